@@ -1,0 +1,37 @@
+"""Staged matrix products of prompts (csrc/gemm_tile.h) at the edges of their tiles, against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# tile of the launch: (T, N, K).  256 x 256 (0.7 of a round of 256 workgroups, one row / column past a tile); 128 x 128 (more than
+# 256 of them); the two K-split forms at whole, ragged and unaligned N; one stage of 64 k, an odd number of stages, two stages
+SHAPES = [(2049, 6145, 64), (2048, 6160, 192), (2300, 2592, 128), (2300, 2590, 320), (300, 200, 128), (257, 130, 256), (1024, 2050, 384),
+          (256, 128, 64), (1100, 2944, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,N,K", SHAPES)
+def test_staged_linear(dtype, T, N, K):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + N + K)
+    x, w, b = (torch.randn(s, generator=g, device="cuda").to(dtype) for s in ((T, K), (N, K), (N,)))
+    code = _lib.seq_dtype_code(dtype)
+    full, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    # an fp32 sum of K products in any order: at most K roundings of 2^-24 of the sum of sizes (and two more for the bias)
+    tol = 2.0 ** -24 * (K + 2) * (size + b.double().abs())
+    out = torch.full((T + 1, N), 7.0, device="cuda")
+    _lib.seq_call("umb_seq_linear", out, x, w, b, T, N, K, 0, code)
+    assert ((out[:T].double() - (full + b.double())).abs() <= tol).all() and bool((out[T] == 7.0).all())
+    out_dt = torch.full((T + 1, N), 7.0, dtype=dtype, device="cuda")
+    _lib.seq_call("umb_seq_linear", out_dt, x, w, None, T, N, K, 1, code)
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11       # unit roundoff of 8 and 11 significant bits
+    assert ((out_dt[:T].double() - full).abs() <= 1.01 * half_ulp * full.abs() + tol + 2.0 ** -25).all() and bool((out_dt[T] == 7.0).all())
+    if N % 2 == 0:                       # stacked halves: silu(gate) * up; |d silu| <= 1.1 |d gate|
+        half = N // 2
+        gate, up, tg, tu = full[:, :half], full[:, half:], tol[:, :half], tol[:, half:]
+        want = gate * torch.sigmoid(gate) * up
+        act = torch.full((T + 1, half), 7.0, dtype=dtype, device="cuda")
+        _lib.seq_call("umb_seq_linear", act, x, w, None, T, N, K, 2, code)
+        bound = 1.02 * half_ulp * want.abs() + 1.1 * tg * up.abs() + gate.abs() * tu + 1e-6 * want.abs() + 2.0 ** -25
+        assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())

@@ -12,6 +12,7 @@
 // A workgroup owns one 16-row output tile and up to 64 tokens; its four waves split K (wave w takes the 32-k steps w, w+4, ...)
 // and their partial tiles are summed through LDS in wave order: the summation order of an output is a function of K alone,
 // never of T or of the row's place in the batch.  K % 8 != 0 (or a tail) falls back to guarded element loads.
+#include "gemm_tile.h"
 #include "seq_common.h"
 
 template <typename P> struct Frag8 { u32x4 v; };
@@ -342,6 +343,113 @@ __global__ __launch_bounds__(256) void seq_linear_wide_kernel(void* __restrict__
   }
 }
 
+// ---- many tokens, both operands dense with whole 64-k stages: the staged product of gemm_tile.h.  DUAL: a wave's RA row tiles are
+// RA / 2 tiles of gate rows and the up rows of the same outputs.  The k order of an output without K-split is the wide kernel's:
+// the same bits.
+template <typename P, int WM, int WN, int RA, int RB, int KS, bool DUAL>
+__global__ __launch_bounds__(64 * WM * WN * KS, RA * RB * KS <= 16 ? 2 : 1)
+void seq_linear_tile_kernel(void* __restrict__ out_, const u16* __restrict__ x, const u16* __restrict__ w, const u16* __restrict__ bias,
+                            int T, int N, int K, int epi, int nbt, float limit, float alpha) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  typedef TileShape<WM, WN, RA, RB, KS> S;
+  constexpr int OUTN = DUAL ? S::BN / 2 : S::BN;
+  const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave_all % S::NW, ks = wave_all / S::NW, j = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
+  const int id = tile_of_block(blockIdx.x, gridDim.x);
+  const int n0 = (id / nbt) * OUTN, t0 = (id % nbt) * S::BT;
+  // rows past the operand's end re-read its last row: their outputs are not stored
+  unsigned voff[S::NPW];
+#pragma unroll
+  for (int i = 0; i < S::NPW; ++i) {
+    const int p = wave + S::NW * i;
+    if (S::NW * i < S::NPA)
+      voff[i] = tile_voff(p, lane, K, [&](int row) {
+        if (!DUAL) return min(n0 + row, N - 1) - n0;
+        const int h = row / (16 * RA), in = row % (16 * RA), up = in / (8 * RA), rr = in % (8 * RA);
+        return min(n0 + h * (8 * RA) + rr, N - 1) - n0 + up * N;
+      });
+    else voff[i] = tile_voff(p - S::NPA, lane, K, [&](int row) { return min(t0 + row, T - 1) - t0; });
+  }
+  f32x4 acc[RA][RB];
+  if (!tile_products<P, WM, WN, RA, RB, KS, false>(acc, smem, w + (long)n0 * K, x + (long)t0 * K, 128, voff, K / 64, wave, ks)) return;
+  const bool v4 = (N & 3) == 0;                              // four outputs of a lane: one store
+#pragma unroll
+  for (int t = 0; t < RB; ++t) {
+    const int tok = t0 + (wn * RB + t) * 16 + j;
+    if (tok >= T) continue;
+#pragma unroll
+    for (int i = 0; i < (DUAL ? RA / 2 : RA); ++i) {
+      const int n = n0 + (DUAL ? wm * (8 * RA) : wm * (16 * RA)) + i * 16 + 4 * g;
+      if (n >= N) continue;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int nn = min(n + r, N - 1);
+        float s = acc[i][t][r] + (bias ? P::to_f(bias[nn]) : 0.f);
+        if constexpr (DUAL) {
+          const float u = acc[i + RA / 2][t][r] + (bias ? P::to_f(bias[N + nn]) : 0.f);
+          s = glu_pair(epi, s, u, limit, alpha);
+        } else if (epi == EPI_RELU2) {
+          const float rl = fmaxf(s, 0.f);
+          s = rl * rl;
+        } else if (epi == EPI_CAP) {
+          s = limit * tanhf(s / limit);
+        }
+        v[r] = s;
+      }
+      const long o = (long)tok * N + n;
+      if (DUAL || epi == EPI_DT || epi == EPI_RELU2) {
+        u16* op = reinterpret_cast<u16*>(out_) + o;
+        if (v4) *reinterpret_cast<u32x2*>(op) = u32x2{pack2<P>(v[0], v[1]), pack2<P>(v[2], v[3])};
+        else
+          for (int r = 0; r < 4; ++r) if (n + r < N) op[r] = P::from_f(v[r]);
+      } else {
+        float* op = reinterpret_cast<float*>(out_) + o;
+        if (v4) *reinterpret_cast<f32x4*>(op) = f32x4{v[0], v[1], v[2], v[3]};
+        else
+          for (int r = 0; r < 4; ++r) if (n + r < N) op[r] = v[r];
+      }
+    }
+  }
+}
+
+template <typename P, int WM, int WN, int RA, int RB, int KS, bool DUAL>
+static int launch_tile_as(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, float limit, float alpha,
+                          hipStream_t st) {
+  typedef TileShape<WM, WN, RA, RB, KS> S;
+  constexpr int OUTN = DUAL ? S::BN / 2 : S::BN;
+  if (ensure_dynamic_lds<seq_linear_tile_kernel<P, WM, WN, RA, RB, KS, DUAL>>(S::LDS) != UMB_OK) return UMB_EHIP;
+  const int nbn = (N + OUTN - 1) / OUTN, nbt = (T + S::BT - 1) / S::BT;
+  hipLaunchKernelGGL((seq_linear_tile_kernel<P, WM, WN, RA, RB, KS, DUAL>), dim3((unsigned)nbn * nbt), dim3(64 * S::NW * KS), S::LDS, st, out,
+                     (const u16*)x, (const u16*)w, (const u16*)bias, T, N, K, epi, nbt, limit, alpha);
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+
+// Which tile: 256 x 256 (8 waves, one workgroup per CU) does 128 x 128 outputs in 0.066 us of the whole chip's time at K = 2048,
+// 128 x 128 (two workgroups per CU) in 0.080, but only whole rounds of 256 workgroups are worth that: it is taken where it fills at
+// least 0.7 of its rounds (T x N x K: 2048 x 16384 x 2048 135 us against 165, 1204 x 28672 x 4096 (0.73) 333 / 363, 1999 x 10240 x 4096
+// (0.62) 214 / 186).  Launches of at most one 128 x 128 workgroup per CU split K over two groups of waves (2048 x 2048 x 8192
+// 73 us / 87), those of at most half as many take tiles of 128 x 64 (300 x 2048 x 2048 13 us / 18).  The kernel before took
+// 225, 474, 290, 137 and 37 us on these five.
+template <typename P, bool DUAL>
+static int launch_tile(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, float limit, float alpha,
+                       hipStream_t st) {
+  const int rows = DUAL ? 2 * N : N;
+  const long big = (long)((rows + 255) / 256) * ((T + 255) / 256), rounds = (big + 255) / 256;
+  if (10 * big >= 7 * 256 * rounds) return launch_tile_as<P, 4, 2, 4, 8, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+  const long mid = (long)((rows + 127) / 128) * ((T + 127) / 128);
+  if (mid <= 128 && K % 128 == 0) return launch_tile_as<P, 2, 2, 4, 2, 2, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+  if (mid <= 256 && K % 128 == 0) return launch_tile_as<P, 2, 2, 4, 4, 2, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+  return launch_tile_as<P, 2, 2, 4, 4, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+}
+
+// whole 64-k stages, 16-byte pieces and stores, 32-bit offsets inside an operand
+static bool tile_ok(const void* out, const void* x, const void* w, int T, int N, int K, int epi) {
+  const long rows = (epi_dual(epi) ? 2L : 1L) * N + 256;
+  return K % 64 == 0 && rows * K < (1L << 31) && ((uintptr_t)out | (uintptr_t)x | (uintptr_t)w) % 16 == 0;
+}
+
 template <typename P>
 static int launch_wide(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
                        const LinExt& ext = LinExt{0, 0, 0, 0, 0, 0, nullptr, nullptr, 0, 0}, int gy = 0) {
@@ -386,6 +494,11 @@ static int launch_vec(void* out, const void* x, const void* w, const void* bias,
   // (the K order of every output is unchanged: a row's value does not depend on which variant computed it)
   const bool dense = gz == 1 && ext.ldx == K && ext.ldo == N && epi != EPI_GATE && epi != EPI_GATE_ROW;
   if (T > 64 && N >= 64 && sizeof(typename El<P>::type) == 2) {
+    if constexpr (sizeof(typename El<P>::type) == 2) {
+      if (VEC && dense && T >= 256 && N >= 128 && tile_ok(out, x, w, T, N, K, epi))
+        return epi_dual(epi) ? launch_tile<P, true>(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, st)
+                             : launch_tile<P, false>(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, st);
+    }
     if (VEC && dense && T >= 256 && N >= 128) return launch_wide<P>(out, x, w, bias, T, N, K, epi, st, LinExt{0, 0, 0, 0, 0, 0, nullptr, nullptr, 0, 0, ext.limit, ext.alpha});      // both operands re-used
     return launch_tt<P, 4, 4, VEC>(out, x, w, bias, T, N, K, epi, st, ext, 0, gz);
   }

@@ -35,3 +35,33 @@ def test_staged_linear(dtype, T, N, K):
         _lib.seq_call("umb_seq_linear", act, x, w, None, T, N, K, 2, code)
         bound = 1.02 * half_ulp * want.abs() + 1.1 * tg * up.abs() + gate.abs() * tu + 1e-6 * want.abs() + 2.0 ** -25
         assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())
+
+
+# wide products of packed dense weights (csrc/dgemm.hip): every tile (one token past 64, a whole one, ragged, 257 = two of 160), K slabs that
+# divide and that do not, a last row tile of 16 rows
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,N,K,S", [(65, 272, 256, 1), (128, 512, 1024, 3), (257, 28672, 128, 1), (300, 4112, 256, 2), (1024, 14336, 128, 1),
+                                     (200, 256, 2048, 5), (513, 2064, 384, 1)])
+def test_wide_dense_product(dtype, T, N, K, S):
+    from umbrella_amd import _lib
+    from umbrella_amd.models.llama import PackedLinear
+    g = torch.Generator(device="cuda").manual_seed(T + N + K)
+    x, w = (torch.randn(s, generator=g, device="cuda").to(dtype) for s in ((T, K), (N, K)))
+    full, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    tol = 2.0 ** -24 * (K + S) * size
+    lin, code = PackedLinear.from_dense(w), _lib.dtype_code(dtype)
+    part = torch.full((S + 1, T, N), 7.0, device="cuda")
+    _lib.call("umb_gemm", part, x, x.stride(0), lin.w, None, T, N, K, 0, S, lin.Rtb, 0, code)
+    assert ((part[:S].double().sum(0) - full).abs() <= tol).all() and bool((part[S] == 7.0).all())
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    out = torch.full((T + 1, N), 7.0, device="cuda")
+    _lib.call("umb_gemm", out, x, x.stride(0), lin.w, None, T, N, K, 0, 1, lin.Rtb, 1, code)
+    assert ((out[:T].double() - full).abs() <= 1.01 * half_ulp * full.abs() + tol + 2.0 ** -25).all() and bool((out[T] == 7.0).all())
+    inter = PackedLinear.from_dense(w, interleave=True)               # gate and up rows in pairs
+    act = torch.full((T + 1, N // 2), 7.0, dtype=dtype, device="cuda")
+    _lib.call("umb_gemm", act, x, x.stride(0), inter.w, None, T, N, K, 0, 1, inter.Rtb, 2, code)
+    gate, up, tg, tu = full[:, :N // 2], full[:, N // 2:], tol[:, :N // 2], tol[:, N // 2:]
+    want = gate * torch.sigmoid(gate) * up
+    # gate, up, silu and the product are each rounded once (|d silu| <= 1.1 |d gate|); 2e-6: the fast exponential
+    bound = 1.05 * half_ulp * (1.1 * gate.abs() * up.abs() + 3 * want.abs()) + 1.1 * tg * up.abs() + 1.1 * gate.abs() * tu + 2e-6 * want.abs() + 2.0 ** -24
+    assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())

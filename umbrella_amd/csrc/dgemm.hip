@@ -1,0 +1,154 @@
+// Wide verify / prompt GEMM of dense 16-bit weights:  out[t][n] = sum_k x[t][k] * W[n][k],  T > 64 tokens, weights in gemm.hip's tile order.
+//
+// Reference call sites: the nn.Linear products of umbrella/models/llama.py (layer_compute, 75-134) at prompts and wide trees.
+//
+// Matrix-pipe bound.  The main loop is that of gemm_tile.h; the packed weights are MFMA fragments already, so a 1-KiB LDS-DMA piece of A
+// is one fragment.  The register-resident kernel it replaces (gemm.hip: 64 x 128 per wave, activations staged through registers, two
+// barriers a step) reached 610 - 730 TFLOP/s on 8B shapes at 1024 tokens; this one 900 - 1200 (figures: dgemm_tile).
+// Split-K partials and epilogues are those of gemm.hip (fp32 [S][T][N]; rounded fp32; SiLU(gate) * up of interleaved rows, S = 1).
+#include "gemm_fused.h"
+#include "gemm_tile.h"
+#include <cstdlib>
+
+template <typename P, int WM, int WN, int RA, int RB, int KS>
+__global__ __launch_bounds__(64 * WM * WN * KS, RA * RB * KS <= 16 ? 2 : 1)
+void dgemm_kernel(const unsigned char* __restrict__ wp, const u16* __restrict__ x, int ldx, int T, int N, int K, int S, int epi, int nbt,
+                  float* __restrict__ out, GemmFused fx) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  typedef TileShape<WM, WN, RA, RB, KS> Sh;
+  const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave_all % Sh::NW, ks = wave_all / Sh::NW, j = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
+  const int id = tile_of_block(blockIdx.x, gridDim.x), tiles = gridDim.x / S;
+  const int sp = id / tiles, tile = id % tiles;
+  const int n0 = (tile / nbt) * Sh::BN, t0 = (tile % nbt) * Sh::BT;
+  const int nst = K / 64, per = (nst + S - 1) / S, st0 = min(nst, sp * per), st1 = min(nst, st0 + per);
+  const int last = (N - n0) / 16 - 1;                        // row tiles and rows past the operand's end re-read its last one: not stored
+  unsigned voff[Sh::NPW];
+#pragma unroll
+  for (int i = 0; i < Sh::NPW; ++i) {
+    const int p = wave + Sh::NW * i;
+    if (Sh::NW * i < Sh::NPA) voff[i] = ((unsigned)min(p >> 1, last) * (unsigned)(K / 32) + (unsigned)(p & 1)) * 1024u + (unsigned)lane * 16u;
+    else voff[i] = tile_voff(p - Sh::NPA, lane, ldx, [&](int row) { return min(t0 + row, T - 1) - t0; });
+  }
+  f32x4 acc[RA][RB];
+  if (st0 < st1) {
+    if (!tile_products<P, WM, WN, RA, RB, KS, true>(acc, smem, wp + ((long)(n0 / 16) * (K / 32) + st0 * 2) * 1024,
+                                                    x + (long)t0 * ldx + st0 * 64, 2048, voff, st1 - st0, wave, ks)) return;
+  } else {                                                   // a slab past the last stage: its partial is zero
+#pragma unroll
+    for (int i = 0; i < RA; ++i)
+#pragma unroll
+      for (int t = 0; t < RB; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (ks) return;
+  }
+#pragma unroll
+  for (int t = 0; t < RB; ++t) {
+    const int tok = t0 + (wn * RB + t) * 16 + j;
+    if (tok >= T) continue;
+    float inv = 1.f;
+    if (fx.ssq_in) {
+      const float* sq = fx.ssq_in + (long)tok * (fx.ssq_stride ? fx.ssq_stride : fx.ssq_groups);
+      float a = 0.f;
+      for (int q = 0; q < fx.ssq_groups; q += 4) { const f32x4 v = *reinterpret_cast<const f32x4*>(sq + q); a += v[0]; a += v[1]; a += v[2]; a += v[3]; }
+      inv = rsqrtf(a / fx.ssq_dim + fx.eps);
+    }
+#pragma unroll
+    for (int i = 0; i < RA; ++i) {
+      const int n = n0 + (wm * RA + i) * 16;
+      if (n >= N) continue;
+      f32x4 v = acc[i][t];
+      if (epi == EPI_SILU) {
+        v *= inv;
+        const float g0 = rnd<P>(v[0]), u0 = rnd<P>(v[1]), g1 = rnd<P>(v[2]), u1 = rnd<P>(v[3]);
+        const float a0 = rnd<P>(g0 / (1.f + __expf(-g0))) * u0, a1 = rnd<P>(g1 / (1.f + __expf(-g1))) * u1;
+        u16* act = reinterpret_cast<u16*>(out);
+        *reinterpret_cast<unsigned*>(act + (long)tok * (N / 2) + n / 2 + g * 2) = pack2<P>(a0, a1);
+      } else {
+        if (epi == EPI_ROUND) { v *= inv; v[0] = rnd<P>(v[0]); v[1] = rnd<P>(v[1]); v[2] = rnd<P>(v[2]); v[3] = rnd<P>(v[3]); }
+        *reinterpret_cast<f32x4*>(out + ((long)sp * T + tok) * N + n + g * 4) = v;
+      }
+    }
+  }
+}
+
+template <typename P, int WM, int WN, int RA, int RB, int KS>
+static int dgemm_launch(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int S, int epi, const GemmFused& fx, hipStream_t st) {
+  typedef TileShape<WM, WN, RA, RB, KS> Sh;
+  static bool attr_done[64] = {};
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  if (dev >= 0 && dev < 64 && !attr_done[dev]) {
+    if (hipFuncSetAttribute((const void*)dgemm_kernel<P, WM, WN, RA, RB, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Sh::LDS) != hipSuccess)
+      return UMB_EHIP;
+    attr_done[dev] = true;
+  }
+  const int nbt = (T + Sh::BT - 1) / Sh::BT;
+  hipLaunchKernelGGL((dgemm_kernel<P, WM, WN, RA, RB, KS>), dim3((unsigned)((N + Sh::BN - 1) / Sh::BN) * nbt * S), dim3(64 * Sh::NW * KS), Sh::LDS, st,
+                     (const unsigned char*)wp, x, ldx, T, N, K, S, epi, nbt, out, fx);
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+
+// The tiles a launch chooses from and what a 64-k stage of one round of 256 workgroups takes (us; one MI355X, bf16 and fp16, random data).
+// 128 x 128 runs two workgroups per CU (a round of 512 takes two); the K-split forms are for launches of at most one workgroup per CU.
+//                        rows tokens stage us
+enum { TILE_256 = 0,   //  256   256   1.5
+       TILE_160 = 1,   //  256   160   1.1     257 tokens are two of these and not two of 256
+       TILE_128 = 2,   //  128   128   0.52
+       TILE_128K = 3,  //  128   128   0.56    K over two groups of waves
+       TILE_64K = 4 }; //  128    64   0.39    the same
+// Least sum of rounds x stages x stage time over the tiles.  28672 x 4096 weights: 257 tokens 74 us (TILE_160; 102 with TILE_256 or
+// TILE_128; the register-resident kernel 141), 385 tokens 102 (TILE_256; 120 - 137; 153), 1024 tokens 200 (TILE_256; 242 - 282; 328);
+// 4096 x 4096, 257 tokens, S = 2: 21 us (TILE_128K; 24 - 27; 52).
+static double dgemm_tile(int T, int N, int K, int S, int* tile) {
+  static const struct { int bn, bt; double us; bool ksplit; } kind[5] = {
+      {256, 256, 1.5, false}, {256, 160, 1.1, false}, {128, 128, 0.52, false}, {128, 128, 0.56, true}, {128, 64, 0.39, true}};
+  const bool even = K % (128 * S) == 0;
+  double best = 1e30;
+  for (int i = 0; i < 5; ++i) {
+    const long wgs = (long)((N + kind[i].bn - 1) / kind[i].bn) * ((T + kind[i].bt - 1) / kind[i].bt) * S, rounds = (wgs + 255) / 256;
+    if (kind[i].ksplit && (rounds > 1 || !even)) continue;
+    // a lone workgroup of the two-per-CU form leaves half the wave slots empty
+    const double cost = rounds * ((K / 64 + S - 1) / S) * (i == TILE_128 && rounds == 1 ? 0.62 : kind[i].us) + 4.0;
+    if (cost < best) { best = cost; *tile = i; }
+  }
+  return best;
+}
+
+template <typename P>
+static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int S, int epi, const GemmFused& fx, hipStream_t st) {
+  int tile = TILE_128;
+  (void)dgemm_tile(T, N, K, S, &tile);
+  switch (tile) {
+    case TILE_256: return dgemm_launch<P, 4, 2, 4, 8, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+    case TILE_160: return dgemm_launch<P, 4, 2, 4, 5, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+    case TILE_128: return dgemm_launch<P, 2, 2, 4, 4, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+    case TILE_128K: return dgemm_launch<P, 2, 2, 4, 4, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+    default: return dgemm_launch<P, 2, 2, 4, 2, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+  }
+}
+
+// Up to 128 tokens against more weights than the last-level cache holds the product is bound by HBM, and gemm.hip's register-resident
+// kernel streams them faster (128256 x 4096, 100 tokens: 195 us, 217 here; 160 tokens: 377, 250 here).
+bool umb_dgemm_ok(const void* x, int ldx, int T, int N, int K, int S, int epi) {
+  static const bool off = getenv("UMB_NO_VGEMM") != nullptr || getenv("UMB_VGEMM_PLAIN") != nullptr;     // gemm.hip's diagnostics
+  return !off && T > 64 && K % 64 == 0 && N % 16 == 0 && ldx % 8 == 0 && (uintptr_t)x % 16 == 0 && epi <= EPI_SILU &&
+         (long)ldx * 512 < (1L << 31) && (T > 128 || (long)N * K * 2 <= (512L << 20));
+}
+
+// K slabs of a wide dense product whose partials are summed by the kernel behind it: the least of the product's time and of what the
+// partials beyond the first cost (written and read, 3 TB/s).  1024 tokens: 6144 x 4096 S = 1, 4096 x 14336 S = 2 (118 -> 99 us)
+int umb_dgemm_split(int T, int N, int K, int S_plan) {
+  int best_s = 1, tile = 0;
+  double best = 1e30;
+  for (int S = 1; S <= S_plan && S <= K / 128 && (long)S * T * N * 4 < (1L << 31); ++S) {
+    const double cost = dgemm_tile(T, N, K, S, &tile) + (S - 1) * (double)T * N * 4 / 3e6;
+    if (cost < best) { best = cost; best_s = S; }
+  }
+  return best_s;
+}
+
+int umb_dgemm(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int S, int epi, const GemmFused& fx, int dtype,
+              hipStream_t st) {
+  DISPATCH_DTYPE(dtype, { return dgemm_any<P>(wp, x, ldx, out, T, N, K, S, epi, fx, st); })
+}

@@ -30,10 +30,12 @@ template <int WM, int WN, int RA, int RB, int KS> struct TileShape {
   static constexpr int NW = WM * WN;                          // waves of one K group
   static constexpr int BN = 16 * WM * RA, BT = 16 * WN * RB;  // rows of A, tokens of B
   static constexpr int NPA = BN / 8, NPB = BT / 8;            // 1-KiB pieces of a stage
-  static constexpr int NPW = (NPA + NPB) / NW;                // pieces a wave fetches per stage
+  static constexpr int NPW = (NPA + NPB + NW - 1) / NW;       // pieces a wave fetches per stage
   static constexpr unsigned SLOT = (NPA + NPB) * 1024u;
-  static constexpr size_t LDS = (size_t)KS * 2 * SLOT;
-  static_assert(NPA % NW == 0 && NPB % NW == 0 && (KS == 1 || RA * RB * NW * 1024u <= LDS), "pieces deal out evenly; a group's tile fits the slots");
+  // where the pieces do not deal out evenly, a wave without a last piece of its own fetches into the KiB behind the slots
+  static constexpr bool EVEN = (NPA + NPB) % NW == 0;
+  static constexpr size_t LDS = (size_t)KS * 2 * SLOT + (EVEN ? 0 : 1024);
+  static_assert(NPA % NW == 0 && (EVEN || KS == 1) && (KS == 1 || RA * RB * NW * 1024u <= LDS), "whole rounds of A pieces; a group's tile fits the slots");
 };
 
 // Row block of a workgroup: the hardware deals consecutive workgroups to the eight XCDs in turn; here the workgroups of one XCD get
@@ -63,7 +65,8 @@ __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned cha
   const unsigned lds0 = (unsigned)(size_t)(lds_char*)smem + (unsigned)ks * 2u * S::SLOT;
   const int n = nst / KS;                                     // stages of this group
   auto issue = [&](int st, int i) {
-    const unsigned dst = lds0 + (unsigned)(st & 1) * S::SLOT + (unsigned)(wave + NW * i) * 1024u;
+    unsigned dst = lds0 + (unsigned)(st & 1) * S::SLOT + (unsigned)(wave + NW * i) * 1024u;
+    if (!S::EVEN && i == NPW - 1 && wave + NW * i >= NPA + S::NPB) dst = lds0 + 2u * S::SLOT;
     const long s = (long)min(st, n - 1) * KS + ks;
     if (NW * i < NPA) tile_dma(voff[i], static_cast<const char*>(abase) + s * astep, dst);
     else tile_dma(voff[i], static_cast<const char*>(bbase) + s * 128, dst);

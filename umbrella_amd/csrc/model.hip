@@ -28,7 +28,9 @@ static inline int dbg_sync(const char* what, hipStream_t st) {
 // CU's ~60 GB/s (0.55 us per split at N = 8192) -- worth more than the last splits give the GEMM when K is short
 // (70B o-proj, T = 13: S = 8 -> 4 costs the GEMM +0.4 us and saves the reduce 2.2 us; 70B down, K = 28672, keeps 8;
 // 8B-AWQ down keeps 8 of its planned 16).  A function of the layer shape only, like the plan itself.
+int umb_dgemm_split(int T, int N, int K, int S_plan);     // dgemm.hip: dense weights, wide forwards
 static inline int eff_s(const UmbLinear& l, int T, bool row_reduce = false) {
+  if (!l.awq && T > 64) return umb_dgemm_split(T, l.N, l.K, l.S);
   int S = umb_gemm_wide_split(T, l.N, l.S);
   if (row_reduce && T <= 64 && l.S_row > 0) return l.S_row;       // the plan's measured choice (umb_gemm_plan2)
   if (row_reduce && T <= 64) {

@@ -65,3 +65,31 @@ def test_wide_dense_product(dtype, T, N, K, S):
     # gate, up, silu and the product are each rounded once (|d silu| <= 1.1 |d gate|); 2e-6: the fast exponential
     bound = 1.05 * half_ulp * (1.1 * gate.abs() * up.abs() + 3 * want.abs()) + 1.1 * tg * up.abs() + 1.1 * gate.abs() * tu + 2e-6 * want.abs() + 2.0 ** -24
     assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())
+
+
+# the chunked kernel of few tokens: token counts around its tiles (8 / 16 / 32 / 48 / 64 and two token tiles), one chunk of K, fewer chunks than
+# ring slots, ragged output rows
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("N,K", [(40, 256), (4134, 512), (272, 1280)])
+def test_few_token_linear(dtype, N, K):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    code = _lib.seq_dtype_code(dtype)
+    x, w, b = (torch.randn(s, generator=g, device="cuda").to(dtype) for s in ((100, K), (N, K), (N,)))
+    full, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    tol = 2.0 ** -24 * (K + 2) * (size + b.double().abs())
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
+    rows = None
+    for T in (1, 8, 9, 17, 33, 48, 64, 65, 100):
+        out = torch.full((T + 1, N), 7.0, device="cuda")
+        _lib.seq_call("umb_seq_linear", out, x[:T].contiguous(), w, b, T, N, K, 0, code)
+        assert ((out[:T].double() - (full[:T] + b.double())).abs() <= tol[:T]).all() and bool((out[T] == 7.0).all())
+        rows = out[:1].clone() if rows is None else rows
+        assert torch.equal(out[:1], rows)                      # the sum's order does not depend on the other rows
+        half = N // 2
+        act = torch.full((T + 1, half), 7.0, dtype=dtype, device="cuda")
+        _lib.seq_call("umb_seq_linear", act, x[:T].contiguous(), w, None, T, N, K, 2, code)
+        gate, up, tg, tu = full[:T, :half], full[:T, half:], tol[:T, :half], tol[:T, half:]
+        want = gate * torch.sigmoid(gate) * up
+        bound = 1.02 * unit * want.abs() + 1.1 * tg * up.abs() + gate.abs() * tu + 1e-6 * want.abs() + 2.0 ** -25
+        assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())

@@ -9,9 +9,9 @@
 // (n = 4 (l / 16) + r, token = l % 16), r = 0..3.  Weights go HBM -> VGPR (every weight element is used by exactly one wave of
 // a <= 64-token launch), as in the skinny GEMM of gemm.hip.
 //
-// A workgroup owns one 16-row output tile and up to 64 tokens; its four waves split K (wave w takes the 32-k steps w, w+4, ...)
+// Few tokens: a workgroup owns 16 (or 32) output rows and up to 64 tokens; its four waves split K (wave w takes the 32-k steps w, w+4, ...)
 // and their partial tiles are summed through LDS in wave order: the summation order of an output is a function of K alone,
-// never of T or of the row's place in the batch.  K % 8 != 0 (or a tail) falls back to guarded element loads.
+// never of the row's place in the batch, and of T only where the many-token kernels take over (launch_vec).  K % 8 != 0 (or a tail) falls back to guarded element loads.
 #include "gemm_tile.h"
 #include "seq_common.h"
 
@@ -468,6 +468,212 @@ static int launch_wide(void* out, const void* x, const void* w, const void* bias
   }
 }
 
+// ---- whole 512-byte pieces of K: both operands of a step staged through LDS in contiguous runs.
+// The kernel above asks for a fragment with one load of 16 rows x 64 B.  Rows of a power-of-two stride sit on the same L2 channel, so
+// such a load takes ~75 cycles of a CU's path whether the rows are weights or tokens, and a launch of 16 and more tokens is bound by
+// its TOKEN fragments (4096 x 14336 weights: 27 us with 1 token, 38 with 16, 80 with 64).  Here a workgroup walks K in chunks of 512
+// bytes per row: LDS-DMA pieces of two rows (whole lines, 4 channels' worth each) into a ring of R slots, R - 1 chunks ahead, one
+// barrier per chunk; the tokens of a chunk are fetched once per workgroup and not once per wave; fragments come from LDS without bank
+// conflicts (pieces 1040 B apart, columns of odd rows XOR 8).  Wave w takes the 32-k steps w, w + 4, ... as above: the same bits.
+// us, cold weights, one MI355X: 4096 x 14336, 1 / 16 / 48 / 64 tokens 27 / 38 / 66 / 80 -> 24 / 25 / 38 / 41; 2048 x 2048, 48 tokens
+// 11.7 -> 7.3; gate/up 28672 x 4096, 1 / 16 / 48 tokens 49 / 58 / 88 -> 42 / 43 / 56 (5.6 TB/s at 1 token).
+template <int NT, int TT, int BP, bool DUAL, int R> struct StreamShape {     // BP: token pieces (8 TT, fewer for very few tokens)
+  static constexpr int AP = (DUAL ? 16 : 8) * NT, NP = AP + BP, PW = (NP + 3) / 4, AT = DUAL ? 2 * NT : NT;
+  static constexpr unsigned PIECE = 1040u, SLOT = NP * PIECE;
+  static constexpr size_t RED = (size_t)AT * 4 * TT * 1024, RING = (size_t)R * SLOT + (NP % 4 ? PIECE : 0);
+  static constexpr size_t LDS = RING > RED ? RING : RED;
+  static_assert(AP % 4 == 0 && R >= 2 && LDS <= 160 * 1024, "whole rounds of weight pieces; the CU's LDS");
+};
+template <typename P, int NT, int TT, int BP, bool DUAL, int R>
+__global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict__ out_, const typename El<P>::type* __restrict__ x,
+                                                                const typename El<P>::type* __restrict__ w,
+                                                                const typename El<P>::type* __restrict__ bias, int T, int N, int K,
+                                                                int epi, LinExt ext) {
+  typedef typename El<P>::type E;
+  typedef StreamShape<NT, TT, BP, DUAL, R> S;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr int EB = sizeof(E), STEPS = 512 / (32 * EB), AT = S::AT;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = lane & 15, g = lane >> 4;
+  int t0 = blockIdx.y * (TT * 16);
+  const int ldx = ext.ldx, ldo = ext.ldo;
+  long obase = (long)blockIdx.z * ext.so;
+  const float* gate = ext.gate ? ext.gate + (long)blockIdx.z * ext.sg : nullptr;
+  x += (long)blockIdx.z * ext.sx;
+  w += (long)blockIdx.z * ext.sw;
+  if (ext.tiles) {                         // grouped: this workgroup's rows and weights come from the tile list
+    const int* td = ext.tiles + 3 * blockIdx.y;
+    const int rows = __builtin_amdgcn_readfirstlane(td[2]);
+    if (rows <= 0) return;
+    const long first = __builtin_amdgcn_readfirstlane(td[1]);
+    w += (long)__builtin_amdgcn_readfirstlane(td[0]) * ext.gs;
+    x += first * ldx;
+    obase += first * ldo;
+    T = rows;
+    t0 = 0;
+  }
+  const int n0 = blockIdx.x * 16 * NT;
+  const unsigned lds0 = (unsigned)(size_t)(lds_char*)smem;
+  // piece p: rows 2 p and 2 p + 1 (lanes 0 - 31, 32 - 63) of the operand; rows past its end re-read the last one: not stored
+  unsigned voff[S::PW];
+#pragma unroll
+  for (int i = 0; i < S::PW; ++i) {
+    const int p = wave + 4 * i, odd = lane >> 5, c = (lane & 31) ^ (odd * 8);
+    if (4 * i < S::AP) {
+      const int r = 2 * p + odd;
+      const int n = DUAL && r >= 16 * NT ? N + min(n0 + r - 16 * NT, N - 1) : min(n0 + r, N - 1);
+      voff[i] = (unsigned)(n - n0) * (unsigned)K * EB + c * 16u;
+    } else {
+      voff[i] = (unsigned)(min(t0 + 2 * (p - S::AP) + odd, T - 1) - t0) * (unsigned)ldx * EB + c * 16u;
+    }
+  }
+  const char* wb = reinterpret_cast<const char*>(w + (long)n0 * K);
+  const char* xb = reinterpret_cast<const char*>(x + (long)t0 * ldx);
+  const int nc = K * EB / 512;
+  auto issue = [&](int c, int slot) {
+    const long at = (long)min(c, nc - 1) * 512;
+#pragma unroll
+    for (int i = 0; i < S::PW; ++i) {
+      unsigned dst = lds0 + (unsigned)slot * S::SLOT + (unsigned)(wave + 4 * i) * S::PIECE;
+      if (S::NP % 4 && i == S::PW - 1 && wave + 4 * i >= S::NP) dst = lds0 + (unsigned)R * S::SLOT;      // a piece of nobody's
+      tile_dma(voff[i], (4 * i < S::AP ? wb : xb) + at, dst);
+    }
+  };
+  f32x4 acc[AT][TT];
+#pragma unroll
+  for (int i = 0; i < AT; ++i)
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) acc[i][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned rowb = (unsigned)(j >> 1) * S::PIECE + (unsigned)(j & 1) * 512u, swz = (unsigned)(j & 1) * 8u;
+  auto frag = [&](unsigned base, int s) {  // 16 rows, the 32 k of step s
+    const auto at = [&](int c) { return *reinterpret_cast<const lds_u32x4*>((size_t)(base + rowb + (((unsigned)c) ^ swz) * 16u)); };
+    Frag8<P> f;
+    if constexpr (EB == 2) f.v = at(s * 4 + g);
+    else {
+      f.lo = __builtin_bit_cast(f32x4, at(s * 8 + 2 * g));
+      f.hi = __builtin_bit_cast(f32x4, at(s * 8 + 2 * g + 1));
+    }
+    return f;
+  };
+#pragma unroll
+  for (int c = 0; c < R - 1; ++c) issue(c, c);
+  int slot = 0;
+  for (int c = 0; c < nc; ++c) {
+    // this wave's pieces of the chunk have landed and its fragments of the chunk before are in registers; behind the barrier that holds
+    // for every wave: the chunk can be read, and the slot of the chunk before filled again
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((R - 2) * S::PW) : "memory");
+    __builtin_amdgcn_s_barrier();
+    issue(c + R - 1, slot == 0 ? R - 1 : slot - 1);
+    const unsigned base = lds0 + (unsigned)slot * S::SLOT;
+#pragma unroll
+    for (int u = 0; u < STEPS / 4; ++u) {
+      const int s = wave + 4 * u;
+      Frag8<P> a[AT], b[TT];
+#pragma unroll
+      for (int i = 0; i < AT; ++i) a[i] = frag(base + (unsigned)(8 * i) * S::PIECE, s);
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) b[tt] = frag(base + (unsigned)(S::AP + 8 * tt) * S::PIECE, s);
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int i = 0; i < AT; ++i) acc[i][tt] = mma8<P>(a[i], b[tt], acc[i][tt]);
+    }
+    slot = slot + 1 == R ? 0 : slot + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  float* red = reinterpret_cast<float*>(smem);                       // [wave][AT][TT][256], over the ring
+#pragma unroll
+  for (int i = 0; i < AT; ++i)
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) *reinterpret_cast<f32x4*>(red + ((wave * AT + i) * TT + tt) * 256 + lane * 4) = acc[i][tt];
+  __syncthreads();
+  const int l = threadIdx.x >> 2, r = threadIdx.x & 3;
+  auto total = [&](int i, int tt) {
+    float s = red[(i * TT + tt) * 256 + threadIdx.x];
+#pragma unroll
+    for (int ww = 1; ww < 4; ++ww) s += red[((ww * AT + i) * TT + tt) * 256 + threadIdx.x];
+    return s;
+  };
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = n0 + nt * 16 + 4 * (l >> 4) + r;
+    if (n >= N) continue;
+    const float bv = bias ? ldf<P>(bias + n) : 0.f;
+    const float bv2 = (DUAL && bias) ? ldf<P>(bias + N + n) : 0.f;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+      const int t = t0 + tt * 16 + (l & 15);
+      if (t >= T) continue;
+      const float s = total(nt, tt) + bv;
+      const long o = obase + (long)t * ldo + n;
+      if constexpr (DUAL) {
+        stf<P>(reinterpret_cast<E*>(out_) + o, glu_pair(epi, s, total(NT + nt, tt) + bv2, ext.limit, ext.alpha));
+      } else if (epi == EPI_DT) {
+        stf<P>(reinterpret_cast<E*>(out_) + o, s);
+      } else if (epi == EPI_RELU2) {
+        const float rl = fmaxf(s, 0.f);
+        stf<P>(reinterpret_cast<E*>(out_) + o, rl * rl);
+      } else if (epi == EPI_GATE) {
+        stf<P>(reinterpret_cast<E*>(out_) + o, s / (1.f + expf(-gate[(long)t * ext.ldg + n])));
+      } else if (epi == EPI_GATE_ROW) {
+        stf<P>(reinterpret_cast<E*>(out_) + o, s / (1.f + expf(-gate[(long)t * ext.ldg])));
+      } else if (epi == EPI_CAP) {
+        reinterpret_cast<float*>(out_)[o] = ext.limit * tanhf(s / ext.limit);
+      } else {
+        reinterpret_cast<float*>(out_)[o] = s;
+      }
+    }
+  }
+}
+
+template <typename P, int NT, int TT, int BP, bool DUAL, int R>
+static int launch_stream_as(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
+                            const LinExt& ext, int gy, int gz) {
+  typedef typename El<P>::type E;
+  typedef StreamShape<NT, TT, BP, DUAL, R> S;
+  if (ensure_dynamic_lds<seq_linear_stream_kernel<P, NT, TT, BP, DUAL, R>>(S::LDS) != UMB_OK) return UMB_EHIP;
+  hipLaunchKernelGGL((seq_linear_stream_kernel<P, NT, TT, BP, DUAL, R>), dim3((N + 16 * NT - 1) / (16 * NT), gy > 0 ? gy : (T + 16 * TT - 1) / (16 * TT), gz),
+                     dim3(256), S::LDS, st, out, (const E*)x, (const E*)w, (const E*)bias, T, N, K, epi, ext);
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+
+// T: tokens of a token tile at most (grouped launches), of the launch otherwise.  Ring depth: as many chunks ahead as leave two
+// workgroups on a CU for one token tile, one workgroup for more (gate/up of 32 tokens: two, 48 us against 51).  32 output rows per
+// workgroup halve the token traffic of launches that stay above one workgroup per CU (32000 x 2048, 48 tokens 51 -> 37 us; 4096 x 4096,
+// 256 workgroups of 16 rows: 12.4 us, 15.3 as 128 of 32).
+template <typename P>
+static int launch_stream(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
+                         const LinExt& ext, int gy = 0, int gz = 1) {
+#define STREAM(NT, TT, BP, DUAL, R) return launch_stream_as<P, NT, TT, BP, DUAL, R>(out, x, w, bias, T, N, K, epi, st, ext, gy, gz)
+  if (epi_dual(epi)) {
+    if (T <= 8) STREAM(1, 1, 4, true, 3);
+    if (T <= 16) STREAM(1, 1, 8, true, 3);
+    if (T <= 32) STREAM(1, 2, 16, true, 2);
+    if (T <= 48) STREAM(1, 3, 24, true, 3);
+    STREAM(1, 4, 32, true, 3);
+  }
+  if (T <= 8) STREAM(1, 1, 4, false, 4);
+  if (T <= 16) STREAM(1, 1, 8, false, 4);
+  if (T <= 32) STREAM(1, 2, 16, false, 3);
+  const bool narrow = (long)((N + 15) / 16) * (gy > 0 ? gy : (T + 63) / 64) * gz <= 256;
+  if (T <= 48) {
+    if (narrow) STREAM(1, 3, 24, false, 3);
+    STREAM(2, 3, 24, false, 3);
+  }
+  if (narrow) STREAM(1, 4, 32, false, 3);
+  STREAM(2, 4, 32, false, 3);
+#undef STREAM
+}
+
+// whole chunks, 16-byte pieces from every row start, 32-bit offsets inside a workgroup's operands
+static bool stream_ok(const void* x, const void* w, int N, int K, int epi, const LinExt& ext, int eb) {
+  auto al = [eb](long n) { return n * eb % 16 == 0; };
+  return (long)K * eb % 512 == 0 && al(ext.ldx) && al(ext.sx) && al(ext.sw) && al(ext.gs) && ((uintptr_t)x | (uintptr_t)w) % 16 == 0 &&
+         ((epi_dual(epi) ? (long)N : 0L) + 64) * K * eb < (1L << 32) && (long)ext.ldx * 64 * eb < (1L << 32);
+}
+
 // gy > 0: the number of token tiles is given (grouped launches); gz: independent problems
 template <typename P, int NT, int TT, bool VEC>
 static int launch_tt(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
@@ -488,17 +694,24 @@ static int launch_tt(void* out, const void* x, const void* w, const void* bias, 
 template <typename P, bool VEC>
 static int launch_vec(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
                       const LinExt& ext, int gz = 1) {
+  const bool dense = gz == 1 && ext.ldx == K && ext.ldo == N && epi != EPI_GATE && epi != EPI_GATE_ROW;
+  const bool stream = VEC && stream_ok(x, w, N, K, epi, ext, sizeof(typename El<P>::type));
+  if constexpr (sizeof(typename El<P>::type) == 2) {
+    // both operands re-used: from 256 tokens on, and for 65 and more where the launch has some 100 tiles of 128 x 128 (cold weights, 100 /
+    // 200 tokens: 18496 x 4096 56 / 72 us, the streaming kernel 84 / 158; 4096 x 4096 41 / 39 us, streaming 18 / 32; 2048 x 8192,
+    // 255 tokens 73 us, streaming 29)
+    const long rows = (long)(epi_dual(epi) ? 2 : 1) * N, tiles = (rows + 127) / 128 * ((T + 127) / 128);
+    if (T > 64 && VEC && dense && N >= 128 && tile_ok(out, x, w, T, N, K, epi) && !(stream && tiles < (T < 256 ? 96 : 49)) &&
+        (T >= 256 || tiles >= 96))
+      return epi_dual(epi) ? launch_tile<P, true>(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, st)
+                           : launch_tile<P, false>(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, st);
+  }
+  if (stream) return launch_stream<P>(out, x, w, bias, T, N, K, epi, st, ext, 0, gz);
   if (T <= 16) return launch_tt<P, 1, 1, VEC>(out, x, w, bias, T, N, K, epi, st, ext, 0, gz);
   if (T <= 32) return launch_tt<P, 1, 2, VEC>(out, x, w, bias, T, N, K, epi, st, ext, 0, gz);
   // many tokens: the launch is bound by fragment loads per MFMA, not by weight bytes -> four output tiles per workgroup
-  // (the K order of every output is unchanged: a row's value does not depend on which variant computed it)
-  const bool dense = gz == 1 && ext.ldx == K && ext.ldo == N && epi != EPI_GATE && epi != EPI_GATE_ROW;
+  // (the K order of every output is unchanged)
   if (T > 64 && N >= 64 && sizeof(typename El<P>::type) == 2) {
-    if constexpr (sizeof(typename El<P>::type) == 2) {
-      if (VEC && dense && T >= 256 && N >= 128 && tile_ok(out, x, w, T, N, K, epi))
-        return epi_dual(epi) ? launch_tile<P, true>(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, st)
-                             : launch_tile<P, false>(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, st);
-    }
     if (VEC && dense && T >= 256 && N >= 128) return launch_wide<P>(out, x, w, bias, T, N, K, epi, st, LinExt{0, 0, 0, 0, 0, 0, nullptr, nullptr, 0, 0, ext.limit, ext.alpha});      // both operands re-used
     return launch_tt<P, 4, 4, VEC>(out, x, w, bias, T, N, K, epi, st, ext, 0, gz);
   }
@@ -572,11 +785,13 @@ static int seq_linear_grouped_any(void* out, const void* x, const void* w, const
   }
   if (tile_rows == 16) {                   // a few rows in all (decoding): one 16-row output tile per workgroup, many workgroups
     DISPATCH_SEQ_DTYPE(dtype, {
+      if (stream_ok(x, w, N, K, epi, ext, sizeof(typename El<P>::type))) return launch_stream<P>(out, x, w, nullptr, 16, N, K, epi, st, ext, max_tiles);
       if (K % 8 == 0 && gs % 8 == 0) return launch_tt<P, 1, 1, true>(out, x, w, nullptr, 16, N, K, epi, st, ext, max_tiles);
       return launch_tt<P, 1, 1, false>(out, x, w, nullptr, 16, N, K, epi, st, ext, max_tiles);
     })
   }
   DISPATCH_SEQ_DTYPE(dtype, {
+    if (stream_ok(x, w, N, K, epi, ext, sizeof(typename El<P>::type))) return launch_stream<P>(out, x, w, nullptr, 64, N, K, epi, st, ext, max_tiles);
     if (K % 8 == 0 && gs % 8 == 0) {
       if (N >= 64 && sizeof(typename El<P>::type) == 2) return launch_tt<P, 4, 4, true>(out, x, w, nullptr, 64, N, K, epi, st, ext, max_tiles);
       return launch_tt<P, 1, 4, true>(out, x, w, nullptr, 64, N, K, epi, st, ext, max_tiles);

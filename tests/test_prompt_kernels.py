@@ -93,3 +93,45 @@ def test_few_token_linear(dtype, N, K):
         want = gate * torch.sigmoid(gate) * up
         bound = 1.02 * unit * want.abs() + 1.1 * tg * up.abs() + gate.abs() * tu + 1e-6 * want.abs() + 2.0 ** -25
         assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())
+
+
+# rows in quads: every workgroup size (64 ... 1024 threads, two quads a thread), a group that ends inside the last wave, several groups
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("W,groups", [(8, 1), (200, 1), (1024, 2), (1200, 1), (3072, 3), (2052, 1), (4096, 1), (4100, 1), (8192, 1)])
+def test_norms_in_quads(dtype, W, groups):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(W + groups)
+    T, eps, code = 3, 1e-5, _lib.seq_dtype_code(dtype)
+    x, y, y2 = (torch.randn(T, W, generator=g, device="cuda") * s for s in (3.0, 50.0, 0.2))
+    w1, w2, w3, w4 = ((1 + 0.2 * torch.randn(W, generator=g, device="cuda")).to(dtype) for _ in range(4))
+
+    def norm(v, w, n=groups):
+        v = v.double().view(T, n, -1)
+        return (v / (v.pow(2).mean(-1, keepdim=True) + eps).sqrt()).view(T, W) * w.double()
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -22}[dtype]
+
+    def close(got, want, u=2.0 ** -21):              # fp32: a handful of roundings of 2^-24, the sum of squares W of them at most (averaged)
+        return bool(((got.double() - want).abs() <= (u + 2.0 ** -20) * want.abs() + 2.0 ** -20).all())
+    out, h = torch.empty(T, W, device="cuda"), torch.full((T + 1, W), 7.0, dtype=dtype, device="cuda")
+    _lib.seq_call("umb_seq_group_norm", out, h, x, None, w1, T, W, groups, eps, code)
+    assert close(out, norm(x, w1)) and close(h[:T], norm(x, w1), unit) and bool((h[T] == 7.0).all())
+    xd = x.clone()
+    _lib.seq_call("umb_seq_resid_norm", xd, h, y, w1, w2, T, W, groups, eps, code)
+    new = x.double() + norm(y, w1)
+    assert close(xd, new) and close(h[:T], norm(new, w2), unit + 2.0 ** -18) and bool((h[T] == 7.0).all())
+    table = torch.randn(11, W, generator=g, device="cuda").to(dtype)
+    ids = torch.tensor([4, 99, -1], dtype=torch.int32, device="cuda")
+    _lib.seq_call("umb_seq_embed_norm", xd, h, table, ids, 1.5, w2, T, W, 11, groups, eps, code)
+    rows = table.double()[[4, 10, 0]] * 1.5
+    assert close(xd, rows) and close(h[:T], norm(rows, w2), unit)
+    xd = x.clone()
+    _lib.seq_call("umb_seq_pair_resid_norm", xd, h, y, y2, w1, w2, 0.5, w3, w4, T, W, eps, code)
+    pair = 0.5 * (norm(y, w1, 1) + norm(y2, w2, 1))
+    new = x.double() + norm(pair, w3, 1)
+    assert close(xd, new, 2.0 ** -19) and close(h[:T], norm(new, w4, 1), unit + 2.0 ** -18)
+    xd = x.clone()
+    _lib.seq_call("umb_hc_seam", xd, h, y, None, None, 0.5, None, w1, 1.0, T, W, 1, eps, code)
+    new = x.double() + 0.5 * y.double()
+    assert close(xd, new) and close(h[:T], norm(new, 1.0 + w1.double(), 1), unit + 2.0 ** -18)
+    _lib.seq_call("umb_hc_embed", xd, h, table, ids, 1.5, None, w1, 1.0, T, W, 11, 1, eps, code)
+    assert close(xd, rows) and close(h[:T], norm(rows, 1.0 + w1.double(), 1), unit)

@@ -51,3 +51,35 @@ template <auto Kernel> static inline int ensure_dynamic_lds(size_t bytes) {
   }
   return UMB_OK;
 }
+
+// ---- rows walked in quads (seq_norm.hip, seq_hyper.hip): four elements in one load of 16 bytes, or of 8 from 16-bit storage
+template <typename P> __device__ __forceinline__ f32x4 ld4(const typename El<P>::type* p) {
+  if constexpr (sizeof(typename El<P>::type) == 4) return *reinterpret_cast<const f32x4*>(p);
+  else {
+    const u32x2 v = *reinterpret_cast<const u32x2*>(p);
+    return f32x4{lo_f<P>(v[0]), hi_f<P>(v[0]), lo_f<P>(v[1]), hi_f<P>(v[1])};
+  }
+}
+template <typename P> __device__ __forceinline__ void st4(typename El<P>::type* p, f32x4 v) {
+  if constexpr (sizeof(typename El<P>::type) == 4) *reinterpret_cast<f32x4*>(p) = v;
+  else *reinterpret_cast<u32x2*>(p) = u32x2{pack2<P>(v[0], v[1]), pack2<P>(v[2], v[3])};
+}
+__device__ __forceinline__ float sq4(f32x4 v) { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3]; }
+
+// whether a (row, group) can be walked in quads (the rows of every operand 16 bytes apart and aligned; 16-bit ones 8)
+static inline bool quads_ok(int W, int groups, const void* a, const void* b = nullptr, const void* c = nullptr, const void* d = nullptr,
+                            const void* e = nullptr, const void* f = nullptr, const void* g = nullptr) {
+  const int gs = W / groups;
+  return gs % 4 == 0 && gs <= 8192 &&
+         ((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d | (uintptr_t)e | (uintptr_t)f | (uintptr_t)g) % 16 == 0;
+}
+#define BY_QUADS(gs, LAUNCH)              \
+  do {                                    \
+    if ((gs) <= 256) LAUNCH(64, 1);       \
+    else if ((gs) <= 512) LAUNCH(128, 1); \
+    else if ((gs) <= 1024) LAUNCH(256, 1); \
+    else if ((gs) <= 2048) LAUNCH(512, 1); \
+    else if ((gs) <= 4096) LAUNCH(1024, 1); \
+    else LAUNCH(1024, 2);                 \
+  } while (0)
+

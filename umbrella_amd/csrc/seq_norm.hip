@@ -314,12 +314,154 @@ __global__ __launch_bounds__(256) void pair_resid_norm_kernel(float* __restrict_
   }
 }
 
+// ---- rows in quads: a workgroup of NT threads owns one (row, group), thread t the quads t, t + NT, ... (NE of them) in registers; every
+// load of the row and of the weights is 8 or 16 bytes wide and issued before the first use, so a seam is one memory round trip, two sums
+// through LDS and the stores.  A decode step has a handful of rows and is latency alone: NT is the group's quads rounded up (1024 at
+// most), one quad per thread up to 4096 elements.  The kernels below (one 4-byte element per lane and load; a wave per group up to
+// 1024, 256 threads beyond) remain for groups that are no multiple of four, longer than 8192, or unaligned (loads and stores: seq_common.h).
+// us of a decode step's launch, one MI355X, 16-bit weights: seam 1 x 4096 10.5 -> 4.8, 16 x 4 x 1024 9.8 -> 5.2; embedding 1 x 4096
+// 40 -> 3.7; final norm 1 x 4096 11.2 -> 4.7; pair seam 1 x 4096 11.7 -> 5.9; of a 2000-token prompt 12.4 -> 8.2 (4 x 512), 10.7 -> 8.9 (2048).
+template <typename P, int NT, int NE>
+__global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__ x, typename El<P>::type* __restrict__ h,
+                                                             const float* __restrict__ y, const typename El<P>::type* __restrict__ w_post,
+                                                             const typename El<P>::type* __restrict__ w_next, int W, int groups, float eps) {
+  __shared__ float red[NT / 64], red2[NT / 64];
+  const int grp = blockIdx.y, gs = W / groups, nq = gs / 4;
+  const long o = (long)blockIdx.x * W + (long)grp * gs;
+  f32x4 yv[NE], xv[NE], wp[NE], wn[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int i = min((int)threadIdx.x + NT * e, nq - 1) * 4;
+    yv[e] = *reinterpret_cast<const f32x4*>(y + o + i);
+    xv[e] = *reinterpret_cast<const f32x4*>(x + o + i);
+    wp[e] = ld4<P>(w_post + grp * gs + i);
+    wn[e] = w_next ? ld4<P>(w_next + grp * gs + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) ss += (int)threadIdx.x + NT * e < nq ? sq4(yv[e]) : 0.f;
+  const float f = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)gs + eps);
+  float s2 = 0.f;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int q = (int)threadIdx.x + NT * e;
+    xv[e] = xv[e] + yv[e] * f * wp[e];
+    if (q < nq) { *reinterpret_cast<f32x4*>(x + o + 4 * q) = xv[e]; s2 += sq4(xv[e]); }
+  }
+  if (!w_next) return;
+  const float f2 = 1.f / sqrtf(block_sum<NT>(s2, red2) / (float)gs + eps);
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int q = (int)threadIdx.x + NT * e;
+    if (q < nq) st4<P>(h + o + 4 * q, xv[e] * f2 * wn[e]);
+  }
+}
+
+// EMBED: the row is embed[tokens[t]] * scale and becomes the residual row as well; otherwise x[rows ? rows[t] : t]
+template <typename P, int NT, int NE, bool EMBED>
+__global__ __launch_bounds__(NT) void norm_quad_kernel(float* __restrict__ out_f32, typename El<P>::type* __restrict__ out_dt,
+                                                       const float* __restrict__ x, const int* __restrict__ rows,
+                                                       const typename El<P>::type* __restrict__ embed, int V, float scale,
+                                                       const typename El<P>::type* __restrict__ w, int W, int groups, float eps) {
+  __shared__ float red[NT / 64];
+  const int t = blockIdx.x, grp = blockIdx.y, gs = W / groups, nq = gs / 4;
+  const int r = rows ? rows[t] : t;
+  const long o = (long)t * W + (long)grp * gs, src = (long)(EMBED ? min(max(r, 0), V - 1) : r) * W + (long)grp * gs;
+  f32x4 xv[NE], wv[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int i = min((int)threadIdx.x + NT * e, nq - 1) * 4;
+    wv[e] = ld4<P>(w + grp * gs + i);
+    xv[e] = EMBED ? ld4<P>(embed + src + i) * scale : *reinterpret_cast<const f32x4*>(x + src + i);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int q = (int)threadIdx.x + NT * e;
+    if (q < nq) {
+      ss += sq4(xv[e]);
+      if (EMBED) *reinterpret_cast<f32x4*>(out_f32 + o + 4 * q) = xv[e];
+    }
+  }
+  const float f = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)gs + eps);
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int q = (int)threadIdx.x + NT * e;
+    if (q >= nq) continue;
+    const f32x4 v = xv[e] * f * wv[e];
+    if (!EMBED && out_f32) *reinterpret_cast<f32x4*>(out_f32 + o + 4 * q) = v;
+    if (out_dt) st4<P>(out_dt + o + 4 * q, v);
+  }
+}
+
+template <typename P, int NT, int NE>
+__global__ __launch_bounds__(NT) void pair_resid_norm_quad_kernel(float* __restrict__ x, typename El<P>::type* __restrict__ h,
+                                                                  const float* __restrict__ y1, const float* __restrict__ y2,
+                                                                  const typename El<P>::type* __restrict__ w1,
+                                                                  const typename El<P>::type* __restrict__ w2, float coef,
+                                                                  const typename El<P>::type* __restrict__ w_post,
+                                                                  const typename El<P>::type* __restrict__ w_next, int W, float eps) {
+  __shared__ float red[4][NT / 64];
+  const long o = (long)blockIdx.x * W;
+  const int nq = W / 4;
+  f32x4 a[NE], b[NE], xv[NE], wa[NE], wb[NE], wp[NE], wn[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int i = min((int)threadIdx.x + NT * e, nq - 1) * 4;
+    a[e] = *reinterpret_cast<const f32x4*>(y1 + o + i);
+    b[e] = *reinterpret_cast<const f32x4*>(y2 + o + i);
+    xv[e] = *reinterpret_cast<const f32x4*>(x + o + i);
+    wa[e] = ld4<P>(w1 + i);
+    wb[e] = ld4<P>(w2 + i);
+    wp[e] = ld4<P>(w_post + i);
+    wn[e] = w_next ? ld4<P>(w_next + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  float sa = 0.f, sb = 0.f;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const bool in = (int)threadIdx.x + NT * e < nq;
+    sa += in ? sq4(a[e]) : 0.f;
+    sb += in ? sq4(b[e]) : 0.f;
+  }
+  const float fa = coef / sqrtf(block_sum<NT>(sa, red[0]) / (float)W + eps), fb = coef / sqrtf(block_sum<NT>(sb, red[1]) / (float)W + eps);
+  float sm = 0.f;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    a[e] = a[e] * fa * wa[e] + b[e] * fb * wb[e];
+    sm += (int)threadIdx.x + NT * e < nq ? sq4(a[e]) : 0.f;
+  }
+  const float fm = 1.f / sqrtf(block_sum<NT>(sm, red[2]) / (float)W + eps);
+  float sx = 0.f;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int q = (int)threadIdx.x + NT * e;
+    xv[e] = xv[e] + a[e] * fm * wp[e];
+    if (q < nq) { *reinterpret_cast<f32x4*>(x + o + 4 * q) = xv[e]; sx += sq4(xv[e]); }
+  }
+  if (!w_next) return;
+  const float fx = 1.f / sqrtf(block_sum<NT>(sx, red[3]) / (float)W + eps);
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int q = (int)threadIdx.x + NT * e;
+    if (q < nq) st4<P>(h + o + 4 * q, xv[e] * fx * wn[e]);
+  }
+}
+
 static inline bool norm_args_ok(int T, int W, int groups) { return T >= 1 && W >= 1 && groups >= 1 && W % groups == 0; }
 
 extern "C" int umb_seq_group_norm(float* out_f32, void* out_dt, const float* x, const int* rows, const void* w, int T, int W,
                                   int groups, float eps, int dtype, hipStream_t st) {
   if (!norm_args_ok(T, W, groups) || !x || !w || (!out_f32 && !out_dt)) return UMB_EINVAL;
   const int gs = W / groups;
+  if (quads_ok(W, groups, out_f32, out_dt, x, w)) {
+#define NORM_QUADS(NT, NE)                                                                                                               \
+  hipLaunchKernelGGL((norm_quad_kernel<P, NT, NE, false>), dim3(T, groups), dim3(NT), 0, st, out_f32, (E*)out_dt, x, rows, (const E*)nullptr, \
+                     0, 1.f, (const E*)w, W, groups, eps)
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(gs, NORM_QUADS); })
+#undef NORM_QUADS
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
   DISPATCH_SEQ_DTYPE(dtype, {
     typedef typename El<P>::type E;
     if (gs > 1024 && gs <= 2048)
@@ -339,6 +481,15 @@ extern "C" int umb_seq_group_norm(float* out_f32, void* out_dt, const float* x, 
 extern "C" int umb_seq_embed_norm(float* x, void* h, const void* embed, const int* tokens, float scale, const void* w, int T, int W,
                                   int V, int groups, float eps, int dtype, hipStream_t st) {
   if (!norm_args_ok(T, W, groups) || !x || !h || !embed || !tokens || !w || V < 1) return UMB_EINVAL;
+  if (quads_ok(W, groups, x, h, embed, w)) {
+#define EMBED_QUADS(NT, NE)                                                                                                            \
+  hipLaunchKernelGGL((norm_quad_kernel<P, NT, NE, true>), dim3(T, groups), dim3(NT), 0, st, x, (E*)h, (const float*)nullptr, tokens, (const E*)embed, \
+                     V, scale, (const E*)w, W, groups, eps)
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W / groups, EMBED_QUADS); })
+#undef EMBED_QUADS
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
   DISPATCH_SEQ_DTYPE(dtype, {
     typedef typename El<P>::type E;
     hipLaunchKernelGGL(embed_norm_kernel<P>, dim3(T, (groups + 3) / 4), dim3(256), 0, st, x, (E*)h, (const E*)embed, tokens,
@@ -351,6 +502,15 @@ extern "C" int umb_seq_embed_norm(float* x, void* h, const void* embed, const in
 extern "C" int umb_seq_resid_norm(float* x, void* h, const float* y, const void* w_post, const void* w_next, int T, int W,
                                   int groups, float eps, int dtype, hipStream_t st) {
   if (!norm_args_ok(T, W, groups) || !x || !y || !w_post || (w_next && !h)) return UMB_EINVAL;
+  if (quads_ok(W, groups, x, h, y, w_post, w_next)) {
+#define SEAM_QUADS(NT, NE)                                                                                                      \
+  hipLaunchKernelGGL((resid_norm_quad_kernel<P, NT, NE>), dim3(T, groups), dim3(NT), 0, st, x, (E*)h, y, (const E*)w_post, (const E*)w_next, \
+                     W, groups, eps)
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W / groups, SEAM_QUADS); })
+#undef SEAM_QUADS
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
   DISPATCH_SEQ_DTYPE(dtype, {
     typedef typename El<P>::type E;
     const int per_lane = (W / groups + 63) / 64;
@@ -408,6 +568,15 @@ extern "C" int umb_seq_resid_canon_step(float* x, void* h, const float* y, const
 extern "C" int umb_seq_pair_resid_norm(float* x, void* h, const float* y1, const float* y2, const void* w1, const void* w2, float coef,
                                        const void* w_post, const void* w_next, int T, int W, float eps, int dtype, hipStream_t st) {
   if (!norm_args_ok(T, W, 1) || !x || !y1 || !y2 || !w1 || !w2 || !w_post || (w_next && !h)) return UMB_EINVAL;
+  if (quads_ok(W, 1, x, h, y1, y2, w1, w2, w_post) && (uintptr_t)w_next % 16 == 0) {
+#define PAIR_QUADS(NT, NE)                                                                                                          \
+  hipLaunchKernelGGL((pair_resid_norm_quad_kernel<P, NT, NE>), dim3(T), dim3(NT), 0, st, x, (E*)h, y1, y2, (const E*)w1, (const E*)w2, coef, \
+                     (const E*)w_post, (const E*)w_next, W, eps)
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, PAIR_QUADS); })
+#undef PAIR_QUADS
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
 #define PAIR_SEAM(EPT)                                                                                                          \
   hipLaunchKernelGGL((pair_resid_norm_kernel<P, EPT>), dim3(T), dim3(256), 0, st, x, (E*)h, y1, y2, (const E*)w1, (const E*)w2, \
                      coef, (const E*)w_post, (const E*)w_next, W, eps)

@@ -141,10 +141,19 @@ int umb_moe_combine(float* y, const float* ye, const int* pos_of, int T, int W, 
  * decay: alpha[t][H D] = sigmoid(W_a2 a + b)^(1/tau), fp32 */
 int umb_gla_decay(float* alpha, const float* proj, int ld, int a_col, const void* w_a2, const void* b_a2, int T, int HD, int rank,
                   float tau, int dtype, umb_stream_t stream);
+/* the logarithm of that decay */
+int umb_gla_decay_log(float* log_alpha, const float* proj, int ld, int a_col, const void* w_a2, const void* b_a2, int T, int HD, int rank,
+                      float tau, int dtype, umb_stream_t stream);
 /* per sequence and head: S <- diag(alpha_t) S + k_t v_t^T ; o_t = S^T (q_t * qscale).  state fp32 [slots][H][D][Dv]; a
  * sequence whose first position is 0 starts from S = 0 whatever its slot holds.  o fp32 [T][H Dv]. */
 int umb_gla_scan(float* o, float* state, const float* proj, int ld, const float* alpha, const int* seq_slot, const int* seq_row0,
                  const int* seq_pos0, const int* seq_len, int B, int H, int D, int Dv, float qscale, umb_stream_t stream);
+/* the same recurrence in chunks of 64 tokens, from the decays' logarithms [T][H D].  _floats: scratch floats of a step of T rows in B
+ * stretches (0: shape not covered); proj and scratch 16-byte aligned, ld % 4 == 0, max_len the longest stretch */
+long umb_gla_scan_chunked_floats(int T, int B, int H, int D, int Dv);
+int umb_gla_scan_chunked(float* o, float* state, const float* proj, int ld, const float* log_alpha, const int* seq_slot,
+                         const int* seq_row0, const int* seq_pos0, const int* seq_len, int T, int B, int max_len, int H, int D, int Dv,
+                         float qscale, float* scratch, long scratch_floats, umb_stream_t stream);
 /* out[t][h] = rms_norm(o[t][h]) * w (w [Dv], shared by heads) * silu(g[t][h]) in `dtype` */
 int umb_gla_gate(void* out, const float* o, const float* proj, int ld, int g_col, const void* w, int T, int H, int Dv, float eps,
                  int dtype, umb_stream_t stream);
@@ -243,6 +252,11 @@ int umb_mingru_scan(void* out, float* state, const float* proj, int ld, int z_co
 int umb_lin_scan(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
                  const float* alpha, int alpha_per_head, int qk_heads, const int* seq_slot, const int* seq_row0,
                  const int* seq_pos0, const int* seq_len, int B, int H, int D, int Dv, float qscale, umb_stream_t stream);
+/* a step of ONE token per sequence (row t at position pos[t] of slot[t]; position 0 starts from S = 0), sums in the order of umb_lin_scan; v and
+ * state 16-byte aligned, Dv and ldv multiples of four */
+int umb_lin_step(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* alpha,
+                 int alpha_per_head, int qk_heads, const int* pos, const int* slot, int T, int H, int D, int Dv, float qscale,
+                 umb_stream_t stream);
 
 /* ---- selective state space with a scalar decay per head (state-space duality).  proj fp32 [T][ld]; from column col0:
  * [z (H Dv) | x (H Dv) | B (G N) | C (G N) | dt (H)].  prep: x, B, C through a causal convolution per channel (w [C][taps],

@@ -135,3 +135,66 @@ def test_norms_in_quads(dtype, W, groups):
     assert close(xd, new) and close(h[:T], norm(new, 1.0 + w1.double(), 1), unit + 2.0 ** -18)
     _lib.seq_call("umb_hc_embed", xd, h, table, ids, 1.5, None, w1, 1.0, T, W, 11, 1, eps, code)
     assert close(xd, rows) and close(h[:T], norm(rows, 1.0 + w1.double(), 1), unit)
+
+
+# the chunked recurrence with a decay per channel: one chunk and a token, ragged stretches (one shorter than a block), a carried state, weak and
+# strong decays (a channel forgets within a token), sizes up to the LDS limit
+@pytest.mark.parametrize("H,D,Dv,lens,strong", [(2, 16, 16, [65], False), (3, 48, 80, [64, 5, 130], False), (2, 128, 256, [200, 1], False),
+                                                (2, 128, 64, [70, 129], True), (1, 112, 32, [333], True)])
+def test_gla_chunks(H, D, Dv, lens, strong):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(D + Dv)
+    T, B, HD = sum(lens), len(lens), H * D
+    ld = 2 * HD + H * Dv + 8
+    proj = torch.randn(T, ld, generator=g, device="cuda")
+    la = -torch.rand(T, HD, generator=g, device="cuda") * (0.2 if not strong else 1.0) * torch.where(
+        torch.rand(HD, generator=g, device="cuda") < (0.5 if strong else 0.0), 60.0, 1.0)
+    state = torch.randn(B + 1, H, D, Dv, generator=g, device="cuda")
+    pos0 = [0 if b % 2 else 7 for b in range(B)]
+    row0 = [sum(lens[:b]) for b in range(B)]
+    slots = [B - b for b in range(B)]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                            # noqa: E731
+    want_o, want_s, size = torch.zeros(T, H, Dv, dtype=torch.float64, device="cuda"), state.double(), torch.zeros(T, H, Dv, dtype=torch.float64, device="cuda")
+    q, k, v = (proj[:, c:c + n].double() for c, n in ((0, HD), (HD, HD), (2 * HD, H * Dv)))
+    for b in range(B):
+        S = want_s[slots[b]] * (0.0 if pos0[b] == 0 else 1.0)
+        A = S.abs()
+        for t in range(row0[b], row0[b] + lens[b]):
+            a = la[t].double().exp().view(H, D, 1)
+            add = k[t].view(H, D, 1) * v[t].view(H, 1, Dv)
+            S, A = a * S + add, a * A + add.abs()
+            want_o[t], size[t] = (S * q[t].view(H, D, 1)).sum(1), (A * q[t].abs().view(H, D, 1)).sum(1)
+        want_s[slots[b]] = S
+    need = _lib.load_seq().umb_gla_scan_chunked_floats(T, B, H, D, Dv)
+    scratch = torch.full((need + 64,), float("nan"), device="cuda")
+    o, st = torch.full((T + 1, H * Dv), 7.0, device="cuda"), state.clone()
+    _lib.seq_call("umb_gla_scan_chunked", o, st, proj, ld, la, i32(slots), i32(row0), i32(pos0), i32(lens), T, B, max(lens), H, D, Dv, 0.5,
+                  scratch, need)
+    # fp32 sums of at most D + 64 products in two stages, every weight an exponential good to 2^-21: far inside 2^-17 of the sum of sizes
+    assert ((o[:T].view(T, H, Dv).double() - 0.5 * want_o).abs() <= 2.0 ** -17 * 0.5 * size + 1e-30).all() and bool((o[T] == 7.0).all())
+    assert ((st[slots].double() - want_s[slots]).abs() <= 2.0 ** -17 * (want_s[slots].abs().amax() + 1)).all()
+    assert torch.equal(st[0], state[0]) and bool(torch.isnan(scratch[need:]).all())
+
+
+@pytest.mark.parametrize("H,D,Dv,per_head,groups", [(2, 16, 8, 0, 2), (4, 40, 60, 1, 2), (1, 128, 256, 0, 1), (2, 130, 64, 0, 2), (2, 256, 4, 1, 1)])
+def test_single_token_recurrence_follows_the_scan(H, D, Dv, per_head, groups):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(D + Dv)
+    T = 3
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")                                     # noqa: E731
+    q, k, v = r(T, groups * D), r(T, groups * D + 4), r(T, H * Dv + 4)
+    alpha = torch.rand(T, H if per_head else H * D, generator=g, device="cuda")
+    state, out = r(T + 2, H, D, Dv), []
+    pos, slot, row, one = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([5, 0, 9], [3, 0, 1], [0, 1, 2], [1, 1, 1]))
+    for step in (True, False):
+        st, o = state.clone(), torch.full((T + 1, H * Dv), 7.0, device="cuda")
+        args = (o, st, q, groups * D, k, groups * D + 4, v, H * Dv + 4, alpha, per_head, groups)
+        if step:
+            _lib.seq_call("umb_lin_step", *args, pos, slot, T, H, D, Dv, 0.25)
+        else:
+            _lib.seq_call("umb_lin_scan", *args, slot, row, pos, one, T, H, D, Dv, 0.25)
+        out.append((o, st))
+    # the sums run in one order; which product of a * S + k * v joins the other unrounded is the compiler's choice
+    bound = 2.0 ** -23 * (state[slot.long()].abs() + k.abs().amax() * v.abs().amax())
+    assert ((out[0][1] - out[1][1])[slot.long()].abs() <= bound).all() and torch.equal(out[0][1][[2, 4]], state[[2, 4]])
+    assert ((out[0][0] - out[1][0]).abs() <= D * q.abs().amax() * bound.amax()).all() and bool((out[0][0][T] == 7.0).all())

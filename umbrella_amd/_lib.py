@@ -309,6 +309,9 @@ SEQ_SIGNATURES = {
     "umb_seq_embed_norm": [_P, _P, _P, _P, _F, _P, _I, _I, _I, _I, _F, _I],
     "umb_seq_resid_norm": [_P, _P, _P, _P, _P, _I, _I, _I, _F, _I],
     "umb_gla_decay": [_P, _P, _I, _I, _P, _P, _I, _I, _I, _F, _I],
+    "umb_gla_decay_log": [_P, _P, _I, _I, _P, _P, _I, _I, _I, _F, _I],
+    "umb_gla_scan_chunked_floats": [_I, _I, _I, _I, _I],
+    "umb_gla_scan_chunked": [_P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _L],
     "umb_gla_scan": [_P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F],
     "umb_gla_gate": [_P, _P, _P, _I, _I, _P, _I, _I, _I, _F, _I],
     "umb_pwa_prep": [_P, _PKV, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I],
@@ -320,6 +323,7 @@ SEQ_SIGNATURES = {
     "umb_hc_read": [_P, _P, _P, _P, _P, _P, _F, _I, _I, _I, _F, _I],
     "umb_mingru_scratch_floats": [_I, _I, _I],
     "umb_mingru_scan": [_P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _P, _L, _I],
+    "umb_lin_step": [_P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _I, _I, _I, _I, _F],
     "umb_lin_scan": [_P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _F],
     "umb_ssd_prep": [_P, _I, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I],
     "umb_ssd_scan_chunked_floats": [_I, _I, _I, _I, _I],
@@ -361,7 +365,7 @@ SEQ_SIGNATURES = {
     "umb_seq_version": [],
 }
 _SEQ_NO_STREAM = {"umb_lat_attend_tiled_ok", "umb_seq_resid_canon_step_ok", "umb_bsa_attend_tiled_ok", "umb_mingru_scratch_floats",
-                  "umb_ssd_scan_chunked_floats", "umb_delta_scan_floats"}          # predicates: no stream argument, the value is the answer
+                  "umb_ssd_scan_chunked_floats", "umb_delta_scan_floats", "umb_gla_scan_chunked_floats"}          # predicates: no stream argument, the value is the answer
 _seq_lib = None
 
 

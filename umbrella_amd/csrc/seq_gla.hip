@@ -13,7 +13,8 @@
 #include "seq_common.h"
 #include <type_traits>
 
-template <typename P>
+// LOG: the decay's logarithm itself, as the chunked form reads it
+template <typename P, bool LOG>
 __global__ __launch_bounds__(256) void gla_decay_kernel(float* __restrict__ alpha, const float* __restrict__ proj, int ld,
                                                         int a_col, const typename El<P>::type* __restrict__ w_a2,
                                                         const typename El<P>::type* __restrict__ b_a2, int HD, int rank,
@@ -27,7 +28,8 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(float* __restrict__ alph
     float z = 0.f;
     for (int i = 0; i < rank; ++i) z += ldf<P>(wr + i) * a_s[i];
     if (b_a2) z += ldf<P>(b_a2 + n);
-    alpha[(long)t * HD + n] = expf(log_sigmoidf_(z) * inv_tau);
+    const float la = log_sigmoidf_(z) * inv_tau;
+    alpha[(long)t * HD + n] = LOG ? la : expf(la);
   }
 }
 
@@ -212,17 +214,28 @@ __global__ __launch_bounds__(256) void gla_gate_kernel(typename El<P>::type* __r
     stf<P>(out + (long)t * H * Dv + (long)h * Dv + i, orow[i] * f * ldf<P>(w + i) * siluf_(gr[i]));
 }
 
-extern "C" int umb_gla_decay(float* alpha, const float* proj, int ld, int a_col, const void* w_a2, const void* b_a2, int T, int HD,
-                             int rank, float tau, int dtype, hipStream_t st) {
+template <bool LOG>
+static int gla_decay_launch(float* alpha, const float* proj, int ld, int a_col, const void* w_a2, const void* b_a2, int T, int HD, int rank,
+                            float tau, int dtype, hipStream_t st) {
   if (T < 1 || HD < 1 || rank < 1 || rank > 8192 || !(tau > 0.f) || !alpha || !proj || !w_a2) return UMB_EINVAL;
   const int gy = (HD + 255) / 256 > 64 ? 64 : (HD + 255) / 256;
   DISPATCH_SEQ_DTYPE(dtype, {
     typedef typename El<P>::type E;
-    hipLaunchKernelGGL(gla_decay_kernel<P>, dim3(T, gy), dim3(256), rank * sizeof(float), st, alpha, proj, ld, a_col,
+    hipLaunchKernelGGL((gla_decay_kernel<P, LOG>), dim3(T, gy), dim3(256), rank * sizeof(float), st, alpha, proj, ld, a_col,
                        (const E*)w_a2, (const E*)b_a2, HD, rank, 1.f / tau);
   })
   UMB_LAUNCH_CHECK();
   return UMB_OK;
+}
+
+extern "C" int umb_gla_decay(float* alpha, const float* proj, int ld, int a_col, const void* w_a2, const void* b_a2, int T, int HD,
+                             int rank, float tau, int dtype, hipStream_t st) {
+  return gla_decay_launch<false>(alpha, proj, ld, a_col, w_a2, b_a2, T, HD, rank, tau, dtype, st);
+}
+
+extern "C" int umb_gla_decay_log(float* log_alpha, const float* proj, int ld, int a_col, const void* w_a2, const void* b_a2, int T, int HD,
+                                 int rank, float tau, int dtype, hipStream_t st) {
+  return gla_decay_launch<true>(log_alpha, proj, ld, a_col, w_a2, b_a2, T, HD, rank, tau, dtype, st);
 }
 
 extern "C" int umb_lin_scan(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
@@ -275,6 +288,401 @@ extern "C" int umb_gla_gate(void* out, const float* o, const float* proj, int ld
     hipLaunchKernelGGL(gla_gate_kernel<P>, dim3((unsigned)((th + 3) / 4)), dim3(256), 0, st, (E*)out, o, proj, ld, g_col,
                        (const E*)w, T, H, Dv, eps);
   })
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+
+// ---- one token per sequence: the state is read and written once, nothing else is large (16 requests x 16 heads x 128 x 256: 67 MB).
+// Workgroup = (64 value columns, head, token): thread (column quad tid % 16, row group r = tid / 16) keeps rows r nr .. of its four
+// columns, all loads in flight at once; the read-out sums rows as the scan does (nr in order, then groups by 8, 4, 2, 1).
+// The scan kernel stages sixteen tokens' operands for the one: 46 us for those 67 MB, 13.6 here (4.9 TB/s); 8 heads x 128 x 256, one request
+// 10.6 -> 5.4.
+template <int RMAX>
+__global__ __launch_bounds__(256) void lin_step_kernel(float* __restrict__ o, float* __restrict__ state, const float* __restrict__ qp, int ldq,
+                                                       const float* __restrict__ kp, int ldk, const float* __restrict__ vp, int ldv,
+                                                       const float* __restrict__ alpha, int aph, int hpg, const int* __restrict__ pos,
+                                                       const int* __restrict__ slot, int H, int D, int Dv, float qscale) {
+  __shared__ __attribute__((aligned(16))) float rowv[3][16 * GLA_MAXR];          // alpha, k, q of the head
+  __shared__ __attribute__((aligned(16))) float red[16][64];
+  const int t = blockIdx.z, h = blockIdx.y, hq = h / hpg, nr = (D + 15) / 16;
+  const int cq = threadIdx.x & 15, r = threadIdx.x >> 4, c = blockIdx.x * 64 + 4 * cq;
+  const bool c_ok = c < Dv;
+  float* sp = state + (((long)slot[t] * H + h) * D) * Dv + (c_ok ? c : 0);
+  f32x4 S[RMAX];
+#pragma unroll
+  for (int i = 0; i < RMAX; ++i) {
+    const int d = r * nr + (i < nr ? i : nr - 1);
+    S[i] = *reinterpret_cast<const f32x4*>(sp + (long)(d < D ? d : D - 1) * Dv);
+  }
+  const f32x4 v = *reinterpret_cast<const f32x4*>(vp + (long)t * ldv + (long)h * Dv + (c_ok ? c : 0));
+  const int d0 = threadIdx.x;
+  if (d0 < D) {
+    rowv[0][d0] = aph ? alpha[(long)t * H + h] : alpha[(long)t * H * D + (long)h * D + d0];
+    rowv[1][d0] = kp[(long)t * ldk + (long)hq * D + d0];
+    rowv[2][d0] = qp[(long)t * ldq + (long)hq * D + d0];
+  }
+  const bool fresh = pos[t] == 0;
+  __syncthreads();
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < RMAX; ++i) {
+    const int d = r * nr + i;
+    if (i < nr && d < D) {
+      const float al = rowv[0][d], kk = rowv[1][d], qq = rowv[2][d];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        S[i][e] = al * (fresh ? 0.f : S[i][e]) + kk * v[e];
+        acc[e] += S[i][e] * qq;
+      }
+      if (c_ok) *reinterpret_cast<f32x4*>(sp + (long)d * Dv) = S[i];
+    }
+  }
+  *reinterpret_cast<f32x4*>(&red[r][4 * cq]) = acc;
+  __syncthreads();
+  const int cc = threadIdx.x;
+  if (cc < 64 && blockIdx.x * 64 + cc < Dv) {
+    float p[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) p[i] = red[i][cc];
+#pragma unroll
+    for (int m = 8; m >= 1; m >>= 1)
+#pragma unroll
+      for (int i = 0; i < m; ++i) p[i] += p[i + m];
+    o[(long)t * (H * Dv) + (long)h * Dv + blockIdx.x * 64 + cc] = p[0] * qscale;
+  }
+}
+
+extern "C" int umb_lin_step(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
+                            const float* alpha, int alpha_per_head, int qk_heads, const int* pos, const int* slot, int T, int H, int D, int Dv,
+                            float qscale, hipStream_t st) {
+  if (T < 1 || T > 65535 || H < 1 || H > 65535 || D < 1 || D > 16 * GLA_MAXR || Dv < 1 || Dv % 4 || qk_heads < 1 || H % qk_heads || !o || !state ||
+      !q || !k || !v || !alpha || !pos || !slot || ldq < qk_heads * D || ldk < qk_heads * D || ldv < H * Dv || ldv % 4 ||
+      ((uintptr_t)v | (uintptr_t)state) % 16)
+    return UMB_EINVAL;
+  const dim3 grid((Dv + 63) / 64, H, T);
+  const int nr = (D + 15) / 16, aph = alpha_per_head ? 1 : 0, hpg = H / qk_heads;
+#define LIN_STEP(R) \
+  hipLaunchKernelGGL(lin_step_kernel<R>, grid, dim3(256), 0, st, o, state, q, ldq, k, ldk, v, ldv, alpha, aph, hpg, pos, slot, H, D, Dv, qscale)
+  if (nr <= 2) LIN_STEP(2);
+  else if (nr <= 4) LIN_STEP(4);
+  else if (nr <= 8) LIN_STEP(8);
+  else LIN_STEP(16);
+#undef LIN_STEP
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+
+// ---- the recurrence in chunks of 64 tokens, for stretches of many.  With one decay per key CHANNEL, c_t = sum of the channel's
+// log decays over the chunk up to and including token t:
+//     S_end = e^(c_64) S_start + sum_s (e^(c_64 - c_s) k_s) v_s^T        o_t = (e^(c_t) q_t)^T S_start + sum_{s <= t} A_ts v_s
+//     A_ts  = sum_d q_td k_sd e^(c_td - c_sd)
+// All exponents are of non-positive numbers.  A's 16 x 16 blocks below the diagonal split the exponent at the start r of the row
+// block, (e^(c_t - r) q_t) . (e^(r - c_s) k_s), a matrix product; in the diagonal blocks the split would need e^(+): there every
+// pair of tokens and channel takes its own exponential.  Four launches, all but the second over (column slice, chunk, head, sequence):
+//   prep   c (prefix sums in double, kept as blocks' starts and offsets inside a block in two 32-bit parts), A, e^(c_t) q_t, e^(c_64 - c_s) k_s
+//   state  every chunk's sum from a zero state        pass   chunks in order: sums become start states, the slot the final one
+//   out    A v + (e^c q)^T S_start
+// fp32 throughout, products on the fp32 matrix pipe.  2048 tokens, 8 heads x 128 x 256 on one MI355X: 670 us token by token (a serial
+// loop on 512 waves) -> 100 (25 + 23 + 15 + 38); 192 tokens 66 -> 45.  D and Dv multiples of 16, D <= 128 (the chunk's q, k and offsets fill the LDS).
+constexpr int GC_Q = 64;
+
+struct GlaChunk {
+  const float *q, *k, *v, *la;             // rows of proj at the q, k, v columns; la [T][H D]
+  int ld, H, D, Dv;
+  const int *seq_slot, *seq_row0, *seq_pos0, *seq_len;
+  float *qt, *kh, *m, *sc, *ac;            // [T][H D] twice, [T][H][64], [chunks][H][D][Dv], [chunks][H][D]
+  float qscale;
+  // chunks of the sequences before b
+  __device__ __forceinline__ int first(int b) const {
+    int n = 0;
+    for (int i = 0; i < b; ++i) n += (seq_len[i] + GC_Q - 1) / GC_Q;
+    return n;
+  }
+};
+
+__device__ __forceinline__ f32x4 gla_mma(f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+  return c;
+}
+
+// grid (chunks, heads, sequences).  One workgroup fills a CU's LDS: 1024 threads, 256 for each diagonal block, whose exponentials are most
+// of the work (256 threads: 40 us for one chunk as for 256 of them)
+__global__ __launch_bounds__(1024) void gla_chunk_prep_kernel(GlaChunk a) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int b = blockIdx.z, h = blockIdx.y, t0 = blockIdx.x * GC_Q, len = a.seq_len[b];
+  if (t0 >= len) return;
+  const int cnt = len - t0 < GC_Q ? len - t0 : GC_Q, D = a.D, LD = D + 4, HD = a.H * D;
+  const long row0 = (long)a.seq_row0[b] + t0;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, g = lane >> 4;
+  double* blk = reinterpret_cast<double*>(sm);   // [5][128]: c at the starts of the four blocks, and at the chunk's end
+  float* rs = sm + 2 * 5 * 128;                  // [64][LD]: c_t less the start of t's block, rounded ..
+  float* rl = rs + GC_Q * LD;                    // [64][LD]: .. and what the rounding left (a channel that forgets at once has sums of hundreds)
+  float* qs = rl + GC_Q * LD;                    // [64][LD]
+  float* ks = qs + GC_Q * LD;                    // [64][LD]
+  if (tid < 512 && (tid & 127) < D) {            // (channel, block): the block's running sums
+    const int d = tid & 127, u = tid >> 7;
+    float l[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int t = 16 * u + i;
+      l[i] = a.la[(row0 + (t < cnt ? t : cnt - 1)) * HD + (long)h * D + d];
+    }
+    double run = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int t = 16 * u + i;
+      run += t < cnt ? (double)l[i] : 0.0;
+      const float hi = (float)run;
+      rs[t * LD + d] = hi;
+      rl[t * LD + d] = (float)(run - (double)hi);
+    }
+    blk[(u + 1) * 128 + d] = run;                // the block's own sum for now
+  }
+  const int dq = D >> 2;
+  for (int x = tid; x < GC_Q * dq; x += 1024) {
+    const int t = x / dq, d = (x - t * dq) * 4;
+    f32x4 qv = f32x4{0.f, 0.f, 0.f, 0.f}, kv = qv;
+    if (t < cnt) {
+      qv = *reinterpret_cast<const f32x4*>(a.q + (row0 + t) * a.ld + (long)h * D + d);
+      kv = *reinterpret_cast<const f32x4*>(a.k + (row0 + t) * a.ld + (long)h * D + d);
+    }
+    *reinterpret_cast<f32x4*>(qs + t * LD + d) = qv;
+    *reinterpret_cast<f32x4*>(ks + t * LD + d) = kv;
+  }
+  __syncthreads();
+  const int nc = a.first(b) + blockIdx.x;
+  if (tid < D) {
+    double run = 0.0;
+    blk[tid] = 0.0;
+#pragma unroll
+    for (int i = 1; i <= 4; ++i) {
+      run += blk[i * 128 + tid];
+      blk[i * 128 + tid] = run;
+    }
+    a.ac[((long)nc * a.H + h) * D + tid] = expf((float)run);
+  }
+  __syncthreads();
+  for (int x = tid; x < GC_Q * dq; x += 1024) {   // what the other launches read: decayed from the chunk's start, to its end
+    const int t = x / dq, d = (x - t * dq) * 4;
+    if (t >= cnt) continue;
+    f32x4 qv = *reinterpret_cast<const f32x4*>(qs + t * LD + d), kv = *reinterpret_cast<const f32x4*>(ks + t * LD + d);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const double c = blk[(t >> 4) * 128 + d + e] + ((double)rs[t * LD + d + e] + (double)rl[t * LD + d + e]);
+      qv[e] *= expf((float)c);
+      kv[e] *= expf((float)(blk[4 * 128 + d + e] - c));
+    }
+    *reinterpret_cast<f32x4*>(a.qt + (row0 + t) * HD + (long)h * D + d) = qv;
+    *reinterpret_cast<f32x4*>(a.kh + (row0 + t) * HD + (long)h * D + d) = kv;
+  }
+  // diagonal block tid / 256: thread (row, column)
+  constexpr float L2E = 1.44269504088896341f;
+  const int tr = (tid >> 4) & 15, ts = tid & 15;
+  {
+    const int t = 16 * (tid >> 8) + tr, s = 16 * (tid >> 8) + ts;
+    float acc = 0.f;
+    if (ts <= tr && t < cnt) {
+      for (int d = 0; d < D; d += 4) {
+        const f32x4 q4 = *reinterpret_cast<const f32x4*>(qs + t * LD + d), k4 = *reinterpret_cast<const f32x4*>(ks + s * LD + d);
+        const f32x4 rt = *reinterpret_cast<const f32x4*>(rs + t * LD + d), r4 = *reinterpret_cast<const f32x4*>(rs + s * LD + d);
+        const f32x4 lt = *reinterpret_cast<const f32x4*>(rl + t * LD + d), l4 = *reinterpret_cast<const f32x4*>(rl + s * LD + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc += q4[e] * k4[e] * __builtin_amdgcn_exp2f(((rt[e] - r4[e]) + (lt[e] - l4[e])) * L2E);
+      }
+    }
+    if (t < cnt) a.m[((row0 + t) * a.H + h) * 64 + s] = acc;
+  }
+  // the six blocks below the diagonal: row block rb, column block cb
+  if (wave < 6) {
+    const int id = wave;
+    const int rb = id < 1 ? 1 : (id < 3 ? 2 : 3), cb = id - rb * (rb - 1) / 2;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int t = 16 * rb + j, s = 16 * cb + j;
+    for (int k0 = 4 * g; k0 < D; k0 += 16) {
+      f32x4 x = *reinterpret_cast<const f32x4*>(qs + t * LD + k0), y = *reinterpret_cast<const f32x4*>(ks + s * LD + k0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] *= expf(rs[t * LD + k0 + e]);           // (an error in a sum that large is an error in nothing)
+        y[e] *= expf((float)(blk[rb * 128 + k0 + e] - (blk[cb * 128 + k0 + e] + ((double)rs[s * LD + k0 + e] + (double)rl[s * LD + k0 + e]))));
+      }
+      acc = gla_mma(x, y, acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tt = 16 * rb + 4 * g + r;
+      if (tt < cnt) a.m[((row0 + tt) * a.H + h) * 64 + 16 * cb + j] = acc[r];
+    }
+  }
+}
+
+// grid (64-column slices, chunks, sequences x heads): wave w the row tiles w, w + 4 of the state, four column tiles
+__global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunk a) {
+  const int b = blockIdx.z / a.H, h = blockIdx.z % a.H, t0 = blockIdx.y * GC_Q, len = a.seq_len[b];
+  if (t0 >= len) return;
+  const int cnt = len - t0 < GC_Q ? len - t0 : GC_Q, D = a.D, Dv = a.Dv, HD = a.H * D;
+  const long row0 = (long)a.seq_row0[b] + t0;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4, p0 = blockIdx.x * 64;
+  f32x4 acc[2][4];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k0 = 0; k0 < GC_Q; k0 += 16) {
+    f32x4 fa[2], fb[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int s = k0 + 4 * g + r, sc = s < cnt ? s : cnt - 1;
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int d = 16 * (wave + 4 * x) + j;
+        const float kv = a.kh[(row0 + sc) * HD + (long)h * D + (d < D ? d : D - 1)];
+        fa[x][r] = s < cnt ? kv : 0.f;
+      }
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        const int p = p0 + 16 * y + j;
+        fb[y][r] = a.v[(row0 + sc) * a.ld + (long)h * Dv + (p < Dv ? p : Dv - 1)];
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 4; ++y) acc[x][y] = gla_mma(fa[x], fb[y], acc[x][y]);
+  }
+  float* dst = a.sc + ((long)(a.first(b) + blockIdx.y) * a.H + h) * D * Dv;
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = 16 * (wave + 4 * x) + 4 * g + r, p = p0 + 16 * y + j;
+        if (d < D && p < Dv) dst[(long)d * Dv + p] = acc[x][y][r];
+      }
+}
+
+// thread per state element of a (sequence, head), chunks in order (eight sums in flight); sc[c] becomes the START state of chunk c
+__global__ __launch_bounds__(256) void gla_chunk_pass_kernel(float* __restrict__ state, GlaChunk a) {
+  const int b = blockIdx.z, h = blockIdx.y;
+  const long e = (long)blockIdx.x * 256 + threadIdx.x, NP = (long)a.D * a.Dv;
+  if (e >= NP) return;
+  const int nch = (a.seq_len[b] + GC_Q - 1) / GC_Q, d = (int)(e / a.Dv);
+  if (nch == 0) return;
+  float* sp = state + ((long)a.seq_slot[b] * a.H + h) * NP + e;
+  float S = a.seq_pos0[b] == 0 ? 0.f : *sp;
+  const long base = a.first(b), step = (long)a.H * NP;
+  float* x = a.sc + (base * a.H + h) * NP + e;
+  const float* ac = a.ac + (base * a.H + h) * a.D + d;
+  for (int c0 = 0; c0 < nch; c0 += 8) {
+    float add[8], dec[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int c = c0 + i < nch ? c0 + i : nch - 1;
+      add[i] = x[c * step];
+      dec[i] = ac[(long)c * a.H * a.D];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (c0 + i < nch) {
+        x[(c0 + i) * step] = S;
+        S = dec[i] * S + add[i];
+      }
+    }
+  }
+  *sp = S;
+}
+
+// grid (64-column slices, chunks, sequences x heads): wave w the read-outs of tokens 16 w .., four column tiles
+__global__ __launch_bounds__(256) void gla_chunk_out_kernel(float* __restrict__ o, GlaChunk a) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  constexpr int LP = 68;
+  const int b = blockIdx.z / a.H, h = blockIdx.z % a.H, t0 = blockIdx.y * GC_Q, len = a.seq_len[b];
+  if (t0 >= len) return;
+  const int cnt = len - t0 < GC_Q ? len - t0 : GC_Q, D = a.D, Dv = a.Dv, HD = a.H * D;
+  const long row0 = (long)a.seq_row0[b] + t0;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, g = lane >> 4, p0 = blockIdx.x * 64;
+  float* vs = sm;                          // [64][LP]
+  float* ss = vs + GC_Q * LP;              // [D][LP]: the chunk's start state
+  const float* s0 = a.sc + ((long)(a.first(b) + blockIdx.y) * a.H + h) * D * Dv;
+  for (int x = tid; x < (GC_Q + D) * 16; x += 256) {
+    const int row = x >> 4, p = (x & 15) * 4, pc = p0 + p < Dv ? p0 + p : Dv - 4;
+    const int t = row < GC_Q ? (row < cnt ? row : cnt - 1) : 0;
+    const float* src = row < GC_Q ? a.v + (row0 + t) * a.ld + (long)h * Dv + pc : s0 + (long)(row - GC_Q) * Dv + pc;
+    *reinterpret_cast<f32x4*>(sm + row * LP + p) = *reinterpret_cast<const f32x4*>(src);
+  }
+  const int t = 16 * wave + j, tc = t < cnt ? t : cnt - 1;
+  f32x4 fm[4], fq[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) fm[i] = i <= wave ? *reinterpret_cast<const f32x4*>(a.m + ((row0 + tc) * a.H + h) * 64 + 16 * i + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) fq[i] = 16 * i < D ? *reinterpret_cast<const f32x4*>(a.qt + (row0 + tc) * HD + (long)h * D + 16 * i + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+  f32x4 acc[4];
+#pragma unroll
+  for (int y = 0; y < 4; ++y) acc[y] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto cols = [&](const float* m, int k0, int y) {          // column 16 y + j, rows k0 + 4 g ..
+    f32x4 f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) f[r] = m[(k0 + 4 * g + r) * LP + 16 * y + j];
+    return f;
+  };
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (16 * i < D) {
+#pragma unroll
+      for (int y = 0; y < 4; ++y) acc[y] = gla_mma(fq[i], cols(ss, 16 * i, y), acc[y]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i <= wave) {
+#pragma unroll
+      for (int y = 0; y < 4; ++y) acc[y] = gla_mma(fm[i], cols(vs, 16 * i, y), acc[y]);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int tt = 16 * wave + 4 * g + r;
+    if (tt >= cnt) continue;
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      const int p = p0 + 16 * y + j;
+      if (p < Dv) o[(row0 + tt) * ((long)a.H * Dv) + (long)h * Dv + p] = acc[y][r] * a.qscale;
+    }
+  }
+}
+
+// floats of scratch for a step of T rows in B stretches; 0: the shape is not covered
+extern "C" long umb_gla_scan_chunked_floats(int T, int B, int H, int D, int Dv) {
+  if (T < 1 || B < 1 || H < 1 || D < 16 || D > 128 || D % 16 || Dv < 16 || Dv % 16) return 0;
+  const long chunks = T / GC_Q + B;                          // whole chunks, and at most one started per stretch
+  return (long)T * H * (2L * D + 64) + chunks * H * ((long)D * Dv + D);
+}
+
+extern "C" int umb_gla_scan_chunked(float* o, float* state, const float* proj, int ld, const float* log_alpha, const int* seq_slot,
+                                    const int* seq_row0, const int* seq_pos0, const int* seq_len, int T, int B, int max_len, int H, int D, int Dv,
+                                    float qscale, float* scratch, long scratch_floats, hipStream_t st) {
+  const long need = umb_gla_scan_chunked_floats(T, B, H, D, Dv);
+  if (need == 0 || need > scratch_floats || !o || !state || !proj || !log_alpha || !scratch || !seq_slot || !seq_row0 || !seq_pos0 || !seq_len ||
+      max_len < 1 || max_len > T || (long)B * H > 65535 || ld < 2 * H * D + H * Dv || ld % 4 || ((uintptr_t)proj | (uintptr_t)scratch) % 16)
+    return UMB_EINVAL;
+  const int chunks = (max_len + GC_Q - 1) / GC_Q, HD = H * D;
+  if (chunks > 65535) return UMB_EINVAL;
+  const long nc = T / GC_Q + B;
+  float* qt = scratch;
+  float* kh = qt + (long)T * HD;
+  float* m = kh + (long)T * HD;
+  float* sc = m + (long)T * H * 64;
+  float* ac = sc + nc * H * D * Dv;
+  const GlaChunk a{proj, proj + HD, proj + 2L * HD, log_alpha, ld, H, D, Dv, seq_slot, seq_row0, seq_pos0, seq_len, qt, kh, m, sc, ac, qscale};
+  const size_t lds1 = (2 * 5 * 128 + 4 * (size_t)GC_Q * (D + 4)) * sizeof(float), lds4 = (size_t)(GC_Q + D) * 68 * sizeof(float);
+  if (ensure_dynamic_lds<gla_chunk_prep_kernel>(lds1) != UMB_OK || ensure_dynamic_lds<gla_chunk_out_kernel>(lds4) != UMB_OK) return UMB_EHIP;
+  hipLaunchKernelGGL(gla_chunk_prep_kernel, dim3(chunks, H, B), dim3(1024), lds1, st, a);
+  hipLaunchKernelGGL(gla_chunk_state_kernel, dim3((Dv + 63) / 64, chunks, B * H), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(gla_chunk_pass_kernel, dim3((unsigned)(((long)D * Dv + 255) / 256), H, B), dim3(256), 0, st, state, a);
+  hipLaunchKernelGGL(gla_chunk_out_kernel, dim3((Dv + 63) / 64, chunks, B * H), dim3(256), lds4, st, o, a);
   UMB_LAUNCH_CHECK();
   return UMB_OK;
 }

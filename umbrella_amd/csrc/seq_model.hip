@@ -137,6 +137,11 @@ static int mix_mingru(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqW
                          Wm, s->max_len, ws->aux, umb_mingru_scratch_floats(s->T, s->B, Wm), m->dtype, st);
 }
 
+// single-token steps of the recurrences take the step kernel where its 16-byte accesses can be made
+static inline bool lin_step_ok(const float* v, int ldv, const float* state, int Dv) {
+  return Dv % 4 == 0 && ldv % 4 == 0 && ((uintptr_t)v | (uintptr_t)state) % 16 == 0;
+}
+
 // softmax attention with a distance bias beside a state-space layer; both read the projection of the same input and write
 // their halves of the row that the one output projection reads: [scale_a * attention | scale_b * state space]
 static int mix_attn_ssd(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWork* ws, const UmbSeqStep* s, hipStream_t st) {
@@ -177,6 +182,8 @@ static int mix_attn_ssd(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSe
   if (need > 0 && need <= spare2_floats && (long)s->B * sH <= 65535)
     SEQ_TRY(umb_ssd_scan_chunked(ws->o, ly.state, sx + inner + sG * N, lds, sx + inner, lds, sx, lds, log_alpha, sG, s->seq_slot,
                                  s->seq_row0, s->seq_pos0, s->seq_len, s->B, s->max_len, sH, N, sDv, spare2, spare2_floats, st));
+  else if (single && lin_step_ok(sx, lds, ly.state, sDv))
+    SEQ_TRY(umb_lin_step(ws->o, ly.state, sx + inner + sG * N, lds, sx + inner, lds, sx, lds, alpha, 1, sG, s->pos, s->slot, T, sH, N, sDv, 1.f, st));
   else
     SEQ_TRY(umb_lin_scan(ws->o, ly.state, sx + inner + sG * N, lds, sx + inner, lds, sx, lds, alpha, 1, sG, s->seq_slot, s->seq_row0,
                          s->seq_pos0, s->seq_len, s->B, sH, N, sDv, 1.f, st));
@@ -196,6 +203,8 @@ static int scan_per_head(float* o, float* state, const float* q, int ldq, const 
   if (need > 0 && need <= scratch_floats && (long)s->B * H <= 65535)
     return umb_ssd_scan_chunked(o, state, q, ldq, k, ldk, v, ldv, log_alpha, H, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, s->B,
                                 s->max_len, H, D, P, scratch, scratch_floats, st);
+  if (s->max_len == 1 && lin_step_ok(v, ldv, state, P))
+    return umb_lin_step(o, state, q, ldq, k, ldk, v, ldv, alpha, 1, H, s->pos, s->slot, s->T, H, D, P, 1.f, st);
   return umb_lin_scan(o, state, q, ldq, k, ldk, v, ldv, alpha, 1, H, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, s->B, H, D, P,
                       1.f, st);
 }
@@ -370,9 +379,23 @@ static int run_mixer(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWo
   } else if (ly.kind == UMB_MIX_GLA) {
     const int H = ly.heads, D = ly.dim, Dv = ly.vdim, HD = H * D;
     if (ld != 2 * HD + 2 * H * Dv + ly.rank || !ly.state) return UMB_EINVAL;
-    SEQ_TRY(umb_gla_decay(ws->aux, ws->proj, ld, 2 * HD + 2 * H * Dv, ly.a2.w, ly.a2.bias, T, HD, ly.rank, ly.tau, dt, st));
-    SEQ_TRY(umb_gla_scan(ws->o, ly.state, ws->proj, ld, ws->aux, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, s->B, H, D,
-                         Dv, ly.qscale, st));
+    // aux: decays (their logarithms) [T][HD] | scratch of the chunked form
+    float* spare = ws->aux + al4((long)T * HD);
+    const long spare_floats = ws->aux_floats - (long)(spare - ws->aux), need = umb_gla_scan_chunked_floats(T, s->B, H, D, Dv);
+    // stretches of three chunks and more side by side, where the shape is covered (8 heads x 128 x 256: 128 tokens 44 us, token by token 45;
+    // 192 tokens 45 / 66; sixteen stretches of 96 134 / 127)
+    const bool chunked = s->max_len >= 192 && need > 0 && need <= spare_floats && (long)s->B * H <= 65535 && ld % 4 == 0;
+    SEQ_TRY((chunked ? umb_gla_decay_log : umb_gla_decay)(ws->aux, ws->proj, ld, 2 * HD + 2 * H * Dv, ly.a2.w, ly.a2.bias, T, HD, ly.rank, ly.tau,
+                                                          dt, st));
+    if (chunked)
+      SEQ_TRY(umb_gla_scan_chunked(ws->o, ly.state, ws->proj, ld, ws->aux, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, T, s->B, s->max_len,
+                                   H, D, Dv, ly.qscale, spare, spare_floats, st));
+    else if (s->max_len == 1 && lin_step_ok(ws->proj + 2L * HD, ld, ly.state, Dv))
+      SEQ_TRY(umb_lin_step(ws->o, ly.state, ws->proj, ld, ws->proj + HD, ld, ws->proj + 2L * HD, ld, ws->aux, 0, H, s->pos, s->slot, T, H, D, Dv,
+                           ly.qscale, st));
+    else
+      SEQ_TRY(umb_gla_scan(ws->o, ly.state, ws->proj, ld, ws->aux, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, s->B, H, D,
+                           Dv, ly.qscale, st));
     SEQ_TRY(umb_gla_gate(ws->mix, ws->o, ws->proj, ld, 2 * HD + H * Dv, ly.head_norm, T, H, Dv, eps, dt, st));
   } else if (ly.kind == UMB_MIX_LATENT) {
     // proj = [dq | dkv (latent + rotated key part) | gate]; the query latent goes up to the heads, its unrotated parts are

@@ -409,6 +409,12 @@ class SeqMixLM(LLMBase):
                 rows = 2 * m.s_groups * up(m.s_state) + inner + 2 * m.s_heads + m.s_heads * (up(m.s_state) + up(m.s_vdim) + 66)
                 ask(aux=m.heads * m.dim + max(rows, 16 * m.heads * (m.vdim + 2) // (16 if T > 64 else 1)) + 48 // T + 2, o=inner,
                     mix=m.heads * m.vdim + inner + 64 // T + 1)
+            elif m.kind == "gla":
+                # aux: decays | scratch of the chunked scan (decayed queries and keys, pair weights, a state per head and 64 tokens,
+                # room for the partial chunks of a few dozen sequences)
+                chunk = m.heads * (m.dim * m.vdim + m.dim)
+                ask(aux=m.heads * (3 * m.dim + 64) + (chunk + 63) // 64 + (min(self.batch_size, 32) * chunk + 64) // T + 1,
+                    o=m.heads * m.vdim, mix=m.heads * m.vdim)
             else:
                 ask(aux=m.heads * m.dim, o=m.heads * m.vdim, mix=m.heads * m.vdim)
             if ly.ff_kind == "moe":

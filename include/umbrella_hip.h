@@ -320,6 +320,13 @@ int umb_beam_expand(const int* top_idx, const float* top_val, int w, int B, int 
  * out5 = {kept, bonus token, eos hit, new num_nodes, raw accept length}; path[i] = i-th accepted tree index */
 int umb_accept_scan(const int* sampled, const int* parents, int* tokens_all, int* n_ptr, int T, const int* eos,
                     int n_eos, int* out5, int* path, umb_stream_t stream);
+/* Boolean attention mask [T][C] (bytes, row stride ld; columns are cache slots; umbrella/models/llama.py:117-134) for the tree-attention
+ * kernels.  scan: per 64-column block b out[2 b] = its first column that some row does not attend (C: none), out[2 b + 1] = one past its
+ * last attended column (0: none); out[2 ceil(C / 64)] = max(slots).  pack: bits [T][W] u64, bit i of word w = column prefix + 64 w + i;
+ * idx [3 T + 1] = {ids, positions, slots, prefix} in 32 bits.  *64: the array holds 64-bit integers */
+int umb_mask_scan(int* out, const void* mask, long ld, int T, int C, const void* slots, int slots64, umb_stream_t stream);
+int umb_mask_pack(void* bits, int W, int* idx, const void* mask, long ld, int T, int C, int prefix, const void* ids, int ids64,
+                  const void* pos, int pos64, const void* slots, int slots64, umb_stream_t stream);
 /* KV_Cache.gather_kv_incremental (umbrella/attn/cache.py:41-49) without the tail memset */
 int umb_kv_compact(void* k_cache, void* vt_cache, const int* res, const int* path, int L, int Hkv, int D, int Lmax,
                    int max_path, int dtype, umb_stream_t stream);

@@ -198,3 +198,54 @@ def test_single_token_recurrence_follows_the_scan(H, D, Dv, per_head, groups):
     bound = 2.0 ** -23 * (state[slot.long()].abs() + k.abs().amax() * v.abs().amax())
     assert ((out[0][1] - out[1][1])[slot.long()].abs() <= bound).all() and torch.equal(out[0][1][[2, 4]], state[[2, 4]])
     assert ((out[0][0] - out[1][0]).abs() <= D * q.abs().amax() * bound.amax()).all() and bool((out[0][0][T] == 7.0).all())
+
+
+@pytest.mark.parametrize("T,C,prefix,end,wide", [(1, 1, 1, 1, True), (1, 65, 65, 65, False), (13, 77, 64, 77, True), (31, 200, 0, 131, True), (40, 640, 600, 640, False),
+                                                 (257, 957, 700, 957, True), (5, 64, 63, 64, True)])
+def test_boolean_mask_scan_and_bits(T, C, prefix, end, wide):
+    from umbrella_amd import _lib
+    from umbrella_amd.models.llama import pack_mask_bits
+    g = torch.Generator().manual_seed(T + C)
+    mask = torch.zeros(T, C + 3, dtype=torch.bool)
+    mask[:, :prefix] = True
+    mask[:, prefix:end] = torch.rand(T, end - prefix, generator=g) < 0.4
+    if end > prefix:
+        mask[0, prefix], mask[T - 1, end - 1] = False, True
+        if T == 1 and end - prefix == 1:
+            mask[0, prefix] = True
+    m = mask.cuda()[:, :C]                                                   # rows further apart than their columns
+    kind = torch.int64 if wide else torch.int32
+    ids, pos, slots = (torch.randint(0, 5000, (T,), generator=g).to(kind).cuda() for _ in range(3))
+    nb = (C + 63) // 64
+    out = torch.full((2 * nb + 2,), -7, dtype=torch.int32, device="cuda")
+    _lib.call("umb_mask_scan", out, m, m.stride(0), T, C, slots, int(wide))
+    got = out.tolist()
+    cols = mask[:, :C].all(0)
+    first = int((~cols).nonzero()[0]) if not bool(cols.all()) else C
+    assert min(got[0:2 * nb:2]) == first and got[2 * nb] == int(slots.max()) and got[2 * nb + 1] == -7
+    assert max(got[1:2 * nb:2]) == int(mask[:, :C].any(0).nonzero()[-1]) + 1
+    pre = max(min(first, C - 1), 0)
+    W = (C - pre + 63) // 64
+    bits, idx = torch.empty(T + 1, W, dtype=torch.int64, device="cuda").fill_(-7), torch.empty(3 * T + 2, dtype=torch.int32, device="cuda").fill_(-7)
+    _lib.call("umb_mask_pack", bits, W, idx, m, m.stride(0), T, C, pre, ids, int(wide), pos, int(wide), slots, int(wide))
+    assert torch.equal(bits[:T].cpu(), pack_mask_bits(mask[:, pre:C])) and bool((bits[T] == -7).all())
+    assert torch.equal(idx[:3 * T], torch.cat([ids, pos, slots]).int()) and idx[3 * T:].tolist() == [pre, -7]
+
+
+def test_a_row_that_attends_everything_attends_nothing_else():
+    """a mask of ones has no column left for bit rows: the row must not see the slot behind its own, whatever that holds"""
+    from umbrella_amd.models.config import LlamaCfg
+    from umbrella_amd.models.llama import Llama
+    from umbrella_amd.models.synthetic import synth_state_small
+    cfg = LlamaCfg(vocab_size=128, hidden_size=256, intermediate_size=256, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2,
+                   head_dim=64, eos_token_id=[], name="tiny")
+    m = Llama("tiny", max_length=128, device="cuda:0", dtype=torch.float16, state_dict=synth_state_small(cfg, 1), config=cfg)
+    m.alloc()
+    ids = torch.arange(20, 29)[None]
+    see = torch.tril(torch.ones(9, 9, dtype=torch.bool))
+    m.inference(ids[:, :8], torch.arange(8)[None], see[:8, :8], torch.arange(8))
+    m.kv_cache.set_rows([9], torch.full((2, 2, 1, 64), 30.0, device="cuda"), torch.full((2, 2, 1, 64), 50.0, device="cuda"))
+    one = m.inference(ids[:, 8:], torch.tensor([[8]]), see[8:], torch.tensor([8]))
+    m.clear()
+    both = m.inference(ids, torch.arange(9)[None], see, torch.arange(9))
+    assert (one[0, 0] - both[0, 8]).abs().max() < 2e-2 * both.abs().max()

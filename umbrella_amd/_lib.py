@@ -176,6 +176,8 @@ SIGNATURES = {
     "umb_sample_rows_uniform": [_P, _P, _I, _I, _P, _P, _F, _F, _I, _F, _P, _I, _I, _I, _P, _P, _P],
     "umb_beam_expand": [_P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P],
     "umb_accept_scan": [_P, _P, _P, _P, _I, _P, _I, _P, _P, _P],
+    "umb_mask_scan": [_P, _P, _L, _I, _I, _P, _I, _P],
+    "umb_mask_pack": [_P, _I, _P, _P, _L, _I, _I, _I, _P, _I, _P, _I, _P, _I, _P],
     "umb_kv_compact": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "umb_set_int": [_P, _I, _P],
     "umb_mask_eos": [_P, _P, _I, _P],

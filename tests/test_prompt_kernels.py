@@ -249,3 +249,131 @@ def test_a_row_that_attends_everything_attends_nothing_else():
     m.clear()
     both = m.inference(ids, torch.arange(9)[None], see, torch.arange(9))
     assert (one[0, 0] - both[0, 8]).abs().max() < 2e-2 * both.abs().max()
+
+
+def _decode_store(lens, G, DK, E, pool, dtype, page, seed):
+    from umbrella_amd.attn.cache import PagedSeqCache
+    c = PagedSeqCache([(G, DK, pool, E)], [], sum(lens), len(lens), "cuda", dtype, page=page)
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    for z in ("k", "v", "kp", "vp"):
+        if c.kv[0][z] is not None:
+            c.kv[0][z].copy_(torch.randn(c.kv[0][z].shape, generator=g, device="cuda"))
+    entries = []
+    for b, n in enumerate(lens):
+        c.open(b)
+        c.extend(b, n, entries)
+    c.write_pages(entries)
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device="cuda")
+    return c, pos, torch.tensor([c.slot(b) for b in range(len(lens))], dtype=torch.int32, device="cuda"), g
+
+
+SHORT, LONG = [1, 15, 16, 17, 40, 65, 256, 257], [1024, 1025, 2049, 3]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,E,maps,lens,window,chunk,keep,extra", [
+    (8, 2, 64, 64, 1, SHORT, 2 ** 30, 0, 0, False), (4, 2, 128, 128, 1, LONG, 2 ** 30, 0, 0, True), (8, 2, 96, 128, 2, SHORT, 100, 0, 0, True),
+    (4, 1, 128, 256, 2, LONG, 2 ** 30, 0, 0, False), (3, 1, 160, 64, 1, SHORT + LONG, 30, 0, 5, True), (6, 3, 32, 256, 1, SHORT, 300, 50, 7, True),
+    (4, 1, 64, 64, 1, [20 + 3 * i for i in range(70)], 64, 0, 3, True), (32, 8, 64, 128, 1, [33] * 140, 512, 0, 0, False)])
+def test_single_token_attention(dtype, H, G, D, E, maps, lens, window, chunk, keep, extra):
+    from umbrella_amd import _lib
+    code = _lib.seq_dtype_code(dtype)
+    c, pos, slot, g = _decode_store(lens, G, maps * D, E, 0, dtype, 16, H + D + E)
+    T, nd = len(lens), 40
+    q = torch.randn(T, H, maps, D, generator=g, device="cuda")
+    gate = torch.randn(T, H * E, generator=g, device="cuda") if extra else None
+    sink = torch.randn(H, generator=g, device="cuda") if extra else None
+    bias = torch.randn(H, nd, generator=g, device="cuda") if extra else None
+    if extra:
+        bias[0, nd - 1] = float("-inf")                   # whole rounds of one head see nothing
+    cap, lam, eps, scale = (6.0 if extra else 0.0), 0.3, 1e-3, D ** -0.5
+    form = _lib.UmbAttnForm(maps, chunk, sink.data_ptr() if extra else None, lam, eps, keep, int(extra))
+    for split in (False, True):
+        out = torch.full((T, H * E + 8), 3.0, dtype=dtype, device="cuda")
+        scratch = torch.empty(T * H * maps * 16 * (E + 2), device="cuda") if split else None
+        _lib.seq_call("umb_attn_attend", out, H * E + 8, q, c.struct(0), gate, H * E if extra else 0, 0 if extra else -1, bias, nd if extra else 0, pos,
+                      slot, T, H, G, D, E, window, scale, 1.25, cap, form, scratch, scratch.numel() if split else 0, code)
+        assert bool((out[:, H * E:] == 3.0).all())
+        for t, n in enumerate(lens):
+            i = n - 1
+            j = torch.arange(n)
+            see = i - j < window
+            if chunk:
+                see &= j // chunk == i // chunk
+            j = j[see | (j < keep)]
+            k, v = (z.double() for z in c.token_rows(0, t, j))                       # [m, G, maps D], [m, G, E]
+            k = k.view(len(j), G, maps, D).repeat_interleave(H // G, 1)
+            s = (q[t].double()[None] * k).sum(-1) * scale                            # [m, H, maps]
+            if cap:
+                s = cap * torch.tanh(s / cap)
+            if extra:
+                s = s + bias.double()[:, torch.clamp(i - j, max=nd - 1).cuda()].T[..., None]
+                p = torch.softmax(torch.cat([s, sink.double()[None, :, None].expand(1, H, maps)]), 0)[:-1]
+            else:
+                p = torch.softmax(s, 0)
+            o = (p[..., None] * v.repeat_interleave(H // G, 1)[:, :, None]).sum(0)   # [H, maps, E]
+            if maps == 2:
+                o = o[:, 0] - lam * o[:, 1]
+                o = o / torch.sqrt(o.pow(2).mean(-1, keepdim=True) + eps)
+            else:
+                o = o[:, 0]
+            o = (1.25 * o).reshape(-1)
+            if extra:
+                o = o * torch.sigmoid(gate[t].double())
+            got = out[t, :H * E].double()
+            # storage rounding of the result; scores of up to 7 in fp32 over at most 2049 keys, then a quotient: 1e-4 of the largest output
+            tol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * o.abs() + 1e-4 * o.abs().max() + 1e-6
+            assert bool(((got - o).abs() <= tol).all()), (t, n, split, float((got - o).abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,lens,window,pool", [(8, 2, 64, SHORT, 2 ** 20, 16), (4, 2, 128, SHORT + LONG, 20, 7), (2, 2, 256, LONG, 513, 3),
+                                                    (32, 8, 128, [90 + i for i in range(40)], 64, 16), (6, 3, 64, [33] * 400, 16, 1)])
+def test_single_token_pooled_attention(dtype, H, G, D, lens, window, pool):
+    from umbrella_amd import _lib
+    code = _lib.seq_dtype_code(dtype)
+    c, pos, slot, g = _decode_store(lens, G, D, D, pool, dtype, 32, H + D + pool)
+    T = len(lens)
+    q, gate = torch.randn(T, H, D, generator=g, device="cuda"), torch.randn(T, H, generator=g, device="cuda")
+    pb = torch.randn(H, generator=g, device="cuda").to(dtype)
+    out = torch.empty(T, H * D, dtype=dtype, device="cuda")
+    _lib.seq_call("umb_pwa_attend", out, q, c.struct(0), gate, H, 0, pb, pos, slot, T, H, G, D, window, pool, D ** -0.5, code)
+    for t, n in list(enumerate(lens))[:50]:
+        i = n - 1
+        j = torch.arange(max(0, i - window + 1), n)
+        k, v = (z.double() for z in c.token_rows(0, t, j))
+        nb = max(i - window + 1, 0) // pool
+        if nb:
+            kp, vp = (z.double() for z in c.pooled_rows(0, t, torch.arange(nb)))
+            k, v = torch.cat([kp, k]), torch.cat([vp, v])
+        k, v = k.repeat_interleave(H // G, 1), v.repeat_interleave(H // G, 1)
+        w = torch.sigmoid((q[t].double()[None] * k).sum(-1) * D ** -0.5 + pb.double())
+        o = ((w[..., None] * v).sum(0) * torch.sigmoid(gate[t].double())[:, None]).reshape(-1)
+        scale = (w[..., None] * v.abs()).sum(0).max()
+        # storage rounding; fp32 sums of up to 2049 terms of that total size (2^-24 each, pairwise over waves and row groups)
+        tol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * o.abs() + 2e-6 * scale + 1e-6
+        assert bool(((out[t].double() - o).abs() <= tol).all()), (t, n, float((out[t].double() - o).abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,pool,page", [(24, 7, 64), (128, 16, 64), (200, 65, 64), (300, 130, 32), (64, 1, 8)])
+def test_pooled_blocks(dtype, D, pool, page):
+    from umbrella_amd import _lib
+    c, pos, slot, g = _decode_store([300, 131, 1], 2, D, D, pool, dtype, page, D + pool)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                                    # noqa: E731
+    p0, n = [64, 0, 0], [236, 131, 1]
+    want = {}
+    for b in range(3):
+        for blk in range((p0[b] + n[b]) // pool):
+            rows = c.token_rows(0, b, torch.arange(blk * pool, (blk + 1) * pool))
+            new = p0[b] <= blk * pool + pool - 1
+            want[b, blk] = [z.float() for z in rows] if new else [z[0].clone() for z in c.pooled_rows(0, b, [blk])]
+    _lib.seq_call("umb_pwa_pool", c.struct(0), slot, i32(p0), i32(n), 3, max(n), 2, D, pool, _lib.seq_dtype_code(dtype))
+    for (b, blk), rows in want.items():
+        for z, r in zip(c.pooled_rows(0, b, [blk]), rows):
+            if r.dim() == 3:                              # added in position order in fp32, then times the rounded 1 / pool
+                s = torch.zeros_like(r[0])
+                for x in r:
+                    s = s + x
+                r = s * torch.tensor(1.0 / pool, dtype=torch.float32, device="cuda")
+            assert torch.equal(z[0], r), (b, blk)

@@ -26,6 +26,7 @@
 // column with eight keys' rows in flight; per-wave running maximum / denominator, merged through LDS in wave order.  Which
 // keys land in which wave and round depends on the query's position alone -- never on the batch or on how a prompt was cut.
 #include "seq_common.h"
+#include "seq_decode.h"
 
 static inline bool bsa_kv_ok(const UmbPagedKV* kv) { return kv && kv->k && kv->v && kv->pages && kv->page >= 1 && kv->max_pages >= 1; }
 
@@ -104,6 +105,77 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, U
 
 constexpr int BSA_MAXC = 8;      // value columns per lane: E <= 512
 
+// positions a token sees: 0 .. kept - 1, then j_lo .. its own; n in all
+struct AttnKeys { int j_lo, kept, n; };
+__device__ __forceinline__ AttnKeys attn_keys(int i, int window, const UmbAttnForm& form) {
+  int j_lo = i - window + 1 > 0 ? i - window + 1 : 0;
+  if (form.chunk > 0) j_lo = max(j_lo, i / form.chunk * form.chunk);
+  const int kept = min(form.keep_first, j_lo);          // first positions in front of the walk
+  return AttnKeys{j_lo, kept, kept + i - j_lo + 1};
+}
+
+// end of a workgroup: the partial sums o_s [nact][RH][Ep], maxima and denominators ml_s [nact][RH][2] (and 2 RH floats behind the nw-th)
+// of its waves, added in wave order; nact <= 16: a row's factors are worked out once, by 16 lanes.
+// part: this split's result goes there instead ([token][row][split][E + 2] = o .., maximum, denominator)
+template <typename P, int RH, int NC, int MAPS>
+__device__ __forceinline__ void attn_finish(typename El<P>::type* __restrict__ out, int ldo, const float* o_s, int Ep, float* ml_s,
+                                            int nact, int nw, float* __restrict__ part, int split, int nsplit,
+                                            const float* __restrict__ proj, int ld, int gate_col, int t, int h0, int H, int E,
+                                            float out_scale, const UmbAttnForm& form) {
+  constexpr int RR = RH / MAPS;
+  const int lane = threadIdx.x & 63;
+  float* row_s = ml_s + nw * RH * 2;                       // [RH][2] maximum, denominator
+  if (threadIdx.x < RH * 16) {
+    const int r = threadIdx.x >> 4, w = threadIdx.x & 15;
+    float* ml = ml_s + (w * RH + r) * 2;
+    const float m = w < nact ? ml[0] : -INFINITY, l = w < nact ? ml[1] : 0.f;
+    const float M = row_max16(m), f = m == -INFINITY ? 0.f : expf(m - M), L = row_add16(l * f);
+    if (w < nact) ml[0] = f;
+    if (w == 0) { row_s[2 * r] = M; row_s[2 * r + 1] = L; }
+  }
+  __syncthreads();
+  auto merged = [&](int r, int d) -> float {               // unnormalised output of row r, column d
+    float o = 0.f;
+    for (int w = 0; w < nact; ++w) o += o_s[(w * RH + r) * Ep + d] * ml_s[(w * RH + r) * 2];
+    return o;
+  };
+  auto denominator = [&](int r) -> float { return row_s[2 * r + 1] + (form.sink ? expf(form.sink[h0 + r / MAPS] - row_s[2 * r]) : 0.f); };
+  auto gate_of = [&](int h, int d) {
+    return gate_col >= 0 ? 1.f / (1.f + expf(-proj[(long)t * ld + gate_col + (form.gate_elem ? h * E + d : h)])) : 1.f;
+  };
+  if (MAPS == 1 || part) {
+    for (int x = threadIdx.x; x < RH * E; x += nw * 64) {
+      const int r = x / E, d = x % E;
+      const float o = merged(r, d);
+      if (part) {
+        float* pr = part + ((((long)t * H + h0) * MAPS + r) * nsplit + split) * (E + 2);
+        pr[d] = o;
+        if (d == 0) { pr[E] = row_s[2 * r]; pr[E + 1] = row_s[2 * r + 1]; }
+        continue;
+      }
+      stf<P>(out + (long)t * ldo + (long)(h0 + r) * E + d, out_scale * gate_of(h0 + r, d) * (o / denominator(r)));
+    }
+  } else {
+    // a wave per head: o = a1 - lambda a2 over its root mean square
+    for (int rr = threadIdx.x >> 6; rr < RR; rr += nw) {
+      float v[NC], ss = 0.f;
+      const float L1 = denominator(MAPS * rr), L2 = denominator(MAPS * rr + MAPS - 1);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int d = min(lane + 64 * c, E - 1);
+        const float o = merged(MAPS * rr, d) / L1 - form.lambda * (merged(MAPS * rr + MAPS - 1, d) / L2);
+        v[c] = o;
+        if (lane + 64 * c < E) ss += o * o;
+      }
+      ss = wave_sum(ss);
+      const float f = out_scale / sqrtf(ss / (float)E + form.eps);
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        if (lane + 64 * c < E) stf<P>(out + (long)t * ldo + (long)(h0 + rr) * E + lane + 64 * c, v[c] * f * gate_of(h0 + rr, lane + 64 * c));
+    }
+  }
+}
+
 // RH rows of the workgroup = RH / MAPS query heads with MAPS maps each (row r: head r / MAPS, map r % MAPS)
 template <typename P, int RH, int NC, int NW, int MAPS>
 __global__ __launch_bounds__(NW * 64) void bsa_attend_kernel(typename El<P>::type* __restrict__ out, int ldo,
@@ -135,10 +207,8 @@ __global__ __launch_bounds__(NW * 64) void bsa_attend_kernel(typename El<P>::typ
     q_s[r * Dp + d] = q[(((long)t * H + h0) * MAPS + r) * D + d];
   }
   __syncthreads();
-  int j_lo = i - window + 1 > 0 ? i - window + 1 : 0;
-  if (form.chunk > 0) j_lo = max(j_lo, i / form.chunk * form.chunk);
-  const int kept = min(form.keep_first, j_lo);          // first positions in front of the walk: keys 0 .. kept - 1, then j_lo .. i
-  const int n_keys = kept + i - j_lo + 1;
+  const AttnKeys keys = attn_keys(i, window, form);
+  const int j_lo = keys.j_lo, kept = keys.kept, n_keys = keys.n;
   const bool vec = (D & 7) == 0 && sizeof(El_) == 2;
   float acc[RH][NC], m_run[RH], l_run[RH];
 #pragma unroll
@@ -248,62 +318,132 @@ __global__ __launch_bounds__(NW * 64) void bsa_attend_kernel(typename El<P>::typ
     if (lane == 0) { ml_s[(wave * RH + r) * 2] = m_run[r]; ml_s[(wave * RH + r) * 2 + 1] = l_run[r]; }
   }
   __syncthreads();
-  // row r of the waves' partials merged in wave order: unnormalised output of column d, maximum and denominator
-  auto merged = [&](int r, int d, float& M, float& L) -> float {
-    M = -INFINITY;
+  attn_finish<P, RH, NC, MAPS>(out, ldo, lds, Ep, ml_s, NW, NW, nsplit > 1 ? part : nullptr, split, nsplit, proj, ld, gate_col, t, h0, H, E,
+                               out_scale, form);
+}
+
+// Attention of single tokens (see seq_decode.h).  Workgroup = (token, RH rows of one key/value head, split); its waves deal the rounds of
+// 16 keys among themselves.  With nsplit > 1 workgroup z takes the spans of ATT_SPAN keys z, z + nsplit, ..; a token whose keys fit one
+// span is finished by workgroup 0 and the others leave at once, so a short context pays neither the split nor the merge.
+// Before -> now, replayed from a graph: 48 tokens behind 40 keys of 64 features 19.1 -> 6.2 us, behind 500 29.4 -> 20.5; one token behind
+// 40 / 2000 keys of 128 features 16.0 -> 7.4 / 19.2 -> 12.8 (spans of 1024: 22.0); two maps, values of 256, one token behind 40 / 1000
+// 23.0 -> 9.5 / 27.2 -> 19.8; 64 tokens behind 1000, 128 features, 81 -> 51 (262 MB of rows, 5.1 TB/s).
+constexpr int ATT_SPAN = 256;
+
+template <typename P, int RH, int LPR, int NW, int MAPS>
+__global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q, UmbPagedKV kv,
+                                                              const float* __restrict__ proj, int ld, int gate_col,
+                                                              const float* __restrict__ bias, int n_dist, const int* __restrict__ pos,
+                                                              const int* __restrict__ slot_, int H, int G, int D, int window, float scale,
+                                                              float out_scale, float softcap, UmbAttnForm form, float* __restrict__ part,
+                                                              int nsplit) {
+  constexpr int E = LPR * 8, KPI = 64 / LPR, VL = 16 / KPI, RR = RH / MAPS;
+  extern __shared__ float lds[];
+  const int split = blockIdx.z, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, quarter = lane >> 4;
+  float* q_s = lds;                                        // [RH][D]
+  float* o_s = lds + RH * D;                               // [NW][RH][E]
+  float* ml_s = o_s + NW * RH * E;                         // [NW][RH][2], [RH][2]
+  const int t = blockIdx.x, h0 = blockIdx.y * RR, g = h0 / (H / G);
+  const int i = pos[t], slot = slot_[t];
+  const AttnKeys keys = attn_keys(i, window, form);
+  const int first = split * ATT_SPAN;
+  if (first >= keys.n) return;
+  const int nact = min(NW, (min(keys.n - first, ATT_SPAN) + 15) / 16);       // waves that get a round
+  auto key_pos = [&](int kx) { return kx < keys.kept ? kx : keys.j_lo + kx - keys.kept; };
+  int base = first + wave * 16;
+  unsigned row = 0;
+  if (wave < nact) row = pkv_tok_row(kv, slot, key_pos(min(base + j, keys.n - 1)), g, G);
+  for (int x = threadIdx.x; x < RH * D; x += NW * 64) q_s[x] = q[((long)t * H + h0) * MAPS * D + x];
+  __syncthreads();
+  if (wave < nact) {
+    float acc[RH * 8], m_run[RH], l_run[RH];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) M = fmaxf(M, ml_s[(w * RH + r) * 2]);
-    float o = 0.f;
-    L = 0.f;
+    for (int r = 0; r < RH; ++r) { m_run[r] = -INFINITY; l_run[r] = 0.f; }
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float mw = ml_s[(w * RH + r) * 2];
-      const float f = mw == -INFINITY ? 0.f : expf(mw - M);
-      o += lds[(w * RH + r) * Ep + d] * f;
-      L += ml_s[(w * RH + r) * 2 + 1] * f;
-    }
-    return o;
-  };
-  auto gate_of = [&](int h, int d) {
-    return gate_col >= 0 ? 1.f / (1.f + expf(-proj[(long)t * ld + gate_col + (form.gate_elem ? h * E + d : h)])) : 1.f;
-  };
-  if (MAPS == 1 || nsplit > 1) {
-    for (int x = threadIdx.x; x < RH * E; x += NW * 64) {
-      const int r = x / E, d = x % E;
-      float M, L;
-      const float o = merged(r, d, M, L);
-      if (nsplit > 1) {                                // partial result of this split: [t][row][split][E + 2] = o.., M, L
-        float* pr = part + ((((long)t * H + h0) * MAPS + r) * nsplit + split) * (E + 2);
-        pr[d] = o;
-        if (d == 0) { pr[E] = M; pr[E + 1] = L; }
-        continue;
+    for (int v = 0; v < RH * 8; ++v) acc[v] = 0.f;
+    const u16* vcol = reinterpret_cast<const u16*>(kv.v) + (lane & (LPR - 1)) * 8;
+    while (base < keys.n) {
+      const int kx = base + j;
+      u32x4 vv[VL];
+#pragma unroll
+      for (int u = 0; u < VL; ++u) vv[u] = *reinterpret_cast<const u32x4*>(vcol + (long)(unsigned)__shfl((int)row, KPI * u + lane / LPR, 64) * E);
+      const u16* kr = reinterpret_cast<const u16*>(kv.k) + (long)row * (MAPS * D) + quarter * 8;
+      const int dist = i - key_pos(min(kx, keys.n - 1));
+      float bv[RR];
+      const int bi = dist < n_dist ? dist : n_dist - 1;
+#pragma unroll
+      for (int r = 0; r < RR; ++r) bv[r] = bias ? bias[(long)(h0 + r) * n_dist + bi] : 0.f;
+      // the next round of this wave: NW rounds on, or in the next of its workgroup's spans
+      int next = base + NW * 16;
+      if (nsplit > 1 && next / ATT_SPAN != base / ATT_SPAN) next += (nsplit - 1) * ATT_SPAN;
+      unsigned next_row = 0;
+      if (next < keys.n) next_row = pkv_tok_row(kv, slot, key_pos(min(next + j, keys.n - 1)), g, G);
+      float s[RH];
+#pragma unroll
+      for (int r = 0; r < RH; ++r) s[r] = 0.f;
+      for (int d = 0; d < D; d += 128) {
+        u32x4 kk[MAPS][4];
+#pragma unroll
+        for (int mp = 0; mp < MAPS; ++mp)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) kk[mp][u] = *reinterpret_cast<const u32x4*>(kr + mp * D + (d + 32 * u < D ? d + 32 * u : 0));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (d + 32 * u >= D) break;
+#pragma unroll
+          for (int mp = 0; mp < MAPS; ++mp) {
+            float kf[8];
+            unpack8<P>(kk[mp][u], kf);
+#pragma unroll
+            for (int r = mp; r < RH; r += MAPS) {
+              const f32x4 qa = *reinterpret_cast<const f32x4*>(q_s + r * D + d + 32 * u + quarter * 8);
+              const f32x4 qb = *reinterpret_cast<const f32x4*>(q_s + r * D + d + 32 * u + quarter * 8 + 4);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) s[r] += qa[e] * kf[e];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) s[r] += qb[e] * kf[4 + e];
+            }
+          }
+        }
       }
-      if (form.sink) L += expf(form.sink[h0 + r] - M);
-      stf<P>(out + (long)t * ldo + (long)(h0 + r) * E + d, out_scale * gate_of(h0 + r, d) * (o / L));
-    }
-  } else {
-    // a wave per head: o = a1 - lambda a2 over its root mean square
-    for (int rr = wave; rr < RR; rr += NW) {
-      float v[NC], ss = 0.f;
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const int d = dcl[c];
-        float M, L1, L2;
-        float o = merged(MAPS * rr, d, M, L1);
-        if (form.sink) L1 += expf(form.sink[h0 + rr] - M);
-        const float a2 = merged(MAPS * rr + MAPS - 1, d, M, L2);
-        if (form.sink) L2 += expf(form.sink[h0 + rr] - M);
-        o = o / L1 - form.lambda * (a2 / L2);
-        v[c] = o;
-        if (lane + 64 * c < E) ss += o * o;
+      for (int r = 0; r < RH; ++r) {
+        float sc = add_rows(s[r]) * scale;
+        if (softcap > 0.f) sc = softcap * tanhf(sc / softcap);
+        const float sv = kx < keys.n ? sc + bv[r / MAPS] : -INFINITY;
+        const float m_new = fmaxf(m_run[r], row_max16(sv));
+        const float m_ref = m_new == -INFINITY ? 0.f : m_new;          // a round of -inf scores alone: weights 0, nothing to rescale
+        const float fac = expf(m_run[r] - m_ref);
+        s[r] = kx < keys.n ? expf(sv - m_ref) : 0.f;
+        l_run[r] = l_run[r] * fac + s[r];
+        m_run[r] = m_new;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[r * 8 + e] *= fac;
       }
-      ss = wave_sum(ss);
-      const float f = out_scale / sqrtf(ss / (float)E + form.eps);
 #pragma unroll
-      for (int c = 0; c < NC; ++c)
-        if (lane + 64 * c < E) stf<P>(out + (long)t * ldo + (long)(h0 + rr) * E + dcl[c], v[c] * f * gate_of(h0 + rr, dcl[c]));
+      for (int u = 0; u < VL; ++u) {
+        float vf[8];
+        unpack8<P>(vv[u], vf);
+#pragma unroll
+        for (int r = 0; r < RH; ++r) {
+          const float w = __shfl(s[r], KPI * u + lane / LPR, 64);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[r * 8 + e] += w * vf[e];
+        }
+      }
+      base = next;
+      row = next_row;
     }
+#pragma unroll
+    for (int r = 0; r < RH; ++r) {
+      const float l = row_add16(l_run[r]);
+      if (lane == 0) { ml_s[(wave * RH + r) * 2] = m_run[r]; ml_s[(wave * RH + r) * 2 + 1] = l; }
+    }
+    store_groups<RH, LPR>(o_s + wave * RH * E, acc, lane);
   }
+  __syncthreads();
+  attn_finish<P, RH, (E + 63) / 64, MAPS>(out, ldo, o_s, E, ml_s, nact, NW, keys.n > ATT_SPAN && nsplit > 1 ? part : nullptr, split, nsplit,
+                                          proj, ld, gate_col, t, h0, H, E, out_scale, form);
 }
 
 // the splits of one (token, head) merged: lane s holds split s's maximum and denominator (a split that had no key carries
@@ -311,8 +451,15 @@ __global__ __launch_bounds__(NW * 64) void bsa_attend_kernel(typename El<P>::typ
 template <typename P, int MAPS>
 __global__ __launch_bounds__(64) void bsa_merge_kernel(typename El<P>::type* __restrict__ out, int ldo, const float* __restrict__ part,
                                                        const float* __restrict__ proj, int ld, int gate_col, int H, int E,
-                                                       int nsplit, float out_scale, UmbAttnForm form) {
+                                                       int splits, float out_scale, UmbAttnForm form, const int* __restrict__ pos,
+                                                       int window) {
   const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+  int nsplit = splits;
+  if (window > 0) {                                       // splits by spans: those that had keys, none if one workgroup did it all
+    const int n = attn_keys(pos[t], window, form).n;
+    if (n <= ATT_SPAN) return;
+    nsplit = min(splits, (n + ATT_SPAN - 1) / ATT_SPAN);
+  }
   auto gate_of = [&](int d) {
     return gate_col >= 0 ? 1.f / (1.f + expf(-proj[(long)t * ld + gate_col + (form.gate_elem ? h * E + d : h)])) : 1.f;
   };
@@ -320,7 +467,7 @@ __global__ __launch_bounds__(64) void bsa_merge_kernel(typename El<P>::type* __r
   float f[MAPS][16], inv[MAPS];
 #pragma unroll
   for (int mp = 0; mp < MAPS; ++mp) {
-    pr[mp] = part + (((long)t * H + h) * MAPS + mp) * nsplit * (E + 2);
+    pr[mp] = part + (((long)t * H + h) * MAPS + mp) * splits * (E + 2);
     const float ms = lane < nsplit ? pr[mp][lane * (E + 2) + E] : -INFINITY;
     const float ls = lane < nsplit ? pr[mp][lane * (E + 2) + E + 1] : 0.f;
     const float M = wave_max(ms);
@@ -416,6 +563,56 @@ static int bsa_launch(dim3 grid, size_t lds, hipStream_t st, void* out, int ldo,
   return UMB_OK;
 }
 
+// the decode kernel: spans of ATT_SPAN keys dealt to several workgroups only where few items leave the chip idle; 16 waves per item as
+// long as every item gets a compute unit of its own (values of 256: their registers do not hold it), 8 while two share one, 4 beyond
+template <typename P>
+static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const float* bias,
+                       int n_dist, const int* pos, const int* slot, int T, int H, int G, int D, int E, int window, float scale,
+                       float out_scale, float softcap, const UmbAttnForm& form, float* scratch, long scratch_floats, hipStream_t st) {
+  const int maps = form.maps, hpg = H / G;
+  int rh = 4;
+  while (rh > maps && hpg % (rh / maps)) rh >>= 1;
+  const int hblocks = H * maps / rh;
+  const long items = (long)T * hblocks;
+  const long most = (long)(form.chunk > 0 && form.chunk < window ? form.chunk : window) + form.keep_first;
+  int nsplit = 1;
+  if (scratch && items <= 64 && most > ATT_SPAN) {
+    nsplit = (int)(512 / items) < 16 ? (int)(512 / items) : 16;
+    if (nsplit > (most + ATT_SPAN - 1) / ATT_SPAN) nsplit = (int)((most + ATT_SPAN - 1) / ATT_SPAN);
+    while (nsplit > 1 && (long)T * H * maps * nsplit * (E + 2) > scratch_floats) nsplit >>= 1;
+  }
+  const int nw = items <= 256 && E < 256 ? 16 : (items <= 1024 ? 8 : 4);
+  const size_t lds = ((size_t)rh * D + (size_t)nw * rh * E + (size_t)(nw + 1) * rh * 2) * sizeof(float);
+#define ATT_GO(RH, LPR, NW, MAPS)                                                                                                     \
+  do {                                                                                                                               \
+    if (ensure_dynamic_lds<attn_decode_kernel<P, RH, LPR, NW, MAPS>>(lds) != UMB_OK) return UMB_EHIP;                                 \
+    hipLaunchKernelGGL((attn_decode_kernel<P, RH, LPR, NW, MAPS>), dim3(T, hblocks, nsplit), dim3(NW * 64), lds, st, (u16*)out, ldo, q,   \
+                       *kv, proj, ld, gate_col, bias, n_dist, pos, slot, H, G, D, window, scale, out_scale, softcap, form, scratch, nsplit); \
+  } while (0)
+#define ATT_NW(RH, LPR, MAPS) do { if (nw == 16) ATT_GO(RH, (LPR < 32 ? LPR : 16), 16, MAPS); else if (nw == 8) ATT_GO(RH, LPR, 8, MAPS); else ATT_GO(RH, LPR, 4, MAPS); } while (0)
+#define ATT_RH(LPR)                                                                                  \
+  do {                                                                                               \
+    if (maps == 2) { if (rh == 4) ATT_NW(4, LPR, 2); else ATT_NW(2, LPR, 2); }                        \
+    else if (rh == 4) ATT_NW(4, LPR, 1); else if (rh == 2) ATT_NW(2, LPR, 1); else ATT_NW(1, LPR, 1); \
+  } while (0)
+  if (E == 64) ATT_RH(8);
+  else if (E == 128) ATT_RH(16);
+  else ATT_RH(32);
+#undef ATT_RH
+#undef ATT_NW
+#undef ATT_GO
+  if (nsplit > 1) {
+    if (maps == 2)
+      hipLaunchKernelGGL((bsa_merge_kernel<P, 2>), dim3(T, H), dim3(64), 0, st, (u16*)out, ldo, scratch, proj, ld, gate_col, H, E, nsplit,
+                         out_scale, form, pos, window);
+    else
+      hipLaunchKernelGGL((bsa_merge_kernel<P, 1>), dim3(T, H), dim3(64), 0, st, (u16*)out, ldo, scratch, proj, ld, gate_col, H, E, nsplit,
+                         out_scale, form, pos, window);
+  }
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+
 extern "C" int umb_attn_attend(void* out, int ldo, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col,
                                const float* bias, int n_dist, const int* pos, const int* slot, int T, int H, int G, int D, int E,
                                int window, float scale, float out_scale, float softcap, const UmbAttnForm* form_, float* scratch,
@@ -425,6 +622,13 @@ extern "C" int umb_attn_attend(void* out, int ldo, const float* q, const UmbPage
     return UMB_EINVAL;
   const UmbAttnForm form = form_ ? *form_ : UmbAttnForm{1, 0, nullptr, 0.f, 0.f, 0, 0};
   if (gate_col >= 0 && (!proj || ld < gate_col + form_gate_cols(form, H, E))) return UMB_EINVAL;
+  if (decode_rows_ok(D, E, dtype, kv)) {
+    if (dtype == UMB_SEQ_BF16)
+      return attn_decode<BF16>(out, ldo, q, kv, proj, ld, gate_col, bias, n_dist, pos, slot, T, H, G, D, E, window, scale, out_scale, softcap,
+                               form, scratch, scratch_floats, st);
+    return attn_decode<F16>(out, ldo, q, kv, proj, ld, gate_col, bias, n_dist, pos, slot, T, H, G, D, E, window, scale, out_scale, softcap,
+                            form, scratch, scratch_floats, st);
+  }
   const int maps = form.maps;
   const int hpg = H / G, nc = (E + 63) / 64;
   const int Dp = (D + 3) & ~3, Ep = (E + 3) & ~3, Mp = Dp > Ep ? Dp : Ep;
@@ -475,10 +679,10 @@ extern "C" int umb_attn_attend(void* out, int ldo, const float* q, const UmbPage
     if (nsplit > 1) {
       if (maps == 2)
         hipLaunchKernelGGL((bsa_merge_kernel<P, 2>), dim3(T, H), dim3(64), 0, st, (El_*)out, ldo, scratch, proj, ld, gate_col, H, E,
-                           nsplit, out_scale, form);
+                           nsplit, out_scale, form, pos, 0);
       else
         hipLaunchKernelGGL((bsa_merge_kernel<P, 1>), dim3(T, H), dim3(64), 0, st, (El_*)out, ldo, scratch, proj, ld, gate_col, H, E,
-                           nsplit, out_scale, form);
+                           nsplit, out_scale, form, pos, 0);
     }
   })
 #undef BSA_RH

@@ -20,6 +20,7 @@
 // Because the weights are not normalised there is no running maximum and no rescaling: a query's output is a plain sum, and
 // each (token, head) sums its keys in position order per lane column -- independent of the batch and of how the prompt was cut.
 #include "seq_common.h"
+#include "seq_decode.h"
 
 // ---- rotary + unit RMS + cache append.  One wave per (token, head slot); head slots 0..H-1 are queries, H..H+G-1 keys.
 template <typename P>
@@ -75,13 +76,16 @@ __global__ __launch_bounds__(256) void pwa_prep_kernel(float* __restrict__ q, Um
   }
 }
 
-// ---- pooled blocks completed by this step: grid (block-in-step, sequence, kv head), one wave each
+// ---- pooled blocks completed by this step: grid (block-in-step, sequence, kv head), a thread per feature.
+// Latency: a handful of workgroups, each a chain of page lookups and loads.  Lane j of a wave looks up position j's row, the rows go round
+// as scalars and sixteen positions are in flight together (one at a time, each behind its own lookup, 16 positions took 19.3 us, now 4.4).
 template <typename P>
-__global__ __launch_bounds__(64) void pwa_pool_kernel(UmbPagedKV kv, const int* __restrict__ seq_slot,
-                                                      const int* __restrict__ seq_pos0, const int* __restrict__ seq_len, int G,
-                                                      int D, int pool) {
+__global__ __launch_bounds__(256) void pwa_pool_kernel(UmbPagedKV kv, const int* __restrict__ seq_slot,
+                                                       const int* __restrict__ seq_pos0, const int* __restrict__ seq_len, int G,
+                                                       int D, int pool) {
   typedef typename El<P>::type E;
-  const int b = blockIdx.y, g = blockIdx.z, lane = threadIdx.x;
+  constexpr int KB = 16;
+  const int b = blockIdx.y, g = blockIdx.z, lane = threadIdx.x & 63;
   const int p0 = seq_pos0[b], n = seq_len[b];
   if (n <= 0) return;
   // blocks whose last position e = blk pool + pool - 1 lies in [p0, p0 + n): blk >= ceil((p0 - pool + 1) / pool) = p0 / pool
@@ -92,15 +96,34 @@ __global__ __launch_bounds__(64) void pwa_pool_kernel(UmbPagedKV kv, const int* 
   const int slot = seq_slot[b];
   const long dst = pkv_blk(kv, slot, blk, pool, g, G, D);
   const float inv = 1.f / (float)pool;
-  for (int d = lane; d < D; d += 64) {
+  for (int d0 = threadIdx.x - lane; d0 < D; d0 += blockDim.x) {           // uniform in a wave
+    const int d = d0 + lane < D ? d0 + lane : D - 1;
     float sk = 0.f, sv = 0.f;
-    for (int j = 0; j < pool; ++j) {
-      const long off = pkv_tok(kv, slot, blk * pool + j, g, G, D) + d;
-      sk += ldf<P>(reinterpret_cast<const E*>(kv.k) + off);
-      sv += ldf<P>(reinterpret_cast<const E*>(kv.v) + off);
+    for (int c = 0; c < pool; c += 64) {
+      const int cnt = pool - c < 64 ? pool - c : 64;
+      const long off = pkv_tok(kv, slot, blk * pool + c + (lane < cnt ? lane : cnt - 1), g, G, D);
+      for (int j0 = 0; j0 < cnt; j0 += KB) {
+        E kk[KB], vv[KB];
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+          const int src = j0 + u < cnt ? j0 + u : cnt - 1;
+          const unsigned lo = __builtin_amdgcn_readlane((unsigned)off, src), hi = __builtin_amdgcn_readlane((unsigned)(off >> 32), src);
+          const long o = (long)(((unsigned long long)hi << 32) | lo) + d;
+          kk[u] = reinterpret_cast<const E*>(kv.k)[o];
+          vv[u] = reinterpret_cast<const E*>(kv.v)[o];
+        }
+#pragma unroll
+        for (int u = 0; u < KB; ++u)
+          if (j0 + u < cnt) {
+            sk += ldf<P>(&kk[u]);
+            sv += ldf<P>(&vv[u]);
+          }
+      }
     }
-    kv.kp[dst + d] = sk * inv;
-    kv.vp[dst + d] = sv * inv;
+    if (d0 + lane < D) {
+      kv.kp[dst + d] = sk * inv;
+      kv.vp[dst + d] = sv * inv;
+    }
   }
 }
 
@@ -278,6 +301,149 @@ __global__ __launch_bounds__(NW * 64) void pwa_attend_kernel(typename El<P>::typ
     for (int w = 1; w < NW; ++w) o += lds[(w * RH + r) * Dp + d];
     const float gate = 1.f / (1.f + expf(-proj[(long)t * ld + gate_col + h0 + r]));
     stf<P>(out + (long)t * H * D + (long)(h0 + r) * D + d, o * gate);
+  }
+}
+
+// ---- attention of single tokens (see seq_decode.h; D = 64, 128 or 256 in 16-bit storage): rounds of 16 pooled entries, then rounds of 16
+// tokens, dealt to the workgroup's waves; weights need no maximum, so the waves' sums are simply added.
+// Before -> now, replayed from a graph, D 128: one token behind 40 / 2000 keys 10.7 -> 4.9 / 30.8 -> 18.0 us, 48 tokens behind 40 20.9 -> 5.7,
+// 64 behind 1000 77 -> 45.
+template <typename P, int RH, int LPR, int NW>
+__global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ out, const float* __restrict__ q, UmbPagedKV kv,
+                                                             const float* __restrict__ proj, int ld, int gate_col,
+                                                             const u16* __restrict__ pos_bias, const int* __restrict__ pos,
+                                                             const int* __restrict__ slot_, int H, int G, int Dr, int window, int pool,
+                                                             float scale) {
+  constexpr int D = LPR * 8, KPI = 64 / LPR, VL = 16 / KPI;      // Dr = D, but not at compile time: or a round's queries are all read ahead
+  __shared__ __attribute__((aligned(16))) float q_s[RH * D];
+  extern __shared__ float o_s[];                           // [NW][RH][D]
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, quarter = lane >> 4;
+  const int t = blockIdx.x, h0 = blockIdx.y * RH, g = h0 / (H / G);
+  const int i = pos[t], slot = slot_[t];
+  const int j_lo = i - window + 1 > 0 ? i - window + 1 : 0;
+  const int n_blk = i - window + 1 >= pool ? (i - window + 1) / pool : 0;
+  const int n_tok = i - j_lo + 1, br = (n_blk + 15) / 16, rounds = br + (n_tok + 15) / 16;
+  const int nact = min(NW, rounds);
+  auto row_of = [&](int rd) {
+    return rd < br ? pkv_blk_row(kv, slot, min(rd * 16 + j, n_blk - 1), pool, g, G)
+                   : pkv_tok_row(kv, slot, j_lo + min((rd - br) * 16 + j, n_tok - 1), g, G);
+  };
+  unsigned row = 0;
+  if (wave < nact) row = row_of(wave);
+  for (int x = threadIdx.x; x < RH * D; x += NW * 64) q_s[x] = q[((long)t * H + h0) * D + x];
+  float bias[RH];
+#pragma unroll
+  for (int r = 0; r < RH; ++r) bias[r] = pos_bias ? P::to_f(pos_bias[h0 + r]) : 0.f;
+  __syncthreads();
+  if (wave < nact) {
+    float acc[RH * 8];
+#pragma unroll
+    for (int v = 0; v < RH * 8; ++v) acc[v] = 0.f;
+    float s[RH];
+    auto dots = [&](const float* kf, int d) {
+      const int at = d + quarter * 8;
+#pragma unroll
+      for (int r = 0; r < RH; ++r) {
+        const f32x4 qa = *reinterpret_cast<const f32x4*>(q_s + r * D + at);
+        const f32x4 qb = *reinterpret_cast<const f32x4*>(q_s + r * D + at + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[r] += qa[e] * kf[e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[r] += qb[e] * kf[4 + e];
+      }
+    };
+    auto weights = [&](bool valid) {
+#pragma unroll
+      for (int r = 0; r < RH; ++r) s[r] = valid ? 1.f / (1.f + expf(-(add_rows(s[r]) * scale + bias[r]))) : 0.f;
+    };
+    auto values = [&](const float* vf, int u) {
+#pragma unroll
+      for (int r = 0; r < RH; ++r) {
+        const float w = __shfl(s[r], KPI * u + lane / LPR, 64);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[r * 8 + e] += w * vf[e];
+      }
+    };
+    int rd = wave;
+    for (; rd < br; rd += NW) {                            // two loops: joined in one they need twice the registers
+      const unsigned next_row = rd + NW < rounds ? row_of(rd + NW) : 0;
+#pragma unroll
+      for (int r = 0; r < RH; ++r) s[r] = 0.f;
+      const float* kr = kv.kp + (long)row * D + quarter * 8;
+      const float* vc = kv.vp + (lane & (LPR - 1)) * 8;
+      for (int d = 0; d < Dr; d += 128) {
+        f32x4 ka[4], kb[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float* kd = kr + (d + 32 * u < Dr ? d + 32 * u : 0);
+          ka[u] = *reinterpret_cast<const f32x4*>(kd);
+          kb[u] = *reinterpret_cast<const f32x4*>(kd + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (d + 32 * u >= Dr) break;
+          const float kf[8] = {ka[u][0], ka[u][1], ka[u][2], ka[u][3], kb[u][0], kb[u][1], kb[u][2], kb[u][3]};
+          dots(kf, d + 32 * u);
+        }
+      }
+      weights(rd * 16 + j < n_blk);
+      // fp32 rows are twice as long as a token's: their values are fetched behind the scores, in registers that held the keys
+      constexpr int VB = VL < 4 ? VL : 4;
+#pragma unroll 1
+      for (int u0 = 0; u0 < VL; u0 += VB) {
+        f32x4 va[VB], vb[VB];
+#pragma unroll
+        for (int u = 0; u < VB; ++u) {
+          const float* vr = vc + (long)(unsigned)__shfl((int)row, KPI * (u0 + u) + lane / LPR, 64) * D;
+          va[u] = *reinterpret_cast<const f32x4*>(vr);
+          vb[u] = *reinterpret_cast<const f32x4*>(vr + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < VB; ++u) {
+          const float vf[8] = {va[u][0], va[u][1], va[u][2], va[u][3], vb[u][0], vb[u][1], vb[u][2], vb[u][3]};
+          values(vf, u0 + u);
+        }
+      }
+      row = next_row;
+    }
+    for (; rd < rounds; rd += NW) {
+      const unsigned next_row = rd + NW < rounds ? row_of(rd + NW) : 0;
+#pragma unroll
+      for (int r = 0; r < RH; ++r) s[r] = 0.f;
+      const u16* kr = reinterpret_cast<const u16*>(kv.k) + (long)row * D + quarter * 8;
+      const u16* vc = reinterpret_cast<const u16*>(kv.v) + (lane & (LPR - 1)) * 8;
+      u32x4 vv[VL];
+#pragma unroll
+      for (int u = 0; u < VL; ++u) vv[u] = *reinterpret_cast<const u32x4*>(vc + (long)(unsigned)__shfl((int)row, KPI * u + lane / LPR, 64) * D);
+      for (int d = 0; d < Dr; d += 128) {
+        u32x4 kk[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) kk[u] = *reinterpret_cast<const u32x4*>(kr + (d + 32 * u < Dr ? d + 32 * u : 0));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (d + 32 * u >= Dr) break;
+          float kf[8];
+          unpack8<P>(kk[u], kf);
+          dots(kf, d + 32 * u);
+        }
+      }
+      weights((rd - br) * 16 + j < n_tok);
+#pragma unroll
+      for (int u = 0; u < VL; ++u) {
+        float vf[8];
+        unpack8<P>(vv[u], vf);
+        values(vf, u);
+      }
+      row = next_row;
+    }
+    store_groups<RH, LPR>(o_s + wave * RH * D, acc, lane);
+  }
+  __syncthreads();
+  for (int x = threadIdx.x; x < RH * D; x += NW * 64) {
+    float o = o_s[x];
+    for (int w = 1; w < nact; ++w) o += o_s[w * RH * D + x];
+    const float gate = 1.f / (1.f + expf(-proj[(long)t * ld + gate_col + h0 + x / D]));
+    out[((long)t * H + h0) * D + x] = P::from_f(o * gate);
   }
 }
 
@@ -483,7 +649,7 @@ extern "C" int umb_pwa_pool(const UmbPagedKV* kv, const int* seq_slot, const int
   if (B < 1 || max_len < 1 || G < 1 || D < 1 || pool < 1 || !pkv_ok(kv) || !seq_slot || !seq_pos0 || !seq_len) return UMB_EINVAL;
   const int nb = max_len / pool + 1;             // at most this many blocks end inside max_len consecutive positions
   DISPATCH_SEQ_DTYPE(dtype, {
-    hipLaunchKernelGGL(pwa_pool_kernel<P>, dim3(nb, B, G), dim3(64), 0, st, *kv, seq_slot, seq_pos0, seq_len, G, D, pool);
+    hipLaunchKernelGGL(pwa_pool_kernel<P>, dim3(nb, B, G), dim3(D > 192 ? 256 : (D + 63) / 64 * 64), 0, st, *kv, seq_slot, seq_pos0, seq_len, G, D, pool);
   })
   UMB_LAUNCH_CHECK();
   return UMB_OK;
@@ -496,6 +662,30 @@ extern "C" int umb_pwa_attend(void* out, const float* q, const UmbPagedKV* kv, c
       !proj || !pos || !slot)
     return UMB_EINVAL;
   const int R = H / G;
+  if (decode_rows_ok(D, D, dtype, kv)) {
+    // 16 waves per item as long as every item gets a compute unit of its own, 8 while two share one, 4 beyond
+    const int rh = R % 4 == 0 ? 4 : (R % 2 == 0 ? 2 : 1);
+    const long items = (long)T * (H / rh);
+    const int nw = items <= 256 ? 16 : (items <= 1024 ? 8 : 4);
+    const size_t lds = (size_t)nw * rh * D * sizeof(float);
+#define PWD_GO(RH, LPR, NW)                                                                                                     \
+  do {                                                                                                                          \
+    if (ensure_dynamic_lds<pwa_decode_kernel<P, RH, LPR, NW>>(lds) != UMB_OK) return UMB_EHIP;                                  \
+    hipLaunchKernelGGL((pwa_decode_kernel<P, RH, LPR, NW>), dim3(T, H / rh), dim3(NW * 64), lds, st, (u16*)out, q, *kv, proj, ld,   \
+                       gate_col, (const u16*)pos_bias, pos, slot, H, G, D, window, pool, scale);                                \
+  } while (0)
+#define PWD_NW(RH, LPR) do { if (nw == 16) PWD_GO(RH, LPR, 16); else if (nw == 8) PWD_GO(RH, LPR, 8); else PWD_GO(RH, LPR, 4); } while (0)
+#define PWD_RH(LPR) do { if (rh == 4) PWD_NW(4, LPR); else if (rh == 2) PWD_NW(2, LPR); else PWD_NW(1, LPR); } while (0)
+#define PWD_D() do { if (D == 64) PWD_RH(8); else if (D == 128) PWD_RH(16); else PWD_RH(32); } while (0)
+    if (dtype == UMB_SEQ_BF16) { using P = BF16; PWD_D(); }
+    else { using P = F16; PWD_D(); }
+#undef PWD_D
+#undef PWD_RH
+#undef PWD_NW
+#undef PWD_GO
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
   const int rh = R % 8 == 0 ? 8 : (R % 4 == 0 ? 4 : (R % 2 == 0 ? 2 : 1));     // heads of one group per workgroup
   const int Dp = (D + 3) & ~3;
   const dim3 grid(T, H / rh);

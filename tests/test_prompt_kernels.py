@@ -377,3 +377,67 @@ def test_pooled_blocks(dtype, D, pool, page):
                     s = s + x
                 r = s * torch.tensor(1.0 / pool, dtype=torch.float32, device="cuda")
             assert torch.equal(z[0], r), (b, blk)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,N,S", [(257, 1024, 3), (300, 36, 1), (259, 2052, 2), (513, 4096, 5), (1024, 4096, 1), (270, 8192, 8), (258, 5120, 4)])
+def test_split_reduce_of_many_rows_is_that_of_few(dtype, T, N, S):
+    """h bit for bit what the launches of up to 256 rows give; the norm's sum of squares runs in another order (fp32): one rounding step"""
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + N)
+    code, eps = _lib.dtype_code(dtype), torch.finfo(dtype).eps
+    part = torch.randn(S, T, N, generator=g, device="cuda")
+    res, w = torch.randn(T, N, generator=g, device="cuda").to(dtype), torch.randn(N, generator=g, device="cuda").to(dtype)
+    for residual, normed in ((res, True), (None, True), (res, False)):
+        h, x = torch.full((T + 1, N), 3.0, dtype=dtype, device="cuda"), torch.full((T + 1, N), 3.0, dtype=dtype, device="cuda")
+        _lib.call("umb_reduce_residual_norm", part, S, T, N, residual, h, x if normed else None, w, 1e-5, code)
+        for lo in range(0, T, 200):
+            n = min(200, T - lo)
+            h1, x1 = torch.empty(n, N, dtype=dtype, device="cuda"), torch.empty(n, N, dtype=dtype, device="cuda")
+            _lib.call("umb_reduce_residual_norm", part[:, lo:lo + n].contiguous(), S, n, N, None if residual is None else residual[lo:lo + n], h1,
+                      x1 if normed else None, w, 1e-5, code)
+            assert torch.equal(h[lo:lo + n], h1)
+            if normed:
+                assert bool(((x[lo:lo + n].float() - x1.float()).abs() <= eps * x1.float().abs() + 1e-7).all())
+        assert bool((h[T] == 3.0).all()) and bool((x[T] == 3.0).all()) and (normed or bool((x == 3.0).all()))
+    if N % 32 == 0:
+        tt = (T + 15) // 16
+        h2, x2 = torch.empty(T, N, dtype=dtype, device="cuda"), torch.zeros(16 * tt * N, dtype=dtype, device="cuda")
+        _lib.call("umb_reduce_residual_norm_fm", part, S, T, N, res, h2, x2, w, 1e-5, tt, code)
+        _lib.call("umb_reduce_residual_norm", part, S, T, N, res, h, x, w, 1e-5, code)
+        fm = x2.view(N // 32, tt, 4, 16, 8).permute(1, 3, 0, 2, 4).reshape(16 * tt, N)[:T]
+        assert torch.equal(fm, x[:T]) and torch.equal(h2, h[:T])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,Hq,Hkv,D,S,paired", [(257, 4, 2, 64, 2, 1), (400, 4, 1, 96, 3, 1), (263, 3, 1, 32, 1, 0), (514, 2, 2, 128, 4, 0), (1024, 5, 1, 256, 8, 1)])
+def test_split_reduce_and_rotation_of_many_tokens_is_that_of_few(dtype, T, Hq, Hkv, D, S, paired):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + D)
+    N, L, code = (Hq + 2 * Hkv) * D, 1536, _lib.dtype_code(dtype)
+    part = torch.randn(S, T, N, generator=g, device="cuda")
+    cos, sin = torch.randn(L, D, generator=g, device="cuda").to(dtype), torch.randn(L, D, generator=g, device="cuda").to(dtype)
+    pos = torch.randint(0, L, (T,), generator=g, device="cuda", dtype=torch.int32)
+    bias = torch.randn(N, generator=g, device="cuda").to(dtype)
+    ssq = torch.rand(T, 7, generator=g, device="cuda") + 0.5
+    runs = {"in a row": torch.arange(T, device="cuda") + 100, "off the grid": torch.arange(T, device="cuda") + 101,
+            "anywhere": torch.randperm(L, generator=g, device="cuda")[:T]}
+    for name, slot in runs.items():
+        slot = slot.to(torch.int32)
+        for b, q2 in ((None, None), (bias, None), (None, ssq), (bias, ssq)):
+            outs = []
+            for step in (T, 200):
+                q = torch.full((T + 1, Hq * D), 3.0, dtype=dtype, device="cuda")
+                kc, vt = torch.full((Hkv, L * D), 3.0, dtype=dtype, device="cuda"), torch.full((Hkv, D * (L + 32)), 3.0, dtype=dtype, device="cuda")
+                for lo in range(0, T, step):
+                    n = min(step, T - lo)
+                    _lib.call("umb_reduce_qkv_rope2", part[:, lo:lo + n].contiguous(), S, n, Hq, Hkv, D, L, pos[lo:lo + n], slot[lo:lo + n], cos, sin,
+                              q[lo:lo + n], kc, vt, paired, b, None if q2 is None else q2[lo:lo + n], 0 if q2 is None else 5, 0 if q2 is None else 7,
+                              0.0 if q2 is None else 40.0, 1e-5, code)
+                outs.append((q, kc, vt))
+            for x, y in zip(*outs):
+                if b is None or q2 is None:
+                    assert torch.equal(x, y), (name, b is not None)
+                else:       # x / rms + bias may be one fp32 rounding or two: then each of the rotation's two products may round the other way
+                    eps = torch.finfo(dtype).eps
+                    assert bool(((x.float() - y.float()).abs() <= 4 * eps * y.float().abs().max()).all()) and (x != y).float().mean() < 1e-2

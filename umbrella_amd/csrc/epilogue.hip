@@ -173,6 +173,62 @@ __global__ __launch_bounds__(1024) void reduce_residual_norm_kernel(const float*
   }
 }
 
+// The same for many rows: NT threads a row with CG column groups each, so that several rows share a compute unit and one row's sum and
+// stores hide behind another's loads.  1024 threads a row left two rows a unit, each waiting for its own loads, sum and stores in turn.
+// Before -> now (us): 257 rows of 4096, 4 splits 11.6 -> 8.4; 1024 rows of 2048, 2 splits 18.2 -> 7.9 (29 MB, 3.7 TB/s); of 4096, one split
+// 19.1 -> 10.8 (42 MB, 3.9 TB/s), 4 splits 25.5 -> 18.0 (92 MB, 5.1 TB/s); of 8192, 8 splits 61.5 -> 56.2 (319 MB, 5.7 TB/s).
+template <typename P, int NT, int CG>
+__global__ __launch_bounds__(NT) void reduce_residual_norm_wide_kernel(const float* __restrict__ part, int S, int T, int N,
+                                                                       const u16* residual, u16* h_out, u16* __restrict__ xn_out,
+                                                                       const u16* __restrict__ w, float eps, int xn_fm_tt) {
+  __shared__ float red[16];
+  const int t = blockIdx.x;
+  const long sstride = (long)T * N;
+  const float* p = part + (long)t * N;
+  f32x4 a[CG];
+  uint2 r[CG], o[CG];
+  int at[CG];
+#pragma unroll
+  for (int c = 0; c < CG; ++c) {
+    at[c] = (c * NT + (int)threadIdx.x) * 4;
+    const int i = at[c] < N ? at[c] : 0;
+    a[c] = LDP(p + i);
+    r[c] = residual ? *reinterpret_cast<const uint2*>(residual + (long)t * N + i) : uint2{0u, 0u};
+  }
+#pragma unroll 4
+  for (int s = 1; s < S; ++s) {
+    f32x4 v[CG];
+#pragma unroll
+    for (int c = 0; c < CG; ++c) v[c] = LDP(p + (long)s * sstride + (at[c] < N ? at[c] : 0));
+#pragma unroll
+    for (int c = 0; c < CG; ++c) a[c] += v[c];                 // fixed order 0..S-1
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CG; ++c) {
+    float x0 = rnd<P>(a[c][0]), x1 = rnd<P>(a[c][1]), x2 = rnd<P>(a[c][2]), x3 = rnd<P>(a[c][3]);
+    if (residual) { x0 += lo_f<P>(r[c].x); x1 += hi_f<P>(r[c].x); x2 += lo_f<P>(r[c].y); x3 += hi_f<P>(r[c].y); }
+    o[c].x = pack2<P>(x0, x1); o[c].y = pack2<P>(x2, x3);
+    if (at[c] < N) {
+      if (h_out) *reinterpret_cast<uint2*>(h_out + (long)t * N + at[c]) = o[c];
+      x0 = lo_f<P>(o[c].x); x1 = hi_f<P>(o[c].x); x2 = lo_f<P>(o[c].y); x3 = hi_f<P>(o[c].y);
+      ss += x0 * x0 + x1 * x1 + x2 * x2 + x3 * x3;
+    }
+  }
+  if (!xn_out) return;
+  ss = block_sum<NT>(ss, red);
+  const float inv = rsqrtf(ss / (float)N + eps);
+#pragma unroll
+  for (int c = 0; c < CG; ++c)
+    if (at[c] < N) {
+      const uint2 g = *reinterpret_cast<const uint2*>(w + at[c]);
+      uint2 x;
+      x.x = pack2<P>(lo_f<P>(o[c].x) * inv * lo_f<P>(g.x), hi_f<P>(o[c].x) * inv * hi_f<P>(g.x));
+      x.y = pack2<P>(lo_f<P>(o[c].y) * inv * lo_f<P>(g.y), hi_f<P>(o[c].y) * inv * hi_f<P>(g.y));
+      *reinterpret_cast<uint2*>(xn_out + (xn_fm_tt ? fm_off(t, at[c], xn_fm_tt) : (long)t * N + at[c])) = x;
+    }
+}
+
 // ---- act[t][i] = silu(gate) * up ; partial rows hold [gate(0..I) | up(I..2I)]
 template <typename P>
 __global__ __launch_bounds__(256) void reduce_silu_mul_kernel(const float* __restrict__ part, int S, int T, int I,
@@ -318,6 +374,142 @@ __global__ __launch_bounds__(64) void reduce_qkv_rope_kernel(const float* __rest
   }
 }
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+// The same for many tokens: a workgroup takes 256 columns of 16 tokens, a wave four of the tokens, a lane four columns of each; the loads of
+// the four tokens are in flight together.  K and V lines hold 4 and 32 keys: with a workgroup per (token, head) they were completed by
+// workgroups on different dies, two bytes at a time; here one workgroup writes whole lines, V four keys a store where the slots run on.
+// Before -> now (us), 32 + 2 * 8 heads: 257 tokens, D 64, 2 splits 8.3 -> 6.2; 1024 tokens, D 64, 2 splits 23.5 -> 10.6, D 128, one split
+// 25.0 -> 13.9 (38 MB, 2.7 TB/s), 4 splits 27.3 -> 23.6 (113 MB, 4.8 TB/s).
+template <typename P, bool PAIRED>
+__global__ __launch_bounds__(256) void reduce_qkv_rope_wide_kernel(const float* __restrict__ part, int S, int T, int Hq, int Hkv, int D,
+                                                                   int Lmax, const int* __restrict__ pos, const int* __restrict__ slot,
+                                                                   const u16* __restrict__ cosT, const u16* __restrict__ sinT,
+                                                                   u16* __restrict__ q_out, u16* __restrict__ kc, u16* __restrict__ vt,
+                                                                   const u16* __restrict__ bias,
+                                                                   const float* __restrict__ ssq_in, int ssq_groups, int ssq_stride,
+                                                                   float ssq_dim, float eps) {
+  constexpr int TT = 4;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int t0 = blockIdx.y * 16 + wave * TT;
+  if (t0 >= T) return;
+  const int N = (Hq + 2 * Hkv) * D, half = D / 2;
+  const int col = blockIdx.x * 256 + 4 * lane;
+  const bool ok = col < N;
+  const int cc = ok ? col : N - 4, hd = cc / D, c = cc - hd * D;
+  // quad: the lane's four columns are what it needs: V features c .. c + 3, or rotation partners packed next to each other (c / 2,
+  // c / 2 + half, c / 2 + 1, ..); otherwise features c / 2, c / 2 + 1 and their partners half a head further on
+  const bool is_v = hd >= Hq + Hkv, quad = is_v || PAIRED;
+  const int d = is_v ? c : c / 2;
+  const long sstride = (long)T * N;
+  f32x4 a[TT];
+  auto fetch = [&](int u, int s) -> f32x4 {
+    const float* row = part + (long)s * sstride + (long)min(t0 + u, T - 1) * N;
+    if (PAIRED) return LDP(row + cc);
+    const f32x2 x = *reinterpret_cast<const f32x2*>(row + (quad ? cc : hd * D + d));
+    const f32x2 y = *reinterpret_cast<const f32x2*>(row + (quad ? cc + 2 : hd * D + d + half));
+    return quad ? f32x4{x[0], x[1], y[0], y[1]} : f32x4{x[0], y[0], x[1], y[1]};
+  };
+  int sl[TT], ps[TT];
+  bool run = true;                                         // four slots in a row, inside one group of eight keys
+#pragma unroll
+  for (int u = 0; u < TT; ++u) {
+    const int t = min(t0 + u, T - 1);
+    sl[u] = slot[t];
+    ps[u] = pos[t];
+    run = run && t0 + u < T && sl[u] == sl[0] + u;
+  }
+#pragma unroll
+  for (int u = 0; u < TT; ++u) a[u] = fetch(u, 0);
+  unsigned ck[TT][4];                                      // cos, sin of features d, d + 1 and of their partners
+#pragma unroll
+  for (int u = 0; u < TT; ++u) {
+    const long ct = (long)ps[u] * D + (is_v ? 0 : d);
+    ck[u][0] = *reinterpret_cast<const unsigned*>(cosT + ct);
+    ck[u][1] = *reinterpret_cast<const unsigned*>(cosT + ct + half);
+    ck[u][2] = *reinterpret_cast<const unsigned*>(sinT + ct);
+    ck[u][3] = *reinterpret_cast<const unsigned*>(sinT + ct + half);
+  }
+  int s = 1;
+  for (; s + 2 < S; s += 3) {                              // three splits of four tokens in flight
+    f32x4 v[3][TT];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int u = 0; u < TT; ++u) v[k][u] = fetch(u, s + k);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int u = 0; u < TT; ++u) a[u] += v[k][u];        // fixed order 0..S-1
+  }
+  for (; s < S; ++s)
+#pragma unroll
+    for (int u = 0; u < TT; ++u) a[u] += fetch(u, s);
+  run = run && (sl[0] & 3) == 0;
+  float b4[4] = {0.f, 0.f, 0.f, 0.f};                      // bias of the lane's columns, in the order of a[u]
+  if (bias) {
+    const u16* bh = bias + hd * D;
+    b4[0] = P::to_f(bh[d]);
+    b4[1] = P::to_f(bh[is_v ? d + 1 : d + half]);
+    b4[2] = P::to_f(bh[is_v ? d + 2 : d + 1]);
+    b4[3] = P::to_f(bh[is_v ? d + 3 : d + 1 + half]);
+  }
+#pragma unroll
+  for (int u = 0; u < TT; ++u) {
+    float inv = 1.f;
+    if (ssq_in) {
+      float q = 0.f;
+      for (int x = lane; x < ssq_groups; x += 64) q += ssq_in[(long)min(t0 + u, T - 1) * ssq_stride + x];
+      inv = rsqrtf(wave_sum(q) / ssq_dim + eps);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = a[u][e] * inv;
+      if (bias) v += b4[e];
+      a[u][e] = rnd<P>(v);
+    }
+  }
+  if (!ok) return;
+  if (is_v) {
+    u16* vo = vt + (long)(hd - Hq - Hkv) * D * VT_LD(Lmax);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (run) {
+        *reinterpret_cast<uint2*>(vo + vt_off(d + e, sl[0], D)) = uint2{pack2<P>(a[0][e], a[1][e]), pack2<P>(a[2][e], a[3][e])};
+      } else {
+#pragma unroll
+        for (int u = 0; u < TT; ++u)
+          if (t0 + u < T) vo[vt_off(d + e, sl[u], D)] = P::from_f(a[u][e]);
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < TT; ++u) {
+    if (t0 + u >= T) break;
+    float oa[2], ob[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      // rotate-half RoPE in the model dtype (each product and the sum are rounded, as eager torch does)
+      const float va = a[u][2 * e], vb = a[u][2 * e + 1];
+      const float ka = e ? hi_f<P>(ck[u][0]) : lo_f<P>(ck[u][0]), kb = e ? hi_f<P>(ck[u][1]) : lo_f<P>(ck[u][1]);
+      const float sa = e ? hi_f<P>(ck[u][2]) : lo_f<P>(ck[u][2]), sb = e ? hi_f<P>(ck[u][3]) : lo_f<P>(ck[u][3]);
+      oa[e] = rnd<P>(mul_rnd<P>(va, ka) + mul_rnd<P>(-vb, sa));
+      ob[e] = rnd<P>(mul_rnd<P>(vb, kb) + mul_rnd<P>(va, sb));
+    }
+    u16 *x, *y;
+    if (hd < Hq) {
+      x = q_out + ((long)(t0 + u) * Hq + hd) * D + d;
+      y = x + half;
+    } else {
+      u16* ko = kc + (long)(hd - Hq) * Lmax * D;           // fragment order inside the head's slab (common.h)
+      x = ko + kc_off(sl[u], d, D);
+      y = ko + kc_off(sl[u], d + half, D);
+    }
+    *reinterpret_cast<unsigned*>(x) = pack2<P>(oa[0], oa[1]);
+    *reinterpret_cast<unsigned*>(y) = pack2<P>(ob[0], ob[1]);
+  }
+}
+
 // ---- embedding gather + per-forward index prep.
 // TREE mode  (tokens_all != null): token i = tokens_all[n + off + i], pos = n + depth[off+i], slot = n + off + i
 // EXPLICIT   : tokens/pos/slot given; they are copied into the workspace arrays the later kernels read.
@@ -434,10 +626,26 @@ extern "C" int umb_rmsnorm(void* out, const void* x, const void* w, float eps, i
 }
 
 // xn_fm_tt: as fm_tt above, for xn_out only
+// more rows than compute units: rows share a unit (both sides at the kernel; 100 rows of 4096, 4 splits: 6.3 -> 7.0 us, 257: 11.6 -> 8.4)
+constexpr int WIDE_ROWS = 257;
 extern "C" int umb_reduce_residual_norm_fm(const void* partial, int S, int T, int N, const void* residual, void* h_out,
                                            void* xn_out, const void* w, float eps, int xn_fm_tt, int dtype, hipStream_t st) {
   if (N % 4 || T < 1 || xn_fm_tt < 0 || (xn_fm_tt && (T > 16 * xn_fm_tt || N % 32))) return UMB_EINVAL;
   const size_t sm = 64 + (size_t)N * 2;
+  if (T >= WIDE_ROWS && S >= 1 && N <= 8192) {
+#define RNW(NT, CG)                                                                                                              \
+  hipLaunchKernelGGL((reduce_residual_norm_wide_kernel<P, NT, CG>), dim3(T), dim3(NT), 0, st, (const float*)partial, S, T, N,    \
+                     (const u16*)residual, (u16*)h_out, (u16*)xn_out, (const u16*)w, eps, xn_fm_tt)
+    DISPATCH_DTYPE(dtype, {
+      if (N <= 1024) RNW(256, 1);
+      else if (N <= 2048) RNW(256, 2);
+      else if (N <= 4096) RNW(256, 4);
+      else RNW(512, 4);
+    })
+#undef RNW
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
   DISPATCH_DTYPE(dtype, {
     hipLaunchKernelGGL((reduce_residual_norm_kernel<P>), dim3(T), dim3(1024), sm, st, (const float*)partial, S, T, N,
                        (const u16*)residual, (u16*)h_out, (u16*)xn_out, (const u16*)w, eps, xn_fm_tt);
@@ -482,6 +690,20 @@ extern "C" int umb_reduce_qkv_rope2(const void* partial, int S, int T, int Hq, i
                                     void* k_cache, void* vt_cache, int paired, const void* bias, const float* ssq_in,
                                     int ssq_groups, int ssq_stride, float ssq_dim, float eps, int dtype, hipStream_t st) {
   if (D % 32 || Lmax % 32 || (ssq_in && (ssq_groups < 1 || ssq_stride < ssq_groups || ssq_dim <= 0.f))) return UMB_EINVAL;   // 32-key x 32-feature cache tiles
+  // from where a workgroup per (token, head) means rounds of them; many splits move the line up (257 tokens, 64 + 8 heads of 128: 2 splits
+  // 12.0 -> 10.2 us, 8 splits 16.4 -> 19.8)
+  if (T >= WIDE_ROWS && T >= 128 * S && S >= 1 && ((uintptr_t)partial % 16 | (uintptr_t)q_out % 4 | (uintptr_t)k_cache % 4 | (uintptr_t)vt_cache % 8 | (uintptr_t)cosT % 4 | (uintptr_t)sinT % 4) == 0) {
+#define QRW(PAIRED)                                                                                                                \
+  hipLaunchKernelGGL((reduce_qkv_rope_wide_kernel<P, PAIRED>), dim3(((Hq + 2 * Hkv) * D + 255) / 256, (T + 15) / 16), dim3(256), 0, st,   \
+                     (const float*)partial, S, T, Hq, Hkv, D, Lmax, pos, slot, (const u16*)cosT, (const u16*)sinT, (u16*)q_out,     \
+                     (u16*)k_cache, (u16*)vt_cache, (const u16*)bias, ssq_in, ssq_groups, ssq_stride, ssq_dim, eps)
+    DISPATCH_DTYPE(dtype, {
+      if (paired) QRW(true); else QRW(false);
+    })
+#undef QRW
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
   DISPATCH_DTYPE(dtype, {
     hipLaunchKernelGGL((reduce_qkv_rope_kernel<P>), dim3(T, Hq + 2 * Hkv), dim3(64), 0, st, (const float*)partial, S, T,
                        Hq, Hkv, D, Lmax, pos, slot, (const u16*)cosT, (const u16*)sinT, (u16*)q_out, (u16*)k_cache,

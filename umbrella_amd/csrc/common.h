@@ -65,12 +65,9 @@ struct BF16 {
   static constexpr float MAGIC_OFF = 128.0f;
   static constexpr unsigned ONE2 = 0x3F803F80u;    // packed (1.0, 1.0)
   __device__ __forceinline__ static float to_f(u16 b) { return __uint_as_float(((unsigned)b) << 16); }
-  __device__ __forceinline__ static u16 from_f(float f) {   // round-to-nearest-even
-    unsigned u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (u16)((u >> 16) | 0x40);   // quiet NaN
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (u16)(u >> 16);
-  }
+  // round-to-nearest-even, NaN made quiet: v_cvt_pk_bf16_f32.  Written out in integers (an add, a bit field, a compare and a select per
+  // value) it was a third of the vector work of the prompt attention kernels; the two agree on all 2^32 inputs.
+  __device__ __forceinline__ static u16 from_f(float f) { return __builtin_bit_cast(u16, (__bf16)f); }
   __device__ __forceinline__ static f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
@@ -107,6 +104,11 @@ template <typename P> __device__ __forceinline__ float rnd_prod(float x, float y
 }
 template <typename P> __device__ __forceinline__ unsigned pack2(float lo, float hi) {
   return (unsigned)P::from_f(lo) | ((unsigned)P::from_f(hi) << 16);
+}
+template <> __device__ __forceinline__ unsigned pack2<BF16>(float lo, float hi) {         // one conversion for both
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f2{lo, hi}), b2));
 }
 template <typename P> __device__ __forceinline__ float lo_f(unsigned w) { return P::to_f((u16)(w & 0xffffu)); }
 template <typename P> __device__ __forceinline__ float hi_f(unsigned w) { return P::to_f((u16)(w >> 16)); }

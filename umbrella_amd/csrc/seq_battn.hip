@@ -714,9 +714,8 @@ extern "C" int umb_bsa_attend(void* out, int ldo, const float* q, const UmbPaged
 constexpr float BSA_LOG2E = 1.4426950408889634f;
 
 template <typename P> __device__ __forceinline__ void split2(float a, float b, unsigned& hi, unsigned& lo) {
-  const u16 ah = P::from_f(a), bh = P::from_f(b);
-  hi = (unsigned)ah | ((unsigned)bh << 16);
-  lo = pack2<P>(a - P::to_f(ah), b - P::to_f(bh));
+  hi = pack2<P>(a, b);
+  lo = pack2<P>(a - lo_f<P>(hi), b - hi_f<P>(hi));
 }
 
 // HPW rows per wave = HPW / MAPS heads with MAPS maps each; every map has its part of the staged key rows, the value fragments of

@@ -461,10 +461,8 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
 template <typename P> __device__ __forceinline__ void split8(const float* v, u32x4& hi, u32x4& lo) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const u16 h0 = P::from_f(v[2 * e]), h1 = P::from_f(v[2 * e + 1]);
-    const u16 l0 = P::from_f(v[2 * e] - P::to_f(h0)), l1 = P::from_f(v[2 * e + 1] - P::to_f(h1));
-    hi[e] = (unsigned)h0 | ((unsigned)h1 << 16);
-    lo[e] = (unsigned)l0 | ((unsigned)l1 << 16);
+    hi[e] = pack2<P>(v[2 * e], v[2 * e + 1]);
+    lo[e] = pack2<P>(v[2 * e] - lo_f<P>(hi[e]), v[2 * e + 1] - hi_f<P>(hi[e]));
   }
 }
 

@@ -318,14 +318,22 @@ __global__ __launch_bounds__(64 * NW, NQ > 1 ? 1 : 2) void tree_attn1_kernel(con
       }
       float pv[8];
       float tmax = NEG_BIG;
+      // a tile every row sees whole (most of a prompt's, and the prefix of a tree's) needs no tests; rows past the last are not stored
+      if (k0 + 32 <= k_hi && __ballot(vbits != 0xffu) == 0) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int key = k0 + gq * 8 + e;
-        float sc = st[e >> 2][e & 3] * scale;
-        const bool vis = row_ok[qi] && key < k_hi && ((vbits >> e) & 1u);
-        sc = vis ? sc : -INFINITY;
-        pv[e] = sc;
-        tmax = fmaxf(tmax, sc);
+        for (int e = 0; e < 8; ++e) {
+          pv[e] = st[e >> 2][e & 3] * scale;
+          tmax = fmaxf(tmax, pv[e]);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int key = k0 + gq * 8 + e;
+          const float sc = st[e >> 2][e & 3] * scale;
+          const bool vis = row_ok[qi] && key < k_hi && ((vbits >> e) & 1u);
+          pv[e] = vis ? sc : -INFINITY;
+          tmax = fmaxf(tmax, pv[e]);
+        }
       }
       tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
       tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
@@ -339,11 +347,12 @@ __global__ __launch_bounds__(64 * NW, NQ > 1 ? 1 : 2) void tree_attn1_kernel(con
       for (int e = 0; e < 4; ++e) pb[e] = pack2<P>(pv[2 * e], pv[2 * e + 1]);
       l[qi] = l[qi] * alpha + psum;
       m[qi] = m_new;
+      if (__ballot(alpha != 1.f)) {                                 // a row's maximum moved
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        o[qi][dt] *= alpha;
-        o[qi][dt] = P::mfma(av[dt], pb, o[qi][dt]);
+        for (int dt = 0; dt < DT; ++dt) o[qi][dt] *= alpha;
       }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[qi][dt] = P::mfma(av[dt], pb, o[qi][dt]);
     }
   };
 

@@ -711,6 +711,9 @@ extern "C" int umb_bsa_attend(void* out, int ldo, const float* q, const UmbPaged
 // exponents, accumulators rescaled only when a maximum moved; the lane's eight weights ARE its share of the B operand of the
 // value product.  Scores and weights keep fp32 accuracy on the 16-bit pipe: the fp32 queries and the fp32 weights enter as
 // high + low 16-bit halves (two products each, 2^-17 relative).
+// NSM / NVM bound the unrolled register arrays; EXACT: they are the counts (the sizes that are used in earnest).  With run-time counts every
+// product stood in a block of its own behind its own LDS read; with a whole step's reads free to move ahead, and steps that every query sees
+// whole left untested, 1999 positions, 32 + 8 heads of 128 went from 212 us to 140, two maps over 617 positions, 64 | 128, from 104 to 71.
 constexpr float BSA_LOG2E = 1.4426950408889634f;
 
 template <typename P> __device__ __forceinline__ void split2(float a, float b, unsigned& hi, unsigned& lo) {
@@ -720,7 +723,7 @@ template <typename P> __device__ __forceinline__ void split2(float a, float b, u
 
 // HPW rows per wave = HPW / MAPS heads with MAPS maps each; every map has its part of the staged key rows, the value fragments of
 // a step serve all rows
-template <typename P, int NSM, int NVM, int HPW, int MAPS>
+template <typename P, int NSM, int NVM, int HPW, int MAPS, bool EXACT>
 __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q,
                                                               UmbPagedKV kv, const float* __restrict__ proj, int ld, int gate_col,
                                                               const float* __restrict__ bias, int n_dist,
@@ -729,6 +732,7 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
                                                               int H, int G, int D, int E, int window, float scale, float out_scale,
                                                               float softcap, UmbAttnForm form) {
   extern __shared__ __attribute__((aligned(16))) u16 bsa_lds[];
+  if constexpr (EXACT) { D = NSM * 32; E = NVM * 16; }      // the counts as constants
   static_assert(HPW % MAPS == 0, "a wave owns whole heads");
   constexpr int HW = HPW / MAPS;                      // heads per wave
   constexpr int NLK = (NSM * 4 * MAPS + 7) / 8, NLV = (NVM * 2 + 7) / 8;     // 16-byte chunks of a key / value row per staging thread
@@ -762,6 +766,7 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     j_lo = max(j_lo, i_first / form.chunk * form.chunk);
     c_lo = i_j / form.chunk * form.chunk;
   }
+  const int lo_all = max(i_last - window + 1, form.chunk > 0 ? i_last / form.chunk * form.chunk : 0);         // first position every query sees
   const int kept = min(form.keep_first, j_lo);        // first positions in front of the walk: step rows 0 .. kept - 1, then j_lo .. i_last
   const int j_off = j_lo - kept;
   const int total = kept + i_last - j_lo + 1;
@@ -806,8 +811,8 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     const int kx = base + sm;
     const bool ok = kx < total;
     const int jk = kx < kept ? kx : j_off + kx;
-    const long offk = ok ? pkv_tok(kv, slot, jk, g, G, DK) : 0;
-    const long offv = ok ? pkv_tok(kv, slot, jk, g, G, E) : 0;
+    const unsigned rw = ok ? pkv_tok_row(kv, slot, jk, g, G) : 0;
+    const long offk = (long)rw * DK, offv = (long)rw * E;
 #pragma unroll
     for (int u = 0; u < NLK; ++u) {
       const int ch = sc + 8 * u;
@@ -820,6 +825,7 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     }
   };
   fetch(0);
+  if (threadIdx.x < 32) *reinterpret_cast<u32x4*>(k_s + threadIdx.x * LD + DK) = u32x4{0u, 0u, 0u, 0u};       // read where a step of 32 runs past D
   for (int base = 0; base < total; base += 32) {
     __syncthreads();                                  // every wave is done with the previous tile
 #pragma unroll
@@ -842,21 +848,18 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     if (base + 32 < total) fetch(base + 32);          // in flight while this step is used
     if (!active) continue;
     // which of the lane's eight keys this query sees, and at what distance: the same for every head
-    bool vis[8];
-    int di[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int kx = base + 16 * (e >> 2) + 4 * g4 + (e & 3);
-      const int jt = kx < kept ? kx : j_off + kx;
-      vis[e] = q_ok && jt <= i_j && ((jt > i_j - window && jt >= c_lo) || jt < form.keep_first);
-      const int dd = i_j - jt;
-      di[e] = dd < 0 ? 0 : (dd < n_dist ? dd : n_dist - 1);
-    }
+    // (a step that every query sees whole needs no tests: rows past the last are not stored)
+    const bool whole = base >= kept && j_off + base + 31 <= i_first && j_off + base >= lo_all;
     float bv[HPW][8];
+    if (bias) {
 #pragma unroll
-    for (int hh = 0; hh < HPW; ++hh)
+      for (int e = 0; e < 8; ++e) {
+        const int kx = base + 16 * (e >> 2) + 4 * g4 + (e & 3);
+        const int dd = i_j - (kx < kept ? kx : j_off + kx), di = dd < 0 ? 0 : (dd < n_dist ? dd : n_dist - 1);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) bv[hh][e] = bias ? bias[(long)hd[hh] * n_dist + di[e]] : 0.f;
+        for (int hh = 0; hh < HPW; ++hh) bv[hh][e] = bias[(long)hd[hh] * n_dist + di];
+      }
+    }
     f32x4 sc2[HPW][2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -869,7 +872,7 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
         if (s < ns) {
 #pragma unroll
           for (int mp = 0; mp < MAPS; ++mp) {
-            const u32x4 kf = d < D ? *reinterpret_cast<const u32x4*>(kr + mp * D + d) : u32x4{0u, 0u, 0u, 0u};
+            const u32x4 kf = *reinterpret_cast<const u32x4*>(kr + (d < D ? mp * D + d : DK));
 #pragma unroll
             for (int hh = mp; hh < HPW; hh += MAPS) {
               sc2[hh][u] = P::mfma(kf, ql[hh][s], sc2[hh][u]);
@@ -886,11 +889,23 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
       float sv[8], mx = -INFINITY;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        float raw = sc2[hh][e >> 2][e & 3] * scale2;
-        if (softcap > 0.f) raw = softcap * tanhf(sc2[hh][e >> 2][e & 3] * scale / softcap) * BSA_LOG2E;      // capped, then to base 2
-        sv[e] = vis[e] ? raw + bv[hh][e] * BSA_LOG2E : -INFINITY;
-        mx = fmaxf(mx, sv[e]);
+        sv[e] = sc2[hh][e >> 2][e & 3] * scale2;
+        if (softcap > 0.f) sv[e] = softcap * tanhf(sc2[hh][e >> 2][e & 3] * scale / softcap) * BSA_LOG2E;      // capped, then to base 2
       }
+      if (bias) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sv[e] += bv[hh][e] * BSA_LOG2E;
+      }
+      if (!whole) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int kx = base + 16 * (e >> 2) + 4 * g4 + (e & 3);
+          const int jt = kx < kept ? kx : j_off + kx;
+          sv[e] = q_ok && jt <= i_j && ((jt > i_j - window && jt >= c_lo) || jt < form.keep_first) ? sv[e] : -INFINITY;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sv[e]);
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float m_new = fmaxf(m_run[hh], mx);
@@ -999,21 +1014,27 @@ extern "C" int umb_attn_attend_tiled(void* out, int ldo, const float* q, const U
   if (gate_col >= 0 && (!proj || ld < gate_col + form_gate_cols(form, H, E))) return UMB_EINVAL;
   const int hpg = H / G, maps = form.maps;
   const size_t lds = ((size_t)32 * (maps * D + 8) + (size_t)E * 36) * sizeof(u16);
-#define BSA_MFMA(NSM, NVM, HPW, MAPS)                                                                                      \
+#define BSA_MFMA(NSM, NVM, HPW, MAPS, EX)                                                                                  \
   do {                                                                                                                     \
     const int hblocks = (hpg + 4 * (HPW / MAPS) - 1) / (4 * (HPW / MAPS));                                                 \
     if ((long)G * hblocks > 65535) return UMB_EINVAL;                                                                      \
     const dim3 grid((max_len + 15) / 16, B, G * hblocks);                                                                  \
-    if (ensure_dynamic_lds<bsa_attend_mfma_kernel<P, NSM, NVM, HPW, MAPS>>(lds) != UMB_OK) return UMB_EHIP;                \
-    hipLaunchKernelGGL((bsa_attend_mfma_kernel<P, NSM, NVM, HPW, MAPS>), grid, dim3(256), lds, st, (u16*)out, ldo, q, *kv, \
+    if (ensure_dynamic_lds<bsa_attend_mfma_kernel<P, NSM, NVM, HPW, MAPS, EX>>(lds) != UMB_OK) return UMB_EHIP;                \
+    hipLaunchKernelGGL((bsa_attend_mfma_kernel<P, NSM, NVM, HPW, MAPS, EX>), grid, dim3(256), lds, st, (u16*)out, ldo, q, *kv, \
                        proj, ld, gate_col, bias, n_dist, seq_slot, seq_row0, seq_pos0, seq_len, H, G, D, E, window, scale, \
                        out_scale, softcap, form);                                                                          \
   } while (0)
 #define BSA_MFMA_SHAPE()                                                                                                   \
-  if (maps == 2) { if (D <= 128 && E <= 128) BSA_MFMA(4, 8, 2, 2); else BSA_MFMA(8, 16, 2, 2); }                           \
-  else if (D <= 64 && E <= 64) { if (hpg > 4) BSA_MFMA(2, 4, 2, 1); else BSA_MFMA(2, 4, 1, 1); }                           \
-  else if (D <= 128 && E <= 128) { if (hpg > 4) BSA_MFMA(4, 8, 2, 1); else BSA_MFMA(4, 8, 1, 1); }                         \
-  else BSA_MFMA(8, 16, 1, 1)
+  if (maps == 2) {                                                                                                         \
+    if (D == 64 && E == 128) BSA_MFMA(2, 8, 2, 2, true);                                                                   \
+    else if (D == 128 && E == 256) BSA_MFMA(4, 16, 2, 2, true);                                                            \
+    else if (D <= 128 && E <= 128) BSA_MFMA(4, 8, 2, 2, false);                                                            \
+    else BSA_MFMA(8, 16, 2, 2, false);                                                                                     \
+  } else if (D == 64 && E == 64) { if (hpg > 4) BSA_MFMA(2, 4, 2, 1, true); else BSA_MFMA(2, 4, 1, 1, true); }             \
+  else if (D == 128 && E == 128) { if (hpg > 4) BSA_MFMA(4, 8, 2, 1, true); else BSA_MFMA(4, 8, 1, 1, true); }             \
+  else if (D <= 64 && E <= 64) BSA_MFMA(2, 4, 1, 1, false);                                                                \
+  else if (D <= 128 && E <= 128) BSA_MFMA(4, 8, 1, 1, false);                                                              \
+  else BSA_MFMA(8, 16, 1, 1, false)
   if (dtype == UMB_SEQ_BF16) { using P = BF16; BSA_MFMA_SHAPE(); }
   else { using P = F16; BSA_MFMA_SHAPE(); }
 #undef BSA_MFMA_SHAPE

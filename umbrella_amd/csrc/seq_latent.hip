@@ -332,16 +332,19 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_kernel(typename El<P>::typ
 //   O^T += V^T P^T: the lane's eight weights ARE its share of the B operand when V^T's k index runs over (tile 0: 4g .. 4g+3,
 //         tile 1: 4g .. 4g+3); V^T (A: 16 features x those 8 keys) is gathered from the LDS tile.
 // The sink joins the denominator at the end.  NSM / NVM bound the unrolled register arrays (key steps of 32 features, value
-// tiles of 16 features); the actual counts are run-time.
-template <typename P, int NSM, int NVM, int HPW>
-__global__ __launch_bounds__(256) void lat_attend_mfma_kernel(u16* __restrict__ out, const float* __restrict__ qa, UmbPagedKV kv,
+// tiles of 16 features); EXACT: they are the counts.  With run-time counts every product stood in a block of its own behind its own LDS
+// read, and the step was that latency sixty times over: 1999 positions, 32 heads, kv_rank 512 + 64: 932 us, exact 526, eight waves on a
+// staged tile instead of four (two a SIMD; they spill 18 registers) 410.
+template <typename P, int NSM, int NVM, int HPW, int NW, bool EXACT>
+__global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restrict__ out, const float* __restrict__ qa, UmbPagedKV kv,
                                                               const u16* __restrict__ sink, const int* __restrict__ seq_slot,
                                                               const int* __restrict__ seq_row0, const int* __restrict__ seq_pos0,
                                                               const int* __restrict__ seq_len, int H, int Dc, int R, int window,
                                                               float scale) {
   extern __shared__ __attribute__((aligned(16))) u16 lat_lds[];
-  constexpr int NLD = (NSM + 1) / 2;                  // 16-byte chunks of a row per staging thread: Dk / 8 chunks over 8 threads
+  constexpr int SR = 2 * NW, NLD = (4 * NSM + SR - 1) / SR;           // staging threads per row, 16-byte chunks of the row for each
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
+  if constexpr (EXACT) { Dc = NVM * 16; R = NSM * 32 - Dc; }          // the counts as constants
   const int Dk = Dc + R, LD = Dk + 8;                 // LDS row stride: 16 bytes of padding spread the key quads over the banks
   const int ns = (Dk + 31) >> 5, nv = Dc >> 4, nch = Dk >> 3;
   constexpr int LT = 36;                              // row stride of the transposed tile: 32 keys + 8 bytes of padding
@@ -350,7 +353,7 @@ __global__ __launch_bounds__(256) void lat_attend_mfma_kernel(u16* __restrict__ 
   const int b = blockIdx.y;
   const int n = seq_len[b], q0 = blockIdx.x * 16;
   if (q0 >= n) return;                                // the whole workgroup
-  const int h0 = (blockIdx.z * 4 + wave) * HPW;
+  const int h0 = (blockIdx.z * NW + wave) * HPW;
   const bool active = h0 < H;                         // a wave without heads still stages rows and meets the barriers
   const int slot = seq_slot[b], row0 = seq_row0[b], pos0 = seq_pos0[b];
   const int nq = n - q0 < 16 ? n - q0 : 16;
@@ -384,7 +387,7 @@ __global__ __launch_bounds__(256) void lat_attend_mfma_kernel(u16* __restrict__ 
     m_run[hh] = -INFINITY;
     l_run[hh] = 0.f;
   }
-  // staging role of a thread: key row sm of the step, 16-byte chunks sc, sc + 8, ... of that row
+  // staging role of a thread: key row sm of the step, 16-byte chunks sc, sc + SR, ... of that row
   const int sm = threadIdx.x & 31, sc = threadIdx.x >> 5;
   u32x4 stage[NLD];
   auto fetch = [&](int base) {
@@ -392,16 +395,17 @@ __global__ __launch_bounds__(256) void lat_attend_mfma_kernel(u16* __restrict__ 
     const long off = kx < total ? pkv_tok(kv, slot, j_lo + kx, 0, 1, Dk) : -1;
 #pragma unroll
     for (int u = 0; u < NLD; ++u) {
-      const int ch = sc + 8 * u;
+      const int ch = sc + SR * u;
       stage[u] = (off >= 0 && ch < nch) ? *reinterpret_cast<const u32x4*>(kbase + off + 8 * ch) : u32x4{0u, 0u, 0u, 0u};
     }
   };
   fetch(0);
+  if (threadIdx.x < 32) *reinterpret_cast<u32x4*>(v_s + threadIdx.x * LD + Dk) = u32x4{0u, 0u, 0u, 0u};       // read where a step of 32 runs past Dk
   for (int base = 0; base < total; base += 32) {
     __syncthreads();                                  // every wave is done with the previous tile
 #pragma unroll
     for (int u = 0; u < NLD; ++u) {
-      const int ch = sc + 8 * u;
+      const int ch = sc + SR * u;
       if (ch < nch) {
         *reinterpret_cast<u32x4*>(v_s + sm * LD + 8 * ch) = stage[u];
         if (8 * ch < Dc) {                            // Dc is a multiple of 16: a chunk is all values or all rotated key part
@@ -426,29 +430,30 @@ __global__ __launch_bounds__(256) void lat_attend_mfma_kernel(u16* __restrict__ 
       for (int s = 0; s < NSM; ++s) {
         const int d = 32 * s + 8 * g4;
         if (s < ns) {
-          const u32x4 kf = d < Dk ? *reinterpret_cast<const u32x4*>(kr + d) : u32x4{0u, 0u, 0u, 0u};
+          const u32x4 kf = *reinterpret_cast<const u32x4*>(kr + (d < Dk ? d : Dk));
 #pragma unroll
           for (int hh = 0; hh < HPW; ++hh) sc2[hh][u] = P::mfma(kf, qf[hh][s], sc2[hh][u]);
         }
       }
     }
-    // which of the lane's eight keys this query sees: the same for every head
-    bool vis[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int jt = j_lo + base + 16 * (e >> 2) + 4 * g4 + (e & 3);
-      vis[e] = q_ok && jt <= i_j && jt > i_j - window;
-    }
+    // a step that every query sees whole needs no tests (rows past the last are not stored)
+    const bool whole = j_lo + base + 31 <= i_first && j_lo + base > i_last - window;
     u32x4 pf[HPW];
 #pragma unroll
     for (int hh = 0; hh < HPW; ++hh) {
       // maxima and exponents in base 2 (scale2 = scale log2 e): one v_exp_f32 per weight
       float sv[8], mx = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        sv[e] = vis[e] ? sc2[hh][e >> 2][e & 3] * scale2 : -INFINITY;
-        mx = fmaxf(mx, sv[e]);
+      for (int e = 0; e < 8; ++e) sv[e] = sc2[hh][e >> 2][e & 3] * scale2;
+      if (!whole) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int jt = j_lo + base + 16 * (e >> 2) + 4 * g4 + (e & 3);
+          sv[e] = q_ok && jt <= i_j && jt > i_j - window ? sv[e] : -INFINITY;
+        }
       }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sv[e]);
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float m_new = fmaxf(m_run[hh], mx);
@@ -511,13 +516,14 @@ __global__ __launch_bounds__(256) void lat_attend_mfma_kernel(u16* __restrict__ 
 // block of 16 heads); its four waves take the 32-key steps w, w + 4, ... of the window (which step lands in which wave depends
 // on the token's position alone) with the same step body as the prompt kernel, then merge their running maxima, sums and
 // partial outputs through LDS in wave order, where the sink joins the denominator.
-template <typename P, int NSM, int NVM>
+template <typename P, int NSM, int NVM, bool EXACT>
 __global__ __launch_bounds__(256) void lat_decode_mfma_kernel(u16* __restrict__ out, const float* __restrict__ qa, UmbPagedKV kv,
                                                               const u16* __restrict__ sink, const int* __restrict__ pos,
                                                               const int* __restrict__ slot_, int H, int Dc, int R, int window,
                                                               float scale) {
   extern __shared__ __attribute__((aligned(16))) u16 lat_lds[];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
+  if constexpr (EXACT) { Dc = NVM * 16; R = NSM * 32 - Dc; }          // the counts as constants
   const int Dk = Dc + R, LD = Dc + 8;
   const int ns = (Dk + 31) >> 5, nv = Dc >> 4;
   u16* v_s = lat_lds + (long)wave * (32 * LD + 32 * 4);
@@ -685,17 +691,19 @@ extern "C" int umb_lat_attend_tiled(void* out, const float* qa, const UmbPagedKV
     return UMB_EINVAL;
   const int Dk = kv_rank + rot_dim;
   const size_t lds = ((size_t)32 * (Dk + 8) + (size_t)kv_rank * 36) * sizeof(u16);
-#define LAT_MFMA(NSM, NVM, HPW)                                                                                            \
+#define LAT_MFMA(NSM, NVM, HPW, NW, EX)                                                                                      \
   do {                                                                                                                     \
-    const dim3 grid((max_len + 15) / 16, B, (H + 4 * HPW - 1) / (4 * HPW));                                                \
-    if (ensure_dynamic_lds<lat_attend_mfma_kernel<P, NSM, NVM, HPW>>(lds) != UMB_OK) return UMB_EHIP;                      \
-    hipLaunchKernelGGL((lat_attend_mfma_kernel<P, NSM, NVM, HPW>), grid, dim3(256), lds, st, (u16*)out, qa, *kv,           \
+    const dim3 grid((max_len + 15) / 16, B, (H + NW * HPW - 1) / (NW * HPW));                                              \
+    if (ensure_dynamic_lds<lat_attend_mfma_kernel<P, NSM, NVM, HPW, NW, EX>>(lds) != UMB_OK) return UMB_EHIP;                  \
+    hipLaunchKernelGGL((lat_attend_mfma_kernel<P, NSM, NVM, HPW, NW, EX>), grid, dim3(NW * 64), lds, st, (u16*)out, qa, *kv,   \
                        (const u16*)sink, seq_slot, seq_row0, seq_pos0, seq_len, H, kv_rank, rot_dim, window, scale);       \
   } while (0)
 #define LAT_MFMA_SHAPE()                                                                                                   \
-  if (Dk <= 128 && kv_rank <= 128) { if (H >= 8) LAT_MFMA(4, 8, 2); else LAT_MFMA(4, 8, 1); }                              \
-  else if (Dk <= 320 && kv_rank <= 256) LAT_MFMA(10, 16, 1);   /* two heads a wave spill to AGPRs here: measured slower */ \
-  else LAT_MFMA(18, 32, 1)
+  if (H > 4 && Dk == 576 && kv_rank == 512) LAT_MFMA(18, 32, 1, 8, true);                                                  \
+  else if (H > 4 && Dk == 288 && kv_rank == 256) LAT_MFMA(9, 16, 1, 8, true);                                              \
+  else if (Dk <= 128 && kv_rank <= 128) { if (H >= 8) LAT_MFMA(4, 8, 2, 4, false); else LAT_MFMA(4, 8, 1, 4, false); }     \
+  else if (Dk <= 320 && kv_rank <= 256) LAT_MFMA(10, 16, 1, 4, false);                                                           \
+  else LAT_MFMA(18, 32, 1, 4, false)
   if (dtype == UMB_SEQ_BF16) { using P = BF16; LAT_MFMA_SHAPE(); }
   else { using P = F16; LAT_MFMA_SHAPE(); }
 #undef LAT_MFMA_SHAPE
@@ -769,14 +777,15 @@ extern "C" int umb_lat_attend(void* out, const float* qa, const UmbPagedKV* kv, 
     const size_t parts = (size_t)4 * (kv_rank / 16) * 64 * sizeof(f32x4) + 4 * 16 * 2 * sizeof(float);
     const size_t lds = tiles > parts ? tiles : parts;
     const dim3 grid(T, (H + 15) / 16);
-#define LAT_DEC(NSM, NVM)                                                                                                  \
+#define LAT_DEC(NSM, NVM, EX)                                                                                              \
   do {                                                                                                                     \
-    if (ensure_dynamic_lds<lat_decode_mfma_kernel<P, NSM, NVM>>(lds) != UMB_OK) return UMB_EHIP;                           \
-    hipLaunchKernelGGL((lat_decode_mfma_kernel<P, NSM, NVM>), grid, dim3(256), lds, st, (u16*)out, qa, *kv,                \
+    if (ensure_dynamic_lds<lat_decode_mfma_kernel<P, NSM, NVM, EX>>(lds) != UMB_OK) return UMB_EHIP;                           \
+    hipLaunchKernelGGL((lat_decode_mfma_kernel<P, NSM, NVM, EX>), grid, dim3(256), lds, st, (u16*)out, qa, *kv,                \
                        (const u16*)sink, pos, slot, H, kv_rank, rot_dim, window, scale);                                   \
   } while (0)
 #define LAT_DEC_SHAPE()                                                                                                    \
-  if (Dk <= 128 && kv_rank <= 128) LAT_DEC(4, 8); else if (Dk <= 320 && kv_rank <= 256) LAT_DEC(10, 16); else LAT_DEC(18, 32)
+  if (Dk == 576 && kv_rank == 512) LAT_DEC(18, 32, true); else if (Dk == 288 && kv_rank == 256) LAT_DEC(9, 16, true);       \
+  else if (Dk <= 128 && kv_rank <= 128) LAT_DEC(4, 8, false); else if (Dk <= 320 && kv_rank <= 256) LAT_DEC(10, 16, false); else LAT_DEC(18, 32, false)
     if (dtype == UMB_SEQ_BF16) { using P = BF16; LAT_DEC_SHAPE(); }
     else { using P = F16; LAT_DEC_SHAPE(); }
 #undef LAT_DEC_SHAPE

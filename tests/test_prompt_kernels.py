@@ -441,3 +441,139 @@ def test_split_reduce_and_rotation_of_many_tokens_is_that_of_few(dtype, T, Hq, H
                 else:       # x / rms + bias may be one fp32 rounding or two: then each of the rotation's two products may round the other way
                     eps = torch.finfo(dtype).eps
                     assert bool(((x.float() - y.float()).abs() <= 4 * eps * y.float().abs().max()).all()) and (x != y).float().mean() < 1e-2
+
+
+def _stretches(lens, news):
+    """rows of a step that brings the last news[b] of lens[b] positions of every sequence"""
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                                    # noqa: E731
+    row0 = [sum(news[:b]) for b in range(len(news))]
+    return i32(row0), i32([n - k for n, k in zip(lens, news)]), i32(news), sum(news)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,E,maps,window,chunk,keep,extra", [
+    (8, 2, 64, 64, 1, 2 ** 30, 0, 0, False), (6, 1, 64, 64, 1, 70, 0, 5, True), (4, 1, 128, 128, 1, 90, 0, 40, True), (12, 2, 128, 128, 1, 2 ** 30, 64, 0, False),
+    (4, 2, 64, 128, 2, 2 ** 30, 50, 0, False), (2, 1, 128, 256, 2, 100, 0, 3, True), (3, 1, 72, 48, 1, 60, 0, 0, True)])
+def test_prompt_attention(dtype, H, G, D, E, maps, window, chunk, keep, extra):
+    from umbrella_amd import _lib
+    code = _lib.seq_dtype_code(dtype)
+    lens, news = [16, 33, 250, 95], [16, 17, 250, 30]
+    c, _, slot, g = _decode_store(lens, G, maps * D, E, 0, dtype, 16, H + D + E)
+    row0, pos0, cnt, T = _stretches(lens, news)
+    nd = 40
+    q = torch.randn(T, H, maps, D, generator=g, device="cuda")
+    gate = torch.randn(T, H, generator=g, device="cuda") if extra else None
+    sink = torch.randn(H, generator=g, device="cuda") if extra else None
+    bias = torch.randn(H, nd, generator=g, device="cuda") if extra else None
+    cap, lam, eps, scale = (6.0 if extra else 0.0), 0.3, 1e-3, D ** -0.5
+    form = _lib.UmbAttnForm(maps, chunk, sink.data_ptr() if extra else None, lam, eps, keep, 0)
+    out = torch.full((T + 1, H * E + 8), 3.0, dtype=dtype, device="cuda")
+    _lib.seq_call("umb_attn_attend_tiled", out, H * E + 8, q, c.struct(0), gate, H if extra else 0, 0 if extra else -1, bias, nd if extra else 0, slot, row0,
+                  pos0, cnt, len(lens), max(news), H, G, D, E, window, scale, 1.25, cap, form, code)
+    assert bool((out[:, H * E:] == 3.0).all()) and bool((out[T] == 3.0).all())
+    for b, (n, k) in enumerate(zip(lens, news)):
+        kk, vv = (z.double() for z in c.token_rows(0, b, torch.arange(n)))
+        kk = kk.view(n, G, maps, D).repeat_interleave(H // G, 1)
+        vv = vv.repeat_interleave(H // G, 1)
+        r0 = int(row0[b])
+        i, j = torch.arange(n - k, n, device="cuda")[:, None], torch.arange(n, device="cuda")[None]
+        see = i - j < window
+        if chunk:
+            see &= j // chunk == i // chunk
+        see = (see | (j < keep)) & (j <= i)
+        s = torch.einsum("thmd,jhmd->thmj", q[r0:r0 + k].double().cpu(), kk.cpu()).cuda() * scale
+        if cap:
+            s = cap * torch.tanh(s / cap)
+        if extra:
+            s = s + bias.double()[:, (i - j).clamp(0, nd - 1)].permute(1, 0, 2)[:, :, None]
+        s = s.masked_fill(~see[:, None, None], float("-inf"))
+        if extra:
+            p = torch.softmax(torch.cat([s, sink.double()[None, :, None, None].expand(k, H, maps, 1)], -1), -1)[..., :-1]
+        else:
+            p = torch.softmax(s, -1)
+        o = torch.einsum("thmj,jhe->thme", p.cpu(), vv.cpu()).cuda()
+        if maps == 2:
+            o = o[:, :, 0] - lam * o[:, :, 1]
+            o = o / torch.sqrt(o.pow(2).mean(-1, keepdim=True) + eps)
+        else:
+            o = o[:, :, 0]
+        o = 1.25 * o * (torch.sigmoid(gate[r0:r0 + k].double())[..., None] if extra else 1.0)
+        # storage rounding; queries and weights split to 2^-17 each (bf16; 2^-22 in fp16), scores of up to 7: 1e-4 of the largest output
+        tol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * o.abs() + 2e-4 * o.abs().max() + 1e-6
+        err = (out[r0:r0 + k, :H * E].double().view(k, H, E) - o).abs()
+        assert bool((err <= tol).all()), (b, float(err.max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,window,pool", [(8, 2, 64, 40, 16), (5, 1, 32, 2 ** 20, 4), (4, 2, 128, 17, 3), (6, 1, 96, 64, 1), (2, 1, 256, 33, 7)])
+def test_prompt_pooled_attention(dtype, H, G, D, window, pool):
+    from umbrella_amd import _lib
+    code = _lib.seq_dtype_code(dtype)
+    lens, news = [16, 33, 250, 95], [16, 17, 250, 30]
+    c, _, slot, g = _decode_store(lens, G, D, D, pool, dtype, 32, H + D + pool)
+    row0, pos0, cnt, T = _stretches(lens, news)
+    q, gate = torch.randn(T, H, D, generator=g, device="cuda"), torch.randn(T, H, generator=g, device="cuda")
+    pb = torch.randn(H, generator=g, device="cuda").to(dtype)
+    out = torch.full((T + 1, H * D), 3.0, dtype=dtype, device="cuda")
+    _lib.seq_call("umb_pwa_attend_tiled", out, q, c.struct(0), gate, H, 0, pb, slot, row0, pos0, cnt, len(lens), max(news), H, G, D, window, pool, D ** -0.5,
+                  code)
+    assert bool((out[T] == 3.0).all())
+    for b, (n, k) in enumerate(zip(lens, news)):
+        nb = max(n - window, 0) // pool
+        kk, vv = (z.double() for z in c.token_rows(0, b, torch.arange(n)))
+        if nb:
+            kp, vp = (z.double() for z in c.pooled_rows(0, b, torch.arange(nb)))
+            kk, vv = torch.cat([kp, kk]), torch.cat([vp, vv])
+        kk, vv = kk.repeat_interleave(H // G, 1).cpu(), vv.repeat_interleave(H // G, 1).cpu()
+        r0 = int(row0[b])
+        i, j = torch.arange(n - k, n)[:, None], torch.arange(n)[None]
+        see = torch.cat([torch.arange(nb)[None] * pool + pool - 1 <= i - window, (j <= i) & (i - j < window)], 1)
+        s = torch.einsum("thd,jhd->thj", q[r0:r0 + k].double().cpu(), kk) * D ** -0.5
+        w = torch.sigmoid(s + pb.double().cpu()[None, :, None]) * see[:, None]
+        gt = torch.sigmoid(gate[r0:r0 + k].double().cpu())[..., None]
+        o, size = torch.einsum("thj,jhd->thd", w, vv) * gt, (torch.einsum("thj,jhd->thd", w, vv.abs()) * gt).max()
+        # storage rounding; queries, pooled rows and weights split to 2^-17 each (bf16), scores of up to 7: 3e-5 of the sum of sizes
+        tol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * o.abs() + 3e-5 * size + 1e-6
+        err = (out[r0:r0 + k].double().cpu().view(k, H, D) - o).abs()
+        assert bool((err <= tol).all()), (b, float(err.max()), float(size))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,Dc,R,window", [(9, 512, 64, 70), (16, 256, 32, 2 ** 20), (8, 256, 64, 33), (4, 512, 64, 2 ** 20), (9, 64, 24, 50)])
+def test_latent_attention_of_prompts_and_of_many_tokens(dtype, H, Dc, R, window):
+    from umbrella_amd import _lib
+    from umbrella_amd.attn.cache import PagedSeqCache
+    code, Dk = _lib.seq_dtype_code(dtype), Dc + R
+    g = torch.Generator(device="cuda").manual_seed(H + Dc + R)
+
+    def case(lens, news, tiled):
+        c = PagedSeqCache([], [], sum(lens), len(lens), "cuda", dtype, page=16, latent_layers=(Dk,))
+        c.latent[0].copy_(torch.randn(c.latent[0].shape, generator=g, device="cuda"))
+        for b, n in enumerate(lens):
+            c.open(b), c.extend(b, n)
+        slot = torch.tensor([c.slot(b) for b in range(len(lens))], dtype=torch.int32, device="cuda")
+        row0, pos0, cnt, T = _stretches(lens, news)
+        qa, sink = torch.randn(T, H, Dk, generator=g, device="cuda"), torch.randn(H, generator=g, device="cuda").to(dtype)
+        out = torch.full((T + 1, H * Dc), 3.0, dtype=dtype, device="cuda")
+        scale = Dk ** -0.5
+        if tiled:
+            _lib.seq_call("umb_lat_attend_tiled", out, qa, c.latent_struct(0), sink, slot, row0, pos0, cnt, len(lens), max(news), H, Dc, R, window, scale, code)
+        else:
+            pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device="cuda")
+            _lib.seq_call("umb_lat_attend", out, qa, c.latent_struct(0), sink, pos, slot, T, H, Dc, R, window, scale, code)
+        assert bool((out[T] == 3.0).all())
+        for b, (n, k) in enumerate(zip(lens, news)):
+            r0 = int(row0[b])
+            rows = c.latent_rows(0, b, torch.arange(n)).double().cpu()
+            i, j = torch.arange(n - k, n)[:, None], torch.arange(n)[None]
+            x = qa[r0:r0 + k].to(dtype).double().cpu()                       # queries enter in the storage type
+            s = (torch.einsum("thd,jd->thj", x, rows) * scale).masked_fill(~((j <= i) & (i - j < window))[:, None], float("-inf"))
+            p = torch.softmax(torch.cat([s, sink.double().cpu()[None, :, None].expand(k, H, 1)], -1), -1)[..., :-1]
+            o = torch.einsum("thj,jd->thd", p, rows[:, :Dc])
+            # weights and the result are rounded to the storage type, each to half a step of its own size
+            u = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+            tol = u * o.abs() + u * torch.einsum("thj,jd->thd", p, rows[:, :Dc].abs()) + 1e-4 * o.abs().max()
+            err = (out[r0:r0 + k].double().cpu().view(k, H, Dc) - o).abs()
+            assert bool((err <= tol).all()), (b, float(err.max()))
+    case([16, 33, 250, 95], [16, 17, 250, 30], True)
+    case([1 + 3 * i for i in range(50)], [1] * 50, False)

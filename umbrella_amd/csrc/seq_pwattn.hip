@@ -448,16 +448,19 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
 }
 
 // ---- prompt attention on the matrix pipe (16-bit storage, D a multiple of 32).
-// Workgroup = (16 consecutive positions of one sequence, one key/value group); its four waves take the group's query heads.
-// Key list of the tile: pooled blocks 0 .. nb(last position) (padded to a multiple of 32), then the tokens from the first
-// position's window start to the last position; a 32-key step is all pooled or all tokens.  Per step and head:
-//   S^T = K Q^T as two 16-key MFMA tiles (A = 16 keys x 32 d straight from the cache rows, B = the queries);
-//   P = visible ? sigmoid(S scale + bias) : 0 in fp32, lane (query j, key quad g) holding keys 4g .. 4g+3 of both tiles --
-//   which IS the lane's share of the B operand of O^T += V^T P^T over the step's 32 keys when V^T's k index runs over
-//   (tile 0: 4g..4g+3, tile 1: 4g..4g+3): no data moves between the two products;
-//   V^T (A operand: 16 d x those 8 keys) is gathered from a [32 keys][D] copy of the value rows in LDS.
+// Workgroup = (16 consecutive positions of one sequence, one key/value group); its four waves take the group's query heads, each wave
+// every fourth one in turn.
+// Key list of the tile: pooled blocks 0 .. nb(last position), then the tokens from the first position's window start to the last
+// position, in steps of 32 keys.  A step is staged ONCE for the four waves: key rows as cached (the A operand of S^T = K Q^T), values
+// transposed (the A operand of O^T += V^T P^T); pooled rows, held in fp32, as high and low halves.  The next step's rows are in flight
+// in registers while this one is used.  Per step and head:
+//   S^T as two 16-key MFMA tiles; P = visible ? sigmoid(S scale + bias) : 0 in fp32, lane (query j, key quad g) holding keys 4g .. 4g+3
+//   of both tiles -- which IS the lane's share of the B operand of the value product.
 // Scores and weights stay fp32-exact on a bf16 / f16 matrix pipe by splitting the fp32 factor into a high and a low 16-bit
-// half (x = hi + lo to 2^-17): q, the pooled means (held in fp32) and the weights go through two MFMAs instead of one.
+// half (x = hi + lo to 2^-17): q, the pooled means (held in fp32) and the weights go through two MFMAs instead of one; the exponential and
+// the reciprocal of the sigmoid (one and two units in the last place, 2^-22) are far below that.
+// It is bound by the vector work between the products.  With every wave staging its own values, gathering them two bytes at a time and
+// testing every key: 38 vector instructions a matrix instruction and 129 us at 2048 positions, 32 + 8 heads of 64, window 512; now 45.
 template <typename P> __device__ __forceinline__ void split8(const float* v, u32x4& hi, u32x4& lo) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -473,15 +476,17 @@ __global__ __launch_bounds__(256) void pwa_attend_mfma_kernel(u16* __restrict__ 
                                                               const int* __restrict__ seq_row0, const int* __restrict__ seq_pos0,
                                                               const int* __restrict__ seq_len, int H, int G, int window, int pool,
                                                               float scale) {
-  constexpr int D = NS * 32, LD = D + 8;              // LDS row stride: 16 bytes of padding spread the key quads over the banks
-  extern __shared__ __attribute__((aligned(16))) u16 vt_all[];
+  constexpr int D = NS * 32, LD = D + 8, LT = 36, NL = (D + 63) / 64;   // row strides of the two tiles; 8-feature chunks of a row per thread
+  constexpr float L2E = 1.4426950408889634f;
+  extern __shared__ __attribute__((aligned(16))) u16 pwa_lds[];
+  u16* k_hi = pwa_lds;                                         // [32][LD]
+  u16* v_hi = k_hi + 32 * LD;                              // [D][LT]
+  u16* k_lo = v_hi + D * LT;                               // the low halves of pooled rows
+  u16* v_lo = k_lo + 32 * LD;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
-  u16* v_hi = vt_all + (long)wave * (2 * 32 * LD + 32 * 4);   // [32][LD] values, [32][LD] low halves (pooled steps), [32] offsets
-  u16* v_lo = v_hi + 32 * LD;
-  long* offs = reinterpret_cast<long*>(v_lo + 32 * LD);
   const int b = blockIdx.y, g = blockIdx.z;
   const int n = seq_len[b], q0 = blockIdx.x * 16;
-  if (q0 >= n) return;
+  if (q0 >= n) return;                                     // the whole workgroup
   const int slot = seq_slot[b], row0 = seq_row0[b], pos0 = seq_pos0[b];
   const int nq = n - q0 < 16 ? n - q0 : 16;
   const int i_first = pos0 + q0, i_last = i_first + nq - 1;
@@ -489,136 +494,164 @@ __global__ __launch_bounds__(256) void pwa_attend_mfma_kernel(u16* __restrict__ 
   const int i_j = i_first + (q_ok ? j : nq - 1);
   const long qrow = row0 + q0 + (q_ok ? j : nq - 1);
   const int nb_j = i_j - window + 1 >= pool ? (i_j - window + 1) / pool : 0;
+  const int nb_first = i_first - window + 1 >= pool ? (i_first - window + 1) / pool : 0;
   const int nb_max = i_last - window + 1 >= pool ? (i_last - window + 1) / pool : 0;
-  const int j_lo = i_first - window + 1 > 0 ? i_first - window + 1 : 0;
-  const int tok0 = (nb_max + 31) & ~31, total = tok0 + (i_last - j_lo + 1);
+  const int j_lo = i_first - window + 1 > 0 ? i_first - window + 1 : 0, n_tok = i_last - j_lo + 1;
   const int R = H / G;
-  for (int r = wave; r < R; r += 4) {
-    const int h = g * R + r;
+  const int sm = threadIdx.x & 31, sc = threadIdx.x >> 5;  // staging role: key row sm of the step, 8-feature chunks sc, sc + 8, ..
+  for (int r0 = 0; r0 < R; r0 += 4) {                      // a wave without a head still stages and meets the barriers
+    const bool active = r0 + wave < R;
+    const int h = g * R + (active ? r0 + wave : R - 1);
     u32x4 qhi[NS], qlo[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       float v[8];
-      const f32x4 a = *reinterpret_cast<const f32x4*>(q + qrow * H * D + (long)h * D + 32 * s + 8 * g4);
-      const f32x4 c = *reinterpret_cast<const f32x4*>(q + qrow * H * D + (long)h * D + 32 * s + 8 * g4 + 4);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(q + qrow * H * D + (long)h * D + 32 * s + 8 * g4);
+      const f32x4 y = *reinterpret_cast<const f32x4*>(q + qrow * H * D + (long)h * D + 32 * s + 8 * g4 + 4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = c[e]; }
+      for (int e = 0; e < 4; ++e) { v[e] = x[e]; v[4 + e] = y[e]; }
       split8<P>(v, qhi[s], qlo[s]);
     }
     const float bias = pos_bias ? P::to_f(pos_bias[h]) : 0.f;
     f32x4 o[2 * NS];
 #pragma unroll
     for (int dt = 0; dt < 2 * NS; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int base = 0; base < total; base += 32) {
-      const bool pooled = base < tok0;
-      // element offsets of the step's 32 keys (-1: no such key)
-      if (lane < 32) {
-        const int kx = base + lane;
-        long off = -1;
-        if (pooled) { if (kx < nb_max) off = pkv_blk(kv, slot, kx, pool, g, G, D); }
-        else if (kx < total) off = pkv_tok(kv, slot, j_lo + (kx - tok0), g, G, D);
-        offs[lane] = off;
+    auto put = [&](u16* ks, u16* vt, int ch, u32x4 kk, u32x4 vv) {
+      *reinterpret_cast<u32x4*>(ks + sm * LD + 8 * ch) = kk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        vt[(8 * ch + 2 * e) * LT + sm] = (u16)(vv[e] & 0xffffu);
+        vt[(8 * ch + 2 * e + 1) * LT + sm] = (u16)(vv[e] >> 16);
       }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      // value rows -> LDS: 32 x D / 8 pieces of 8 features, NS pieces... (4 D / 64 = 2 NS per lane)
-#pragma unroll
-      for (int i = 0; i < 2 * NS; ++i) {
-        const int p = lane + 64 * i, m = p / (D / 8), dp = (p % (D / 8)) * 8;
-        const long off = offs[m];
-        u32x4 hi = u32x4{0u, 0u, 0u, 0u}, lo = u32x4{0u, 0u, 0u, 0u};
-        if (off >= 0) {
-          if (pooled) {
-            float v[8];
-            const f32x4 a = *reinterpret_cast<const f32x4*>(kv.vp + off + dp);
-            const f32x4 c = *reinterpret_cast<const f32x4*>(kv.vp + off + dp + 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = c[e]; }
-            split8<P>(v, hi, lo);
-          } else {
-            hi = *reinterpret_cast<const u32x4*>(reinterpret_cast<const u16*>(kv.v) + off + dp);
-          }
-        }
-        *reinterpret_cast<u32x4*>(v_hi + m * LD + dp) = hi;
-        if (pooled) *reinterpret_cast<u32x4*>(v_lo + m * LD + dp) = lo;
-      }
-      // scores of the two 16-key tiles
-      f32x4 sc[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        sc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const long off = offs[16 * u + j];
-        const long offc = off >= 0 ? off : 0;
-        if (pooled) {
-#pragma unroll
-          for (int s = 0; s < NS; ++s) {
-            float v[8];
-            const f32x4 a = *reinterpret_cast<const f32x4*>(kv.kp + offc + 32 * s + 8 * g4);
-            const f32x4 c = *reinterpret_cast<const f32x4*>(kv.kp + offc + 32 * s + 8 * g4 + 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = c[e]; }
-            u32x4 khi, klo;
-            split8<P>(v, khi, klo);
-            sc[u] = P::mfma(khi, qhi[s], sc[u]);
-            sc[u] = P::mfma(khi, qlo[s], sc[u]);
-            sc[u] = P::mfma(klo, qhi[s], sc[u]);
-          }
-        } else {
-          u32x4 kf[NS];
-#pragma unroll
-          for (int s = 0; s < NS; ++s)
-            kf[s] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const u16*>(kv.k) + offc + 32 * s + 8 * g4);
-#pragma unroll
-          for (int s = 0; s < NS; ++s) {
-            sc[u] = P::mfma(kf[s], qhi[s], sc[u]);
-            sc[u] = P::mfma(kf[s], qlo[s], sc[u]);
-          }
-        }
-      }
-      // weights: lane (query j, quad g4) holds keys 16 u + 4 g4 + r of the step
+    };
+    auto key_tile = [&](const u16* ks, int u, int s) { return *reinterpret_cast<const u32x4*>(ks + (16 * u + j) * LD + 32 * s + 8 * g4); };
+    auto value_tile = [&](const u16* vt, int dt) {
+      const u16* vr = vt + (16 * dt + j) * LT + 4 * g4;
+      const u32x2 t0 = *reinterpret_cast<const u32x2*>(vr), t1 = *reinterpret_cast<const u32x2*>(vr + 16);
+      return u32x4{t0[0], t0[1], t1[0], t1[1]};
+    };
+    // whole: every key of the step is seen by every query (rows past the last are not stored); else lane's key 16 u + 4 g4 + rr by `sees`
+    auto weights = [&](f32x4 (&s2)[2], bool whole, auto sees, u32x4& hi, u32x4& lo) {
       float w[8];
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int e = 0; e < 8; ++e) w[e] = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(s2[e >> 2][e & 3] * scale + bias) * L2E));
+      if (!whole) {
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int kk = base + 16 * u + 4 * g4 + rr;
-          bool vis;
-          if (pooled) vis = kk < nb_j;
-          else { const int jt = j_lo + (kk - tok0); vis = jt <= i_j && jt > i_j - window; }
-          w[4 * u + rr] = (vis && q_ok) ? 1.f / (1.f + expf(-(sc[u][rr] * scale + bias))) : 0.f;
-        }
-      u32x4 phi, plo;
-      split8<P>(w, phi, plo);
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      // O^T[d][query] += V^T[d][keys] P^T[keys][query]: lane (d row j of tile dt, quad g4) gathers its 8 keys' values
+        for (int e = 0; e < 8; ++e) w[e] = q_ok && sees(16 * (e >> 2) + 4 * g4 + (e & 3)) ? w[e] : 0.f;
+      }
+      split8<P>(w, hi, lo);
+    };
+
+    // ---- pooled blocks: fp32 rows
+    f32x4 pk[NL][2], pv[NL][2];
+    auto fetch_pooled = [&](int base) {
+      const long off = (long)pkv_blk_row(kv, slot, min(base + sm, nb_max - 1), pool, g, G) * D;
 #pragma unroll
-      for (int dt = 0; dt < 2 * NS; ++dt) {
-        unsigned e[8];
-#pragma unroll
-        for (int m = 0; m < 8; ++m) e[m] = v_hi[((m >> 2) * 16 + 4 * g4 + (m & 3)) * LD + 16 * dt + j];
-        const u32x4 va = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-        o[dt] = P::mfma(va, phi, o[dt]);
-        o[dt] = P::mfma(va, plo, o[dt]);
-        if (pooled) {
-#pragma unroll
-          for (int m = 0; m < 8; ++m) e[m] = v_lo[((m >> 2) * 16 + 4 * g4 + (m & 3)) * LD + 16 * dt + j];
-          const u32x4 vl = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-          o[dt] = P::mfma(vl, phi, o[dt]);
+      for (int u = 0; u < NL; ++u) {
+        const int ch = sc + 8 * u;
+        if (D % 64 == 0 || ch < D / 8) {
+          pk[u][0] = *reinterpret_cast<const f32x4*>(kv.kp + off + 8 * ch);
+          pk[u][1] = *reinterpret_cast<const f32x4*>(kv.kp + off + 8 * ch + 4);
+          pv[u][0] = *reinterpret_cast<const f32x4*>(kv.vp + off + 8 * ch);
+          pv[u][1] = *reinterpret_cast<const f32x4*>(kv.vp + off + 8 * ch + 4);
         }
       }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+    };
+    if (nb_max > 0) fetch_pooled(0);
+    for (int base = 0; base < nb_max; base += 32) {
+      __syncthreads();                                     // every wave is done with the previous tile
+#pragma unroll
+      for (int u = 0; u < NL; ++u) {
+        const int ch = sc + 8 * u;
+        if (D % 64 == 0 || ch < D / 8) {
+          u32x4 kh, kl, vh, vl;
+          float t[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[e] = pk[u][e >> 2][e & 3];
+          split8<P>(t, kh, kl);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[e] = pv[u][e >> 2][e & 3];
+          split8<P>(t, vh, vl);
+          put(k_hi, v_hi, ch, kh, vh);
+          put(k_lo, v_lo, ch, kl, vl);
+        }
+      }
+      __syncthreads();
+      if (base + 32 < nb_max) fetch_pooled(base + 32);
+      if (!active) continue;
+      f32x4 s2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const u32x4 kh = key_tile(k_hi, u, s);
+          s2[u] = P::mfma(kh, qlo[s], s2[u]);
+          s2[u] = P::mfma(key_tile(k_lo, u, s), qhi[s], s2[u]);
+          s2[u] = P::mfma(kh, qhi[s], s2[u]);
+        }
+      u32x4 phi, plo;
+      weights(s2, base + 32 <= nb_first, [&](int k) { return base + k < nb_j; }, phi, plo);
+#pragma unroll
+      for (int dt = 0; dt < 2 * NS; ++dt) {
+        const u32x4 vh = value_tile(v_hi, dt);
+        o[dt] = P::mfma(vh, plo, o[dt]);
+        o[dt] = P::mfma(value_tile(v_lo, dt), phi, o[dt]);
+        o[dt] = P::mfma(vh, phi, o[dt]);
+      }
+    }
+
+    // ---- tokens
+    u32x4 tk[NL], tv[NL];
+    auto fetch_tokens = [&](int base) {
+      const long off = (long)pkv_tok_row(kv, slot, j_lo + min(base + sm, n_tok - 1), g, G) * D;
+#pragma unroll
+      for (int u = 0; u < NL; ++u) {
+        const int ch = sc + 8 * u;
+        if (D % 64 == 0 || ch < D / 8) {
+          tk[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const u16*>(kv.k) + off + 8 * ch);
+          tv[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const u16*>(kv.v) + off + 8 * ch);
+        }
+      }
+    };
+    fetch_tokens(0);
+    for (int base = 0; base < n_tok; base += 32) {
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < NL; ++u) {
+        const int ch = sc + 8 * u;
+        if (D % 64 == 0 || ch < D / 8) put(k_hi, v_hi, ch, tk[u], tv[u]);
+      }
+      __syncthreads();
+      if (base + 32 < n_tok) fetch_tokens(base + 32);
+      if (!active) continue;
+      f32x4 s2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const u32x4 kh = key_tile(k_hi, u, s);
+          s2[u] = P::mfma(kh, qlo[s], s2[u]);
+          s2[u] = P::mfma(kh, qhi[s], s2[u]);
+        }
+      const int jt = j_lo + base;
+      u32x4 phi, plo;
+      weights(s2, jt + 31 <= i_first && jt > i_last - window, [&](int k) { return jt + k <= i_j && jt + k > i_j - window; }, phi, plo);
+#pragma unroll
+      for (int dt = 0; dt < 2 * NS; ++dt) {
+        const u32x4 vh = value_tile(v_hi, dt);
+        o[dt] = P::mfma(vh, plo, o[dt]);
+        o[dt] = P::mfma(vh, phi, o[dt]);
+      }
     }
     // lane holds O^T[d = 16 dt + 4 g4 + rr][query j]
-    if (q_ok) {
+    if (q_ok && active) {
       const float gate = 1.f / (1.f + expf(-proj[qrow * ld + gate_col + h]));
 #pragma unroll
       for (int dt = 0; dt < 2 * NS; ++dt) {
-        u32x2 pk;
-        pk[0] = pack2<P>(o[dt][0] * gate, o[dt][1] * gate);
-        pk[1] = pack2<P>(o[dt][2] * gate, o[dt][3] * gate);
-        *reinterpret_cast<u32x2*>(out + qrow * H * D + (long)h * D + 16 * dt + 4 * g4) = pk;
+        u32x2 pk2;
+        pk2[0] = pack2<P>(o[dt][0] * gate, o[dt][1] * gate);
+        pk2[1] = pack2<P>(o[dt][2] * gate, o[dt][3] * gate);
+        *reinterpret_cast<u32x2*>(out + qrow * H * D + (long)h * D + 16 * dt + 4 * g4) = pk2;
       }
     }
   }
@@ -723,7 +756,7 @@ extern "C" int umb_pwa_attend_tiled(void* out, const float* q, const UmbPagedKV*
       !pkv_ok(kv) || !proj || !seq_slot || !seq_row0 || !seq_pos0 || !seq_len || dtype == UMB_SEQ_F32)
     return UMB_EINVAL;
   const dim3 grid((max_len + 15) / 16, B, G);
-  const size_t lds = 4 * (size_t)(2 * 32 * (D + 8) + 128) * sizeof(u16);
+  const size_t lds = 2 * ((size_t)32 * (D + 8) + (size_t)D * 36) * sizeof(u16);
 #define PWA_MFMA_CASE(NS)                                                                                                  \
   case NS:                                                                                                                 \
     if (ensure_dynamic_lds<pwa_attend_mfma_kernel<P, NS>>(lds) != UMB_OK) return UMB_EHIP;                                 \

@@ -577,3 +577,59 @@ def test_latent_attention_of_prompts_and_of_many_tokens(dtype, H, Dc, R, window)
             assert bool((err <= tol).all()), (b, float(err.max()))
     case([16, 33, 250, 95], [16, 17, 250, 30], True)
     case([1 + 3 * i for i in range(50)], [1] * 50, False)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("H,G,D,E,maps,layout,rot,append,norm,mixed", [(8, 2, 64, 64, 1, 0, 64, 1, 1, True), (3, 1, 128, 96, 2, 1, 80, 1, 0, False),
+                                                                       (7, 7, 24, 128, 1, 1, 0, 1, 1, True), (30, 2, 100, 40, 1, 0, 50, 0, 1, False)])
+def test_many_slots_are_prepared_as_few_are(dtype, H, G, D, E, maps, layout, rot, append, norm, mixed):
+    """norm, rotation and append of many (token, head) slots against launches of few: an fp32 sum of squares in another order"""
+    from umbrella_amd import _lib
+    T, step, code = 2400, 60, _lib.seq_dtype_code(dtype)
+    g = torch.Generator(device="cuda").manual_seed(D + E)
+    c, _, _, _ = _decode_store([T], G, maps * D, E, 0, dtype, 32, 1)
+    d, _, _, _ = _decode_store([T], G, maps * D, E, 0, dtype, 32, 2)
+    HQ, GK, GV = maps * H, append * maps * G, append * G
+    ld = HQ * D + GK * D + GV * E + 5
+    proj, freq = torch.randn(T, ld, generator=g, device="cuda"), torch.rand(64, generator=g, device="cuda")
+    wq, wk = (torch.randn(D, generator=g, device="cuda").to(dtype) for _ in range(2))
+    pos, slot = torch.arange(T, device="cuda", dtype=torch.int32), torch.zeros(T, device="cuda", dtype=torch.int32)
+    firsts = torch.randn(T, G * E, generator=g, device="cuda")
+    outs = []
+    for store, n in ((c, T), (d, step)):
+        q, keep = torch.empty(T, HQ * D, device="cuda"), torch.zeros(T, G * E, device="cuda")
+        for lo in range(0, T, n):
+            m = _lib.UmbValueMix(firsts[lo:].data_ptr(), keep[lo:].data_ptr(), 0.3, 0.0) if mixed else None
+            _lib.seq_call("umb_attn_prep_mix", q[lo:], store.struct(0), proj[lo:lo + n], ld, append, wq if norm else None, wk if norm else None, norm, norm,
+                          pos[lo:lo + n], slot[lo:lo + n], freq if rot else None, rot, layout, 1.1, n, H, G, D, E, maps, 0.1, 100, 1e-5, m, code)
+        outs.append([q, keep] + ([store.kv[0]["k"], store.kv[0]["v"]] if append else []))
+    eps = torch.finfo(dtype).eps
+    for i, (x, y) in enumerate(zip(*outs)):
+        if i >= 2:                                         # pages of the two stores hold the same sequence in the same order
+            x, y = x.float()[:T // 32], y.float()[:T // 32]
+        size = y.abs().max()
+        assert bool(((x - y).abs() <= (4e-6 * size if i < 2 else eps * y.abs() + 4e-6 * size)).all()), i
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,G,D,rot", [(8, 2, 64, 64), (9, 3, 128, 40), (30, 2, 22, 0)])
+def test_many_pooled_slots_are_prepared_as_few_are(dtype, H, G, D, rot):
+    from umbrella_amd import _lib
+    T, code = 1700, _lib.seq_dtype_code(dtype)
+    g = torch.Generator(device="cuda").manual_seed(D)
+    proj, freq = torch.randn(T, (H + G) * D + 3, generator=g, device="cuda"), torch.rand(64, generator=g, device="cuda")
+    pos, slot = torch.arange(T, device="cuda", dtype=torch.int32), torch.zeros(T, device="cuda", dtype=torch.int32)
+    outs = []
+    for seed, n in ((1, T), (2, 100)):
+        c, _, _, _ = _decode_store([T], G, D, D, 5, dtype, 32, seed)
+        q = torch.empty(T, H * D, device="cuda")
+        for lo in range(0, T, n):
+            _lib.seq_call("umb_pwa_prep", q[lo:], c.struct(0), proj[lo:lo + n], proj.shape[1], pos[lo:lo + n], slot[lo:lo + n], freq if rot else None, n, H, G,
+                          D, rot, 1e-5, code)
+        k, v = c.token_rows(0, 0, torch.arange(T))
+        outs.append((q, k.float(), v.float()))
+    eps = torch.finfo(dtype).eps
+    assert torch.equal(outs[0][2], outs[1][2])
+    for i in range(2):
+        x, y = outs[0][i], outs[1][i]
+        assert bool(((x - y).abs() <= (0 if i == 0 else eps) * y.abs() + 4e-6 * y.abs().max()).all())

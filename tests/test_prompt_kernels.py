@@ -251,6 +251,39 @@ def test_a_row_that_attends_everything_attends_nothing_else():
     assert (one[0, 0] - both[0, 8]).abs().max() < 2e-2 * both.abs().max()
 
 
+def test_masks_that_are_accepted_in_any_layout():
+    """one row of any stride, rows and columns to spare, no column: the logits are those of the same mask laid out plainly"""
+    from umbrella_amd.models.config import LlamaCfg
+    from umbrella_amd.models.llama import Llama
+    from umbrella_amd.models.synthetic import synth_state_small
+    cfg = LlamaCfg(vocab_size=128, hidden_size=256, intermediate_size=256, num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2,
+                   head_dim=64, eos_token_id=[], name="tiny")
+    m = Llama("tiny", max_length=128, device="cuda:0", dtype=torch.float16, state_dict=synth_state_small(cfg, 1), config=cfg)
+    m.alloc()
+    ids, at = torch.arange(20, 29)[None], torch.arange(9)
+    see = torch.tril(torch.ones(9, 9, dtype=torch.bool)).cuda()
+    m.inference(ids, at[None], see, at)
+
+    def row(mask, pos=torch.tensor([[8]]), slots=torch.tensor([8])):
+        return m.inference(ids[:, 8:], pos, mask, slots).clone()
+    some = torch.tensor([1, 0, 1, 1, 0, 1, 1, 0, 1], dtype=torch.bool, device="cuda")
+    for one in (torch.ones(9, dtype=torch.bool, device="cuda"), some):
+        want = row(one.clone()[None])
+        assert torch.equal(row(one[:, None].clone().T), want)                            # strides (1, 1)
+        assert torch.equal(row(torch.stack([one, ~one], 1)[:, :1].T), want)              # a column of a wider array
+    want = row(torch.ones(1, 9, dtype=torch.bool, device="cuda"))
+    assert torch.equal(row(torch.ones(1, 1, dtype=torch.bool, device="cuda").expand(1, 9)), want)     # strides (0, 0)
+    full = m.inference(ids, at[None], see, at).clone()
+    m.kv_cache.kv_offset = 9
+    spare = torch.cat([see, torch.zeros(2, 9, dtype=torch.bool, device="cuda")])
+    got = m.inference(ids, torch.arange(11)[None], spare, torch.arange(12))              # rows, positions and slots to spare
+    assert torch.allclose(got, full, rtol=0, atol=2e-3 * float(full.abs().max())) and m.kv_cache.kv_offset == 12
+    first = m.inference(ids[:, :1], at[None, :1], see[:1, :1], at[:1])
+    assert torch.equal(m.inference(ids[:, :1], at[None, :1], see[:1, :0], at[:1]), first)
+    with pytest.raises(AssertionError):
+        m.inference(ids, at[None], see[:8], at)
+
+
 def _decode_store(lens, G, DK, E, pool, dtype, page, seed):
     from umbrella_amd.attn.cache import PagedSeqCache
     c = PagedSeqCache([(G, DK, pool, E)], [], sum(lens), len(lens), "cuda", dtype, page=page)

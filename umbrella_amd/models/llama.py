@@ -176,6 +176,17 @@ def pack_mask_bits(mask: torch.Tensor) -> torch.Tensor:
     return (m.view(T, W, 64) << sh).sum(dim=-1)     # wraps into the sign bit as intended
 
 
+def mask_rows(mask: torch.Tensor, T: int):
+    """The first T rows of a mask as the mask kernels walk them -> (bool mask of unit column stride, row stride >= its columns).  A
+    dimension of size one counts as contiguous whatever its stride, so a lone row's stride is not to be read."""
+    mask = mask[:T]
+    mask = mask if mask.dtype == torch.bool else mask != 0
+    Cn = mask.shape[1]
+    if (Cn > 1 and mask.stride(1) != 1) or (T > 1 and mask.stride(0) < Cn):
+        mask = mask.contiguous()
+    return mask, (mask.stride(0) if T > 1 else Cn)
+
+
 class Llama(LLMBase):
     CHUNK = 64          # rows of the default workspace (tree / generic forwards)
     PREFILL_CHUNK = 1024  # prompt tokens per forward when the workspace allows: the matrix-bound verify GEMM streams the
@@ -690,15 +701,16 @@ class Llama(LLMBase):
             t = t.reshape(-1).to(dev)
             return (t if t.dtype in (torch.int32, torch.int64) else t.long()).contiguous()
         ids, pos, slots = index(input_ids), index(position_ids), index(storage_ids)
-        mask = attention_mask.to(dev)
-        mask = mask if mask.dtype == torch.bool else mask != 0
-        mask = mask if mask.stride(1) == 1 and mask.stride(0) >= mask.shape[1] else mask.contiguous()
-        T, Cn = ids.shape[0], mask.shape[1]
-        assert mask.shape[0] == T and pos.shape[0] == T and slots.shape[0] == T, (tuple(mask.shape), T)
+        T = ids.shape[0]
+        assert attention_mask.shape[0] >= T and pos.shape[0] >= T and slots.shape[0] >= T, (tuple(attention_mask.shape), T)
+        mask, ld = mask_rows(attention_mask.to(dev), T)
+        Cn = mask.shape[1]
+        if Cn == 0:                                 # no columns: the first slot alone
+            mask, ld, Cn = torch.ones(T, 1, dtype=torch.bool, device=dev), 1, 1
         wide = [int(t.dtype == torch.int64) for t in (ids, pos, slots)]
         nb = (Cn + 63) // 64
         scan = torch.empty(2 * nb + 1, dtype=torch.int32, device=dev)
-        _lib.call("umb_mask_scan", scan, mask, mask.stride(0), T, Cn, slots, wide[2])
+        _lib.call("umb_mask_scan", scan, mask, ld, T, Cn, slots, wide[2])
         scan = scan.tolist()
         prefix, kv_end = min(scan[0:2 * nb:2]), max(scan[1:2 * nb:2])    # columns every row attends in front; one past the last attended
         if kv_end <= prefix:                        # nothing behind the prefix: its last column becomes the masked part (a null mask is causal)
@@ -707,7 +719,7 @@ class Llama(LLMBase):
         W = (nmk + 63) // 64
         bits = torch.empty(T, W, dtype=torch.int64, device=dev)
         idx = torch.empty(3 * T + 1, dtype=torch.int32, device=dev)
-        _lib.call("umb_mask_pack", bits, W, idx, mask, mask.stride(0), T, Cn, prefix, ids, wide[0], pos, wide[1], slots, wide[2])
+        _lib.call("umb_mask_pack", bits, W, idx, mask, ld, T, Cn, prefix, ids, wide[0], pos, wide[1], slots, wide[2])
         pre = idx[3 * T:]
         V = self.config.vocab_size
         out = torch.empty(T, V, dtype=torch.float32, device=dev)
@@ -716,7 +728,8 @@ class Llama(LLMBase):
             self.forward_explicit(idx[lo:hi], idx[T + lo:T + hi], idx[2 * T + lo:2 * T + hi], pre,
                                   mask_bits=bits[lo:hi], mask_words=W, n_mask_keys=nmk, head_from=0)
             out[lo:hi] = self._bufs["logits"][:hi - lo]
-        self.kv_cache.kv_offset = max(self.kv_cache.kv_offset, scan[2 * nb] + 1)
+        last = scan[2 * nb] if slots.shape[0] == T else int(slots.max().item())
+        self.kv_cache.kv_offset = max(self.kv_cache.kv_offset, last + 1)
         return out[None]
 
     def graph_inference(self, input_ids, storage_ids, position_ids=None, attention_mask=None):

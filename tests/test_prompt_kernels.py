@@ -80,7 +80,7 @@ def test_few_token_linear(dtype, N, K):
     tol = 2.0 ** -24 * (K + 2) * (size + b.double().abs())
     unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
     rows = None
-    for T in (1, 8, 9, 17, 33, 48, 64, 65, 100):
+    for T in (1, 2, 7, 8, 9, 17, 33, 48, 64, 65, 100):
         out = torch.full((T + 1, N), 7.0, device="cuda")
         _lib.seq_call("umb_seq_linear", out, x[:T].contiguous(), w, b, T, N, K, 0, code)
         assert ((out[:T].double() - (full[:T] + b.double())).abs() <= tol[:T]).all() and bool((out[T] == 7.0).all())

@@ -483,6 +483,18 @@ template <int NT, int TT, int BP, bool DUAL, int R> struct StreamShape {     // 
   static constexpr size_t RED = (size_t)AT * 4 * TT * 1024, RING = (size_t)R * SLOT + (NP % 4 ? PIECE : 0);
   static constexpr size_t LDS = RING > RED ? RING : RED;
   static_assert(AP % 4 == 0 && R >= 2 && LDS <= 160 * 1024, "whole rounds of weight pieces; the CU's LDS");
+  static_assert(BP % TT == 0 && (BP == 8 * TT || TT == 1), "token tiles of whole pieces");
+  // place of a tile's row inside a slot; a token tile staged in part repeats its pieces: columns that are not stored
+  static constexpr unsigned row_at(int first_piece, int pieces, int row) { return (unsigned)(first_piece + (row >> 1) % pieces) * PIECE + (unsigned)(row & 1) * 512u; }
+  static constexpr unsigned weight_row(int tile, int row) { return row_at(8 * tile, 8, row); }
+  static constexpr unsigned token_row(int tile, int row) { return row_at(AP + 8 * tile, BP / TT, row); }
+  static constexpr bool rows_inside_slot() {
+    for (int row = 0; row < 16; ++row) {
+      for (int i = 0; i < AT; ++i) if (weight_row(i, row) + 512u > (unsigned)AP * PIECE) return false;
+      for (int i = 0; i < TT; ++i) if (token_row(i, row) < (unsigned)AP * PIECE || token_row(i, row) + 512u > SLOT) return false;
+    }
+    return true;
+  }
 };
 template <typename P, int NT, int TT, int BP, bool DUAL, int R>
 __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict__ out_, const typename El<P>::type* __restrict__ x,
@@ -491,6 +503,7 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
                                                                 int epi, LinExt ext) {
   typedef typename El<P>::type E;
   typedef StreamShape<NT, TT, BP, DUAL, R> S;
+  static_assert(S::rows_inside_slot(), "a fragment reads rows of the slot it belongs to and no others");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int EB = sizeof(E), STEPS = 512 / (32 * EB), AT = S::AT;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -544,9 +557,9 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
   for (int i = 0; i < AT; ++i)
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) acc[i][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const unsigned rowb = (unsigned)(j >> 1) * S::PIECE + (unsigned)(j & 1) * 512u, swz = (unsigned)(j & 1) * 8u;
-  auto frag = [&](unsigned base, int s) {  // 16 rows, the 32 k of step s
-    const auto at = [&](int c) { return *reinterpret_cast<const lds_u32x4*>((size_t)(base + rowb + (((unsigned)c) ^ swz) * 16u)); };
+  const unsigned wrow = S::weight_row(0, j), trow = S::token_row(0, j), swz = (unsigned)(j & 1) * 8u;
+  auto frag = [&](unsigned base, int s) {  // this lane's part of 16 rows, the 32 k of step s
+    const auto at = [&](int c) { return *reinterpret_cast<const lds_u32x4*>((size_t)(base + (((unsigned)c) ^ swz) * 16u)); };
     Frag8<P> f;
     if constexpr (EB == 2) f.v = at(s * 4 + g);
     else {
@@ -570,9 +583,9 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
       const int s = wave + 4 * u;
       Frag8<P> a[AT], b[TT];
 #pragma unroll
-      for (int i = 0; i < AT; ++i) a[i] = frag(base + (unsigned)(8 * i) * S::PIECE, s);
+      for (int i = 0; i < AT; ++i) a[i] = frag(base + wrow + (unsigned)(8 * i) * S::PIECE, s);
 #pragma unroll
-      for (int tt = 0; tt < TT; ++tt) b[tt] = frag(base + (unsigned)(S::AP + 8 * tt) * S::PIECE, s);
+      for (int tt = 0; tt < TT; ++tt) b[tt] = frag(base + trow + (unsigned)(8 * tt) * S::PIECE, s);
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt)
 #pragma unroll

@@ -176,6 +176,43 @@ def test_gla_chunks(H, D, Dv, lens, strong):
     assert torch.equal(st[0], state[0]) and bool(torch.isnan(scratch[need:]).all())
 
 
+@pytest.mark.parametrize("T,at", [(200, 70), (200, 64), (200, 135), (197, 196), (130, 0)])
+@pytest.mark.parametrize("kind", ["inf", "nan", "forget"])
+def test_gla_chunks_stay_causal_for_values_that_are_not_finite(kind, T, at):
+    """an infinite or NaN value spoils its own token and later ones, as token by token; a log decay of -inf is a decay of zero"""
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + at)
+    H, D, Dv = 2, 32, 80
+    HD, ld = H * D, 2 * H * D + H * Dv + 8
+    proj, la = torch.randn(T, ld, generator=g, device="cuda"), -0.2 * torch.rand(T, HD, generator=g, device="cuda")
+    state = torch.randn(1, H, D, Dv, generator=g, device="cuda")
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                            # noqa: E731
+    need = _lib.load_seq().umb_gla_scan_chunked_floats(T, 1, H, D, Dv)
+    scratch = torch.empty(need, device="cuda")
+
+    def chunked(p, log_decay):
+        o, st = torch.empty(T, H * Dv, device="cuda"), state.clone()
+        _lib.seq_call("umb_gla_scan_chunked", o, st, p, ld, log_decay, i32([0]), i32([0]), i32([3]), i32([T]), T, 1, T, H, D, Dv, 0.5, scratch, need)
+        return o, st
+    o0, _ = chunked(proj, la)
+    if kind == "forget":
+        la[at, ::3] = float("-inf")
+        la[min(at + 1, T - 1), 1::3] = float("-inf")
+    else:
+        proj[at, 2 * HD + 5] = float(kind)
+        proj[at, 2 * HD + Dv + 7] = -float(kind)
+    o1, s1 = chunked(proj, la)
+    o2, s2 = torch.empty(T, H * Dv, device="cuda"), state.clone()
+    _lib.seq_call("umb_gla_scan", o2, s2, proj, ld, la.exp(), i32([0]), i32([0]), i32([3]), i32([T]), 1, H, D, Dv, 0.5)
+    assert torch.equal(o1.isfinite(), o2.isfinite()) and torch.equal(s1.isfinite(), s2.isfinite())
+    assert bool(o1.isfinite().all()) == (kind == "forget")
+    fin, size = o2.isfinite(), float(o2[o2.isfinite()].abs().max())
+    # sums of a few hundred products in another order: 2^-24 times their number at most, of the largest output
+    assert float((o1 - o2)[fin].abs().max()) <= 2.0 ** -14 * size and float((s1 - s2)[s2.isfinite()].abs().max()) <= 2.0 ** -14 * float(state.abs().max() + size)
+    if kind != "forget":
+        assert torch.equal(o1[:at // 16 * 16], o0[:at // 16 * 16])               # blocks in front are what they were
+
+
 @pytest.mark.parametrize("H,D,Dv,per_head,groups", [(2, 16, 8, 0, 2), (4, 40, 60, 1, 2), (1, 128, 256, 0, 1), (2, 130, 64, 0, 2), (2, 256, 4, 1, 1)])
 def test_single_token_recurrence_follows_the_scan(H, D, Dv, per_head, groups):
     from umbrella_amd import _lib

@@ -384,7 +384,10 @@ extern "C" int umb_lin_step(float* o, float* state, const float* q, int ldq, con
 //   out    A v + (e^c q)^T S_start
 // fp32 throughout, products on the fp32 matrix pipe.  2048 tokens, 8 heads x 128 x 256 on one MI355X: 670 us token by token (a serial
 // loop on 512 waves) -> 100 (25 + 23 + 15 + 38); 192 tokens 66 -> 45.  D and Dv multiples of 16, D <= 128 (the chunk's q, k and offsets fill the LDS).
+// Values that are not finite stay where the recurrence has them: a log decay below GC_LA (a decay of zero in fp32, -inf included) is taken
+// as that; later tokens of a block meet an infinite value with weight zero, so such a block is summed token by token.
 constexpr int GC_Q = 64;
+constexpr float GC_LA = -128.f;
 
 struct GlaChunk {
   const float *q, *k, *v, *la;             // rows of proj at the q, k, v columns; la [T][H D]
@@ -426,7 +429,8 @@ __global__ __launch_bounds__(1024) void gla_chunk_prep_kernel(GlaChunk a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int t = 16 * u + i;
-      l[i] = a.la[(row0 + (t < cnt ? t : cnt - 1)) * HD + (long)h * D + d];
+      const float la = a.la[(row0 + (t < cnt ? t : cnt - 1)) * HD + (long)h * D + d];
+      l[i] = la < GC_LA ? GC_LA : la;            // a NaN stays one
     }
     double run = 0.0;
 #pragma unroll
@@ -543,7 +547,8 @@ __global__ __launch_bounds__(256) void gla_chunk_state_kernel(GlaChunk a) {
 #pragma unroll
       for (int y = 0; y < 4; ++y) {
         const int p = p0 + 16 * y + j;
-        fb[y][r] = a.v[(row0 + sc) * a.ld + (long)h * Dv + (p < Dv ? p : Dv - 1)];
+        const float vv = a.v[(row0 + sc) * a.ld + (long)h * Dv + (p < Dv ? p : Dv - 1)];
+        fb[y][r] = s < cnt ? vv : 0.f;
       }
     }
 #pragma unroll
@@ -606,11 +611,15 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(float* __restrict__ 
   float* vs = sm;                          // [64][LP]
   float* ss = vs + GC_Q * LP;              // [D][LP]: the chunk's start state
   const float* s0 = a.sc + ((long)(a.first(b) + blockIdx.y) * a.H + h) * D * Dv;
+  bool odd = false;                        // a value that is not finite
   for (int x = tid; x < (GC_Q + D) * 16; x += 256) {
     const int row = x >> 4, p = (x & 15) * 4, pc = p0 + p < Dv ? p0 + p : Dv - 4;
     const int t = row < GC_Q ? (row < cnt ? row : cnt - 1) : 0;
     const float* src = row < GC_Q ? a.v + (row0 + t) * a.ld + (long)h * Dv + pc : s0 + (long)(row - GC_Q) * Dv + pc;
-    *reinterpret_cast<f32x4*>(sm + row * LP + p) = *reinterpret_cast<const f32x4*>(src);
+    const f32x4 v = *reinterpret_cast<const f32x4*>(src);
+    *reinterpret_cast<f32x4*>(sm + row * LP + p) = v;
+    const f32x4 z = v - v;                 // zero, or NaN
+    odd = odd || (row < GC_Q && !(z[0] + z[1] + z[2] + z[3] == 0.f));
   }
   const int t = 16 * wave + j, tc = t < cnt ? t : cnt - 1;
   f32x4 fm[4], fq[8];
@@ -618,7 +627,7 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(float* __restrict__ 
   for (int i = 0; i < 4; ++i) fm[i] = i <= wave ? *reinterpret_cast<const f32x4*>(a.m + ((row0 + tc) * a.H + h) * 64 + 16 * i + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < 8; ++i) fq[i] = 16 * i < D ? *reinterpret_cast<const f32x4*>(a.qt + (row0 + tc) * HD + (long)h * D + 16 * i + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
-  __syncthreads();
+  odd = __syncthreads_or(odd);
   f32x4 acc[4];
 #pragma unroll
   for (int y = 0; y < 4; ++y) acc[y] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -637,9 +646,19 @@ __global__ __launch_bounds__(256) void gla_chunk_out_kernel(float* __restrict__ 
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    if (i <= wave) {
+    if (i < wave || (i == wave && !odd)) {
 #pragma unroll
       for (int y = 0; y < 4; ++y) acc[y] = gla_mma(fm[i], cols(vs, 16 * i, y), acc[y]);
+    }
+  }
+  if (odd) {                               // the wave's own block: no product with a later token's value
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tt = 16 * wave + 4 * g + r;
+      const float* mr = a.m + ((row0 + (tt < cnt ? tt : cnt - 1)) * a.H + h) * 64;
+      for (int u = 16 * wave; u <= tt; ++u)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) acc[y][r] += mr[u] * vs[u * LP + 16 * y + j];
     }
   }
 #pragma unroll

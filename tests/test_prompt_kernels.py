@@ -176,6 +176,30 @@ def test_gla_chunks(H, D, Dv, lens, strong):
     assert torch.equal(st[0], state[0]) and bool(torch.isnan(scratch[need:]).all())
 
 
+@pytest.mark.parametrize("decay", [0.01, 1.0, 4.0])
+@pytest.mark.parametrize("u", [0, 3])
+def test_gla_chunks_weigh_as_well_as_token_by_token(decay, u):
+    """single weights e^(sum of log decays) inside a block, read out by values of one: relative, however small the weight"""
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(int(decay * 100) + u)
+    D, Dv, T = 16, 16, 64
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                            # noqa: E731
+    need = _lib.load_seq().umb_gla_scan_chunked_floats(T, 1, 1, D, Dv)
+    proj, scratch = torch.zeros(T, 2 * D + Dv, device="cuda"), torch.empty(need, device="cuda")
+    proj[:, 0], proj[:, D] = 1.0, 1.0
+    own = torch.arange(16 * u, 16 * u + 16, device="cuda")
+    proj[own, 2 * D + torch.arange(16, device="cuda")] = 1.0
+    la = -2 * decay * torch.rand(T, D, generator=g, device="cuda")
+    o, st = torch.empty(T, Dv, device="cuda"), torch.zeros(1, 1, D, Dv, device="cuda")
+    _lib.seq_call("umb_gla_scan_chunked", o, st, proj, 2 * D + Dv, la, i32([0]), i32([0]), i32([0]), i32([T]), T, 1, T, 1, D, Dv, 1.0, scratch, need)
+    c = la[:, 0].double().cumsum(0)[own]
+    want = (c[:, None] - c[None]).exp().tril()
+    see = want > 2.0 ** -120
+    # the exponential unit's last place (2^-23), the exponent's rest to first order (2^-26) and one rounding behind it
+    assert float(((o[own].double() - want).abs() / want.clamp(min=1e-300))[see].max()) <= 4 * 2.0 ** -24
+    assert bool((o[own][~see].abs() < 2.0 ** -119).all())
+
+
 @pytest.mark.parametrize("T,at", [(200, 70), (200, 64), (200, 135), (197, 196), (130, 0)])
 @pytest.mark.parametrize("kind", ["inf", "nan", "forget"])
 def test_gla_chunks_stay_causal_for_values_that_are_not_finite(kind, T, at):

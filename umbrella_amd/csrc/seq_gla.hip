@@ -379,15 +379,29 @@ extern "C" int umb_lin_step(float* o, float* state, const float* q, int ldq, con
 // All exponents are of non-positive numbers.  A's 16 x 16 blocks below the diagonal split the exponent at the start r of the row
 // block, (e^(c_t - r) q_t) . (e^(r - c_s) k_s), a matrix product; in the diagonal blocks the split would need e^(+): there every
 // pair of tokens and channel takes its own exponential.  Four launches, all but the second over (column slice, chunk, head, sequence):
-//   prep   c (prefix sums in double, kept as blocks' starts and offsets inside a block in two 32-bit parts), A, e^(c_t) q_t, e^(c_64 - c_s) k_s
+//   prep   c (prefix sums in double and base 2, kept as blocks' starts and offsets inside a block in two 32-bit parts), A, e^(c_t) q_t,
+//          e^(c_64 - c_s) k_s
 //   state  every chunk's sum from a zero state        pass   chunks in order: sums become start states, the slot the final one
 //   out    A v + (e^c q)^T S_start
 // fp32 throughout, products on the fp32 matrix pipe.  2048 tokens, 8 heads x 128 x 256 on one MI355X: 670 us token by token (a serial
-// loop on 512 waves) -> 100 (25 + 23 + 15 + 38); 192 tokens 66 -> 45.  D and Dv multiples of 16, D <= 128 (the chunk's q, k and offsets fill the LDS).
+// loop on 512 waves) -> 92; 192 tokens 66 -> 45.  D and Dv multiples of 16, D <= 128 (the chunk's q, k and offsets fill the LDS).
 // Values that are not finite stay where the recurrence has them: a log decay below GC_LA (a decay of zero in fp32, -inf included) is taken
 // as that; later tokens of a block meet an infinite value with weight zero, so such a block is summed token by token.
 constexpr int GC_Q = 64;
 constexpr float GC_LA = -128.f;
+// An offset inside a block as r + l / ln 2: r a multiple of 2^-12 (below 4096: 24 bits, so a difference of two is exact), l small.
+// e^(difference) = 2^dr (1 + dl) is then good to 2^-22 however large it is, where an exponent x rounded to 32 bits costs x 2^-24.  Relative error
+// of the weights inside a block, largest / root mean square in 2^-24, decays of 4 a token: 2.1 / 0.58; with the rounded exponent 149 / 19;
+// token by token 7.9 / 1.3.
+constexpr double GC_LOG2E = 1.4426950408889634, GC_LN2 = 0.6931471805599453;
+__device__ __forceinline__ float gla_exp(float r, float l) {
+  const float v = __builtin_amdgcn_exp2f(r);
+  return fmaf(v, l, v);
+}
+__device__ __forceinline__ float gla_exp(double c) {        // 2^c
+  const float r = (float)c;
+  return gla_exp(r, (float)((c - (double)r) * GC_LN2));
+}
 
 struct GlaChunk {
   const float *q, *k, *v, *la;             // rows of proj at the q, k, v columns; la [T][H D]
@@ -419,8 +433,8 @@ __global__ __launch_bounds__(1024) void gla_chunk_prep_kernel(GlaChunk a) {
   const long row0 = (long)a.seq_row0[b] + t0;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, g = lane >> 4;
   double* blk = reinterpret_cast<double*>(sm);   // [5][128]: c at the starts of the four blocks, and at the chunk's end
-  float* rs = sm + 2 * 5 * 128;                  // [64][LD]: c_t less the start of t's block, rounded ..
-  float* rl = rs + GC_Q * LD;                    // [64][LD]: .. and what the rounding left (a channel that forgets at once has sums of hundreds)
+  float* rs = sm + 2 * 5 * 128;                  // [64][LD]: c_t less the start of t's block: r ..
+  float* rl = rs + GC_Q * LD;                    // [64][LD]: .. and l
   float* qs = rl + GC_Q * LD;                    // [64][LD]
   float* ks = qs + GC_Q * LD;                    // [64][LD]
   if (tid < 512 && (tid & 127) < D) {            // (channel, block): the block's running sums
@@ -436,10 +450,10 @@ __global__ __launch_bounds__(1024) void gla_chunk_prep_kernel(GlaChunk a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int t = 16 * u + i;
-      run += t < cnt ? (double)l[i] : 0.0;
-      const float hi = (float)run;
-      rs[t * LD + d] = hi;
-      rl[t * LD + d] = (float)(run - (double)hi);
+      run += t < cnt ? GC_LOG2E * (double)l[i] : 0.0;
+      const double r = rint(run * 4096.0) / 4096.0;
+      rs[t * LD + d] = (float)r;
+      rl[t * LD + d] = (float)((run - r) * GC_LN2);
     }
     blk[(u + 1) * 128 + d] = run;                // the block's own sum for now
   }
@@ -464,7 +478,7 @@ __global__ __launch_bounds__(1024) void gla_chunk_prep_kernel(GlaChunk a) {
       run += blk[i * 128 + tid];
       blk[i * 128 + tid] = run;
     }
-    a.ac[((long)nc * a.H + h) * D + tid] = expf((float)run);
+    a.ac[((long)nc * a.H + h) * D + tid] = gla_exp(run);
   }
   __syncthreads();
   for (int x = tid; x < GC_Q * dq; x += 1024) {   // what the other launches read: decayed from the chunk's start, to its end
@@ -473,15 +487,14 @@ __global__ __launch_bounds__(1024) void gla_chunk_prep_kernel(GlaChunk a) {
     f32x4 qv = *reinterpret_cast<const f32x4*>(qs + t * LD + d), kv = *reinterpret_cast<const f32x4*>(ks + t * LD + d);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const double c = blk[(t >> 4) * 128 + d + e] + ((double)rs[t * LD + d + e] + (double)rl[t * LD + d + e]);
-      qv[e] *= expf((float)c);
-      kv[e] *= expf((float)(blk[4 * 128 + d + e] - c));
+      const double c = blk[(t >> 4) * 128 + d + e] + ((double)rs[t * LD + d + e] + GC_LOG2E * (double)rl[t * LD + d + e]);
+      qv[e] *= gla_exp(c);
+      kv[e] *= gla_exp(blk[4 * 128 + d + e] - c);
     }
     *reinterpret_cast<f32x4*>(a.qt + (row0 + t) * HD + (long)h * D + d) = qv;
     *reinterpret_cast<f32x4*>(a.kh + (row0 + t) * HD + (long)h * D + d) = kv;
   }
   // diagonal block tid / 256: thread (row, column)
-  constexpr float L2E = 1.44269504088896341f;
   const int tr = (tid >> 4) & 15, ts = tid & 15;
   {
     const int t = 16 * (tid >> 8) + tr, s = 16 * (tid >> 8) + ts;
@@ -492,7 +505,7 @@ __global__ __launch_bounds__(1024) void gla_chunk_prep_kernel(GlaChunk a) {
         const f32x4 rt = *reinterpret_cast<const f32x4*>(rs + t * LD + d), r4 = *reinterpret_cast<const f32x4*>(rs + s * LD + d);
         const f32x4 lt = *reinterpret_cast<const f32x4*>(rl + t * LD + d), l4 = *reinterpret_cast<const f32x4*>(rl + s * LD + d);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc += q4[e] * k4[e] * __builtin_amdgcn_exp2f(((rt[e] - r4[e]) + (lt[e] - l4[e])) * L2E);
+        for (int e = 0; e < 4; ++e) acc += q4[e] * k4[e] * gla_exp(rt[e] - r4[e], lt[e] - l4[e]);
       }
     }
     if (t < cnt) a.m[((row0 + t) * a.H + h) * 64 + s] = acc;
@@ -507,8 +520,8 @@ __global__ __launch_bounds__(1024) void gla_chunk_prep_kernel(GlaChunk a) {
       f32x4 x = *reinterpret_cast<const f32x4*>(qs + t * LD + k0), y = *reinterpret_cast<const f32x4*>(ks + s * LD + k0);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        x[e] *= expf(rs[t * LD + k0 + e]);           // (an error in a sum that large is an error in nothing)
-        y[e] *= expf((float)(blk[rb * 128 + k0 + e] - (blk[cb * 128 + k0 + e] + ((double)rs[s * LD + k0 + e] + (double)rl[s * LD + k0 + e]))));
+        x[e] *= gla_exp(rs[t * LD + k0 + e], rl[t * LD + k0 + e]);
+        y[e] *= gla_exp(blk[rb * 128 + k0 + e] - (blk[cb * 128 + k0 + e] + ((double)rs[s * LD + k0 + e] + GC_LOG2E * (double)rl[s * LD + k0 + e])));
       }
       acc = gla_mma(x, y, acc);
     }

@@ -505,10 +505,17 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
 //   S^T as two 16-key MFMA tiles; P = visible ? sigmoid(S scale + bias) : 0 in fp32, lane (query j, key quad g) holding keys 4g .. 4g+3
 //   of both tiles -- which IS the lane's share of the B operand of the value product.
 // Scores and weights stay fp32-exact on a bf16 / f16 matrix pipe by splitting the fp32 factor into a high and a low 16-bit
-// half (x = hi + lo to 2^-17): q, the pooled means (held in fp32) and the weights go through two MFMAs instead of one; the exponential and
-// the reciprocal of the sigmoid (one and two units in the last place, 2^-22) are far below that.
+// half (x = hi + lo to 2^-17 in bf16, 2^-22 in fp16): q, the pooled means (held in fp32) and the weights go through two MFMAs instead of one.
 // It is bound by the vector work between the products.  With every wave staging its own values, gathering them two bytes at a time and
-// testing every key: 38 vector instructions a matrix instruction and 129 us at 2048 positions, 32 + 8 heads of 64, window 512; now 45.
+// testing every key: 38 vector instructions a matrix instruction and 121 us at 2048 positions, 32 + 8 heads of 64, window 512; now 57.
+// A quarter of that is the sigmoid: with the exponential and the reciprocal as the units give them 45, but its error then grows with the score
+// (relative, root mean square in 2^-24: 1.7 within scores of 8 and 6.1 within 30; as below 0.64 and 0.56, a full divide the same).
+// 1 / (1 + e^-x): the quotient by one Newton step, which rounds as the divide does
+__device__ __forceinline__ float sigmoid_rcp(float x) {
+  const float d = 1.f + expf(-x), r = __builtin_amdgcn_rcpf(d), w = fmaf(fmaf(-d, r, 1.f), r, r);
+  return d < 1e37f ? w : r;                                // d infinite, or r next to the smallest number: no step
+}
+
 template <typename P> __device__ __forceinline__ void split8(const float* v, u32x4& hi, u32x4& lo) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -525,7 +532,6 @@ __global__ __launch_bounds__(256) void pwa_attend_mfma_kernel(u16* __restrict__ 
                                                               const int* __restrict__ seq_len, int H, int G, int window, int pool,
                                                               float scale) {
   constexpr int D = NS * 32, LD = D + 8, LT = 36, NL = (D + 63) / 64;   // row strides of the two tiles; 8-feature chunks of a row per thread
-  constexpr float L2E = 1.4426950408889634f;
   extern __shared__ __attribute__((aligned(16))) u16 pwa_lds[];
   u16* k_hi = pwa_lds;                                         // [32][LD]
   u16* v_hi = k_hi + 32 * LD;                              // [D][LT]
@@ -582,7 +588,7 @@ __global__ __launch_bounds__(256) void pwa_attend_mfma_kernel(u16* __restrict__ 
     auto weights = [&](f32x4 (&s2)[2], bool whole, auto sees, u32x4& hi, u32x4& lo) {
       float w[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) w[e] = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(s2[e >> 2][e & 3] * scale + bias) * L2E));
+      for (int e = 0; e < 8; ++e) w[e] = sigmoid_rcp(s2[e >> 2][e & 3] * scale + bias);
       if (!whole) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) w[e] = q_ok && sees(16 * (e >> 2) + 4 * g4 + (e & 3)) ? w[e] : 0.f;

@@ -251,7 +251,7 @@ __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x,
     if (q < nq) { *reinterpret_cast<f32x4*>(x + o + 4 * q) = a; ss += sq4(xv[e]); }
   }
   if (!w_next) return;
-  const float f = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)W + eps);
+  const float f = 1.f / sqrtf(row_sum<NT>(ss, red) / (float)W + eps);
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int q = (int)threadIdx.x + NT * e;
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(NT) void hc_embed_quad_kernel(float* __restrict__ x
     if (q < nq) { *reinterpret_cast<f32x4*>(x + o + 4 * q) = v; ss += sq4(ev[e]); }
   }
   if (!h) return;
-  const float f = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)W + eps);
+  const float f = 1.f / sqrtf(row_sum<NT>(ss, red) / (float)W + eps);
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int q = (int)threadIdx.x + NT * e;

@@ -340,7 +340,7 @@ __global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) ss += (int)threadIdx.x + NT * e < nq ? sq4(yv[e]) : 0.f;
-  const float f = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)gs + eps);
+  const float f = 1.f / sqrtf(row_sum<NT>(ss, red) / (float)gs + eps);
   float s2 = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__
     if (q < nq) { *reinterpret_cast<f32x4*>(x + o + 4 * q) = xv[e]; s2 += sq4(xv[e]); }
   }
   if (!w_next) return;
-  const float f2 = 1.f / sqrtf(block_sum<NT>(s2, red2) / (float)gs + eps);
+  const float f2 = 1.f / sqrtf(row_sum<NT>(s2, red2) / (float)gs + eps);
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int q = (int)threadIdx.x + NT * e;
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(NT) void norm_quad_kernel(float* __restrict__ out_f
       if (EMBED) *reinterpret_cast<f32x4*>(out_f32 + o + 4 * q) = xv[e];
     }
   }
-  const float f = 1.f / sqrtf(block_sum<NT>(ss, red) / (float)gs + eps);
+  const float f = 1.f / sqrtf(row_sum<NT>(ss, red) / (float)gs + eps);
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int q = (int)threadIdx.x + NT * e;
@@ -423,14 +423,14 @@ __global__ __launch_bounds__(NT) void pair_resid_norm_quad_kernel(float* __restr
     sa += in ? sq4(a[e]) : 0.f;
     sb += in ? sq4(b[e]) : 0.f;
   }
-  const float fa = coef / sqrtf(block_sum<NT>(sa, red[0]) / (float)W + eps), fb = coef / sqrtf(block_sum<NT>(sb, red[1]) / (float)W + eps);
+  const float fa = coef / sqrtf(row_sum<NT>(sa, red[0]) / (float)W + eps), fb = coef / sqrtf(row_sum<NT>(sb, red[1]) / (float)W + eps);
   float sm = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     a[e] = a[e] * fa * wa[e] + b[e] * fb * wb[e];
     sm += (int)threadIdx.x + NT * e < nq ? sq4(a[e]) : 0.f;
   }
-  const float fm = 1.f / sqrtf(block_sum<NT>(sm, red[2]) / (float)W + eps);
+  const float fm = 1.f / sqrtf(row_sum<NT>(sm, red[2]) / (float)W + eps);
   float sx = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
@@ -439,7 +439,7 @@ __global__ __launch_bounds__(NT) void pair_resid_norm_quad_kernel(float* __restr
     if (q < nq) { *reinterpret_cast<f32x4*>(x + o + 4 * q) = xv[e]; sx += sq4(xv[e]); }
   }
   if (!w_next) return;
-  const float fx = 1.f / sqrtf(block_sum<NT>(sx, red[3]) / (float)W + eps);
+  const float fx = 1.f / sqrtf(row_sum<NT>(sx, red[3]) / (float)W + eps);
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int q = (int)threadIdx.x + NT * e;

@@ -95,6 +95,120 @@ def test_few_token_linear(dtype, N, K):
         assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())
 
 
+UNIT = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}
+
+
+def _bounded(got, want, tol, unit=0.0):
+    """tol: of the fp32 value; unit: its rounding to storage"""
+    return bool(((got.double() - want).abs() <= 1.02 * unit * want.abs() + tol + 2.0 ** -25).all())
+
+
+# whole 512-byte chunks of K in a batch of problems, row strides beyond the row, output gates: launches of few workgroups (the ring) and of more
+# than one per unit (the one-tile kernels); one chunk and several
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,N,K", [(3, 40, 512), (5, 72, 256), (40, 200, 256), (2, 130, 1280)])
+@pytest.mark.parametrize("T", [1, 7, 17, 48, 70, 300])
+def test_batched_linear_in_whole_chunks(dtype, B, N, K, T):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + N + K)
+    code, ldx, ldo = _lib.seq_dtype_code(dtype), B * K + 256, B * N + 5
+    x, w = torch.randn(T, ldx, generator=g, device="cuda").to(dtype), torch.randn(B, N, K, generator=g, device="cuda").to(dtype)
+    gate = torch.randn(T, B * N + 3, generator=g, device="cuda")
+    xs = x[:, :B * K].double().view(T, B, K).transpose(0, 1).contiguous()
+    wt = w.double().transpose(1, 2).contiguous()
+    full, size = (torch.bmm(a, b).transpose(0, 1).reshape(T, B * N) for a, b in ((xs, wt), (xs.abs(), wt.abs())))
+    tol = 2.0 ** -24 * (K + 2) * size
+    for epi in (0, 1, 3, 7):
+        out = torch.full((T + 1, ldo), 7.0, dtype=torch.float32 if epi == 0 else dtype, device="cuda")
+        _lib.seq_call("umb_seq_linear_batched", out, x, w, T, N, K, ldx, ldo, B, K, N * K, N, epi, gate if epi > 1 else None, B * N + 3,
+                      N if epi == 3 else 1, code)
+        f = 1.0
+        if epi == 3:
+            f = torch.sigmoid(gate[:, :B * N].double())
+        elif epi == 7:
+            f = torch.sigmoid(gate[:, :B].double()).repeat_interleave(N, 1)
+        # a quotient by 1 + e^-gate behind the sum: 2^-22 of it
+        assert _bounded(out[:T, :B * N], full * f, tol + 2.0 ** -22 * (full * f).abs(), UNIT[dtype] if epi else 0.0), epi
+        assert bool((out[T] == 7.0).all()) and bool((out[:, B * N:] == 7.0).all())
+
+
+def _glu(kind, gate, up):
+    if kind == 5:                                          # limit 1.5, alpha 1.7
+        gate, up = gate.clamp(max=1.5), up.clamp(-1.5, 1.5)
+        return gate * torch.sigmoid(1.7 * gate) * (up + 1)
+    if kind == 6:
+        return torch.nn.functional.gelu(gate, approximate="tanh") * up
+    return torch.nn.functional.silu(gate) * up
+
+
+# tile lists in whole chunks: whole, partial and empty tiles, every epilogue; output rows few and many, so that both kernels run
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("tile_rows", [16, 64])
+@pytest.mark.parametrize("N,K", [(72, 512), (1500, 256), (40, 1280)])
+def test_grouped_linear_in_whole_chunks(dtype, tile_rows, N, K):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(tile_rows + N + K)
+    code, E = _lib.seq_dtype_code(dtype), 4
+    tiles = [(2, 0, tile_rows), (2, tile_rows, 3), (0, tile_rows + 3, 1), (3, tile_rows + 4, tile_rows - 1), (0, 0, 0), (1, 2 * tile_rows + 3, 9)]
+    T = 2 * tile_rows + 12
+    grp = torch.zeros(T, dtype=torch.long, device="cuda")
+    for e, r0, n in tiles:
+        grp[r0:r0 + n] = e
+    tl = torch.tensor(tiles, dtype=torch.int32, device="cuda")
+    x, w = torch.randn(T, K, generator=g, device="cuda").to(dtype), (0.1 * torch.randn(E, 2 * N, K, generator=g, device="cuda")).to(dtype)
+    full, size = torch.empty(T, 2 * N, dtype=torch.float64, device="cuda"), torch.empty(T, 2 * N, dtype=torch.float64, device="cuda")
+    for e in range(E):
+        full[grp == e], size[grp == e] = x[grp == e].double() @ w[e].double().T, x[grp == e].double().abs() @ w[e].double().abs().T
+    tol = 2.0 ** -24 * (K + 2) * size
+    gate, up, tg, tu = full[:, :N], full[:, N:], tol[:, :N], tol[:, N:]
+    for epi in (0, 1, 4, 2, 5, 6):
+        dual = epi in (2, 5, 6)
+        out = torch.full((T + 1, N if dual else 2 * N), 7.0, dtype=torch.float32 if epi == 0 else dtype, device="cuda")
+        if epi == 5:
+            _lib.seq_call("umb_seq_linear_grouped_glu", out, x, w, tl, len(tiles), tile_rows, 2 * N * K, 2 * N, K, 1.5, 1.7, code)
+        else:
+            _lib.seq_call("umb_seq_linear_grouped", out, x, w, tl, len(tiles), tile_rows, 2 * N * K, 2 * N, K, epi, code)
+        if dual:                                           # |d act / d gate| <= 1.2 for the three, |act| <= |gate| + 0.3
+            want = _glu(epi, gate, up)
+            assert _bounded(out[:T], want, 1.2 * tg * (up.abs() + 1) + (gate.abs() + 0.3) * tu + 2e-6 * (want.abs() + up.abs()), UNIT[dtype]), epi
+        elif epi == 4:
+            want = full.clamp(min=0).pow(2)
+            assert _bounded(out[:T], want, 2 * tol * full.abs() + tol * tol + 2.0 ** -23 * want, UNIT[dtype])
+        else:
+            assert _bounded(out[:T], full, tol, UNIT[dtype] if epi else 0.0)
+        assert bool((out[T] == 7.0).all())
+
+
+# the remaining epilogues of the dense products: the ring (whole chunks, few tokens) and the staged tiles (many tokens)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,N,K", [(5, 72, 512), (30, 200, 256), (60, 40, 768), (300, 260, 192), (257, 2304, 128)])
+def test_epilogues_of_linears(dtype, T, N, K):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + N + K)
+    code = _lib.seq_dtype_code(dtype)
+    x, w, b = torch.randn(T, K, generator=g, device="cuda").to(dtype), (0.1 * torch.randn(N, K, generator=g, device="cuda")).to(dtype), torch.randn(N, generator=g, device="cuda").to(dtype)
+    full, size = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
+    tol = 2.0 ** -24 * (K + 3) * size
+    out = torch.full((T + 1, N), 7.0, dtype=dtype, device="cuda")
+    _lib.seq_call("umb_seq_linear", out, x, w, b, T, N, K, 4, code)
+    want = full.clamp(min=0).pow(2)
+    assert _bounded(out[:T], want, 2 * tol * full.abs() + tol * tol + 2.0 ** -23 * want, UNIT[dtype]) and bool((out[T] == 7.0).all())
+    cap = torch.full((T + 1, N), 7.0, device="cuda")
+    _lib.seq_call("umb_seq_linear_cap", cap, x, w, b, T, N, K, 2.5, code)
+    assert _bounded(cap[:T], 2.5 * torch.tanh(full / 2.5), tol + 2e-6) and bool((cap[T] == 7.0).all())      # a tangent of 2^-22 at most
+    half = N // 2
+    gate, up, tg, tu = full[:, :half], full[:, half:], tol[:, :half], tol[:, half:]
+    for epi in (2, 5, 6):
+        act = torch.full((T + 1, half), 7.0, dtype=dtype, device="cuda")
+        if epi == 5:
+            _lib.seq_call("umb_seq_linear_glu", act, x, w, b, T, N, K, 1.5, 1.7, code)
+        else:
+            _lib.seq_call("umb_seq_linear", act, x, w, b, T, N, K, epi, code)
+        want = _glu(epi, gate, up)
+        assert _bounded(act[:T], want, 1.2 * tg * (up.abs() + 1) + (gate.abs() + 0.3) * tu + 2e-6 * (want.abs() + up.abs()), UNIT[dtype]), epi
+        assert bool((act[T] == 7.0).all())
+
+
 # rows in quads: every workgroup size (64 ... 1024 threads, two quads a thread), a group that ends inside the last wave, several groups
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("W,groups", [(8, 1), (200, 1), (1024, 2), (1200, 1), (3072, 3), (2052, 1), (4096, 1), (4100, 1), (8192, 1)])

@@ -656,6 +656,7 @@ static int launch_stream_as(void* out, const void* x, const void* w, const void*
 // workgroups on a CU for one token tile, one workgroup for more (gate/up of 32 tokens: two, 48 us against 51).  32 output rows per
 // workgroup halve the token traffic of launches that stay above one workgroup per CU (32000 x 2048, 48 tokens 51 -> 37 us; 4096 x 4096,
 // 256 workgroups of 16 rows: 12.4 us, 15.3 as 128 of 32).
+static inline bool stream_narrow(int N, int token_tiles, int gz) { return (long)((N + 15) / 16) * token_tiles * gz <= 256; }
 template <typename P>
 static int launch_stream(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
                          const LinExt& ext, int gy = 0, int gz = 1) {
@@ -670,7 +671,7 @@ static int launch_stream(void* out, const void* x, const void* w, const void* bi
   if (T <= 8) STREAM(1, 1, 4, false, 4);
   if (T <= 16) STREAM(1, 1, 8, false, 4);
   if (T <= 32) STREAM(1, 2, 16, false, 3);
-  const bool narrow = (long)((N + 15) / 16) * (gy > 0 ? gy : (T + 63) / 64) * gz <= 256;
+  const bool narrow = stream_narrow(N, gy > 0 ? (gy + 1) / 2 : (T + 63) / 64, gz);    // about half of a tile list is in use
   if (T <= 48) {
     if (narrow) STREAM(1, 3, 24, false, 3);
     STREAM(2, 3, 24, false, 3);
@@ -685,6 +686,33 @@ static bool stream_ok(const void* x, const void* w, int N, int K, int epi, const
   auto al = [eb](long n) { return n * eb % 16 == 0; };
   return (long)K * eb % 512 == 0 && al(ext.ldx) && al(ext.sx) && al(ext.sw) && al(ext.gs) && ((uintptr_t)x | (uintptr_t)w) % 16 == 0 &&
          ((epi_dual(epi) ? (long)N : 0L) + 64) * K * eb < (1L << 32) && (long)ext.ldx * 64 * eb < (1L << 32);
+}
+
+// Where the ring pays.  A workgroup fills three chunks before its first product and its LDS lets two of them on a unit, where the
+// one-tile kernel has eight: with K of few chunks and more workgroups than units the latter is ahead, and a batch of prompts re-uses both
+// operands, which its 64 x 64 tiles do and the ring's 32 rows do not.  us, one-tile kernel / ring, one MI355X, bf16: 32 x (512 x 256), 65 tokens
+// 9.3 / 15.1; 32 x (128 x 512), 128 tokens 12.8 / 7.8 (256 workgroups), 200 15.6 / 15.9, 2000 66 / 114; 16384 x 1536, one token 10.3 / 11.2;
+// 16384 x 256, 32 tokens 5.5 / 6.3; fp32 2048 x 256, 300 tokens 10.4 / 12.2, 32 x (256 x 512), 300 tokens 62 / 49.
+static bool stream_pays(int T, int N, int K, int epi, int gz, int eb) {
+  const long chunks = (long)K * eb / 512;
+  const int rows = !epi_dual(epi) && T > 32 && !stream_narrow(N, (T + 63) / 64, gz) ? 32 : 16;
+  const int tokens = T <= 16 ? 16 : T <= 32 ? 32 : T <= 48 ? 48 : 64;
+  const long wgs = (long)((N + rows - 1) / rows) * ((T + tokens - 1) / tokens) * gz;
+  if (wgs <= 256) return true;
+  if (T <= 4 && eb == 2 && gz == 1) return chunks >= 8 || (epi_dual(epi) ? chunks > 2 || wgs <= 384 : wgs <= 512);
+  if (T <= 64) return eb == 4 || chunks > 1 || wgs <= 384;
+  return eb == 4 ? chunks > 2 : chunks > 1 && gz == 1;
+}
+// The same for tile lists, whose tiles in use are not known here (bf16, eight experts, two a token; us, one-tile kernel / ring): tiles of
+// 16 rows, single matrices: 2048 x 2048 12.7 / 14.5 at 4 tokens, 4096 x 1024 15.2 / 18.7 at 16, 4096 x 3584 47 / 43, 1024 x 2048 8.8 / 8.4;
+// gate and up together 28672 x 4096 94 / 81.  Tiles of 64 rows: 4096 x 1024 17.5 / 23.3 at 64 tokens, gate and up 8192 x 2048 37 / 38, 3584 x 4096
+// 56 / 62 at 33; 1024 x 1024 12 / 7.3; fp32 2048 x 512 16.6 / 18.2 at 33, 2048 x 2048 67 / 54.
+static bool stream_pays_grouped(int tile_rows, int N, int K, int epi, int eb) {
+  const long chunks = (long)K * eb / 512;
+  const bool dual = epi_dual(epi);
+  if (eb == 4) return tile_rows == 16 || chunks >= 16 || (dual ? 2 : 1) * N <= 128 * chunks;
+  if (tile_rows == 16) return dual || chunks >= 12 || N <= 128 * chunks;
+  return dual ? chunks >= 12 || 2 * N <= 384 * chunks : N <= 384 * chunks && N < 3584;
 }
 
 // gy > 0: the number of token tiles is given (grouped launches); gz: independent problems
@@ -708,7 +736,8 @@ template <typename P, bool VEC>
 static int launch_vec(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
                       const LinExt& ext, int gz = 1) {
   const bool dense = gz == 1 && ext.ldx == K && ext.ldo == N && epi != EPI_GATE && epi != EPI_GATE_ROW;
-  const bool stream = VEC && stream_ok(x, w, N, K, epi, ext, sizeof(typename El<P>::type));
+  constexpr int EB = sizeof(typename El<P>::type);
+  const bool stream = VEC && stream_ok(x, w, N, K, epi, ext, EB) && stream_pays(T, N, K, epi, gz, EB);
   if constexpr (sizeof(typename El<P>::type) == 2) {
     // both operands re-used: from 256 tokens on, and for 65 and more where the launch has some 100 tiles of 128 x 128 (cold weights, 100 /
     // 200 tokens: 18496 x 4096 56 / 72 us, the streaming kernel 84 / 158; 4096 x 4096 41 / 39 us, streaming 18 / 32; 2048 x 8192,
@@ -798,13 +827,15 @@ static int seq_linear_grouped_any(void* out, const void* x, const void* w, const
   }
   if (tile_rows == 16) {                   // a few rows in all (decoding): one 16-row output tile per workgroup, many workgroups
     DISPATCH_SEQ_DTYPE(dtype, {
-      if (stream_ok(x, w, N, K, epi, ext, sizeof(typename El<P>::type))) return launch_stream<P>(out, x, w, nullptr, 16, N, K, epi, st, ext, max_tiles);
+      constexpr int EB = sizeof(typename El<P>::type);
+      if (stream_ok(x, w, N, K, epi, ext, EB) && stream_pays_grouped(16, N, K, epi, EB)) return launch_stream<P>(out, x, w, nullptr, 16, N, K, epi, st, ext, max_tiles);
       if (K % 8 == 0 && gs % 8 == 0) return launch_tt<P, 1, 1, true>(out, x, w, nullptr, 16, N, K, epi, st, ext, max_tiles);
       return launch_tt<P, 1, 1, false>(out, x, w, nullptr, 16, N, K, epi, st, ext, max_tiles);
     })
   }
   DISPATCH_SEQ_DTYPE(dtype, {
-    if (stream_ok(x, w, N, K, epi, ext, sizeof(typename El<P>::type))) return launch_stream<P>(out, x, w, nullptr, 64, N, K, epi, st, ext, max_tiles);
+    constexpr int EB = sizeof(typename El<P>::type);
+    if (stream_ok(x, w, N, K, epi, ext, EB) && stream_pays_grouped(64, N, K, epi, EB)) return launch_stream<P>(out, x, w, nullptr, 64, N, K, epi, st, ext, max_tiles);
     if (K % 8 == 0 && gs % 8 == 0) {
       if (N >= 64 && sizeof(typename El<P>::type) == 2) return launch_tt<P, 4, 4, true>(out, x, w, nullptr, 64, N, K, epi, st, ext, max_tiles);
       return launch_tt<P, 1, 4, true>(out, x, w, nullptr, 64, N, K, epi, st, ext, max_tiles);

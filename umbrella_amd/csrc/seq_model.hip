@@ -142,6 +142,17 @@ static inline bool lin_step_ok(const float* v, int ldv, const float* state, int 
   return Dv % 4 == 0 && ldv % 4 == 0 && ((uintptr_t)v | (uintptr_t)state) % 16 == 0;
 }
 
+// Whether a step's gated linear attention runs in chunks: from three whole chunks on, where their time is the lesser one.  Token by token it
+// is the longest stretch's serial walk or all rows' share of the chip; in chunks every stretch, however short, is a chunk of full cost per
+// head, and the grid has the longest stretch's chunks for each of them (both fitted, us, one MI355X).  Token by token / in chunks, heads x
+// keys x values 8 x 128 x 256: 192 tokens 68 / 47, 2000 654 / 95, 8 stretches of 200 155 / 104, one of 192 beside 15 single tokens 72 / 113 (16 heads
+// 76 / 187), 300 beside 20 of 20 111 / 148; 32 x 64 x 64: 192 52 / 33, 192 beside 15 of 100 77 / 120, 32 of 192 207 / 290.
+static inline bool gla_chunks_pay(int T, int B, int max_len, int H, int D, int Dv) {
+  const double serial = max_len * (0.17 + 0.0013 * D), rows = 3.4e-7 * T * H * (double)D * Dv;
+  const double chunks = 30 + 1e-5 * (T / 64 + B) * H * (double)D * Dv + 5e-4 * ((max_len + 63) / 64) * (double)B * H * D;
+  return max_len >= 192 && chunks < (serial > rows ? serial : rows);
+}
+
 // softmax attention with a distance bias beside a state-space layer; both read the projection of the same input and write
 // their halves of the row that the one output projection reads: [scale_a * attention | scale_b * state space]
 static int mix_attn_ssd(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWork* ws, const UmbSeqStep* s, hipStream_t st) {
@@ -382,9 +393,8 @@ static int run_mixer(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWo
     // aux: decays (their logarithms) [T][HD] | scratch of the chunked form
     float* spare = ws->aux + al4((long)T * HD);
     const long spare_floats = ws->aux_floats - (long)(spare - ws->aux), need = umb_gla_scan_chunked_floats(T, s->B, H, D, Dv);
-    // stretches of three chunks and more side by side, where the shape is covered (8 heads x 128 x 256: 128 tokens 44 us, token by token 45;
-    // 192 tokens 45 / 66; sixteen stretches of 96 134 / 127)
-    const bool chunked = s->max_len >= 192 && need > 0 && need <= spare_floats && (long)s->B * H <= 65535 && ld % 4 == 0;
+    const bool chunked = need > 0 && need <= spare_floats && (long)s->B * H <= 65535 && ld % 4 == 0 &&
+                         gla_chunks_pay(T, s->B, s->max_len, H, D, Dv);
     SEQ_TRY((chunked ? umb_gla_decay_log : umb_gla_decay)(ws->aux, ws->proj, ld, 2 * HD + 2 * H * Dv, ly.a2.w, ly.a2.bias, T, HD, ly.rank, ly.tau,
                                                           dt, st));
     if (chunked)

@@ -209,13 +209,15 @@ def test_epilogues_of_linears(dtype, T, N, K):
         assert bool((act[T] == 7.0).all())
 
 
-# rows in quads: every workgroup size (64 ... 1024 threads, two quads a thread), a group that ends inside the last wave, several groups
+# rows in quads: every workgroup size (64 ... 1024 threads, up to four quads a thread where rows are many), a group that ends inside the last
+# wave, several groups; small groups of many rows, a wave each
+@pytest.mark.parametrize("T", [3, 402])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("W,groups", [(8, 1), (200, 1), (1024, 2), (1200, 1), (3072, 3), (2052, 1), (4096, 1), (4100, 1), (8192, 1)])
-def test_norms_in_quads(dtype, W, groups):
+@pytest.mark.parametrize("W,groups", [(192, 3), (8, 1), (200, 1), (1024, 2), (1200, 1), (3072, 3), (2052, 1), (4096, 1), (4100, 1), (8192, 1)])
+def test_norms_in_quads(dtype, W, groups, T):
     from umbrella_amd import _lib
     g = torch.Generator(device="cuda").manual_seed(W + groups)
-    T, eps, code = 3, 1e-5, _lib.seq_dtype_code(dtype)
+    eps, code = 1e-5, _lib.seq_dtype_code(dtype)
     x, y, y2 = (torch.randn(T, W, generator=g, device="cuda") * s for s in (3.0, 50.0, 0.2))
     w1, w2, w3, w4 = ((1 + 0.2 * torch.randn(W, generator=g, device="cuda")).to(dtype) for _ in range(4))
 
@@ -234,9 +236,9 @@ def test_norms_in_quads(dtype, W, groups):
     new = x.double() + norm(y, w1)
     assert close(xd, new) and close(h[:T], norm(new, w2), unit + 2.0 ** -18) and bool((h[T] == 7.0).all())
     table = torch.randn(11, W, generator=g, device="cuda").to(dtype)
-    ids = torch.tensor([4, 99, -1], dtype=torch.int32, device="cuda")
+    ids = torch.tensor([4, 99, -1] * (T // 3), dtype=torch.int32, device="cuda")
     _lib.seq_call("umb_seq_embed_norm", xd, h, table, ids, 1.5, w2, T, W, 11, groups, eps, code)
-    rows = table.double()[[4, 10, 0]] * 1.5
+    rows = table.double()[[4, 10, 0] * (T // 3)] * 1.5
     assert close(xd, rows) and close(h[:T], norm(rows, w2), unit)
     xd = x.clone()
     _lib.seq_call("umb_seq_pair_resid_norm", xd, h, y, y2, w1, w2, 0.5, w3, w4, T, W, eps, code)
@@ -258,7 +260,8 @@ def test_scale_of_a_normed_row(W):
     g = torch.Generator(device="cuda").manual_seed(W)
     T = 4000
     x, w, h = 3 * torch.randn(T, W, generator=g, device="cuda"), torch.ones(W, device="cuda"), torch.empty(T, W, device="cuda")
-    _lib.seq_call("umb_seq_group_norm", h, None, x, None, w, T, W, 1, 1e-6, _lib.seq_dtype_code(torch.float32))
+    for lo, n in [(200 * i, 200) for i in range(15)] + [(3000, 1000)]:          # launches of few rows and of many
+        _lib.seq_call("umb_seq_group_norm", h[lo:], None, x[lo:], None, w, n, W, 1, 1e-6, _lib.seq_dtype_code(torch.float32))
     v = x.double()
     want = v / (v.pow(2).mean(-1, keepdim=True) + 1e-6).sqrt()
     err = (h.double() * want).sum(-1) / want.pow(2).sum(-1) - 1

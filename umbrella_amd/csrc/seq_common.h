@@ -87,15 +87,27 @@ template <int NT> __device__ __forceinline__ float row_sum(float v, float* red /
 static inline bool quads_ok(int W, int groups, const void* a, const void* b = nullptr, const void* c = nullptr, const void* d = nullptr,
                             const void* e = nullptr, const void* f = nullptr, const void* g = nullptr) {
   const int gs = W / groups;
-  return gs % 4 == 0 && gs <= 8192 &&
+  return gs % 4 == 0 && gs <= 8192 && groups <= 65535 &&
          ((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d | (uintptr_t)e | (uintptr_t)f | (uintptr_t)g) % 16 == 0;
 }
-#define BY_QUADS(gs, LAUNCH)              \
+// Groups of at most 64 elements leave three quarters of a wave idle, which shows once there are a few workgroups per unit: a wave per group
+// there (2000 x 3 x 64: embedding 3.3 us, 3.7 in quads, final norm 3.1 / 3.4)
+static inline bool quads_fill(int gs, long rows) { return gs > 64 || rows < 1024; }
+// Rows beyond 1024 elements: one quad a thread where rows are few; from 400 rows on the chip is full either way and two or four quads a thread let
+// several rows share a compute unit, one's loads behind another's sums (us, 4-byte elements by 256 threads / one quad / these: pair seam
+// 700 x 3072 10.0 / 11.4 / 8.6, seam 2000 x 4096 27.5 / 21.1 / 19.7, one-stream seam 2000 x 4096 19.3 / 20.4 / 19.6, embedding 2000 x 3072 11.5 /
+// 12.9 / 11.4; 256 rows: one quad is ahead or equal).
+constexpr long QUAD_ROWS = 400;
+#define BY_QUADS(gs, rows, LAUNCH)        \
   do {                                    \
     if ((gs) <= 256) LAUNCH(64, 1);       \
     else if ((gs) <= 512) LAUNCH(128, 1); \
     else if ((gs) <= 1024) LAUNCH(256, 1); \
-    else if ((gs) <= 2048) LAUNCH(512, 1); \
+    else if ((rows) >= QUAD_ROWS) {       \
+      if ((gs) <= 2048) LAUNCH(256, 2);   \
+      else if ((gs) <= 4096) LAUNCH(256, 4); \
+      else LAUNCH(512, 4);                \
+    } else if ((gs) <= 2048) LAUNCH(512, 1); \
     else if ((gs) <= 4096) LAUNCH(1024, 1); \
     else LAUNCH(1024, 2);                 \
   } while (0)

@@ -299,7 +299,7 @@ extern "C" int umb_hc_embed(float* x, void* h, const void* embed, const int* tok
 #define HC_EMBED_QUADS(NT, NE)                                                                                                          \
   hipLaunchKernelGGL((hc_embed_quad_kernel<P, NT, NE>), dim3(T), dim3(NT), 0, st, x, (E*)h, (const E*)embed, tokens, scale, in, (const E*)w, offset, W, \
                      V, eps)
-    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, HC_EMBED_QUADS); })
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, (long)T, HC_EMBED_QUADS); })
 #undef HC_EMBED_QUADS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
@@ -343,7 +343,7 @@ extern "C" int umb_hc_seam(float* x, void* h, const float* y, const float* mix, 
   if (S == 1 && quads_ok(W, 1, x, h, y, w_next)) {
 #define HC_SEAM_QUADS(NT, NE)                                                                                                       \
   hipLaunchKernelGGL((hc_seam_quad_kernel<P, NT, NE>), dim3(T), dim3(NT), 0, st, x, (E*)h, y, mix, out, m, in_next, (const E*)w_next, offset, W, eps)
-    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, HC_SEAM_QUADS); })
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, (long)T, HC_SEAM_QUADS); })
 #undef HC_SEAM_QUADS
     UMB_LAUNCH_CHECK();
     return UMB_OK;

@@ -453,11 +453,11 @@ extern "C" int umb_seq_group_norm(float* out_f32, void* out_dt, const float* x, 
                                   int groups, float eps, int dtype, hipStream_t st) {
   if (!norm_args_ok(T, W, groups) || !x || !w || (!out_f32 && !out_dt)) return UMB_EINVAL;
   const int gs = W / groups;
-  if (quads_ok(W, groups, out_f32, out_dt, x, w)) {
+  if (quads_ok(W, groups, out_f32, out_dt, x, w) && quads_fill(gs, (long)T * groups)) {
 #define NORM_QUADS(NT, NE)                                                                                                               \
   hipLaunchKernelGGL((norm_quad_kernel<P, NT, NE, false>), dim3(T, groups), dim3(NT), 0, st, out_f32, (E*)out_dt, x, rows, (const E*)nullptr, \
                      0, 1.f, (const E*)w, W, groups, eps)
-    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(gs, NORM_QUADS); })
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(gs, (long)T * groups, NORM_QUADS); })
 #undef NORM_QUADS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
@@ -481,11 +481,11 @@ extern "C" int umb_seq_group_norm(float* out_f32, void* out_dt, const float* x, 
 extern "C" int umb_seq_embed_norm(float* x, void* h, const void* embed, const int* tokens, float scale, const void* w, int T, int W,
                                   int V, int groups, float eps, int dtype, hipStream_t st) {
   if (!norm_args_ok(T, W, groups) || !x || !h || !embed || !tokens || !w || V < 1) return UMB_EINVAL;
-  if (quads_ok(W, groups, x, h, embed, w)) {
+  if (quads_ok(W, groups, x, h, embed, w) && quads_fill(W / groups, (long)T * groups)) {
 #define EMBED_QUADS(NT, NE)                                                                                                            \
   hipLaunchKernelGGL((norm_quad_kernel<P, NT, NE, true>), dim3(T, groups), dim3(NT), 0, st, x, (E*)h, (const float*)nullptr, tokens, (const E*)embed, \
                      V, scale, (const E*)w, W, groups, eps)
-    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W / groups, EMBED_QUADS); })
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W / groups, (long)T * groups, EMBED_QUADS); })
 #undef EMBED_QUADS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
@@ -506,7 +506,7 @@ extern "C" int umb_seq_resid_norm(float* x, void* h, const float* y, const void*
 #define SEAM_QUADS(NT, NE)                                                                                                      \
   hipLaunchKernelGGL((resid_norm_quad_kernel<P, NT, NE>), dim3(T, groups), dim3(NT), 0, st, x, (E*)h, y, (const E*)w_post, (const E*)w_next, \
                      W, groups, eps)
-    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W / groups, SEAM_QUADS); })
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W / groups, (long)T * groups, SEAM_QUADS); })
 #undef SEAM_QUADS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
@@ -572,7 +572,7 @@ extern "C" int umb_seq_pair_resid_norm(float* x, void* h, const float* y1, const
 #define PAIR_QUADS(NT, NE)                                                                                                          \
   hipLaunchKernelGGL((pair_resid_norm_quad_kernel<P, NT, NE>), dim3(T), dim3(NT), 0, st, x, (E*)h, y1, y2, (const E*)w1, (const E*)w2, coef, \
                      (const E*)w_post, (const E*)w_next, W, eps)
-    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, PAIR_QUADS); })
+    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, (long)T, PAIR_QUADS); })
 #undef PAIR_QUADS
     UMB_LAUNCH_CHECK();
     return UMB_OK;

@@ -665,6 +665,7 @@ static int bsa_launch(dim3 grid, size_t lds, hipStream_t st, void* out, int ldo,
 
 // the decode kernel: spans of ATT_SPAN keys dealt to several workgroups only where few items leave the chip idle; 16 waves per item as
 // long as every item gets a compute unit of its own (values of 256: their registers do not hold it), 8 while two share one, 4 beyond
+// (us with 8 / 4 waves, 32 + 8 heads of 128: 1024 items behind 30 / 200 keys 12.8 / 8.4, 30.2 / 27.5; 512 items behind 500 28.8 / 36.7)
 template <typename P>
 static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const float* bias,
                        int n_dist, const int* pos, const int* slot, int T, int H, int G, int D, int E, int window, float scale,
@@ -681,7 +682,7 @@ static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv,
     if (nsplit > (most + ATT_SPAN - 1) / ATT_SPAN) nsplit = (int)((most + ATT_SPAN - 1) / ATT_SPAN);
     while (nsplit > 1 && (long)T * H * maps * nsplit * (E + 2) > scratch_floats) nsplit >>= 1;
   }
-  const int nw = items <= 256 && E < 256 ? 16 : (items <= 1024 ? 8 : 4);
+  const int nw = items <= 256 && E < 256 ? 16 : (items <= 512 ? 8 : 4);
   const size_t lds = ((size_t)rh * D + (size_t)nw * rh * E + (size_t)(nw + 1) * rh * 2) * sizeof(float);
 #define ATT_GO(RH, LPR, NW, MAPS)                                                                                                     \
   do {                                                                                                                               \

@@ -757,10 +757,11 @@ extern "C" int umb_pwa_attend(void* out, const float* q, const UmbPagedKV* kv, c
     return UMB_EINVAL;
   const int R = H / G;
   if (decode_rows_ok(D, D, dtype, kv)) {
-    // 16 waves per item as long as every item gets a compute unit of its own, 8 while two share one, 4 beyond
+    // 16 waves per item as long as every item gets a compute unit of its own, 8 while two share one, 4 beyond (us with 8 / 4 waves, 32 + 8 heads of
+    // 64: 1024 items behind 30 / 200 keys 12.7 / 7.8, 24.9 / 20.1, 768 behind 200 19.1 / 12.9; 512 items of 128 behind 500 25.4 / 30.0)
     const int rh = R % 4 == 0 ? 4 : (R % 2 == 0 ? 2 : 1);
     const long items = (long)T * (H / rh);
-    const int nw = items <= 256 ? 16 : (items <= 1024 ? 8 : 4);
+    const int nw = items <= 256 ? 16 : (items <= 512 ? 8 : 4);
     const size_t lds = (size_t)nw * rh * D * sizeof(float);
 #define PWD_GO(RH, LPR, NW)                                                                                                     \
   do {                                                                                                                          \

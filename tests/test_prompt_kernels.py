@@ -680,7 +680,12 @@ def _stretches(lens, news):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H,G,D,E,maps,window,chunk,keep,extra", [
     (8, 2, 64, 64, 1, 2 ** 30, 0, 0, False), (6, 1, 64, 64, 1, 70, 0, 5, True), (4, 1, 128, 128, 1, 90, 0, 40, True), (12, 2, 128, 128, 1, 2 ** 30, 64, 0, False),
-    (4, 2, 64, 128, 2, 2 ** 30, 50, 0, False), (2, 1, 128, 256, 2, 100, 0, 3, True), (3, 1, 72, 48, 1, 60, 0, 0, True)])
+    (4, 2, 64, 128, 2, 2 ** 30, 50, 0, False), (2, 1, 128, 256, 2, 100, 0, 3, True), (3, 1, 72, 48, 1, 60, 0, 0, True),
+    # every count of 32-feature steps and 16-column tiles, whole and not, each direction first to overflow its size; more heads than a workgroup has waves
+    (8, 1, 96, 96, 1, 2 ** 30, 0, 0, False), (5, 1, 80, 32, 1, 50, 0, 2, True), (2, 2, 16, 112, 1, 70, 0, 0, False), (6, 1, 104, 128, 1, 2 ** 30, 30, 0, True),
+    (2, 1, 192, 192, 1, 40, 0, 0, True), (3, 1, 136, 48, 1, 2 ** 30, 0, 0, False), (1, 1, 256, 256, 1, 2 ** 30, 0, 0, True), (2, 1, 24, 208, 1, 60, 0, 0, False),
+    (2, 1, 40, 48, 2, 2 ** 30, 0, 0, True), (2, 2, 128, 128, 2, 60, 0, 0, False), (1, 1, 72, 144, 2, 2 ** 30, 0, 0, True), (2, 1, 160, 160, 2, 2 ** 30, 40, 0, False),
+    (1, 1, 256, 256, 2, 80, 0, 5, True)])
 def test_prompt_attention(dtype, H, G, D, E, maps, window, chunk, keep, extra):
     from umbrella_amd import _lib
     code = _lib.seq_dtype_code(dtype)
@@ -708,7 +713,8 @@ def test_prompt_attention(dtype, H, G, D, E, maps, window, chunk, keep, extra):
         if chunk:
             see &= j // chunk == i // chunk
         see = (see | (j < keep)) & (j <= i)
-        s = torch.einsum("thmd,jhmd->thmj", q[r0:r0 + k].double().cpu(), kk.cpu()).cuda() * scale
+        s, s_size = (torch.einsum("thmd,jhmd->thmj", x.cpu(), y.cpu()).cuda() * scale for x, y in
+                     ((q[r0:r0 + k].double(), kk), (q[r0:r0 + k].double().abs(), kk.abs())))
         if cap:
             s = cap * torch.tanh(s / cap)
         if extra:
@@ -718,15 +724,24 @@ def test_prompt_attention(dtype, H, G, D, E, maps, window, chunk, keep, extra):
             p = torch.softmax(torch.cat([s, sink.double()[None, :, None, None].expand(k, H, maps, 1)], -1), -1)[..., :-1]
         else:
             p = torch.softmax(s, -1)
-        o = torch.einsum("thmj,jhe->thme", p.cpu(), vv.cpu()).cuda()
+        # o = sum p v, p a quotient of weights: a score's error counts twice, a weight's split once.  A split keeps 2^-17 (bf16) or 2^-22 (fp16) of
+        # its number, an fp32 sum of D products D 2^-24 of their size, base-2 scores within 20 round to 2^-20; fp16 weights next to zero lose 2^-25
+        split = 2.0 ** (-17 if dtype == torch.bfloat16 else -22)
+        s_err = (split + D * 2.0 ** -24) * s_size.masked_fill(~see[:, None, None], 0.0).amax(-1) + 2.0 ** -20
+        rel, lost = 2 * s_err + split + 2.0 ** -20, 0.0 if dtype == torch.bfloat16 else 2.0 ** -25
+        o, size = (torch.einsum("thmj,jhe->thme", p.cpu(), v.cpu()).cuda() for v in (vv, vv.abs()))
+        gone = lost * torch.einsum("tj,jhe->the", see.double(), vv.abs().contiguous())[:, :, None]
+        o_err = rel[..., None] * size + gone
         if maps == 2:
-            o = o[:, :, 0] - lam * o[:, :, 1]
-            o = o / torch.sqrt(o.pow(2).mean(-1, keepdim=True) + eps)
+            o, o_err = o[:, :, 0] - lam * o[:, :, 1], o_err[:, :, 0] + lam * o_err[:, :, 1]
+            rms = torch.sqrt(o.pow(2).mean(-1, keepdim=True) + eps)
+            o = o / rms
+            o_err = o_err / rms + o.abs() * torch.sqrt(o_err.pow(2).mean(-1, keepdim=True)) / rms
         else:
-            o = o[:, :, 0]
-        o = 1.25 * o * (torch.sigmoid(gate[r0:r0 + k].double())[..., None] if extra else 1.0)
-        # storage rounding; queries and weights split to 2^-17 each (bf16; 2^-22 in fp16), scores of up to 7: 1e-4 of the largest output
-        tol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * o.abs() + 2e-4 * o.abs().max() + 1e-6
+            o, o_err = o[:, :, 0], o_err[:, :, 0]
+        f = 1.25 * (torch.sigmoid(gate[r0:r0 + k].double())[..., None] if extra else 1.0)
+        o, o_err = o * f, o_err * f
+        tol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * o.abs() + o_err + 2.0 ** -20 * o.abs() + 2.0 ** -25
         err = (out[r0:r0 + k, :H * E].double().view(k, H, E) - o).abs()
         assert bool((err <= tol).all()), (b, float(err.max()))
 

@@ -803,8 +803,7 @@ extern "C" int umb_bsa_attend(void* out, int ldo, const float* q, const UmbPaged
 }
 
 // ---- prompt attention on the matrix pipe (16-bit storage; D a multiple of 8, E a multiple of 16).
-// Workgroup = (16 consecutive positions of one sequence, one key/value head, a block of 4 HPW of its query heads); wave w owns
-// HPW heads.  The tile's keys -- from the first position's window start to the last position -- are walked in steps of 32 by
+// Workgroup = (16 consecutive positions of one sequence, one key/value head, four of its query heads), a wave per head.  The tile's keys -- from the first position's window start to the last position -- are walked in steps of 32 by
 // the whole workgroup: the step's 32 cached key rows and value rows are staged ONCE into LDS (keys as cached: the A operand of
 // S^T = K Q^T; values transposed: the A operand of O^T += V^T P^T) and serve every head of the workgroup; the next step's rows
 // are in flight in registers while the current one is used.  Per step and head: two 16-key score tiles; the bias of the
@@ -812,9 +811,13 @@ extern "C" int umb_bsa_attend(void* out, int ldo, const float* q, const UmbPaged
 // exponents, accumulators rescaled only when a maximum moved; the lane's eight weights ARE its share of the B operand of the
 // value product.  Scores and weights keep fp32 accuracy on the 16-bit pipe: the fp32 queries and the fp32 weights enter as
 // high + low 16-bit halves (two products each, 2^-17 relative).
-// NSM / NVM bound the unrolled register arrays; EXACT: they are the counts (the sizes that are used in earnest).  With run-time counts every
-// product stood in a block of its own behind its own LDS read; with a whole step's reads free to move ahead, and steps that every query sees
-// whole left untested, 1999 positions, 32 + 8 heads of 128 went from 212 us to 140, two maps over 617 positions, 64 | 128, from 104 to 71.
+// Products per step at compile time: NSM steps of 32 features and NVM tiles of 16 columns, the least of a few sizes that hold D and E, with zeros
+// behind a key row's D columns.  With run-time counts every product stood in a block of its own behind its own LDS read; with a whole step's
+// reads free to move ahead, and steps that every query sees whole left untested, 1999 positions, 32 + 8 heads of 128 went from 212 us to 140, two
+// maps over 617 positions, 64 | 128, from 104 to 71.  FULL: D and E fill them, staging then tests nothing (2000 positions of 128: 158 us,
+// 162 without).  us, run-time / these counts, 2000 positions: heads of 96 86 / 75, of 112 242 / 202, of 256 216 / 156, two maps of 128 | 128 273 / 179.
+// Two heads a wave, sharing the value fragments, are behind wherever a launch is not several rounds of workgroups: 600 positions, 64 + 8 heads
+// of 128 67 against 55, of 64 42 / 35 (2000 positions 195 / 198, 134 / 121).
 constexpr float BSA_LOG2E = 1.4426950408889634f;
 
 template <typename P> __device__ __forceinline__ void split2(float a, float b, unsigned& hi, unsigned& lo) {
@@ -822,9 +825,13 @@ template <typename P> __device__ __forceinline__ void split2(float a, float b, u
   lo = pack2<P>(a - lo_f<P>(hi), b - hi_f<P>(hi));
 }
 
-// HPW rows per wave = HPW / MAPS heads with MAPS maps each; every map has its part of the staged key rows, the value fragments of
-// a step serve all rows
-template <typename P, int NSM, int NVM, int HPW, int MAPS, bool EXACT>
+// MAPS rows per wave, the maps of its head; every map has its part of the staged key rows, the value fragments of a step serve both
+template <int NSM, int NVM, int MAPS> struct BsaTile {
+  static constexpr int KD = NSM * 32, LD = MAPS * KD + 8;       // a map's part of a staged key row; row stride: 16 bytes of padding spread the banks
+  static constexpr int LT = 36;                                 // row stride of the transposed value tile: 32 keys + 8 bytes of padding
+  static constexpr size_t LDS = ((size_t)32 * LD + (size_t)NVM * 16 * LT) * sizeof(u16);
+};
+template <typename P, int NSM, int NVM, int MAPS, bool FULL>
 __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q,
                                                               UmbPagedKV kv, const float* __restrict__ proj, int ld, int gate_col,
                                                               const float* __restrict__ bias, int n_dist,
@@ -833,16 +840,15 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
                                                               int H, int G, int D, int E, int window, float scale, float out_scale,
                                                               float softcap, UmbAttnForm form) {
   extern __shared__ __attribute__((aligned(16))) u16 bsa_lds[];
-  if constexpr (EXACT) { D = NSM * 32; E = NVM * 16; }      // the counts as constants
-  static_assert(HPW % MAPS == 0, "a wave owns whole heads");
-  constexpr int HW = HPW / MAPS;                      // heads per wave
+  typedef BsaTile<NSM, NVM, MAPS> Tile;
+  if constexpr (FULL) { D = NSM * 32; E = NVM * 16; }
+  constexpr int HPW = MAPS;                           // rows of scores per wave
   constexpr int NLK = (NSM * 4 * MAPS + 7) / 8, NLV = (NVM * 2 + 7) / 8;     // 16-byte chunks of a key / value row per staging thread
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
-  const int DK = MAPS * D, LD = DK + 8;               // LDS row stride of the key tile: 16 bytes of padding spread the banks
-  const int ns = (D + 31) >> 5, nv = E >> 4, nck = DK >> 3, ncv = E >> 3;
-  constexpr int LT = 36;                              // row stride of the transposed value tile: 32 keys + 8 bytes of padding
-  u16* k_s = bsa_lds;                                 // [32][LD]
-  u16* v_t = bsa_lds + 32 * LD;                       // [E][LT]
+  constexpr int KD = Tile::KD, LD = Tile::LD, LT = Tile::LT;
+  const int DK = MAPS * D, nv = E >> 4, nck = DK >> 3, ncv = E >> 3;
+  u16* k_s = bsa_lds;                                 // [32][LD], zero past a map's D columns
+  u16* v_t = bsa_lds + 32 * LD;                       // [16 NVM][LT], rows past E as they are: they reach columns that are not stored
   const int b = blockIdx.y;
   // How many keys a tile sees depends on its place in the chunk (or, without a window, in the sequence).  Workgroups that share a CU
   // are about 256 apart in launch order, which is the same tile of another head block: every other run of 256 takes the tiles from the
@@ -851,10 +857,10 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
   const int tile = (row / run) & 1 ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x;
   const int n = seq_len[b], q0 = tile * 16;
   if (q0 >= n) return;                                // the whole workgroup
-  const int hpg = H / G, hblocks = (hpg + 4 * HW - 1) / (4 * HW);
+  const int hpg = H / G, hblocks = (hpg + 3) / 4;
   const int g = blockIdx.z / hblocks;
-  const int hl0 = ((blockIdx.z % hblocks) * 4 + wave) * HW;         // first of the wave's heads inside the group
-  const bool active = hl0 < hpg;                      // a wave without heads still stages rows and meets the barriers
+  const int hl = blockIdx.z % hblocks * 4 + wave;     // the wave's head inside the group
+  const bool active = hl < hpg;                       // a wave without one still stages rows and meets the barriers
   const int slot = seq_slot[b], row0 = seq_row0[b], pos0 = seq_pos0[b];
   const int nq = n - q0 < 16 ? n - q0 : 16;
   const int i_first = pos0 + q0, i_last = i_first + nq - 1;
@@ -877,19 +883,16 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
   u32x4 qh[HPW][NSM], ql[HPW][NSM];
   f32x4 o[HPW][NVM];
   float m_run[HPW], l_run[HPW];
-  bool h_ok[HPW];
-  int hd[HPW];
+  const int hd = g * hpg + (active ? hl : hpg - 1);
 #pragma unroll
   for (int hh = 0; hh < HPW; ++hh) {
-    h_ok[hh] = hl0 + hh / MAPS < hpg;
-    hd[hh] = g * hpg + (h_ok[hh] ? hl0 + hh / MAPS : hpg - 1);
-    const float* qr = q + ((qrow * H + hd[hh]) * MAPS + hh % MAPS) * D;
+    const float* qr = q + ((qrow * H + hd) * MAPS + hh) * D;
 #pragma unroll
     for (int s = 0; s < NSM; ++s) {
       const int d = 32 * s + 8 * g4;
       qh[hh][s] = u32x4{0u, 0u, 0u, 0u};
       ql[hh][s] = u32x4{0u, 0u, 0u, 0u};
-      if (s < ns && d < D) {
+      if (d < D) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(qr + d), c = *reinterpret_cast<const f32x4*>(qr + d + 4);
         unsigned hi[4], lo[4];
         split2<P>(a[0], a[1], hi[0], lo[0]);
@@ -926,13 +929,15 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     }
   };
   fetch(0);
-  if (threadIdx.x < 32) *reinterpret_cast<u32x4*>(k_s + threadIdx.x * LD + DK) = u32x4{0u, 0u, 0u, 0u};       // read where a step of 32 runs past D
+  const int pad = (KD - D) >> 3;                      // 16-byte chunks a map's part is short of its steps
+  for (int x = threadIdx.x; x < 32 * MAPS * pad; x += 256)
+    *reinterpret_cast<u32x4*>(k_s + (x & 31) * LD + (x >> 5) / pad * KD + D + 8 * ((x >> 5) % pad)) = u32x4{0u, 0u, 0u, 0u};
   for (int base = 0; base < total; base += 32) {
     __syncthreads();                                  // every wave is done with the previous tile
 #pragma unroll
     for (int u = 0; u < NLK; ++u) {
       const int ch = sc + 8 * u;
-      if (ch < nck) *reinterpret_cast<u32x4*>(k_s + sm * LD + 8 * ch) = stk[u];
+      if (ch < nck) *reinterpret_cast<u32x4*>(k_s + sm * LD + 8 * ch + (MAPS == 2 && 8 * ch >= D ? KD - D : 0)) = stk[u];
     }
 #pragma unroll
     for (int u = 0; u < NLV; ++u) {
@@ -951,14 +956,13 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     // which of the lane's eight keys this query sees, and at what distance: the same for every head
     // (a step that every query sees whole needs no tests: rows past the last are not stored)
     const bool whole = base >= kept && j_off + base + 31 <= i_first && j_off + base >= lo_all;
-    float bv[HPW][8];
+    float bv[8];
     if (bias) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int kx = base + 16 * (e >> 2) + 4 * g4 + (e & 3);
         const int dd = i_j - (kx < kept ? kx : j_off + kx), di = dd < 0 ? 0 : (dd < n_dist ? dd : n_dist - 1);
-#pragma unroll
-        for (int hh = 0; hh < HPW; ++hh) bv[hh][e] = bias[(long)hd[hh] * n_dist + di];
+        bv[e] = bias[(long)hd * n_dist + di];
       }
     }
     f32x4 sc2[HPW][2];
@@ -969,17 +973,11 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
       const u16* kr = k_s + (16 * u + j) * LD;
 #pragma unroll
       for (int s = 0; s < NSM; ++s) {
-        const int d = 32 * s + 8 * g4;
-        if (s < ns) {
 #pragma unroll
-          for (int mp = 0; mp < MAPS; ++mp) {
-            const u32x4 kf = *reinterpret_cast<const u32x4*>(kr + (d < D ? mp * D + d : DK));
-#pragma unroll
-            for (int hh = mp; hh < HPW; hh += MAPS) {
-              sc2[hh][u] = P::mfma(kf, ql[hh][s], sc2[hh][u]);
-              sc2[hh][u] = P::mfma(kf, qh[hh][s], sc2[hh][u]);
-            }
-          }
+        for (int mp = 0; mp < MAPS; ++mp) {
+          const u32x4 kf = *reinterpret_cast<const u32x4*>(kr + mp * KD + 32 * s + 8 * g4);
+          sc2[mp][u] = P::mfma(kf, ql[mp][s], sc2[mp][u]);
+          sc2[mp][u] = P::mfma(kf, qh[mp][s], sc2[mp][u]);
         }
       }
     }
@@ -995,7 +993,7 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
       }
       if (bias) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sv[e] += bv[hh][e] * BSA_LOG2E;
+        for (int e = 0; e < 8; ++e) sv[e] += bv[e] * BSA_LOG2E;
       }
       if (!whole) {
 #pragma unroll
@@ -1024,9 +1022,7 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
       m_run[hh] = m_new;
       if (__ballot(fac != 1.f)) {                                    // the maximum moved for some row of the tile
 #pragma unroll
-        for (int dt = 0; dt < NVM; ++dt) {
-          if (dt < nv) { o[hh][dt][0] *= fac; o[hh][dt][1] *= fac; o[hh][dt][2] *= fac; o[hh][dt][3] *= fac; }
-        }
+        for (int dt = 0; dt < NVM; ++dt) { o[hh][dt][0] *= fac; o[hh][dt][1] *= fac; o[hh][dt][2] *= fac; o[hh][dt][3] *= fac; }
       }
       unsigned hi[4], lo[4];
 #pragma unroll
@@ -1037,60 +1033,53 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     // O^T[d][query] += V^T[d][keys] P^T[keys][query]: lane (d row j of tile dt, quad g4) reads its 8 keys' values
 #pragma unroll
     for (int dt = 0; dt < NVM; ++dt) {
-      if (dt < nv) {
-        const u16* vr = v_t + (16 * dt + j) * LT + 4 * g4;
-        const u32x2 t0 = *reinterpret_cast<const u32x2*>(vr), t1 = *reinterpret_cast<const u32x2*>(vr + 16);
-        const u32x4 va = u32x4{t0[0], t0[1], t1[0], t1[1]};
+      const u16* vr = v_t + (16 * dt + j) * LT + 4 * g4;
+      const u32x2 t0 = *reinterpret_cast<const u32x2*>(vr), t1 = *reinterpret_cast<const u32x2*>(vr + 16);
+      const u32x4 va = u32x4{t0[0], t0[1], t1[0], t1[1]};
 #pragma unroll
-        for (int hh = 0; hh < HPW; ++hh) {
-          o[hh][dt] = P::mfma(va, pl[hh], o[hh][dt]);
-          o[hh][dt] = P::mfma(va, ph[hh], o[hh][dt]);
-        }
+      for (int hh = 0; hh < HPW; ++hh) {
+        o[hh][dt] = P::mfma(va, pl[hh], o[hh][dt]);
+        o[hh][dt] = P::mfma(va, ph[hh], o[hh][dt]);
       }
     }
   }
   // lane holds O^T[d = 16 dt + 4 g4 + rr][query j]
   if (q_ok && active) {
+    const bool gate_head = gate_col >= 0 && !form.gate_elem;
+    const float gt = gate_head ? 1.f / (1.f + expf(-proj[qrow * ld + gate_col + hd])) : 1.f;
+    const float* ge = gate_col >= 0 && form.gate_elem ? proj + qrow * ld + gate_col + (long)hd * E : nullptr;
+    float l[MAPS];
 #pragma unroll
-    for (int hh = 0; hh < HPW; hh += MAPS) {
-      if (!h_ok[hh]) continue;
-      const bool gate_head = gate_col >= 0 && !form.gate_elem;
-      const float gt = gate_head ? 1.f / (1.f + expf(-proj[qrow * ld + gate_col + hd[hh]])) : 1.f;
-      const float* ge = gate_col >= 0 && form.gate_elem ? proj + qrow * ld + gate_col + (long)hd[hh] * E : nullptr;
-      float l[MAPS];
-#pragma unroll
-      for (int mp = 0; mp < MAPS; ++mp)
-        l[mp] = l_run[hh + mp] + (form.sink ? __builtin_amdgcn_exp2f(form.sink[hd[hh]] * BSA_LOG2E - m_run[hh + mp]) : 0.f);
-      float inv = out_scale * gt / l[0];
-      if constexpr (MAPS == 2) {                      // o = a1 - lambda a2 over the root mean square of the head's E columns
-        const float i1 = 1.f / l[0], i2 = form.lambda / l[1];
-        float ss = 0.f;
-#pragma unroll
-        for (int dt = 0; dt < NVM; ++dt) {
-          if (dt < nv) {
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-              const float v = o[hh][dt][rr] * i1 - o[hh + 1][dt][rr] * i2;
-              o[hh][dt][rr] = v;
-              ss += v * v;
-            }
-          }
-        }
-        ss += __shfl_xor(ss, 16, 64);                 // the query's column quads: lanes j, j + 16, j + 32, j + 48 (all active)
-        ss += __shfl_xor(ss, 32, 64);
-        inv = out_scale * gt / sqrtf(ss / (float)E + form.eps);
-      }
-      u16* orow = out + qrow * ldo + (long)hd[hh] * E;
+    for (int mp = 0; mp < MAPS; ++mp) l[mp] = l_run[mp] + (form.sink ? __builtin_amdgcn_exp2f(form.sink[hd] * BSA_LOG2E - m_run[mp]) : 0.f);
+    float inv = out_scale * gt / l[0];
+    if constexpr (MAPS == 2) {                        // o = a1 - lambda a2 over the root mean square of the head's E columns
+      const float i1 = 1.f / l[0], i2 = form.lambda / l[1];
+      float ss = 0.f;
 #pragma unroll
       for (int dt = 0; dt < NVM; ++dt) {
         if (dt < nv) {
 #pragma unroll
           for (int rr = 0; rr < 4; ++rr) {
-            const int d = 16 * dt + 4 * g4 + rr;
-            float v = o[hh][dt][rr] * inv;
-            if (ge) v /= 1.f + expf(-ge[d]);
-            orow[d] = P::from_f(v);
+            const float v = o[0][dt][rr] * i1 - o[1][dt][rr] * i2;
+            o[0][dt][rr] = v;
+            ss += v * v;
           }
+        }
+      }
+      ss += __shfl_xor(ss, 16, 64);                   // the query's column quads: lanes j, j + 16, j + 32, j + 48 (all active)
+      ss += __shfl_xor(ss, 32, 64);
+      inv = out_scale * gt / sqrtf(ss / (float)E + form.eps);
+    }
+    u16* orow = out + qrow * ldo + (long)hd * E;
+#pragma unroll
+    for (int dt = 0; dt < NVM; ++dt) {
+      if (dt < nv) {
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) {
+          const int d = 16 * dt + 4 * g4 + rr;
+          float v = o[0][dt][rr] * inv;
+          if (ge) v /= 1.f + expf(-ge[d]);
+          orow[d] = P::from_f(v);
         }
       }
     }
@@ -1114,31 +1103,34 @@ extern "C" int umb_attn_attend_tiled(void* out, int ldo, const float* q, const U
   const UmbAttnForm form = form_ ? *form_ : UmbAttnForm{1, 0, nullptr, 0.f, 0.f, 0, 0};
   if (gate_col >= 0 && (!proj || ld < gate_col + form_gate_cols(form, H, E))) return UMB_EINVAL;
   const int hpg = H / G, maps = form.maps;
-  const size_t lds = ((size_t)32 * (maps * D + 8) + (size_t)E * 36) * sizeof(u16);
-#define BSA_MFMA(NSM, NVM, HPW, MAPS, EX)                                                                                  \
+#define BSA_MFMA_AS(NSM, NVM, MAPS, FULL)                                                                               \
   do {                                                                                                                     \
-    const int hblocks = (hpg + 4 * (HPW / MAPS) - 1) / (4 * (HPW / MAPS));                                                 \
+    const int hblocks = (hpg + 3) / 4;                                                                                     \
     if ((long)G * hblocks > 65535) return UMB_EINVAL;                                                                      \
     const dim3 grid((max_len + 15) / 16, B, G * hblocks);                                                                  \
-    if (ensure_dynamic_lds<bsa_attend_mfma_kernel<P, NSM, NVM, HPW, MAPS, EX>>(lds) != UMB_OK) return UMB_EHIP;                \
-    hipLaunchKernelGGL((bsa_attend_mfma_kernel<P, NSM, NVM, HPW, MAPS, EX>), grid, dim3(256), lds, st, (u16*)out, ldo, q, *kv, \
+    constexpr size_t lds = BsaTile<NSM, NVM, MAPS>::LDS;                                                                   \
+    if (ensure_dynamic_lds<bsa_attend_mfma_kernel<P, NSM, NVM, MAPS, FULL>>(lds) != UMB_OK) return UMB_EHIP;          \
+    hipLaunchKernelGGL((bsa_attend_mfma_kernel<P, NSM, NVM, MAPS, FULL>), grid, dim3(256), lds, st, (u16*)out, ldo, q, *kv, \
                        proj, ld, gate_col, bias, n_dist, seq_slot, seq_row0, seq_pos0, seq_len, H, G, D, E, window, scale, \
                        out_scale, softcap, form);                                                                          \
   } while (0)
+#define BSA_MFMA(NSM, NVM, MAPS)                                                                                      \
+  do { if (D == 32 * NSM && E == 16 * NVM) BSA_MFMA_AS(NSM, NVM, MAPS, true); else BSA_MFMA_AS(NSM, NVM, MAPS, false); } while (0)
 #define BSA_MFMA_SHAPE()                                                                                                   \
   if (maps == 2) {                                                                                                         \
-    if (D == 64 && E == 128) BSA_MFMA(2, 8, 2, 2, true);                                                                   \
-    else if (D == 128 && E == 256) BSA_MFMA(4, 16, 2, 2, true);                                                            \
-    else if (D <= 128 && E <= 128) BSA_MFMA(4, 8, 2, 2, false);                                                            \
-    else BSA_MFMA(8, 16, 2, 2, false);                                                                                     \
-  } else if (D == 64 && E == 64) { if (hpg > 4) BSA_MFMA(2, 4, 2, 1, true); else BSA_MFMA(2, 4, 1, 1, true); }             \
-  else if (D == 128 && E == 128) { if (hpg > 4) BSA_MFMA(4, 8, 2, 1, true); else BSA_MFMA(4, 8, 1, 1, true); }             \
-  else if (D <= 64 && E <= 64) BSA_MFMA(2, 4, 1, 1, false);                                                                \
-  else if (D <= 128 && E <= 128) BSA_MFMA(4, 8, 1, 1, false);                                                              \
-  else BSA_MFMA(8, 16, 1, 1, false)
+    if (D <= 64 && E <= 128) BSA_MFMA(2, 8, 2);                                                                         \
+    else if (D <= 128 && E <= 128) BSA_MFMA(4, 8, 2);                                                                   \
+    else if (D <= 128) BSA_MFMA(4, 16, 2);                                                                              \
+    else BSA_MFMA(8, 16, 2);                                                                                            \
+  } else if (D <= 64 && E <= 64) BSA_MFMA(2, 4, 1);                                                                     \
+  else if (D <= 96 && E <= 96) BSA_MFMA(3, 6, 1);                                                                       \
+  else if (D <= 128 && E <= 128) BSA_MFMA(4, 8, 1);                                                                     \
+  else if (D <= 192 && E <= 192) BSA_MFMA(6, 12, 1);                                                                    \
+  else BSA_MFMA(8, 16, 1)
   if (dtype == UMB_SEQ_BF16) { using P = BF16; BSA_MFMA_SHAPE(); }
   else { using P = F16; BSA_MFMA_SHAPE(); }
 #undef BSA_MFMA_SHAPE
+#undef BSA_MFMA_AS
 #undef BSA_MFMA
   UMB_LAUNCH_CHECK();
   return UMB_OK;

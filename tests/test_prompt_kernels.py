@@ -781,7 +781,10 @@ def test_prompt_pooled_attention(dtype, H, G, D, window, pool):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("H,Dc,R,window", [(9, 512, 64, 70), (16, 256, 32, 2 ** 20), (8, 256, 64, 33), (4, 512, 64, 2 ** 20), (9, 64, 24, 50)])
+@pytest.mark.parametrize("H,Dc,R,window", [(9, 512, 64, 70), (16, 256, 32, 2 ** 20), (8, 256, 64, 33), (4, 512, 64, 2 ** 20), (9, 64, 24, 50),
+    # every count of feature steps and value tiles, whole and not, either first to overflow its size; few heads and more than eight
+    (8, 128, 0, 40), (3, 96, 32, 2 ** 20), (5, 144, 8, 60), (16, 256, 48, 2 ** 20), (6, 272, 0, 50), (7, 384, 64, 2 ** 20), (4, 368, 40, 45), (12, 400, 40, 70),
+    (2, 512, 0, 2 ** 20)])
 def test_latent_attention_of_prompts_and_of_many_tokens(dtype, H, Dc, R, window):
     from umbrella_amd import _lib
     from umbrella_amd.attn.cache import PagedSeqCache
@@ -818,6 +821,8 @@ def test_latent_attention_of_prompts_and_of_many_tokens(dtype, H, Dc, R, window)
             err = (out[r0:r0 + k].double().cpu().view(k, H, Dc) - o).abs()
             assert bool((err <= tol).all()), (b, float(err.max()))
     case([16, 33, 250, 95], [16, 17, 250, 30], True)
+    if H > 4:                                              # enough workgroups of eight waves
+        case([1100, 60, 1100], [1100, 17, 1090], True) if Dc <= 384 else case([330] * 6, [330] * 6, True)
     case([1 + 3 * i for i in range(50)], [1] * 50, False)
 
 

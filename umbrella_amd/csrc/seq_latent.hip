@@ -319,7 +319,7 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_kernel(typename El<P>::typ
 }
 
 // ---- prompt attention on the matrix pipe (16-bit storage; Dk a multiple of 8, kv_rank a multiple of 16).
-// Workgroup = (16 consecutive positions of one sequence, a block of 4 HPW heads); wave w owns HPW heads.  The tile's keys -- from
+// Workgroup = (16 consecutive positions of one sequence, a block of NW HPW heads); wave w owns HPW heads.  The tile's keys -- from
 // the first position's window start to the last position -- are walked in steps of 32 by the whole workgroup: the step's 32
 // cached rows (all Dk features) are staged ONCE into a shared LDS tile and serve every head of the workgroup, as keys and as
 // values; the next step's rows are already in flight (in registers) while the current one is used, so the one global round
@@ -331,11 +331,15 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_kernel(typename El<P>::typ
 //         finished over the four lanes of a query by two shuffles; accumulators are rescaled when the maximum grows;
 //   O^T += V^T P^T: the lane's eight weights ARE its share of the B operand when V^T's k index runs over (tile 0: 4g .. 4g+3,
 //         tile 1: 4g .. 4g+3); V^T (A: 16 features x those 8 keys) is gathered from the LDS tile.
-// The sink joins the denominator at the end.  NSM / NVM bound the unrolled register arrays (key steps of 32 features, value
-// tiles of 16 features); EXACT: they are the counts.  With run-time counts every product stood in a block of its own behind its own LDS
-// read, and the step was that latency sixty times over: 1999 positions, 32 heads, kv_rank 512 + 64: 932 us, exact 526, eight waves on a
-// staged tile instead of four (two a SIMD; they spill 18 registers) 410.
-template <typename P, int NSM, int NVM, int HPW, int NW, bool EXACT>
+// The sink joins the denominator at the end.  Products per step at compile time: NSM steps of 32 features and NVM tiles of 16, the least of a few
+// sizes that hold Dk and Dc, with zeros behind a row's Dk features; FULL: they are the counts.  With run-time counts every product stood in a
+// block of its own behind its own LDS read, and the step was that latency sixty times over: 2000 positions, 32 heads, kv_rank + rotary 512 + 64
+// 962 us, with counts and four waves 497, eight waves on a staged step (two a SIMD; they spill 16 registers) 372; 384 + 64 849 -> 241.
+template <int NSM, int NVM> struct LatTile {
+  static constexpr int LD = NSM * 32 + 8, LT = 36;              // row strides of a step's rows and of its transposed values: 16 and 8 bytes of padding
+  static constexpr size_t LDS = ((size_t)32 * LD + (size_t)NVM * 16 * LT) * sizeof(u16);
+};
+template <typename P, int NSM, int NVM, int HPW, int NW, bool FULL>
 __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restrict__ out, const float* __restrict__ qa, UmbPagedKV kv,
                                                               const u16* __restrict__ sink, const int* __restrict__ seq_slot,
                                                               const int* __restrict__ seq_row0, const int* __restrict__ seq_pos0,
@@ -344,12 +348,11 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
   extern __shared__ __attribute__((aligned(16))) u16 lat_lds[];
   constexpr int SR = 2 * NW, NLD = (4 * NSM + SR - 1) / SR;           // staging threads per row, 16-byte chunks of the row for each
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
-  if constexpr (EXACT) { Dc = NVM * 16; R = NSM * 32 - Dc; }          // the counts as constants
-  const int Dk = Dc + R, LD = Dk + 8;                 // LDS row stride: 16 bytes of padding spread the key quads over the banks
-  const int ns = (Dk + 31) >> 5, nv = Dc >> 4, nch = Dk >> 3;
-  constexpr int LT = 36;                              // row stride of the transposed tile: 32 keys + 8 bytes of padding
-  u16* v_s = lat_lds;                                 // [32][LD]: the step's rows as cached (keys: A operand of S^T = K Q^T)
-  u16* v_t = lat_lds + 32 * LD;                       // [Dc][LT]: their first Dc features transposed (values: A operand of O^T)
+  if constexpr (FULL) { Dc = NVM * 16; R = NSM * 32 - Dc; }
+  constexpr int LD = LatTile<NSM, NVM>::LD, LT = LatTile<NSM, NVM>::LT;
+  const int Dk = Dc + R, nv = Dc >> 4, nch = Dk >> 3;
+  u16* v_s = lat_lds;                                 // [32][LD]: the step's rows as cached, zero past Dk (keys: A operand of S^T = K Q^T)
+  u16* v_t = lat_lds + 32 * LD;                       // [16 NVM][LT]: their first Dc features transposed (values: A operand of O^T); the rest as it is
   const int b = blockIdx.y;
   const int n = seq_len[b], q0 = blockIdx.x * 16;
   if (q0 >= n) return;                                // the whole workgroup
@@ -377,7 +380,7 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
     for (int s = 0; s < NSM; ++s) {
       const int d = 32 * s + 8 * g4;
       qf[hh][s] = u32x4{0u, 0u, 0u, 0u};
-      if (s < ns && d < Dk) {
+      if (d < Dk) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(qr + d), c = *reinterpret_cast<const f32x4*>(qr + d + 4);
         qf[hh][s] = u32x4{pack2<P>(a[0], a[1]), pack2<P>(a[2], a[3]), pack2<P>(c[0], c[1]), pack2<P>(c[2], c[3])};
       }
@@ -400,7 +403,8 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
     }
   };
   fetch(0);
-  if (threadIdx.x < 32) *reinterpret_cast<u32x4*>(v_s + threadIdx.x * LD + Dk) = u32x4{0u, 0u, 0u, 0u};       // read where a step of 32 runs past Dk
+  if (threadIdx.x < 32)
+    for (int ch = nch; ch <= NSM * 4; ++ch) *reinterpret_cast<u32x4*>(v_s + threadIdx.x * LD + 8 * ch) = u32x4{0u, 0u, 0u, 0u};
   for (int base = 0; base < total; base += 32) {
     __syncthreads();                                  // every wave is done with the previous tile
 #pragma unroll
@@ -428,12 +432,9 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
       const u16* kr = v_s + (16 * u + j) * LD;
 #pragma unroll
       for (int s = 0; s < NSM; ++s) {
-        const int d = 32 * s + 8 * g4;
-        if (s < ns) {
-          const u32x4 kf = *reinterpret_cast<const u32x4*>(kr + (d < Dk ? d : Dk));
+        const u32x4 kf = *reinterpret_cast<const u32x4*>(kr + 32 * s + 8 * g4);
 #pragma unroll
-          for (int hh = 0; hh < HPW; ++hh) sc2[hh][u] = P::mfma(kf, qf[hh][s], sc2[hh][u]);
-        }
+        for (int hh = 0; hh < HPW; ++hh) sc2[hh][u] = P::mfma(kf, qf[hh][s], sc2[hh][u]);
       }
     }
     // a step that every query sees whole needs no tests (rows past the last are not stored)
@@ -471,22 +472,18 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
       m_run[hh] = m_new;
       if (__ballot(fac != 1.f)) {                                    // the maximum moved for some row of the tile
 #pragma unroll
-        for (int dt = 0; dt < NVM; ++dt) {
-          if (dt < nv) { o[hh][dt][0] *= fac; o[hh][dt][1] *= fac; o[hh][dt][2] *= fac; o[hh][dt][3] *= fac; }
-        }
+        for (int dt = 0; dt < NVM; ++dt) { o[hh][dt][0] *= fac; o[hh][dt][1] *= fac; o[hh][dt][2] *= fac; o[hh][dt][3] *= fac; }
       }
       pf[hh] = u32x4{pack2<P>(w[0], w[1]), pack2<P>(w[2], w[3]), pack2<P>(w[4], w[5]), pack2<P>(w[6], w[7])};
     }
     // O^T[d][query] += V^T[d][keys] P^T[keys][query]: lane (d row j of tile dt, quad g4) reads its 8 keys' values
 #pragma unroll
     for (int dt = 0; dt < NVM; ++dt) {
-      if (dt < nv) {
-        const u16* vr = v_t + (16 * dt + j) * LT + 4 * g4;
-        const u32x2 t0 = *reinterpret_cast<const u32x2*>(vr), t1 = *reinterpret_cast<const u32x2*>(vr + 16);
-        const u32x4 va = u32x4{t0[0], t0[1], t1[0], t1[1]};
+      const u16* vr = v_t + (16 * dt + j) * LT + 4 * g4;
+      const u32x2 t0 = *reinterpret_cast<const u32x2*>(vr), t1 = *reinterpret_cast<const u32x2*>(vr + 16);
+      const u32x4 va = u32x4{t0[0], t0[1], t1[0], t1[1]};
 #pragma unroll
-        for (int hh = 0; hh < HPW; ++hh) o[hh][dt] = P::mfma(va, pf[hh], o[hh][dt]);
-      }
+      for (int hh = 0; hh < HPW; ++hh) o[hh][dt] = P::mfma(va, pf[hh], o[hh][dt]);
     }
   }
   // lane holds O^T[d = 16 dt + 4 g4 + rr][query j]
@@ -516,16 +513,16 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
 // block of 16 heads); its four waves take the 32-key steps w, w + 4, ... of the window (which step lands in which wave depends
 // on the token's position alone) with the same step body as the prompt kernel, then merge their running maxima, sums and
 // partial outputs through LDS in wave order, where the sink joins the denominator.
-template <typename P, int NSM, int NVM, bool EXACT>
+template <typename P, int NSM, int NVM, bool FULL>
 __global__ __launch_bounds__(256) void lat_decode_mfma_kernel(u16* __restrict__ out, const float* __restrict__ qa, UmbPagedKV kv,
                                                               const u16* __restrict__ sink, const int* __restrict__ pos,
                                                               const int* __restrict__ slot_, int H, int Dc, int R, int window,
                                                               float scale) {
   extern __shared__ __attribute__((aligned(16))) u16 lat_lds[];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
-  if constexpr (EXACT) { Dc = NVM * 16; R = NSM * 32 - Dc; }          // the counts as constants
-  const int Dk = Dc + R, LD = Dc + 8;
-  const int ns = (Dk + 31) >> 5, nv = Dc >> 4;
+  if constexpr (FULL) { Dc = NVM * 16; R = NSM * 32 - Dc; }            // no test at a row's loads: 14 us, 16 with, at 48 tokens behind 40, 512 + 64
+  constexpr int LD = NVM * 16 + 8;
+  const int Dk = Dc + R, nv = Dc >> 4;
   u16* v_s = lat_lds + (long)wave * (32 * LD + 32 * 4);
   long* offs = reinterpret_cast<long*>(v_s + 32 * LD);
   const int t = blockIdx.x, h = blockIdx.y * 16 + j;
@@ -543,7 +540,7 @@ __global__ __launch_bounds__(256) void lat_decode_mfma_kernel(u16* __restrict__ 
     for (int s = 0; s < NSM; ++s) {
       const int d = 32 * s + 8 * g4;
       qf[s] = u32x4{0u, 0u, 0u, 0u};
-      if (s < ns && d < Dk) {
+      if (d < Dk) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(qr + d), c = *reinterpret_cast<const f32x4*>(qr + d + 4);
         qf[s] = u32x4{pack2<P>(a[0], a[1]), pack2<P>(a[2], a[3]), pack2<P>(c[0], c[1]), pack2<P>(c[2], c[3])};
       }
@@ -588,12 +585,10 @@ __global__ __launch_bounds__(256) void lat_decode_mfma_kernel(u16* __restrict__ 
 #pragma unroll
       for (int s = 0; s < NSM; ++s) {
         const int d = 32 * s + 8 * g4;
-        kf[s] = (s < ns && d < Dk && off >= 0) ? *reinterpret_cast<const u32x4*>(kr + d) : u32x4{0u, 0u, 0u, 0u};
+        kf[s] = (d < Dk && off >= 0) ? *reinterpret_cast<const u32x4*>(kr + d) : u32x4{0u, 0u, 0u, 0u};
       }
 #pragma unroll
-      for (int s = 0; s < NSM; ++s) {
-        if (s < ns) sc[u] = P::mfma(kf[s], qf[s], sc[u]);
-      }
+      for (int s = 0; s < NSM; ++s) sc[u] = P::mfma(kf[s], qf[s], sc[u]);
     }
     float sv[8], mx = -INFINITY;                                // maxima and exponents in base 2: one v_exp_f32 per weight
 #pragma unroll
@@ -620,22 +615,18 @@ __global__ __launch_bounds__(256) void lat_decode_mfma_kernel(u16* __restrict__ 
     m_run = m_new;
     if (__ballot(fac != 1.f)) {
 #pragma unroll
-      for (int dt = 0; dt < NVM; ++dt) {
-        if (dt < nv) { o[dt][0] *= fac; o[dt][1] *= fac; o[dt][2] *= fac; o[dt][3] *= fac; }
-      }
+      for (int dt = 0; dt < NVM; ++dt) { o[dt][0] *= fac; o[dt][1] *= fac; o[dt][2] *= fac; o[dt][3] *= fac; }
     }
     const u32x4 pf = u32x4{pack2<P>(w[0], w[1]), pack2<P>(w[2], w[3]), pack2<P>(w[4], w[5]), pack2<P>(w[6], w[7])};
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int dt = 0; dt < NVM; ++dt) {
-      if (dt < nv) {
-        unsigned e[8];
+      unsigned e[8];
 #pragma unroll
-        for (int m = 0; m < 8; ++m) e[m] = v_s[((m >> 2) * 16 + 4 * g4 + (m & 3)) * LD + 16 * dt + j];
-        const u32x4 va = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-        o[dt] = P::mfma(va, pf, o[dt]);
-      }
+      for (int m = 0; m < 8; ++m) e[m] = v_s[((m >> 2) * 16 + 4 * g4 + (m & 3)) * LD + 16 * dt + j];
+      const u32x4 va = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
+      o[dt] = P::mfma(va, pf, o[dt]);
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -690,24 +681,34 @@ extern "C" int umb_lat_attend_tiled(void* out, const float* qa, const UmbPagedKV
       !umb_lat_attend_tiled_ok(H, kv_rank, rot_dim, dtype))
     return UMB_EINVAL;
   const int Dk = kv_rank + rot_dim;
-  const size_t lds = ((size_t)32 * (Dk + 8) + (size_t)kv_rank * 36) * sizeof(u16);
-#define LAT_MFMA(NSM, NVM, HPW, NW, EX)                                                                                      \
+  // Eight waves share a staged step where there is a workgroup of them for most compute units and the walk is long or its rows are; four, and
+  // twice the workgroups, elsewhere (us with 4 / 8 waves, kv_rank + rotary, heads, positions: 512 + 64, 32: 16 16 / 24, 600 111 / 120, 2000
+  // 497 / 372, 8 x 300 174 / 157; 384 + 64, 32: 600 69 / 76, 2000 249 / 241, 8 x 300 98 / 106; 256 + 32, 16: 600 39 / 48, 2000 55 / 53, 8 x 300 41 / 48)
+  const long eights = (long)((max_len + 15) / 16) * B * ((H + 7) / 8);
+  const bool eight = H > 4 && eights >= 200 && (kv_rank > 384 || max_len >= 1000);
+#define LAT_MFMA_AS(NSM, NVM, HPW, NW, FULL)                                                                               \
   do {                                                                                                                     \
     const dim3 grid((max_len + 15) / 16, B, (H + NW * HPW - 1) / (NW * HPW));                                              \
-    if (ensure_dynamic_lds<lat_attend_mfma_kernel<P, NSM, NVM, HPW, NW, EX>>(lds) != UMB_OK) return UMB_EHIP;                  \
-    hipLaunchKernelGGL((lat_attend_mfma_kernel<P, NSM, NVM, HPW, NW, EX>), grid, dim3(NW * 64), lds, st, (u16*)out, qa, *kv,   \
+    constexpr size_t lds = LatTile<NSM, NVM>::LDS;                                                                         \
+    if (ensure_dynamic_lds<lat_attend_mfma_kernel<P, NSM, NVM, HPW, NW, FULL>>(lds) != UMB_OK) return UMB_EHIP;            \
+    hipLaunchKernelGGL((lat_attend_mfma_kernel<P, NSM, NVM, HPW, NW, FULL>), grid, dim3(NW * 64), lds, st, (u16*)out, qa, *kv, \
                        (const u16*)sink, seq_slot, seq_row0, seq_pos0, seq_len, H, kv_rank, rot_dim, window, scale);       \
   } while (0)
+#define LAT_MFMA(NSM, NVM, HPW, NW)                                                                                        \
+  do { if (Dk == 32 * NSM && kv_rank == 16 * NVM) LAT_MFMA_AS(NSM, NVM, HPW, NW, true); else LAT_MFMA_AS(NSM, NVM, HPW, NW, false); } while (0)
+#define LAT_MFMA_WAVES(NSM, NVM) do { if (eight) LAT_MFMA(NSM, NVM, 1, 8); else LAT_MFMA(NSM, NVM, 1, 4); } while (0)
 #define LAT_MFMA_SHAPE()                                                                                                   \
-  if (H > 4 && Dk == 576 && kv_rank == 512) LAT_MFMA(18, 32, 1, 8, true);                                                  \
-  else if (H > 4 && Dk == 288 && kv_rank == 256) LAT_MFMA(9, 16, 1, 8, true);                                              \
-  else if (Dk <= 128 && kv_rank <= 128) { if (H >= 8) LAT_MFMA(4, 8, 2, 4, false); else LAT_MFMA(4, 8, 1, 4, false); }     \
-  else if (Dk <= 320 && kv_rank <= 256) LAT_MFMA(10, 16, 1, 4, false);                                                           \
-  else LAT_MFMA(18, 32, 1, 4, false)
+  if (Dk <= 128 && kv_rank <= 128) { if (H >= 8) LAT_MFMA(4, 8, 2, 4); else LAT_MFMA(4, 8, 1, 4); }                        \
+  else if (Dk <= 288 && kv_rank <= 256) LAT_MFMA_WAVES(9, 16);                                                             \
+  else if (Dk <= 320 && kv_rank <= 256) LAT_MFMA_WAVES(10, 16);                                                            \
+  else if (Dk <= 448 && kv_rank <= 384) LAT_MFMA_WAVES(14, 24);                                                            \
+  else LAT_MFMA_WAVES(18, 32)
   if (dtype == UMB_SEQ_BF16) { using P = BF16; LAT_MFMA_SHAPE(); }
   else { using P = F16; LAT_MFMA_SHAPE(); }
 #undef LAT_MFMA_SHAPE
+#undef LAT_MFMA_WAVES
 #undef LAT_MFMA
+#undef LAT_MFMA_AS
   UMB_LAUNCH_CHECK();
   return UMB_OK;
 }
@@ -773,23 +774,26 @@ extern "C" int umb_lat_attend(void* out, const float* qa, const UmbPagedKV* kv, 
   if (H >= 4 && T >= lat_dec_min && umb_lat_attend_tiled_ok(H, kv_rank, rot_dim, dtype)) {
     // 16-bit storage: sixteen heads of a token form the query tile of the matrix-pipe kernel
     const int Dk = kv_rank + rot_dim;
-    const size_t tiles = 4 * (size_t)(32 * (kv_rank + 8) + 128) * sizeof(u16);
-    const size_t parts = (size_t)4 * (kv_rank / 16) * 64 * sizeof(f32x4) + 4 * 16 * 2 * sizeof(float);
-    const size_t lds = tiles > parts ? tiles : parts;
     const dim3 grid(T, (H + 15) / 16);
-#define LAT_DEC(NSM, NVM, EX)                                                                                              \
+#define LAT_DEC_AS(NSM, NVM, FULL)                                                                                         \
   do {                                                                                                                     \
-    if (ensure_dynamic_lds<lat_decode_mfma_kernel<P, NSM, NVM, EX>>(lds) != UMB_OK) return UMB_EHIP;                           \
-    hipLaunchKernelGGL((lat_decode_mfma_kernel<P, NSM, NVM, EX>), grid, dim3(256), lds, st, (u16*)out, qa, *kv,                \
+    constexpr size_t tiles = 4 * (size_t)(32 * (NVM * 16 + 8) + 128) * sizeof(u16);                                        \
+    constexpr size_t parts = (size_t)4 * NVM * 64 * sizeof(f32x4) + 4 * 16 * 2 * sizeof(float);                            \
+    constexpr size_t lds = tiles > parts ? tiles : parts;                                                                  \
+    if (ensure_dynamic_lds<lat_decode_mfma_kernel<P, NSM, NVM, FULL>>(lds) != UMB_OK) return UMB_EHIP;                     \
+    hipLaunchKernelGGL((lat_decode_mfma_kernel<P, NSM, NVM, FULL>), grid, dim3(256), lds, st, (u16*)out, qa, *kv,          \
                        (const u16*)sink, pos, slot, H, kv_rank, rot_dim, window, scale);                                   \
   } while (0)
+#define LAT_DEC(NSM, NVM)                                                                                                  \
+  do { if (Dk == 32 * NSM && kv_rank == 16 * NVM) LAT_DEC_AS(NSM, NVM, true); else LAT_DEC_AS(NSM, NVM, false); } while (0)
 #define LAT_DEC_SHAPE()                                                                                                    \
-  if (Dk == 576 && kv_rank == 512) LAT_DEC(18, 32, true); else if (Dk == 288 && kv_rank == 256) LAT_DEC(9, 16, true);       \
-  else if (Dk <= 128 && kv_rank <= 128) LAT_DEC(4, 8, false); else if (Dk <= 320 && kv_rank <= 256) LAT_DEC(10, 16, false); else LAT_DEC(18, 32, false)
+  if (Dk <= 128 && kv_rank <= 128) LAT_DEC(4, 8); else if (Dk <= 288 && kv_rank <= 256) LAT_DEC(9, 16);                     \
+  else if (Dk <= 320 && kv_rank <= 256) LAT_DEC(10, 16); else if (Dk <= 448 && kv_rank <= 384) LAT_DEC(14, 24); else LAT_DEC(18, 32)
     if (dtype == UMB_SEQ_BF16) { using P = BF16; LAT_DEC_SHAPE(); }
     else { using P = F16; LAT_DEC_SHAPE(); }
 #undef LAT_DEC_SHAPE
 #undef LAT_DEC
+#undef LAT_DEC_AS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
   }

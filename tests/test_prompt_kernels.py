@@ -832,7 +832,7 @@ def test_latent_attention_of_prompts_and_of_many_tokens(dtype, H, Dc, R, window)
 def test_many_slots_are_prepared_as_few_are(dtype, H, G, D, E, maps, layout, rot, append, norm, mixed):
     """norm, rotation and append of many (token, head) slots against launches of few: an fp32 sum of squares in another order"""
     from umbrella_amd import _lib
-    T, step, code = 2400, 60, _lib.seq_dtype_code(dtype)
+    T, step, code = 2880, 60, _lib.seq_dtype_code(dtype)
     g = torch.Generator(device="cuda").manual_seed(D + E)
     c, _, _, _ = _decode_store([T], G, maps * D, E, 0, dtype, 32, 1)
     d, _, _, _ = _decode_store([T], G, maps * D, E, 0, dtype, 32, 2)

@@ -616,8 +616,9 @@ extern "C" int umb_attn_prep_mix(float* q, const UmbPagedKV* kv, const float* pr
              temp_coef, temp_every, eps, mix ? *mix : UmbValueMix{nullptr, nullptr, 0.f, 0.f}};
   const UmbPagedKV none{};
   const long items = (long)T * (a.HQ + a.GK + a.GV);
-  // from two rounds of waves over the chip on (2304 items take a wave each in 4.2 us)
-  if (items >= 16384 && D <= 128 && E <= 128) {
+  // from three rounds of waves over the chip on (us, a wave each / four: 17600 items of two maps 9.2 / 10.5, 19200 of 64 10.2 / 9.9, 30800 of two maps
+  // 13.9 / 13.5, 96000 37.9 / 29.3)
+  if (items >= 24576 && D <= 128 && E <= 128) {
     const int groups = (a.HQ + a.GK + a.GV + 3) / 4;
     DISPATCH_SEQ_DTYPE(dtype, {
       typedef typename El<P>::type El_;

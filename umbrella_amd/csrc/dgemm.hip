@@ -131,10 +131,12 @@ static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, i
 // Up to 128 tokens against more weights than the last-level cache holds the product is bound by HBM, and gemm.hip's register-resident
 // kernel streams them faster (128256 x 4096, 100 tokens: 195 us, 217 here; 160 tokens: 377, 250 here).  It holds up to 144 tokens in one pass,
 // and stays ahead there where the 256-row tiles of such a launch are more than one per compute unit (129 tokens, it / here: 128256 x 4096 198 /
-// 245 us, 73728 x 4608 192 / 219; 65536 x 5120, one round, 175 / 145; 145 tokens 377 / 245).
+// 245 us, 73728 x 4608 192 / 219, 128256 x 2048 111 / 122; 65536 x 5120, one round, 175 / 145; 145 tokens 377 / 245).  Less weight of such a
+// launch already stays ahead there (65 tokens, 100352 x 2560 101 / 125) unless K is short (256000 x 1024 127 / 117).
 bool umb_dgemm_ok(const void* x, int ldx, int T, int N, int K, int S, int epi) {
   static const bool off = getenv("UMB_NO_VGEMM") != nullptr || getenv("UMB_VGEMM_PLAIN") != nullptr;     // gemm.hip's diagnostics
-  const bool streams = (long)N * K * 2 > (512L << 20) && (T <= 128 || (T <= 144 && (N + 255) / 256 > 256));
+  const long bytes = (long)N * K * 2;
+  const bool streams = (T <= 128 && bytes > (512L << 20)) || (T <= 144 && N > 65536 && K >= 1536 && bytes > (448L << 20));
   return !off && T > 64 && K % 64 == 0 && N % 16 == 0 && ldx % 8 == 0 && (uintptr_t)x % 16 == 0 && epi <= EPI_SILU &&
          (long)ldx * 512 < (1L << 31) && !streams;
 }

@@ -637,7 +637,9 @@ def test_split_reduce_of_many_rows_is_that_of_few(dtype, T, N, S):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("T,Hq,Hkv,D,S,paired", [(257, 4, 2, 64, 2, 1), (400, 4, 1, 96, 3, 1), (263, 3, 1, 32, 1, 0), (514, 2, 2, 128, 4, 0), (1024, 5, 1, 256, 8, 1)])
+@pytest.mark.parametrize("T,Hq,Hkv,D,S,paired", [(257, 4, 2, 64, 2, 1), (400, 4, 1, 96, 3, 1), (263, 3, 1, 32, 1, 0), (514, 2, 2, 128, 4, 0), (1024, 5, 1, 256, 8, 1),
+    # enough columns and few enough splits for a workgroup per 256 columns of 16 tokens
+    (263, 20, 6, 64, 2, 1), (400, 8, 4, 96, 3, 1), (259, 48, 2, 32, 1, 0), (514, 4, 2, 128, 2, 0), (700, 8, 1, 64, 4, 1), (1023, 5, 1, 256, 3, 1), (258, 5, 1, 256, 1, 0)])
 def test_split_reduce_and_rotation_of_many_tokens_is_that_of_few(dtype, T, Hq, Hkv, D, S, paired):
     from umbrella_amd import _lib
     g = torch.Generator(device="cuda").manual_seed(T + D)

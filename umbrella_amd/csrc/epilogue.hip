@@ -690,9 +690,13 @@ extern "C" int umb_reduce_qkv_rope2(const void* partial, int S, int T, int Hq, i
                                     void* k_cache, void* vt_cache, int paired, const void* bias, const float* ssq_in,
                                     int ssq_groups, int ssq_stride, float ssq_dim, float eps, int dtype, hipStream_t st) {
   if (D % 32 || Lmax % 32 || (ssq_in && (ssq_groups < 1 || ssq_stride < ssq_groups || ssq_dim <= 0.f))) return UMB_EINVAL;   // 32-key x 32-feature cache tiles
-  // from where a workgroup per (token, head) means rounds of them; many splits move the line up (257 tokens, 64 + 8 heads of 128: 2 splits
-  // 12.0 -> 10.2 us, 8 splits 16.4 -> 19.8)
-  if (T >= WIDE_ROWS && T >= 128 * S && S >= 1 && ((uintptr_t)partial % 16 | (uintptr_t)q_out % 4 | (uintptr_t)k_cache % 4 | (uintptr_t)vt_cache % 8 | (uintptr_t)cosT % 4 | (uintptr_t)sinT % 4) == 0) {
+  // From where a workgroup per (token, head) means rounds of them.  A wave of four tokens walks the splits one after the other where those have a
+  // wave per token: few splits only, fewer where a head's two halves are far apart in memory and not next to each other (us, a workgroup per
+  // head / this, halves apart: 1024 tokens, 32 + 8 heads of 128, 1 / 2 / 3 / 4 / 8 splits 25.3 / 18.5, 24.8 / 22.1, 25.1 / 25.2, 25.6 / 26.8, 36 / 41, heads of
+  // 64, 4 splits 23.6 / 15.7; 2048 tokens, 8 + 1 of 256, 3 splits 17.4 / 21.2; 257 tokens, 8 + 2 of 64, 2 splits 4.8 / 5.4)
+  const int most = D <= 64 ? 4 : (paired ? 3 : (D <= 128 ? 2 : 1));
+  if (T >= WIDE_ROWS && T >= 128 * S && S >= 1 && S <= most && (long)T * (Hq + 2 * Hkv) * D >= 400000 &&
+      ((uintptr_t)partial % 16 | (uintptr_t)q_out % 4 | (uintptr_t)k_cache % 4 | (uintptr_t)vt_cache % 8 | (uintptr_t)cosT % 4 | (uintptr_t)sinT % 4) == 0) {
 #define QRW(PAIRED)                                                                                                                \
   hipLaunchKernelGGL((reduce_qkv_rope_wide_kernel<P, PAIRED>), dim3(((Hq + 2 * Hkv) * D + 255) / 256, (T + 15) / 16), dim3(256), 0, st,   \
                      (const float*)partial, S, T, Hq, Hkv, D, Lmax, pos, slot, (const u16*)cosT, (const u16*)sinT, (u16*)q_out,     \

@@ -24,7 +24,8 @@
 // attend (vector pipe, any dtype and head size): workgroup = (token, RH query heads of ONE key/value head, so one pass over
 // the keys serves them all); waves take 64-key rounds by round number; score phase lane = key, value phase lane = value
 // column with eight keys' rows in flight; per-wave running maximum / denominator, merged through LDS in wave order.  Which
-// keys land in which wave and round depends on the query's position alone -- never on the batch or on how a prompt was cut.
+// keys land in which wave and round depends on the query's position and on the launch (waves an item, splits of a token's keys, prompt tiles):
+// the same token in another batch, or of a prompt cut elsewhere, agrees to fp32 rounding and not bit for bit.
 #include "seq_common.h"
 #include "seq_decode.h"
 

@@ -172,8 +172,8 @@ __global__ __launch_bounds__(256) void lat_front_kernel(typename El<P>::type* __
 // in position order; inside a round lane = key for the scores (the key's row against the queries in LDS), then lane = value
 // column for the weighted sum, the round's weights broadcast one key at a time.  Each wave keeps a running maximum and
 // denominator per head (the usual rescaling when the maximum grows); the waves' partial results are merged through LDS in
-// wave order together with the sink.  Which keys land in which wave and round depends on the query's position alone -- never
-// on the batch or on how the prompt was cut.
+// wave order together with the sink.  Which keys land in which wave and round depends on the query's position and on NW, which follows the
+// number of workgroups.
 constexpr int LAT_MAXC = 16;     // value columns per lane: kv_rank <= 1024
 
 template <typename P, int RH, int NC, int NW>

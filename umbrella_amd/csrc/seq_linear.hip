@@ -11,7 +11,8 @@
 //
 // Few tokens: a workgroup owns 16 (or 32) output rows and up to 64 tokens; its four waves split K (wave w takes the 32-k steps w, w+4, ...)
 // and their partial tiles are summed through LDS in wave order: the summation order of an output is a function of K alone,
-// never of the row's place in the batch, and of T only where the many-token kernels take over (launch_vec).  K % 8 != 0 (or a tail) falls back to guarded element loads.
+// never of the row's place in the batch, and of T only where the many-token kernels take over (launch_vec).  K % 8 != 0 (or a tail)
+// falls back to guarded element loads.
 #include "gemm_tile.h"
 #include "seq_common.h"
 

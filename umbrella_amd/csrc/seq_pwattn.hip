@@ -17,8 +17,9 @@
 // sequence.  The pooled mean is always taken over the cached (rounded) values in position order: the same numbers whether
 // the tokens arrived in one step or one by one.
 //
-// Because the weights are not normalised there is no running maximum and no rescaling: a query's output is a plain sum, and
-// each (token, head) sums its keys in position order per lane column -- independent of the batch and of how the prompt was cut.
+// Because the weights are not normalised there is no running maximum and no rescaling: a query's output is a plain sum.  A wave adds its
+// rounds of keys in position order; how many waves share a query follows the launch (prompt tiles, or the number of (token, head block)
+// items), so the same token in another batch, or of a prompt cut elsewhere, agrees to fp32 rounding and not bit for bit.
 #include "seq_common.h"
 #include "seq_decode.h"
 
@@ -178,8 +179,7 @@ __global__ __launch_bounds__(256) void pwa_pool_kernel(UmbPagedKV kv, const int*
 // ---- attention.  Workgroup = (token, RH query heads of one key/value group): the heads of a group read the same keys and
 // values, so one pass over the keys serves all of them.  The NW waves take the 64-key rounds w, w + NW, ... of the key list
 // (pooled blocks first, then the window's tokens, both in position order) and their partial sums are added through LDS in
-// wave order -- which keys land in which wave depends on the query's position alone, never on the batch or on how the prompt
-// was cut.  Score phase: lane = key, 16-byte loads along the key's row against the queries held in LDS.  Value phase:
+// wave order: which keys land in which wave depends on the query's position and on NW.  Score phase: lane = key, 16-byte loads along the key's row against the queries held in LDS.  Value phase:
 // lane = value column, the round's weights broadcast one key at a time.
 constexpr int PWA_MAXC = 4;      // value columns per lane: D <= 256
 

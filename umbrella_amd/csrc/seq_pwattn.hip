@@ -179,8 +179,8 @@ __global__ __launch_bounds__(256) void pwa_pool_kernel(UmbPagedKV kv, const int*
 // ---- attention.  Workgroup = (token, RH query heads of one key/value group): the heads of a group read the same keys and
 // values, so one pass over the keys serves all of them.  The NW waves take the 64-key rounds w, w + NW, ... of the key list
 // (pooled blocks first, then the window's tokens, both in position order) and their partial sums are added through LDS in
-// wave order: which keys land in which wave depends on the query's position and on NW.  Score phase: lane = key, 16-byte loads along the key's row against the queries held in LDS.  Value phase:
-// lane = value column, the round's weights broadcast one key at a time.
+// wave order: which keys land in which wave depends on the query's position and on NW.  Score phase: lane = key, 16-byte loads along
+// the key's row against the queries held in LDS.  Value phase: lane = value column, the round's weights broadcast one key at a time.
 constexpr int PWA_MAXC = 4;      // value columns per lane: D <= 256
 
 template <typename P, int RH, int NC, int NW>

@@ -806,7 +806,8 @@ extern "C" int umb_bsa_attend(void* out, int ldo, const float* q, const UmbPaged
 
 // ---- prompt attention on the matrix pipe (16-bit storage; D a multiple of 8, E a multiple of 16).
 // Workgroup = (16 consecutive positions of one sequence, one key/value head, four of its query heads), a wave per head.  The tile's
-// keys -- from the first position's window start to the last position -- are walked in steps of 32 by the whole workgroup: the step's 32 cached key rows and value rows are staged ONCE into LDS (keys as cached: the A operand of
+// keys -- from the first position's window start to the last position -- are walked in steps of 32 by the whole workgroup: the
+// step's 32 cached key rows and value rows are staged ONCE into LDS (keys as cached: the A operand of
 // S^T = K Q^T; values transposed: the A operand of O^T += V^T P^T) and serve every head of the workgroup; the next step's rows
 // are in flight in registers while the current one is used.  Per step and head: two 16-key score tiles; the bias of the
 // lane's eight (query, key) pairs, fetched by distance before the products are issued; online softmax in fp32 with base-2

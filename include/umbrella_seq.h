@@ -59,6 +59,12 @@ typedef struct UmbSeqLinear { const void* w; const void* bias; int32_t N, K; } U
 int umb_seq_linear(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, int dtype,
                    umb_stream_t stream);
 
+/* A product of few tokens (T <= 64) whose K is summed in `parts` slabs: out fp32 [parts][T][N], the sum over the slabs is the result (bias in
+ * the first one's).  umb_seq_linear_split: the number of slabs that pays for these operands (1 .. 4; 1: umb_seq_linear; no stream). */
+int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype);
+int umb_seq_linear_parts(float* out, const void* x, const void* w, const void* bias, int T, int N, int K, int parts, int dtype,
+                         umb_stream_t stream);
+
 /* The same product for `batch` independent problems (blockIdx.z): problem b reads x + b sx (rows ldx apart), weights
  * w + b sw ([N][K]) and writes out + b so (rows ldo apart); strides in elements; no bias.  epi 0 / 1 as above;
  * epi 3: out in `dtype` = acc * sigmoid(gate[t ldg + b sg + n]) (gate fp32); epi 7: the same with ONE gate per row and problem,
@@ -87,11 +93,17 @@ int umb_seq_embed_norm(float* x, void* h, const void* embed, const int* tokens, 
 /* x <- x + group_norm(y) * w_post ; if w_next: h <- group_norm(x) * w_next in `dtype`   (y fp32 [T][W]) */
 int umb_seq_resid_norm(float* x, void* h, const float* y, const void* w_post, const void* w_next, int T, int W, int groups,
                        float eps, int dtype, umb_stream_t stream);
+/* the same with y in 1 .. 4 slabs [parts][T][W] whose sum is meant (umb_seq_linear_parts); where the seam's own kernel does not add them
+ * they are summed into the first slab before it */
+int umb_seq_resid_norm_parts(float* x, void* h, float* y, int parts, const void* w_post, const void* w_next, int T, int W, int groups,
+                             float eps, int dtype, umb_stream_t stream);
 
 /* m = coef (norm(y1) * w1 + norm(y2) * w2); x <- x + norm(m) * w_post; if w_next: h <- norm(x) * w_next in `dtype` (plain RMS
  * norms over the row; y1, y2 fp32 [T][W]): the seam behind two mixers side by side */
 int umb_seq_pair_resid_norm(float* x, void* h, const float* y1, const float* y2, const void* w1, const void* w2, float coef,
                             const void* w_post, const void* w_next, int T, int W, float eps, int dtype, umb_stream_t stream);
+int umb_seq_pair_resid_norm_parts(float* x, void* h, float* y1, int parts1, float* y2, int parts2, const void* w1, const void* w2, float coef,
+                                  const void* w_post, const void* w_next, int T, int W, float eps, int dtype, umb_stream_t stream);
 
 /* x[t] <- embed[tokens[t]] * scale (fp32) */
 int umb_seq_embed(float* x, const void* embed, const int* tokens, float scale, int T, int W, int V, int dtype,
@@ -231,6 +243,8 @@ int umb_hc_embed(float* x, void* h, const void* embed, const int* tokens, float 
                  float offset, int T, int W, int V, int S, float eps, int dtype, umb_stream_t stream);
 int umb_hc_seam(float* x, void* h, const float* y, const float* mix, const float* out, float m, const float* in_next,
                 const void* w_next, float offset, int T, int W, int S, float eps, int dtype, umb_stream_t stream);
+int umb_hc_seam_parts(float* x, void* h, float* y, int parts, const float* mix, const float* out, float m, const float* in_next,
+                      const void* w_next, float offset, int T, int W, int S, float eps, int dtype, umb_stream_t stream);
 int umb_hc_read(float* u_out, void* h, const float* x, const int* rows, const float* in, const void* w, float offset, int R,
                 int W, int S, float eps, int dtype, umb_stream_t stream);
 
@@ -573,6 +587,7 @@ typedef struct UmbSeqWork {
   void* h2;            /* parallel blocks: normed input of the feed-forward [Tmax][W] dtype */
   float* y2;           /* parallel blocks: feed-forward output; mixers with two output projections: the second [Tmax][W] fp32 */
   float* v_first;      /* values that later layers of the step mix in [Tmax][kv_heads vdim] fp32 (null when no layer does) */
+  int64_t y_floats;    /* floats in y, and in y2 where there is one (0: Tmax W): room for the slabs of split products */
 } UmbSeqWork;
 
 typedef struct UmbSeqStep {

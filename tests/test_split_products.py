@@ -1,0 +1,76 @@
+"""Products of few tokens whose K is summed in slabs, and the seams that add the slabs: against the sum of the slabs in float64."""
+import pytest
+import torch
+
+U = 2.0 ** -24
+DTYPES = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
+
+
+def _code(name):
+    from umbrella_amd import _lib
+    return {"bf16": _lib.BF16, "fp16": _lib.F16, "fp32": _lib.F32}[name]
+
+
+def test_split_rule_stays_inside_what_the_product_takes():
+    from umbrella_amd import _lib
+    split = _lib.load_seq().umb_seq_linear_split
+    ptr = 1 << 20
+    for code, item in ((_lib.BF16, 2), (_lib.F32, 4)):
+        for T in (1, 16, 17, 32, 33, 64, 65, 2000):
+            for N in (1, 16, 1000, 2048, 2049, 2730, 4096, 4097, 32000):
+                for K in (8, 200, 256, 512, 1024, 2048, 2304, 8192, 14336):
+                    parts = split(ptr, ptr, T, N, K, code)
+                    assert 1 <= parts <= 4 and (parts == 1 or (T <= 64 and K * item % 512 == 0 and parts * 4 <= K * item // 512)), (T, N, K)
+        assert split(ptr + 8, ptr, 1, 2048, 8192, code) == 1 and split(ptr, ptr + 8, 1, 2048, 8192, code) == 1     # no 16-byte pieces
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("T,N,chunks,parts", [(1, 16, 2, 2), (1, 2048, 8, 2), (16, 40, 7, 3), (17, 2049, 5, 4), (33, 4096, 16, 2), (48, 130, 32, 4),
+                                              (64, 2047, 33, 4)])
+def test_slabs_add_up_to_the_product(dtype, T, N, chunks, parts):
+    from umbrella_amd import _lib
+    dt, K = DTYPES[dtype], chunks * 512 // DTYPES[dtype].itemsize
+    g = torch.Generator().manual_seed(T * N + chunks)
+    x, w, b = (torch.randn(s, generator=g).to(dt) for s in ((T, K), (N, K), (N,)))
+    out = torch.full((parts + 1, T, N), 7.0, device="cuda:0")
+    _lib.seq_call("umb_seq_linear_parts", out, x.cuda(), w.cuda(), b.cuda(), T, N, K, parts, _code(dtype))
+    assert bool((out[parts] == 7.0).all())                     # and nothing behind the last slab
+    want = x.double() @ w.double().T + b.double()
+    bound = 4 * U * K ** 0.5 * (x.double().abs() @ w.double().abs().T + b.double().abs())      # fp32 sums of K products
+    assert ((out[:parts].double().cpu().sum(0) - want).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,groups", [(64, 1), (4096, 1), (2048, 4), (201, 3), (8200, 1)])
+@pytest.mark.parametrize("parts", [1, 2, 3, 4])
+def test_seams_add_the_slabs(W, groups, parts):
+    """every seam over slabs gives what it gives over their sum, formed in the same order"""
+    from umbrella_amd import _lib
+    g = torch.Generator().manual_seed(W + parts)
+    for T in (1, 5, 450 if W <= 4096 else 3):
+        x, w1, w2, w3, w4 = (torch.randn(s, generator=g).cuda() for s in ((T, W), (W,), (W,), (W,), (W,)))
+        y, y2 = (torch.randn(parts, T, W, generator=g).cuda() for _ in range(2))
+
+        def total(t):
+            s = t[0].clone()
+            for p in range(1, parts):
+                s += t[p]
+            return s
+        outs = []
+        for slabs in (True, False):
+            a, b, n = (y.clone(), y2.clone(), parts) if slabs else (total(y), total(y2), 1)
+            xs = [x.clone() for _ in range(3)]
+            hs = [torch.empty_like(x) for _ in range(3)]
+            _lib.seq_call("umb_seq_resid_norm_parts", xs[0], hs[0], a.clone(), n, w1, w2, T, W, groups, 1e-5, _lib.F32)
+            _lib.seq_call("umb_seq_pair_resid_norm_parts", xs[1], hs[1], a.clone(), n, b, n, w1, w2, 0.5, w3, w4, T, W, 1e-5, _lib.F32)
+            _lib.seq_call("umb_hc_seam_parts", xs[2], hs[2], a.clone(), n, None, None, 0.5, None, w1, 1.0, T, W, 1, 1e-5, _lib.F32)
+            outs.append(xs + hs)
+        for got, want in zip(*outs):
+            assert torch.equal(got, want)
+        xs = torch.randn(T, 2, W, generator=g).cuda()             # several streams: the slabs are summed in front of the seam
+        hs = [torch.empty(T, W, device="cuda:0") for _ in range(2)]
+        both = [xs.clone(), xs.clone()]
+        _lib.seq_call("umb_hc_seam_parts", both[0], hs[0], y.clone(), parts, None, None, 0.5, None, w1, 1.0, T, W, 2, 1e-5, _lib.F32)
+        _lib.seq_call("umb_hc_seam", both[1], hs[1], total(y), None, None, 0.5, None, w1, 1.0, T, W, 2, 1e-5, _lib.F32)
+        assert torch.equal(both[0], both[1]) and torch.equal(hs[0], hs[1])

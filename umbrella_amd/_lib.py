@@ -274,7 +274,7 @@ class UmbSeqWork(C.Structure):
                 ("Tmax", C.c_int32), ("Rmax", C.c_int32), ("moe_sel", C.c_void_p), ("moe_wt", C.c_void_p),
                 ("moe_pos", C.c_void_p), ("moe_tiles", C.c_void_p), ("moe_xs", C.c_void_p), ("moe_act", C.c_void_p),
                 ("moe_y", C.c_void_p), ("moe_max_tiles", C.c_int64), ("aux_floats", C.c_int64),
-                ("h2", C.c_void_p), ("y2", C.c_void_p), ("v_first", C.c_void_p)]
+                ("h2", C.c_void_p), ("y2", C.c_void_p), ("v_first", C.c_void_p), ("y_floats", C.c_int64)]
 
 
 class UmbSeqStep(C.Structure):
@@ -288,6 +288,11 @@ _PKV = C.POINTER(UmbPagedKV)
 _FORM = C.POINTER(UmbAttnForm)
 SEQ_SIGNATURES = {
     "umb_seq_linear": [_P, _P, _P, _P, _I, _I, _I, _I, _I],
+    "umb_seq_linear_split": [_P, _P, _I, _I, _I, _I],
+    "umb_seq_linear_parts": [_P, _P, _P, _P, _I, _I, _I, _I, _I],
+    "umb_seq_resid_norm_parts": [_P, _P, _P, _I, _P, _P, _I, _I, _I, _F, _I],
+    "umb_seq_pair_resid_norm_parts": [_P, _P, _P, _I, _P, _I, _P, _P, _F, _P, _P, _I, _I, _F, _I],
+    "umb_hc_seam_parts": [_P, _P, _P, _I, _P, _P, _F, _P, _P, _F, _I, _I, _I, _F, _I],
     "umb_seq_linear_batched": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _L, _L, _I, _P, _I, _I, _I],
     "umb_seq_linear_grouped": [_P, _P, _P, _P, _I, _I, _L, _I, _I, _I, _I],
     "umb_seq_embed": [_P, _P, _P, _F, _I, _I, _I, _I],
@@ -366,7 +371,7 @@ SEQ_SIGNATURES = {
     "umb_sample_rows": [_P, _P, _I, _I, _P, _P, _F, _F, _I, _F, _P, _I, _P, _P],
     "umb_seq_version": [],
 }
-_SEQ_NO_STREAM = {"umb_lat_attend_tiled_ok", "umb_seq_resid_canon_step_ok", "umb_bsa_attend_tiled_ok", "umb_mingru_scratch_floats",
+_SEQ_NO_STREAM = {"umb_lat_attend_tiled_ok", "umb_seq_linear_split", "umb_seq_resid_canon_step_ok", "umb_bsa_attend_tiled_ok", "umb_mingru_scratch_floats",
                   "umb_ssd_scan_chunked_floats", "umb_delta_scan_floats", "umb_gla_scan_chunked_floats"}          # predicates: no stream argument, the value is the answer
 _seq_lib = None
 

@@ -64,6 +64,26 @@ template <typename P> __device__ __forceinline__ void st4(typename El<P>::type* 
   if constexpr (sizeof(typename El<P>::type) == 4) *reinterpret_cast<f32x4*>(p) = v;
   else *reinterpret_cast<u32x2*>(p) = u32x2{pack2<P>(v[0], v[1]), pack2<P>(v[2], v[3])};
 }
+// A sublayer's output may stand in `parts` slabs (at most PARTS_MAX, `slab` floats apart) of partial sums: a product whose K was split.
+// y holds this thread's quads of slab 0; the others' are added in order, their loads all in flight.
+constexpr int PARTS_MAX = 4;
+template <int NE, typename Off> __device__ __forceinline__ void add_parts(f32x4 (&y)[NE], const float* __restrict__ src, int parts, long slab, Off off) {
+  if (parts == 1) return;
+  f32x4 a[NE], b[NE], c[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const float* p = src + off(e) + slab;
+    a[e] = *reinterpret_cast<const f32x4*>(p);
+    if (parts > 2) b[e] = *reinterpret_cast<const f32x4*>(p + slab);
+    if (parts > 3) c[e] = *reinterpret_cast<const f32x4*>(p + 2 * slab);
+  }
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    y[e] += a[e];
+    if (parts > 2) y[e] += b[e];
+    if (parts > 3) y[e] += c[e];
+  }
+}
 __device__ __forceinline__ float sq4(f32x4 v) { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3]; }
 
 // block_sum of a row's squares with the waves' sums added in pairs: with 16 of them one after the other the scale of a row of 4096 was off by

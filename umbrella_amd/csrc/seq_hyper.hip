@@ -229,7 +229,7 @@ template <typename P, int NT, int NE>
 __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x, typename El<P>::type* __restrict__ h, const float* __restrict__ y,
                                                           const float* __restrict__ mix, const float* __restrict__ out, float m,
                                                           const float* __restrict__ in_next, const typename El<P>::type* __restrict__ w_next,
-                                                          float offset, int W, float eps) {
+                                                          float offset, int W, float eps, int parts, long slab) {
   __shared__ float red[NT / 64];
   const long o = (long)blockIdx.x * W;
   const int nq = W / 4;
@@ -242,6 +242,7 @@ __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x,
     yv[e] = *reinterpret_cast<const f32x4*>(y + o + i);
     wn[e] = w_next ? ld4<P>(w_next + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  add_parts<NE>(yv, y, parts, slab, [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; });
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
@@ -337,23 +338,33 @@ static int hc_seam_launch(float* x, void* h, const float* y, const float* mix, c
   return UMB_OK;
 }
 
-extern "C" int umb_hc_seam(float* x, void* h, const float* y, const float* mix, const float* out, float m, const float* in_next,
-                           const void* w_next, float offset, int T, int W, int S, float eps, int dtype, hipStream_t st) {
-  if (T < 1 || W < 1 || S < 1 || S > HC_MAXS || !x || !y || (w_next && !h)) return UMB_EINVAL;
+int seq_sum_parts(float* y, int parts, long slab, hipStream_t st);
+
+extern "C" int umb_hc_seam_parts(float* x, void* h, float* y, int parts, const float* mix, const float* out, float m, const float* in_next,
+                                 const void* w_next, float offset, int T, int W, int S, float eps, int dtype, hipStream_t st) {
+  if (T < 1 || W < 1 || S < 1 || S > HC_MAXS || !x || !y || (w_next && !h) || parts < 1 || parts > PARTS_MAX) return UMB_EINVAL;
+  const long slab = (long)T * W;
   if (S == 1 && quads_ok(W, 1, x, h, y, w_next)) {
 #define HC_SEAM_QUADS(NT, NE)                                                                                                       \
-  hipLaunchKernelGGL((hc_seam_quad_kernel<P, NT, NE>), dim3(T), dim3(NT), 0, st, x, (E*)h, y, mix, out, m, in_next, (const E*)w_next, offset, W, eps)
+  hipLaunchKernelGGL((hc_seam_quad_kernel<P, NT, NE>), dim3(T), dim3(NT), 0, st, x, (E*)h, y, mix, out, m, in_next, (const E*)w_next, offset, W, eps, \
+                     parts, slab)
     DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, (long)T, HC_SEAM_QUADS); })
 #undef HC_SEAM_QUADS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
   }
+  if (const int rc = seq_sum_parts(y, parts, slab, st)) return rc;
   DISPATCH_SEQ_DTYPE(dtype, {
     if (S == 1) return hc_seam_launch<P, 1>(x, h, y, mix, out, m, in_next, w_next, offset, T, W, S, eps, st);
     if (S == 2) return hc_seam_launch<P, 2>(x, h, y, mix, out, m, in_next, w_next, offset, T, W, S, eps, st);
     if (S <= 4) return hc_seam_launch<P, 4>(x, h, y, mix, out, m, in_next, w_next, offset, T, W, S, eps, st);
     return hc_seam_launch<P, HC_MAXS>(x, h, y, mix, out, m, in_next, w_next, offset, T, W, S, eps, st);
   })
+}
+
+extern "C" int umb_hc_seam(float* x, void* h, const float* y, const float* mix, const float* out, float m, const float* in_next,
+                           const void* w_next, float offset, int T, int W, int S, float eps, int dtype, hipStream_t st) {
+  return umb_hc_seam_parts(x, h, const_cast<float*>(y), 1, mix, out, m, in_next, w_next, offset, T, W, S, eps, dtype, st);      // one slab is only read
 }
 
 extern "C" int umb_hc_read(float* u_out, void* h, const float* x, const int* rows, const float* in, const void* w, float offset,

@@ -15,6 +15,7 @@
 // falls back to guarded element loads.
 #include "gemm_tile.h"
 #include "seq_common.h"
+#include <algorithm>
 
 template <typename P> struct Frag8 { u32x4 v; };
 template <> struct Frag8<F32> { f32x4 lo, hi; };
@@ -90,6 +91,7 @@ struct LinExt {
   const float* gate;
   int ldg, sg;
   float limit, alpha;      // EPI_CLAMP_GLU; EPI_CAP: out = limit tanh(acc / limit), fp32
+  int parts;               // > 1: blockIdx.z is a slab of K and not a problem; its sums go to out + z so, the bias into slab 0's
 };
 static inline LinExt lin_dense(int N, int K) { return LinExt{K, N, 0, 0, 0, 0, nullptr, nullptr, 0, 0}; }
 
@@ -543,7 +545,14 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
   }
   const char* wb = reinterpret_cast<const char*>(w + (long)n0 * K);
   const char* xb = reinterpret_cast<const char*>(x + (long)t0 * ldx);
-  const int nc = K * EB / 512;
+  int nc = K * EB / 512;
+  if (ext.parts > 1) {                     // this workgroup's slab of K: chunks c0 .. c0 + nc - 1
+    const int c0 = nc * (int)blockIdx.z / ext.parts;
+    nc = nc * ((int)blockIdx.z + 1) / ext.parts - c0;
+    wb += (long)c0 * 512;
+    xb += (long)c0 * 512;
+    if (blockIdx.z) bias = nullptr;
+  }
   auto issue = [&](int c, int slot) {
     const long at = (long)min(c, nc - 1) * 512;
 #pragma unroll
@@ -781,6 +790,33 @@ extern "C" int umb_seq_linear(void* out, const void* x, const void* w, const voi
                               hipStream_t st) {
   if (!epi_plain(epi)) return UMB_EINVAL;                   // the others have constants: umb_seq_linear_glu, umb_seq_linear_cap
   return seq_linear_any(out, x, w, bias, T, N, K, epi, 0.f, 0.f, dtype, st);
+}
+
+// Slabs of K for a product whose partial sums the kernel behind it adds (the seams), 1: none.  One workgroup per 16 output rows leaves half
+// of the compute units idle below 128 of them, and from 33 tokens on a unit's path is full of token pieces that two slabs with 32 output
+// rows each halve; a slab is four chunks at least (shorter ones are all prologue).  us at 1 / 16 / 48 tokens, bf16, cold weights, one MI355X,
+// 1 slab -> this rule's: 2048 x 8192 10.5 / 12.1 / 18.9 -> 8.8 / 9.5 / 10.8 (4); 2048 x 2048 4.6 / 5.0 / 7.2 -> 3.9 / 4.1 / 5.4 (2); 2560 x 6912 9.3 / 11.1 /
+// 15.3 -> 8.3 / 9.9 / 10.6 (3); 4096 x 14336, 48 tokens 37 -> 26 (2), and 1 / 16 tokens 24.0 / 24.7 stay whole (24.3 / 25.6 in two).
+extern "C" int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype) {
+  if (T < 1 || T > 64 || N < 1 || K < 1) return 1;
+  const int eb = (int)seq_elem_bytes(dtype), chunks = (int)((long)K * eb / 512), blocks = (N + 15) / 16;
+  if (!stream_ok(x, w, N, K, EPI_F32, lin_dense(N, K), eb)) return 1;
+  const int parts = std::min(std::min(512 / blocks, 4), chunks / 4);
+  return parts < 2 || (parts == 2 && blocks > 128 && T <= 32) ? 1 : parts;
+}
+
+extern "C" int umb_seq_linear_parts(float* out, const void* x, const void* w, const void* bias, int T, int N, int K, int parts, int dtype,
+                                    hipStream_t st) {
+  if (T < 1 || N < 1 || K < 1 || parts < 1 || !out || !x || !w) return UMB_EINVAL;
+  if (parts == 1) return umb_seq_linear(out, x, w, bias, T, N, K, EPI_F32, dtype, st);
+  LinExt ext = lin_dense(N, K);
+  ext.so = (long)T * N;
+  ext.parts = parts;
+  DISPATCH_SEQ_DTYPE(dtype, {
+    constexpr int EB = sizeof(typename El<P>::type);
+    if (parts > (long)K * EB / 512 || !stream_ok(x, w, N, K, EPI_F32, ext, EB)) return UMB_EINVAL;
+    return launch_stream<P>(out, x, w, bias, T, N, K, EPI_F32, st, ext, 0, parts);
+  })
 }
 
 extern "C" int umb_seq_linear_glu(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, float limit,

@@ -34,6 +34,14 @@ static inline int lin(const UmbSeqLinear& l, void* out, const void* x, int T, in
   return umb_seq_linear(out, x, l.w, l.bias, T, l.N, l.K, epi, dtype, st);
 }
 
+// a sublayer's last product, summed in slabs where that pays and the seam behind it adds them (*parts; null: it does not)
+static int lin_y(const UmbSeqLinear& l, float* y, const UmbSeqWork* ws, const void* x, int T, int* parts, int dtype, hipStream_t st) {
+  int n = parts ? umb_seq_linear_split(x, l.w, T, l.N, l.K, dtype) : 1;
+  if ((long)n * T * l.N > ws->y_floats) n = 1;
+  if (parts) *parts = n;
+  return n > 1 ? umb_seq_linear_parts(y, x, l.w, l.bias, T, l.N, l.K, n, dtype, st) : lin(l, y, x, T, 0, dtype, st);
+}
+
 static const void* first_norm_of(const UmbSeqModel* m, int l) { return l < m->L ? m->layers[l].norm1 : nullptr; }
 
 // What a sublayer reads.  With a pre-norm the seam kernel has already left norm(x) * w in ws->h.  Without one the sublayer
@@ -52,7 +60,7 @@ static int sublayer_input(const UmbSeqModel* m, const UmbSeqWork* ws, const UmbS
 // The seam behind a sublayer: x <- x + norm(y) * w_post, and what the NEXT sublayer reads.  With a pre-norm that is
 // norm(x) * w_next (same kernel).  Without one, a step of one token per sequence also runs the next sublayer's convolution
 // and state update here (*h_ready); longer steps leave it to sublayer_input, where a token's neighbours are complete.
-static int seam(const UmbSeqModel* m, const UmbSeqWork* ws, const UmbSeqStep* s, const void* w_post, const void* w_next,
+static int seam(const UmbSeqModel* m, const UmbSeqWork* ws, const UmbSeqStep* s, int parts, const void* w_post, const void* w_next,
                 const void* next_canon, float* next_state, bool* h_ready, hipStream_t st) {
   const int T = s->T, W = m->W;
   *h_ready = false;
@@ -61,7 +69,7 @@ static int seam(const UmbSeqModel* m, const UmbSeqWork* ws, const UmbSeqStep* s,
     return umb_seq_resid_canon_step(ws->x, ws->h, ws->y, w_post, next_canon, next_state, s->pos, s->slot, T, W, m->groups,
                                     m->canon_taps, m->eps, m->dtype, st);
   }
-  return umb_seq_resid_norm(ws->x, ws->h, ws->y, w_post, w_next, T, W, m->groups, m->eps, m->dtype, st);
+  return umb_seq_resid_norm_parts(ws->x, ws->h, ws->y, parts, w_post, w_next, T, W, m->groups, m->eps, m->dtype, st);
 }
 
 // the first product of a feed-forward with its activation as epilogue: silu(gate) * up, gelu(gate) * up or the capped form over
@@ -72,20 +80,21 @@ static int lin_act(const UmbSeqLayer& ly, const UmbSeqLinear& l, float limit, vo
   return lin(l, out, x, T, act_epi(ly.act_kind), dt, st);
 }
 
-// feed-forward of h_in (dtype [T][W]) into y_out (fp32 [T][W])
+// feed-forward of h_in (dtype [T][W]) into y_out (fp32 [T][W], in *parts slabs where the caller takes them)
 static int feed_forward(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWork* ws, const UmbSeqStep* s, const void* h_in,
-                        float* y_out, hipStream_t st) {
+                        float* y_out, int* parts, hipStream_t st) {
   const int T = s->T, W = m->W, dt = m->dtype;
+  if (parts) *parts = 1;
   const int epi = act_epi(ly.act_kind), stack = ly.act_kind == UMB_ACT_RELU2 ? 1 : 2;
   if (ly.ff_kind == UMB_FF_GATED) {
     SEQ_TRY(lin_act(ly, ly.gu, ly.act_limit, ws->act, h_in, T, dt, st));
-    return lin(ly.down, y_out, ws->act, T, 0, dt, st);
+    return lin_y(ly.down, y_out, ws, ws->act, T, parts, dt, st);
   }
   if (ly.ff_kind == UMB_FF_POLYNORM) {
     if (!ly.act || ly.gu.N != ly.ff) return UMB_EINVAL;
     SEQ_TRY(lin(ly.gu, ws->proj, h_in, T, 0, dt, st));                         // "up" alone
     SEQ_TRY(umb_polynorm(ws->act, ws->proj, ly.act, T, ly.ff, m->eps, dt, st));
-    return lin(ly.down, y_out, ws->act, T, 0, dt, st);
+    return lin_y(ly.down, y_out, ws, ws->act, T, parts, dt, st);
   }
   if (ly.ff_kind == UMB_FF_MOE) {
     const int E = ly.experts, top = ly.top, F = ly.expert_ff;
@@ -480,7 +489,7 @@ static int forward_parallel_blocks(const UmbSeqModel* m, const UmbSeqWork* ws, c
     SEQ_TRY(lin(ly.proj, ws->proj, ws->h, T, 0, dt, st));
     SEQ_TRY(run_mixer(m, ly, ws, s, st));
     SEQ_TRY(lin(ly.out, ws->y, ws->mix, T, 0, dt, st));
-    if (ly.has_mlp) SEQ_TRY(feed_forward(m, ly, ws, s, ws->h2, ws->y2, st));
+    if (ly.has_mlp) SEQ_TRY(feed_forward(m, ly, ws, s, ws->h2, ws->y2, nullptr, st));
     const float* y2 = ly.has_mlp ? ws->y2 : nullptr;
     const void* w1 = nl ? nl->norm1 : nullptr;
     const void* w2 = nl && nl->has_mlp ? nl->norm2 : nullptr;
@@ -523,24 +532,27 @@ extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const
   else
     SEQ_TRY(umb_seq_embed(ws->x, m->embed, s->tokens, m->embed_scale, T, W, m->V, dt, st));
   bool h_ready = false;
+  int parts = 1, parts2 = 1;
+  // where the slabs of the sublayer's output are counted; a next sublayer that reads through a convolution takes whole sums (its seam's kernel)
+  auto slabs = [&](const void* w_next, const void* canon) { parts = 1; return !hyper && !w_next && canon ? nullptr : &parts; };
   for (int l = 0; l < m->L; ++l) {
     const UmbSeqLayer& ly = m->layers[l];
     const UmbSeqLayer* nl = l + 1 < m->L ? &m->layers[l + 1] : nullptr;
     if (!hyper) SEQ_TRY(sublayer_input(m, ws, s, ly.norm1, ly.canon1, ly.canon_state1, h_ready, st));
     SEQ_TRY(lin(ly.proj, ws->proj, ws->h, T, 0, dt, st));
     SEQ_TRY(run_mixer(m, ly, ws, s, st));
-    SEQ_TRY(lin(ly.out, ws->y, ws->mix, T, 0, dt, st));
+    SEQ_TRY(lin_y(ly.out, ws->y, ws, ws->mix, T, ly.has_mlp ? slabs(ly.norm2, ly.canon2) : slabs(first_norm_of(m, l + 1), nl ? nl->canon1 : nullptr), dt, st));
     if (hyper) {
       // write of this sublayer and read of the next one (the feed-forward, the next layer's mixer, or nothing) in one launch
       const float* in2 = ly.has_mlp ? ly.hc2_in : (nl ? nl->hc1_in : nullptr);
       const void* w2 = ly.has_mlp ? ly.norm2 : (nl ? nl->norm1 : nullptr);
       if ((ly.has_mlp || nl) && !w2) return UMB_EINVAL;
-      SEQ_TRY(umb_hc_seam(ws->x, ws->h, ws->y, ly.hc1_mix, ly.hc1_out, m->resid_mult, in2, w2, m->norm_offset, T, W, S, eps, dt, st));
+      SEQ_TRY(umb_hc_seam_parts(ws->x, ws->h, ws->y, parts, ly.hc1_mix, ly.hc1_out, m->resid_mult, in2, w2, m->norm_offset, T, W, S, eps, dt, st));
       if (ly.has_mlp) {
-        SEQ_TRY(feed_forward(m, ly, ws, s, ws->h, ws->y, st));
+        SEQ_TRY(feed_forward(m, ly, ws, s, ws->h, ws->y, &parts, st));
         if (nl && !nl->norm1) return UMB_EINVAL;
-        SEQ_TRY(umb_hc_seam(ws->x, ws->h, ws->y, ly.hc2_mix, ly.hc2_out, m->resid_mult, nl ? nl->hc1_in : nullptr,
-                            nl ? nl->norm1 : nullptr, m->norm_offset, T, W, S, eps, dt, st));
+        SEQ_TRY(umb_hc_seam_parts(ws->x, ws->h, ws->y, parts, ly.hc2_mix, ly.hc2_out, m->resid_mult, nl ? nl->hc1_in : nullptr,
+                                  nl ? nl->norm1 : nullptr, m->norm_offset, T, W, S, eps, dt, st));
       }
       if (s->trace) SEQ_TRY(umb_hc_read(s->trace + (long)l * T * W, nullptr, ws->x, nullptr, nullptr, nullptr, 0.f, T, W, S, eps, dt, st));
       continue;
@@ -548,17 +560,17 @@ extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const
     const void* next = ly.has_mlp ? ly.norm2 : first_norm_of(m, l + 1);
     if (ly.kind == UMB_MIX_ATTN_DELTA) {
       const void* right = static_cast<char*>(ws->mix) + mix_right(ly, T) * seq_elem_bytes(dt);
-      SEQ_TRY(lin(ly.out2, ws->y2, right, T, 0, dt, st));
-      SEQ_TRY(umb_seq_pair_resid_norm(ws->x, ws->h, ws->y, ws->y2, ly.out_norm_a, ly.out_norm_b, ly.pair_coef, ly.norm1b, next, T, W, eps, dt,
-                                      st));
+      SEQ_TRY(lin_y(ly.out2, ws->y2, ws, right, T, &parts2, dt, st));
+      SEQ_TRY(umb_seq_pair_resid_norm_parts(ws->x, ws->h, ws->y, parts, ws->y2, parts2, ly.out_norm_a, ly.out_norm_b, ly.pair_coef, ly.norm1b,
+                                            next, T, W, eps, dt, st));
       h_ready = false;
     } else
-      SEQ_TRY(seam(m, ws, s, ly.norm1b, next, ly.has_mlp ? ly.canon2 : (nl ? nl->canon1 : nullptr),
+      SEQ_TRY(seam(m, ws, s, parts, ly.norm1b, next, ly.has_mlp ? ly.canon2 : (nl ? nl->canon1 : nullptr),
   ly.has_mlp ? ly.canon_state2 : (nl ? nl->canon_state1 : nullptr), &h_ready, st));
     if (ly.has_mlp) {
       SEQ_TRY(sublayer_input(m, ws, s, ly.norm2, ly.canon2, ly.canon_state2, h_ready, st));
-      SEQ_TRY(feed_forward(m, ly, ws, s, ws->h, ws->y, st));
-      SEQ_TRY(seam(m, ws, s, ly.norm2b, first_norm_of(m, l + 1), nl ? nl->canon1 : nullptr, nl ? nl->canon_state1 : nullptr,
+      SEQ_TRY(feed_forward(m, ly, ws, s, ws->h, ws->y, slabs(first_norm_of(m, l + 1), nl ? nl->canon1 : nullptr), st));
+      SEQ_TRY(seam(m, ws, s, parts, ly.norm2b, first_norm_of(m, l + 1), nl ? nl->canon1 : nullptr, nl ? nl->canon_state1 : nullptr,
                    &h_ready, st));
     }
     if (s->trace) {

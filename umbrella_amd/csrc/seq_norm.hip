@@ -324,7 +324,8 @@ __global__ __launch_bounds__(256) void pair_resid_norm_kernel(float* __restrict_
 template <typename P, int NT, int NE>
 __global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__ x, typename El<P>::type* __restrict__ h,
                                                              const float* __restrict__ y, const typename El<P>::type* __restrict__ w_post,
-                                                             const typename El<P>::type* __restrict__ w_next, int W, int groups, float eps) {
+                                                             const typename El<P>::type* __restrict__ w_next, int W, int groups, float eps,
+                                                             int parts, long slab) {
   __shared__ float red[NT / 64], red2[NT / 64];
   const int grp = blockIdx.y, gs = W / groups, nq = gs / 4;
   const long o = (long)blockIdx.x * W + (long)grp * gs;
@@ -337,6 +338,7 @@ __global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__
     wp[e] = ld4<P>(w_post + grp * gs + i);
     wn[e] = w_next ? ld4<P>(w_next + grp * gs + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  add_parts<NE>(yv, y, parts, slab, [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; });
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) ss += (int)threadIdx.x + NT * e < nq ? sq4(yv[e]) : 0.f;
@@ -400,7 +402,8 @@ __global__ __launch_bounds__(NT) void pair_resid_norm_quad_kernel(float* __restr
                                                                   const typename El<P>::type* __restrict__ w1,
                                                                   const typename El<P>::type* __restrict__ w2, float coef,
                                                                   const typename El<P>::type* __restrict__ w_post,
-                                                                  const typename El<P>::type* __restrict__ w_next, int W, float eps) {
+                                                                  const typename El<P>::type* __restrict__ w_next, int W, float eps,
+                                                                  int parts1, int parts2, long slab) {
   __shared__ float red[4][NT / 64];
   const long o = (long)blockIdx.x * W;
   const int nq = W / 4;
@@ -416,6 +419,9 @@ __global__ __launch_bounds__(NT) void pair_resid_norm_quad_kernel(float* __restr
     wp[e] = ld4<P>(w_post + i);
     wn[e] = w_next ? ld4<P>(w_next + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  const auto at = [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; };
+  add_parts<NE>(a, y1, parts1, slab, at);
+  add_parts<NE>(b, y2, parts2, slab, at);
   float sa = 0.f, sb = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
@@ -499,18 +505,35 @@ extern "C" int umb_seq_embed_norm(float* x, void* h, const void* embed, const in
   return UMB_OK;
 }
 
-extern "C" int umb_seq_resid_norm(float* x, void* h, const float* y, const void* w_post, const void* w_next, int T, int W,
-                                  int groups, float eps, int dtype, hipStream_t st) {
-  if (!norm_args_ok(T, W, groups) || !x || !y || !w_post || (w_next && !h)) return UMB_EINVAL;
-  if (quads_ok(W, groups, x, h, y, w_post, w_next)) {
+// slabs 1 .. parts - 1 added onto slab 0, for a seam that is not walked in quads
+__global__ __launch_bounds__(256) void sum_parts_kernel(float* __restrict__ y, int parts, long slab) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= slab) return;
+  float v = y[i];
+  for (int p = 1; p < parts; ++p) v += y[i + p * slab];
+  y[i] = v;
+}
+int seq_sum_parts(float* y, int parts, long slab, hipStream_t st) {
+  if (parts < 2) return UMB_OK;
+  hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)((slab + 255) / 256)), dim3(256), 0, st, y, parts, slab);
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+
+extern "C" int umb_seq_resid_norm_parts(float* x, void* h, float* y, int parts, const void* w_post, const void* w_next, int T, int W,
+                                        int groups, float eps, int dtype, hipStream_t st) {
+  if (!norm_args_ok(T, W, groups) || !x || !y || !w_post || (w_next && !h) || parts < 1 || parts > PARTS_MAX) return UMB_EINVAL;
+  const long slab = (long)T * W;
+  if (quads_ok(W, groups, x, h, y, w_post, w_next) && (parts == 1 || W % 4 == 0)) {
 #define SEAM_QUADS(NT, NE)                                                                                                      \
   hipLaunchKernelGGL((resid_norm_quad_kernel<P, NT, NE>), dim3(T, groups), dim3(NT), 0, st, x, (E*)h, y, (const E*)w_post, (const E*)w_next, \
-                     W, groups, eps)
+                     W, groups, eps, parts, slab)
     DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W / groups, (long)T * groups, SEAM_QUADS); })
 #undef SEAM_QUADS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
   }
+  if (const int rc = seq_sum_parts(y, parts, slab, st)) return rc;
   DISPATCH_SEQ_DTYPE(dtype, {
     typedef typename El<P>::type E;
     const int per_lane = (W / groups + 63) / 64;
@@ -534,6 +557,11 @@ extern "C" int umb_seq_resid_norm(float* x, void* h, const float* y, const void*
   })
   UMB_LAUNCH_CHECK();
   return UMB_OK;
+}
+
+extern "C" int umb_seq_resid_norm(float* x, void* h, const float* y, const void* w_post, const void* w_next, int T, int W, int groups, float eps,
+                                  int dtype, hipStream_t st) {
+  return umb_seq_resid_norm_parts(x, h, const_cast<float*>(y), 1, w_post, w_next, T, W, groups, eps, dtype, st);      // one slab is only read
 }
 
 extern "C" int umb_seq_resid_canon_step_ok(int W, int groups) {
@@ -565,18 +593,24 @@ extern "C" int umb_seq_resid_canon_step(float* x, void* h, const float* y, const
   return UMB_OK;
 }
 
-extern "C" int umb_seq_pair_resid_norm(float* x, void* h, const float* y1, const float* y2, const void* w1, const void* w2, float coef,
-                                       const void* w_post, const void* w_next, int T, int W, float eps, int dtype, hipStream_t st) {
-  if (!norm_args_ok(T, W, 1) || !x || !y1 || !y2 || !w1 || !w2 || !w_post || (w_next && !h)) return UMB_EINVAL;
+extern "C" int umb_seq_pair_resid_norm_parts(float* x, void* h, float* y1, int parts1, float* y2, int parts2, const void* w1, const void* w2,
+                                             float coef, const void* w_post, const void* w_next, int T, int W, float eps, int dtype,
+                                             hipStream_t st) {
+  if (!norm_args_ok(T, W, 1) || !x || !y1 || !y2 || !w1 || !w2 || !w_post || (w_next && !h) || parts1 < 1 || parts1 > PARTS_MAX ||
+      parts2 < 1 || parts2 > PARTS_MAX)
+    return UMB_EINVAL;
+  const long slab = (long)T * W;
   if (quads_ok(W, 1, x, h, y1, y2, w1, w2, w_post) && (uintptr_t)w_next % 16 == 0) {
 #define PAIR_QUADS(NT, NE)                                                                                                          \
   hipLaunchKernelGGL((pair_resid_norm_quad_kernel<P, NT, NE>), dim3(T), dim3(NT), 0, st, x, (E*)h, y1, y2, (const E*)w1, (const E*)w2, coef, \
-                     (const E*)w_post, (const E*)w_next, W, eps)
+                     (const E*)w_post, (const E*)w_next, W, eps, parts1, parts2, slab)
     DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, (long)T, PAIR_QUADS); })
 #undef PAIR_QUADS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
   }
+  if (const int rc = seq_sum_parts(y1, parts1, slab, st)) return rc;
+  if (const int rc = seq_sum_parts(y2, parts2, slab, st)) return rc;
 #define PAIR_SEAM(EPT)                                                                                                          \
   hipLaunchKernelGGL((pair_resid_norm_kernel<P, EPT>), dim3(T), dim3(256), 0, st, x, (E*)h, y1, y2, (const E*)w1, (const E*)w2, \
                      coef, (const E*)w_post, (const E*)w_next, W, eps)
@@ -590,4 +624,10 @@ extern "C" int umb_seq_pair_resid_norm(float* x, void* h, const float* y1, const
 #undef PAIR_SEAM
   UMB_LAUNCH_CHECK();
   return UMB_OK;
+}
+
+extern "C" int umb_seq_pair_resid_norm(float* x, void* h, const float* y1, const float* y2, const void* w1, const void* w2, float coef,
+                                       const void* w_post, const void* w_next, int T, int W, float eps, int dtype, hipStream_t st) {
+  return umb_seq_pair_resid_norm_parts(x, h, const_cast<float*>(y1), 1, const_cast<float*>(y2), 1, w1, w2, coef, w_post, w_next, T, W, eps, dtype,
+                                       st);                  // one slab is only read
 }

@@ -423,11 +423,12 @@ class SeqMixLM(LLMBase):
             elif ly.ff:
                 ask(act=ly.ff, proj=ly.ff if ly.ff_kind == "polynorm" else 1)
         f32, i32 = torch.float32, torch.int32
+        y_rows = max(T, 4 * min(T, 64))                 # few-token products leave up to four slabs of partial sums
         b = self._bufs = dict(
             x=torch.zeros(T, max(1, c.streams) * c.width, dtype=f32, device=dev), h=torch.zeros(T, c.width, dtype=dt, device=dev),
             proj=torch.zeros(T, need["proj"], dtype=f32, device=dev), aux=torch.zeros(T, need["aux"], dtype=f32, device=dev),
             o=torch.zeros(T, need["o"], dtype=f32, device=dev), mix=torch.zeros(T, need["mix"], dtype=dt, device=dev),
-            act=torch.zeros(T, need["act"], dtype=dt, device=dev), y=torch.zeros(T, c.width, dtype=f32, device=dev),
+            act=torch.zeros(T, need["act"], dtype=dt, device=dev), y=torch.zeros(y_rows, c.width, dtype=f32, device=dev),
             logits=torch.zeros(R, c.vocab_size, dtype=f32, device=dev))
         ws = self._ws = UmbSeqWork()
         for k in ("x", "h", "proj", "aux", "o", "mix", "act", "y", "logits"):
@@ -436,7 +437,7 @@ class SeqMixLM(LLMBase):
             b["h2"] = torch.zeros(T, c.width, dtype=dt, device=dev)
             ws.h2 = b["h2"].data_ptr()
         if c.block == "parallel" or any(ly.mixer.kind == "attention_delta" for ly in c.layers):
-            b["y2"] = torch.zeros(T, c.width, dtype=f32, device=dev)     # its output; the second output projection's
+            b["y2"] = torch.zeros(y_rows, c.width, dtype=f32, device=dev)     # its output; the second output projection's
             ws.y2 = b["y2"].data_ptr()
         if self._v_width:                               # values that later layers of the step mix in
             b["v_first"] = torch.zeros(T, self._v_width, dtype=f32, device=dev)
@@ -451,7 +452,7 @@ class SeqMixLM(LLMBase):
             for k in ("moe_sel", "moe_wt", "moe_pos", "moe_tiles", "moe_xs", "moe_act", "moe_y"):
                 setattr(ws, k, b[k].data_ptr())
             ws.moe_max_tiles = tiles
-        ws.Tmax, ws.Rmax, ws.aux_floats = T, R, b["aux"].numel()
+        ws.Tmax, ws.Rmax, ws.aux_floats, ws.y_floats = T, R, b["aux"].numel(), b["y"].numel()
         self.ws_tokens, self.logit_rows = T, R
 
     @property

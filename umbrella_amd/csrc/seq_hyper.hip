@@ -234,13 +234,15 @@ __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x,
   const long o = (long)blockIdx.x * W;
   const int nq = W / 4;
   const float mx = mix ? mix[0] : 1.f, ot = out ? out[0] : 1.f, in0 = in_next ? in_next[0] : 1.f;
+  // read either way (without a next norm from the row's first slab): behind a test the load is a round trip of its own
+  const typename El<P>::type* wq = w_next ? w_next : reinterpret_cast<const typename El<P>::type*>(y);
   f32x4 xv[NE], yv[NE], wn[NE];
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int i = min((int)threadIdx.x + NT * e, nq - 1) * 4;
     xv[e] = *reinterpret_cast<const f32x4*>(x + o + i);
     yv[e] = *reinterpret_cast<const f32x4*>(y + o + i);
-    wn[e] = w_next ? ld4<P>(w_next + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+    wn[e] = ld4<P>(wq + i);
   }
   add_parts<NE>(yv, y, parts, slab, [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; });
   float ss = 0.f;
@@ -269,12 +271,13 @@ __global__ __launch_bounds__(NT) void hc_embed_quad_kernel(float* __restrict__ x
   const long o = (long)blockIdx.x * W, src = (long)min(max(tokens[blockIdx.x], 0), V - 1) * W;
   const int nq = W / 4;
   const float in0 = in ? in[0] : 1.f;
+  const typename El<P>::type* wq = h ? w : embed;
   f32x4 ev[NE], wv[NE];
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int i = min((int)threadIdx.x + NT * e, nq - 1) * 4;
     ev[e] = ld4<P>(embed + src + i);
-    wv[e] = h ? ld4<P>(w + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+    wv[e] = ld4<P>(wq + i);
   }
   float ss = 0.f;
 #pragma unroll

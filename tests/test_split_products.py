@@ -41,6 +41,39 @@ def test_slabs_add_up_to_the_product(dtype, T, N, chunks, parts):
     assert ((out[:parts].double().cpu().sum(0) - want).abs() <= bound).all()
 
 
+# more row blocks than the chip holds workgroups (16 rows a block up to 32 tokens and in gate/up, 32 beyond): one block past it, ragged, a third
+# round; as many chunks as the ring has slots, one less (not run on), and more; 65 tokens: two token tiles
+RUNS = [(1, 16 * 768 + 1, 4), (8, 16 * 1600 - 3, 5), (16, 16 * 513, 4), (16, 16 * 512, 9), (17, 16 * 257 - 8, 3), (32, 16 * 530 + 2, 4), (32, 16 * 300, 2),
+        (33, 32 * 256 + 2, 3), (48, 32 * 520 - 6, 8), (64, 32 * 257, 7), (65, 32 * 130, 4)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("T,N,chunks", RUNS)
+def test_streams_run_on_from_block_to_block(dtype, T, N, chunks):
+    from umbrella_amd import _lib
+    dt, K = DTYPES[dtype], chunks * 512 // DTYPES[dtype].itemsize
+    g = torch.Generator(device="cuda").manual_seed(T * N + chunks)
+    x, w, b = (torch.randn(s, generator=g, device="cuda").to(dt) for s in ((T, K), (N, K), (N,)))
+    want, size = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
+    bound = 4 * U * K ** 0.5 * size
+    out = torch.full((T + 1, N), 7.0, device="cuda")
+    _lib.seq_call("umb_seq_linear", out, x, w, b, T, N, K, 0, _code(dtype))
+    assert ((out[:T].double() - want).abs() <= bound).all() and bool((out[T] == 7.0).all())
+    half = N // 2
+    for n in {half, N // 2 * 2}:                               # stacked halves of half and of whole height: silu(gate) * up
+        w2 = torch.cat([w[:n], w[:n].flip(0)]).contiguous()
+        full = x.double() @ w2.double().T
+        size = x.double().abs() @ w2.double().abs().T
+        gate, up, tol = full[:, :n], full[:, n:], 4 * U * K ** 0.5 * size
+        act = torch.full((T + 1, n), 7.0, dtype=dt, device="cuda")
+        _lib.seq_call("umb_seq_linear", act, x, w2, None, T, 2 * n, K, 2, _code(dtype))
+        ref = gate * torch.sigmoid(gate) * up
+        ulp = {"bf16": 2.0 ** -8, "fp32": 2.0 ** -23}[dtype]
+        slack = 1.1 * tol[:, :n] * up.abs() + gate.abs() * tol[:, n:] + 1.02 * ulp * ref.abs() + 1e-6 * ref.abs() + 1e-20
+        assert ((act[:T].double() - ref).abs() <= slack).all() and bool((act[T] == 7.0).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("W,groups", [(64, 1), (4096, 1), (2048, 4), (201, 3), (8200, 1)])
 @pytest.mark.parametrize("parts", [1, 2, 3, 4])

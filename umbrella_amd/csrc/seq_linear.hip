@@ -10,8 +10,8 @@
 // a <= 64-token launch), as in the skinny GEMM of gemm.hip.
 //
 // Few tokens: a workgroup owns 16 (or 32) output rows and up to 64 tokens; its four waves split K (wave w takes the 32-k steps w, w+4, ...)
-// and their partial tiles are summed through LDS in wave order: the summation order of an output is a function of K alone,
-// never of the row's place in the batch, and of T only where the many-token kernels take over (launch_vec).  K % 8 != 0 (or a tail)
+// and their partial tiles are summed through LDS in wave order: the summation order of an output is a function of K and of its row block,
+// never of the row's place in the batch, and of T only where another kernel or another block height takes over (launch_vec, launch_stream).  K % 8 != 0 (or a tail)
 // falls back to guarded element loads.
 #include "gemm_tile.h"
 #include "seq_common.h"
@@ -91,7 +91,9 @@ struct LinExt {
   const float* gate;
   int ldg, sg;
   float limit, alpha;      // EPI_CLAMP_GLU; EPI_CAP: out = limit tanh(acc / limit), fp32
-  int parts;               // > 1: blockIdx.z is a slab of K and not a problem; its sums go to out + z so, the bias into slab 0's
+  // streaming kernel.  parts > 1: blockIdx.z is a slab of K and not a problem, part_chunks 512-byte chunks (one more in the first ones); its sums go to
+  // out + z so, the bias into slab 0's.  step: distance of a workgroup's row blocks (gridDim.x, read with the other arguments)
+  int parts, part_chunks, step;
 };
 static inline LinExt lin_dense(int N, int K) { return LinExt{K, N, 0, 0, 0, 0, nullptr, nullptr, 0, 0}; }
 
@@ -477,15 +479,14 @@ static int launch_wide(void* out, const void* x, const void* w, const void* bias
 // its TOKEN fragments (4096 x 14336 weights: 27 us with 1 token, 38 with 16, 80 with 64).  Here a workgroup walks K in chunks of 512
 // bytes per row: LDS-DMA pieces of two rows (whole lines, 4 channels' worth each) into a ring of R slots, R - 1 chunks ahead, one
 // barrier per chunk; the tokens of a chunk are fetched once per workgroup and not once per wave; fragments come from LDS without bank
-// conflicts (pieces 1040 B apart, columns of odd rows XOR 8).  Wave w takes the 32-k steps w, w + 4, ... as above: the same bits.
+// conflicts (pieces 1040 B apart, columns of odd rows XOR 8).  Wave w takes the 32-k steps w, w + 4, ... of a chunk.
 // us, cold weights, one MI355X: 4096 x 14336, 1 / 16 / 48 / 64 tokens 27 / 38 / 66 / 80 -> 24 / 25 / 38 / 41; 2048 x 2048, 48 tokens
 // 11.7 -> 7.3; gate/up 28672 x 4096, 1 / 16 / 48 tokens 49 / 58 / 88 -> 42 / 43 / 56 (5.6 TB/s at 1 token).
 template <int NT, int TT, int BP, bool DUAL, int R> struct StreamShape {     // BP: token pieces (8 TT, fewer for very few tokens)
   static constexpr int AP = (DUAL ? 16 : 8) * NT, NP = AP + BP, PW = (NP + 3) / 4, AT = DUAL ? 2 * NT : NT;
   static constexpr unsigned PIECE = 1040u, SLOT = NP * PIECE;
-  static constexpr size_t RED = (size_t)AT * 4 * TT * 1024, RING = (size_t)R * SLOT + (NP % 4 ? PIECE : 0);
-  static constexpr size_t LDS = RING > RED ? RING : RED;
-  static_assert(AP % 4 == 0 && R >= 2 && LDS <= 160 * 1024, "whole rounds of weight pieces; the CU's LDS");
+  static constexpr size_t RED = (size_t)AT * 4 * TT * 1024, LDS = (size_t)R * SLOT + (NP % 4 ? PIECE : 0);
+  static_assert(AP % 4 == 0 && R >= 2 && LDS <= 160 * 1024 && RED <= SLOT, "whole rounds of weight pieces; the CU's LDS");
   static_assert(BP % TT == 0 && (BP == 8 * TT || TT == 1), "token tiles of whole pieces");
   // place of a tile's row inside a slot; a token tile staged in part repeats its pieces: columns that are not stored
   static constexpr unsigned row_at(int first_piece, int pieces, int row) { return (unsigned)(first_piece + (row >> 1) % pieces) * PIECE + (unsigned)(row & 1) * 512u; }
@@ -499,7 +500,10 @@ template <int NT, int TT, int BP, bool DUAL, int R> struct StreamShape {     // 
     return true;
   }
 };
-template <typename P, int NT, int TT, int BP, bool DUAL, int R>
+// The row blocks that one XCD works on side by side (every eighth) walk K from eight places: in step they would all ask for the same 512 bytes
+// of rows a power of two apart, which stand on a quarter of the L2's channels (10240 x 4096, 48 tokens: 32.1 -> 26.3 us; 32000 x 2048, 1 token 27.9 -> 24.2).
+__device__ __forceinline__ int first_chunk(int block, int chunks) { return ((block >> 3) & 7) * chunks / 8; }
+template <typename P, int NT, int TT, int BP, bool DUAL, int R, bool RUN>
 __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict__ out_, const typename El<P>::type* __restrict__ x,
                                                                 const typename El<P>::type* __restrict__ w,
                                                                 const typename El<P>::type* __restrict__ bias, int T, int N, int K,
@@ -512,7 +516,7 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, g = lane >> 4;
   int t0 = blockIdx.y * (TT * 16);
-  const int ldx = ext.ldx, ldo = ext.ldo;
+  const int ldx = ext.ldx, ldo = ext.ldo, parts = ext.parts, step = ext.step;
   long obase = (long)blockIdx.z * ext.so;
   const float* gate = ext.gate ? ext.gate + (long)blockIdx.z * ext.sg : nullptr;
   x += (long)blockIdx.z * ext.sx;
@@ -528,38 +532,47 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
     T = rows;
     t0 = 0;
   }
-  const int n0 = blockIdx.x * 16 * NT;
   const unsigned lds0 = (unsigned)(size_t)(lds_char*)smem;
   // piece p: rows 2 p and 2 p + 1 (lanes 0 - 31, 32 - 63) of the operand; rows past its end re-read the last one: not stored
   unsigned voff[S::PW];
+  auto rows_of_block = [&](int n0) {       // the weight pieces' offsets from row n0
 #pragma unroll
-  for (int i = 0; i < S::PW; ++i) {
-    const int p = wave + 4 * i, odd = lane >> 5, c = (lane & 31) ^ (odd * 8);
-    if (4 * i < S::AP) {
-      const int r = 2 * p + odd;
+    for (int i = 0; i < S::AP / 4; ++i) {
+      const int odd = lane >> 5, c = (lane & 31) ^ (odd * 8), r = 2 * (wave + 4 * i) + odd;
       const int n = DUAL && r >= 16 * NT ? N + min(n0 + r - 16 * NT, N - 1) : min(n0 + r, N - 1);
       voff[i] = (unsigned)(n - n0) * (unsigned)K * EB + c * 16u;
-    } else {
-      voff[i] = (unsigned)(min(t0 + 2 * (p - S::AP) + odd, T - 1) - t0) * (unsigned)ldx * EB + c * 16u;
     }
+  };
+#pragma unroll
+  for (int i = S::AP / 4; i < S::PW; ++i) {
+    const int odd = lane >> 5, c = (lane & 31) ^ (odd * 8);
+    voff[i] = (unsigned)(min(t0 + 2 * (wave + 4 * i - S::AP) + odd, T - 1) - t0) * (unsigned)ldx * EB + c * 16u;
   }
-  const char* wb = reinterpret_cast<const char*>(w + (long)n0 * K);
+  const char* wb = reinterpret_cast<const char*>(w);
   const char* xb = reinterpret_cast<const char*>(x + (long)t0 * ldx);
   int nc = K * EB / 512;
-  if (ext.parts > 1) {                     // this workgroup's slab of K: chunks c0 .. c0 + nc - 1
-    const int c0 = nc * (int)blockIdx.z / ext.parts;
-    nc = nc * ((int)blockIdx.z + 1) / ext.parts - c0;
+  if (parts > 1) {                         // this workgroup's slab of K: chunks c0 .. c0 + nc - 1
+    const int z = blockIdx.z, longer = nc - parts * ext.part_chunks, c0 = z * ext.part_chunks + min(z, longer);
+    nc = ext.part_chunks + (z < longer);
     wb += (long)c0 * 512;
     xb += (long)c0 * 512;
-    if (blockIdx.z) bias = nullptr;
+    if (z) bias = nullptr;
   }
-  auto issue = [&](int c, int slot) {
-    const long at = (long)min(c, nc - 1) * 512;
+  // the row blocks of this workgroup, blockIdx.x, + step, ...: their chunks are ONE sequence, the ring runs on over the end of a block
+  const int nb = (N + 16 * NT - 1) / (16 * NT);
+  int fb = blockIdx.x, left = nc;          // the block that is fetched, its chunks that are still to come
+  int col = first_chunk(fb, nc);                // and the next of them: they are taken in turn from this one on
+  const char* fw = wb + (long)fb * (16 * NT) * K * EB;
+  rows_of_block(fb * (16 * NT));
+  auto issue = [&](int slot) {
+    const long at = (long)col * 512;
+    col = col + 1 == nc ? 0 : col + 1;     // past the last chunk of all: fetched again, never read
+    --left;
 #pragma unroll
     for (int i = 0; i < S::PW; ++i) {
       unsigned dst = lds0 + (unsigned)slot * S::SLOT + (unsigned)(wave + 4 * i) * S::PIECE;
       if (S::NP % 4 && i == S::PW - 1 && wave + 4 * i >= S::NP) dst = lds0 + (unsigned)R * S::SLOT;      // a piece of nobody's
-      tile_dma(voff[i], (4 * i < S::AP ? wb : xb) + at, dst);
+      tile_dma(voff[i], (4 * i < S::AP ? fw : xb) + at, dst);
     }
   };
   f32x4 acc[AT][TT];
@@ -579,87 +592,123 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
     return f;
   };
 #pragma unroll
-  for (int c = 0; c < R - 1; ++c) issue(c, c);
+  for (int c = 0; c < R - 1; ++c) issue(c);
   int slot = 0;
-  for (int c = 0; c < nc; ++c) {
-    // this wave's pieces of the chunk have landed and its fragments of the chunk before are in registers; behind the barrier that holds
-    // for every wave: the chunk can be read, and the slot of the chunk before filled again
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((R - 2) * S::PW) : "memory");
-    __builtin_amdgcn_s_barrier();
-    issue(c + R - 1, slot == 0 ? R - 1 : slot - 1);
-    const unsigned base = lds0 + (unsigned)slot * S::SLOT;
+  for (int block = blockIdx.x; block < nb; block += step) {
+    const int n0 = block * 16 * NT;
 #pragma unroll
-    for (int u = 0; u < STEPS / 4; ++u) {
-      const int s = wave + 4 * u;
-      Frag8<P> a[AT], b[TT];
+    for (int i = 0; i < AT; ++i)
 #pragma unroll
-      for (int i = 0; i < AT; ++i) a[i] = frag(base + wrow + (unsigned)(8 * i) * S::PIECE, s);
+      for (int tt = 0; tt < TT; ++tt) acc[i][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    unsigned base = lds0;
+    for (int c = 0; c < nc; ++c) {
+      // this wave's pieces of the chunk have landed and its fragments of the chunk before are in registers; behind the barrier that holds
+      // for every wave: the chunk can be read, and the slot of the chunk before filled again
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((R - 2) * S::PW) : "memory");
+      __builtin_amdgcn_s_barrier();
+      if (RUN && __builtin_expect(left == 0 && fb + step < nb, 0)) {
+        fb += step;
+        left = nc;
+        col = first_chunk(fb, nc);
+        fw = wb + (long)fb * (16 * NT) * K * EB;
+        rows_of_block(fb * (16 * NT));
+      }
+      issue(slot == 0 ? R - 1 : slot - 1);
+      base = lds0 + (unsigned)slot * S::SLOT;
 #pragma unroll
-      for (int tt = 0; tt < TT; ++tt) b[tt] = frag(base + trow + (unsigned)(8 * tt) * S::PIECE, s);
+      for (int u = 0; u < STEPS / 4; ++u) {
+        const int s = wave + 4 * u;
+        Frag8<P> a[AT], b[TT];
 #pragma unroll
-      for (int tt = 0; tt < TT; ++tt)
+        for (int i = 0; i < AT; ++i) a[i] = frag(base + wrow + (unsigned)(8 * i) * S::PIECE, s);
 #pragma unroll
-        for (int i = 0; i < AT; ++i) acc[i][tt] = mma8<P>(a[i], b[tt], acc[i][tt]);
+        for (int tt = 0; tt < TT; ++tt) b[tt] = frag(base + trow + (unsigned)(8 * tt) * S::PIECE, s);
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+          for (int i = 0; i < AT; ++i) acc[i][tt] = mma8<P>(a[i], b[tt], acc[i][tt]);
+      }
+      slot = slot + 1 == R ? 0 : slot + 1;
     }
-    slot = slot + 1 == R ? 0 : slot + 1;
-  }
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  float* red = reinterpret_cast<float*>(smem);                       // [wave][AT][TT][256], over the ring
+    // the waves' tiles are added in the slot of the block's last chunk, which the next block's first barrier hands back to the ring
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    const unsigned red = base;                                         // [wave][AT][TT][256] floats
 #pragma unroll
-  for (int i = 0; i < AT; ++i)
+    for (int i = 0; i < AT; ++i)
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) *reinterpret_cast<f32x4*>(red + ((wave * AT + i) * TT + tt) * 256 + lane * 4) = acc[i][tt];
-  __syncthreads();
-  const int l = threadIdx.x >> 2, r = threadIdx.x & 3;
-  auto total = [&](int i, int tt) {
-    float s = red[(i * TT + tt) * 256 + threadIdx.x];
+      for (int tt = 0; tt < TT; ++tt) *reinterpret_cast<lds_f32x4*>((size_t)(red + (((wave * AT + i) * TT + tt) * 256 + lane * 4) * 4u)) = acc[i][tt];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    const int l = threadIdx.x >> 2, r = threadIdx.x & 3;
+    auto total = [&](int i, int tt) {
+      const auto at = [&](int ww) { return *reinterpret_cast<const lds_f32*>((size_t)(red + (((ww * AT + i) * TT + tt) * 256 + threadIdx.x) * 4u)); };
+      float s = at(0);
 #pragma unroll
-    for (int ww = 1; ww < 4; ++ww) s += red[((ww * AT + i) * TT + tt) * 256 + threadIdx.x];
-    return s;
-  };
+      for (int ww = 1; ww < 4; ++ww) s += at(ww);
+      return s;
+    };
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int n = n0 + nt * 16 + 4 * (l >> 4) + r;
-    if (n >= N) continue;
-    const float bv = bias ? ldf<P>(bias + n) : 0.f;
-    const float bv2 = (DUAL && bias) ? ldf<P>(bias + N + n) : 0.f;
+    for (int nt = 0; nt < NT; ++nt) {
+      const int n = n0 + nt * 16 + 4 * (l >> 4) + r;
+      if (n >= N) continue;
+      const float bv = bias ? ldf<P>(bias + n) : 0.f;
+      const float bv2 = (DUAL && bias) ? ldf<P>(bias + N + n) : 0.f;
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      const int t = t0 + tt * 16 + (l & 15);
-      if (t >= T) continue;
-      const float s = total(nt, tt) + bv;
-      const long o = obase + (long)t * ldo + n;
-      if constexpr (DUAL) {
-        stf<P>(reinterpret_cast<E*>(out_) + o, glu_pair(epi, s, total(NT + nt, tt) + bv2, ext.limit, ext.alpha));
-      } else if (epi == EPI_DT) {
-        stf<P>(reinterpret_cast<E*>(out_) + o, s);
-      } else if (epi == EPI_RELU2) {
-        const float rl = fmaxf(s, 0.f);
-        stf<P>(reinterpret_cast<E*>(out_) + o, rl * rl);
-      } else if (epi == EPI_GATE) {
-        stf<P>(reinterpret_cast<E*>(out_) + o, s / (1.f + expf(-gate[(long)t * ext.ldg + n])));
-      } else if (epi == EPI_GATE_ROW) {
-        stf<P>(reinterpret_cast<E*>(out_) + o, s / (1.f + expf(-gate[(long)t * ext.ldg])));
-      } else if (epi == EPI_CAP) {
-        reinterpret_cast<float*>(out_)[o] = ext.limit * tanhf(s / ext.limit);
-      } else {
-        reinterpret_cast<float*>(out_)[o] = s;
+      for (int tt = 0; tt < TT; ++tt) {
+        const int t = t0 + tt * 16 + (l & 15);
+        if (t >= T) continue;
+        const float s = total(nt, tt) + bv;
+        const long o = obase + (long)t * ldo + n;
+        if constexpr (DUAL) {
+          stf<P>(reinterpret_cast<E*>(out_) + o, glu_pair(epi, s, total(NT + nt, tt) + bv2, ext.limit, ext.alpha));
+        } else if (epi == EPI_DT) {
+          stf<P>(reinterpret_cast<E*>(out_) + o, s);
+        } else if (epi == EPI_RELU2) {
+          const float rl = fmaxf(s, 0.f);
+          stf<P>(reinterpret_cast<E*>(out_) + o, rl * rl);
+        } else if (epi == EPI_GATE) {
+          stf<P>(reinterpret_cast<E*>(out_) + o, s / (1.f + expf(-gate[(long)t * ext.ldg + n])));
+        } else if (epi == EPI_GATE_ROW) {
+          stf<P>(reinterpret_cast<E*>(out_) + o, s / (1.f + expf(-gate[(long)t * ext.ldg])));
+        } else if (epi == EPI_CAP) {
+          reinterpret_cast<float*>(out_)[o] = ext.limit * tanhf(s / ext.limit);
+        } else {
+          reinterpret_cast<float*>(out_)[o] = s;
+        }
       }
     }
+    if (!RUN) break;
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // nothing of this wave may still be writing LDS
 }
 
+template <typename P, int NT, int TT, int BP, bool DUAL, int R, bool RUN>
+static int launch_stream_grid(dim3 grid, void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
+                              LinExt ext) {
+  typedef typename El<P>::type E;
+  typedef StreamShape<NT, TT, BP, DUAL, R> S;
+  if (ensure_dynamic_lds<seq_linear_stream_kernel<P, NT, TT, BP, DUAL, R, RUN>>(S::LDS) != UMB_OK) return UMB_EHIP;
+  ext.step = (int)grid.x;
+  hipLaunchKernelGGL((seq_linear_stream_kernel<P, NT, TT, BP, DUAL, R, RUN>), grid, dim3(256), S::LDS, st, out, (const E*)x, (const E*)w, (const E*)bias,
+                     T, N, K, epi, ext);
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+// RUN: a launch of more row blocks than the chip holds runs on from block to block inside its workgroups, the ring filled across their ends: a new
+// workgroup's first chunks and its last sums would stand bare (us, rounds of workgroups / this, both in turn from eight places: 32000 x 2048 at 1 /
+// 16 / 32 / 48 / 64 tokens 26.1 / 29.4 / 35.7 / 35.9 / 40.1 -> 24.2 / 27.1 / 33.4 / 31.3 / 36.4; gate/up 16384 x 2048, 48 tokens 18.2 -> 16.8).  Fewer
+// blocks: the code around the ring is 0.3 us more than it gives.  Gate/up of at most 32 tokens: two workgroups a unit cover for one another, equal.
 template <typename P, int NT, int TT, int BP, bool DUAL, int R>
 static int launch_stream_as(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
                             const LinExt& ext, int gy, int gz) {
-  typedef typename El<P>::type E;
-  typedef StreamShape<NT, TT, BP, DUAL, R> S;
-  if (ensure_dynamic_lds<seq_linear_stream_kernel<P, NT, TT, BP, DUAL, R>>(S::LDS) != UMB_OK) return UMB_EHIP;
-  hipLaunchKernelGGL((seq_linear_stream_kernel<P, NT, TT, BP, DUAL, R>), dim3((N + 16 * NT - 1) / (16 * NT), gy > 0 ? gy : (T + 16 * TT - 1) / (16 * TT), gz),
-                     dim3(256), S::LDS, st, out, (const E*)x, (const E*)w, (const E*)bias, T, N, K, epi, ext);
-  UMB_LAUNCH_CHECK();
-  return UMB_OK;
+  const int blocks = (N + 16 * NT - 1) / (16 * NT), ty = gy > 0 ? gy : (T + 16 * TT - 1) / (16 * TT);
+  constexpr int HELD = 256 * (int)(160 * 1024 / StreamShape<NT, TT, BP, DUAL, R>::LDS);      // workgroups that the chip holds at once
+  constexpr bool narrow = NT == 1 && TT > 2 && !DUAL;                                        // stream_narrow: never that many blocks
+  if constexpr (!narrow && (!DUAL || TT > 2))
+    if (ty == 1 && gz == 1 && blocks > HELD && (long)K * sizeof(typename El<P>::type) / 512 >= R)
+      return launch_stream_grid<P, NT, TT, BP, DUAL, R, true>(dim3(HELD), out, x, w, bias, T, N, K, epi, st, ext);
+  return launch_stream_grid<P, NT, TT, BP, DUAL, R, false>(dim3(blocks, ty, gz), out, x, w, bias, T, N, K, epi, st, ext);
 }
 
 // T: tokens of a token tile at most (grouped launches), of the launch otherwise.  Ring depth: as many chunks ahead as leave two
@@ -812,6 +861,7 @@ extern "C" int umb_seq_linear_parts(float* out, const void* x, const void* w, co
   LinExt ext = lin_dense(N, K);
   ext.so = (long)T * N;
   ext.parts = parts;
+  ext.part_chunks = (int)((long)K * seq_elem_bytes(dtype) / 512) / parts;
   DISPATCH_SEQ_DTYPE(dtype, {
     constexpr int EB = sizeof(typename El<P>::type);
     if (parts > (long)K * EB / 512 || !stream_ok(x, w, N, K, EPI_F32, ext, EB)) return UMB_EINVAL;

@@ -107,3 +107,20 @@ def test_seams_add_the_slabs(W, groups, parts):
         _lib.seq_call("umb_hc_seam_parts", both[0], hs[0], y.clone(), parts, None, None, 0.5, None, w1, 1.0, T, W, 2, 1e-5, _lib.F32)
         _lib.seq_call("umb_hc_seam", both[1], hs[1], total(y), None, None, 0.5, None, w1, 1.0, T, W, 2, 1e-5, _lib.F32)
         assert torch.equal(both[0], both[1]) and torch.equal(hs[0], hs[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("N,chunks", [(4134, 2), (4134, 8), (2048, 9), (9000, 12)])
+def test_a_row_is_summed_in_one_order_whatever_the_batch(dtype, N, chunks):
+    """K from several places, one or two row tiles a workgroup, workgroups that run on: the same bits for a token alone and among others"""
+    from umbrella_amd import _lib
+    dt, K = DTYPES[dtype], chunks * 512 // DTYPES[dtype].itemsize
+    g = torch.Generator(device="cuda").manual_seed(N + chunks)
+    x, w = (torch.randn(s, generator=g, device="cuda").to(dt) for s in ((64, K), (N, K)))
+    full = torch.empty(64, N, device="cuda")
+    _lib.seq_call("umb_seq_linear", full, x, w, None, 64, N, K, 0, _code(dtype))
+    for lo, n in ((0, 1), (5, 8), (7, 16), (30, 17), (20, 33), (10, 48)):
+        part = torch.empty(n, N, device="cuda")
+        _lib.seq_call("umb_seq_linear", part, x[lo:lo + n].contiguous(), w, None, n, N, K, 0, _code(dtype))
+        assert torch.equal(part, full[lo:lo + n])

@@ -10,8 +10,8 @@
 // a <= 64-token launch), as in the skinny GEMM of gemm.hip.
 //
 // Few tokens: a workgroup owns 16 (or 32) output rows and up to 64 tokens; its four waves split K (wave w takes the 32-k steps w, w+4, ...)
-// and their partial tiles are summed through LDS in wave order: the summation order of an output is a function of K and of its row block,
-// never of the row's place in the batch, and of T only where another kernel or another block height takes over (launch_vec, launch_stream).  K % 8 != 0 (or a tail)
+// and their partial tiles are summed through LDS in wave order: the summation order of an output is a function of K and of its row of W,
+// never of the token's place in the batch, and of T only where the many-token kernels take over (launch_vec).  K % 8 != 0 (or a tail)
 // falls back to guarded element loads.
 #include "gemm_tile.h"
 #include "seq_common.h"
@@ -92,8 +92,8 @@ struct LinExt {
   int ldg, sg;
   float limit, alpha;      // EPI_CLAMP_GLU; EPI_CAP: out = limit tanh(acc / limit), fp32
   // streaming kernel.  parts > 1: blockIdx.z is a slab of K and not a problem, part_chunks 512-byte chunks (one more in the first ones); its sums go to
-  // out + z so, the bias into slab 0's.  step: distance of a workgroup's row blocks (gridDim.x, read with the other arguments)
-  int parts, part_chunks, step;
+  // out + z so, the bias into slab 0's.  step: distance of a workgroup's row blocks (gridDim.x, read with the other arguments); turn: first_chunk
+  int parts, part_chunks, step, turn;
 };
 static inline LinExt lin_dense(int N, int K) { return LinExt{K, N, 0, 0, 0, 0, nullptr, nullptr, 0, 0}; }
 
@@ -502,7 +502,9 @@ template <int NT, int TT, int BP, bool DUAL, int R> struct StreamShape {     // 
 };
 // The row blocks that one XCD works on side by side (every eighth) walk K from eight places: in step they would all ask for the same 512 bytes
 // of rows a power of two apart, which stand on a quarter of the L2's channels (10240 x 4096, 48 tokens: 32.1 -> 26.3 us; 32000 x 2048, 1 token 27.9 -> 24.2).
-__device__ __forceinline__ int first_chunk(int block, int chunks) { return ((block >> 3) & 7) * chunks / 8; }
+// The place follows from the row and K alone, whatever the tokens of the launch.  From eight chunks on and not in grouped or batched launches:
+// those leave some shapes to the kernel above by their tokens, and a row is summed in one order in both (turn: 7, or 0).
+__device__ __forceinline__ int first_chunk(int row, int chunks, int turn) { return ((row >> 7) & turn) * chunks / 8; }
 template <typename P, int NT, int TT, int BP, bool DUAL, int R, bool RUN>
 __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict__ out_, const typename El<P>::type* __restrict__ x,
                                                                 const typename El<P>::type* __restrict__ w,
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, g = lane >> 4;
   int t0 = blockIdx.y * (TT * 16);
-  const int ldx = ext.ldx, ldo = ext.ldo, parts = ext.parts, step = ext.step;
+  const int ldx = ext.ldx, ldo = ext.ldo, parts = ext.parts, step = ext.step, turn = ext.turn;
   long obase = (long)blockIdx.z * ext.so;
   const float* gate = ext.gate ? ext.gate + (long)blockIdx.z * ext.sg : nullptr;
   x += (long)blockIdx.z * ext.sx;
@@ -561,7 +563,7 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
   // the row blocks of this workgroup, blockIdx.x, + step, ...: their chunks are ONE sequence, the ring runs on over the end of a block
   const int nb = (N + 16 * NT - 1) / (16 * NT);
   int fb = blockIdx.x, left = nc;          // the block that is fetched, its chunks that are still to come
-  int col = first_chunk(fb, nc);                // and the next of them: they are taken in turn from this one on
+  int col = first_chunk(fb * (16 * NT), nc, turn);                // and the next of them: they are taken in turn from this one on
   const char* fw = wb + (long)fb * (16 * NT) * K * EB;
   rows_of_block(fb * (16 * NT));
   auto issue = [&](int slot) {
@@ -609,7 +611,7 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
       if (RUN && __builtin_expect(left == 0 && fb + step < nb, 0)) {
         fb += step;
         left = nc;
-        col = first_chunk(fb, nc);
+        col = first_chunk(fb * (16 * NT), nc, turn);
         fw = wb + (long)fb * (16 * NT) * K * EB;
         rows_of_block(fb * (16 * NT));
       }
@@ -701,12 +703,14 @@ static int launch_stream_grid(dim3 grid, void* out, const void* x, const void* w
 // blocks: the code around the ring is 0.3 us more than it gives.  Gate/up of at most 32 tokens: two workgroups a unit cover for one another, equal.
 template <typename P, int NT, int TT, int BP, bool DUAL, int R>
 static int launch_stream_as(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
-                            const LinExt& ext, int gy, int gz) {
+                            LinExt ext, int gy, int gz) {
+  const long chunks = (long)K * sizeof(typename El<P>::type) / 512;
+  ext.turn = chunks >= 8 && gy == 0 && (gz == 1 || ext.parts > 1) ? 7 : 0;
   const int blocks = (N + 16 * NT - 1) / (16 * NT), ty = gy > 0 ? gy : (T + 16 * TT - 1) / (16 * TT);
   constexpr int HELD = 256 * (int)(160 * 1024 / StreamShape<NT, TT, BP, DUAL, R>::LDS);      // workgroups that the chip holds at once
   constexpr bool narrow = NT == 1 && TT > 2 && !DUAL;                                        // stream_narrow: never that many blocks
   if constexpr (!narrow && (!DUAL || TT > 2))
-    if (ty == 1 && gz == 1 && blocks > HELD && (long)K * sizeof(typename El<P>::type) / 512 >= R)
+    if (ty == 1 && gz == 1 && blocks > HELD && chunks >= R)
       return launch_stream_grid<P, NT, TT, BP, DUAL, R, true>(dim3(HELD), out, x, w, bias, T, N, K, epi, st, ext);
   return launch_stream_grid<P, NT, TT, BP, DUAL, R, false>(dim3(blocks, ty, gz), out, x, w, bias, T, N, K, epi, st, ext);
 }

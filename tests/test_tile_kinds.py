@@ -1,0 +1,64 @@
+"""Staged products of prompts (csrc/gemm_tile.h): every tile that a launch chooses from, at ragged edges, with rows stored as whole lines, in quads
+and one by one, with K of one stage, fewer stages than the ring has slots, and more; against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (T, N, K) of single matrices by the tile that they get; N % 8 == 0, N % 4 == 0 and odd
+SHAPES = [(1600, 8184, 64), (2049, 6145, 320), (2049, 6148, 192),               # 256 x 256
+          (1300, 6145, 128), (1300, 8188, 64), (2300, 8184, 192),               # 256 x 192
+          (900, 8184, 64), (1101, 8190, 192), (2049, 8188, 320),                # 256 x 160
+          (1101, 6152, 192), (1300, 5001, 128), (2300, 2592, 320),              # 256 x 128
+          (257, 6148, 64), (257, 8184, 320), (2300, 2050, 192),                 # 256 x 96
+          (257, 200, 64), (300, 1001, 192), (1000, 1028, 320),                  # 128 x 128
+          (257, 2048, 128), (300, 1004, 384), (2049, 129, 128)]                 # 128 x 64
+
+
+@pytest.mark.parametrize("T,N,K", SHAPES)
+def test_every_tile(T, N, K):
+    from umbrella_amd import _lib
+    dtype = torch.bfloat16 if K % 128 else torch.float16
+    code, half_ulp = _lib.seq_dtype_code(dtype), 2.0 ** -8 if K % 128 else 2.0 ** -11
+    g = torch.Generator(device="cuda").manual_seed(T + N + K)
+    x, w, b = (torch.randn(s, generator=g, device="cuda").to(dtype) for s in ((T, K), (N, K), (N,)))
+    full, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    tol = 2.0 ** -24 * (K + 2) * (size + b.double().abs())                     # an fp32 sum of K products in any order, and the bias
+    out = torch.full((T + 1, N), 7.0, device="cuda")
+    _lib.seq_call("umb_seq_linear", out, x, w, b, T, N, K, 0, code)
+    assert ((out[:T].double() - (full + b.double())).abs() <= tol).all() and bool((out[T] == 7.0).all())
+    out = torch.full((T + 1, N), 7.0, dtype=dtype, device="cuda")
+    _lib.seq_call("umb_seq_linear", out, x, w, None, T, N, K, 1, code)
+    assert ((out[:T].double() - full).abs() <= 1.01 * half_ulp * full.abs() + tol + 2.0 ** -25).all() and bool((out[T] == 7.0).all())
+    n = N // 2                                                                 # stacked halves: |d silu| <= 1.1 |d gate|
+    gate, up, tg, tu = full[:, :n], full[:, n:2 * n], tol[:, :n], tol[:, n:2 * n]
+    act = torch.full((T + 1, n), 7.0, dtype=dtype, device="cuda")
+    _lib.seq_call("umb_seq_linear", act, x, w[:2 * n].contiguous(), None, T, 2 * n, K, 2, code)
+    want = gate * torch.sigmoid(gate) * up
+    bound = 1.02 * half_ulp * want.abs() + 1.1 * tg * up.abs() + gate.abs() * tu + 1e-6 * want.abs() + 2.0 ** -25
+    assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())
+
+
+# packed weights: the same tiles, K in slabs of one stage, of an even and an odd number, and a slab past the last stage
+@pytest.mark.parametrize("T,N,K,S", [(1600, 8176, 128, 1), (1300, 6160, 128, 1), (900, 8176, 128, 1), (1101, 6160, 128, 1), (257, 6160, 128, 1),
+                                     (300, 1008, 640, 3), (1300, 5008, 384, 4), (257, 2048, 256, 2), (300, 1008, 128, 2)])
+def test_every_tile_of_packed_weights(T, N, K, S):
+    from umbrella_amd import _lib
+    from umbrella_amd.models.llama import PackedLinear
+    dtype = torch.float16 if K > 128 else torch.bfloat16
+    half_ulp = 2.0 ** -11 if K > 128 else 2.0 ** -8
+    g = torch.Generator(device="cuda").manual_seed(T + N + K)
+    x, w = (torch.randn(s, generator=g, device="cuda").to(dtype) for s in ((T, K), (N, K)))
+    full, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    tol = 2.0 ** -24 * (K + S) * size
+    lin, code = PackedLinear.from_dense(w), _lib.dtype_code(dtype)
+    part = torch.full((S + 1, T, N), 7.0, device="cuda")
+    _lib.call("umb_gemm", part, x, x.stride(0), lin.w, None, T, N, K, 0, S, lin.Rtb, 0, code)
+    assert ((part[:S].double().sum(0) - full).abs() <= tol).all() and bool((part[S] == 7.0).all())
+    inter = PackedLinear.from_dense(w, interleave=True)                        # gate and up rows in pairs
+    act = torch.full((T + 1, N // 2), 7.0, dtype=dtype, device="cuda")
+    _lib.call("umb_gemm", act, x, x.stride(0), inter.w, None, T, N, K, 0, 1, inter.Rtb, 2, code)
+    gate, up, tg, tu = full[:, :N // 2], full[:, N // 2:], tol[:, :N // 2], tol[:, N // 2:]
+    want = gate * torch.sigmoid(gate) * up
+    bound = 1.05 * half_ulp * (1.1 * gate.abs() * up.abs() + 3 * want.abs()) + 1.1 * tg * up.abs() + 1.1 * gate.abs() * tu + 2e-6 * want.abs() + 2.0 ** -24
+    assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())

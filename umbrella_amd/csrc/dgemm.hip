@@ -11,7 +11,7 @@
 #include <cstdlib>
 
 template <typename P, int WM, int WN, int RA, int RB, int KS>
-__global__ __launch_bounds__(64 * WM * WN * KS, RA * RB * KS <= 16 ? 2 : 1)
+__global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS == 4 ? 2 : 1)
 void dgemm_kernel(const unsigned char* __restrict__ wp, const u16* __restrict__ x, int ldx, int T, int N, int K, int S, int epi, int nbt,
                   float* __restrict__ out, GemmFused fx) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -41,10 +41,12 @@ void dgemm_kernel(const unsigned char* __restrict__ wp, const u16* __restrict__ 
       for (int t = 0; t < RB; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (ks) return;
   }
+  const int nw = n0 + wm * RA * 16;                          // this wave's first row of W
+  const unsigned strip = (unsigned)(size_t)(lds_char*)smem + (unsigned)wave * (KS == 2 ? RA * RB * 1024u : TileRows<16, RA>::BYTES);
+  static_assert(TileRows<16, RA>::BYTES <= RA * RB * 1024u && TileRows<16, RA>::BYTES * Sh::NW <= Sh::LDS, "a strip per wave");
 #pragma unroll
   for (int t = 0; t < RB; ++t) {
-    const int tok = t0 + (wn * RB + t) * 16 + j;
-    if (tok >= T) continue;
+    const int tile0 = t0 + (wn * RB + t) * 16, tok = min(tile0 + j, T - 1);
     float inv = 1.f;
     if (fx.ssq_in) {
       const float* sq = fx.ssq_in + (long)tok * (fx.ssq_stride ? fx.ssq_stride : fx.ssq_groups);
@@ -52,21 +54,28 @@ void dgemm_kernel(const unsigned char* __restrict__ wp, const u16* __restrict__ 
       for (int q = 0; q < fx.ssq_groups; q += 4) { const f32x4 v = *reinterpret_cast<const f32x4*>(sq + q); a += v[0]; a += v[1]; a += v[2]; a += v[3]; }
       inv = rsqrtf(a / fx.ssq_dim + fx.eps);
     }
+    if (epi == EPI_SILU) {
+      unsigned d[RA];
 #pragma unroll
-    for (int i = 0; i < RA; ++i) {
-      const int n = n0 + (wm * RA + i) * 16;
-      if (n >= N) continue;
-      f32x4 v = acc[i][t];
-      if (epi == EPI_SILU) {
-        v *= inv;
+      for (int i = 0; i < RA; ++i) {
+        const f32x4 v = acc[i][t] * inv;
         const float g0 = rnd<P>(v[0]), u0 = rnd<P>(v[1]), g1 = rnd<P>(v[2]), u1 = rnd<P>(v[3]);
-        const float a0 = rnd<P>(g0 / (1.f + __expf(-g0))) * u0, a1 = rnd<P>(g1 / (1.f + __expf(-g1))) * u1;
-        u16* act = reinterpret_cast<u16*>(out);
-        *reinterpret_cast<unsigned*>(act + (long)tok * (N / 2) + n / 2 + g * 2) = pack2<P>(a0, a1);
-      } else {
-        if (epi == EPI_ROUND) { v *= inv; v[0] = rnd<P>(v[0]); v[1] = rnd<P>(v[1]); v[2] = rnd<P>(v[2]); v[3] = rnd<P>(v[3]); }
-        *reinterpret_cast<f32x4*>(out + ((long)sp * T + tok) * N + n + g * 4) = v;
+        d[i] = pack2<P>(rnd<P>(g0 / (1.f + __expf(-g0))) * u0, rnd<P>(g1 / (1.f + __expf(-g1))) * u1);
       }
+      u16* act = reinterpret_cast<u16*>(out) + nw / 2;       // N % 16 == 0: rows of whole 16-byte groups
+      tile_rows_out<4, RA>(strip, d, [&](int row, int at, u32x4 b) {
+        if (tile0 + row < T && nw + at < N) *reinterpret_cast<u32x4*>(act + (long)(tile0 + row) * (N / 2) + at / 2) = b;
+      });
+    } else {
+      f32x4 v[RA];
+#pragma unroll
+      for (int i = 0; i < RA; ++i) {
+        v[i] = acc[i][t];
+        if (epi == EPI_ROUND) { v[i] *= inv; v[i][0] = rnd<P>(v[i][0]); v[i][1] = rnd<P>(v[i][1]); v[i][2] = rnd<P>(v[i][2]); v[i][3] = rnd<P>(v[i][3]); }
+      }
+      tile_rows_out<16, RA>(strip, v, [&](int row, int at, u32x4 b) {
+        if (tile0 + row < T && nw + at / 4 < N) *reinterpret_cast<u32x4*>(out + ((long)sp * T + tile0 + row) * N + nw + at / 4) = b;
+      });
     }
   }
 }
@@ -89,41 +98,18 @@ static int dgemm_launch(const void* wp, const u16* x, int ldx, float* out, int T
   return UMB_OK;
 }
 
-// The tiles a launch chooses from and what a 64-k stage of one round of 256 workgroups takes (us; one MI355X, bf16 and fp16, random data).
-// 128 x 128 runs two workgroups per CU (a round of 512 takes two); the K-split forms are for launches of at most one workgroup per CU.
-//                        rows tokens stage us
-enum { TILE_256 = 0,   //  256   256   1.5
-       TILE_160 = 1,   //  256   160   1.1     257 tokens are two of these and not two of 256
-       TILE_128 = 2,   //  128   128   0.52
-       TILE_128K = 3,  //  128   128   0.56    K over two groups of waves
-       TILE_64K = 4 }; //  128    64   0.39    the same
-// Least sum of rounds x stages x stage time over the tiles.  28672 x 4096 weights: 257 tokens 74 us (TILE_160; 102 with TILE_256 or
-// TILE_128; the register-resident kernel 141), 385 tokens 102 (TILE_256; 120 - 137; 153), 1024 tokens 200 (TILE_256; 242 - 282; 328);
-// 4096 x 4096, 257 tokens, S = 2: 21 us (TILE_128K; 24 - 27; 52).
-static double dgemm_tile(int T, int N, int K, int S, int* tile) {
-  static const struct { int bn, bt; double us; bool ksplit; } kind[5] = {
-      {256, 256, 1.5, false}, {256, 160, 1.1, false}, {128, 128, 0.52, false}, {128, 128, 0.56, true}, {128, 64, 0.39, true}};
-  const bool even = K % (128 * S) == 0;
-  double best = 1e30;
-  for (int i = 0; i < 5; ++i) {
-    const long wgs = (long)((N + kind[i].bn - 1) / kind[i].bn) * ((T + kind[i].bt - 1) / kind[i].bt) * S, rounds = (wgs + 255) / 256;
-    if (kind[i].ksplit && (rounds > 1 || !even)) continue;
-    // a lone workgroup of the two-per-CU form leaves half the wave slots empty
-    const double cost = rounds * ((K / 64 + S - 1) / S) * (i == TILE_128 && rounds == 1 ? 0.62 : kind[i].us) + 4.0;
-    if (cost < best) { best = cost; *tile = i; }
-  }
-  return best;
-}
+// the tile by tile_kind (gemm_tile.h)
+static int dgemm_tile(int T, int N, int K, int S, double* us = nullptr) { return tile_kind(T, N, (K / 64 + S - 1) / S, S, K % (128 * S) == 0, us); }
 
 template <typename P>
 static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int S, int epi, const GemmFused& fx, hipStream_t st) {
-  int tile = TILE_128;
-  (void)dgemm_tile(T, N, K, S, &tile);
-  switch (tile) {
+  switch (dgemm_tile(T, N, K, S)) {
     case TILE_256: return dgemm_launch<P, 4, 2, 4, 8, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+    case TILE_192: return dgemm_launch<P, 4, 2, 4, 6, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     case TILE_160: return dgemm_launch<P, 4, 2, 4, 5, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
-    case TILE_128: return dgemm_launch<P, 2, 2, 4, 4, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
-    case TILE_128K: return dgemm_launch<P, 2, 2, 4, 4, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+    case TILE_128W: return dgemm_launch<P, 4, 2, 4, 4, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+    case TILE_96: return dgemm_launch<P, 4, 2, 4, 3, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+    case TILE_128: return dgemm_launch<P, 2, 4, 4, 2, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     default: return dgemm_launch<P, 2, 2, 4, 2, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
   }
 }
@@ -133,21 +119,23 @@ static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, i
 // and stays ahead there where the 256-row tiles of such a launch are more than one per compute unit (129 tokens, it / here: 128256 x 4096 198 /
 // 245 us, 73728 x 4608 192 / 219, 128256 x 2048 111 / 122; 65536 x 5120, one round, 175 / 145; 145 tokens 377 / 245).  Less weight of such a
 // launch already stays ahead there (65 tokens, 100352 x 2560 101 / 125) unless K is short (256000 x 1024 127 / 117).
-bool umb_dgemm_ok(const void* x, int ldx, int T, int N, int K, int S, int epi) {
+bool umb_dgemm_ok(const void* x, const void* out, int ldx, int T, int N, int K, int S, int epi) {
   static const bool off = getenv("UMB_NO_VGEMM") != nullptr || getenv("UMB_VGEMM_PLAIN") != nullptr;     // gemm.hip's diagnostics
   const long bytes = (long)N * K * 2;
   const bool streams = (T <= 128 && bytes > (512L << 20)) || (T <= 144 && N > 65536 && K >= 1536 && bytes > (448L << 20));
-  return !off && T > 64 && K % 64 == 0 && N % 16 == 0 && ldx % 8 == 0 && (uintptr_t)x % 16 == 0 && epi <= EPI_SILU &&
+  return !off && T > 64 && K % 64 == 0 && N % 16 == 0 && ldx % 8 == 0 && ((uintptr_t)x | (uintptr_t)out) % 16 == 0 && epi <= EPI_SILU &&
          (long)ldx * 512 < (1L << 31) && !streams;
 }
 
-// K slabs of a wide dense product whose partials are summed by the kernel behind it: the least of the product's time and of what the
-// partials beyond the first cost (written and read, 3 TB/s).  1024 tokens: 6144 x 4096 S = 1, 4096 x 14336 S = 2 (118 -> 99 us)
+// K slabs of a wide dense product whose partials are summed by the kernel behind it: the least of the product's time and of what reading the
+// partials beyond the first costs there (8 TB/s: they come from the last-level cache).  1024 tokens: 6144 x 4096 S = 1, 4096 x 14336 S = 4 in 256 x 256
+// tiles (93 us and 13.1 in the residual behind it; S = 2 in 256 x 128 102 and 10.3; whole 190)
 int umb_dgemm_split(int T, int N, int K, int S_plan) {
-  int best_s = 1, tile = 0;
-  double best = 1e30;
+  int best_s = 1;
+  double best = 1e30, us = 0.0;
   for (int S = 1; S <= S_plan && S <= K / 128 && (long)S * T * N * 4 < (1L << 31); ++S) {
-    const double cost = dgemm_tile(T, N, K, S, &tile) + (S - 1) * (double)T * N * 4 / 3e6;
+    (void)dgemm_tile(T, N, K, S, &us);
+    const double cost = us + (S - 1) * (double)T * N * 4 / 8e6;
     if (cost < best) { best = cost; best_s = S; }
   }
   return best_s;

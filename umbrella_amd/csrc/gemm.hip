@@ -1608,7 +1608,7 @@ extern "C" int umb_gemm_fused(void* out, const void* x, int ldx, const void* wpa
     return launch_tt<F16, 2>(wpacked, meta, (const u16*)x, ldx, (float*)out, T, N, K, R, S, epi, fx, st, tb);
   DISPATCH_DTYPE(dtype, {
     if (awq) return launch_tt<P, 1>(wpacked, meta, (const u16*)x, ldx, (float*)out, T, N, K, R, S, epi, fx, st, tb);
-    if (umb_dgemm_ok(x, ldx, T, N, K, S, epi))
+    if (umb_dgemm_ok(x, out, ldx, T, N, K, S, epi))
       return umb_dgemm(wpacked, (const u16*)x, ldx, (float*)out, T, N, K, S, epi, fx, dtype, st);
     return launch_tt<P, 0>(wpacked, meta, (const u16*)x, ldx, (float*)out, T, N, K, R, S, epi, fx, st, tb);
   })

@@ -29,6 +29,6 @@ int umb_vgemm_w(const void* wp, const void* meta, const u16* x, int ldx, float* 
                 const GemmFused& fx, hipStream_t st);
 
 // dgemm.hip: the wide (T > 64) GEMM of dense 16-bit weights, gemm.hip's tile order and epilogues
-bool umb_dgemm_ok(const void* x, int ldx, int T, int N, int K, int S, int epi);
+bool umb_dgemm_ok(const void* x, const void* out, int ldx, int T, int N, int K, int S, int epi);
 int umb_dgemm(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int S, int epi, const GemmFused& fx, int dtype,
               hipStream_t st);

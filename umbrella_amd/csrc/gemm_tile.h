@@ -6,10 +6,12 @@
 // it, 64 x 128 (4 x 8) for three quarters.  Hence:
 //   * operands go HBM / L2 -> LDS by LDS-DMA (1-KiB pieces of 8 rows x 128 B: whole lines, no VGPR on the way, no address arithmetic
 //     in the loop); the 16-byte column of a row is XOR-swizzled on the SOURCE side, so fragment reads meet no bank conflict;
-//   * two slots of 64 k.  ONE barrier per stage stands between its two 32-k phases: when a wave arrives there it has every fragment
-//     of the stage in registers, so behind the barrier the slot is free for the stage after the next, and the next stage (whose
-//     pieces every wave has waited for) can be read: the fragments of a phase are requested, one per few products, while the
-//     products of the phase before run, across the stage boundary too, and a stage's pieces have a whole stage to arrive.
+//   * a ring of two to four slots of 64 k, as many as the LDS holds.  ONE barrier per stage stands between its two 32-k phases: when a
+//     wave arrives there it has every fragment of the stage in registers, so behind the barrier the slot is free for the stage NS
+//     further on, and the next stage (whose pieces every wave has waited for) can be read: the fragments of a phase are requested, one
+//     per few products, while the products of the phase before run, across the stage boundary too, and a stage's pieces have
+//     NS - 1 stages to arrive.  With two slots no stage is shorter than the 1.0 us that pieces take from L2: 256 x 128 outputs 1.05 -> 0.86
+//     us a stage with three, 256 x 160 1.1 -> 0.95 - 1.05, 128 x 128 (eight waves, four slots; before: K over two groups of four, 0.55) 0.49.
 // K-split (KS = 2): two groups of WM x WN waves take alternate stages in slots of their own and their tiles are added (group 0 +
 // group 1) at the end: two waves per SIMD where a launch has at most one workgroup per CU.
 // Measured against the register-staged kernel it replaces (bf16, random data, one MI355X; both sides in seq_linear.hip).
@@ -34,11 +36,42 @@ template <int WM, int WN, int RA, int RB, int KS> struct TileShape {
   static constexpr int NPA = BN / 8, NPB = BT / 8;            // 1-KiB pieces of a stage
   static constexpr int NPW = (NPA + NPB + NW - 1) / NW;       // pieces a wave fetches per stage
   static constexpr unsigned SLOT = (NPA + NPB) * 1024u;
+  static constexpr int PER_CU = NW * KS == 4 ? 2 : 1;         // workgroups that share a CU
   // where the pieces do not deal out evenly, a wave without a last piece of its own fetches into the KiB behind the slots
   static constexpr bool EVEN = (NPA + NPB) % NW == 0;
-  static constexpr size_t LDS = (size_t)KS * 2 * SLOT + (EVEN ? 0 : 1024);
-  static_assert(NPA % NW == 0 && (EVEN || KS == 1) && (KS == 1 || RA * RB * NW * 1024u <= LDS), "whole rounds of A pieces; a group's tile fits the slots");
+  static constexpr int FIT = (int)((160 * 1024 / PER_CU - (EVEN ? 0 : 1024)) / (KS * SLOT)), NS = FIT < 4 ? FIT : 4;      // slots of a ring
+  static constexpr size_t LDS = (size_t)KS * NS * SLOT + (EVEN ? 0 : 1024);
+  static_assert(NS >= 2 && NPA % NW == 0 && (EVEN || KS == 1) && (KS == 1 || RA * RB * NW * 1024u <= LDS), "whole rounds of A pieces; a group's tile fits the slots");
 };
+
+// The tiles a launch chooses from, and what a 64-k stage of a whole round of 256 workgroups takes (us; one MI355X, bf16, random data).  Few sizes
+// of a prompt fill rounds of one tile; between 0.46 (256 x 256) and 1.4 ns a stage, row and token the right one is the one that fills best.
+//                       rows tokens stage
+enum { TILE_256 = 0,  //  256   256  1.42
+       TILE_192 = 1,  //  256   192  1.20
+       TILE_160 = 2,  //  256   160  1.04
+       TILE_128W = 3, //  256   128  0.86
+       TILE_96 = 4,   //  256    96  0.73
+       TILE_128 = 5,  //  128   128  0.49
+       TILE_64K = 6,  //  128    64  0.38   K over two groups of waves
+       TILE_KINDS = 7 };
+// us of a launch: 4, and for each round its stages, 2 in front of them and 14 for 256 x 256 outputs behind them; a last round that is not
+// full takes a little less (its share of the memory path is larger).  rows: of A; stages: of one slab; S: slabs
+static inline double tile_cost(int kind, int T, int rows, int stages, int S) {
+  static const struct { int bn, bt; double us; } k[TILE_KINDS] = {{256, 256, 1.42}, {256, 192, 1.20}, {256, 160, 1.04}, {256, 128, 0.86},
+                                                                 {256, 96, 0.73}, {128, 128, 0.49}, {128, 64, 0.38}};
+  const long wgs = (long)((rows + k[kind].bn - 1) / k[kind].bn) * ((T + k[kind].bt - 1) / k[kind].bt) * S, rest = wgs % 256;
+  const double load = rest / 256.0, products = stages * k[kind].us, out = 2.1e-4 * k[kind].bn * k[kind].bt;
+  return 4.0 + (wgs / 256) * (products + out + 2.0) + (rest ? products * (0.8 + 0.2 * load) + out * load + 2.0 : 0.0);
+}
+// the least of them (the K-split one takes an even number of stages)
+static inline int tile_kind(int T, int rows, int stages, int S, bool even, double* us = nullptr) {
+  int best = 0;
+  for (int i = 1; i < TILE_KINDS; ++i)
+    if ((i != TILE_64K || even) && tile_cost(i, T, rows, stages, S) < tile_cost(best, T, rows, stages, S)) best = i;
+  if (us) *us = tile_cost(best, T, rows, stages, S);
+  return best;
+}
 
 // Row block of a workgroup: the hardware deals consecutive workgroups to the eight XCDs in turn; here the workgroups of one XCD get
 // consecutive tile numbers, so that the tiles its L2 serves share operand rows.
@@ -57,18 +90,19 @@ template <typename F> __device__ __forceinline__ unsigned tile_voff(int p, int l
 // abase / bbase: the operands at k = 0 of the tile (a stage advances them by astep / 128 bytes); voff: per-lane byte offsets of this
 // wave's pieces (NPA / NW of A, then those of B).  FRAG: A lies in 1-KiB fragments already (lane l's 16 bytes at 16 l): its pieces are
 // the fragments (16 rows, 32 k) in the order row tile, k half.  nst: stages of 64 k (a multiple of KS).  On return acc is complete in
-// the waves of group 0; returns whether this wave is one of them.
+// the waves of group 0, which may use their share of LDS from then on (16 RA RB KiB / 16 a wave with a K split, else LDS / NW); returns whether
+// this wave is one of them.
 template <typename P, int WM, int WN, int RA, int RB, int KS, bool FRAG>
 __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned char* smem, const void* abase, const void* bbase, long astep,
                                               const unsigned (&voff)[TileShape<WM, WN, RA, RB, KS>::NPW], int nst, int wave, int ks) {
   typedef TileShape<WM, WN, RA, RB, KS> S;
-  constexpr int NW = S::NW, NPA = S::NPA, NPW = S::NPW, NF = RA + RB, NM = RA * RB;
+  constexpr int NW = S::NW, NPA = S::NPA, NPW = S::NPW, NF = RA + RB, NM = RA * RB, NS = S::NS;
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
-  const unsigned lds0 = (unsigned)(size_t)(lds_char*)smem + (unsigned)ks * 2u * S::SLOT;
+  const unsigned lds0 = (unsigned)(size_t)(lds_char*)smem + (unsigned)(ks * S::NS) * S::SLOT;
   const int n = nst / KS;                                     // stages of this group
-  auto issue = [&](int st, int i) {
-    unsigned dst = lds0 + (unsigned)(st & 1) * S::SLOT + (unsigned)(wave + NW * i) * 1024u;
-    if (!S::EVEN && i == NPW - 1 && wave + NW * i >= NPA + S::NPB) dst = lds0 + 2u * S::SLOT;
+  auto issue = [&](int st, unsigned slot, int i) {
+    unsigned dst = lds0 + slot + (unsigned)(wave + NW * i) * 1024u;
+    if (!S::EVEN && i == NPW - 1 && wave + NW * i >= NPA + S::NPB) dst = lds0 + (unsigned)NS * S::SLOT;
     const long s = (long)min(st, n - 1) * KS + ks;
     if (NW * i < NPA) tile_dma(voff[i], static_cast<const char*>(abase) + s * astep, dst);
     else tile_dma(voff[i], static_cast<const char*>(bbase) + s * 128, dst);
@@ -82,44 +116,47 @@ __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned cha
 #pragma unroll
     for (int t = 0; t < RB; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   u32x4 fa[2][RA], fb[2][RB];
-  auto read = [&](int st, int kh, int i) {                    // the i-th fragment of a phase, in the order the products want them
-    const unsigned base = lds0 + (unsigned)(st & 1) * S::SLOT;
+  auto read = [&](unsigned slot, int kh, int i) {             // the i-th fragment of a phase, in the order the products want them
+    const unsigned base = lds0 + slot;
     const unsigned ao = base + (FRAG ? (unsigned)(kh * 1024 + lane * 16) : foff[kh]);
     if (i == 0) fa[kh][0] = *reinterpret_cast<const lds_u32x4*>((size_t)(ao + (unsigned)(wm * RA) * 2048u));
     else if (i <= RB) fb[kh][i - 1] = *reinterpret_cast<const lds_u32x4*>((size_t)(base + foff[kh] + NPA * 1024u + (unsigned)(wn * RB + i - 1) * 2048u));
     else fa[kh][i - RB] = *reinterpret_cast<const lds_u32x4*>((size_t)(ao + (unsigned)(wm * RA + i - RB) * 2048u));
   };
+  unsigned slot = 0, next = S::SLOT;                          // of the stage whose products run, and of the one behind it
   auto phase = [&](auto half, int st) {
     constexpr int KH = decltype(half)::value;
     constexpr int GAP = NM / NF > 0 ? NM / NF : 1, DG = NM / NPW > 0 ? NM / NPW : 1;   // products per fragment read, per piece
     static_assert(GAP * (NF - 1) < NM && DG * (NPW - 1) < NM, "every read and every piece has a product to hide behind");
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-      if (m % GAP == 0 && m / GAP < NF) read(KH == 0 ? st : st + 1, KH ^ 1, m / GAP);
-      if (KH == 1 && m % DG == 0 && m / DG < NPW) issue(st + 2, m / DG);
+      if (m % GAP == 0 && m / GAP < NF) read(KH == 0 ? slot : next, KH ^ 1, m / GAP);
+      if (KH == 1 && m % DG == 0 && m / DG < NPW) issue(st + NS, slot, m / DG);
       acc[m / RB][m % RB] = P::mfma(fa[KH][m / RB], fb[KH][m % RB], acc[m / RB][m % RB]);
       if ((m + 1) % GAP == 0) __builtin_amdgcn_sched_barrier(0);
     }
   };
 #pragma unroll
-  for (int i = 0; i < NPW; ++i) issue(0, i);
+  for (int c = 0; c < NS; ++c)
 #pragma unroll
-  for (int i = 0; i < NPW; ++i) issue(1, i);
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NPW) : "memory");
+    for (int i = 0; i < NPW; ++i) issue(c, c * S::SLOT, i);
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NS - 1) * NPW) : "memory");
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int i = 0; i < NF; ++i) read(0, 0, i);
   for (int st = 0; st < n; ++st) {
     phase(std::integral_constant<int, 0>{}, st);
     // every fragment of stage st is in registers, and this wave's pieces of stage st + 1 are in LDS
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NS - 2) * NPW) : "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     phase(std::integral_constant<int, 1>{}, st);
+    slot = next;
+    next = next == (NS - 1) * S::SLOT ? 0u : next + S::SLOT;
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // nothing of this wave may still be writing LDS
+  __builtin_amdgcn_s_barrier();                                 // and none reads a slot any more
   if constexpr (KS == 2) {
-    __builtin_amdgcn_s_barrier();
     f32x4* red = reinterpret_cast<f32x4*>(smem) + wave * NM * 64 + lane;
     if (ks == 1) {
 #pragma unroll
@@ -131,4 +168,33 @@ __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned cha
     for (int i = 0; i < NM; ++i) acc[i / RB][i % RB] += red[i * 64];
   }
   return true;
+}
+
+// Outputs of one token tile of a wave, on their way to rows of memory.  After the products lane (j, g) holds, for each of NI row tiles, the QB
+// bytes of token j behind 4 g outputs: stored from there, an instruction writes 16 rows of 4 QB bytes with neighbouring lanes on different
+// rows, and the stores of a launch take as long as a third of its products (8192 x 2048 outputs, K = 2048, bf16: 72 us, 48 without
+// stores).  Through a strip of LDS of the wave's own they leave as whole lines: put(row, byte, 16 bytes) with neighbouring lanes on
+// neighbouring bytes.  `strip`: its LDS address, TileRows::BYTES of it; rows of it are 16 bytes more than the data apart.
+template <int QB, int NI> struct TileRows {
+  static constexpr int ROW = NI * 4 * QB, STRIDE = ROW + 16, LPR = ROW / 16, RPI = 64 / LPR;       // lanes a row, rows an instruction
+  static constexpr unsigned BYTES = 16u * STRIDE;
+  static_assert(ROW % 16 == 0 && 64 % LPR == 0 && 16 % RPI == 0, "whole rows");
+};
+template <int QB, int NI, typename V, typename Put>
+__device__ __forceinline__ void tile_rows_out(unsigned strip, const V (&v)[NI], Put put) {
+  typedef TileRows<QB, NI> R;
+  typedef __attribute__((address_space(3))) V lds_v;
+  static_assert(sizeof(V) == QB, "a lane's bytes of a row tile");
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) *reinterpret_cast<lds_v*>((size_t)(strip + (unsigned)(j * R::STRIDE + (i * 4 + g) * QB))) = v[i];
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int k = 0; k < 16 / R::RPI; ++k) {
+    const int row = k * R::RPI + lane / R::LPR, at = lane % R::LPR * 16;
+    put(row, at, *reinterpret_cast<const lds_u32x4*>((size_t)(strip + (unsigned)(row * R::STRIDE + at))));
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }

@@ -86,16 +86,16 @@ __device__ __forceinline__ float glu_pair(int epi, float g, float u, float limit
 // EPI_GATE_ROW by sigmoid(gate[t ldg + z sg]): one number per row and problem.
 struct LinExt {
   int ldx, ldo;
+  // streaming kernel.  parts > 1: blockIdx.z is a slab of K and not a problem, part_chunks 512-byte chunks (one more in the first ones); its sums go to
+  // out + z so, the bias into slab 0's.  step: distance of a workgroup's row blocks (gridDim.x, read with the other arguments); turn: first_chunk
+  int parts, part_chunks, step, turn;
   long sx, sw, so, gs;
   const int* tiles;
   const float* gate;
   int ldg, sg;
   float limit, alpha;      // EPI_CLAMP_GLU; EPI_CAP: out = limit tanh(acc / limit), fp32
-  // streaming kernel.  parts > 1: blockIdx.z is a slab of K and not a problem, part_chunks 512-byte chunks (one more in the first ones); its sums go to
-  // out + z so, the bias into slab 0's.  step: distance of a workgroup's row blocks (gridDim.x, read with the other arguments); turn: first_chunk
-  int parts, part_chunks, step, turn;
 };
-static inline LinExt lin_dense(int N, int K) { return LinExt{K, N, 0, 0, 0, 0, nullptr, nullptr, 0, 0}; }
+static inline LinExt lin_dense(int N, int K) { return LinExt{K, N, 0, 0, 0, 0, 0, 0, 0, 0, nullptr, nullptr, 0, 0, 0.f, 0.f}; }
 
 // NT output tiles x TT token tiles of 16 per workgroup (each wave holds all NT x TT accumulator tiles of its K share: one weight
 // fragment meets TT token fragments and one token fragment NT weight fragments, so a launch of many tokens moves
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(256) void seq_linear_wide_kernel(void* __restrict__
 // RA / 2 tiles of gate rows and the up rows of the same outputs.  The k order of an output without K-split is the wide kernel's:
 // the same bits.
 template <typename P, int WM, int WN, int RA, int RB, int KS, bool DUAL>
-__global__ __launch_bounds__(64 * WM * WN * KS, RA * RB * KS <= 16 ? 2 : 1)
+__global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS == 4 ? 2 : 1)
 void seq_linear_tile_kernel(void* __restrict__ out_, const u16* __restrict__ x, const u16* __restrict__ w, const u16* __restrict__ bias,
                             int T, int N, int K, int epi, int nbt, float limit, float alpha) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -377,19 +377,20 @@ void seq_linear_tile_kernel(void* __restrict__ out_, const u16* __restrict__ x, 
   }
   f32x4 acc[RA][RB];
   if (!tile_products<P, WM, WN, RA, RB, KS, false>(acc, smem, w + (long)n0 * K, x + (long)t0 * K, 128, voff, K / 64, wave, ks)) return;
-  const bool v4 = (N & 3) == 0;                              // four outputs of a lane: one store
+  constexpr int NI = DUAL ? RA / 2 : RA;
+  const int nw = n0 + (DUAL ? wm * (8 * RA) : wm * (16 * RA));         // this wave's first output
+  const bool half = DUAL || epi == EPI_DT || epi == EPI_RELU2;
+  const unsigned strip = (unsigned)(size_t)(lds_char*)smem + (unsigned)wave * (KS == 2 ? RA * RB * 1024u : TileRows<16, RA>::BYTES);
+  static_assert(TileRows<16, RA>::BYTES <= RA * RB * 1024u && TileRows<16, RA>::BYTES * S::NW <= S::LDS, "a strip per wave");
 #pragma unroll
   for (int t = 0; t < RB; ++t) {
-    const int tok = t0 + (wn * RB + t) * 16 + j;
-    if (tok >= T) continue;
+    const int tile0 = t0 + (wn * RB + t) * 16, tok = tile0 + j;
+    f32x4 v[NI];
 #pragma unroll
-    for (int i = 0; i < (DUAL ? RA / 2 : RA); ++i) {
-      const int n = n0 + (DUAL ? wm * (8 * RA) : wm * (16 * RA)) + i * 16 + 4 * g;
-      if (n >= N) continue;
-      float v[4];
+    for (int i = 0; i < NI; ++i) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int nn = min(n + r, N - 1);
+        const int nn = min(nw + i * 16 + 4 * g + r, N - 1);
         float s = acc[i][t][r] + (bias ? P::to_f(bias[nn]) : 0.f);
         if constexpr (DUAL) {
           const float u = acc[i + RA / 2][t][r] + (bias ? P::to_f(bias[N + nn]) : 0.f);
@@ -400,19 +401,38 @@ void seq_linear_tile_kernel(void* __restrict__ out_, const u16* __restrict__ x, 
         } else if (epi == EPI_CAP) {
           s = limit * tanhf(s / limit);
         }
-        v[r] = s;
+        v[i][r] = s;
       }
+    }
+    if (half && N % 8 == 0) {                                // rows of whole 16-byte groups: whole lines at a time
+      u32x2 d[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) d[i] = u32x2{pack2<P>(v[i][0], v[i][1]), pack2<P>(v[i][2], v[i][3])};
+      tile_rows_out<8, NI>(strip, d, [&](int row, int at, u32x4 b) {
+        if (tile0 + row < T && nw + at / 2 < N) *reinterpret_cast<u32x4*>(reinterpret_cast<u16*>(out_) + (long)(tile0 + row) * N + nw + at / 2) = b;
+      });
+      continue;
+    }
+    if (!DUAL && !half && N % 4 == 0) {
+      tile_rows_out<16, NI>(strip, v, [&](int row, int at, u32x4 b) {
+        if (tile0 + row < T && nw + at / 4 < N) *reinterpret_cast<u32x4*>(reinterpret_cast<float*>(out_) + (long)(tile0 + row) * N + nw + at / 4) = b;
+      });
+      continue;
+    }
+    if (tok >= T) continue;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int n = nw + i * 16 + 4 * g;
       const long o = (long)tok * N + n;
-      if (DUAL || epi == EPI_DT || epi == EPI_RELU2) {
-        u16* op = reinterpret_cast<u16*>(out_) + o;
-        if (v4) *reinterpret_cast<u32x2*>(op) = u32x2{pack2<P>(v[0], v[1]), pack2<P>(v[2], v[3])};
-        else
-          for (int r = 0; r < 4; ++r) if (n + r < N) op[r] = P::from_f(v[r]);
-      } else {
-        float* op = reinterpret_cast<float*>(out_) + o;
-        if (v4) *reinterpret_cast<f32x4*>(op) = f32x4{v[0], v[1], v[2], v[3]};
-        else
-          for (int r = 0; r < 4; ++r) if (n + r < N) op[r] = v[r];
+      if (n < N && half && N % 4 == 0) {
+        *reinterpret_cast<u32x2*>(reinterpret_cast<u16*>(out_) + o) = u32x2{pack2<P>(v[i][0], v[i][1]), pack2<P>(v[i][2], v[i][3])};
+        continue;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (n + r >= N) continue;
+        if (half) reinterpret_cast<u16*>(out_)[o + r] = P::from_f(v[i][r]);
+        else reinterpret_cast<float*>(out_)[o + r] = v[i][r];
       }
     }
   }
@@ -431,22 +451,21 @@ static int launch_tile_as(void* out, const void* x, const void* w, const void* b
   return UMB_OK;
 }
 
-// Which tile: 256 x 256 (8 waves, one workgroup per CU) does 128 x 128 outputs in 0.066 us of the whole chip's time at K = 2048,
-// 128 x 128 (two workgroups per CU) in 0.080, but only whole rounds of 256 workgroups are worth that: it is taken where it fills at
-// least 0.7 of its rounds (T x N x K: 2048 x 16384 x 2048 135 us against 165, 1204 x 28672 x 4096 (0.73) 333 / 363, 1999 x 10240 x 4096
-// (0.62) 214 / 186).  Launches of at most one 128 x 128 workgroup per CU split K over two groups of waves (2048 x 2048 x 8192
-// 73 us / 87), those of at most half as many take tiles of 128 x 64 (300 x 2048 x 2048 13 us / 18).  The kernel before took
-// 225, 474, 290, 137 and 37 us on these five.
+// us at T x N x K, two kinds of 256 x 256 / 128 x 128 tiles by a fixed share of a round (the rule before) -> tile_kind's: 1101 x 16384 x 2048 gate/up 109 -> 83,
+// 2048 x 5120 x 2048 70 -> 48, 1101 x 2048 x 8192 79 -> 62, 2048 x 2048 x 2048 30 -> 22, 2466 x 4096 x 14336 376 -> 230, 700 x 4096 x 4096 47 -> 35, 512 x 2048 x 8192
+// 73 -> 53; 2048 x 16384 x 2048 gate/up 126 -> 121 and 2048 x 28672 x 4096 412 -> 404 keep their tiles.
 template <typename P, bool DUAL>
 static int launch_tile(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, float limit, float alpha,
                        hipStream_t st) {
-  const int rows = DUAL ? 2 * N : N;
-  const long big = (long)((rows + 255) / 256) * ((T + 255) / 256), rounds = (big + 255) / 256;
-  if (10 * big >= 7 * 256 * rounds) return launch_tile_as<P, 4, 2, 4, 8, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
-  const long mid = (long)((rows + 127) / 128) * ((T + 127) / 128);
-  if (mid <= 128 && K % 128 == 0) return launch_tile_as<P, 2, 2, 4, 2, 2, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
-  if (mid <= 256 && K % 128 == 0) return launch_tile_as<P, 2, 2, 4, 4, 2, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
-  return launch_tile_as<P, 2, 2, 4, 4, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+  switch (tile_kind(T, DUAL ? 2 * N : N, K / 64, 1, K % 128 == 0)) {
+    case TILE_256: return launch_tile_as<P, 4, 2, 4, 8, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+    case TILE_192: return launch_tile_as<P, 4, 2, 4, 6, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+    case TILE_160: return launch_tile_as<P, 4, 2, 4, 5, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+    case TILE_128W: return launch_tile_as<P, 4, 2, 4, 4, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+    case TILE_96: return launch_tile_as<P, 4, 2, 4, 3, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+    case TILE_128: return launch_tile_as<P, 2, 4, 4, 2, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+    default: return launch_tile_as<P, 2, 2, 4, 2, 2, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+  }
 }
 
 // whole 64-k stages, 16-byte pieces and stores, 32-bit offsets inside an operand
@@ -457,7 +476,7 @@ static bool tile_ok(const void* out, const void* x, const void* w, int T, int N,
 
 template <typename P>
 static int launch_wide(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
-                       const LinExt& ext = LinExt{0, 0, 0, 0, 0, 0, nullptr, nullptr, 0, 0}, int gy = 0) {
+                       const LinExt& ext, int gy = 0) {
   if constexpr (sizeof(typename El<P>::type) == 2) {
     const unsigned ty = gy > 0 ? gy : (T + 127) / 128;
     if (epi_dual(epi))
@@ -632,7 +651,9 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
       }
       slot = slot + 1 == R ? 0 : slot + 1;
     }
-    // the waves' tiles are added in the slot of the block's last chunk, which the next block's first barrier hands back to the ring
+    // the waves' tiles are added in the slot of the block's last chunk, which the next block's first barrier hands back to the ring; behind the
+    // last block nothing of this wave may be writing LDS any more (waited for here, not behind the stores: those need no wait)
+    if (!RUN || block + step >= nb) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     const unsigned red = base;                                         // [wave][AT][TT][256] floats
@@ -682,7 +703,6 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
     }
     if (!RUN) break;
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // nothing of this wave may still be writing LDS
 }
 
 template <typename P, int NT, int TT, int BP, bool DUAL, int R, bool RUN>
@@ -817,7 +837,7 @@ static int launch_vec(void* out, const void* x, const void* w, const void* bias,
   // many tokens: the launch is bound by fragment loads per MFMA, not by weight bytes -> four output tiles per workgroup
   // (the K order of every output is unchanged)
   if (T > 64 && N >= 64 && sizeof(typename El<P>::type) == 2) {
-    if (VEC && dense && T >= 256 && N >= 128) return launch_wide<P>(out, x, w, bias, T, N, K, epi, st, LinExt{0, 0, 0, 0, 0, 0, nullptr, nullptr, 0, 0, ext.limit, ext.alpha});      // both operands re-used
+    if (VEC && dense && T >= 256 && N >= 128) return launch_wide<P>(out, x, w, bias, T, N, K, epi, st, ext);      // both operands re-used
     return launch_tt<P, 4, 4, VEC>(out, x, w, bias, T, N, K, epi, st, ext, 0, gz);
   }
   return launch_tt<P, 1, 4, VEC>(out, x, w, bias, T, N, K, epi, st, ext, 0, gz);
@@ -891,7 +911,7 @@ extern "C" int umb_seq_linear_batched(void* out, const void* x, const void* w, i
   if (T < 1 || N < 1 || K < 1 || batch < 1 || batch > 65535 || ldx < K || ldo < N || !out || !x || !w ||
       !(epi == EPI_F32 || epi == EPI_DT || epi == EPI_GATE || epi == EPI_GATE_ROW) || ((epi == EPI_GATE || epi == EPI_GATE_ROW) && !gate))
     return UMB_EINVAL;
-  const LinExt ext{ldx, ldo, sx, sw, so, 0, nullptr, gate, ldg, sg};
+  const LinExt ext{ldx, ldo, 0, 0, 0, 0, sx, sw, so, 0, nullptr, gate, ldg, sg, 0.f, 0.f};
   // 16-byte loads need every row start aligned: the strides as well as K
   const bool vec = K % 8 == 0 && ldx % 8 == 0 && sx % 8 == 0 && sw % 8 == 0;
   DISPATCH_SEQ_DTYPE(dtype, {
@@ -910,7 +930,7 @@ static int seq_linear_grouped_any(void* out, const void* x, const void* w, const
     if (N & 1) return UMB_EINVAL;
     N >>= 1;
   }
-  const LinExt ext{K, N, 0, 0, 0, gs, tiles, nullptr, 0, 0, limit, alpha};
+  const LinExt ext{K, N, 0, 0, 0, 0, 0, 0, 0, gs, tiles, nullptr, 0, 0, limit, alpha};
   if (tile_rows == 128) {                  // many rows per group: both operands staged through LDS (16-bit storage only)
     if (dtype == UMB_SEQ_F32 || K % 8 || gs % 8) return UMB_EINVAL;
     if (dtype == UMB_SEQ_BF16) return launch_wide<BF16>(out, x, w, nullptr, 128, N, K, epi, st, ext, max_tiles);

@@ -59,8 +59,9 @@ typedef struct UmbSeqLinear { const void* w; const void* bias; int32_t N, K; } U
 int umb_seq_linear(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, int dtype,
                    umb_stream_t stream);
 
-/* A product of few tokens (T <= 64) whose K is summed in `parts` slabs: out fp32 [parts][T][N], the sum over the slabs is the result (bias in
- * the first one's).  umb_seq_linear_split: the number of slabs that pays for these operands (1 .. 4; 1: umb_seq_linear; no stream). */
+/* A product whose K is summed in `parts` slabs: out fp32 [parts][T][N], the sum over the slabs is the result (bias in the first one's).  Up to 64
+ * tokens whole 512-byte chunks of K, beyond them 16-bit storage and K % 64 == 0; 16-byte aligned operands.  umb_seq_linear_split: the number of
+ * slabs that pays for these operands (1 .. 4; 1: umb_seq_linear; no stream). */
 int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype);
 int umb_seq_linear_parts(float* out, const void* x, const void* w, const void* bias, int T, int N, int K, int parts, int dtype,
                          umb_stream_t stream);

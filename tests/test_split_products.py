@@ -20,17 +20,20 @@ def test_split_rule_stays_inside_what_the_product_takes():
             for N in (1, 16, 1000, 2048, 2049, 2730, 4096, 4097, 32000):
                 for K in (8, 200, 256, 512, 1024, 2048, 2304, 8192, 14336):
                     parts = split(ptr, ptr, T, N, K, code)
-                    assert 1 <= parts <= 4 and (parts == 1 or (T <= 64 and K * item % 512 == 0 and parts * 4 <= K * item // 512)), (T, N, K)
+                    assert 1 <= parts <= 4 and (parts == 1 or (T <= 64 and K * item % 512 == 0 and parts * 4 <= K * item // 512) or
+                                                            (T > 64 and item == 2 and N >= 128 and K % 64 == 0 and parts * 4 <= K // 64)), (T, N, K)
         assert split(ptr + 8, ptr, 1, 2048, 8192, code) == 1 and split(ptr, ptr + 8, 1, 2048, 8192, code) == 1     # no 16-byte pieces
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("T,N,chunks,parts", [(1, 16, 2, 2), (1, 2048, 8, 2), (16, 40, 7, 3), (17, 2049, 5, 4), (33, 4096, 16, 2), (48, 130, 32, 4),
-                                              (64, 2047, 33, 4)])
+                                              (64, 2047, 33, 4), (65, 130, 2, 4), (257, 1001, 3, 4), (300, 2048, 5, 2), (1101, 520, 4, 3)])
 def test_slabs_add_up_to_the_product(dtype, T, N, chunks, parts):
     from umbrella_amd import _lib
     dt, K = DTYPES[dtype], chunks * 512 // DTYPES[dtype].itemsize
+    if T > 64 and dtype == "fp32":
+        pytest.skip("slabs of many tokens are for 16-bit storage")
     g = torch.Generator().manual_seed(T * N + chunks)
     x, w, b = (torch.randn(s, generator=g).to(dt) for s in ((T, K), (N, K), (N,)))
     out = torch.full((parts + 1, T, N), 7.0, device="cuda:0")

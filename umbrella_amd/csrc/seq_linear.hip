@@ -354,14 +354,16 @@ __global__ __launch_bounds__(256) void seq_linear_wide_kernel(void* __restrict__
 template <typename P, int WM, int WN, int RA, int RB, int KS, bool DUAL>
 __global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS == 4 ? 2 : 1)
 void seq_linear_tile_kernel(void* __restrict__ out_, const u16* __restrict__ x, const u16* __restrict__ w, const u16* __restrict__ bias,
-                            int T, int N, int K, int epi, int nbt, float limit, float alpha) {
+                            int T, int N, int K, int epi, int nbt, int slabs, float limit, float alpha) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   typedef TileShape<WM, WN, RA, RB, KS> S;
   constexpr int OUTN = DUAL ? S::BN / 2 : S::BN;
   const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = wave_all % S::NW, ks = wave_all / S::NW, j = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
-  const int id = tile_of_block(blockIdx.x, gridDim.x);
-  const int n0 = (id / nbt) * OUTN, t0 = (id % nbt) * S::BT;
+  const int id = tile_of_block(blockIdx.x, gridDim.x), tiles = gridDim.x / slabs, sp = id / tiles, tile = id - sp * tiles;
+  const int n0 = (tile / nbt) * OUTN, t0 = (tile % nbt) * S::BT;
+  // slab sp of K (one more stage in the first ones): its sums go to out + sp T N, the bias into slab 0's
+  const int each = K / 64 / slabs, longer = K / 64 - each * slabs, st0 = sp * each + min(sp, longer), stages = each + (sp < longer);
   // rows past the operand's end re-read its last row: their outputs are not stored
   unsigned voff[S::NPW];
 #pragma unroll
@@ -376,7 +378,12 @@ void seq_linear_tile_kernel(void* __restrict__ out_, const u16* __restrict__ x, 
     else voff[i] = tile_voff(p - S::NPA, lane, K, [&](int row) { return min(t0 + row, T - 1) - t0; });
   }
   f32x4 acc[RA][RB];
-  if (!tile_products<P, WM, WN, RA, RB, KS, false>(acc, smem, w + (long)n0 * K, x + (long)t0 * K, 128, voff, K / 64, wave, ks)) return;
+  if (!tile_products<P, WM, WN, RA, RB, KS, false>(acc, smem, w + (long)n0 * K + st0 * 64, x + (long)t0 * K + st0 * 64, 128, voff, stages, wave, ks))
+    return;
+  if (sp) {
+    out_ = reinterpret_cast<float*>(out_) + (long)sp * T * N;
+    bias = nullptr;
+  }
   constexpr int NI = DUAL ? RA / 2 : RA;
   const int nw = n0 + (DUAL ? wm * (8 * RA) : wm * (16 * RA));         // this wave's first output
   const bool half = DUAL || epi == EPI_DT || epi == EPI_RELU2;
@@ -439,14 +446,14 @@ void seq_linear_tile_kernel(void* __restrict__ out_, const u16* __restrict__ x, 
 }
 
 template <typename P, int WM, int WN, int RA, int RB, int KS, bool DUAL>
-static int launch_tile_as(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, float limit, float alpha,
-                          hipStream_t st) {
+static int launch_tile_as(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, int slabs, float limit,
+                          float alpha, hipStream_t st) {
   typedef TileShape<WM, WN, RA, RB, KS> S;
   constexpr int OUTN = DUAL ? S::BN / 2 : S::BN;
   if (ensure_dynamic_lds<seq_linear_tile_kernel<P, WM, WN, RA, RB, KS, DUAL>>(S::LDS) != UMB_OK) return UMB_EHIP;
   const int nbn = (N + OUTN - 1) / OUTN, nbt = (T + S::BT - 1) / S::BT;
-  hipLaunchKernelGGL((seq_linear_tile_kernel<P, WM, WN, RA, RB, KS, DUAL>), dim3((unsigned)nbn * nbt), dim3(64 * S::NW * KS), S::LDS, st, out,
-                     (const u16*)x, (const u16*)w, (const u16*)bias, T, N, K, epi, nbt, limit, alpha);
+  hipLaunchKernelGGL((seq_linear_tile_kernel<P, WM, WN, RA, RB, KS, DUAL>), dim3((unsigned)nbn * nbt * slabs), dim3(64 * S::NW * KS), S::LDS, st,
+                     out, (const u16*)x, (const u16*)w, (const u16*)bias, T, N, K, epi, nbt, slabs, limit, alpha);
   UMB_LAUNCH_CHECK();
   return UMB_OK;
 }
@@ -455,16 +462,16 @@ static int launch_tile_as(void* out, const void* x, const void* w, const void* b
 // 2048 x 5120 x 2048 70 -> 48, 1101 x 2048 x 8192 79 -> 62, 2048 x 2048 x 2048 30 -> 22, 2466 x 4096 x 14336 376 -> 230, 700 x 4096 x 4096 47 -> 35, 512 x 2048 x 8192
 // 73 -> 53; 2048 x 16384 x 2048 gate/up 126 -> 121 and 2048 x 28672 x 4096 412 -> 404 keep their tiles.
 template <typename P, bool DUAL>
-static int launch_tile(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, float limit, float alpha,
-                       hipStream_t st) {
-  switch (tile_kind(T, DUAL ? 2 * N : N, K / 64, 1, K % 128 == 0)) {
-    case TILE_256: return launch_tile_as<P, 4, 2, 4, 8, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
-    case TILE_192: return launch_tile_as<P, 4, 2, 4, 6, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
-    case TILE_160: return launch_tile_as<P, 4, 2, 4, 5, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
-    case TILE_128W: return launch_tile_as<P, 4, 2, 4, 4, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
-    case TILE_96: return launch_tile_as<P, 4, 2, 4, 3, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
-    case TILE_128: return launch_tile_as<P, 2, 4, 4, 2, 1, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
-    default: return launch_tile_as<P, 2, 2, 4, 2, 2, DUAL>(out, x, w, bias, T, N, K, epi, limit, alpha, st);
+static int launch_tile(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, int slabs, float limit,
+                       float alpha, hipStream_t st) {
+  switch (tile_kind(T, DUAL ? 2 * N : N, (K / 64 + slabs - 1) / slabs, slabs, K % (128 * slabs) == 0)) {
+    case TILE_256: return launch_tile_as<P, 4, 2, 4, 8, 1, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
+    case TILE_192: return launch_tile_as<P, 4, 2, 4, 6, 1, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
+    case TILE_160: return launch_tile_as<P, 4, 2, 4, 5, 1, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
+    case TILE_128W: return launch_tile_as<P, 4, 2, 4, 4, 1, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
+    case TILE_96: return launch_tile_as<P, 4, 2, 4, 3, 1, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
+    case TILE_128: return launch_tile_as<P, 2, 4, 4, 2, 1, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
+    default: return launch_tile_as<P, 2, 2, 4, 2, 2, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
   }
 }
 
@@ -815,6 +822,14 @@ static int launch_tt(void* out, const void* x, const void* w, const void* bias, 
   return UMB_OK;
 }
 
+// Whether a dense product of more than 64 tokens takes the staged tiles (stream: the streaming kernel takes it otherwise).  Both operands are
+// re-used: from 256 tokens on, and for 65 and more where the launch has some 100 tiles of 128 x 128 (cold weights, 100 / 200 tokens: 18496 x 4096
+// 56 / 72 us, the streaming kernel 84 / 158; 4096 x 4096 41 / 39 us, streaming 18 / 32; 2048 x 8192, 255 tokens 73 us, streaming 29)
+static bool tiles_pay(int T, long rows, bool stream) {
+  const long tiles = (rows + 127) / 128 * ((T + 127) / 128);
+  return !(stream && tiles < (T < 256 ? 96 : 49)) && (T >= 256 || tiles >= 96);
+}
+
 template <typename P, bool VEC>
 static int launch_vec(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, hipStream_t st,
                       const LinExt& ext, int gz = 1) {
@@ -822,14 +837,9 @@ static int launch_vec(void* out, const void* x, const void* w, const void* bias,
   constexpr int EB = sizeof(typename El<P>::type);
   const bool stream = VEC && stream_ok(x, w, N, K, epi, ext, EB) && stream_pays(T, N, K, epi, gz, EB);
   if constexpr (sizeof(typename El<P>::type) == 2) {
-    // both operands re-used: from 256 tokens on, and for 65 and more where the launch has some 100 tiles of 128 x 128 (cold weights, 100 /
-    // 200 tokens: 18496 x 4096 56 / 72 us, the streaming kernel 84 / 158; 4096 x 4096 41 / 39 us, streaming 18 / 32; 2048 x 8192,
-    // 255 tokens 73 us, streaming 29)
-    const long rows = (long)(epi_dual(epi) ? 2 : 1) * N, tiles = (rows + 127) / 128 * ((T + 127) / 128);
-    if (T > 64 && VEC && dense && N >= 128 && tile_ok(out, x, w, T, N, K, epi) && !(stream && tiles < (T < 256 ? 96 : 49)) &&
-        (T >= 256 || tiles >= 96))
-      return epi_dual(epi) ? launch_tile<P, true>(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, st)
-                           : launch_tile<P, false>(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, st);
+    if (T > 64 && VEC && dense && N >= 128 && tile_ok(out, x, w, T, N, K, epi) && tiles_pay(T, (long)(epi_dual(epi) ? 2 : 1) * N, stream))
+      return epi_dual(epi) ? launch_tile<P, true>(out, x, w, bias, T, N, K, epi, 1, ext.limit, ext.alpha, st)
+                           : launch_tile<P, false>(out, x, w, bias, T, N, K, epi, 1, ext.limit, ext.alpha, st);
   }
   if (stream) return launch_stream<P>(out, x, w, bias, T, N, K, epi, st, ext, 0, gz);
   if (T <= 16) return launch_tt<P, 1, 1, VEC>(out, x, w, bias, T, N, K, epi, st, ext, 0, gz);
@@ -870,10 +880,35 @@ extern "C" int umb_seq_linear(void* out, const void* x, const void* w, const voi
 // rows each halve; a slab is four chunks at least (shorter ones are all prologue).  us at 1 / 16 / 48 tokens, bf16, cold weights, one MI355X,
 // 1 slab -> this rule's: 2048 x 8192 10.5 / 12.1 / 18.9 -> 8.8 / 9.5 / 10.8 (4); 2048 x 2048 4.6 / 5.0 / 7.2 -> 3.9 / 4.1 / 5.4 (2); 2560 x 6912 9.3 / 11.1 /
 // 15.3 -> 8.3 / 9.9 / 10.6 (3); 4096 x 14336, 48 tokens 37 -> 26 (2), and 1 / 16 tokens 24.0 / 24.7 stay whole (24.3 / 25.6 in two).
+//
+// Many tokens: the staged tiles, where rounds of them fill better with K in slabs than the whole K does: the least of the product's time and of
+// reading the slabs beyond the first in the kernel behind it (8 TB/s, they come from the last-level cache), against the whole K on the tiles or on
+// the streaming kernel (0.50 us a chunk and round of 16 rows x 64 tokens a workgroup, 0.78 of 32).  us, whole / this: 4096 x 14336 at 100 / 300 / 1101 /
+// 1999 tokens 46 / 95 / 171 / 198 -> 33 / 52 / 121 / 178; 2048 x 8192 at 128 / 300 / 1101 20.9 / 47 / 62 -> 20.9 / 22 / 42; 4096 x 4096 at 1101 53 -> 42.
+static int tile_slabs(int T, int N, int K, bool stream) {
+  double best = 1e30, us = 0.0;
+  if (tiles_pay(T, N, stream)) {
+    (void)tile_kind(T, N, K / 64, 1, K % 128 == 0, &best);
+  } else if (stream) {
+    const bool narrow = stream_narrow(N, (T + 63) / 64, 1);
+    const long wgs = (long)((N + (narrow ? 15 : 31)) / (narrow ? 16 : 32)) * ((T + 63) / 64);
+    best = 2.5 + (wgs + 255) / 256 * (K / 256) * (narrow ? 0.50 : 0.78);
+  }
+  int best_s = 1;
+  for (int S = 2; S <= 4 && S * 4 <= K / 64; ++S) {
+    (void)tile_kind(T, N, (K / 64 + S - 1) / S, S, K % (128 * S) == 0, &us);
+    us += (S - 1) * (double)T * N * 4 / 8e6;
+    if (us < best) { best = us; best_s = S; }
+  }
+  return best_s;
+}
+
 extern "C" int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype) {
-  if (T < 1 || T > 64 || N < 1 || K < 1) return 1;
+  if (T < 1 || N < 1 || K < 1) return 1;
   const int eb = (int)seq_elem_bytes(dtype), chunks = (int)((long)K * eb / 512), blocks = (N + 15) / 16;
-  if (!stream_ok(x, w, N, K, EPI_F32, lin_dense(N, K), eb)) return 1;
+  const bool stream = stream_ok(x, w, N, K, EPI_F32, lin_dense(N, K), eb);
+  if (T > 64) return eb == 2 && N >= 128 && tile_ok(nullptr, x, w, T, N, K, EPI_F32) ? tile_slabs(T, N, K, stream && stream_pays(T, N, K, EPI_F32, 1, eb)) : 1;
+  if (!stream) return 1;
   const int parts = std::min(std::min(512 / blocks, 4), chunks / 4);
   return parts < 2 || (parts == 2 && blocks > 128 && T <= 32) ? 1 : parts;
 }
@@ -886,6 +921,12 @@ extern "C" int umb_seq_linear_parts(float* out, const void* x, const void* w, co
   ext.so = (long)T * N;
   ext.parts = parts;
   ext.part_chunks = (int)((long)K * seq_elem_bytes(dtype) / 512) / parts;
+  if (T > 64) {
+    if (parts > K / 64 || !tile_ok(out, x, w, T, N, K, EPI_F32)) return UMB_EINVAL;
+    if (dtype == UMB_SEQ_BF16) return launch_tile<BF16, false>(out, x, w, bias, T, N, K, EPI_F32, parts, 0.f, 0.f, st);
+    if (dtype == UMB_SEQ_F16) return launch_tile<F16, false>(out, x, w, bias, T, N, K, EPI_F32, parts, 0.f, 0.f, st);
+    return UMB_EINVAL;
+  }
   DISPATCH_SEQ_DTYPE(dtype, {
     constexpr int EB = sizeof(typename El<P>::type);
     if (parts > (long)K * EB / 512 || !stream_ok(x, w, N, K, EPI_F32, ext, EB)) return UMB_EINVAL;

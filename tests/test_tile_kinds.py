@@ -62,3 +62,25 @@ def test_every_tile_of_packed_weights(T, N, K, S):
     want = gate * torch.sigmoid(gate) * up
     bound = 1.05 * half_ulp * (1.1 * gate.abs() * up.abs() + 3 * want.abs()) + 1.1 * tg * up.abs() + 1.1 * gate.abs() * tu + 2e-6 * want.abs() + 2.0 ** -24
     assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())
+
+
+@pytest.mark.parametrize("T", [1, 300])
+@pytest.mark.parametrize("epi", [2, 6])
+def test_gates_far_from_zero(T, epi):
+    """gated epilogues at the ends of their exponential, at infinities and NaN: what torch gives in 64 bits, on few tokens and on tiles"""
+    from umbrella_amd import _lib
+    K, vals = 64, [0.0, -0.0, 1e-20, 3.0, -3.0, 30.0, -30.0, 86.0, -86.0, 200.0, -200.0, 3e38, float("inf"), float("nan")]
+    n = 128
+    w = torch.zeros(2 * n, K, device="cuda", dtype=torch.bfloat16)
+    w[:n, 0], w[n:, 1] = 1.0, 1.0                              # gate = x[0], up = x[1]
+    for v in vals:
+        x = torch.zeros(T, K, device="cuda", dtype=torch.bfloat16)
+        x[:, 0], x[:, 1] = v, 1.0
+        act = torch.empty(T, n, device="cuda", dtype=torch.bfloat16)
+        _lib.seq_call("umb_seq_linear", act, x, w, None, T, 2 * n, K, epi, _lib.BF16)
+        g = x[0, 0].double().cpu()
+        if v == float("inf") or v != v:                        # 0 * inf in the other products of the row: everything is NaN
+            assert bool(torch.isnan(act).all())
+            continue
+        want = g * torch.sigmoid(g) if epi == 2 else torch.nn.functional.gelu(g, approximate="tanh")
+        assert ((act.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-30).all(), v

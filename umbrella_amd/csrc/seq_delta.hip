@@ -171,6 +171,69 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(float* __restrict__ q, 
   }
 }
 
+// The same for few taps, rows in quads: LPS lanes hold a slot's row four channels each and go down eight tokens, so a projection row is fetched
+// (8 + TAPS - 1) / 8 times and not TAPS times, 16 bytes a lane, with all rows in flight.  A wave per token and slot with single channels took
+// 70 us for 2466 tokens of 8 + 8 + 16 slots of 128 (80 MB), this 27 (3 TB/s).
+template <typename P, int TAPS, int LPS>
+__global__ __launch_bounds__(256) void delta_prep_quad_kernel(float* __restrict__ q, float* __restrict__ k, int ldqk, int Dp,
+                                                              float* __restrict__ v, float* __restrict__ beta, float* __restrict__ lg,
+                                                              DeltaIn in, const typename El<P>::type* __restrict__ conv_w,
+                                                              const int* __restrict__ pos, const int* __restrict__ slot_, int T, float qscale,
+                                                              int packs) {
+  constexpr int NT = 8, SPW = 64 / LPS, NR = NT + TAPS - 1;
+  const int item = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  const int t0 = __builtin_amdgcn_readfirstlane(item / packs) * NT, lane = threadIdx.x & 63, l = lane % LPS;
+  if (t0 >= T) return;
+  const int hs = (item - t0 / NT * packs) * SPW + lane / LPS, per = 2 * in.Hk + in.H, nt = min(NT, T - t0), D = in.D, E = in.E, C = in.C();
+  if (hs > per) return;
+  if (hs == per) {                                       // the gates of the tokens
+    for (int i = l; i < nt * in.H; i += LPS) {
+      const int t = t0 + i / in.H, h = i % in.H;
+      const float* pr = in.proj + (long)t * in.ld + in.col0 + C + in.H * E;
+      beta[(long)t * in.H + h] = 1.f / (1.f + expf(-pr[h]));
+      lg[(long)t * in.H + h] = -expf(in.a_log[h]) * delta_softplus(pr[in.H + h] + in.dt_bias[h]);
+    }
+    return;
+  }
+  const bool is_v = hs >= 2 * in.Hk, is_q = hs < in.Hk;
+  const int width = is_v ? E : D, col = is_v ? 2 * in.qk() + (hs - 2 * in.Hk) * E : hs * D;
+  for (int c0 = 4 * l; c0 < (is_v ? E : 4 * LPS); c0 += 4 * LPS) {     // one round for q and k, with every lane in the sum
+    const int c = col + min(c0, width - 4);
+    f32x4 x[NR], wq[TAPS];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) x[r] = *reinterpret_cast<const f32x4*>(in.proj + (long)min(max(t0 - (TAPS - 1) + r, 0), T - 1) * in.ld + in.col0 + c);
+#pragma unroll
+    for (int i = 0; i < TAPS; ++i) wq[i] = ld4<P>(conv_w + (long)c * TAPS + 4 * i);
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      if (u >= nt) break;
+      const int t = t0 + u, p = pos[t], slot = slot_[t];
+      f32x4 acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) {
+        const int d = TAPS - 1 - j;                      // tap j looks d positions back: this step's row, the ring's, or none
+        f32x4 xv = x[u + j];
+        if (d > 0 && !(t - d >= 0 && slot_[t - d] == slot))
+          xv = d <= p ? *reinterpret_cast<const f32x4*>(in.ring + ((long)slot * TAPS + (p - d) % TAPS) * C + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += wq[(e * TAPS + j) / 4][(e * TAPS + j) % 4] * xv[e];
+      }
+      f32x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = c0 < width ? siluf_(acc[e]) : 0.f;
+      if (is_v) {
+        *reinterpret_cast<f32x4*>(v + ((long)t * in.H + (hs - 2 * in.Hk)) * E + c0) = y;
+        continue;
+      }
+      float ss = sq4(y);
+#pragma unroll
+      for (int o = LPS / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      const float f = (is_q ? qscale : 1.f) / sqrtf(ss + DELTA_UNIT_EPS);
+      if (c0 < Dp) *reinterpret_cast<f32x4*>((is_q ? q : k) + (long)t * ldqk + (long)(is_q ? hs : hs - in.Hk) * Dp + c0) = y * f;       // zeros from D to Dp
+    }
+  }
+}
+
 // ---- the recurrence in chunks of 64 tokens.  With c_t = log g_1 + .. + log g_t inside a chunk and S_0 the state before it,
 //     u_t = beta_t (v_t - e^(c_t) S_0^T k_t - sum_{s < t} e^(c_t - c_s) (k_s . k_t) u_s)
 // is a unit lower triangular system (I + A) U = diag(beta) V - diag(beta e^c) K S_0, A_ts = beta_t e^(c_t - c_s) (k_t . k_s).  So
@@ -494,6 +557,25 @@ extern "C" int umb_delta_prep(float* q, float* k, int ldqk, float* v, float* bet
     return UMB_EINVAL;
   const DeltaIn in{proj, ld, col0, Hk, H, D, E, taps, ring, dt_bias, a_log};
   const long items = (long)T * (2 * Hk + H + 1);
+  if ((taps == 3 || taps == 4) && D % 4 == 0 && E % 4 == 0 && ld % 4 == 0 && col0 % 4 == 0 && ldqk % 4 == 0 &&
+      ((uintptr_t)proj | (uintptr_t)ring | (uintptr_t)conv_w | (uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16 == 0) {
+#define DELTA_QUADS(TAPS, LPS)                                                                                                          \
+  do {                                                                                                                                  \
+    const int packs = (2 * Hk + H + 1 + 64 / LPS - 1) / (64 / LPS);                                                                     \
+    hipLaunchKernelGGL((delta_prep_quad_kernel<P, TAPS, LPS>), dim3((unsigned)(((T + 7) / 8 * (long)packs + 3) / 4)), dim3(256), 0, st, q, k, ldqk, \
+                       up16(D), v, beta, log_g, in, (const El_*)conv_w, pos, slot, T, 1.f / sqrtf((float)D), packs);                    \
+  } while (0)
+    DISPATCH_SEQ_DTYPE(dtype, {
+      typedef typename El<P>::type El_;
+      if (taps == 4 && D <= 128) DELTA_QUADS(4, 32);
+      else if (taps == 4) DELTA_QUADS(4, 64);
+      else if (D <= 128) DELTA_QUADS(3, 32);
+      else DELTA_QUADS(3, 64);
+    })
+#undef DELTA_QUADS
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
   DISPATCH_SEQ_DTYPE(dtype, {
     typedef typename El<P>::type El_;
     hipLaunchKernelGGL(delta_prep_kernel<P>, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, st, q, k, ldqk, up16(D), v, beta, log_g, in,

@@ -67,19 +67,6 @@ static inline bool epi_dual(int epi) { return epi == EPI_SILU_MUL || epi == EPI_
 static inline bool epi_plain(int epi) {
   return epi == EPI_F32 || epi == EPI_DT || epi == EPI_SILU_MUL || epi == EPI_RELU2 || epi == EPI_GELU_MUL;
 }
-// z / (1 + e^-u) as exactly as expf and a division give it, in two thirds of their instructions: the exponent of 2 in whole and rest (v_exp_f32 on the
-// rest), no cases beyond |u| = 88, and one step on the quotient.  Infinities and NaN as there (the step is dropped where it is not a number).
-// Error of z = u over |u| < 30 against 64 bits, in 2^-24 of the value: largest 2.96, root mean square 0.641, both as there.  A prompt's gated
-// feed-forward does 64 of these a lane behind its products (16384 x 2048, 2048 tokens: 125 us -> 111 with them, the biases and the choice of
-// the epilogue out of the loop over tokens).
-__device__ __forceinline__ float over_one_plus_exp(float z, float u) {
-#pragma clang fp contract(off)
-  const float c = __builtin_amdgcn_fmed3f(u, -88.f, 88.f), h = -c * 1.44269502f, n = __builtin_rintf(h);
-  const float l = fmaf(-c, 1.92596303e-8f, fmaf(-c, 1.44269502f, -h));         // log2(e) in two parts
-  const float d = 1.f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((h - n) + l), (int)n);
-  const float r = __builtin_amdgcn_rcpf(d), q = z * r, p = fmaf(fmaf(-q, d, z), r, q);
-  return p == p ? p : q;
-}
 // 0.5 z (1 + tanh(u)) with u = sqrt(2 / pi) (z + 0.044715 z^3), as z / (1 + e^(-2 u)): the same function, one exponential, and no
 // cancellation where tanh is near -1
 __device__ __forceinline__ float gelu_tanhf_(float z) { return over_one_plus_exp(z, 1.5957691216057308f * (z + 0.044715f * z * z * z)); }

@@ -84,3 +84,32 @@ def test_gates_far_from_zero(T, epi):
             continue
         want = g * torch.sigmoid(g) if epi == 2 else torch.nn.functional.gelu(g, approximate="tanh")
         assert ((act.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-30).all(), v
+
+
+# per-head products on tiles (96 of them and more) and just below, ragged tokens and rows, one stage and several, row strides beyond the row; outputs
+# whose rows are no whole 16-byte groups stay where they were
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,N,K,pad", [(32, 385, 128, 64, 8), (7, 900, 200, 192, 0), (50, 257, 72, 320, 24), (12, 1024, 64, 128, 8), (24, 500, 130, 64, 2)])
+def test_batched_tiles(dtype, B, T, N, K, pad):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + N + K)
+    code, ldx, per = _lib.seq_dtype_code(dtype), B * K + pad, N + pad
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    x, w = torch.randn(T, ldx, generator=g, device="cuda").to(dtype), torch.randn(B, N, K, generator=g, device="cuda").to(dtype)
+    gate = torch.randn(T, B * N, generator=g, device="cuda")
+    xs, wt = x[:, :B * K].double().view(T, B, K).transpose(0, 1).contiguous(), w.double().transpose(1, 2).contiguous()
+    full, size = (torch.bmm(a, b).transpose(0, 1) for a, b in ((xs, wt), (xs.abs(), wt.abs())))          # [T][B][N]
+    tol = 2.0 ** -24 * (K + 2) * size
+    for epi in (0, 1, 3, 7):
+        out = torch.full((T + 1, B * per), 7.0, dtype=torch.float32 if epi == 0 else dtype, device="cuda")
+        _lib.seq_call("umb_seq_linear_batched", out, x, w, T, N, K, ldx, B * per, B, K, N * K, per, epi, gate if epi > 1 else None, B * N,
+                      N if epi == 3 else 1, code)
+        f = 1.0
+        if epi == 3:
+            f = torch.sigmoid(gate.double()).view(T, B, N)
+        elif epi == 7:
+            f = torch.sigmoid(gate[:, :B].double())[..., None]
+        got = out[:T].double().view(T, B, per)
+        want = full * f
+        bound = tol + 2.0 ** -22 * want.abs() + (0.0 if epi == 0 else 1.02 * half_ulp * want.abs() + 2.0 ** -25)
+        assert ((got[..., :N] - want).abs() <= bound).all() and bool((got[..., N:] == 7.0).all()) and bool((out[T] == 7.0).all())

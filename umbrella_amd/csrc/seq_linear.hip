@@ -486,6 +486,82 @@ static int launch_tile_as(void* out, const void* x, const void* w, const void* b
   return UMB_OK;
 }
 
+// ---- many tokens of a batch of small problems (per-head products): the same main loop, rows with strides of their own, 128 x 128 tiles of four
+// waves, two workgroups a CU: K is a few stages, and one's stores run beside the other's products.  us, 64 x 64 tiles from L2 / this, bf16:
+// 32 heads, fp32 out 512 x 128 at 128 / 400 / 1999 tokens 8.1 / 22.8 / 83 -> 5.9 / 9.1 / 29 (147 MB out), gated 128 x 512 6.9 / 16.7 / 58 -> 9.7 / 10.5 / 21;
+// 16 heads 256 x 64 at 256 / 1101 5.7 / 15.9 -> 5.9 / 7.7, gated 64 x 256 at 400 / 1101 6.5 / 12.1 -> 8.4 / 8.5.  So from 96 tiles on.
+template <typename P>
+__global__ __launch_bounds__(256, 2) void seq_linear_tile_batched_kernel(void* __restrict__ out_, const u16* __restrict__ x, const u16* __restrict__ w,
+                                                                          int T, int N, int K, int epi, int nbt, int nbn, LinExt ext) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr int WN = 2, RA = 4, RB = 4;
+  typedef TileShape<2, WN, RA, RB, 1> S;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
+  const int id = tile_of_block(blockIdx.x, gridDim.x), column = __builtin_amdgcn_readfirstlane(id / nbt), z = __builtin_amdgcn_readfirstlane(column / nbn);
+  const int n0 = (column - z * nbn) * S::BN, t0 = (id - column * nbt) * S::BT;
+  unsigned voff[S::NPW];
+#pragma unroll
+  for (int i = 0; i < S::NPW; ++i) {
+    const int p = wave + S::NW * i;
+    if (S::NW * i < S::NPA) voff[i] = tile_voff(p, lane, K, [&](int row) { return min(n0 + row, N - 1) - n0; });
+    else voff[i] = tile_voff(p - S::NPA, lane, ext.ldx, [&](int row) { return min(t0 + row, T - 1) - t0; });
+  }
+  f32x4 acc[RA][RB];
+  (void)tile_products<P, 2, WN, RA, RB, 1, false>(acc, smem, w + z * ext.sw + (long)n0 * K, x + z * ext.sx + (long)t0 * ext.ldx, 128, voff, K / 64, wave, 0);
+  const int nw = n0 + wm * (16 * RA);
+  const long obase = z * ext.so;
+  const float* gate = ext.gate ? ext.gate + (long)z * ext.sg : nullptr;
+  const unsigned strip = (unsigned)(size_t)(lds_char*)smem + (unsigned)wave * TileRows<16, RA>::BYTES;
+#pragma unroll
+  for (int t = 0; t < RB; ++t) {
+    const int tile0 = t0 + (wn * RB + t) * 16;
+    f32x4 v[RA];
+#pragma unroll
+    for (int i = 0; i < RA; ++i) v[i] = acc[i][t];
+    if (gate) {
+      const float* gr = gate + (long)min(tile0 + j, T - 1) * ext.ldg;
+      const float row = epi == EPI_GATE_ROW ? gr[0] : 0.f;
+#pragma unroll
+      for (int i = 0; i < RA; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[i][r] = over_one_plus_exp(v[i][r], epi == EPI_GATE_ROW ? row : gr[min(nw + i * 16 + 4 * g + r, N - 1)]);
+    }
+    if (epi == EPI_F32) {
+      tile_rows_out<16, RA>(strip, v, [&](int row, int at, u32x4 b) {
+        if (tile0 + row < T && nw + at / 4 < N) *reinterpret_cast<u32x4*>(reinterpret_cast<float*>(out_) + obase + (long)(tile0 + row) * ext.ldo + nw + at / 4) = b;
+      });
+      continue;
+    }
+    u32x2 d[RA];
+#pragma unroll
+    for (int i = 0; i < RA; ++i) d[i] = u32x2{pack2<P>(v[i][0], v[i][1]), pack2<P>(v[i][2], v[i][3])};
+    tile_rows_out<8, RA>(strip, d, [&](int row, int at, u32x4 b) {
+      if (tile0 + row < T && nw + at / 2 < N) *reinterpret_cast<u32x4*>(reinterpret_cast<u16*>(out_) + obase + (long)(tile0 + row) * ext.ldo + nw + at / 2) = b;
+    });
+  }
+}
+
+// whole 64-k stages, every row of every problem 16-byte aligned and stored in whole 16-byte groups, 32-bit offsets inside an operand
+template <typename P>
+static bool tile_batched_ok(const void* out, const void* x, const void* w, int T, int N, int K, int epi, const LinExt& ext, int batch) {
+  if constexpr (sizeof(typename El<P>::type) == 4) return false;
+  const int per = epi == EPI_F32 ? 4 : 8;                    // outputs of 16 bytes
+  if ((long)((N + 127) / 128) * ((T + 127) / 128) * batch < 96) return false;
+  return T >= 128 && N >= 64 && K % 64 == 0 && N % per == 0 && ext.ldo % per == 0 && ext.so % per == 0 && ext.ldx % 8 == 0 && ext.sx % 8 == 0 &&
+         ext.sw % 8 == 0 && ((uintptr_t)out | (uintptr_t)x | (uintptr_t)w) % 16 == 0 && (long)ext.ldx * 256 < (1L << 31) && (N + 128L) * K < (1L << 31);
+}
+template <typename P>
+static int launch_tile_batched(void* out, const void* x, const void* w, int T, int N, int K, int epi, const LinExt& ext, int batch, hipStream_t st) {
+  typedef TileShape<2, 2, 4, 4, 1> S;
+  if (ensure_dynamic_lds<seq_linear_tile_batched_kernel<P>>(S::LDS) != UMB_OK) return UMB_EHIP;
+  const int nbn = (N + S::BN - 1) / S::BN, nbt = (T + S::BT - 1) / S::BT;
+  if ((long)nbn * nbt * batch > 0x7fffffffL) return UMB_EINVAL;
+  hipLaunchKernelGGL(seq_linear_tile_batched_kernel<P>, dim3((unsigned)nbn * nbt * batch), dim3(256), S::LDS, st, out, (const u16*)x, (const u16*)w, T, N, K,
+                     epi, nbt, nbn, ext);
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+
 // us at T x N x K, two kinds of 256 x 256 / 128 x 128 tiles by a fixed share of a round (the rule before) -> tile_kind's: 1101 x 16384 x 2048 gate/up 109 -> 83,
 // 2048 x 5120 x 2048 70 -> 48, 1101 x 2048 x 8192 79 -> 62, 2048 x 2048 x 2048 30 -> 22, 2466 x 4096 x 14336 376 -> 230, 700 x 4096 x 4096 47 -> 35, 512 x 2048 x 8192
 // 73 -> 53; 2048 x 16384 x 2048 gate/up 126 -> 121 and 2048 x 28672 x 4096 412 -> 404 keep their tiles.
@@ -984,6 +1060,8 @@ extern "C" int umb_seq_linear_batched(void* out, const void* x, const void* w, i
   // 16-byte loads need every row start aligned: the strides as well as K
   const bool vec = K % 8 == 0 && ldx % 8 == 0 && sx % 8 == 0 && sw % 8 == 0;
   DISPATCH_SEQ_DTYPE(dtype, {
+    if constexpr (sizeof(typename El<P>::type) == 2)
+      if (tile_batched_ok<P>(out, x, w, T, N, K, epi, ext, batch)) return launch_tile_batched<P>(out, x, w, T, N, K, epi, ext, batch, st);
     if (vec) return launch_vec<P, true>(out, x, w, nullptr, T, N, K, epi, st, ext, batch);
     return launch_vec<P, false>(out, x, w, nullptr, T, N, K, epi, st, ext, batch);
   })

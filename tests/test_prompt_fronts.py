@@ -1,5 +1,5 @@
 """What stands between a prompt's projection and its mixer, walked in quads: against the kernels of single channels, which take the same numbers from
-columns that are not 16-byte aligned."""
+columns that are not 16-byte aligned.  And attention of more than 1024 query tiles against float64."""
 import pytest
 import torch
 
@@ -42,3 +42,44 @@ def test_delta_fronts(dtype, taps, Hk, H, D, E):
     assert (outs[0][2] - outs[1][2]).abs().max() <= 2e-6 * outs[1][2].abs().max()          # sums of 3 or 4 products
     for a, b in zip(outs[0][:2], outs[1][:2]):                 # unit rows: sums of D squares in another order
         assert (a - b).abs().max() <= 4e-7 * D ** 0.5
+
+
+# more than 1024 tiles of 16 rows: ragged rows, prefixes around a 64-key step and none, a cache that ends inside one (Lmax an odd multiple of 32),
+# trees and causal prompts, stale keys behind the valid ones
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,Hq,Hkv,T,prefix,spare", [(128, 64, 8, 257, 63, 0), (128, 32, 8, 530, 0, 32), (64, 32, 8, 515, 65, 32), (64, 12, 4, 1400, 1, 0),
+                                                     (32, 32, 32, 529, 130, 96), (32, 40, 8, 430, 0, 32)])
+def test_attention_of_many_tiles(dtype, D, Hq, Hkv, T, prefix, spare):
+    import numpy as np
+    from umbrella_amd.attn.cache import VT_PAD, k_to_frag, vt_to_frag
+    from umbrella_amd import _lib
+    from umbrella_amd.models.llama import pack_mask_bits
+    S, g = prefix + T, Hq // Hkv
+    Lmax = (S + 31) // 32 * 32 + spare
+    gen = torch.Generator().manual_seed(T + D)
+    q, k, v = (torch.randn(n, h, D, generator=gen).to(dtype) for n, h in ((T, Hq), (S, Hkv), (S, Hkv)))
+    kc, vt = torch.full((Hkv, Lmax, D), 7.0, dtype=dtype), torch.full((Hkv, D, Lmax + VT_PAD), -9.0, dtype=dtype)
+    kc[:, :S], vt[:, :, :S] = k.permute(1, 0, 2), v.permute(1, 2, 0)
+    kc, vt, qd = k_to_frag(kc).cuda(), vt_to_frag(vt).cuda(), q.cuda()
+    rs = np.random.RandomState(T)
+    tree = torch.zeros(T, T, dtype=torch.bool)
+    for i in range(T):
+        if i:
+            tree[i] = tree[max(0, i - 1 - rs.randint(0, min(i, 24)))]
+        tree[i, i] = True
+    pre = torch.tensor([prefix], dtype=torch.int32, device="cuda")
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for bits, see in ((pack_mask_bits(tree).cuda(), tree), (None, torch.ones(T, T).tril().bool())):
+        out = torch.full((T + 1, Hq, D), 3.0, dtype=dtype, device="cuda")
+        _lib.call("umb_tree_attn", out, qd, kc, vt, None, None, pre, bits, 0 if bits is None else bits.shape[1], T, T, Hq, Hkv, D, Lmax, 256, 1,
+                  D ** -0.5, None, _lib.dtype_code(dtype))
+        mask = torch.cat([torch.ones(T, prefix, dtype=torch.bool), see], dim=1).cuda()
+        for h in range(Hkv):
+            kd, vd = k[:, h].double().cuda(), v[:, h].double().cuda()
+            for a in range(h * g, h * g + g):
+                p = torch.softmax(((q[:, a].double().cuda() @ kd.T) * D ** -0.5).masked_fill(~mask, -torch.inf), dim=-1)
+                want = p @ vd
+                # weights rounded to storage (a relative unit each), the result rounded once
+                bound = 1.1 * unit * (p @ vd.abs()) + 1.1 * unit * want.abs() + 1e-5
+                assert ((out[:T, a].double() - want).abs() <= bound).all()
+        assert bool((out[T] == 3.0).all())

@@ -21,6 +21,7 @@
 //   grid = (Hkv, query-tile groups, key splits); partial (m, l, O) per split are
 //   merged by attn_combine_kernel.
 #include "common.h"
+#include "gemm_tile.h"
 
 #define NEG_BIG (-1.0e30f)
 
@@ -491,6 +492,170 @@ __global__ __launch_bounds__(64 * NW, NQ > 1 ? 1 : 2) void tree_attn1_kernel(con
   }
 }
 
+// ---- many query tiles (wide trees, prompt chunks): four waves of one 16-row query tile each share the keys.
+// A wave per workgroup that walks 32 keys at a time (tree_attn1_kernel) is a chain -- products, maximum, two exchanges between lanes, exponents,
+// products -- of some 900 cycles per tile, two waves a SIMD, and pulls 16 KiB through the CU's path to L2 for each.  Here 64 keys make a step: one
+// chain for twice the work, its exchanges by lane swaps instead of through LDS, exponents in base 2 (one multiplication less); their K and V^T
+// (contiguous in the cache's fragment order) go to LDS by LDS-DMA once for the four tiles, one barrier a step; a fragment is read as it lies, a
+// contiguous KiB.  Two workgroups share a CU.  us, one MI355X, a wave each / this: 1024 causal
+// tokens of 32 + 8 heads of 128 behind 0 / 1024 keys 36 / 69 -> 25 / 46, of 64 24 / 42 -> 17 / 29; 257 tree rows of 64 + 8 heads behind 700 33 -> 25;
+// 769 behind 500 72 -> 54.  32 rows a wave (half the LDS reads, one wave a SIMD): 40 / 69.
+// max over lanes l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ float quad_max(float v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+template <typename P, int D>
+__global__ __launch_bounds__(256, 2) void wide_attn_kernel(const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vt,
+                                                           const int* __restrict__ prefix_p, int T, int Hq, int Hkv, int Lmax, int mask_words,
+                                                           int n_mask_keys, const unsigned long long* __restrict__ mask_bits, float scale,
+                                                           u16* __restrict__ out, int fold) {
+  constexpr int DS = D / 32, DT = D / 16, R = D == 128 ? 2 : 4, PW = D / 16;      // slots; 1-KiB pieces a wave fetches of a step
+  constexpr unsigned SLOT = 256u * D, HALF = SLOT / 2;                            // K | V^T of 64 keys
+  __shared__ __attribute__((aligned(16))) unsigned char ring[R * SLOT];
+  __shared__ int tops[4];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, gq = lane >> 4;
+  // later rows see more keys: they start first, or, where two workgroups a CU hold them all, each with an early one
+  const int ny = gridDim.y, y = blockIdx.y, h = blockIdx.x, four = fold && y >= (ny + 1) / 2 ? y - (ny + 1) / 2 : ny - 1 - y;
+  const int g = Hq / Hkv, nrows = T * g, row = four * 64 + wv * 16 + j;
+  const bool row_ok = row < nrows;
+  const int t = row_ok ? row / g : 0, hq = h * g + (row_ok ? row % g : 0);
+  const unsigned lds0 = (unsigned)(size_t)(lds_char*)ring;
+  const char* kbase = reinterpret_cast<const char*>(kc + (long)h * Lmax * D);
+  const char* vbase = reinterpret_cast<const char*>(vt + (long)h * D * VT_LD(Lmax));
+  const unsigned voff = (unsigned)lane * 16u;
+  auto issue = [&](int st, unsigned slot) {                  // waves 0 and 1 fetch K, 2 and 3 V^T
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {                           // (a piece past the cache is its last one again: keys that no tile walks)
+      const long at = min((long)st * HALF + ((wv & 1) * PW + i) * 1024, (long)Lmax * D * 2 - 1024);
+      tile_dma(voff, (wv < 2 ? kbase : vbase) + at, lds0 + slot + (unsigned)(wv * PW + i) * 1024u);
+    }
+  };
+#pragma unroll
+  for (int c = 0; c < R - 1; ++c) issue(c, c * SLOT);        // their place follows from the workgroup alone: under way before the prefix is known
+  const u32x4 zero4 = {0u, 0u, 0u, 0u};
+  u32x4 bq[DS];
+#pragma unroll
+  for (int ds = 0; ds < DS; ++ds)
+    bq[ds] = row_ok ? *reinterpret_cast<const u32x4*>(q + ((long)t * Hq + hq) * D + ds * 32 + gq * 8) : zero4;
+  const int prefix = *prefix_p, kv_end = prefix + n_mask_keys;
+  int k_hi = kv_end, k_all = kv_end;                         // behind the last key that this tile, and any of the four, sees
+  {
+    int top = -1;
+    if (row_ok && mask_bits) {
+      const unsigned long long* mrow = mask_bits + (long)t * mask_words;
+      for (int w = mask_words - 1; w >= 0; --w) {
+        const unsigned long long x = mrow[w];
+        if (x) { top = w * 64 + 63 - __clzll((long long)x); break; }
+      }
+    } else if (row_ok) {
+      top = t;
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) top = max(top, __shfl_xor(top, off, 64));
+    if (lane == 0) tops[wv] = top;
+    __syncthreads();
+    k_hi = min(k_hi, prefix + top + 1);
+    k_all = min(k_all, prefix + max(max(tops[0], tops[1]), max(tops[2], tops[3])) + 1);
+  }
+  const float scale2 = scale * 1.44269504088896341f;         // scores in base 2
+  float m = NEG_BIG, l = 0.f;
+  f32x4 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int ns = (k_all + 63) / 64;
+  unsigned slot = 0;
+  for (int st = 0; st < ns; ++st) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((R - 2) * PW) : "memory");
+    __builtin_amdgcn_s_barrier();
+    issue(st + R - 1, slot == 0 ? (R - 1) * SLOT : slot - SLOT);
+    const unsigned base = lds0 + slot + voff;
+    slot = slot == (R - 1) * SLOT ? 0 : slot + SLOT;
+    const int k0 = st * 64;
+    if (k0 >= k_hi) continue;
+    auto frag = [&](unsigned at) { return *reinterpret_cast<const lds_u32x4*>((size_t)(base + at)); };
+    f32x4 sc[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) sc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds)                          // (four chains side by side)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) sc[s] = P::mfma(frag((unsigned)(s * DS + ds) * 1024u), bq[ds], sc[s]);
+    u32x4 av[2][DT];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) av[c][dt] = frag(HALF + (unsigned)(c * DT + dt) * 1024u);
+    // sc[2 c + s][r]: key k0 + 32 c + 8 gq + 4 s + r.  Visible keys of this lane's eight of each tile, as in tree_attn1_kernel
+    unsigned vbits[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int bfirst = k0 + 32 * c + gq * 8 - prefix;
+      vbits[c] = 0xffu;
+      if (k0 + 32 * c + 32 > prefix && bfirst > -8) {
+        const int neg = max(-bfirst, 0);
+        unsigned v;
+        if (mask_bits) {
+          const int lo = max(bfirst, 0), wi = lo >> 6, sh = lo & 63;
+          const unsigned long long* mrow = mask_bits + (long)t * mask_words;
+          const unsigned long long w0 = mrow[min(wi, mask_words - 1)], w1 = mrow[min(wi + 1, mask_words - 1)];
+          unsigned long long x = w0 >> sh;
+          if (sh) x |= w1 << (64 - sh);
+          v = (unsigned)x & 0xffu;
+        } else {
+          const int n = min(max(t - max(bfirst, 0) + 1, 0), 8);
+          v = (1u << n) - 1u;
+        }
+        vbits[c] = ((v << neg) | ((1u << neg) - 1u)) & 0xffu;
+      }
+    }
+    float pv[16], tmax = NEG_BIG;
+    const bool whole = k0 + 64 <= k_hi && __ballot((vbits[0] & vbits[1]) != 0xffu) == 0;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) pv[e] = sc[e >> 2][e & 3] * scale2;
+    if (!whole) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const bool vis = row_ok && k0 + 32 * (e >> 3) + gq * 8 + (e & 7) < k_hi && ((vbits[e >> 3] >> (e & 7)) & 1u);
+        pv[e] = vis ? pv[e] : -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, pv[e]);
+    const float m_new = fmaxf(m, quad_max(tmax)), alpha = __builtin_amdgcn_exp2f(m - m_new);
+    float psum[2] = {0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 16; ++e) { pv[e] = __builtin_amdgcn_exp2f(pv[e] - m_new); psum[e >> 3] += pv[e]; }
+    u32x4 pb[2];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) pb[e >> 2][e & 3] = pack2<P>(pv[2 * e], pv[2 * e + 1]);
+    l = l * alpha + (psum[0] + psum[1]);
+    m = m_new;
+    if (__ballot(alpha != 1.f)) {                            // a row's maximum moved
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] = P::mfma(av[c][dt], pb[c], o[dt]);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");            // nothing of this wave may be writing LDS any more, and no wave reads it
+  __builtin_amdgcn_s_barrier();
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  u32x2 d[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) d[dt] = u32x2{pack2<P>(o[dt][0] * inv, o[dt][1] * inv), pack2<P>(o[dt][2] * inv, o[dt][3] * inv)};
+  tile_rows_out<8, DT>(lds0 + (unsigned)wv * TileRows<8, DT>::BYTES, d, [&](int r, int at, u32x4 b) {
+    const int rw = four * 64 + wv * 16 + r;
+    if (rw < nrows) *reinterpret_cast<u32x4*>(out + ((long)(rw / g) * Hq + h * g + rw % g) * D + at / 2) = b;
+  });
+}
+
 // merge the per-split partials: one wave per (t, hq) row
 template <typename P, int D>
 __global__ __launch_bounds__(256) void attn_combine_kernel(u16* __restrict__ out, const float* __restrict__ po,
@@ -560,12 +725,29 @@ extern "C" int umb_tree_attn2(void* out, const void* q, const void* k_cache, con
     single_max = one_env > 0 ? one_env : 1024;
     if (single_max < KBK) single_max = KBK;
   }
+  // More than 1024 query tiles: four waves a compute unit and more, which share their keys (us, a wave each / this: 1032 tiles 32.9 / 25.3, 1024 without a
+  // prefix 12.6 / 13.3, 768 14.1 / 16.5, 520 behind 700 keys 19.1 / 23.5)
+  static const int nw_env = getenv("UMB_ATTN_NW") ? atoi(getenv("UMB_ATTN_NW")) : 0;
+  if (Hkv * nqt > 1024 && !nw_env && !no_single && !out_fm_tt && ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)vt_cache | (uintptr_t)out) % 16 == 0) {
+    const dim3 grid(Hkv, (nrows + 63) / 64);
+    const int fold = (long)grid.x * grid.y <= 512;
+#define WIDE_(DD)                                                                                                                  \
+  hipLaunchKernelGGL((wide_attn_kernel<P, DD>), grid, dim3(256), 0, st, (const u16*)q, (const u16*)k_cache, (const u16*)vt_cache,   \
+                     prefix_len, T, Hq, Hkv, Lmax, mask_words, n_mask_keys, (const unsigned long long*)mask_bits, scale, (u16*)out, fold)
+    DISPATCH_DTYPE(dtype, {
+      if (D == 128) WIDE_(128);
+      else if (D == 64) WIDE_(64);
+      else WIDE_(32);
+    })
+#undef WIDE_
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
   const int spans = (Lmax + KBK - 1) / KBK;
   if ((counters || spans == 1) && nqt <= 65535 && spans <= max_splits && !no_single) {
     // Waves per (kv head, query tile): eight while the tiles are few (narrow trees: the keys of a tile are spread over
     // the waves and merged in LDS); with many tiles the chip is filled by tiles instead and a wave walks more keys,
     // so the per-block prologue and merge are paid 4x / 8x less often.
-    static const int nw_env = getenv("UMB_ATTN_NW") ? atoi(getenv("UMB_ATTN_NW")) : 0;
     const int nblk = Hkv * nqt;
     const int nw = nw_env ? nw_env : nblk >= 1792 ? 1 : nblk >= 512 ? 2 : 8;   // fragment-ordered cache: T = 505 (2024 pairs) 31.8 (1) vs 35.1 (2) us, T = 385 (1544) 25.9 vs 24.4
     static const int nq_env = getenv("UMB_ATTN_NQ") ? atoi(getenv("UMB_ATTN_NQ")) : 0;

@@ -83,3 +83,39 @@ def test_attention_of_many_tiles(dtype, D, Hq, Hkv, T, prefix, spare):
                 bound = 1.1 * unit * (p @ vd.abs()) + 1.1 * unit * want.abs() + 1e-5
                 assert ((out[:T, a].double() - want).abs() <= bound).all()
         assert bool((out[T] == 3.0).all())
+
+
+# every count of 16-row tiles a wave (full, ragged, none), chunks of one token, whole and with a tail, heads that do not fill the eight XCDs
+@pytest.mark.parametrize("D,E,Hk,H", [(16, 16, 1, 3), (33, 24, 2, 2), (64, 40, 1, 2), (80, 16, 3, 3), (96, 130, 1, 1), (128, 128, 4, 8), (144, 20, 1, 2),
+                                      (208, 48, 1, 1), (256, 33, 1, 2)])
+def test_delta_chunks(D, E, Hk, H):
+    from umbrella_amd import _lib
+    lens, first = [64, 1, 63, 200, 129], [0, 7, 3, 0, 64]
+    T, B, Dp = sum(lens), len(lens), (D + 15) // 16 * 16
+    g = torch.Generator(device="cuda").manual_seed(D + E)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")                   # noqa: E731
+    ldqk = Hk * Dp + 8
+    q, k = (torch.nn.functional.normalize(rnd(T, Hk, D), dim=-1) for _ in range(2))
+    v, beta, lg, state = rnd(T, H, E), torch.rand(T, H, generator=g, device="cuda"), -0.2 * torch.rand(T, H, generator=g, device="cuda"), rnd(B, H, D, E)
+    qd, kd = torch.full((2, T, ldqk), 5.0, device="cuda")
+    for dst, src in ((qd, q), (kd, k)):
+        dst[:, :Hk * Dp] = torch.nn.functional.pad(src, (0, Dp - D)).reshape(T, Hk * Dp)
+    row0 = [sum(lens[:i]) for i in range(B)]
+    meta = [torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([2, 0, 4, 1, 3], row0, first, lens)]
+    got, out = state.clone(), torch.full((T + 1, H, E), 3.0, device="cuda")
+    scratch = torch.full((_lib.load_seq().umb_delta_scan_floats(T, H, D, E),), 6.0, device="cuda")
+    _lib.seq_call("umb_delta_scan", out, got, qd, kd, ldqk, v, beta, lg, *meta, T, B, max(lens), Hk, H, D, E, scratch, scratch.numel())
+    for b, slot in enumerate([2, 0, 4, 1, 3]):
+        S = torch.zeros(H, D, E, dtype=torch.float64, device="cuda") if first[b] == 0 else state[slot].double()
+        want = torch.empty(lens[b], H, E, dtype=torch.float64, device="cuda")
+        for i in range(lens[b]):
+            t = row0[b] + i
+            qt, kt = (z[t].double().repeat_interleave(H // Hk, dim=0) for z in (q, k))
+            S = S * lg[t].double().exp()[:, None, None]
+            u = beta[t].double()[:, None] * (v[t].double() - (S * kt[:, :, None]).sum(1))
+            S = S + kt[:, :, None] * u[:, None, :]
+            want[i] = (S * qt[:, :, None]).sum(1)
+        # sums of D + 64 products of 32-bit numbers through a triangular system of unit keys
+        bound = 3e-5
+        assert (out[row0[b]:row0[b] + lens[b]] - want).norm() <= bound * want.norm() and (got[slot] - S).norm() <= bound * S.norm()
+    assert bool((out[T] == 3.0).all())

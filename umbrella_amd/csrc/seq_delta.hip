@@ -259,30 +259,66 @@ __device__ __forceinline__ f32x4 mma4(f32x4 a, f32x4 b, f32x4 c) {
   return c;
 }
 
-// (1) grid (chunks, value heads, sequences)
-__global__ __launch_bounds__(256) void delta_chunk_solve_kernel(DeltaChunk a) {
+// (1) grid (chunks, value heads, sequences).  One chunk is a chain: prefix sums, k . k, four inverses, sixteen solves.  Eight waves, K alone in
+// LDS and two workgroups a unit: q . k, which nothing waits for, is read from memory and runs beside the inverses.  Every load that depends on
+// nothing but the chunk leaves long before its use, NK (>= Dp / 16) of a kind at once: k, the wave's part of q and the decays at the start, its
+// values before the inverses.  In loops of In loops of a run-time count they came one by one, a round trip each.
+// 2466 tokens in five stretches, 16 heads of 128: 73 us -> 44; 61 tokens, 32 heads 25 -> 16.
+template <int NK>
+__global__ __launch_bounds__(512, NK <= 8 ? 4 : 2) void delta_chunk_solve_kernel(DeltaChunk a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int b = blockIdx.z, h = blockIdx.y, t0 = blockIdx.x * DC_Q, len = a.seq_len[b];
   if (t0 >= len) return;
   const int cnt = len - t0 < DC_Q ? len - t0 : DC_Q, H = a.H, Dp = a.Dp, LK = Dp + 4, hk = h / (H / a.Hk);
   const long row0 = (long)a.seq_row0[b] + t0;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   double* cum = reinterpret_cast<double*>(sm);   // [64]
   float* be = sm + 128;                          // [64] beta (0 past the stretch)
   float* ecs = be + 64;                          // [64] e^(c_t)
   float* As = ecs + 64;                          // [64][68]: -A
   float* Td = As + 64 * 68;                      // [4][16][20]: inverses of the diagonal blocks of I + A
   float* Ks = Td + 4 * 16 * 20;                  // [64][LK]
-  float* Qs = Ks + 64 * LK;                      // [64][LK]
+  const int nk = Dp >> 4, nt = nk + (a.Ep >> 4), dq = Dp >> 2;
+  f32x4 kv[(NK + 1) / 2], qv[NK], V[4];
+#pragma unroll
+  for (int i = 0; i < (NK + 1) / 2; ++i) {       // quad x of the chunk: row x / dq
+    const int x = min(tid + 512 * i, 64 * dq - 1), r = x / dq;
+    kv[i] = *reinterpret_cast<const f32x4*>(a.k + (row0 + min(r, cnt - 1)) * a.ldqk + (long)hk * Dp + (x - r * dq) * 4);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const long at = (row0 + min(lane, cnt - 1)) * H + h;
+  const float lg = a.lg[at], bt = a.beta[at];
+  // row tiles of the wave's first tile of q . k, and the values of its first solve for them (from tile nk on)
+  const int vt = wave < nk ? wave + (nk - wave + 7) / 8 * 8 : wave;
+  auto pair_row = [](int id) { return id < 1 ? 0 : (id < 3 ? 1 : (id < 6 ? 2 : 3)); };
+  auto load_q = [&](int id) __attribute__((always_inline)) {
+    const float* p = a.q + (row0 + min(16 * pair_row(id) + j, cnt - 1)) * a.ldqk + (long)hk * Dp + 4 * g;
+#pragma unroll
+    for (int i = 0; i < NK; ++i) qv[i] = *reinterpret_cast<const f32x4*>(p + 16 * min(i, nk - 1));
+  };
+  auto load_v = [&](int tile) __attribute__((always_inline)) {
+    const float* v = a.v + (row0 * H + h) * a.E + min(16 * (tile - nk) + j, a.E - 1);
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) V[rb][r] = v[(long)min(16 * rb + 4 * g + r, cnt - 1) * H * a.E];
+  };
+  load_q(wave ^ 4);
+#pragma unroll
+  for (int i = 0; i < (NK + 1) / 2; ++i) {
+    const int x = tid + 512 * i, r = x / dq;
+    if (x < 64 * dq) *reinterpret_cast<f32x4*>(Ks + r * LK + (x - r * dq) * 4) = r < cnt ? kv[i] : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   if (wave == 0) {
-    double v = lane < cnt ? (double)a.lg[(row0 + lane) * H + h] : 0.0;
+    double v = lane < cnt ? (double)lg : 0.0;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const double u = __shfl_up(v, o, 64);
       if (lane >= o) v += u;
     }
     cum[lane] = v;
-    be[lane] = lane < cnt ? a.beta[(row0 + lane) * H + h] : 0.f;
+    be[lane] = lane < cnt ? bt : 0.f;
     const float e = expf((float)v), w = expf((float)(__shfl(v, 63, 64) - v));
     ecs[lane] = e;
     if (lane < cnt) {
@@ -290,38 +326,40 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(DeltaChunk a) {
       a.ew[(long)h * a.T + row0 + lane] = w;
     }
   }
-  const int dq = Dp >> 2;
-  for (int x = tid; x < 64 * dq; x += 256) {
-    const int s = x / dq, d = (x - s * dq) * 4;
-    f32x4 kv = f32x4{0.f, 0.f, 0.f, 0.f}, qv = kv;
-    if (s < cnt) {
-      kv = *reinterpret_cast<const f32x4*>(a.k + (row0 + s) * a.ldqk + (long)hk * Dp + d);
-      qv = *reinterpret_cast<const f32x4*>(a.q + (row0 + s) * a.ldqk + (long)hk * Dp + d);
-    }
-    *reinterpret_cast<f32x4*>(Ks + s * LK + d) = kv;
-    *reinterpret_cast<f32x4*>(Qs + s * LK + d) = qv;
-  }
   __syncthreads();
-  // k . k and q . k, the ten 16 x 16 tiles on and below the diagonal of each
-  for (int id = wave; id < 20; id += 4) {
-    const int pair = id < 10 ? id : id - 10;
-    const int rb = pair < 1 ? 0 : (pair < 3 ? 1 : (pair < 6 ? 2 : 3)), cb = pair - rb * (rb + 1) / 2;
-    const float* X = (id < 10 ? Ks : Qs) + (16 * rb + j) * LK + 4 * g;
+  // the ten 16 x 16 tiles on and below the diagonal of k . k and, with row t of q past the stretch its last one, of q . k
+  auto pair = [&](int id, auto of_q) __attribute__((always_inline)) {
+    constexpr bool QK = decltype(of_q)::value;
+    const int rb = pair_row(id), cb = id - rb * (rb + 1) / 2;
     const float* Y = Ks + (16 * cb + j) * LK + 4 * g;
+    const float* X = Ks + (16 * rb + j) * LK + 4 * g;
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < Dp; k0 += 16) acc = mma4(*reinterpret_cast<const f32x4*>(X + k0), *reinterpret_cast<const f32x4*>(Y + k0), acc);
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const f32x4 y = *reinterpret_cast<const f32x4*>(Y + 16 * min(i, nk - 1)), x = QK ? qv[i] : *reinterpret_cast<const f32x4*>(X + 16 * min(i, nk - 1));
+      if (i < nk) acc = mma4(x, y, acc);
+    }
     const int s = 16 * cb + j;
     const double cs = cum[s];
+    float e[4], bt4[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 16 * rb + 4 * g + r;
-      const float e = s <= t ? expf((float)(cum[t] - cs)) : 0.f;
-      if (id < 10) As[t * 68 + s] = s < t ? -be[t] * e * acc[r] : 0.f;
-      else if (t < cnt) a.m[((row0 + t) * H + h) * 64 + s] = e * acc[r];
+      e[r] = expf((float)(cum[t] - cs));
+      bt4[r] = be[t];
     }
-  }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = 16 * rb + 4 * g + r;
+      if (!QK) As[t * 68 + s] = s < t ? -bt4[r] * e[r] * acc[r] : 0.f;
+      else if (t < cnt) a.m[((row0 + t) * H + h) * 64 + s] = s <= t ? e[r] * acc[r] : 0.f;
+    }
+  };
+  for (int id = wave; id < 10; id += 8) pair(id, std::false_type{});
   __syncthreads();
-  {                                              // wave w inverts diagonal block w: lane = column, rows one after another
+  if (vt < nt) load_v(vt);
+  __builtin_amdgcn_sched_barrier(0);
+  if (wave < 4) {                                // wave w inverts diagonal block w: lane = column, rows one after another
     float x[16];
     const float* Ab = As + (16 * wave) * 68 + 16 * wave;
 #pragma unroll
@@ -335,23 +373,32 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(DeltaChunk a) {
       for (int t = 0; t < 16; ++t) Td[(wave * 16 + t) * 20 + j] = x[t];
     }
   }
+  pair(wave ^ 4, std::true_type{});
+  if ((wave ^ 4) < 2) {
+    load_q((wave ^ 4) + 8);
+    pair((wave ^ 4) + 8, std::true_type{});
+  }
   __syncthreads();
-  const int nk = Dp >> 4, nt = nk + (a.Ep >> 4);
-  for (int tile = wave; tile < nt; tile += 4) {
+  for (int tile = wave; tile < nt; tile += 8) {
+    asm volatile("" ::: "memory");               // (A and the inverses are read again for each tile: fourteen quads would be held otherwise)
     const bool isW = tile < nk;
     const int col = 16 * (isW ? tile : tile - nk) + j;
     f32x4 U[4];
+    if (isW) {
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) U[rb][r] = ecs[16 * rb + 4 * g + r] * Ks[(16 * rb + 4 * g + r) * LK + col];
+    } else {
+      if (tile != vt) load_v(tile);
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) U[rb][r] = 16 * rb + 4 * g + r < cnt && col < a.E ? V[rb][r] : 0.f;
+    }
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
-      f32x4 acc;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * rb + 4 * g + r;
-        float x;
-        if (isW) x = ecs[t] * Ks[t * LK + col];
-        else x = (t < cnt && col < a.E) ? a.v[((row0 + t) * H + h) * a.E + col] : 0.f;
-        acc[r] = be[t] * x;
-      }
+      f32x4 acc = U[rb] * *reinterpret_cast<const f32x4*>(be + 16 * rb + 4 * g);
 #pragma unroll
       for (int cb = 0; cb < rb; ++cb) acc = mma4(*reinterpret_cast<const f32x4*>(As + (16 * rb + j) * 68 + 16 * cb + 4 * g), U[cb], acc);
       U[rb] = mma4(*reinterpret_cast<const f32x4*>(Td + (rb * 16 + j) * 20 + 4 * g), acc, f32x4{0.f, 0.f, 0.f, 0.f});
@@ -368,98 +415,141 @@ __global__ __launch_bounds__(256) void delta_chunk_solve_kernel(DeltaChunk a) {
   }
 }
 
-// (2) grid (16-column slices, value heads, sequences).  Wave w keeps TPW 16-row tiles of the state slice (from tile w TPW) as
+// (2) a workgroup per 16-column slice of a (value head, sequence).  Wave w keeps TPW 16-row tiles of the state slice (rows 16 TPW w ..) as
 // accumulators; the waves' shares of Wk S and Q S meet in LDS; wave w owns read-out rows 16 w .. of the chunk.
-template <int TPW> struct DeltaFrag {
-  f32x4 wk[4][TPW], q[4][TPW], kt[4][TPW], m[4], uv[4], ew[4], ec;
-  float eq;
-};
-
-template <int TPW, bool PRE>
-__global__ __launch_bounds__(256) void delta_chunk_scan_kernel(float* __restrict__ o, float* __restrict__ state, DeltaChunk a) {
-  extern __shared__ __attribute__((aligned(16))) float red[];        // [2][4 waves][8 tiles][256]
-  const int b = blockIdx.z, h = blockIdx.y, H = a.H, Dp = a.Dp, D = a.D, E = a.E;
+//   * A chunk's operands stay in ONE set of registers: Wk and Q of the next chunk are asked for once its products have taken them (they
+//     arrive beside the read-out), the rest at the end (they arrive beside the next chunk's first products).  With two whole sets the kernel held
+//     one wave a SIMD; it is a chain of loads, products and an exchange, and two of them fill each other's waits.
+//   * The slices of a head read the same Wk, Q, K and M: they run on one XCD and share its L2 (dealt out by blockIdx they each missed in
+//     another one).
+//     2466 tokens in five stretches, 16 heads of 128, both together: 133 us -> 94.
+//   * IL (the waves' tiles are all of D): row p of tile x is state row TPW p + x of the wave's, so a lane's Wk and Q are TPW quads of one line and its K^T one load of TPW.
+template <int TPW, bool IL>
+__global__ __launch_bounds__(256, TPW <= 2 ? 2 : 1) void delta_chunk_scan_kernel(float* __restrict__ o, float* __restrict__ state, DeltaChunk a, int slices,
+                                                                                 int items) {
+  extern __shared__ __attribute__((aligned(16))) float red[];        // [2][4 waves][8 tiles][256], [2][2][64]
+  const int turn = blockIdx.x >> 3, slice = turn % slices, item = turn / slices * 8 + (blockIdx.x & 7);
+  if (item >= items) return;
+  const int b = item / a.H, h = item - b * a.H, H = a.H, Dp = a.Dp, D = a.D, E = a.E;
   const int n = a.seq_len[b];
   if (n <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, g = lane >> 4, hk = h / (H / a.Hk);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);         // uniform: what depends on it stays in scalar registers
-  const int col = blockIdx.x * 16 + j;
+  const int col = slice * 16 + j;
   const bool c_ok = col < E;
   const long row0 = a.seq_row0[b];
   float* sp = state + (((long)a.seq_slot[b] * H + h) * D) * E + (c_ok ? col : 0);
   const bool fresh = a.seq_pos0[b] == 0;
+  auto row_of = [&](int x, int p) { return IL ? 16 * wave * TPW + TPW * p + x : 16 * (wave * TPW + x) + p; };
   f32x4 S[TPW];
 #pragma unroll
   for (int x = 0; x < TPW; ++x)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int d = 16 * (wave * TPW + x) + 4 * g + r;
+      const int d = row_of(x, 4 * g + r);
       S[x][r] = (!fresh && c_ok && d < D) ? sp[(long)d * E] : 0.f;
     }
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
   const int nch = (n + DC_Q - 1) / DC_Q;
   const int ldw = H * Dp, ldu = H * a.Ep, ldm = H * 64, ldk = a.ldqk;
+  typedef float part __attribute__((ext_vector_type(TPW)));
+  part kt_[4][4];
+  f32x4 wk_[4][TPW], q_[4][TPW], m_[4], uv_[4];
+  float decay_, eq_;
   // The operands of a chunk.  Every load is unconditional: a row past the stretch reads the last row instead, and what it brings
-  // has no effect -- its weight ew is 0, M is 0 above the diagonal, its read-out is not stored.  In a full chunk the row of lane
-  // (j, g) is its lane part plus a uniform part, so an address is a scalar base and one of a few lane offsets.
-  auto load = [&](int ch, DeltaFrag<TPW>& f) {
+  // has no effect -- its weight is taken as 0, M is 0 above the diagonal, its read-out is not stored.  Nothing is done to a value where it
+  // is loaded: that would be a wait for it.  In a full chunk the row of lane (j, g) is its lane part plus a uniform part, so an address is a
+  // scalar base and one of five lane offsets; a stretch's last chunk, and rows too far apart for those, go row by row.
+  auto in_dp = [&](int x) { return IL || 16 * (wave * TPW + x) < Dp; };       // uniform; a tile that is not reads the last one
+  auto tile_at = [&](int x) { return IL ? 0 : min(16 * (wave * TPW + x), Dp - 16) - 16 * wave * TPW; };
+  const bool near = ldk < (1 << 24) && ldu < (1 << 24);
+  const unsigned jw = (unsigned)(j * ldw + (IL ? 4 * TPW : 4) * g) * 4u, jk = (unsigned)(j * ldk + (IL ? 4 * TPW : 4) * g) * 4u, jm = (unsigned)(j * ldm + 4 * g) * 4u;
+  const unsigned gk = (unsigned)(4 * g * ldk + (IL ? TPW : 1) * j) * 4u, gu = (unsigned)(4 * g * ldu + j) * 4u;
+  // rows u + j / rows u + 4 g + r of an operand at p
+  auto at_j = [&](auto full, int cnt, const float* p, int ld, int u, unsigned lane_off, int quad) __attribute__((always_inline)) {
+    return full ? reinterpret_cast<const float*>(reinterpret_cast<const char*>(p + (long)u * ld) + lane_off) : p + (long)min(u + j, cnt - 1) * ld + quad * g;
+  };
+  auto at_g = [&](auto full, int cnt, const float* p, int ld, int u, unsigned lane_off, int per) __attribute__((always_inline)) {
+    return full ? reinterpret_cast<const float*>(reinterpret_cast<const char*>(p + (long)u * ld) + lane_off) : p + (long)min(u + 4 * g, cnt - 1) * ld + per * j;
+  };
+  auto load_first = [&](int ch) __attribute__((always_inline)) {              // the decays, Wk and Q
     const int cnt = n - ch * DC_Q < DC_Q ? n - ch * DC_Q : DC_Q;
-    const long base = row0 + (long)ch * DC_Q;
-    const float* wk = a.wk + base * ldw + (long)h * Dp + 16 * wave * TPW;
-    const float* q = a.q + base * ldk + (long)hk * Dp + 16 * wave * TPW;
-    const float* k = a.k + base * ldk + (long)hk * Dp + 16 * wave * TPW;
-    const float* uv = a.uv + base * ldu + (long)h * a.Ep + blockIdx.x * 16;
-    const float* m = a.m + base * ldm + (long)h * 64;
+    int base = (int)row0 + ch * DC_Q;
+    asm volatile("" : "+s"(base));             // (or every load's address is kept and stepped on in registers of its own)
+    const float* wk = a.wk + (long)base * ldw + (long)h * Dp + 16 * wave * TPW;
+    const float* q = a.q + (long)base * ldk + (long)hk * Dp + 16 * wave * TPW;
     const float* ec = a.ec + (long)h * a.T + base;
     const float* ew = a.ew + (long)h * a.T + base;
-    auto fill = [&](auto full) {
-      // row of an operand whose lanes run over rows (u + j) / over groups of four rows (u + 4 g + r): uniform and lane part
-      auto at_j = [&](const float* p, int ld, int u) {
-        return full ? p + u * ld + (unsigned)(j * ld) : p + (unsigned)((u + j < cnt ? u + j : cnt - 1) * ld);
-      };
-      auto at_g = [&](const float* p, int ld, int u) {
-        return full ? p + u * ld + (unsigned)(4 * g * ld) : p + (unsigned)((u + 4 * g < cnt ? u + 4 * g : cnt - 1) * ld);
-      };
+    decay_ = (wave == 0 ? ec : ew)[min(lane, cnt - 1)];        // waves 0 and 1 hand these to all
+    eq_ = ec[cnt - 1];
+    auto fill = [&](auto full) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int x = 0; x < TPW; ++x) {
-          if (16 * (wave * TPW + x) < Dp) {                          // uniform
-            f.wk[i][x] = *reinterpret_cast<const f32x4*>(at_j(wk + 16 * x, ldw, 16 * i) + 4 * g);
-            f.q[i][x] = *reinterpret_cast<const f32x4*>(at_j(q + 16 * x, ldk, 16 * i) + 4 * g);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) f.kt[i][x][r] = at_g(k + 16 * x, ldk, 16 * i + r)[j];
-          } else {
-            f.wk[i][x] = f.q[i][x] = f.kt[i][x] = zero;
-          }
+          wk_[i][x] = *reinterpret_cast<const f32x4*>(at_j(full, cnt, wk + tile_at(x) + (IL ? 4 * x : 0), ldw, 16 * i, jw, IL ? 4 * TPW : 4));
+          q_[i][x] = *reinterpret_cast<const f32x4*>(at_j(full, cnt, q + tile_at(x) + (IL ? 4 * x : 0), ldk, 16 * i, jk, IL ? 4 * TPW : 4));
         }
+    };
+    if (cnt == DC_Q && near) fill(std::true_type{});
+    else fill(std::false_type{});
+  };
+  auto load_rest = [&](int ch) __attribute__((always_inline)) {               // Uv, M and K^T
+    const int cnt = n - ch * DC_Q < DC_Q ? n - ch * DC_Q : DC_Q;
+    int base = (int)row0 + ch * DC_Q;
+    asm volatile("" : "+s"(base));
+    const float* k = a.k + (long)base * ldk + (long)hk * Dp + 16 * wave * TPW;
+    const float* uv = a.uv + (long)base * ldu + (long)h * a.Ep + slice * 16;
+    const float* m = a.m + (long)base * ldm + (long)h * 64;
+    auto fill = [&](auto full) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) uv_[i][r] = *at_g(full, cnt, uv, ldu, 16 * i + r, gu, 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m_[i] = *reinterpret_cast<const f32x4*>(at_j(full, cnt, m + 16 * min(i, wave), ldm, 16 * wave, jm, 4));    // (i > wave: not used)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          f.uv[i][r] = at_g(uv, ldu, 16 * i + r)[j];
-          f.ew[i][r] = at_g(ew, 1, 16 * i + r)[0];
-          if (!full && 16 * i + 4 * g + r >= cnt) f.ew[i][r] = 0.f;
-        }
-        if (i <= wave) f.m[i] = *reinterpret_cast<const f32x4*>(at_j(m + 16 * i, ldm, 16 * wave) + 4 * g);
-        else f.m[i] = zero;
-      }
+          if constexpr (IL) {
+            kt_[i][r] = *reinterpret_cast<const part*>(at_g(full, cnt, k, ldk, 16 * i + r, gk, TPW));
+          } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) f.ec[r] = at_g(ec, 1, 16 * wave + r)[0];
+            for (int x = 0; x < TPW; ++x) kt_[i][r][x] = *at_g(full, cnt, k + tile_at(x), ldk, 16 * i + r, gk, 1);
+          }
+        }
     };
-    if (cnt == DC_Q) fill(std::true_type{});
+    if (cnt == DC_Q && near) fill(std::true_type{});
     else fill(std::false_type{});
-    f.eq = ec[cnt - 1];
   };
-  auto compute = [&](int ch, const DeltaFrag<TPW>& f) {
+  load_first(0);
+  __builtin_amdgcn_sched_barrier(0);             // in this order, as the loop asks for them: a wait then leaves the younger ones in flight
+  load_rest(0);
+  for (int ch = 0;; ++ch) {
     const int cnt = n - ch * DC_Q < DC_Q ? n - ch * DC_Q : DC_Q;
     float* rb = red + (ch & 1) * (4 * 8 * 256);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       f32x4 w = zero, q = zero;
 #pragma unroll
-      for (int x = 0; x < TPW; ++x) { w = mma4(f.wk[i][x], S[x], w); q = mma4(f.q[i][x], S[x], q); }
+      for (int x = 0; x < TPW; ++x) {
+        if (!in_dp(x)) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {                                // IL: the quads are those of the line
+          const int y = IL ? (TPW * r + x) / 4 : x, e = IL ? (TPW * r + x) % 4 : r;
+          w = __builtin_amdgcn_mfma_f32_16x16x4f32(wk_[i][y][e], S[x][r], w, 0, 0, 0);
+          q = __builtin_amdgcn_mfma_f32_16x16x4f32(q_[i][y][e], S[x][r], q, 0, 0, 0);
+        }
+      }
       *reinterpret_cast<f32x4*>(rb + (wave * 8 + i) * 256 + lane * 4) = w;
       *reinterpret_cast<f32x4*>(rb + (wave * 8 + 4 + i) * 256 + lane * 4) = q;
     }
+    float* dec = red + 2 * (4 * 8 * 256) + (ch & 1) * 128;           // e^(c_t), e^(c_end - c_t) and 0 behind the stretch
+    if (wave < 2) dec[tid] = wave == 0 || lane < cnt ? decay_ : 0.f;
+    const float eq = eq_;
+    load_first(min(ch + 1, nch - 1));            // (on every path, for the same reason)
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     f32x4 U[4], out = zero;
 #pragma unroll
@@ -467,58 +557,49 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(float* __restrict
       f32x4 s = *reinterpret_cast<const f32x4*>(rb + i * 256 + lane * 4);
 #pragma unroll
       for (int w = 1; w < 4; ++w) s += *reinterpret_cast<const f32x4*>(rb + (w * 8 + i) * 256 + lane * 4);
-      U[i] = f.uv[i] - s;
+      U[i] = uv_[i] - s;
     }
 #pragma unroll
     for (int w = 0; w < 4; ++w) out += *reinterpret_cast<const f32x4*>(rb + (w * 8 + 4 + wave) * 256 + lane * 4);
-    out *= f.ec;
+    out *= *reinterpret_cast<const f32x4*>(dec + 16 * wave + 4 * g);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (i <= wave) out = mma4(f.m[i], U[i], out);
+      if (i <= wave) out = mma4(m_[i], U[i], out);
 #pragma unroll
-    for (int x = 0; x < TPW; ++x) S[x] *= f.eq;
+    for (int x = 0; x < TPW; ++x) S[x] *= eq;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const f32x4 ue = U[i] * f.ew[i];
+      const f32x4 ue = U[i] * *reinterpret_cast<const f32x4*>(dec + 64 + 16 * i + 4 * g);
 #pragma unroll
-      for (int x = 0; x < TPW; ++x) S[x] = mma4(f.kt[i][x], ue, S[x]);
+      for (int x = 0; x < TPW; ++x) {
+        if (!in_dp(x)) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt_[i][r][x], ue[r], S[x], 0, 0, 0);
+      }
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 16 * wave + 4 * g + r;
       if (t < cnt && c_ok) o[((row0 + (long)ch * DC_Q + t) * H + h) * E + col] = out[r];
     }
-  };
-  if constexpr (PRE) {                           // the next chunk's operands are in flight while a chunk is worked on
-    DeltaFrag<TPW> f0, f1;
-    load(0, f0);
-    for (int ch = 0; ch < nch; ch += 2) {
-      if (ch + 1 < nch) load(ch + 1, f1);
-      compute(ch, f0);
-      if (ch + 1 < nch) {
-        if (ch + 2 < nch) load(ch + 2, f0);
-        compute(ch + 1, f1);
-      }
-    }
-  } else {
-    for (int ch = 0; ch < nch; ++ch) {
-      DeltaFrag<TPW> f;
-      load(ch, f);
-      compute(ch, f);
-    }
+    if (ch + 1 == nch) break;
+    __builtin_amdgcn_sched_barrier(0);
+    load_rest(ch + 1);
   }
+  int g_out = g;
+  asm volatile("" : "+v"(g_out));                // (or these addresses are kept from the loads in front on)
 #pragma unroll
   for (int x = 0; x < TPW; ++x)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int d = 16 * (wave * TPW + x) + 4 * g + r;
+      const int d = row_of(x, 4 * g_out + r);
       if (c_ok && d < D) sp[(long)d * E] = S[x][r];
     }
 }
 
 static inline int up16(int n) { return (n + 15) & ~15; }
 static inline size_t delta_solve_lds(int Dp) {
-  return ((size_t)128 + 64 + 64 + 64 * 68 + 4 * 16 * 20 + 2 * 64 * (size_t)(Dp + 4)) * sizeof(float);
+  return ((size_t)128 + 64 + 64 + 64 * 68 + 4 * 16 * 20 + 64 * (size_t)(Dp + 4)) * sizeof(float);
 }
 static inline bool delta_in_ok(const float* proj, int ld, int col0, const void* conv_w, const float* ring, const float* dt_bias,
                                const float* a_log, int T, int Hk, int H, int D, int E, int taps) {
@@ -606,16 +687,28 @@ extern "C" int umb_delta_scan(float* o, float* state, const float* q, const floa
   float* uv = m + n * 64;
   float* ec = uv + n * Ep;
   DeltaChunk a{q, k, v, beta, log_g, wk, uv, m, ec, ec + n, T, ldqk, Hk, H, D, Dp, E, Ep, seq_slot, seq_row0, seq_pos0, seq_len};
-  const size_t lds1 = delta_solve_lds(Dp), lds2 = (size_t)2 * 4 * 8 * 256 * sizeof(float);
-  if (ensure_dynamic_lds<delta_chunk_solve_kernel>(lds1) != UMB_OK) return UMB_EHIP;
-  hipLaunchKernelGGL(delta_chunk_solve_kernel, dim3((max_len + DC_Q - 1) / DC_Q, H, B), dim3(256), lds1, st, a);
-#define DELTA_SCAN(TPW, PRE)                                                                                              \
+  const size_t lds1 = delta_solve_lds(Dp), lds2 = (size_t)(2 * 4 * 8 * 256 + 2 * 2 * 64) * sizeof(float);
+#define DELTA_SOLVE(NK)                                                                                                   \
   do {                                                                                                                    \
-    if (ensure_dynamic_lds<delta_chunk_scan_kernel<TPW, PRE>>(lds2) != UMB_OK) return UMB_EHIP;                           \
-    hipLaunchKernelGGL((delta_chunk_scan_kernel<TPW, PRE>), dim3(Ep / 16, H, B), dim3(256), lds2, st, o, state, a);       \
+    if (ensure_dynamic_lds<delta_chunk_solve_kernel<NK>>(lds1) != UMB_OK) return UMB_EHIP;                                \
+    hipLaunchKernelGGL(delta_chunk_solve_kernel<NK>, dim3((max_len + DC_Q - 1) / DC_Q, H, B), dim3(512), lds1, st, a);    \
   } while (0)
-  if (Dp <= 64) DELTA_SCAN(1, true);
-  else if (Dp <= 128) DELTA_SCAN(2, true);
+  if (Dp <= 32) DELTA_SOLVE(2);
+  else if (Dp <= 64) DELTA_SOLVE(4);
+  else if (Dp <= 128) DELTA_SOLVE(8);
+  else DELTA_SOLVE(16);
+#undef DELTA_SOLVE
+  const long items = (long)H * B, blocks = (items + 7) / 8 * 8 * (Ep / 16);
+  if (blocks > 0x7fffffffL) return UMB_EINVAL;
+#define DELTA_SCAN(TPW, IL)                                                                                               \
+  do {                                                                                                                    \
+    if (ensure_dynamic_lds<delta_chunk_scan_kernel<TPW, IL>>(lds2) != UMB_OK) return UMB_EHIP;                            \
+    hipLaunchKernelGGL((delta_chunk_scan_kernel<TPW, IL>), dim3((unsigned)blocks), dim3(256), lds2, st, o, state, a, Ep / 16, (int)items); \
+  } while (0)
+  if (Dp <= 64) DELTA_SCAN(1, false);
+  else if (Dp == 128) DELTA_SCAN(2, true);
+  else if (Dp < 128) DELTA_SCAN(2, false);
+  else if (Dp == 256) DELTA_SCAN(4, true);
   else DELTA_SCAN(4, false);
 #undef DELTA_SCAN
   UMB_LAUNCH_CHECK();

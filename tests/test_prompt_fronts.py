@@ -119,3 +119,43 @@ def test_delta_chunks(D, E, Hk, H):
         bound = 3e-5
         assert (out[row0[b]:row0[b] + lens[b]] - want).norm() <= bound * want.norm() and (got[slot] - S).norm() <= bound * S.norm()
     assert bool((out[T] == 3.0).all())
+
+
+# the rows of a step come from several pages, whole and cut anywhere: what the cache's page size is must not show
+@pytest.mark.parametrize("D,E,maps,keep,chunk", [(128, 128, 1, 0, 0), (72, 48, 1, 37, 0), (64, 128, 2, 0, 61), (24, 16, 1, 3, 0), (256, 208, 1, 0, 0)])
+def test_prompt_attention_of_any_page_size(D, E, maps, keep, chunk):
+    from umbrella_amd import _lib
+    from umbrella_amd.attn.cache import PagedSeqCache
+    lens, news, H, G, window, Dc, R = [201, 40, 131], [201, 1, 97], 4, 2, 90, E // 16 * 16, D // 8 * 8
+    T, dtype = sum(news), torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")                   # noqa: E731
+    keys, vals, lat = ([rnd(n, *s).to(dtype) for n in lens] for s in ((G, maps * D), (G, E), (Dc + R,)))
+    q, qa = rnd(T, H, maps, D), rnd(T, H, Dc + R)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")              # noqa: E731
+    row0, pos0, cnt = i32([sum(news[:b]) for b in range(3)]), i32([n - k for n, k in zip(lens, news)]), i32(news)
+    outs = []
+    for page in (16, 7, 1, 256):
+        c = PagedSeqCache([(G, maps * D, 0, E)], [], sum(lens) + 3 * page, 3, "cuda", dtype, page=page, latent_layers=(Dc + R,))
+        entries = []
+        for b, n in enumerate(lens):
+            c.open(b)
+            c.extend(b, n, entries)
+        c.write_pages(entries)
+        for b, n in enumerate(lens):
+            at = torch.arange(n, device="cuda")
+            pg = c.pages_dev[c.slot(b)].long()[at // page]
+            c.kv[0]["k"][pg, :, at % page] = keys[b]
+            c.kv[0]["v"][pg, :, at % page] = vals[b]
+            c.latent[0][pg, at % page] = lat[b]
+        slot = i32([c.slot(b) for b in range(3)])
+        out, lout = torch.full((T + 1, H * E), 3.0, dtype=dtype, device="cuda"), torch.full((T + 1, H * Dc), 3.0, dtype=dtype, device="cuda")
+        form = _lib.UmbAttnForm(maps, chunk, None, 0.3, 1e-3, keep, 0)
+        _lib.seq_call("umb_attn_attend_tiled", out, H * E, q, c.struct(0), None, 0, -1, None, 0, slot, row0, pos0, cnt, 3, max(news), H, G, D, E, window,
+                      D ** -0.5, 1.0, 0.0, form, _lib.seq_dtype_code(dtype))
+        _lib.seq_call("umb_lat_attend_tiled", lout, qa, c.latent_struct(0), None, slot, row0, pos0, cnt, 3, max(news), H, Dc, R, window, (Dc + R) ** -0.5,
+                      _lib.seq_dtype_code(dtype))
+        outs.append((out, lout))
+    assert bool((outs[0][0][T] == 3.0).all()) and bool((outs[0][1][T] == 3.0).all()) and bool(outs[0][0].isfinite().all())
+    for o in outs[1:]:
+        assert torch.equal(o[0], outs[0][0]) and torch.equal(o[1], outs[0][1])

@@ -28,6 +28,7 @@
 // the same token in another batch, or of a prompt cut elsewhere, agrees to fp32 rounding and not bit for bit.
 #include "seq_common.h"
 #include "seq_decode.h"
+#include "seq_rows.h"
 
 static inline bool bsa_kv_ok(const UmbPagedKV* kv) { return kv && kv->k && kv->v && kv->pages && kv->page >= 1 && kv->max_pages >= 1; }
 
@@ -807,18 +808,18 @@ extern "C" int umb_bsa_attend(void* out, int ldo, const float* q, const UmbPaged
 // ---- prompt attention on the matrix pipe (16-bit storage; D a multiple of 8, E a multiple of 16).
 // Workgroup = (16 consecutive positions of one sequence, one key/value head, four of its query heads), a wave per head.  The tile's
 // keys -- from the first position's window start to the last position -- are walked in steps of 32 by the whole workgroup: the
-// step's 32 cached key rows and value rows are staged ONCE into LDS (keys as cached: the A operand of
-// S^T = K Q^T; values transposed: the A operand of O^T += V^T P^T) and serve every head of the workgroup; the next step's rows
-// are in flight in registers while the current one is used.  Per step and head: two 16-key score tiles; the bias of the
-// lane's eight (query, key) pairs, fetched by distance before the products are issued; online softmax in fp32 with base-2
+// step's 32 cached key rows and value rows stand ONCE in LDS (seq_rows.h) and serve every head of the workgroup; the next step's
+// are on their way to a second buffer while the current one is used.  Per step and head: two 16-key score tiles; the bias of the
+// lane's eight (query, key) pairs, fetched by distance a step ahead; online softmax in fp32 with base-2
 // exponents, accumulators rescaled only when a maximum moved; the lane's eight weights ARE its share of the B operand of the
 // value product.  Scores and weights keep fp32 accuracy on the 16-bit pipe: the fp32 queries and the fp32 weights enter as
 // high + low 16-bit halves (two products each, 2^-17 relative).
 // Products per step at compile time: NSM steps of 32 features and NVM tiles of 16 columns, the least of a few sizes that hold D and E, with zeros
 // behind a key row's D columns.  With run-time counts every product stood in a block of its own behind its own LDS read; with a whole step's
-// reads free to move ahead, and steps that every query sees whole left untested, 1999 positions, 32 + 8 heads of 128 went from 212 us to 140, two
-// maps over 617 positions, 64 | 128, from 104 to 71.  FULL: D and E fill them, staging then tests nothing (2000 positions of 128: 158 us,
-// 162 without).  us, run-time / these counts, 2000 positions: heads of 96 86 / 75, of 112 242 / 202, of 256 216 / 156, two maps of 128 | 128 273 / 179.
+// reads free to move ahead, and steps that every query sees whole left untested, 1999 positions, 32 + 8 heads of 128 went from 212 us to 141, two
+// maps over 617 positions, 64 | 128, from 104 to 71; rows by LDS-DMA, transposed reads in place of 2-byte stores, one barrier a step and fragments read
+// ahead of their products: 117 and 59, two maps of 128 | 256 over 2000 positions 252 -> 182.
+// FULL: D and E fill them, staging then tests nothing (2000 positions of 128: 158 us, 162 without).  us, run-time / these counts, 2000 positions: heads of 96 86 / 75, of 112 242 / 202, of 256 216 / 156, two maps of 128 | 128 273 / 179.
 // Two heads a wave, sharing the value fragments, are behind wherever a launch is not several rounds of workgroups: 600 positions, 64 + 8 heads
 // of 128 67 against 55, of 64 42 / 35 (2000 positions 195 / 198, 134 / 121).
 constexpr float BSA_LOG2E = 1.4426950408889634f;
@@ -830,9 +831,10 @@ template <typename P> __device__ __forceinline__ void split2(float a, float b, u
 
 // MAPS rows per wave, the maps of its head; every map has its part of the staged key rows, the value fragments of a step serve both
 template <int NSM, int NVM, int MAPS> struct BsaTile {
-  static constexpr int KD = NSM * 32, LD = MAPS * KD + 8;       // a map's part of a staged key row; row stride: 16 bytes of padding spread the banks
-  static constexpr int LT = 36;                                 // row stride of the transposed value tile: 32 keys + 8 bytes of padding
-  static constexpr size_t LDS = ((size_t)32 * LD + (size_t)NVM * 16 * LT) * sizeof(u16);
+  typedef RowTile<4 * NSM * MAPS> Keys;                         // a map's part of a key row is NSM steps wide
+  typedef RowTile<2 * NVM> Values;
+  static constexpr unsigned STEP = Keys::BYTES + Values::BYTES;
+  static constexpr size_t LDS = 2 * STEP + 2 * 32 * sizeof(unsigned);
 };
 template <typename P, int NSM, int NVM, int MAPS, bool FULL>
 __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q,
@@ -846,12 +848,10 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
   typedef BsaTile<NSM, NVM, MAPS> Tile;
   if constexpr (FULL) { D = NSM * 32; E = NVM * 16; }
   constexpr int HPW = MAPS;                           // rows of scores per wave
-  constexpr int NLK = (NSM * 4 * MAPS + 7) / 8, NLV = (NVM * 2 + 7) / 8;     // 16-byte chunks of a key / value row per staging thread
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
-  constexpr int KD = Tile::KD, LD = Tile::LD, LT = Tile::LT;
-  const int DK = MAPS * D, nv = E >> 4, nck = DK >> 3, ncv = E >> 3;
-  u16* k_s = bsa_lds;                                 // [32][LD], zero past a map's D columns
-  u16* v_t = bsa_lds + 32 * LD;                       // [16 NVM][LT], rows past E as they are: they reach columns that are not stored
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
+  const int DK = MAPS * D, nv = E >> 4, ncd = D >> 3, ncv = E >> 3;
+  const unsigned lds0 = (unsigned)(size_t)(lds_char*)bsa_lds;          // two buffers of a step's key rows and value rows
+  unsigned* tab = reinterpret_cast<unsigned*>(bsa_lds + Tile::STEP);   // [2][32]: where two steps' rows stand in the cache
   const int b = blockIdx.y;
   // How many keys a tile sees depends on its place in the chunk (or, without a window, in the sequence).  Workgroups that share a CU
   // are about 256 apart in launch order, which is the same tile of another head block: every other run of 256 takes the tiles from the
@@ -883,10 +883,39 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
   const float scale2 = scale * BSA_LOG2E;
   const u16* kbase = reinterpret_cast<const u16*>(kv.k);
   const u16* vbase = reinterpret_cast<const u16*>(kv.v);
+  auto key_at = [&](int kx) { return kx < kept ? kx : j_off + kx; };
+  auto row_pos = [&](int kx) { return key_at(min(kx, total - 1)); };            // behind the last key the last one again, masked
+  auto issue = [&](int st) __attribute__((always_inline)) {
+    const unsigned to = lds0 + (unsigned)(st & 1) * Tile::STEP;
+    auto row_of = [&](int r) { return tab[(st & 1) * 32 + r]; };
+    rows_issue<4 * NSM * MAPS, 4>(kbase, DK, to, wave, lane, row_of, [&](int c) {
+      if (FULL && Tile::Keys::CH == 4 * NSM * MAPS) return c;
+      const int mp = MAPS == 2 && c >= 4 * NSM ? 1 : 0, cc = c - mp * 4 * NSM;
+      return cc < ncd ? mp * ncd + cc : -1;           // zeros past a map's D columns
+    });
+    rows_issue<2 * NVM, 4>(vbase, E, to + Tile::Keys::BYTES, wave, lane, row_of, [&](int c) { return (FULL && Tile::Values::CH == 2 * NVM) || c < ncv ? c : -1; });
+  };
+  const int hd = g * hpg + (active ? hl : hpg - 1);
+  float bnext[8];
+  auto ask_bias = [&](int base) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int dd = i_j - key_at(base + 16 * (e >> 2) + 4 * g4 + (e & 3)), di = dd < 0 ? 0 : (dd < n_dist ? dd : n_dist - 1);
+      bnext[e] = bias[(long)hd * n_dist + di];
+    }
+  };
+  RowKeys<4 * NSM * MAPS> keys(j, g4);
+  RowValues<2 * NVM> values(j, g4);
+  const int steps = (total + 31) / 32;
+  RowAsked next{};
+  if (threadIdx.x < 64) tab[threadIdx.x] = pkv_tok_row(kv, slot, row_pos(threadIdx.x), g, G);
+  if (threadIdx.x < 32) next.ask(kv, slot, row_pos(64 + threadIdx.x));
+  if (bias) ask_bias(0);
+  __syncthreads();
+  issue(0);                                           // on its way beside the queries
   u32x4 qh[HPW][NSM], ql[HPW][NSM];
   f32x4 o[HPW][NVM];
   float m_run[HPW], l_run[HPW];
-  const int hd = g * hpg + (active ? hl : hpg - 1);
 #pragma unroll
   for (int hh = 0; hh < HPW; ++hh) {
     const float* qr = q + ((qrow * H + hd) * MAPS + hh) * D;
@@ -911,78 +940,45 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     m_run[hh] = -INFINITY;
     l_run[hh] = 0.f;
   }
-  // staging role of a thread: key row sm of the step, 16-byte chunks sc, sc + 8, ... of that row (keys and values)
-  const int sm = threadIdx.x & 31, sc = threadIdx.x >> 5;
-  u32x4 stk[NLK], stv[NLV];
-  auto fetch = [&](int base) {
-    const int kx = base + sm;
-    const bool ok = kx < total;
-    const int jk = kx < kept ? kx : j_off + kx;
-    const unsigned rw = ok ? pkv_tok_row(kv, slot, jk, g, G) : 0;
-    const long offk = (long)rw * DK, offv = (long)rw * E;
-#pragma unroll
-    for (int u = 0; u < NLK; ++u) {
-      const int ch = sc + 8 * u;
-      stk[u] = (ok && ch < nck) ? *reinterpret_cast<const u32x4*>(kbase + offk + 8 * ch) : u32x4{0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int u = 0; u < NLV; ++u) {
-      const int ch = sc + 8 * u;
-      stv[u] = (ok && ch < ncv) ? *reinterpret_cast<const u32x4*>(vbase + offv + 8 * ch) : u32x4{0u, 0u, 0u, 0u};
-    }
-  };
-  fetch(0);
-  const int pad = (KD - D) >> 3;                      // 16-byte chunks a map's part is short of its steps
-  for (int x = threadIdx.x; x < 32 * MAPS * pad; x += 256)
-    *reinterpret_cast<u32x4*>(k_s + (x & 31) * LD + (x >> 5) / pad * KD + D + 8 * ((x >> 5) % pad)) = u32x4{0u, 0u, 0u, 0u};
-  for (int base = 0; base < total; base += 32) {
-    __syncthreads();                                  // every wave is done with the previous tile
-#pragma unroll
-    for (int u = 0; u < NLK; ++u) {
-      const int ch = sc + 8 * u;
-      if (ch < nck) *reinterpret_cast<u32x4*>(k_s + sm * LD + 8 * ch + (MAPS == 2 && 8 * ch >= D ? KD - D : 0)) = stk[u];
-    }
-#pragma unroll
-    for (int u = 0; u < NLV; ++u) {
-      const int ch = sc + 8 * u;
-      if (ch < ncv) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v_t[(8 * ch + 2 * e) * LT + sm] = (u16)(stv[u][e] & 0xffffu);
-          v_t[(8 * ch + 2 * e + 1) * LT + sm] = (u16)(stv[u][e] >> 16);
-        }
-      }
-    }
-    __syncthreads();
-    if (base + 32 < total) fetch(base + 32);          // in flight while this step is used
-    if (!active) continue;
-    // which of the lane's eight keys this query sees, and at what distance: the same for every head
-    // (a step that every query sees whole needs no tests: rows past the last are not stored)
-    const bool whole = base >= kept && j_off + base + 31 <= i_first && j_off + base >= lo_all;
+  for (int st = 0; st < steps; ++st) {
+    const int base = st * 32;
+    // the step's rows have landed and nobody reads the step before any more: its buffer and its half of the table are free
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
     float bv[8];
     if (bias) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int kx = base + 16 * (e >> 2) + 4 * g4 + (e & 3);
-        const int dd = i_j - (kx < kept ? kx : j_off + kx), di = dd < 0 ? 0 : (dd < n_dist ? dd : n_dist - 1);
-        bv[e] = bias[(long)hd * n_dist + di];
-      }
+      for (int e = 0; e < 8; ++e) bv[e] = bnext[e];
     }
+    if (threadIdx.x < 32) tab[(st & 1) * 32 + threadIdx.x] = next.row(kv, g, G);      // (in front of the issue: a wait for the look-up must not wait for that)
+    if (st + 1 < steps) issue(st + 1);
+    if (threadIdx.x < 32) next.ask(kv, slot, row_pos(base + 96 + threadIdx.x));
+    if (bias) ask_bias(base + 32);
+    if (!active) continue;
+    keys.at_step(lds0 + (unsigned)(st & 1) * Tile::STEP);
+    values.at_step(lds0 + (unsigned)(st & 1) * Tile::STEP + Tile::Keys::BYTES);
+    // which of the lane's eight keys this query sees, and at what distance: the same for every head
+    // (a step that every query sees whole needs no tests: rows past the last are not stored)
+    const bool whole = base >= kept && j_off + base + 31 <= i_first && j_off + base >= lo_all;
+    // fragments are read FR of them ahead of their products, the values' first ones in front of the softmax
+    constexpr int FR = 4, NK = 2 * NSM * MAPS;
+    u32x4 fr[FR];
     f32x4 sc2[HPW][2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int hh = 0; hh < HPW; ++hh) sc2[hh][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const u16* kr = k_s + (16 * u + j) * LD;
+    auto key_frag = [&](int i) { return keys(i & 1, (i >> 1) % MAPS * NSM + (i >> 1) / MAPS); };         // (step of the map's features, map, key tile)
 #pragma unroll
-      for (int s = 0; s < NSM; ++s) {
+    for (int i = 0; i < FR; ++i) fr[i] = key_frag(i);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int mp = 0; mp < MAPS; ++mp) {
-          const u32x4 kf = *reinterpret_cast<const u32x4*>(kr + mp * KD + 32 * s + 8 * g4);
-          sc2[mp][u] = P::mfma(kf, ql[mp][s], sc2[mp][u]);
-          sc2[mp][u] = P::mfma(kf, qh[mp][s], sc2[mp][u]);
-        }
-      }
+    for (int i = 0; i < NK; ++i) {
+      const int u = i & 1, mp = (i >> 1) % MAPS, s = (i >> 1) / MAPS;
+      sc2[mp][u] = P::mfma(fr[i % FR], ql[mp][s], sc2[mp][u]);
+      sc2[mp][u] = P::mfma(fr[i % FR], qh[mp][s], sc2[mp][u]);
+      fr[i % FR] = i + FR < NK ? key_frag(i + FR) : values(i + FR - NK);
+      __builtin_amdgcn_sched_barrier(0);
     }
     u32x4 ph[HPW], pl[HPW];
 #pragma unroll
@@ -990,9 +986,10 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
       // maxima and exponents in base 2 (scale2 = scale log2 e): one v_exp_f32 per weight
       float sv[8], mx = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        sv[e] = sc2[hh][e >> 2][e & 3] * scale2;
-        if (softcap > 0.f) sv[e] = softcap * tanhf(sc2[hh][e >> 2][e & 3] * scale / softcap) * BSA_LOG2E;      // capped, then to base 2
+      for (int e = 0; e < 8; ++e) sv[e] = sc2[hh][e >> 2][e & 3] * scale2;
+      if (softcap > 0.f) {                                           // (one test for all: eight of them stood between the products and the maximum)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sv[e] = softcap * tanhf(sc2[hh][e >> 2][e & 3] * scale / softcap) * BSA_LOG2E;      // capped, then to base 2
       }
       if (bias) {
 #pragma unroll
@@ -1008,9 +1005,7 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sv[e]);
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run[hh], mx);
+      const float m_new = fmaxf(m_run[hh], rows_quad_max(mx));
       const float m_ref = m_new == -INFINITY ? 0.f : m_new;          // a row that has seen no key yet: all weights 0
       const float fac = __builtin_amdgcn_exp2f(m_run[hh] - m_ref);
       float w[8], sum = 0.f;
@@ -1019,9 +1014,7 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
         w[e] = __builtin_amdgcn_exp2f(sv[e] - m_ref);
         sum += w[e];
       }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
-      l_run[hh] = l_run[hh] * fac + sum;
+      l_run[hh] = l_run[hh] * fac + sum;                             // this lane's keys: added over the four lanes behind the walk
       m_run[hh] = m_new;
       if (__ballot(fac != 1.f)) {                                    // the maximum moved for some row of the tile
 #pragma unroll
@@ -1036,15 +1029,19 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     // O^T[d][query] += V^T[d][keys] P^T[keys][query]: lane (d row j of tile dt, quad g4) reads its 8 keys' values
 #pragma unroll
     for (int dt = 0; dt < NVM; ++dt) {
-      const u16* vr = v_t + (16 * dt + j) * LT + 4 * g4;
-      const u32x2 t0 = *reinterpret_cast<const u32x2*>(vr), t1 = *reinterpret_cast<const u32x2*>(vr + 16);
-      const u32x4 va = u32x4{t0[0], t0[1], t1[0], t1[1]};
 #pragma unroll
       for (int hh = 0; hh < HPW; ++hh) {
-        o[hh][dt] = P::mfma(va, pl[hh], o[hh][dt]);
-        o[hh][dt] = P::mfma(va, ph[hh], o[hh][dt]);
+        o[hh][dt] = P::mfma(fr[(dt + NK) % FR], pl[hh], o[hh][dt]);
+        o[hh][dt] = P::mfma(fr[(dt + NK) % FR], ph[hh], o[hh][dt]);
       }
+      if (dt + FR < NVM) fr[(dt + NK) % FR] = values(dt + FR);
+      __builtin_amdgcn_sched_barrier(0);
     }
+  }
+#pragma unroll
+  for (int hh = 0; hh < HPW; ++hh) {
+    l_run[hh] += __shfl_xor(l_run[hh], 16, 64);
+    l_run[hh] += __shfl_xor(l_run[hh], 32, 64);
   }
   // lane holds O^T[d = 16 dt + 4 g4 + rr][query j]
   if (q_ok && active) {

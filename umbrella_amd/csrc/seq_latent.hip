@@ -17,6 +17,7 @@
 // Two front ends: queries through a latent of their own (lat_prep norms both latents and appends, an up-projection follows,
 // lat_qsplit takes its result apart), or queries straight from the fused input projection (lat_front: one launch for all of it).
 #include "seq_common.h"
+#include "seq_rows.h"
 #include <cstdlib>
 
 constexpr float LOG2E = 1.4426950408889634f;
@@ -321,23 +322,23 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_kernel(typename El<P>::typ
 // ---- prompt attention on the matrix pipe (16-bit storage; Dk a multiple of 8, kv_rank a multiple of 16).
 // Workgroup = (16 consecutive positions of one sequence, a block of NW HPW heads); wave w owns HPW heads.  The tile's keys -- from
 // the first position's window start to the last position -- are walked in steps of 32 by the whole workgroup: the step's 32
-// cached rows (all Dk features) are staged ONCE into a shared LDS tile and serve every head of the workgroup, as keys and as
-// values; the next step's rows are already in flight (in registers) while the current one is used, so the one global round
-// trip of a step hides behind its matrix products, and the small tile leaves room for several workgroups per CU.
+// cached rows (all Dk features) stand ONCE in LDS and serve every head of the workgroup, as keys and as values (seq_rows.h); the next
+// step's are on their way to a second buffer while the current one is used.
 // Per step and head:
 //   S^T = K Q^T as two 16-key MFMA tiles (A = 16 keys x 32 features read from the LDS tile, B = the queries, rounded to the
 //         storage dtype once, when the tile starts);
 //   online softmax in fp32: lane (query j, key quad g) holds keys 4g .. 4g+3 of both tiles; the row maximum and sum are
-//         finished over the four lanes of a query by two shuffles; accumulators are rescaled when the maximum grows;
+//         finished over the four lanes of a query by lane swaps, the sum behind the walk; accumulators are rescaled when the maximum grows;
 //   O^T += V^T P^T: the lane's eight weights ARE its share of the B operand when V^T's k index runs over (tile 0: 4g .. 4g+3,
-//         tile 1: 4g .. 4g+3); V^T (A: 16 features x those 8 keys) is gathered from the LDS tile.
+//         tile 1: 4g .. 4g+3); V^T (A: 16 features x those 8 keys) is read transposed from the LDS tile.
 // The sink joins the denominator at the end.  Products per step at compile time: NSM steps of 32 features and NVM tiles of 16, the least of a few
 // sizes that hold Dk and Dc, with zeros behind a row's Dk features; FULL: they are the counts.  With run-time counts every product stood in a
-// block of its own behind its own LDS read, and the step was that latency sixty times over: 2000 positions, 32 heads, kv_rank + rotary 512 + 64
-// 962 us, with counts and four waves 497, eight waves on a staged step (two a SIMD; they spill 16 registers) 372; 384 + 64 849 -> 241.
-template <int NSM, int NVM> struct LatTile {
-  static constexpr int LD = NSM * 32 + 8, LT = 36;              // row strides of a step's rows and of its transposed values: 16 and 8 bytes of padding
-  static constexpr size_t LDS = ((size_t)32 * LD + (size_t)NVM * 16 * LT) * sizeof(u16);
+// block of its own behind its own LDS read, and the step was that latency sixty times over.  2000 positions, 32 heads, kv_rank + rotary 512 + 64:
+// run-time counts 962 us, counts, rows staged through registers and values transposed by 2-byte stores behind two barriers 376, by LDS-DMA with
+// transposed reads 270, fragments read ahead of their products 178; 384 + 64 849 / 233 / - / 150, 256 + 32 of 16 heads - / 84 / - / 59.
+template <int NSM> struct LatTile {
+  typedef RowTile<4 * NSM> Rows;
+  static constexpr size_t LDS = 2 * Rows::BYTES + 2 * 32 * sizeof(unsigned);
 };
 template <typename P, int NSM, int NVM, int HPW, int NW, bool FULL>
 __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restrict__ out, const float* __restrict__ qa, UmbPagedKV kv,
@@ -346,15 +347,14 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
                                                               const int* __restrict__ seq_len, int H, int Dc, int R, int window,
                                                               float scale) {
   extern __shared__ __attribute__((aligned(16))) u16 lat_lds[];
-  constexpr int SR = 2 * NW, NLD = (4 * NSM + SR - 1) / SR;           // staging threads per row, 16-byte chunks of the row for each
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
+  typedef typename LatTile<NSM>::Rows Rows;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
   if constexpr (FULL) { Dc = NVM * 16; R = NSM * 32 - Dc; }
-  constexpr int LD = LatTile<NSM, NVM>::LD, LT = LatTile<NSM, NVM>::LT;
   const int Dk = Dc + R, nv = Dc >> 4, nch = Dk >> 3;
-  u16* v_s = lat_lds;                                 // [32][LD]: the step's rows as cached, zero past Dk (keys: A operand of S^T = K Q^T)
-  u16* v_t = lat_lds + 32 * LD;                       // [16 NVM][LT]: their first Dc features transposed (values: A operand of O^T); the rest as it is
+  const unsigned lds0 = (unsigned)(size_t)(lds_char*)lat_lds;          // two buffers of a step's rows
+  unsigned* tab = reinterpret_cast<unsigned*>(lat_lds + Rows::BYTES);  // [2][32]: where two steps' rows stand in the cache
   const int b = blockIdx.y;
-  const int n = seq_len[b], q0 = blockIdx.x * 16;
+  const int n = seq_len[b], q0 = (int)(gridDim.x - 1 - blockIdx.x) * 16;         // late tiles see more keys: they start first
   if (q0 >= n) return;                                // the whole workgroup
   const int h0 = (blockIdx.z * NW + wave) * HPW;
   const bool active = h0 < H;                         // a wave without heads still stages rows and meets the barriers
@@ -368,6 +368,20 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
   const int total = i_last - j_lo + 1;
   const float scale2 = scale * LOG2E;
   const u16* kbase = reinterpret_cast<const u16*>(kv.k);
+  // (behind the last key the last one again, masked)
+  auto row_id = [&](int kx) { return pkv_tok_row(kv, slot, j_lo + min(kx, total - 1), 0, 1); };
+  auto issue = [&](int st) __attribute__((always_inline)) {
+    rows_issue<4 * NSM, NW>(kbase, Dk, lds0 + (unsigned)(st & 1) * Rows::BYTES, wave, lane, [&](int r) { return tab[(st & 1) * 32 + r]; },
+                            [&](int c) { return (FULL && Rows::CH == 4 * NSM) || c < nch ? c : -1; });
+  };
+  RowKeys<4 * NSM> keys(j, g4);
+  RowValues<4 * NSM> values(j, g4);
+  const int steps = (total + 31) / 32;
+  RowAsked next{};
+  if (threadIdx.x < 64) tab[threadIdx.x] = row_id(threadIdx.x);
+  if (threadIdx.x < 32) next.ask(kv, slot, j_lo + min(64 + (int)threadIdx.x, total - 1));
+  __syncthreads();
+  issue(0);                                           // on its way beside the queries
   u32x4 qf[HPW][NSM];
   f32x4 o[HPW][NVM];
   float m_run[HPW], l_run[HPW];
@@ -390,52 +404,36 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
     m_run[hh] = -INFINITY;
     l_run[hh] = 0.f;
   }
-  // staging role of a thread: key row sm of the step, 16-byte chunks sc, sc + SR, ... of that row
-  const int sm = threadIdx.x & 31, sc = threadIdx.x >> 5;
-  u32x4 stage[NLD];
-  auto fetch = [&](int base) {
-    const int kx = base + sm;
-    const long off = kx < total ? pkv_tok(kv, slot, j_lo + kx, 0, 1, Dk) : -1;
-#pragma unroll
-    for (int u = 0; u < NLD; ++u) {
-      const int ch = sc + SR * u;
-      stage[u] = (off >= 0 && ch < nch) ? *reinterpret_cast<const u32x4*>(kbase + off + 8 * ch) : u32x4{0u, 0u, 0u, 0u};
-    }
-  };
-  fetch(0);
-  if (threadIdx.x < 32)
-    for (int ch = nch; ch <= NSM * 4; ++ch) *reinterpret_cast<u32x4*>(v_s + threadIdx.x * LD + 8 * ch) = u32x4{0u, 0u, 0u, 0u};
-  for (int base = 0; base < total; base += 32) {
-    __syncthreads();                                  // every wave is done with the previous tile
-#pragma unroll
-    for (int u = 0; u < NLD; ++u) {
-      const int ch = sc + SR * u;
-      if (ch < nch) {
-        *reinterpret_cast<u32x4*>(v_s + sm * LD + 8 * ch) = stage[u];
-        if (8 * ch < Dc) {                            // Dc is a multiple of 16: a chunk is all values or all rotated key part
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            v_t[(8 * ch + 2 * e) * LT + sm] = (u16)(stage[u][e] & 0xffffu);
-            v_t[(8 * ch + 2 * e + 1) * LT + sm] = (u16)(stage[u][e] >> 16);
-          }
-        }
-      }
-    }
-    __syncthreads();
-    if (base + 32 < total) fetch(base + 32);          // in flight while this step is used
+  for (int st = 0; st < steps; ++st) {
+    const int base = st * 32;
+    // the step's rows have landed and nobody reads the step before any more: its buffer and its half of the table are free
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (threadIdx.x < 32) tab[(st & 1) * 32 + threadIdx.x] = next.row(kv, 0, 1);      // (in front of the issue: a wait for the look-up must not wait for that)
+    if (st + 1 < steps) issue(st + 1);
+    if (threadIdx.x < 32) next.ask(kv, slot, j_lo + min(base + 96 + (int)threadIdx.x, total - 1));
     if (!active) continue;
+    keys.at_step(lds0 + (unsigned)(st & 1) * Rows::BYTES);
+    values.at_step(lds0 + (unsigned)(st & 1) * Rows::BYTES);
+    // fragments are read FR products ahead of theirs, the values' first ones in front of the softmax: with the reads left to the compiler each stood
+    // right in front of its product, a wait of LDS latency sixty times a step
+    constexpr int FR = 4;
+    u32x4 fr[FR];
     f32x4 sc2[HPW][2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int hh = 0; hh < HPW; ++hh) sc2[hh][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const u16* kr = v_s + (16 * u + j) * LD;
 #pragma unroll
-      for (int s = 0; s < NSM; ++s) {
-        const u32x4 kf = *reinterpret_cast<const u32x4*>(kr + 32 * s + 8 * g4);
+    for (int i = 0; i < FR; ++i) fr[i] = keys(i & 1, i >> 1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int hh = 0; hh < HPW; ++hh) sc2[hh][u] = P::mfma(kf, qf[hh][s], sc2[hh][u]);
-      }
+    for (int i = 0; i < 2 * NSM; ++i) {
+#pragma unroll
+      for (int hh = 0; hh < HPW; ++hh) sc2[hh][i & 1] = P::mfma(fr[i % FR], qf[hh][i >> 1], sc2[hh][i & 1]);
+      const int nx = i + FR;
+      fr[i % FR] = nx < 2 * NSM ? keys(nx & 1, nx >> 1) : values(nx - 2 * NSM);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // a step that every query sees whole needs no tests (rows past the last are not stored)
     const bool whole = j_lo + base + 31 <= i_first && j_lo + base > i_last - window;
@@ -455,9 +453,7 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sv[e]);
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m_run[hh], mx);
+      const float m_new = fmaxf(m_run[hh], rows_quad_max(mx));
       const float m_ref = m_new == -INFINITY ? 0.f : m_new;          // a row that has seen no key yet: all weights 0
       const float fac = __builtin_amdgcn_exp2f(m_run[hh] - m_ref);
       float w[8], sum = 0.f;
@@ -466,9 +462,7 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
         w[e] = __builtin_amdgcn_exp2f(sv[e] - m_ref);
         sum += w[e];
       }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
-      l_run[hh] = l_run[hh] * fac + sum;
+      l_run[hh] = l_run[hh] * fac + sum;                             // this lane's keys: added over the four lanes behind the walk
       m_run[hh] = m_new;
       if (__ballot(fac != 1.f)) {                                    // the maximum moved for some row of the tile
 #pragma unroll
@@ -479,12 +473,16 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
     // O^T[d][query] += V^T[d][keys] P^T[keys][query]: lane (d row j of tile dt, quad g4) reads its 8 keys' values
 #pragma unroll
     for (int dt = 0; dt < NVM; ++dt) {
-      const u16* vr = v_t + (16 * dt + j) * LT + 4 * g4;
-      const u32x2 t0 = *reinterpret_cast<const u32x2*>(vr), t1 = *reinterpret_cast<const u32x2*>(vr + 16);
-      const u32x4 va = u32x4{t0[0], t0[1], t1[0], t1[1]};
 #pragma unroll
-      for (int hh = 0; hh < HPW; ++hh) o[hh][dt] = P::mfma(va, pf[hh], o[hh][dt]);
+      for (int hh = 0; hh < HPW; ++hh) o[hh][dt] = P::mfma(fr[(dt + 2 * NSM) % FR], pf[hh], o[hh][dt]);
+      if (dt + FR < NVM) fr[(dt + 2 * NSM) % FR] = values(dt + FR);
+      __builtin_amdgcn_sched_barrier(0);
     }
+  }
+#pragma unroll
+  for (int hh = 0; hh < HPW; ++hh) {
+    l_run[hh] += __shfl_xor(l_run[hh], 16, 64);
+    l_run[hh] += __shfl_xor(l_run[hh], 32, 64);
   }
   // lane holds O^T[d = 16 dt + 4 g4 + rr][query j]
   if (q_ok && active) {
@@ -682,14 +680,15 @@ extern "C" int umb_lat_attend_tiled(void* out, const float* qa, const UmbPagedKV
     return UMB_EINVAL;
   const int Dk = kv_rank + rot_dim;
   // Eight waves share a staged step where there is a workgroup of them for most compute units and the walk is long or its rows are; four, and
-  // twice the workgroups, elsewhere (us with 4 / 8 waves, kv_rank + rotary, heads, positions: 512 + 64, 32: 16 16 / 24, 600 111 / 120, 2000
-  // 497 / 372, 8 x 300 174 / 157; 384 + 64, 32: 600 69 / 76, 2000 249 / 241, 8 x 300 98 / 106; 256 + 32, 16: 600 39 / 48, 2000 55 / 53, 8 x 300 41 / 48)
+  // twice the workgroups, elsewhere (us with 4 / 8 waves, kv_rank + rotary, heads, positions: 512 + 64, 32: 16 14 / 22, 300 30 / 40, 600 62 / 60,
+  // 2000 250 / 178, 8 x 300 114 / 98; 8 heads, 8 x 300 45 / 40; 384 + 64, 32: 600 52 / 52, 2000 156 / 151, 8 x 300 73 / 81; 256 + 32, 16: 1200 53 / 56,
+  // 2000 64 / 60, 8 x 300 33 / 39)
   const long eights = (long)((max_len + 15) / 16) * B * ((H + 7) / 8);
-  const bool eight = H > 4 && eights >= 200 && (kv_rank > 384 || max_len >= 1000);
+  const bool eight = H > 4 && eights >= (kv_rank > 384 ? 150 : 200) && (kv_rank > 384 || max_len >= 1000);
 #define LAT_MFMA_AS(NSM, NVM, HPW, NW, FULL)                                                                               \
   do {                                                                                                                     \
     const dim3 grid((max_len + 15) / 16, B, (H + NW * HPW - 1) / (NW * HPW));                                              \
-    constexpr size_t lds = LatTile<NSM, NVM>::LDS;                                                                         \
+    constexpr size_t lds = LatTile<NSM>::LDS;                                                                              \
     if (ensure_dynamic_lds<lat_attend_mfma_kernel<P, NSM, NVM, HPW, NW, FULL>>(lds) != UMB_OK) return UMB_EHIP;            \
     hipLaunchKernelGGL((lat_attend_mfma_kernel<P, NSM, NVM, HPW, NW, FULL>), grid, dim3(NW * 64), lds, st, (u16*)out, qa, *kv, \
                        (const u16*)sink, seq_slot, seq_row0, seq_pos0, seq_len, H, kv_rank, rot_dim, window, scale);       \

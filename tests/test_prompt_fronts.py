@@ -159,3 +159,30 @@ def test_prompt_attention_of_any_page_size(D, E, maps, keep, chunk):
     assert bool((outs[0][0][T] == 3.0).all()) and bool((outs[0][1][T] == 3.0).all()) and bool(outs[0][0].isfinite().all())
     for o in outs[1:]:
         assert torch.equal(o[0], outs[0][0]) and torch.equal(o[1], outs[0][1])
+
+
+@pytest.mark.parametrize("D,E,maps,n", [(128, 128, 1, 1), (64, 64, 1, 129), (128, 256, 2, 70), (128, 128, 1, 192)])
+def test_single_token_in_a_cache_of_one_span(D, E, maps, n):
+    """a page table of less than one span of keys: no splits and no merge behind them, the bits of a large cache"""
+    from umbrella_amd import _lib
+    from umbrella_amd.attn.cache import PagedSeqCache
+    H, G, dtype = 8, 2, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")                   # noqa: E731
+    keys, vals, q = rnd(n, G, maps * D).to(dtype), rnd(n, G, E).to(dtype), rnd(1, H, maps, D)
+    pos, scratch, outs = torch.tensor([n - 1], dtype=torch.int32, device="cuda"), torch.full((H * maps * 16 * (E + 2),), 4.0, device="cuda"), []
+    for room in (n, 4000):
+        c = PagedSeqCache([(G, maps * D, 0, E)], [], room, 1, "cuda", dtype, page=16)
+        entries = []
+        c.open(0)
+        c.extend(0, n, entries)
+        c.write_pages(entries)
+        at = torch.arange(n, device="cuda")
+        pg = c.pages_dev[c.slot(0)].long()[at // 16]
+        c.kv[0]["k"][pg, :, at % 16], c.kv[0]["v"][pg, :, at % 16] = keys, vals
+        out, slot = torch.full((2, H * E), 3.0, dtype=dtype, device="cuda"), torch.tensor([c.slot(0)], dtype=torch.int32, device="cuda")
+        _lib.seq_call("umb_attn_attend", out, H * E, q, c.struct(0), None, 0, -1, None, 0, pos, slot, 1, H, G, D, E, 2 ** 30, D ** -0.5, 1.0, 0.0,
+                      _lib.UmbAttnForm(maps, 0, None, 0.3, 1e-3, 0, 0), scratch, scratch.numel(), _lib.seq_dtype_code(dtype))
+        assert bool((out[1] == 3.0).all()) and bool(out.isfinite().all())
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])

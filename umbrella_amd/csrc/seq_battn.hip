@@ -27,6 +27,7 @@
 // keys land in which wave and round depends on the query's position and on the launch (waves an item, splits of a token's keys, prompt tiles):
 // the same token in another batch, or of a prompt cut elsewhere, agrees to fp32 rounding and not bit for bit.
 #include "seq_common.h"
+#include <algorithm>
 #include "seq_decode.h"
 #include "seq_rows.h"
 
@@ -678,7 +679,9 @@ static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv,
   while (rh > maps && hpg % (rh / maps)) rh >>= 1;
   const int hblocks = H * maps / rh;
   const long items = (long)T * hblocks;
-  const long most = (long)(form.chunk > 0 && form.chunk < window ? form.chunk : window) + form.keep_first;
+  // keys a token can have: by the mask's form and by what a sequence's page table holds.  Within one span nobody splits, and the merge behind it would
+  // find nothing to do: one token of 8B widths in a cache of 192 positions, three layers 56 us -> 41 without the merges (4.6 us each)
+  const long most = std::min((long)(form.chunk > 0 && form.chunk < window ? form.chunk : window) + form.keep_first, (long)kv->max_pages * kv->page);
   int nsplit = 1;
   if (scratch && items <= 64 && most > ATT_SPAN) {
     nsplit = (int)(512 / items) < 16 ? (int)(512 / items) : 16;

@@ -583,12 +583,12 @@ typedef struct UmbSeqWork {
   void* moe_xs;       /* [pairs][W] dtype */
   void* moe_act;      /* [pairs][max expert_ff] dtype */
   float* moe_y;       /* [pairs][W] fp32 */
-  int64_t moe_max_tiles;
+  int32_t moe_max_tiles;
+  int32_t y_rows;      /* rows of W floats in y, and in y2 where there is one: room for the slabs of split products (0: no slabs) */
   int64_t aux_floats;  /* floats in aux (what a step does not use of it serves as scratch) */
   void* h2;            /* parallel blocks: normed input of the feed-forward [Tmax][W] dtype */
   float* y2;           /* parallel blocks: feed-forward output; mixers with two output projections: the second [Tmax][W] fp32 */
   float* v_first;      /* values that later layers of the step mix in [Tmax][kv_heads vdim] fp32 (null when no layer does) */
-  int64_t y_floats;    /* floats in y, and in y2 where there is one (0: Tmax W): room for the slabs of split products */
 } UmbSeqWork;
 
 typedef struct UmbSeqStep {

@@ -98,11 +98,40 @@ static int dgemm_launch(const void* wp, const u16* x, int ldx, float* out, int T
   return UMB_OK;
 }
 
+// Up to 128 tokens a launch is a round or two of any tile, and what is left to choose is the order in which K is summed: that of recorded
+// greedy continuations behind 96-token prompts, whose near-ties a different rounding of the cached keys would decide otherwise.  Five tiles by
+// rounds x stages, K over two groups of waves where a launch has at most one workgroup per compute unit.
+static int dgemm_narrow(int T, int N, int K, int S, double* us) {
+  static const struct { int bn, bt; double us; bool ksplit; } kind[5] = {
+      {256, 256, 1.5, false}, {256, 160, 1.1, false}, {128, 128, 0.52, false}, {128, 128, 0.56, true}, {128, 64, 0.39, true}};
+  const bool even = K % (128 * S) == 0;
+  int best = 2;
+  *us = 1e30;
+  for (int i = 0; i < 5; ++i) {
+    const long wgs = (long)((N + kind[i].bn - 1) / kind[i].bn) * ((T + kind[i].bt - 1) / kind[i].bt) * S, rounds = (wgs + 255) / 256;
+    if (kind[i].ksplit && (rounds > 1 || !even)) continue;
+    // a lone workgroup of the two-per-CU form (128 x 128) leaves half the wave slots empty
+    const double cost = rounds * ((K / 64 + S - 1) / S) * (i == 2 && rounds == 1 ? 0.62 : kind[i].us) + 4.0;
+    if (cost < *us) { *us = cost; best = i; }
+  }
+  return best;
+}
+
 // the tile by tile_kind (gemm_tile.h)
 static int dgemm_tile(int T, int N, int K, int S, double* us = nullptr) { return tile_kind(T, N, (K / 64 + S - 1) / S, S, K % (128 * S) == 0, us); }
 
 template <typename P>
 static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int S, int epi, const GemmFused& fx, hipStream_t st) {
+  if (T <= 128) {
+    double us;
+    switch (dgemm_narrow(T, N, K, S, &us)) {
+      case 0: return dgemm_launch<P, 4, 2, 4, 8, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+      case 1: return dgemm_launch<P, 4, 2, 4, 5, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+      case 2: return dgemm_launch<P, 2, 2, 4, 4, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+      case 3: return dgemm_launch<P, 2, 2, 4, 4, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+      default: return dgemm_launch<P, 2, 2, 4, 2, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+    }
+  }
   switch (dgemm_tile(T, N, K, S)) {
     case TILE_256: return dgemm_launch<P, 4, 2, 4, 8, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     case TILE_192: return dgemm_launch<P, 4, 2, 4, 6, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
@@ -134,8 +163,9 @@ int umb_dgemm_split(int T, int N, int K, int S_plan) {
   int best_s = 1;
   double best = 1e30, us = 0.0;
   for (int S = 1; S <= S_plan && S <= K / 128 && (long)S * T * N * 4 < (1L << 31); ++S) {
-    (void)dgemm_tile(T, N, K, S, &us);
-    const double cost = us + (S - 1) * (double)T * N * 4 / 8e6;
+    if (T <= 128) (void)dgemm_narrow(T, N, K, S, &us);
+    else (void)dgemm_tile(T, N, K, S, &us);
+    const double cost = us + (S - 1) * (double)T * N * 4 / (T <= 128 ? 3e6 : 8e6);
     if (cost < best) { best = cost; best_s = S; }
   }
   return best_s;

@@ -492,14 +492,13 @@ __global__ __launch_bounds__(64 * NW, NQ > 1 ? 1 : 2) void tree_attn1_kernel(con
   }
 }
 
-// ---- many query tiles (wide trees, prompt chunks): four waves of one 16-row query tile each share the keys.
+// ---- many causal query tiles (prompt chunks): four waves of one 16-row query tile each share the keys.
 // A wave per workgroup that walks 32 keys at a time (tree_attn1_kernel) is a chain -- products, maximum, two exchanges between lanes, exponents,
 // products -- of some 900 cycles per tile, two waves a SIMD, and pulls 16 KiB through the CU's path to L2 for each.  Here 64 keys make a step: one
 // chain for twice the work, its exchanges by lane swaps instead of through LDS, exponents in base 2 (one multiplication less); their K and V^T
 // (contiguous in the cache's fragment order) go to LDS by LDS-DMA once for the four tiles, one barrier a step; a fragment is read as it lies, a
 // contiguous KiB.  Two workgroups share a CU.  us, one MI355X, a wave each / this: 1024 causal
-// tokens of 32 + 8 heads of 128 behind 0 / 1024 keys 36 / 69 -> 25 / 46, of 64 24 / 42 -> 17 / 29; 257 tree rows of 64 + 8 heads behind 700 33 -> 25;
-// 769 behind 500 72 -> 54.  32 rows a wave (half the LDS reads, one wave a SIMD): 40 / 69.
+// tokens of 32 + 8 heads of 128 behind 0 / 1024 keys 36 / 69 -> 25 / 46, of 64 24 / 42 -> 17 / 29.  32 rows a wave (half the LDS reads, one wave a SIMD): 40 / 69.
 // max over lanes l, l ^ 16, l ^ 32, l ^ 48
 __device__ __forceinline__ float quad_max(float v) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -509,9 +508,8 @@ __device__ __forceinline__ float quad_max(float v) {
 }
 template <typename P, int D>
 __global__ __launch_bounds__(256, 2) void wide_attn_kernel(const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vt,
-                                                           const int* __restrict__ prefix_p, int T, int Hq, int Hkv, int Lmax, int mask_words,
-                                                           int n_mask_keys, const unsigned long long* __restrict__ mask_bits, float scale,
-                                                           u16* __restrict__ out, int fold) {
+                                                           const int* __restrict__ prefix_p, int T, int Hq, int Hkv, int Lmax, int n_mask_keys,
+                                                           float scale, u16* __restrict__ out, int fold) {
   constexpr int DS = D / 32, DT = D / 16, R = D == 128 ? 2 : 4, PW = D / 16;      // slots; 1-KiB pieces a wave fetches of a step
   constexpr unsigned SLOT = 256u * D, HALF = SLOT / 2;                            // K | V^T of 64 keys
   __shared__ __attribute__((aligned(16))) unsigned char ring[R * SLOT];
@@ -543,16 +541,7 @@ __global__ __launch_bounds__(256, 2) void wide_attn_kernel(const u16* __restrict
   const int prefix = *prefix_p, kv_end = prefix + n_mask_keys;
   int k_hi = kv_end, k_all = kv_end;                         // behind the last key that this tile, and any of the four, sees
   {
-    int top = -1;
-    if (row_ok && mask_bits) {
-      const unsigned long long* mrow = mask_bits + (long)t * mask_words;
-      for (int w = mask_words - 1; w >= 0; --w) {
-        const unsigned long long x = mrow[w];
-        if (x) { top = w * 64 + 63 - __clzll((long long)x); break; }
-      }
-    } else if (row_ok) {
-      top = t;
-    }
+    int top = row_ok ? t : -1;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) top = max(top, __shfl_xor(top, off, 64));
     if (lane == 0) tops[wv] = top;
@@ -596,18 +585,8 @@ __global__ __launch_bounds__(256, 2) void wide_attn_kernel(const u16* __restrict
       vbits[c] = 0xffu;
       if (k0 + 32 * c + 32 > prefix && bfirst > -8) {
         const int neg = max(-bfirst, 0);
-        unsigned v;
-        if (mask_bits) {
-          const int lo = max(bfirst, 0), wi = lo >> 6, sh = lo & 63;
-          const unsigned long long* mrow = mask_bits + (long)t * mask_words;
-          const unsigned long long w0 = mrow[min(wi, mask_words - 1)], w1 = mrow[min(wi + 1, mask_words - 1)];
-          unsigned long long x = w0 >> sh;
-          if (sh) x |= w1 << (64 - sh);
-          v = (unsigned)x & 0xffu;
-        } else {
-          const int n = min(max(t - max(bfirst, 0) + 1, 0), 8);
-          v = (1u << n) - 1u;
-        }
+        const int n = min(max(t - max(bfirst, 0) + 1, 0), 8);
+        const unsigned v = (1u << n) - 1u;
         vbits[c] = ((v << neg) | ((1u << neg) - 1u)) & 0xffu;
       }
     }
@@ -725,15 +704,16 @@ extern "C" int umb_tree_attn2(void* out, const void* q, const void* k_cache, con
     single_max = one_env > 0 ? one_env : 1024;
     if (single_max < KBK) single_max = KBK;
   }
-  // More than 1024 query tiles: four waves a compute unit and more, which share their keys (us, a wave each / this: 1032 tiles 32.9 / 25.3, 1024 without a
+  // More than 1024 causal query tiles (prompts; under a tree's mask the order of a row's sums stays the one of recorded continuations, whose near-ties
+  // another one decides otherwise): four waves a compute unit and more, which share their keys (us, a wave each / this: 1032 tiles 32.9 / 25.3, 1024 without a
   // prefix 12.6 / 13.3, 768 14.1 / 16.5, 520 behind 700 keys 19.1 / 23.5)
   static const int nw_env = getenv("UMB_ATTN_NW") ? atoi(getenv("UMB_ATTN_NW")) : 0;
-  if (Hkv * nqt > 1024 && !nw_env && !no_single && !out_fm_tt && ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)vt_cache | (uintptr_t)out) % 16 == 0) {
+  if (Hkv * nqt > 1024 && !mask_bits && !nw_env && !no_single && !out_fm_tt && ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)vt_cache | (uintptr_t)out) % 16 == 0) {
     const dim3 grid(Hkv, (nrows + 63) / 64);
     const int fold = (long)grid.x * grid.y <= 512;
 #define WIDE_(DD)                                                                                                                  \
   hipLaunchKernelGGL((wide_attn_kernel<P, DD>), grid, dim3(256), 0, st, (const u16*)q, (const u16*)k_cache, (const u16*)vt_cache,   \
-                     prefix_len, T, Hq, Hkv, Lmax, mask_words, n_mask_keys, (const unsigned long long*)mask_bits, scale, (u16*)out, fold)
+                     prefix_len, T, Hq, Hkv, Lmax, n_mask_keys, scale, (u16*)out, fold)
     DISPATCH_DTYPE(dtype, {
       if (D == 128) WIDE_(128);
       else if (D == 64) WIDE_(64);

@@ -113,3 +113,47 @@ def test_batched_tiles(dtype, B, T, N, K, pad):
         want = full * f
         bound = tol + 2.0 ** -22 * want.abs() + (0.0 if epi == 0 else 1.02 * half_ulp * want.abs() + 2.0 ** -25)
         assert ((got[..., :N] - want).abs() <= bound).all() and bool((got[..., N:] == 7.0).all()) and bool((out[T] == 7.0).all())
+
+
+# gates whose exponential leaves the normal range, infinities, NaN: fp32 on few tokens and many, 16 bits on tiles
+GATES = [0.0, -0.0, 1e-38, 5.0, 88.5, 200.0, 3e38, float("inf"), -86.9, -87.4, -88.0, -88.6, -89.0, -100.0, -200.0, -3e38, float("-inf"), float("nan")]
+
+
+@pytest.mark.parametrize("dtype,T", [(torch.float32, 1), (torch.float32, 300), (torch.bfloat16, 300)])
+def test_gates_to_the_ends_of_their_range(dtype, T):
+    """silu(gate) * up of the biases alone: the products are zero"""
+    from umbrella_amd import _lib
+    K, n = 128, 144
+    gate = torch.tensor((GATES * n)[:n]).to(dtype)
+    x, w = torch.zeros(T, K, device="cuda", dtype=dtype), torch.zeros(2 * n, K, device="cuda", dtype=dtype)
+    act = torch.empty(T, n, device="cuda", dtype=dtype)
+    _lib.seq_call("umb_seq_linear", act, x, w, torch.cat([gate, torch.ones(n, dtype=dtype)]).cuda(), T, 2 * n, K, 2, _lib.seq_dtype_code(dtype))
+    z = gate.double()
+    want = (z / (1.0 + torch.exp(-z))).expand(T, n)
+    # 3.1 units of 2^-24; e^-z beyond 32 bits (|z| > 88.72) gives 0; one rounding to 16 bits, whose least steps are 2^-133
+    half = dtype == torch.bfloat16
+    bound = (3.1 * 2.0 ** -24 + (2.0 ** -8 if half else 0.0)) * want.abs() + want.abs() * (z < -88.72) + 2.0 ** (-134 if half else -149)
+    got = act.double().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    ok = ~torch.isnan(want)
+    assert torch.equal(got[ok].isinf(), want[ok].isinf()) and ((got - want).abs() <= bound)[ok & ~want.isinf()].all()
+
+
+@pytest.mark.parametrize("epi", [3, 7])
+def test_batched_gates_to_the_ends_of_their_range(epi):
+    """the gate of a per-head product on tiles: a gate that is no number is seen in the result"""
+    from umbrella_amd import _lib
+    B, T, N, K = 32, 300, 128, 64
+    g = torch.Generator(device="cuda").manual_seed(epi)
+    x, w = (torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16) for s in ((T, B * K), (B, N, K)))
+    gate = torch.tensor((GATES * (T * B * N // len(GATES) + 1))[:T * B * N], device="cuda").view(T, B * N).contiguous()
+    out = torch.empty(T, B * N, device="cuda", dtype=torch.bfloat16)
+    _lib.seq_call("umb_seq_linear_batched", out, x, w, T, N, K, B * K, B * N, B, K, N * K, N, epi, gate, B * N, N if epi == 3 else 1, _lib.BF16)
+    xs, wt = x.double().view(T, B, K).transpose(0, 1).contiguous(), w.double().transpose(1, 2).contiguous()
+    full, size = (torch.bmm(a, b).transpose(0, 1) for a, b in ((xs, wt), (xs.abs(), wt.abs())))
+    s = torch.sigmoid(gate.double()).view(T, B, N) if epi == 3 else torch.sigmoid(gate[:, :B].double())[..., None].expand(T, B, N)
+    want, got = full * s, out.double().view(T, B, N)
+    assert torch.equal(got.isnan(), want.isnan())
+    # the product's sums, one rounding to 16 bits (least steps 2^-133), gates whose exponential is beyond 32 bits
+    bound = 2.0 ** -24 * (K + 4) * size * s + 1.02 * 2.0 ** -8 * want.abs() + want.abs() * (s < 2.95e-39) + 2.0 ** -134
+    assert ((got - want).abs() <= bound)[~want.isnan()].all()

@@ -85,6 +85,34 @@ def test_attention_of_many_tiles(dtype, D, Hq, Hkv, T, prefix, spare):
         assert bool((out[T] == 3.0).all())
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,T,prefix", [(128, 32, 8, 530, 0), (64, 32, 8, 515, 65), (32, 40, 8, 530, 20)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_values_that_are_not_finite_reach_one_tile_of_keys(D, Hq, Hkv, T, prefix, bad):
+    """prompts of more than 1024 query tiles: a value that a token does not see is weighted with zero inside its tile of 32 keys, and read nowhere else"""
+    from umbrella_amd.attn.cache import VT_PAD, k_to_frag, vt_to_frag
+    from umbrella_amd import _lib
+    S, g, dtype = prefix + T, Hq // Hkv, torch.bfloat16
+    Lmax = (S + 31) // 32 * 32
+    gen = torch.Generator().manual_seed(T + D)
+    q, k, v = (torch.randn(n, h, D, generator=gen).to(dtype) for n, h in ((T, Hq), (S, Hkv), (S, Hkv)))
+    pre, outs = torch.tensor([prefix], dtype=torch.int32, device="cuda"), []
+    for key in (None, (prefix + 32) // 64 * 64 + 40, (prefix + 300) // 64 * 64 + 32):       # in the later half of 64 keys
+        kc, vt = torch.zeros(Hkv, Lmax, D, dtype=dtype), torch.zeros(Hkv, D, Lmax + VT_PAD, dtype=dtype)
+        kc[:, :S], vt[:, :, :S] = k.permute(1, 0, 2), v.permute(1, 2, 0)
+        if key is not None:
+            vt[:, :, key] = bad
+        out = torch.empty(T, Hq, D, dtype=dtype, device="cuda")
+        _lib.call("umb_tree_attn", out, q.cuda(), k_to_frag(kc).cuda(), vt_to_frag(vt).cuda(), None, None, pre, None, 0, T, T, Hq, Hkv, D, Lmax, 256, 1,
+                  D ** -0.5, None, _lib.dtype_code(dtype))
+        outs.append(out)
+        if key is not None:
+            # a tile of 16 rows ends with the token of its last row: those whose keys end in front of the bad one's tile
+            ends = [prefix + min((16 * (r // 16) + 15) // g, T - 1) + 1 for r in range(T * g)]
+            clean = [t for t in range(T) if max(ends[t * g:t * g + g]) <= key // 32 * 32]
+            assert clean and torch.equal(out[clean], outs[0][clean])
+            assert bool((~out[key - prefix:].isfinite()).any())
+
+
 # every count of 16-row tiles a wave (full, ragged, none), chunks of one token, whole and with a tail, heads that do not fill the eight XCDs
 @pytest.mark.parametrize("D,E,Hk,H", [(16, 16, 1, 3), (33, 24, 2, 2), (64, 40, 1, 2), (80, 16, 3, 3), (96, 130, 1, 1), (128, 128, 4, 8), (144, 20, 1, 2),
                                       (208, 48, 1, 1), (256, 33, 1, 2)])

@@ -600,6 +600,10 @@ __global__ __launch_bounds__(256, 2) void wide_attn_kernel(const u16* __restrict
         const bool vis = row_ok && k0 + 32 * (e >> 3) + gq * 8 + (e & 7) < k_hi && ((vbits[e >> 3] >> (e & 7)) & 1u);
         pv[e] = vis ? pv[e] : -INFINITY;
       }
+      if (k0 + 32 >= k_hi) {                                 // 32 keys that no row sees: weight 0, but a value that is not finite would come through
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) av[1][dt] = zero4;
+      }
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, pv[e]);

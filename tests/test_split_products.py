@@ -25,6 +25,17 @@ def test_split_rule_stays_inside_what_the_product_takes():
         assert split(ptr + 8, ptr, 1, 2048, 8192, code) == 1 and split(ptr, ptr + 8, 1, 2048, 8192, code) == 1     # no 16-byte pieces
 
 
+def test_up_to_64_tokens_the_number_of_slabs_follows_from_the_weights():
+    """a token's sums are the same whatever else is in its step"""
+    from umbrella_amd import _lib
+    split = _lib.load_seq().umb_seq_linear_split
+    ptr = 1 << 20
+    for code in (_lib.BF16, _lib.F16, _lib.F32):
+        for N in (16, 192, 1000, 2048, 2049, 2560, 2720, 2721, 3072, 4096, 4097, 5120, 8192, 32000):
+            for K in (192, 512, 1024, 2048, 2304, 4096, 8192, 14336):
+                assert len({split(ptr, ptr, T, N, K, code) for T in range(1, 65)}) == 1, (N, K)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("T,N,chunks,parts", [(1, 16, 2, 2), (1, 2048, 8, 2), (16, 40, 7, 3), (17, 2049, 5, 4), (33, 4096, 16, 2), (48, 130, 32, 4),
@@ -127,3 +138,22 @@ def test_a_row_is_summed_in_one_order_whatever_the_batch(dtype, N, chunks):
         part = torch.empty(n, N, device="cuda")
         _lib.seq_call("umb_seq_linear", part, x[lo:lo + n].contiguous(), w, None, n, N, K, 0, _code(dtype))
         assert torch.equal(part, full[lo:lo + n])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("N,K", [(2048, 2048), (2600, 4096), (4096, 4096), (4096, 14336), (4112, 4096)])
+def test_a_row_has_one_order_in_slabs_too(dtype, N, K):
+    """what a sublayer's last product of up to 64 tokens leaves, slab by slab: the same bits for a token alone and among others"""
+    from umbrella_amd import _lib
+    dt, lib = DTYPES[dtype], _lib.load_seq()
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    x, w = (torch.randn(s, generator=g, device="cuda").to(dt) for s in ((64, K), (N, K)))
+    outs = []
+    for lo, n in ((0, 64), (0, 1), (5, 8), (7, 16), (30, 32), (20, 33), (10, 48)):
+        part = x[lo:lo + n].contiguous()
+        parts = lib.umb_seq_linear_split(part.data_ptr(), w.data_ptr(), n, N, K, _code(dtype))
+        out = torch.empty(parts, n, N, device="cuda")
+        _lib.seq_call("umb_seq_linear_parts", out, part, w, None, n, N, K, parts, _code(dtype))
+        outs.append(out)
+        assert out.shape[0] == outs[0].shape[0] and torch.equal(out, outs[0][:, lo:lo + n])

@@ -979,11 +979,14 @@ extern "C" int umb_seq_linear(void* out, const void* x, const void* w, const voi
   return seq_linear_any(out, x, w, bias, T, N, K, epi, 0.f, 0.f, dtype, st);
 }
 
-// Slabs of K for a product whose partial sums the kernel behind it adds (the seams), 1: none.  One workgroup per 16 output rows leaves half
-// of the compute units idle below 128 of them, and from 33 tokens on a unit's path is full of token pieces that two slabs with 32 output
-// rows each halve; a slab is four chunks at least (shorter ones are all prologue).  us at 1 / 16 / 48 tokens, bf16, cold weights, one MI355X,
-// 1 slab -> this rule's: 2048 x 8192 10.5 / 12.1 / 18.9 -> 8.8 / 9.5 / 10.8 (4); 2048 x 2048 4.6 / 5.0 / 7.2 -> 3.9 / 4.1 / 5.4 (2); 2560 x 6912 9.3 / 11.1 /
-// 15.3 -> 8.3 / 9.9 / 10.6 (3); 4096 x 14336, 48 tokens 37 -> 26 (2), and 1 / 16 tokens 24.0 / 24.7 stay whole (24.3 / 25.6 in two).
+// Slabs of K for a product whose partial sums the kernel behind it adds (the seams), 1: none.  Up to 64 tokens their number follows from the weights
+// alone, so a token's sums are the same whatever else is in its step.  One workgroup per 16 output rows leaves half of the compute units idle below
+// 128 of them, and from 33 tokens on a unit's path is full of token pieces that slabs with 32 output rows each halve; a slab is four chunks at
+// least (shorter ones are all prologue).  us at 1 / 16 / 48 tokens, bf16, cold weights, one MI355X, 1 slab -> this rule's: 2048 x 8192 10.5 / 12.1 / 18.9 ->
+// 8.8 / 9.5 / 10.8 (4); 2048 x 2048 4.6 / 5.0 / 7.2 -> 3.9 / 4.1 / 5.4 (2); 2560 x 6912 9.3 / 11.1 / 15.3 -> 8.3 / 9.9 / 10.6 (3).  Two slabs of more than 128
+// workgroups are behind up to 32 tokens and ahead beyond (with the seam behind it, 1 / 16 / 32 / 48 tokens, 1 -> 2: 4096 x 14336 27.3 / 27.7 / 33.6 /
+// 41.3 -> 28.0 / 29.2 / 35.6 / 31.7, 4096 x 4096 11.4 / 12.4 / 14.3 / 16.4 -> 12.0 / 13.3 / 15.2 / 14.9, 4096 x 8192 18.6 / 17.9 / 21.0 / 24.7 -> 21.6 / 20.8 /
+// 23.1 / 22.5): K whole, for decoding of small batches.
 //
 // Many tokens: the staged tiles, where rounds of them fill better with K in slabs than the whole K does: the least of the product's time and of
 // reading the slabs beyond the first in the kernel behind it (8 TB/s, they come from the last-level cache), against the whole K on the tiles or on
@@ -1014,7 +1017,7 @@ extern "C" int umb_seq_linear_split(const void* x, const void* w, int T, int N, 
   if (T > 64) return eb == 2 && N >= 128 && tile_ok(nullptr, x, w, T, N, K, EPI_F32) ? tile_slabs(T, N, K, stream && stream_pays(T, N, K, EPI_F32, 1, eb)) : 1;
   if (!stream) return 1;
   const int parts = std::min(std::min(512 / blocks, 4), chunks / 4);
-  return parts < 2 || (parts == 2 && blocks > 128 && T <= 32) ? 1 : parts;
+  return parts < 2 || (parts == 2 && blocks > 128) ? 1 : parts;
 }
 
 extern "C" int umb_seq_linear_parts(float* out, const void* x, const void* w, const void* bias, int T, int N, int K, int parts, int dtype,

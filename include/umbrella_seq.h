@@ -61,7 +61,7 @@ int umb_seq_linear(void* out, const void* x, const void* w, const void* bias, in
 
 /* A product whose K is summed in `parts` slabs: out fp32 [parts][T][N], the sum over the slabs is the result (bias in the first one's).  Up to 64
  * tokens whole 512-byte chunks of K, beyond them 16-bit storage and K % 64 == 0; 16-byte aligned operands.  umb_seq_linear_split: the number of
- * slabs that pays for these operands (1 .. 4; 1: umb_seq_linear; no stream). */
+ * slabs that pays for these operands (1 .. 4; 1: umb_seq_linear; no stream); slabs times tokens are at most 8192 beyond one slab. */
 int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype);
 int umb_seq_linear_parts(float* out, const void* x, const void* w, const void* bias, int T, int N, int K, int parts, int dtype,
                          umb_stream_t stream);
@@ -584,7 +584,8 @@ typedef struct UmbSeqWork {
   void* moe_act;      /* [pairs][max expert_ff] dtype */
   float* moe_y;       /* [pairs][W] fp32 */
   int32_t moe_max_tiles;
-  int32_t y_rows;      /* rows of W floats in y, and in y2 where there is one: room for the slabs of split products (0: no slabs) */
+  int32_t y_rows;      /* rows of W floats in y, and in y2 where there is one: room for the slabs of split products.  max(Tmax, min(4 Tmax, 8192))
+                          hold them all; where slabs do not fit a product is summed whole (0: everywhere; parallel blocks never split) */
   int64_t aux_floats;  /* floats in aux (what a step does not use of it serves as scratch) */
   void* h2;            /* parallel blocks: normed input of the feed-forward [Tmax][W] dtype */
   float* y2;           /* parallel blocks: feed-forward output; mixers with two output projections: the second [Tmax][W] fp32 */

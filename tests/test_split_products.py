@@ -36,6 +36,20 @@ def test_up_to_64_tokens_the_number_of_slabs_follows_from_the_weights():
                 assert len({split(ptr, ptr, T, N, K, code) for T in range(1, 65)}) == 1, (N, K)
 
 
+def test_slabs_fit_the_room_that_a_workspace_has():
+    """the number of slabs follows from the step and not from the workspace that earlier steps left: what pays among those that fit"""
+    from umbrella_amd import _lib
+    split = _lib.load_seq().umb_seq_linear_split
+    ptr, seen = 1 << 20, set()
+    for T in (1, 64, 65, 300, 2047, 2048, 2049, 2300, 2730, 2731, 4000, 4096, 4097, 6000, 8192, 8193, 20000):
+        for N in (128, 1024, 2048, 4096, 8192):
+            for K in (512, 2048, 4096, 8192, 14336):
+                parts = split(ptr, ptr, T, N, K, _lib.BF16)
+                assert parts * T <= max(T, min(4 * T, 8192)), (T, N, K, parts)
+                seen.add((T, parts))
+    assert (2049, 3) in seen and (2731, 2) in seen and (4096, 2) in seen
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("T,N,chunks,parts", [(1, 16, 2, 2), (1, 2048, 8, 2), (16, 40, 7, 3), (17, 2049, 5, 4), (33, 4096, 16, 2), (48, 130, 32, 4),

@@ -992,6 +992,8 @@ extern "C" int umb_seq_linear(void* out, const void* x, const void* w, const voi
 // reading the slabs beyond the first in the kernel behind it (8 TB/s, they come from the last-level cache), against the whole K on the tiles or on
 // the streaming kernel (0.50 us a chunk and round of 16 rows x 64 tokens a workgroup, 0.78 of 32).  us, whole / this: 4096 x 14336 at 100 / 300 / 1101 /
 // 1999 tokens 46 / 95 / 171 / 198 -> 33 / 52 / 121 / 178; 2048 x 8192 at 128 / 300 / 1101 20.9 / 47 / 62 -> 20.9 / 22 / 42; 4096 x 4096 at 1101 53 -> 42.
+// Their number follows from the tokens and the weights and not from the room that a caller happens to have: at most SLAB_ROWS rows of partial sums.
+constexpr int SLAB_ROWS = 8192;
 static int tile_slabs(int T, int N, int K, bool stream) {
   double best = 1e30, us = 0.0;
   if (tiles_pay(T, N, stream)) {
@@ -1002,7 +1004,7 @@ static int tile_slabs(int T, int N, int K, bool stream) {
     best = 2.5 + (wgs + 255) / 256 * (K / 256) * (narrow ? 0.50 : 0.78);
   }
   int best_s = 1;
-  for (int S = 2; S <= 4 && S * 4 <= K / 64; ++S) {
+  for (int S = 2; S <= 4 && S * 4 <= K / 64 && S <= SLAB_ROWS / T; ++S) {
     (void)tile_kind(T, N, (K / 64 + S - 1) / S, S, K % (128 * S) == 0, &us);
     us += (S - 1) * (double)T * N * 4 / 8e6;
     if (us < best) { best = us; best_s = S; }

@@ -34,7 +34,8 @@ static inline int lin(const UmbSeqLinear& l, void* out, const void* x, int T, in
   return umb_seq_linear(out, x, l.w, l.bias, T, l.N, l.K, epi, dtype, st);
 }
 
-// a sublayer's last product, summed in slabs where that pays and the seam behind it adds them (*parts; null: it does not)
+// a sublayer's last product, summed in slabs where that pays and the seam behind it adds them (*parts; null: it does not).  A workspace with less
+// than the documented room gets whole sums where slabs do not fit
 static int lin_y(const UmbSeqLinear& l, float* y, const UmbSeqWork* ws, const void* x, int T, int* parts, int dtype, hipStream_t st) {
   int n = parts ? umb_seq_linear_split(x, l.w, T, l.N, l.K, dtype) : 1;
   if ((long)n * T > ws->y_rows) n = 1;

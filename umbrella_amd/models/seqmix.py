@@ -423,7 +423,8 @@ class SeqMixLM(LLMBase):
             elif ly.ff:
                 ask(act=ly.ff, proj=ly.ff if ly.ff_kind == "polynorm" else 1)
         f32, i32 = torch.float32, torch.int32
-        y_rows = max(T, min(4 * T, 8192))               # products leave up to four slabs of partial sums
+        # products leave up to four slabs of partial sums, 8192 rows of them at most: y and y2 have room for all (parallel blocks take whole sums)
+        y_rows = T if c.block == "parallel" else max(T, min(4 * T, 8192))
         b = self._bufs = dict(
             x=torch.zeros(T, max(1, c.streams) * c.width, dtype=f32, device=dev), h=torch.zeros(T, c.width, dtype=dt, device=dev),
             proj=torch.zeros(T, need["proj"], dtype=f32, device=dev), aux=torch.zeros(T, need["aux"], dtype=f32, device=dev),

@@ -219,3 +219,22 @@ def test_forwards_in_slabs(kind, dtype):
             # fp32 sums in another order; 16 bits: a rounding of 2^-9 that falls the other way in some of a few dozen places of a layer
             assert (got - want).norm() <= (2e-5 if dtype == "fp32" else 2e-2) * want.norm(), (kind, lens)
         assert T > 64 and dtype == "fp32" or not torch.equal(runs[0][-1], runs[1][-1])        # sums in slabs they were
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["groups", "pair", "one stream"])
+def test_a_workspace_of_single_floats(kind):
+    """outputs of a sublayer that are not 16-byte aligned: whole sums, as a product without slabs takes them"""
+    m, _ = _split_models()[kind](torch.bfloat16, max_length=700)
+    m.reserve(600)
+    g, runs = torch.Generator().manual_seed(4), []
+    ids = torch.randint(0, 90, (600,), generator=g).tolist()
+    for off in (0, 1):
+        bufs = [torch.full((4 * 600 * 1024 + 4,), 5.0, device="cuda") for _ in range(2)]
+        m._ws.y, m._ws.y2 = (b.data_ptr() + 4 * off for b in bufs)
+        m.clear()
+        m.open(0)
+        runs.append(m.forward_batch([(0, ids)]).double().clone())
+        assert all(bool((b[:off] == 5.0).all()) and bool((b[off + 4 * 600 * 1024:] == 5.0).all()) for b in bufs)
+    # a rounding of 2^-9 that falls the other way in some of a few dozen places of a layer
+    assert (runs[0] - runs[1]).norm() <= 2e-2 * runs[0].norm()

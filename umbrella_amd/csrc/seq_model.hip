@@ -35,10 +35,10 @@ static inline int lin(const UmbSeqLinear& l, void* out, const void* x, int T, in
 }
 
 // a sublayer's last product, summed in slabs where that pays and the seam behind it adds them (*parts; null: it does not).  A workspace with less
-// than the documented room gets whole sums where slabs do not fit
+// than the documented room gets whole sums where slabs do not fit, one that is not 16-byte aligned everywhere (many tokens' slabs leave as 16-byte stores)
 static int lin_y(const UmbSeqLinear& l, float* y, const UmbSeqWork* ws, const void* x, int T, int* parts, int dtype, hipStream_t st) {
   int n = parts ? umb_seq_linear_split(x, l.w, T, l.N, l.K, dtype) : 1;
-  if ((long)n * T > ws->y_rows) n = 1;
+  if ((long)n * T > ws->y_rows || (uintptr_t)y % 16) n = 1;
   if (parts) *parts = n;
   return n > 1 ? umb_seq_linear_parts(y, x, l.w, l.bias, T, l.N, l.K, n, dtype, st) : lin(l, y, x, T, 0, dtype, st);
 }

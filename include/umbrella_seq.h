@@ -63,6 +63,8 @@ int umb_seq_linear(void* out, const void* x, const void* w, const void* bias, in
  * tokens whole 512-byte chunks of K, beyond them 16-bit storage and K % 64 == 0; 16-byte aligned operands.  umb_seq_linear_split: the number of
  * slabs that pays for these operands (1 .. 4; 1: umb_seq_linear; no stream); slabs times tokens are at most 8192 beyond one slab. */
 int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype);
+/* the staged tile (csrc/gemm_tile.h's TILE_*) of a product of T tokens and `rows` rows of W whose K is summed in slabs (no stream) */
+int umb_seq_tile_kind(int T, int rows, int K, int slabs);
 int umb_seq_linear_parts(float* out, const void* x, const void* w, const void* bias, int T, int N, int K, int parts, int dtype,
                          umb_stream_t stream);
 

@@ -3,19 +3,34 @@ and one by one, with K of one stage, fewer stages than the ring has slots, and m
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
-
 # (T, N, K) of single matrices by the tile that they get; N % 8 == 0, N % 4 == 0 and odd
-SHAPES = [(1600, 8184, 64), (2049, 6145, 320), (2049, 6148, 192),               # 256 x 256
-          (1300, 6145, 128), (1300, 8188, 64), (2300, 8184, 192),               # 256 x 192
-          (900, 8184, 64), (1101, 8190, 192), (2049, 8188, 320),                # 256 x 160
-          (1101, 6152, 192), (1300, 5001, 128), (2300, 2592, 320),              # 256 x 128
-          (257, 6148, 64), (257, 8184, 320), (2300, 2050, 192),                 # 256 x 96
-          (257, 200, 64), (300, 1001, 192), (1000, 1028, 320),                  # 128 x 128
-          (257, 2048, 128), (300, 1004, 384), (2049, 129, 128)]                 # 128 x 64
+TILES = ["256", "192", "160", "128 wide", "96", "128", "64 split"]          # csrc/gemm_tile.h, in its order
+SHAPES = [(*shape, tile) for tile, shapes in {
+    "256": [(1600, 8184, 64), (2049, 6145, 320), (2049, 6148, 192)],                                  # 256 rows x 256 tokens
+    "192": [(1300, 6145, 128), (1300, 8188, 64), (2300, 5124, 320)],
+    "160": [(2300, 8184, 192), (900, 8184, 64), (1101, 8190, 192), (2049, 8188, 320)],
+    "128 wide": [(1101, 6152, 192), (1300, 5001, 128), (2300, 2592, 320)],
+    "96": [(257, 6148, 64), (1025, 4112, 320), (2300, 2050, 192)],
+    "128": [(257, 8184, 320), (257, 200, 64), (300, 1001, 192), (1000, 1028, 320)],                   # 128 x 128
+    "64 split": [(257, 2048, 128), (300, 1004, 384), (2049, 129, 128)]}.items() for shape in shapes]  # 128 x 64, K over two groups of waves
+# packed weights: (T, N, K, S), K in slabs of one stage, of an even and an odd number, and a slab past the last stage
+PACKED = [(1600, 8176, 128, 1, "256"), (1300, 6160, 128, 1, "192"), (900, 8176, 128, 1, "160"), (1101, 6160, 128, 1, "128 wide"),
+          (257, 8176, 128, 1, "96"), (1025, 4112, 384, 1, "96"), (257, 6160, 128, 1, "64 split"), (300, 1008, 640, 3, "128"),
+          (1300, 5008, 384, 4, "192"), (257, 2048, 256, 2, "64 split"), (300, 1008, 128, 2, "128")]
 
 
-@pytest.mark.parametrize("T,N,K", SHAPES)
+def test_shapes_get_the_tiles_they_are_listed_for():
+    from umbrella_amd import _lib
+    kind = _lib.load_seq().umb_seq_tile_kind
+    for *shape, tile in SHAPES:
+        assert TILES[kind(*shape, 1)] == tile, shape
+    for *shape, tile in PACKED:
+        assert TILES[kind(*shape)] == tile, shape
+    assert {s[-1] for s in SHAPES} == {s[-1] for s in PACKED} == set(TILES)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,N,K", [s[:3] for s in SHAPES])
 def test_every_tile(T, N, K):
     from umbrella_amd import _lib
     dtype = torch.bfloat16 if K % 128 else torch.float16
@@ -39,9 +54,8 @@ def test_every_tile(T, N, K):
     assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())
 
 
-# packed weights: the same tiles, K in slabs of one stage, of an even and an odd number, and a slab past the last stage
-@pytest.mark.parametrize("T,N,K,S", [(1600, 8176, 128, 1), (1300, 6160, 128, 1), (900, 8176, 128, 1), (1101, 6160, 128, 1), (257, 6160, 128, 1),
-                                     (300, 1008, 640, 3), (1300, 5008, 384, 4), (257, 2048, 256, 2), (300, 1008, 128, 2)])
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,N,K,S", [s[:4] for s in PACKED])
 def test_every_tile_of_packed_weights(T, N, K, S):
     from umbrella_amd import _lib
     from umbrella_amd.models.llama import PackedLinear
@@ -64,6 +78,7 @@ def test_every_tile_of_packed_weights(T, N, K, S):
     assert ((act[:T].double() - want).abs() <= bound).all() and bool((act[T] == 7.0).all())
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 300])
 @pytest.mark.parametrize("epi", [2, 6])
 def test_gates_far_from_zero(T, epi):
@@ -88,6 +103,7 @@ def test_gates_far_from_zero(T, epi):
 
 # per-head products on tiles (96 of them and more) and just below, ragged tokens and rows, one stage and several, row strides beyond the row; outputs
 # whose rows are no whole 16-byte groups stay where they were
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,T,N,K,pad", [(32, 385, 128, 64, 8), (7, 900, 200, 192, 0), (50, 257, 72, 320, 24), (12, 1024, 64, 128, 8), (24, 500, 130, 64, 2)])
 def test_batched_tiles(dtype, B, T, N, K, pad):
@@ -119,6 +135,7 @@ def test_batched_tiles(dtype, B, T, N, K, pad):
 GATES = [0.0, -0.0, 1e-38, 5.0, 88.5, 200.0, 3e38, float("inf"), -86.9, -87.4, -88.0, -88.6, -89.0, -100.0, -200.0, -3e38, float("-inf"), float("nan")]
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype,T", [(torch.float32, 1), (torch.float32, 300), (torch.bfloat16, 300)])
 def test_gates_to_the_ends_of_their_range(dtype, T):
     """silu(gate) * up of the biases alone: the products are zero"""
@@ -139,6 +156,7 @@ def test_gates_to_the_ends_of_their_range(dtype, T):
     assert torch.equal(got[ok].isinf(), want[ok].isinf()) and ((got - want).abs() <= bound)[ok & ~want.isinf()].all()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("epi", [3, 7])
 def test_batched_gates_to_the_ends_of_their_range(epi):
     """the gate of a per-head product on tiles: a gate that is no number is seen in the result"""

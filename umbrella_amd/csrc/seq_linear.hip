@@ -1012,6 +1012,11 @@ static int tile_slabs(int T, int N, int K, bool stream) {
   return best_s;
 }
 
+extern "C" int umb_seq_tile_kind(int T, int rows, int K, int slabs) {
+  if (T < 1 || rows < 1 || K < 64 || slabs < 1) return UMB_EINVAL;
+  return tile_kind(T, rows, (K / 64 + slabs - 1) / slabs, slabs, K % (128 * slabs) == 0);
+}
+
 extern "C" int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype) {
   if (T < 1 || N < 1 || K < 1) return 1;
   const int eb = (int)seq_elem_bytes(dtype), chunks = (int)((long)K * eb / 512), blocks = (N + 15) / 16;

@@ -83,7 +83,7 @@ template <typename P> __device__ __forceinline__ void st4(typename El<P>::type* 
 // y holds this thread's quads of slab 0; the others' are added in order, their loads all in flight.
 constexpr int PARTS_MAX = 4;
 template <int NE, typename Off> __device__ __forceinline__ void add_parts(f32x4 (&y)[NE], const float* __restrict__ src, int parts, long slab, Off off) {
-  if (parts == 1) return;
+  if (parts == 1) return;                            // (the other output of a pair)
   f32x4 a[NE], b[NE], c[NE];
 #pragma unroll
   for (int e = 0; e < NE; ++e) {

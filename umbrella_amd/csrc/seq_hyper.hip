@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void hc_embed_kernel(float* __restrict__ x, ty
 // One stream, rows in quads: a workgroup of NT threads, NE quads per thread, every load issued before the first use (the reasons are
 // those of seq_norm.hip's quad kernels).  48 x 2048, 16-bit weights: seam 6.0 -> 4.5 us, embedding 8.2 -> 4.6;
 // 1999 x 4096: seam 18.7 -> 12.7.
-template <typename P, int NT, int NE>
+template <typename P, int NT, int NE, bool SLABS>
 __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x, typename El<P>::type* __restrict__ h, const float* __restrict__ y,
                                                           const float* __restrict__ mix, const float* __restrict__ out, float m,
                                                           const float* __restrict__ in_next, const typename El<P>::type* __restrict__ w_next,
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x,
   const long o = (long)blockIdx.x * W;
   const int nq = W / 4;
   const float mx = mix ? mix[0] : 1.f, ot = out ? out[0] : 1.f, in0 = in_next ? in_next[0] : 1.f;
-  // read either way (without a next norm from the row's first slab): behind a test the load is a round trip of its own
+  // one quad a thread: read either way (without a next norm from the row's first slab), as in resid_norm_quad_kernel
   const typename El<P>::type* wq = w_next ? w_next : reinterpret_cast<const typename El<P>::type*>(y);
   f32x4 xv[NE], yv[NE], wn[NE];
 #pragma unroll
@@ -242,9 +242,9 @@ __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x,
     const int i = min((int)threadIdx.x + NT * e, nq - 1) * 4;
     xv[e] = *reinterpret_cast<const f32x4*>(x + o + i);
     yv[e] = *reinterpret_cast<const f32x4*>(y + o + i);
-    wn[e] = ld4<P>(wq + i);
+    wn[e] = NE == 1 || w_next ? ld4<P>(wq + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  add_parts<NE>(yv, y, parts, slab, [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; });
+  if constexpr (SLABS) add_parts<NE>(yv, y, parts, slab, [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; });
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
@@ -348,11 +348,19 @@ extern "C" int umb_hc_seam_parts(float* x, void* h, float* y, int parts, const f
   if (T < 1 || W < 1 || S < 1 || S > HC_MAXS || !x || !y || (w_next && !h) || parts < 1 || parts > PARTS_MAX) return UMB_EINVAL;
   const long slab = (long)T * W;
   if (S == 1 && quads_ok(W, 1, x, h, y, w_next)) {
-#define HC_SEAM_QUADS(NT, NE)                                                                                                       \
-  hipLaunchKernelGGL((hc_seam_quad_kernel<P, NT, NE>), dim3(T), dim3(NT), 0, st, x, (E*)h, y, mix, out, m, in_next, (const E*)w_next, offset, W, eps, \
-                     parts, slab)
-    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, (long)T, HC_SEAM_QUADS); })
+#define HC_SEAM_AS(NT, NE, SLABS)                                                                                                   \
+  hipLaunchKernelGGL((hc_seam_quad_kernel<P, NT, NE, SLABS>), dim3(T), dim3(NT), 0, st, x, (E*)h, y, mix, out, m, in_next, (const E*)w_next, \
+                     offset, W, eps, parts, slab)
+#define HC_SEAM_QUADS(NT, NE) HC_SEAM_AS(NT, NE, false)
+#define HC_SEAM_SLABS(NT, NE) HC_SEAM_AS(NT, NE, true)
+    DISPATCH_SEQ_DTYPE(dtype, {
+      typedef typename El<P>::type E;
+      if (parts == 1) BY_QUADS(W, (long)T, HC_SEAM_QUADS);
+      else BY_QUADS(W, (long)T, HC_SEAM_SLABS);
+    })
+#undef HC_SEAM_SLABS
 #undef HC_SEAM_QUADS
+#undef HC_SEAM_AS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
   }

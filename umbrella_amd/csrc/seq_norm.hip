@@ -321,7 +321,9 @@ __global__ __launch_bounds__(256) void pair_resid_norm_kernel(float* __restrict_
 // 1024, 256 threads beyond) remain for groups that are no multiple of four, longer than 8192, or unaligned (loads and stores: seq_common.h).
 // us of a decode step's launch, one MI355X, 16-bit weights: seam 1 x 4096 10.5 -> 4.8, 16 x 4 x 1024 9.8 -> 5.2; embedding 1 x 4096
 // 40 -> 3.7; final norm 1 x 4096 11.2 -> 4.7; pair seam 1 x 4096 11.7 -> 5.9; of a 2000-token prompt 12.4 -> 8.2 (4 x 512), 10.7 -> 8.9 (2048).
-template <typename P, int NT, int NE>
+// SLABS: the sublayer's output in `parts` slabs.  A variant of its own: the registers of three slabs a quad cost whole outputs of long rows an eighth and
+// more of their time (fp32 weights, 1000 x 4096 / 8192: 9.6 / 20.4 us, 11.9 / 25.6 with a test of `parts`).
+template <typename P, int NT, int NE, bool SLABS>
 __global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__ x, typename El<P>::type* __restrict__ h,
                                                              const float* __restrict__ y, const typename El<P>::type* __restrict__ w_post,
                                                              const typename El<P>::type* __restrict__ w_next, int W, int groups, float eps,
@@ -329,7 +331,8 @@ __global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__
   __shared__ float red[NT / 64], red2[NT / 64];
   const int grp = blockIdx.y, gs = W / groups, nq = gs / 4;
   const long o = (long)blockIdx.x * W + (long)grp * gs;
-  const typename El<P>::type* wq = w_next ? w_next : w_post;   // read either way: behind a test the load is a round trip of its own
+  // one quad a thread (few rows): read either way, behind a test the load is a round trip of its own; more of them (many rows): only if it is wanted
+  const typename El<P>::type* wq = w_next ? w_next : w_post;
   f32x4 yv[NE], xv[NE], wp[NE], wn[NE];
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
@@ -337,9 +340,9 @@ __global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__
     yv[e] = *reinterpret_cast<const f32x4*>(y + o + i);
     xv[e] = *reinterpret_cast<const f32x4*>(x + o + i);
     wp[e] = ld4<P>(w_post + grp * gs + i);
-    wn[e] = ld4<P>(wq + grp * gs + i);
+    wn[e] = NE == 1 || w_next ? ld4<P>(wq + grp * gs + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  add_parts<NE>(yv, y, parts, slab, [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; });
+  if constexpr (SLABS) add_parts<NE>(yv, y, parts, slab, [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; });
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) ss += (int)threadIdx.x + NT * e < nq ? sq4(yv[e]) : 0.f;
@@ -397,7 +400,7 @@ __global__ __launch_bounds__(NT) void norm_quad_kernel(float* __restrict__ out_f
   }
 }
 
-template <typename P, int NT, int NE>
+template <typename P, int NT, int NE, bool SLABS>
 __global__ __launch_bounds__(NT) void pair_resid_norm_quad_kernel(float* __restrict__ x, typename El<P>::type* __restrict__ h,
                                                                   const float* __restrict__ y1, const float* __restrict__ y2,
                                                                   const typename El<P>::type* __restrict__ w1,
@@ -419,11 +422,13 @@ __global__ __launch_bounds__(NT) void pair_resid_norm_quad_kernel(float* __restr
     wa[e] = ld4<P>(w1 + i);
     wb[e] = ld4<P>(w2 + i);
     wp[e] = ld4<P>(w_post + i);
-    wn[e] = ld4<P>(wq + i);
+    wn[e] = NE == 1 || w_next ? ld4<P>(wq + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  const auto at = [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; };
-  add_parts<NE>(a, y1, parts1, slab, at);
-  add_parts<NE>(b, y2, parts2, slab, at);
+  if constexpr (SLABS) {
+    const auto at = [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; };
+    add_parts<NE>(a, y1, parts1, slab, at);
+    add_parts<NE>(b, y2, parts2, slab, at);
+  }
   float sa = 0.f, sb = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
@@ -527,11 +532,19 @@ extern "C" int umb_seq_resid_norm_parts(float* x, void* h, float* y, int parts, 
   if (!norm_args_ok(T, W, groups) || !x || !y || !w_post || (w_next && !h) || parts < 1 || parts > PARTS_MAX) return UMB_EINVAL;
   const long slab = (long)T * W;
   if (quads_ok(W, groups, x, h, y, w_post, w_next) && (parts == 1 || W % 4 == 0)) {
-#define SEAM_QUADS(NT, NE)                                                                                                      \
-  hipLaunchKernelGGL((resid_norm_quad_kernel<P, NT, NE>), dim3(T, groups), dim3(NT), 0, st, x, (E*)h, y, (const E*)w_post, (const E*)w_next, \
-                     W, groups, eps, parts, slab)
-    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W / groups, (long)T * groups, SEAM_QUADS); })
+#define SEAM_AS(NT, NE, SLABS)                                                                                                  \
+  hipLaunchKernelGGL((resid_norm_quad_kernel<P, NT, NE, SLABS>), dim3(T, groups), dim3(NT), 0, st, x, (E*)h, y, (const E*)w_post, \
+                     (const E*)w_next, W, groups, eps, parts, slab)
+#define SEAM_QUADS(NT, NE) SEAM_AS(NT, NE, false)
+#define SEAM_SLABS(NT, NE) SEAM_AS(NT, NE, true)
+    DISPATCH_SEQ_DTYPE(dtype, {
+      typedef typename El<P>::type E;
+      if (parts == 1) BY_QUADS(W / groups, (long)T * groups, SEAM_QUADS);
+      else BY_QUADS(W / groups, (long)T * groups, SEAM_SLABS);
+    })
+#undef SEAM_SLABS
 #undef SEAM_QUADS
+#undef SEAM_AS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
   }
@@ -603,11 +616,19 @@ extern "C" int umb_seq_pair_resid_norm_parts(float* x, void* h, float* y1, int p
     return UMB_EINVAL;
   const long slab = (long)T * W;
   if (quads_ok(W, 1, x, h, y1, y2, w1, w2, w_post) && (uintptr_t)w_next % 16 == 0) {
-#define PAIR_QUADS(NT, NE)                                                                                                          \
-  hipLaunchKernelGGL((pair_resid_norm_quad_kernel<P, NT, NE>), dim3(T), dim3(NT), 0, st, x, (E*)h, y1, y2, (const E*)w1, (const E*)w2, coef, \
-                     (const E*)w_post, (const E*)w_next, W, eps, parts1, parts2, slab)
-    DISPATCH_SEQ_DTYPE(dtype, { typedef typename El<P>::type E; BY_QUADS(W, (long)T, PAIR_QUADS); })
+#define PAIR_AS(NT, NE, SLABS)                                                                                                      \
+  hipLaunchKernelGGL((pair_resid_norm_quad_kernel<P, NT, NE, SLABS>), dim3(T), dim3(NT), 0, st, x, (E*)h, y1, y2, (const E*)w1, (const E*)w2, \
+                     coef, (const E*)w_post, (const E*)w_next, W, eps, parts1, parts2, slab)
+#define PAIR_QUADS(NT, NE) PAIR_AS(NT, NE, false)
+#define PAIR_SLABS(NT, NE) PAIR_AS(NT, NE, true)
+    DISPATCH_SEQ_DTYPE(dtype, {
+      typedef typename El<P>::type E;
+      if (parts1 == 1 && parts2 == 1) BY_QUADS(W, (long)T, PAIR_QUADS);
+      else BY_QUADS(W, (long)T, PAIR_SLABS);
+    })
+#undef PAIR_SLABS
 #undef PAIR_QUADS
+#undef PAIR_AS
     UMB_LAUNCH_CHECK();
     return UMB_OK;
   }

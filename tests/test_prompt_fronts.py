@@ -17,10 +17,15 @@ def _steps(lens, first, dev="cuda"):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("taps", [3, 4])
 @pytest.mark.parametrize("Hk,H,D,E", [(2, 4, 24, 40), (1, 1, 128, 128), (3, 3, 100, 300), (2, 2, 132, 8), (1, 2, 256, 64), (8, 16, 128, 128)])
-def test_delta_fronts(dtype, taps, Hk, H, D, E):
+@pytest.mark.parametrize("many", [False, True])              # a wave each, and enough of them for quads
+def test_delta_fronts(dtype, taps, Hk, H, D, E, many):
     from umbrella_amd import _lib
     lens, first = [1, 9, 2, 17, 8, 3, 1], [0, 5, 1, 0, 2, 40, 3]
-    T, C, Dp = sum(lens), 2 * Hk * D + H * E, (D + 15) // 16 * 16
+    C, Dp = 2 * Hk * D + H * E, (D + 15) // 16 * 16
+    if many:
+        n = min(1200000 // C + 1, 20000 // (2 * Hk + H + 1) + 1)
+        lens, first = lens + [n // 2 + 3, 5, n // 2], first + [0, 7, 2]
+    T = sum(lens)
     pos, slot = _steps(lens, first)
     g = torch.Generator(device="cuda").manual_seed(D + E + taps)
     cols = C + H * E + 2 * H

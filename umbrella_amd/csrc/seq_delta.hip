@@ -262,7 +262,7 @@ __device__ __forceinline__ f32x4 mma4(f32x4 a, f32x4 b, f32x4 c) {
 // (1) grid (chunks, value heads, sequences).  One chunk is a chain: prefix sums, k . k, four inverses, sixteen solves.  Eight waves, K alone in
 // LDS and two workgroups a unit: q . k, which nothing waits for, is read from memory and runs beside the inverses.  Every load that depends on
 // nothing but the chunk leaves long before its use, NK (>= Dp / 16) of a kind at once: k, the wave's part of q and the decays at the start, its
-// values before the inverses.  In loops of In loops of a run-time count they came one by one, a round trip each.
+// values before the inverses.  In loops of a run-time count they came one by one, a round trip each.
 // 2466 tokens in five stretches, 16 heads of 128: 73 us -> 44; 61 tokens, 32 heads 25 -> 16.
 template <int NK>
 __global__ __launch_bounds__(512, NK <= 8 ? 4 : 2) void delta_chunk_solve_kernel(DeltaChunk a) {
@@ -638,7 +638,13 @@ extern "C" int umb_delta_prep(float* q, float* k, int ldqk, float* v, float* bet
     return UMB_EINVAL;
   const DeltaIn in{proj, ld, col0, Hk, H, D, E, taps, ring, dt_bias, a_log};
   const long items = (long)T * (2 * Hk + H + 1);
-  if ((taps == 3 || taps == 4) && D % 4 == 0 && E % 4 == 0 && ld % 4 == 0 && col0 % 4 == 0 && ldqk % 4 == 0 &&
+  // Quads from 1.2 million channels or 20000 slots on: a wave of eight tokens is a chain of some 9 us, in which fewer are long done a wave each.  us, a wave
+  // a slot / quads, 4 taps, 16-bit weights: 8 + 8 + 16 slots of 128, 48 / 195 / 317 / 488 / 2441 tokens 5.6 / 7.9 / 10.7 / 14.0 / 66 against 9.3 / 9.6 / 9.9 / 10.7 /
+  // 25; 4 + 4 + 4 of 64, 260 / 1041 / 1692 / 6510 tokens 4.8 / 8.7 / 14.3 / 45 against 9.3 / 9.7 / 10.9 / 22; 2 + 2 + 4 of 256, 97 / 634 / 976 7.3 / 12.7 / 22.7 against
+  // 9.7 / 10.5 / 11.8; 3 taps, 2 + 2 + 4 of 24 and 40, 1562 / 2343 / 3125 7.9 / 10.3 / 12.6 against 9.0 / 9.9 / 10.0.  Up to 64 tokens a token's sums are
+  // the same whatever else is in its step.
+  const bool many = T > 64 && (T * (2L * Hk * D + (long)H * E) >= 1200000 || items >= 20000);
+  if (many && (taps == 3 || taps == 4) && D % 4 == 0 && E % 4 == 0 && ld % 4 == 0 && col0 % 4 == 0 && ldqk % 4 == 0 &&
       ((uintptr_t)proj | (uintptr_t)ring | (uintptr_t)conv_w | (uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16 == 0) {
 #define DELTA_QUADS(TAPS, LPS)                                                                                                          \
   do {                                                                                                                                  \

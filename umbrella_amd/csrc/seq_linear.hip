@@ -488,8 +488,9 @@ static int launch_tile_as(void* out, const void* x, const void* w, const void* b
 
 // ---- many tokens of a batch of small problems (per-head products): the same main loop, rows with strides of their own, 128 x 128 tiles of four
 // waves, two workgroups a CU: K is a few stages, and one's stores run beside the other's products.  us, 64 x 64 tiles from L2 / this, bf16:
-// 32 heads, fp32 out 512 x 128 at 128 / 400 / 1999 tokens 8.1 / 22.8 / 83 -> 5.9 / 9.1 / 29 (147 MB out), gated 128 x 512 6.9 / 16.7 / 58 -> 9.7 / 10.5 / 21;
-// 16 heads 256 x 64 at 256 / 1101 5.7 / 15.9 -> 5.9 / 7.7, gated 64 x 256 at 400 / 1101 6.5 / 12.1 -> 8.4 / 8.5.  So from 96 tiles on.
+// 32 heads, fp32 out 512 x 128 at 128 / 400 / 1999 tokens 8.1 / 22.8 / 83 -> 5.9 / 9.1 / 29 (147 MB out), a gate per output 128 x 512 at
+// 300 / 2048 19.7 / 64 -> 11.2 / 24; 16 heads 256 x 64 at 256 / 1101 5.7 / 15.9 -> 5.9 / 7.7, gated 64 x 256 at 700 / 2048 10.6 / 14.0 -> 9.5 / 9.9.  So from 96
+// tiles on.
 template <typename P>
 __global__ __launch_bounds__(256, 2) void seq_linear_tile_batched_kernel(void* __restrict__ out_, const u16* __restrict__ x, const u16* __restrict__ w,
                                                                           int T, int N, int K, int epi, int nbt, int nbn, LinExt ext) {
@@ -512,6 +513,22 @@ __global__ __launch_bounds__(256, 2) void seq_linear_tile_batched_kernel(void* _
   const long obase = z * ext.so;
   const float* gate = ext.gate ? ext.gate + (long)z * ext.sg : nullptr;
   const unsigned strip = (unsigned)(size_t)(lds_char*)smem + (unsigned)wave * TileRows<16, RA>::BYTES;
+  // the gates of all outputs are asked for at once, four (N % 4 == 0 here) or a row's one for all: fetched one by one in front of their quotients they were
+  // four round trips of 16 loads, and up to a few hundred tiles the 64 x 64 ones were ahead (us, gate per output, those / one by one / at once: 16 x (256 x 64),
+  // 300 tokens 9.8 / 14.0 / 8.5; 32 x (512 x 128), 128 tokens 11.6 / 14.8 / 9.2, 2048 168 / 82 / 49; 64 x (64 x 64), 256 tokens 9.5 / 13.7 / 8.5)
+  typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
+  f32x4 gv[RB][RA];
+  if (gate) {
+#pragma unroll
+    for (int t = 0; t < RB; ++t) {
+      const float* gr = gate + (long)min(t0 + (wn * RB + t) * 16 + j, T - 1) * ext.ldg;
+#pragma unroll
+      for (int i = 0; i < RA; ++i) {
+        if (epi == EPI_GATE_ROW) gv[t][i] = i ? gv[t][0] : f32x4{gr[0], gr[0], gr[0], gr[0]};
+        else gv[t][i] = *reinterpret_cast<const quad*>(gr + min(nw + i * 16 + 4 * g, N - 4));
+      }
+    }
+  }
 #pragma unroll
   for (int t = 0; t < RB; ++t) {
     const int tile0 = t0 + (wn * RB + t) * 16;
@@ -519,12 +536,10 @@ __global__ __launch_bounds__(256, 2) void seq_linear_tile_batched_kernel(void* _
 #pragma unroll
     for (int i = 0; i < RA; ++i) v[i] = acc[i][t];
     if (gate) {
-      const float* gr = gate + (long)min(tile0 + j, T - 1) * ext.ldg;
-      const float row = epi == EPI_GATE_ROW ? gr[0] : 0.f;
 #pragma unroll
       for (int i = 0; i < RA; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[i][r] = over_one_plus_exp(v[i][r], epi == EPI_GATE_ROW ? row : gr[min(nw + i * 16 + 4 * g + r, N - 1)]);
+        for (int r = 0; r < 4; ++r) v[i][r] = over_one_plus_exp(v[i][r], gv[t][i][r]);
     }
     if (epi == EPI_F32) {
       tile_rows_out<16, RA>(strip, v, [&](int row, int at, u32x4 b) {

@@ -49,11 +49,13 @@ def test_delta_fronts(dtype, taps, Hk, H, D, E, many):
         assert (a - b).abs().max() <= 4e-7 * D ** 0.5
 
 
-# more than 1024 tiles of 16 rows: ragged rows, prefixes around a 64-key step and none, a cache that ends inside one (Lmax an odd multiple of 32),
-# trees and causal prompts, stale keys behind the valid ones
+# more than 1024 tiles of 16 rows, and heads of 64 and 32 also more than 1791 (four waves share the keys of causal prompts from there on; trees have a
+# wave or two a tile): ragged rows, prefixes around a 64-key step and none, a cache that ends inside one (Lmax an odd multiple of 32), stale keys behind
+# the valid ones
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D,Hq,Hkv,T,prefix,spare", [(128, 64, 8, 257, 63, 0), (128, 32, 8, 530, 0, 32), (64, 32, 8, 515, 65, 32), (64, 12, 4, 1400, 1, 0),
-                                                     (32, 32, 32, 529, 130, 96), (32, 40, 8, 430, 0, 32)])
+                                                     (32, 32, 32, 529, 130, 96), (32, 40, 8, 430, 0, 32), (64, 32, 8, 900, 65, 32),
+                                                     (64, 24, 8, 1200, 1, 0), (32, 32, 32, 900, 130, 96), (32, 40, 8, 720, 0, 32)])
 def test_attention_of_many_tiles(dtype, D, Hq, Hkv, T, prefix, spare):
     import numpy as np
     from umbrella_amd.attn.cache import VT_PAD, k_to_frag, vt_to_frag
@@ -90,10 +92,10 @@ def test_attention_of_many_tiles(dtype, D, Hq, Hkv, T, prefix, spare):
         assert bool((out[T] == 3.0).all())
 
 
-@pytest.mark.parametrize("D,Hq,Hkv,T,prefix", [(128, 32, 8, 530, 0), (64, 32, 8, 515, 65), (32, 40, 8, 530, 20)])
+@pytest.mark.parametrize("D,Hq,Hkv,T,prefix", [(128, 32, 8, 530, 0), (64, 32, 8, 900, 65), (32, 40, 8, 720, 20)])
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_values_that_are_not_finite_reach_one_tile_of_keys(D, Hq, Hkv, T, prefix, bad):
-    """prompts of more than 1024 query tiles: a value that a token does not see is weighted with zero inside its tile of 32 keys, and read nowhere else"""
+    """prompts of many query tiles: a value that a token does not see is weighted with zero inside its tile of 32 keys, and read nowhere else"""
     from umbrella_amd.attn.cache import VT_PAD, k_to_frag, vt_to_frag
     from umbrella_amd import _lib
     S, g, dtype = prefix + T, Hq // Hkv, torch.bfloat16

@@ -708,11 +708,14 @@ extern "C" int umb_tree_attn2(void* out, const void* q, const void* k_cache, con
     single_max = one_env > 0 ? one_env : 1024;
     if (single_max < KBK) single_max = KBK;
   }
-  // More than 1024 causal query tiles (prompts; under a tree's mask the order of a row's sums stays the one of recorded continuations, whose near-ties
-  // another one decides otherwise): four waves a compute unit and more, which share their keys (us, a wave each / this: 1032 tiles 32.9 / 25.3, 1024 without a
-  // prefix 12.6 / 13.3, 768 14.1 / 16.5, 520 behind 700 keys 19.1 / 23.5)
+  // Many causal query tiles (prompts; under a tree's mask the order of a row's sums stays the one of recorded continuations, whose near-ties another one
+  // decides otherwise): four waves a compute unit and more, which share their keys.  From 1792 tiles on, where the kernel below goes on with one wave a tile,
+  // it is behind everywhere; heads of 128 from 1025 on, which costs a little without a prefix and gives more behind one.  us, the kernel below / this, behind
+  // 0 / 500 / 1000 keys: heads of 128, 1040 tiles 15.2 / 26.1 / 39.4 against 16.3 / 23.8 / 32.0, 1296 tiles 16.2 / 30.9 / 45.2 against 16.7 / 25.6 / 34.0, 2048
+  // 34.2 / 48.0 / 61.6 against 23.6 / 32.9 / 42.3; of 64, 1040 tiles 10.5 / 15.3 / 20.8 against 12.5 / 17.9 / 23.7, 1536 12.8 / 19.3 / 25.2 against 13.5 / 20.1 / 25.9, 1792
+  // 21.9 / 31.5 / 40.3 against 15.5 / 21.6 / 27.6; of 32, 1536 16.5 / 21.5 / 35.2 against 18.8 / 23.8 / 28.4, 1792 31.6 / 42.2 / 45.3 against 21.5 / 26.5 / 31.1
   static const int nw_env = getenv("UMB_ATTN_NW") ? atoi(getenv("UMB_ATTN_NW")) : 0;
-  if (Hkv * nqt > 1024 && !mask_bits && !nw_env && !no_single && !out_fm_tt && ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)vt_cache | (uintptr_t)out) % 16 == 0) {
+  if (Hkv * nqt >= (D == 128 ? 1025 : 1792) && !mask_bits && !nw_env && !no_single && !out_fm_tt && ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)vt_cache | (uintptr_t)out) % 16 == 0) {
     const dim3 grid(Hkv, (nrows + 63) / 64);
     const int fold = (long)grid.x * grid.y <= 512;
 #define WIDE_(DD)                                                                                                                  \

@@ -499,13 +499,6 @@ __global__ __launch_bounds__(64 * NW, NQ > 1 ? 1 : 2) void tree_attn1_kernel(con
 // (contiguous in the cache's fragment order) go to LDS by LDS-DMA once for the four tiles, one barrier a step; a fragment is read as it lies, a
 // contiguous KiB.  Two workgroups share a CU.  us, one MI355X, a wave each / this: 1024 causal
 // tokens of 32 + 8 heads of 128 behind 0 / 1024 keys 36 / 69 -> 25 / 46, of 64 24 / 42 -> 17 / 29.  32 rows a wave (half the LDS reads, one wave a SIMD): 40 / 69.
-// max over lanes l, l ^ 16, l ^ 32, l ^ 48
-__device__ __forceinline__ float quad_max(float v) {
-  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
 template <typename P, int D>
 __global__ __launch_bounds__(256, 2) void wide_attn_kernel(const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vt,
                                                            const int* __restrict__ prefix_p, int T, int Hq, int Hkv, int Lmax, int n_mask_keys,

@@ -98,20 +98,24 @@ static int dgemm_launch(const void* wp, const u16* x, int ldx, float* out, int T
   return UMB_OK;
 }
 
-// Up to 128 tokens a launch is a round or two of any tile, and what is left to choose is the order in which K is summed: that of recorded
-// greedy continuations behind 96-token prompts, whose near-ties a different rounding of the cached keys would decide otherwise.  Five tiles by
-// rounds x stages, K over two groups of waves where a launch has at most one workgroup per compute unit.
+// Up to 128 tokens what a tile decides besides its time is whether K is split over two groups of waves, and so the order in which K is summed: that of
+// recorded greedy continuations behind 96-token prompts, whose near-ties another rounding of the cached keys would decide otherwise.  So the tiles
+// there are chosen as they were when those were recorded: five of them, by rounds x stages and the stage times of two-slot rings (only their order
+// counts now, the rings are deeper).  128 is where those prompts end, not where another rule begins to pay: by tile_kind the same launches take as
+// long, but for many rows in few rounds (us, this / tile_kind's, 65 / 128 tokens: gate/up 28672 x 4096 63.7 / 65.1 against 50.9 / 60.7, 32000 x 4096 65.9 / 67.5
+// against 56.9 / 60.4, 6144 x 4096 in four slabs 19.4 / 20.4 against 15.8 / 17.5; 4096 x 4096, 4096 x 14336, 3072 x 2048, 2048 x 8192 within 2 %).
+enum { NARROW_256 = 0, NARROW_160 = 1, NARROW_128 = 2, NARROW_128K = 3, NARROW_64K = 4, NARROW_KINDS = 5 };
 static int dgemm_narrow(int T, int N, int K, int S, double* us) {
-  static const struct { int bn, bt; double us; bool ksplit; } kind[5] = {
+  static const struct { int bn, bt; double us; bool ksplit; } kind[NARROW_KINDS] = {
       {256, 256, 1.5, false}, {256, 160, 1.1, false}, {128, 128, 0.52, false}, {128, 128, 0.56, true}, {128, 64, 0.39, true}};
   const bool even = K % (128 * S) == 0;
-  int best = 2;
+  int best = NARROW_128;
   *us = 1e30;
-  for (int i = 0; i < 5; ++i) {
+  for (int i = 0; i < NARROW_KINDS; ++i) {
     const long wgs = (long)((N + kind[i].bn - 1) / kind[i].bn) * ((T + kind[i].bt - 1) / kind[i].bt) * S, rounds = (wgs + 255) / 256;
     if (kind[i].ksplit && (rounds > 1 || !even)) continue;
-    // a lone workgroup of the two-per-CU form (128 x 128) leaves half the wave slots empty
-    const double cost = rounds * ((K / 64 + S - 1) / S) * (i == 2 && rounds == 1 ? 0.62 : kind[i].us) + 4.0;
+    // a lone workgroup of the two-per-CU form leaves half the wave slots empty
+    const double cost = rounds * ((K / 64 + S - 1) / S) * (i == NARROW_128 && rounds == 1 ? 0.62 : kind[i].us) + 4.0;
     if (cost < *us) { *us = cost; best = i; }
   }
   return best;
@@ -125,10 +129,10 @@ static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, i
   if (T <= 128) {
     double us;
     switch (dgemm_narrow(T, N, K, S, &us)) {
-      case 0: return dgemm_launch<P, 4, 2, 4, 8, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
-      case 1: return dgemm_launch<P, 4, 2, 4, 5, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
-      case 2: return dgemm_launch<P, 2, 2, 4, 4, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
-      case 3: return dgemm_launch<P, 2, 2, 4, 4, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+      case NARROW_256: return dgemm_launch<P, 4, 2, 4, 8, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+      case NARROW_160: return dgemm_launch<P, 4, 2, 4, 5, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+      case NARROW_128: return dgemm_launch<P, 2, 2, 4, 4, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
+      case NARROW_128K: return dgemm_launch<P, 2, 2, 4, 4, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
       default: return dgemm_launch<P, 2, 2, 4, 2, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     }
   }

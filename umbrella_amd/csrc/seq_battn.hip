@@ -679,8 +679,9 @@ static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv,
   while (rh > maps && hpg % (rh / maps)) rh >>= 1;
   const int hblocks = H * maps / rh;
   const long items = (long)T * hblocks;
-  // keys a token can have: by the mask's form and by what a sequence's page table holds.  Within one span nobody splits, and the merge behind it would
-  // find nothing to do: one token of 8B widths in a cache of 192 positions, three layers 56 us -> 41 without the merges (4.6 us each)
+  // keys a token can have: by the mask's form and by the pages there are (a page table has room for the whole pool).  So this sees only a pool that is one
+  // span of keys altogether, a single short conversation's: nobody splits there, and the merge behind it would find nothing to do (one token of 8B
+  // widths in a cache of 192 positions, three layers 56 us -> 41 without the merges, 4.6 us each).  In a larger pool a short sequence's merge still runs.
   const long most = std::min((long)(form.chunk > 0 && form.chunk < window ? form.chunk : window) + form.keep_first, (long)kv->max_pages * kv->page);
   int nsplit = 1;
   if (scratch && items <= 64 && most > ATT_SPAN) {
@@ -1008,7 +1009,7 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sv[e]);
-      const float m_new = fmaxf(m_run[hh], rows_quad_max(mx));
+      const float m_new = fmaxf(m_run[hh], quad_max(mx));
       const float m_ref = m_new == -INFINITY ? 0.f : m_new;          // a row that has seen no key yet: all weights 0
       const float fac = __builtin_amdgcn_exp2f(m_run[hh] - m_ref);
       float w[8], sum = 0.f;

@@ -453,7 +453,7 @@ __global__ __launch_bounds__(NW * 64) void lat_attend_mfma_kernel(u16* __restric
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sv[e]);
-      const float m_new = fmaxf(m_run[hh], rows_quad_max(mx));
+      const float m_new = fmaxf(m_run[hh], quad_max(mx));
       const float m_ref = m_new == -INFINITY ? 0.f : m_new;          // a row that has seen no key yet: all weights 0
       const float fac = __builtin_amdgcn_exp2f(m_run[hh] - m_ref);
       float w[8], sum = 0.f;

@@ -89,10 +89,3 @@ template <int CHUNKS> struct RowValues {
     return u32x4{lo[0], lo[1], hi[0], hi[1]};
   }
 };
-// max over lanes l, l ^ 16, l ^ 32, l ^ 48, by lane swaps instead of through LDS
-__device__ __forceinline__ float rows_quad_max(float v) {
-  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}

@@ -28,19 +28,21 @@ __device__ __forceinline__ float log_sigmoidf_(float x) { return fminf(x, 0.f) -
 // z / (1 + e^-u) as exactly as expf and a division give it, in two thirds of their instructions: e^-u as a power of two, its exponent taken apart
 // into a whole number and a rest (Cody and Waite; v_exp_f32 on the rest), and one step on the quotient.  Numerator and denominator are a quarter of
 // what they are, so that the reciprocal of a denominator of up to 2^128 is none that v_rcp_f32 flushes to zero; beyond it e^-u is infinite and the
-// quotient 0, as there.  The bounds on u keep a NaN, and v_div_fixup_f32 gives what a division does of infinities, zeros and NaN.
+// quotient 0, as there.  Infinities and NaN of z as there (the step is dropped where it is not a number).  A NaN of u alone is lost in its bounds:
+// gated_ below is for a u that z does not follow from.
 // Error of z = u against 64 bits, in 2^-24 of the value, over |u| < 30 / -88.7 < u < -87.2: largest 3.04 / 2.01, root mean square 0.582 / 0.604,
 // all as there.  A prompt's gated feed-forward does 64 of these a lane behind its products (16384 x 2048, 2048 tokens: 125 us -> 111 with them, the
 // biases and the choice of the epilogue out of the loop over tokens).
 __device__ __forceinline__ float over_one_plus_exp(float z, float u) {
 #pragma clang fp contract(off)
-  const float c = __builtin_elementwise_maximum(__builtin_elementwise_minimum(u, 110.f), -110.f), h = -c * 1.44269502f, n = __builtin_rintf(h);
+  const float c = __builtin_amdgcn_fmed3f(u, -110.f, 110.f), h = -c * 1.44269502f, n = __builtin_rintf(h);
   const float l = fmaf(-c, 1.92596303e-8f, fmaf(-c, 1.44269502f, -h));         // log2(e) in two parts
   const float d = fmaf(__builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((h - n) + l), (int)n), 0.25f, 0.25f), t = 0.25f * z;
-  const float r = __builtin_amdgcn_rcpf(d), q = t * r;
-  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, d, t), r, q), d, t);
+  const float r = __builtin_amdgcn_rcpf(d), q = t * r, p = fmaf(fmaf(-q, d, t), r, q);
+  return p == p ? p : q;
 }
 __device__ __forceinline__ float siluf_(float x) { return over_one_plus_exp(x, x); }
+__device__ __forceinline__ float gated_(float z, float u) { const float y = over_one_plus_exp(z, u); return u == u ? y : u; }
 
 // ---- paged key/value store: element offsets (in elements) of one token's / one pooled block's D-vector
 __device__ __forceinline__ long pkv_tok(const UmbPagedKV& kv, int slot, int pos, int g, int G, int D) {

@@ -539,7 +539,7 @@ __global__ __launch_bounds__(256, 2) void seq_linear_tile_batched_kernel(void* _
 #pragma unroll
       for (int i = 0; i < RA; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[i][r] = over_one_plus_exp(v[i][r], gv[t][i][r]);
+        for (int r = 0; r < 4; ++r) v[i][r] = gated_(v[i][r], gv[t][i][r]);
     }
     if (epi == EPI_F32) {
       tile_rows_out<16, RA>(strip, v, [&](int row, int at, u32x4 b) {

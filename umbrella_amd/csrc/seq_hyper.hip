@@ -234,7 +234,7 @@ __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x,
   const long o = (long)blockIdx.x * W;
   const int nq = W / 4;
   const float mx = mix ? mix[0] : 1.f, ot = out ? out[0] : 1.f, in0 = in_next ? in_next[0] : 1.f;
-  // one quad a thread: read either way (without a next norm from the row's first slab), as in resid_norm_quad_kernel
+  // few quads a thread, or slabs: read either way (without a next norm from the row's first slab), as in resid_norm_quad_kernel
   const typename El<P>::type* wq = w_next ? w_next : reinterpret_cast<const typename El<P>::type*>(y);
   f32x4 xv[NE], yv[NE], wn[NE];
 #pragma unroll
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x,
     const int i = min((int)threadIdx.x + NT * e, nq - 1) * 4;
     xv[e] = *reinterpret_cast<const f32x4*>(x + o + i);
     yv[e] = *reinterpret_cast<const f32x4*>(y + o + i);
-    wn[e] = NE == 1 || w_next ? ld4<P>(wq + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+    wn[e] = NE <= 2 || SLABS || w_next ? ld4<P>(wq + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   if constexpr (SLABS) add_parts<NE>(yv, y, parts, slab, [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; });
   float ss = 0.f;

@@ -331,7 +331,9 @@ __global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__
   __shared__ float red[NT / 64], red2[NT / 64];
   const int grp = blockIdx.y, gs = W / groups, nq = gs / 4;
   const long o = (long)blockIdx.x * W + (long)grp * gs;
-  // one quad a thread (few rows): read either way, behind a test the load is a round trip of its own; more of them (many rows): only if it is wanted
+  // one quad a thread (few rows), or slabs: read either way, behind a test the load is a round trip of its own; several quads of whole outputs (many
+  // rows): only if it is wanted (us, fp32 weights, 2048 rows of 2048: 9.6, read either way 10.4; the seams of a forward of 2466 rows,
+  // slabs and 16 bits: 85 read either way, 91 behind the test)
   const typename El<P>::type* wq = w_next ? w_next : w_post;
   f32x4 yv[NE], xv[NE], wp[NE], wn[NE];
 #pragma unroll
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(NT) void resid_norm_quad_kernel(float* __restrict__
     yv[e] = *reinterpret_cast<const f32x4*>(y + o + i);
     xv[e] = *reinterpret_cast<const f32x4*>(x + o + i);
     wp[e] = ld4<P>(w_post + grp * gs + i);
-    wn[e] = NE == 1 || w_next ? ld4<P>(wq + grp * gs + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+    wn[e] = NE == 1 || SLABS || w_next ? ld4<P>(wq + grp * gs + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   if constexpr (SLABS) add_parts<NE>(yv, y, parts, slab, [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; });
   float ss = 0.f;
@@ -422,7 +424,7 @@ __global__ __launch_bounds__(NT) void pair_resid_norm_quad_kernel(float* __restr
     wa[e] = ld4<P>(w1 + i);
     wb[e] = ld4<P>(w2 + i);
     wp[e] = ld4<P>(w_post + i);
-    wn[e] = NE == 1 || w_next ? ld4<P>(wq + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+    wn[e] = NE == 1 || SLABS || w_next ? ld4<P>(wq + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   if constexpr (SLABS) {
     const auto at = [&](int e) { return o + min((int)threadIdx.x + NT * e, nq - 1) * 4; };

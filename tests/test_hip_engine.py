@@ -819,3 +819,47 @@ def test_static_engine_defaults_to_the_reference_sampler(dev):
     assert torch.equal(eng.uniform_samples.cpu(), torch.rand(3, eng.tree_size, generator=torch.Generator().manual_seed(11)))
     e2, _ = static_engine(g, dev, torch.float16, self_draft=True, hip_graph=False, temperature=0.7, seed=11, reference_sampler=False)
     assert e2.uniform_samples is None
+
+
+def test_captures_beside_another_threads_event_queries(dev):
+    """a process group's watchdog asks for the events of collectives that a warm-up issued, from a thread of its own, while an iteration, a stage or a
+    batched step is captured: neither the thread nor the capture meets an error"""
+    import threading
+    import seqmix_helpers as sm
+    from hip_helpers import static_engine
+    from umbrella_amd.parallel import _capture
+    event, errors, polls, stop = torch.cuda.Event(), [], [0], threading.Event()
+    event.record()
+    torch.cuda.synchronize()
+
+    def watch():
+        try:
+            while not stop.is_set():
+                event.query()
+                polls[0] += 1
+        except Exception as e:
+            errors.append(e)
+    x = torch.zeros(64, device=dev)
+    m, _ = sm.build(sm.CONFIGS["mixed"], torch.bfloat16)
+    m.use_graph = True
+    m.open(0)
+    m.forward_batch([(0, [1, 2, 3])])
+    thread = threading.Thread(target=watch)
+    thread.start()
+    try:
+        before = polls[0]
+        graph = _capture(lambda: [x.add_(1.0) for _ in range(2000)], dev)
+        for token in range(4):                                    # eager, captured and replayed
+            m.forward_batch([(0, [token])])
+        eng, _ = static_engine(G, dev, torch.float16, self_draft=True)
+        out = eng.generate(input_ids=PROMPT, max_new_tokens=8)["generated_tokens"]
+        assert polls[0] > before
+    finally:
+        stop.set()
+        thread.join()
+    assert not errors, errors
+    assert eng._graph is not None and len(out) >= 8
+    x.zero_()
+    for _ in range(3):
+        graph.replay()
+    assert bool((x == 6000.0).all())

@@ -245,7 +245,7 @@ def _capture(run, device):
     torch.cuda.current_stream().wait_stream(s)
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    with torch.cuda.graph(g, capture_error_mode="thread_local"):       # (other threads go on asking for events: a process group's watchdog)
         run()
     torch.cuda.synchronize()
     return g

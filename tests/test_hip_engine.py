@@ -825,6 +825,7 @@ def test_captures_beside_another_threads_event_queries(dev):
     """a process group's watchdog asks for the events of collectives that a warm-up issued, from a thread of its own, while an iteration, a stage or a
     batched step is captured: neither the thread nor the capture meets an error"""
     import threading
+    import time
     import seqmix_helpers as sm
     from hip_helpers import static_engine
     from umbrella_amd.parallel import _capture
@@ -837,6 +838,7 @@ def test_captures_beside_another_threads_event_queries(dev):
             while not stop.is_set():
                 event.query()
                 polls[0] += 1
+                time.sleep(2e-4)
         except Exception as e:
             errors.append(e)
     x = torch.zeros(64, device=dev)

@@ -6,12 +6,17 @@
 // it, 64 x 128 (4 x 8) for three quarters.  Hence:
 //   * operands go HBM / L2 -> LDS by LDS-DMA (1-KiB pieces of 8 rows x 128 B: whole lines, no VGPR on the way, no address arithmetic
 //     in the loop); the 16-byte column of a row is XOR-swizzled on the SOURCE side, so fragment reads meet no bank conflict;
-//   * a ring of two to four slots of 64 k, as many as the LDS holds.  ONE barrier per stage stands between its two 32-k phases: when a
-//     wave arrives there it has every fragment of the stage in registers, so behind the barrier the slot is free for the stage NS
-//     further on, and the next stage (whose pieces every wave has waited for) can be read: the fragments of a phase are requested, one
-//     per few products, while the products of the phase before run, across the stage boundary too, and a stage's pieces have
-//     NS - 1 stages to arrive.  With two slots no stage is shorter than the 1.0 us that pieces take from L2: 256 x 128 outputs 1.05 -> 0.86
-//     us a stage with three, 256 x 160 1.1 -> 0.95 - 1.05, 128 x 128 (eight waves, four slots; before: K over two groups of four, 0.55) 0.49.
+//   * a ring of two to four slots of 64 k for each operand, as many as the LDS holds.  ONE barrier per stage stands between its two 32-k
+//     phases: when a wave arrives there it has every fragment of the stage in registers, so behind the barrier the slot is free for the
+//     stage a ring's length further on, and the next stage (whose pieces every wave has waited for) can be read: the fragments of a phase are
+//     requested, one per few products, while the products of the phase before run, across the stage boundary too.  With two slots the
+//     pieces that are asked for last have half a stage to arrive, and no stage is shorter than the 1.0 us that they take from L2: 256 x 128 outputs
+//     1.05 -> 0.86 us a stage with three, 256 x 160 1.1 -> 0.95 - 1.05, 128 x 128 (eight waves, four slots; before: K over two groups of four,
+//     0.55) 0.49.  256 x 256 and 256 x 192 outputs have no room for three of both, but for three of A (the weights, which come from further away) and two
+//     of B, whose pieces are then asked for first: 1.47 -> 1.36 and 1.36 -> 1.19 us a stage (K 4096 -> 8192, 256 workgroups; on zeros, without the
+//     power limit, 2048 x 8192 x 4096 91 -> 78 us; 1024 x 28672 x 4096 197 -> 192).  Four waves of 128 x 128 outputs (a third less LDS traffic, sums in
+//     AGPRs) on the same rings: 105 us where these take 101, 88 on zeros.
+//   * the last stages ask for nothing: pieces past the end would be waited for behind the last product.
 // K-split (KS = 2): two groups of WM x WN waves take alternate stages in slots of their own and their tiles are added (group 0 +
 // group 1) at the end: two waves per SIMD where a launch has at most one workgroup per CU.
 // Measured against the register-staged kernel it replaces (bf16, random data, one MI355X; both sides in seq_linear.hip).
@@ -35,13 +40,16 @@ template <int WM, int WN, int RA, int RB, int KS> struct TileShape {
   static constexpr int BN = 16 * WM * RA, BT = 16 * WN * RB;  // rows of A, tokens of B
   static constexpr int NPA = BN / 8, NPB = BT / 8;            // 1-KiB pieces of a stage
   static constexpr int NPW = (NPA + NPB + NW - 1) / NW;       // pieces a wave fetches per stage
-  static constexpr unsigned SLOT = (NPA + NPB) * 1024u;
+  static constexpr unsigned SA = NPA * 1024u, SB = NPB * 1024u, SLOT = SA + SB;
   static constexpr int PER_CU = NW * KS == 4 ? 2 : 1;         // workgroups that share a CU
   // where the pieces do not deal out evenly, a wave without a last piece of its own fetches into the KiB behind the slots
   static constexpr bool EVEN = (NPA + NPB) % NW == 0;
-  static constexpr int FIT = (int)((160 * 1024 / PER_CU - (EVEN ? 0 : 1024)) / (KS * SLOT)), NS = FIT < 4 ? FIT : 4;      // slots of a ring
-  static constexpr size_t LDS = (size_t)KS * NS * SLOT + (EVEN ? 0 : 1024);
-  static_assert(NS >= 2 && NPA % NW == 0 && (EVEN || KS == 1) && (KS == 1 || RA * RB * NW * 1024u <= LDS), "whole rounds of A pieces; a group's tile fits the slots");
+  static constexpr unsigned ROOM = 160u * 1024 / PER_CU - (EVEN ? 0 : 1024);
+  static constexpr int FIT = (int)(ROOM / (KS * SLOT)), NSB = FIT < 4 ? FIT : 4;               // slots of B's ring
+  static constexpr int NSA = NSB == 2 && KS * (3 * SA + 2 * SB) <= ROOM ? 3 : NSB;             // and of A's
+  static constexpr unsigned RINGS = NSA * SA + NSB * SB;
+  static constexpr size_t LDS = (size_t)KS * RINGS + (EVEN ? 0 : 1024);
+  static_assert(NSB >= 2 && NPA % NW == 0 && (EVEN || KS == 1) && (KS == 1 || RA * RB * NW * 1024u <= LDS), "whole rounds of A pieces; a group's tile fits the slots");
 };
 
 // The tiles a launch chooses from, and what a 64-k stage of a whole round of 256 workgroups takes (us; one MI355X, bf16, random data).  Few sizes
@@ -96,15 +104,16 @@ template <typename P, int WM, int WN, int RA, int RB, int KS, bool FRAG>
 __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned char* smem, const void* abase, const void* bbase, long astep,
                                               const unsigned (&voff)[TileShape<WM, WN, RA, RB, KS>::NPW], int nst, int wave, int ks) {
   typedef TileShape<WM, WN, RA, RB, KS> S;
-  constexpr int NW = S::NW, NPA = S::NPA, NPW = S::NPW, NF = RA + RB, NM = RA * RB, NS = S::NS;
+  constexpr int NW = S::NW, NPA = S::NPA, NPW = S::NPW, PA = NPA / NW, PB = NPW - PA, NF = RA + RB, NM = RA * RB, NSA = S::NSA, NSB = S::NSB;
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
-  const unsigned lds0 = (unsigned)(size_t)(lds_char*)smem + (unsigned)(ks * S::NS) * S::SLOT;
+  const unsigned lds0 = (unsigned)(size_t)(lds_char*)smem + (unsigned)ks * S::RINGS, lds1 = lds0 + NSA * S::SA;
   const int n = nst / KS;                                     // stages of this group
-  auto issue = [&](int st, unsigned slot, int i) {
-    unsigned dst = lds0 + slot + (unsigned)(wave + NW * i) * 1024u;
-    if (!S::EVEN && i == NPW - 1 && wave + NW * i >= NPA + S::NPB) dst = lds0 + (unsigned)NS * S::SLOT;
+  auto issue = [&](int st, unsigned slot, int i) {            // pieces 0 .. PA - 1 are A's; slot: of the ring they go to
+    const unsigned p = (unsigned)(wave + NW * i);
+    unsigned dst = i < PA ? lds0 + slot + p * 1024u : lds1 + slot + (p - NPA) * 1024u;
+    if (!S::EVEN && i == NPW - 1 && wave + NW * i >= NPA + S::NPB) dst = lds0 + S::RINGS;
     const long s = (long)min(st, n - 1) * KS + ks;
-    if (NW * i < NPA) tile_dma(voff[i], static_cast<const char*>(abase) + s * astep, dst);
+    if (i < PA) tile_dma(voff[i], static_cast<const char*>(abase) + s * astep, dst);
     else tile_dma(voff[i], static_cast<const char*>(bbase) + s * 128, dst);
   };
   // fragment (16 rows, 32 k) of two row pieces: lane (j, g) reads row j, 16-byte column 4 kh + g
@@ -116,44 +125,66 @@ __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned cha
 #pragma unroll
     for (int t = 0; t < RB; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   u32x4 fa[2][RA], fb[2][RB];
-  auto read = [&](unsigned slot, int kh, int i) {             // the i-th fragment of a phase, in the order the products want them
-    const unsigned base = lds0 + slot;
-    const unsigned ao = base + (FRAG ? (unsigned)(kh * 1024 + lane * 16) : foff[kh]);
+  auto read = [&](unsigned sa, unsigned sb, int kh, int i) {  // the i-th fragment of a phase, in the order the products want them
+    const unsigned ao = lds0 + sa + (FRAG ? (unsigned)(kh * 1024 + lane * 16) : foff[kh]), bo = lds1 + sb + foff[kh];
     if (i == 0) fa[kh][0] = *reinterpret_cast<const lds_u32x4*>((size_t)(ao + (unsigned)(wm * RA) * 2048u));
-    else if (i <= RB) fb[kh][i - 1] = *reinterpret_cast<const lds_u32x4*>((size_t)(base + foff[kh] + NPA * 1024u + (unsigned)(wn * RB + i - 1) * 2048u));
+    else if (i <= RB) fb[kh][i - 1] = *reinterpret_cast<const lds_u32x4*>((size_t)(bo + (unsigned)(wn * RB + i - 1) * 2048u));
     else fa[kh][i - RB] = *reinterpret_cast<const lds_u32x4*>((size_t)(ao + (unsigned)(wm * RA + i - RB) * 2048u));
   };
-  unsigned slot = 0, next = S::SLOT;                          // of the stage whose products run, and of the one behind it
-  auto phase = [&](auto half, int st) {
-    constexpr int KH = decltype(half)::value;
+  unsigned sa = 0, sb = 0, na = S::SA, nb = S::SB;            // slots of the stage whose products run, and of the one behind it
+  // the products of one half of stage st; FETCH: 2 the stages NSA and NSB further on are asked for (behind the barrier), 1 B's alone, 0 none
+  auto phase = [&](auto half, auto fetch, auto more, int st) {
+    constexpr int KH = decltype(half)::value, FETCH = decltype(fetch)::value;
+    constexpr bool READ = KH == 0 || decltype(more)::value;
     constexpr int GAP = NM / NF > 0 ? NM / NF : 1, DG = NM / NPW > 0 ? NM / NPW : 1;   // products per fragment read, per piece
     static_assert(GAP * (NF - 1) < NM && DG * (NPW - 1) < NM, "every read and every piece has a product to hide behind");
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-      if (m % GAP == 0 && m / GAP < NF) read(KH == 0 ? slot : next, KH ^ 1, m / GAP);
-      if (KH == 1 && m % DG == 0 && m / DG < NPW) issue(st + NS, slot, m / DG);
+      if (READ && m % GAP == 0 && m / GAP < NF) read(KH == 0 ? sa : na, KH == 0 ? sb : nb, KH ^ 1, m / GAP);
+      if (KH == 1 && m % DG == 0 && m / DG < NPW) {
+        const int i = NSA > NSB ? (m / DG < PB ? PA + m / DG : m / DG - PB) : m / DG;            // the shorter ring's pieces first
+        if (i >= PA ? FETCH > 0 : FETCH > 1) issue(st + (i < PA ? NSA : NSB), i < PA ? sa : sb, i);
+      }
       acc[m / RB][m % RB] = P::mfma(fa[KH][m / RB], fb[KH][m % RB], acc[m / RB][m % RB]);
       if ((m + 1) % GAP == 0) __builtin_amdgcn_sched_barrier(0);
     }
   };
-#pragma unroll
-  for (int c = 0; c < NS; ++c)
-#pragma unroll
-    for (int i = 0; i < NPW; ++i) issue(c, c * S::SLOT, i);
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NS - 1) * NPW) : "memory");
-  __builtin_amdgcn_s_barrier();
-#pragma unroll
-  for (int i = 0; i < NF; ++i) read(0, 0, i);
-  for (int st = 0; st < n; ++st) {
-    phase(std::integral_constant<int, 0>{}, st);
+  // a stage; LEFT: what may still be on its way when its successor has to be there
+  auto stage = [&](auto left, auto fetch, auto more, int st) {
+    phase(std::integral_constant<int, 0>{}, fetch, more, st);
     // every fragment of stage st is in registers, and this wave's pieces of stage st + 1 are in LDS
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NS - 2) * NPW) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(decltype(left)::value) : "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    phase(std::integral_constant<int, 1>{}, st);
-    slot = next;
-    next = next == (NS - 1) * S::SLOT ? 0u : next + S::SLOT;
-  }
+    phase(std::integral_constant<int, 1>{}, fetch, more, st);
+    sa = na;
+    sb = nb;
+    na = na == (NSA - 1) * S::SA ? 0u : na + S::SA;
+    nb = nb == (NSB - 1) * S::SB ? 0u : nb + S::SB;
+  };
+#pragma unroll
+  for (int c = 0; c < NSA; ++c)
+#pragma unroll
+    for (int i = 0; i < NPW; ++i)
+      if (i < PA || c < NSB) issue(c, c * (i < PA ? S::SA : S::SB), i);
+  constexpr int ALONE = NSA > NSB ? PA : 0;                   // A's pieces of the stage that only its ring holds
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NSB - 1) * NPW + ALONE) : "memory");
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < NF; ++i) read(0, 0, 0, i);
+  int st = 0;
+  for (; st < n - NSA; ++st) stage(std::integral_constant<int, (NSB - 2) * NPW + ALONE>{}, std::integral_constant<int, 2>{}, std::true_type{}, st);
+  // the last NSA stages: nothing is asked for that no stage will use
+  auto last = [&](auto t_) {
+    constexpr int t = decltype(t_)::value, LEFT = (NSB - 2 - t > 0 ? NSB - 2 - t : 0) * NPW + (t == 0 ? ALONE : 0);
+    if (st < n) stage(std::integral_constant<int, LEFT>{}, std::integral_constant<int, (t < NSA - NSB)>{}, std::integral_constant<bool, (t < NSA - 1)>{}, st);
+    ++st;
+  };
+  last(std::integral_constant<int, 0>{});
+  last(std::integral_constant<int, 1>{});
+  if constexpr (NSA > 2) last(std::integral_constant<int, 2>{});
+  if constexpr (NSA > 3) last(std::integral_constant<int, 3>{});
+  static_assert(NSA >= 2 && NSA <= 4 && (NSA == NSB || (NSA == 3 && NSB == 2)), "the last stages above");
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // nothing of this wave may still be writing LDS
   __builtin_amdgcn_s_barrier();                                 // and none reads a slot any more
   if constexpr (KS == 2) {

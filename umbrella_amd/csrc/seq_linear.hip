@@ -21,10 +21,10 @@ template <typename P> struct Frag8 { u32x4 v; };
 template <> struct Frag8<F32> { f32x4 lo, hi; };
 
 template <typename P, bool VEC>
-__device__ __forceinline__ Frag8<P> load8(const typename El<P>::type* __restrict__ row, bool ok, int k, int K) {
+__device__ __forceinline__ Frag8<P> load8(const typename El<P>::type* __restrict__ row, int k, int K) {
   Frag8<P> f;
   if constexpr (VEC) {                      // K % 8 == 0: k < K means the whole 8-group is inside, 16-byte aligned
-    const bool in = ok && k < K;
+    const bool in = k < K;
     if constexpr (sizeof(typename El<P>::type) == 2) {
       f.v = in ? *reinterpret_cast<const u32x4*>(row + k) : u32x4{0u, 0u, 0u, 0u};
     } else {
@@ -35,12 +35,12 @@ __device__ __forceinline__ Frag8<P> load8(const typename El<P>::type* __restrict
     if constexpr (sizeof(typename El<P>::type) == 2) {
       unsigned e[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) e[i] = (ok && k + i < K) ? (unsigned)row[k + i] : 0u;
+      for (int i = 0; i < 8; ++i) e[i] = (k + i < K) ? (unsigned)row[k + i] : 0u;
       f.v = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
     } else {
       float e[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) e[i] = (ok && k + i < K) ? row[k + i] : 0.f;
+      for (int i = 0; i < 8; ++i) e[i] = (k + i < K) ? row[k + i] : 0.f;
       f.lo = f32x4{e[0], e[1], e[2], e[3]};
       f.hi = f32x4{e[4], e[5], e[6], e[7]};
     }
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void seq_linear_kernel(void* __restrict__ out_
   typedef typename El<P>::type E;
   static_assert(!DUAL || NT <= 2, "gate and up partials of NT x TT tiles must fit the LDS");
   __shared__ float red[DUAL ? 2 : 1][4][NT * TT][256];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int j = lane & 15, g = lane >> 4;
   int t0 = blockIdx.y * (TT * 16);
   const int ldx = ext.ldx, ldo = ext.ldo;
@@ -134,22 +134,22 @@ __global__ __launch_bounds__(256) void seq_linear_kernel(void* __restrict__ out_
     T = rows;
     t0 = 0;
   }
-  const E* wrow[NT];
-  bool n_ok[NT];
+  const E* wrow[NT];                       // rows past an operand's end read its last one: what they give is not stored
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int n_row = (blockIdx.x * NT + nt) * 16 + j;
-    n_ok[nt] = n_row < N;
-    wrow[nt] = w + (long)(n_ok[nt] ? n_row : 0) * K;
-  }
+  for (int nt = 0; nt < NT; ++nt) wrow[nt] = w + (long)min((int)(blockIdx.x * NT + nt) * 16 + j, N - 1) * K;
   const long half = DUAL ? (long)N * K : 0;
   const E* xrow[TT];
-  bool t_ok[TT];
 #pragma unroll
-  for (int tt = 0; tt < TT; ++tt) {
-    const int t = t0 + tt * 16 + j;
-    t_ok[tt] = t < T;
-    xrow[tt] = x + (long)(t_ok[tt] ? t : 0) * ldx;
+  for (int tt = 0; tt < TT; ++tt) xrow[tt] = x + (long)min(t0 + tt * 16 + j, T - 1) * ldx;
+  // thread (l = tid / 4, r = tid % 4) finishes output (n = 4 (l / 16) + r, token = l % 16) of every tile; its biases are asked for beside the
+  // operands: behind the sums they were a round trip of their own
+  const int l = threadIdx.x >> 2, r = threadIdx.x & 3;
+  float bv[NT], bv2[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int n = min((int)(blockIdx.x * NT + nt) * 16 + 4 * (l >> 4) + r, N - 1);
+    bv[nt] = bias ? ldf<P>(bias + n) : 0.f;
+    bv2[nt] = (DUAL && bias) ? ldf<P>(bias + N + n) : 0.f;
   }
   f32x4 acc[NT][TT], acc2[NT][TT];
 #pragma unroll
@@ -158,23 +158,24 @@ __global__ __launch_bounds__(256) void seq_linear_kernel(void* __restrict__ out_
     for (int nt = 0; nt < NT; ++nt) { acc[nt][tt] = f32x4{0.f, 0.f, 0.f, 0.f}; acc2[nt][tt] = f32x4{0.f, 0.f, 0.f, 0.f}; }
   }
 
-  constexpr int UN = (NT * TT == 1) ? (DUAL ? 8 : 16) : 2;        // 32-k steps in flight per wave (a single-tile launch is latency-bound:
-                                                    // K = 2048 is two round trips per wave instead of four)
-  for (int k0 = wave * 32; k0 < K; k0 += 128 * UN) {
-    Frag8<P> a[UN][NT], a2[UN][NT], b[UN][TT];
+  // this wave's 32-k steps k0, k0 + 128, ...: `un` of them in flight at once.  (A step past K is zeros; the loads and, in fp32, eight products of it
+  // cost as much as any other's, see UN.)
+  auto steps = [&](auto un, int k0) __attribute__((always_inline)) {
+    constexpr int U = decltype(un)::value;
+    Frag8<P> a[U][NT], a2[U][NT], b[U][TT];
 #pragma unroll
-    for (int u = 0; u < UN; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int k = k0 + u * 128 + g * 8;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        a[u][nt] = load8<P, VEC>(wrow[nt], n_ok[nt], k, K);
-        if constexpr (DUAL) a2[u][nt] = load8<P, VEC>(wrow[nt] + half, n_ok[nt], k, K);
+        a[u][nt] = load8<P, VEC>(wrow[nt], k, K);
+        if constexpr (DUAL) a2[u][nt] = load8<P, VEC>(wrow[nt] + half, k, K);
       }
 #pragma unroll
-      for (int tt = 0; tt < TT; ++tt) b[u][tt] = load8<P, VEC>(xrow[tt], t_ok[tt], k, K);
+      for (int tt = 0; tt < TT; ++tt) b[u][tt] = load8<P, VEC>(xrow[tt], k, K);
     }
 #pragma unroll
-    for (int u = 0; u < UN; ++u) {
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt) {
 #pragma unroll
@@ -184,7 +185,16 @@ __global__ __launch_bounds__(256) void seq_linear_kernel(void* __restrict__ out_
         }
       }
     }
-  }
+  };
+  // A single tile's launch is latency-bound: all its steps in flight, up to 16 (8 of both halves), K = 2048 in one round trip.  The last ones by the
+  // least power of two that holds them: as 16 whatever K is, K = 192 in fp32 was fourteen steps of zeros, 112 of 128 products.
+  constexpr int UN = (NT * TT == 1) ? (DUAL ? 8 : 16) : 2;
+  int k0 = wave * 32;
+  for (; K - k0 > 128 * (UN / 2); k0 += 128 * UN) steps(std::integral_constant<int, UN>{}, k0);
+  if constexpr (UN > 8) if (K - k0 > 128 * 4) { steps(std::integral_constant<int, 8>{}, k0); k0 = K; }
+  if constexpr (UN > 4) if (K - k0 > 128 * 2) { steps(std::integral_constant<int, 4>{}, k0); k0 = K; }
+  if constexpr (UN > 2) if (K - k0 > 128) { steps(std::integral_constant<int, 2>{}, k0); k0 = K; }
+  if (K > k0) steps(std::integral_constant<int, 1>{}, k0);
 #pragma unroll
   for (int tt = 0; tt < TT; ++tt) {
 #pragma unroll
@@ -194,14 +204,10 @@ __global__ __launch_bounds__(256) void seq_linear_kernel(void* __restrict__ out_
     }
   }
   __syncthreads();
-  // thread (l = tid / 4, r = tid % 4) finishes output (n = 4 (l / 16) + r, token = l % 16) of every tile
-  const int l = threadIdx.x >> 2, r = threadIdx.x & 3;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int n = (blockIdx.x * NT + nt) * 16 + 4 * (l >> 4) + r;
     if (n >= N) continue;
-    const float bv = bias ? ldf<P>(bias + n) : 0.f;
-    const float bv2 = (DUAL && bias) ? ldf<P>(bias + N + n) : 0.f;
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
       const int t = t0 + tt * 16 + (l & 15);
@@ -209,12 +215,12 @@ __global__ __launch_bounds__(256) void seq_linear_kernel(void* __restrict__ out_
       float s = red[0][0][nt * TT + tt][threadIdx.x];
 #pragma unroll
       for (int ww = 1; ww < 4; ++ww) s += red[0][ww][nt * TT + tt][threadIdx.x];
-      s += bv;
+      s += bv[nt];
       if constexpr (DUAL) {
         float u = red[1][0][nt * TT + tt][threadIdx.x];
 #pragma unroll
         for (int ww = 1; ww < 4; ++ww) u += red[1][ww][nt * TT + tt][threadIdx.x];
-        u += bv2;
+        u += bv2[nt];
         stf<P>(reinterpret_cast<E*>(out_) + obase + (long)t * ldo + n, glu_pair(epi, s, u, ext.limit, ext.alpha));
       } else if (epi == EPI_DT) {
         stf<P>(reinterpret_cast<E*>(out_) + obase + (long)t * ldo + n, s);

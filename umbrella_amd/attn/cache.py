@@ -137,6 +137,18 @@ class TreeKVCache:
         self.kv_offset = kv_len
 
 
+def send(host: torch.Tensor, device, into: torch.Tensor = None) -> torch.Tensor:
+    """A host tensor's values on the device (in `into`, if given), in the order of the current stream, without waiting for it: they leave
+    from pinned memory of their own, which torch's allocator hands out again once the copy has run.  Refused under capture, as a copy
+    that waits is: a replay would read memory that is somebody else's by then."""
+    if torch.device(device).type != "cuda":
+        return host.to(device) if into is None else into.copy_(host)
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("host values cannot be sent to the device while the stream is capturing")
+    host = torch.empty(host.shape, dtype=host.dtype, pin_memory=True).copy_(host)
+    return host.to(device, non_blocking=True) if into is None else into.copy_(host, non_blocking=True)
+
+
 class PagedSeqCache:
     """Paged key/value store, pooled blocks and recurrent-state slots for MANY sequences (the sequence-mixer models of
     libumbrella_seq.so; device-side statement: csrc/seq_common.h ``pkv_tok`` / ``pkv_blk``).
@@ -250,7 +262,7 @@ class PagedSeqCache:
         """page-table entries [(place, page)] to the device, stream-ordered, in ONE host copy: a copy per sequence kept the host 20 us
         each (48 sequences that start together: 9.44 -> 8.34 ms for a whole call of 17 steps)"""
         if entries:
-            at, page = torch.tensor(entries, dtype=torch.long).t().contiguous().to(self.device)
+            at, page = send(torch.tensor(entries, dtype=torch.long).t().contiguous(), self.device)
             self.pages_dev.view(-1)[at] = page.to(torch.int32)
 
     # ---- semantic access (tests, tools): never on the hot path

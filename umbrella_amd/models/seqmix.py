@@ -26,11 +26,12 @@ from __future__ import annotations
 import ctypes as C
 import os
 
+import numpy as np
 import torch
 
 from .. import _lib
 from .._lib import UmbSeqLayer, UmbSeqLinear, UmbSeqModel, UmbSeqStep, UmbSeqWork
-from ..attn.cache import PagedSeqCache
+from ..attn.cache import PagedSeqCache, send
 from .base import LLMBase
 from .config import SeqMixCfg, rotary_frequencies, rotary_table
 
@@ -478,11 +479,11 @@ class SeqMixLM(LLMBase):
         [rows wanted, V] (a view of the workspace, valid until the next step) in the order of parts and of want; with
         trace also the residual stream after every layer [L, T, W]."""
         cache, dev = self.kv_cache, self.device
-        toks, pos, slot, seq_slot, row0, pos0, lens, rows = [], [], [], [], [], [], [], []
+        toks, seq_slot, row0, pos0, lens, rows, counts = [], [], [], [], [], [], []
         entries = []                                 # page-table entries of all parts, written at once
         try:
             for i, (sid, ids) in enumerate(parts):
-                ids = [int(v) for v in (ids.tolist() if isinstance(ids, torch.Tensor) else ids)]
+                ids = list(map(int, ids.tolist() if isinstance(ids, torch.Tensor) else ids))
                 n = len(ids)
                 if n == 0:
                     raise ValueError("a part of a step needs at least one token")
@@ -490,24 +491,33 @@ class SeqMixLM(LLMBase):
                     raise RuntimeError(f"sequence {sid!r} would exceed max_length {self.max_length}")
                 p0, sl = cache.extend(sid, n, entries), cache.slot(sid)
                 seq_slot.append(sl), row0.append(len(toks)), pos0.append(p0), lens.append(n)
-                w = [n - 1] if want is None else list(want[i])
-                rows.extend(len(toks) + int(k) for k in w)
-                toks.extend(ids), pos.extend(range(p0, p0 + n)), slot.extend([sl] * n)
+                w = [n - 1] if want is None else list(map(int, want[i]))
+                rows.extend(w), counts.append(len(w)), toks.extend(ids)
         finally:                                     # a part that is refused leaves those before it extended
             cache.write_pages(entries)
         T, B, R = len(toks), len(parts), len(rows)
         self.reserve(T, max(R, 1))
-        host = torch.tensor(toks + pos + slot + seq_slot + row0 + pos0 + lens + rows, dtype=torch.int32)
+        # tokens, their positions and slots | per sequence: slot, first row, first position, length | rows whose logits are wanted.  Up to a few
+        # thousand rows: filled by array operations, and sent without waiting -- a copy that waits for the stream leaves the device idle
+        # while the host makes the step's launches, and a step's host work cannot run beside the step before it
+        meta_host = torch.empty(3 * T + 4 * B + R, dtype=torch.int32)
+        at = meta_host.numpy()
+        first, n_of = np.asarray(row0), np.asarray(lens)
+        at[:T] = toks
+        at[T:2 * T] = np.arange(T) + np.repeat(np.asarray(pos0) - first, n_of)
+        at[2 * T:3 * T] = np.repeat(np.asarray(seq_slot), n_of)
+        at[3 * T:3 * T + 4 * B] = seq_slot + row0 + pos0 + lens
+        at[3 * T + 4 * B:] = np.asarray(rows, dtype=np.int64) + np.repeat(first, counts)
         graphed = self.use_graph and not trace and T == B and str(dev).startswith("cuda")     # a pure decode step
         key = (T, R)
         if graphed:
             entry = self._graphs.get(key)
             if entry is None:
-                entry = self._graphs[key] = {"meta": torch.zeros(host.numel(), dtype=torch.int32, device=dev), "graph": None, "runs": 0}
+                entry = self._graphs[key] = {"meta": torch.zeros(meta_host.numel(), dtype=torch.int32, device=dev), "graph": None, "runs": 0}
             meta = entry["meta"]
-            meta.copy_(host)
+            send(meta_host, dev, into=meta)
         else:
-            meta = host.to(dev)
+            meta = send(meta_host, dev)
         o = [0, T, 2 * T, 3 * T, 3 * T + B, 3 * T + 2 * B, 3 * T + 3 * B, 3 * T + 4 * B]
         p = meta.data_ptr()
         s = UmbSeqStep()

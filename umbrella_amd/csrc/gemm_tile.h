@@ -35,6 +35,12 @@ __device__ __forceinline__ void tile_dma(unsigned voff, const void* sbase, unsig
                :: "v"(voff), "s"(sbase), "s"(ldsaddr) : "memory", "m0");
 }
 
+// the same for what is read once: not kept in L2 in the place of what is
+__device__ __forceinline__ void tile_dma_once(unsigned voff, const void* sbase, unsigned ldsaddr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
+               :: "v"(voff), "s"(sbase), "s"(ldsaddr) : "memory", "m0");
+}
+
 template <int WM, int WN, int RA, int RB, int KS> struct TileShape {
   static constexpr int NW = WM * WN;                          // waves of one K group
   static constexpr int BN = 16 * WM * RA, BT = 16 * WN * RB;  // rows of A, tokens of B

@@ -717,6 +717,11 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
   int col = first_chunk(fb * (16 * NT), nc, turn);                // and the next of them: they are taken in turn from this one on
   const char* fw = wb + (long)fb * (16 * NT) * K * EB;
   rows_of_block(fb * (16 * NT));
+  // Weights that one workgroup alone reads do not stay in L2: left there they push out the code, tokens, tables and partial sums of the dozen
+  // small kernels around a product, each of which then fetched its own from further away (us, kept / not: one token, gate/up 28672 x 4096 41.9 / 41.1,
+  // two-map attention 11.6 / 9.7, delta rule 10.2 / 8.4; a whole call of 17 steps, 8B widths, 16 requests 8936 / 8531, one 7290 / 6824).  From 33 tokens
+  // on the tokens' own pieces are more than the weights, and 48 tokens of 1B widths were 2 % slower for it.  Tile lists: two tiles may share weights.
+  const bool once = TT <= 2 && !ext.tiles;
   auto issue = [&](int slot) {
     const long at = (long)col * 512;
     col = col + 1 == nc ? 0 : col + 1;     // past the last chunk of all: fetched again, never read
@@ -725,7 +730,9 @@ __global__ __launch_bounds__(256) void seq_linear_stream_kernel(void* __restrict
     for (int i = 0; i < S::PW; ++i) {
       unsigned dst = lds0 + (unsigned)slot * S::SLOT + (unsigned)(wave + 4 * i) * S::PIECE;
       if (S::NP % 4 && i == S::PW - 1 && wave + 4 * i >= S::NP) dst = lds0 + (unsigned)R * S::SLOT;      // a piece of nobody's
-      tile_dma(voff[i], (4 * i < S::AP ? fw : xb) + at, dst);
+      if (4 * i >= S::AP) tile_dma(voff[i], xb + at, dst);
+      else if (once) tile_dma_once(voff[i], fw + at, dst);
+      else tile_dma(voff[i], fw + at, dst);
     }
   };
   f32x4 acc[AT][TT];

@@ -65,6 +65,9 @@ int umb_seq_linear(void* out, const void* x, const void* w, const void* bias, in
 int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype);
 /* the staged tile (csrc/gemm_tile.h's TILE_*) of a product of T tokens and `rows` rows of W whose K is summed in slabs (no stream) */
 int umb_seq_tile_kind(int T, int rows, int K, int slabs);
+/* Whether that launch (whole K) takes its whole rounds of 256 x 256 tiles and the rows behind them in tiles of fewer tokens: 7 x (256-row columns of the
+   whole rounds) + the tile behind them, 0 where it does not. */
+int umb_seq_tile_mix(int T, int rows, int K);
 int umb_seq_linear_parts(float* out, const void* x, const void* w, const void* bias, int T, int N, int K, int parts, int dtype,
                          umb_stream_t stream);
 

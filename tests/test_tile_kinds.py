@@ -175,3 +175,31 @@ def test_batched_gates_to_the_ends_of_their_range(epi):
     # the product's sums, one rounding to 16 bits (least steps 2^-133), gates whose exponential is beyond 32 bits
     bound = 2.0 ** -24 * (K + 4) * size * s + 1.02 * 2.0 ** -8 * want.abs() + want.abs() * (s < 2.95e-39) + 2.0 ** -134
     assert ((got - want).abs() <= bound)[~want.isnan()].all()
+
+
+# whole rounds of 256 x 256 tiles with the columns behind them in another tile: (T, N, K, columns, tile); rows stored as whole lines, in quads, one by one
+MIXED = [(1027, 22488, 192, 51, "192"), (1318, 18735, 64, 42, "192"), (1030, 22029, 192, 51, "160"), (1559, 14468, 64, 36, "160"), (486, 37771, 192, 128, "128 wide"),
+         (1162, 17976, 320, 51, "128 wide"), (643, 30628, 64, 85, "96"), (491, 32774, 192, 128, "96")]
+MIXED_PACKED = [(1308, 18720, 128, 42, "192"), (1540, 14496, 256, 36, "160"), (483, 37152, 128, 128, "128 wide"), (482, 32928, 384, 128, "96")]
+
+
+def test_mixed_shapes_get_the_tiles_they_are_listed_for():
+    from umbrella_amd import _lib
+    for T, N, K, columns, tile in MIXED + MIXED_PACKED:
+        got = _lib.load_seq().umb_seq_tile_mix(T, N, K)
+        assert (got // len(TILES), TILES[got % len(TILES)]) == (columns, tile), (T, N, K)
+    assert {m[-1] for m in MIXED} == {m[-1] for m in MIXED_PACKED} == {"192", "160", "128 wide", "96"}
+    for T, N, K in [(2048, 16384, 2048), (256, 65536, 64), (1024, 8192, 4096), (300, 1000, 64)]:         # whole rounds, or less than one
+        assert _lib.load_seq().umb_seq_tile_mix(T, N, K) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,N,K", [s[:3] for s in MIXED])
+def test_mixed_tiles(T, N, K):
+    test_every_tile(T, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,N,K", [s[:3] for s in MIXED_PACKED])
+def test_mixed_tiles_of_packed_weights(T, N, K):
+    test_every_tile_of_packed_weights(T, N, K, 1)

@@ -10,17 +10,14 @@
 #include "gemm_tile.h"
 #include <cstdlib>
 
+// A workgroup of the launch: tile number `tile` of nbt token tiles a column, slab sp of S, the columns from row `first` on.
 template <typename P, int WM, int WN, int RA, int RB, int KS>
-__global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS == 4 ? 2 : 1)
-void dgemm_kernel(const unsigned char* __restrict__ wp, const u16* __restrict__ x, int ldx, int T, int N, int K, int S, int epi, int nbt,
-                  float* __restrict__ out, GemmFused fx) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+__device__ __forceinline__ void dgemm_block(unsigned char* smem, const unsigned char* __restrict__ wp, const u16* __restrict__ x, int ldx, int T, int N, int K,
+                                            int S, int epi, int nbt, float* __restrict__ out, const GemmFused& fx, int tile, int sp, int first) {
   typedef TileShape<WM, WN, RA, RB, KS> Sh;
   const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = wave_all % Sh::NW, ks = wave_all / Sh::NW, j = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
-  const int id = tile_of_block(blockIdx.x, gridDim.x), tiles = gridDim.x / S;
-  const int sp = id / tiles, tile = id % tiles;
-  const int n0 = (tile / nbt) * Sh::BN, t0 = (tile % nbt) * Sh::BT;
+  const int n0 = first + (tile / nbt) * Sh::BN, t0 = (tile % nbt) * Sh::BT;
   const int nst = K / 64, per = (nst + S - 1) / S, st0 = min(nst, sp * per), st1 = min(nst, st0 + per);
   const int last = (N - n0) / 16 - 1;                        // row tiles and rows past the operand's end re-read its last one: not stored
   unsigned voff[Sh::NPW];
@@ -81,6 +78,45 @@ void dgemm_kernel(const unsigned char* __restrict__ wp, const u16* __restrict__ 
 }
 
 template <typename P, int WM, int WN, int RA, int RB, int KS>
+__global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS == 4 ? 2 : 1)
+void dgemm_kernel(const unsigned char* __restrict__ wp, const u16* __restrict__ x, int ldx, int T, int N, int K, int S, int epi, int nbt,
+                  float* __restrict__ out, GemmFused fx) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int id = tile_of_block(blockIdx.x, gridDim.x), tiles = gridDim.x / S;
+  dgemm_block<P, WM, WN, RA, RB, KS>(smem, wp, x, ldx, T, N, K, S, epi, nbt, out, fx, id % tiles, id / tiles, 0);
+}
+
+// whole rounds of 256 x 256 tiles (the first `whole` workgroups), then the rows behind them in tiles of fewer tokens (tile_mix)
+template <typename P, int RB>
+__global__ __launch_bounds__(512, 1)
+void dgemm_mixed_kernel(const unsigned char* __restrict__ wp, const u16* __restrict__ x, int ldx, int T, int N, int K, int epi, int nbt, int nbt_tail,
+                        int whole, int first, float* __restrict__ out, GemmFused fx) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int b = blockIdx.x;
+  if (b < whole) dgemm_block<P, 4, 2, 4, 8, 1>(smem, wp, x, ldx, T, N, K, 1, epi, nbt, out, fx, tile_of_block(b, whole), 0, 0);
+  else dgemm_block<P, 4, 2, 4, RB, 1>(smem, wp, x, ldx, T, N, K, 1, epi, nbt_tail, out, fx, tile_of_block(b - whole, gridDim.x - whole), 0, first);
+}
+
+template <typename P, int RB>
+static int dgemm_launch_mixed(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int epi, int columns, const GemmFused& fx, hipStream_t st) {
+  typedef TileShape<4, 2, 4, 8, 1> Sh;
+  typedef TileShape<4, 2, 4, RB, 1> Tail;
+  constexpr int LDS = (int)(Sh::LDS > Tail::LDS ? Sh::LDS : Tail::LDS);
+  static bool attr_done[64] = {};
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  if (dev >= 0 && dev < 64 && !attr_done[dev]) {
+    if (hipFuncSetAttribute((const void*)dgemm_mixed_kernel<P, RB>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return UMB_EHIP;
+    attr_done[dev] = true;
+  }
+  const int first = columns * Sh::BN, nbt = (T + Sh::BT - 1) / Sh::BT, nbt_tail = (T + Tail::BT - 1) / Tail::BT, whole = columns * nbt;
+  hipLaunchKernelGGL((dgemm_mixed_kernel<P, RB>), dim3((unsigned)whole + (N - first + Sh::BN - 1) / Sh::BN * nbt_tail), dim3(512), LDS, st,
+                     (const unsigned char*)wp, x, ldx, T, N, K, epi, nbt, nbt_tail, whole, first, out, fx);
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+
+template <typename P, int WM, int WN, int RA, int RB, int KS>
 static int dgemm_launch(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int S, int epi, const GemmFused& fx, hipStream_t st) {
   typedef TileShape<WM, WN, RA, RB, KS> Sh;
   static bool attr_done[64] = {};
@@ -136,7 +172,18 @@ static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, i
       default: return dgemm_launch<P, 2, 2, 4, 2, 2>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     }
   }
-  switch (dgemm_tile(T, N, K, S)) {
+  double us;
+  const int kind = dgemm_tile(T, N, K, S, &us);
+  if (S == 1) {
+    const TileMix mix = tile_mix(T, N, K / 64, us);
+#define MIXED(KIND, RB) if (mix.columns && mix.tail == KIND) return dgemm_launch_mixed<P, RB>(wp, x, ldx, out, T, N, K, epi, mix.columns, fx, st)
+    MIXED(TILE_192, 6);
+    MIXED(TILE_160, 5);
+    MIXED(TILE_128W, 4);
+    MIXED(TILE_96, 3);
+#undef MIXED
+  }
+  switch (kind) {
     case TILE_256: return dgemm_launch<P, 4, 2, 4, 8, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     case TILE_192: return dgemm_launch<P, 4, 2, 4, 6, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     case TILE_160: return dgemm_launch<P, 4, 2, 4, 5, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);

@@ -87,6 +87,29 @@ static inline int tile_kind(int T, int rows, int stages, int S, bool even, doubl
   return best;
 }
 
+// More 256 x 256 tiles than whole rounds of 256 workgroups: the whole rounds take the first `columns` 256-row columns, the columns that are left go in
+// tiles of `tail`'s tokens (256 rows too) behind them in the same launch, chosen as above (the first of them run beside the last round's end).  columns 0: no.
+// What it may save is the last round's idle share, so it has to be 3 % ahead.
+struct TileMix { int columns, tail; };
+static inline TileMix tile_mix(int T, int rows, int stages, double single) {
+  static const struct { int kind, bt; double us; } k[4] = {{TILE_192, 192, 1.20}, {TILE_160, 160, 1.04}, {TILE_128W, 128, 0.86}, {TILE_96, 96, 0.73}};
+  const long nbt = (T + 255) / 256, all = (rows + 255L) / 256 * nbt, rounds = all / 256;
+  TileMix best{0, 0};
+  if (rounds == 0 || all % 256 == 0 || nbt > 256) return best;
+  const int columns = (int)(256 * rounds / nbt);
+  const long tail = (rows + 255) / 256 - columns, spare = 256 * rounds - columns * nbt;
+  if (tail <= 0) return best;
+  const double main = 4.0 + rounds * (stages * 1.42 + 2.1e-4 * 256 * 256 + 2.0);
+  double least = 0.97 * single;
+  for (int i = 0; i < 4; ++i) {
+    const long wgs = tail * ((T + k[i].bt - 1) / k[i].bt) - spare, rest = wgs > 0 ? wgs % 256 : 0;
+    const double load = rest / 256.0, products = stages * k[i].us, out = 2.1e-4 * 256 * k[i].bt;
+    const double us = main + (wgs > 0 ? wgs / 256 * (products + out + 2.0) : 0.0) + (rest ? products * (0.8 + 0.2 * load) + out * load + 2.0 : 0.0);
+    if (us < least) { least = us; best = TileMix{columns, k[i].kind}; }
+  }
+  return best;
+}
+
 // Row block of a workgroup: the hardware deals consecutive workgroups to the eight XCDs in turn; here the workgroups of one XCD get
 // consecutive tile numbers, so that the tiles its L2 serves share operand rows.
 __device__ __forceinline__ int tile_of_block(int b, int nb) {

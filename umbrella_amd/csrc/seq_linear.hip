@@ -364,19 +364,16 @@ __global__ __launch_bounds__(256) void seq_linear_wide_kernel(void* __restrict__
 // ---- many tokens, both operands dense with whole 64-k stages: the staged product of gemm_tile.h.  DUAL: a wave's RA row tiles are
 // RA / 2 tiles of gate rows and the up rows of the same outputs.  The k order of an output without K-split is the wide kernel's:
 // the same bits.
+// A workgroup of the launch: tile number id of nbt token tiles a column, slab sp of K, the columns from row `first` on.
 template <typename P, int WM, int WN, int RA, int RB, int KS, bool DUAL>
-__global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS == 4 ? 2 : 1)
-void seq_linear_tile_kernel(void* __restrict__ out_, const u16* __restrict__ x, const u16* __restrict__ w, const u16* __restrict__ bias,
-                            int T, int N, int K, int epi, int nbt, int slabs, float limit, float alpha) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+__device__ __forceinline__ void tile_block(unsigned char* smem, void* __restrict__ out_, const u16* __restrict__ x, const u16* __restrict__ w,
+                                           const u16* __restrict__ bias, int T, int N, int K, int epi, int nbt, int slabs, float limit, float alpha,
+                                           int tile, int sp, int first) {
   typedef TileShape<WM, WN, RA, RB, KS> S;
   constexpr int OUTN = DUAL ? S::BN / 2 : S::BN;
   const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = wave_all % S::NW, ks = wave_all / S::NW, j = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
-  // (quotients go through the vector pipe: named uniform, or the addresses built on them are not)
-  const int id = tile_of_block(blockIdx.x, gridDim.x), tiles = __builtin_amdgcn_readfirstlane(gridDim.x / slabs);
-  const int sp = __builtin_amdgcn_readfirstlane(id / tiles), tile = id - sp * tiles, column = __builtin_amdgcn_readfirstlane(tile / nbt);
-  const int n0 = column * OUTN, t0 = (tile - column * nbt) * S::BT;
+  const int column = __builtin_amdgcn_readfirstlane(tile / nbt), n0 = first + column * OUTN, t0 = (tile - column * nbt) * S::BT;
   // slab sp of K (one more stage in the first ones): its sums go to out + sp T N, the bias into slab 0's
   const int each = __builtin_amdgcn_readfirstlane(K / 64 / slabs), longer = K / 64 - each * slabs, st0 = sp * each + min(sp, longer), stages = each + (sp < longer);
   // rows past the operand's end re-read its last row: their outputs are not stored
@@ -477,6 +474,43 @@ void seq_linear_tile_kernel(void* __restrict__ out_, const u16* __restrict__ x, 
     else if (epi == EPI_CAP) finish(std::integral_constant<int, EPI_CAP>{});
     else finish(std::integral_constant<int, EPI_F32>{});
   }
+}
+
+template <typename P, int WM, int WN, int RA, int RB, int KS, bool DUAL>
+__global__ __launch_bounds__(64 * WM * WN * KS, WM * WN * KS == 4 ? 2 : 1)
+void seq_linear_tile_kernel(void* __restrict__ out, const u16* __restrict__ x, const u16* __restrict__ w, const u16* __restrict__ bias,
+                            int T, int N, int K, int epi, int nbt, int slabs, float limit, float alpha) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  // (quotients go through the vector pipe: named uniform, or the addresses built on them are not)
+  const int id = tile_of_block(blockIdx.x, gridDim.x), tiles = __builtin_amdgcn_readfirstlane(gridDim.x / slabs), sp = __builtin_amdgcn_readfirstlane(id / tiles);
+  tile_block<P, WM, WN, RA, RB, KS, DUAL>(smem, out, x, w, bias, T, N, K, epi, nbt, slabs, limit, alpha, id - sp * tiles, sp, 0);
+}
+
+// Whole rounds of 256 x 256 tiles (the first `whole` workgroups), then the columns that are left in tiles of fewer tokens (tile_mix): a last round of
+// 256 x 256 tiles takes as long as the others however few it has.
+template <typename P, int RB, bool DUAL>
+__global__ __launch_bounds__(512, 1)
+void seq_linear_mixed_kernel(void* __restrict__ out, const u16* __restrict__ x, const u16* __restrict__ w, const u16* __restrict__ bias,
+                             int T, int N, int K, int epi, int nbt, int nbt_tail, int whole, int first, float limit, float alpha) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int b = blockIdx.x;
+  if (b < whole) tile_block<P, 4, 2, 4, 8, 1, DUAL>(smem, out, x, w, bias, T, N, K, epi, nbt, 1, limit, alpha, tile_of_block(b, whole), 0, 0);
+  else tile_block<P, 4, 2, 4, RB, 1, DUAL>(smem, out, x, w, bias, T, N, K, epi, nbt_tail, 1, limit, alpha, tile_of_block(b - whole, gridDim.x - whole), 0, first);
+}
+
+template <typename P, int RB, bool DUAL>
+static int launch_mixed(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, int columns, float limit, float alpha,
+                        hipStream_t st) {
+  typedef TileShape<4, 2, 4, 8, 1> S;
+  typedef TileShape<4, 2, 4, RB, 1> Tail;
+  constexpr int OUTN = DUAL ? S::BN / 2 : S::BN;
+  constexpr size_t LDS = S::LDS > Tail::LDS ? S::LDS : Tail::LDS;
+  if (ensure_dynamic_lds<seq_linear_mixed_kernel<P, RB, DUAL>>(LDS) != UMB_OK) return UMB_EHIP;
+  const int first = columns * OUTN, nbt = (T + S::BT - 1) / S::BT, nbt_tail = (T + Tail::BT - 1) / Tail::BT, whole = columns * nbt;
+  hipLaunchKernelGGL((seq_linear_mixed_kernel<P, RB, DUAL>), dim3((unsigned)whole + (N - first + OUTN - 1) / OUTN * nbt_tail), dim3(512), LDS, st,
+                     out, (const u16*)x, (const u16*)w, (const u16*)bias, T, N, K, epi, nbt, nbt_tail, whole, first, limit, alpha);
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
 }
 
 template <typename P, int WM, int WN, int RA, int RB, int KS, bool DUAL>
@@ -589,7 +623,18 @@ static int launch_tile_batched(void* out, const void* x, const void* w, int T, i
 template <typename P, bool DUAL>
 static int launch_tile(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, int slabs, float limit,
                        float alpha, hipStream_t st) {
-  switch (tile_kind(T, DUAL ? 2 * N : N, (K / 64 + slabs - 1) / slabs, slabs, K % (128 * slabs) == 0)) {
+  double us;
+  const int kind = tile_kind(T, DUAL ? 2 * N : N, (K / 64 + slabs - 1) / slabs, slabs, K % (128 * slabs) == 0, &us);
+  if (slabs == 1) {
+    const TileMix mix = tile_mix(T, DUAL ? 2 * N : N, K / 64, us);
+#define MIXED(KIND, RB) if (mix.columns && mix.tail == KIND) return launch_mixed<P, RB, DUAL>(out, x, w, bias, T, N, K, epi, mix.columns, limit, alpha, st)
+    MIXED(TILE_192, 6);
+    MIXED(TILE_160, 5);
+    MIXED(TILE_128W, 4);
+    MIXED(TILE_96, 3);
+#undef MIXED
+  }
+  switch (kind) {
     case TILE_256: return launch_tile_as<P, 4, 2, 4, 8, 1, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
     case TILE_192: return launch_tile_as<P, 4, 2, 4, 6, 1, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
     case TILE_160: return launch_tile_as<P, 4, 2, 4, 5, 1, DUAL>(out, x, w, bias, T, N, K, epi, slabs, limit, alpha, st);
@@ -1043,6 +1088,14 @@ static int tile_slabs(int T, int N, int K, bool stream) {
 extern "C" int umb_seq_tile_kind(int T, int rows, int K, int slabs) {
   if (T < 1 || rows < 1 || K < 64 || slabs < 1) return UMB_EINVAL;
   return tile_kind(T, rows, (K / 64 + slabs - 1) / slabs, slabs, K % (128 * slabs) == 0);
+}
+
+extern "C" int umb_seq_tile_mix(int T, int rows, int K) {
+  if (T < 1 || rows < 1 || K < 64) return UMB_EINVAL;
+  double us;
+  (void)tile_kind(T, rows, K / 64, 1, K % 128 == 0, &us);
+  const TileMix mix = tile_mix(T, rows, K / 64, us);
+  return mix.columns * TILE_KINDS + mix.tail;
 }
 
 extern "C" int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype) {

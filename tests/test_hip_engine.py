@@ -865,3 +865,20 @@ def test_captures_beside_another_threads_event_queries(dev):
     for _ in range(3):
         graph.replay()
     assert bool((x == 6000.0).all())
+
+
+def test_prompt_in_one_chunk_and_in_many(dev):
+    """1500 tokens in one forward (more 16-row query tiles than 1024 tokens have, several spans of keys each) and in forwards of 256"""
+    from hip_helpers import hip_model
+    P, got = 1500, []
+    ids = torch.randint(0, G["target_cfg"]["vocab_size"], (P,), generator=torch.Generator().manual_seed(3)).to(torch.int32).to(dev)
+    for chunk in (2048, 256):
+        m, _ = hip_model(dict(G["target_cfg"], max_position_embeddings=4096), G["seeds"]["target"], 2600, torch.float16, dev)
+        assert m.PREFILL_CHUNK == 2048
+        m.reserve(min(chunk, P), logit_rows=64)
+        first = m.prefill_tokens(ids, 0).clone()
+        step = m.inference(ids[None, :3].long(), torch.tensor([[P, P + 1, P + 1]], device=dev),
+                           torch.ones(3, P + 3, dtype=torch.bool, device=dev).tril(P), torch.arange(P, P + 3, device=dev))
+        got.append((first, step[0]))
+    for a, b in zip(*got):
+        assert torch.isfinite(a).all() and (a - b).abs().max() < 0.06          # fp16 keys behind another order of sums, as in TOL

@@ -191,7 +191,9 @@ class Llama(LLMBase):
     CHUNK = 64          # rows of the default workspace (tree / generic forwards)
     PREFILL_CHUNK = 1024  # prompt tokens per forward when the workspace allows: the matrix-bound verify GEMM streams the
                           # weights once per chunk (70B-AWQ, 2048-token prompt: 4.2 k tok/s at 128, 6.1 k at 256, 6.7 k at
-                          # 512, 7.0 k at 1024; 1B: 53 k / 94 k / 155 k / 211 k).  1024 = rows of the attention counters.
+                          # 512, 7.0 k at 1024; 1B: 53 k / 94 k / 155 k / 211 k)
+    PREFILL_CHUNK_DENSE = 2048   # the same of 16-bit weights, whose products have no limit of 1024 rows: fewer partial sums, whole rounds of tiles, one walk
+                                 # over the keys (8B widths, 2048-token prompt and one token: 8526 -> 7751 us)
 
     def __init__(self, model_name: str, batch_size: int = 1, max_length: int = 256, device: str = "cuda:0",
                  dtype=torch.float16, offload: bool = False, cuda_graph: bool = False, state_dict=None,
@@ -229,6 +231,8 @@ class Llama(LLMBase):
         if self.sched == "auto":
             self.sched = "split" if (self.config.awq or self.config.hidden_size >= 4096) else "ll"
         c = self.config
+        if not c.awq:
+            self.PREFILL_CHUNK = self.PREFILL_CHUNK_DENSE
         if c.attention_bias:
             self.fused = False                    # projection bias: default / low-latency schedules only
         self.hidden_size, self.num_heads, self.head_dim = c.hidden_size, c.num_attention_heads, c.head_dim
@@ -601,9 +605,10 @@ class Llama(LLMBase):
         maxn = max(N for (N, K, S) in self._plans.values())
         if not hasattr(self, "_counters"):          # self-resetting arrival counters (zero between launches)
             self._counters = torch.zeros(maxn // 64 + 64, dtype=torch.int32, device=dev)
-            g = c.num_attention_heads // c.num_key_value_heads
-            self._attn_counters = torch.zeros(c.num_key_value_heads * ((1024 * g + 15) // 16) + 64, dtype=torch.int32,
-                                              device=dev)      # one per (kv head, 16-row query tile), T <= 1024
+        g = c.num_attention_heads // c.num_key_value_heads
+        tiles = c.num_key_value_heads * ((max(1024, T) * g + 15) // 16) + 64                # one per (kv head, 16-row query tile)
+        if not hasattr(self, "_attn_counters") or self._attn_counters.numel() < tiles:
+            self._attn_counters = torch.zeros(tiles, dtype=torch.int32, device=dev)
         ws = self._ws = UmbWorkspace()
         ws.h, ws.xn, ws.q, ws.attn, ws.act = (w[k].data_ptr() for k in ("h", "xn", "q", "attn", "act"))
         ws.partial, ws.attn_po, ws.attn_ml = w["partial"].data_ptr(), w["po"].data_ptr(), w["ml"].data_ptr()

@@ -232,6 +232,11 @@ int umb_lat_front(void* qn, float* qa, const UmbPagedKV* kv, const float* proj, 
  * denominator (exp(sink[h]): no key, no value, not scaled; sink may be null); out [T][H][kv_rank] in `dtype`. */
 int umb_lat_attend(void* out, const float* qa, const UmbPagedKV* kv, const void* sink, const int* pos, const int* slot, int T,
                    int H, int kv_rank, int rot_dim, int window, float scale, int dtype, umb_stream_t stream);
+/* the same with room for partial results: where a token's heads are few workgroups, spans of 64 keys go to several (as many as 16; T H <= 256 and kv_rank
+ * of 64, 128, 256 or 512: scratch of T H 16 (kv_rank + 2) floats holds them all, less of it fewer; null: none) */
+int umb_lat_attend_split(void* out, const float* qa, const UmbPagedKV* kv, const void* sink, const int* pos, const int* slot, int T,
+                         int H, int kv_rank, int rot_dim, int window, float scale, float* scratch, long scratch_floats, int dtype,
+                         umb_stream_t stream);
 /* the same for steps that bring stretches of a sequence, on the matrix pipe: workgroups own 16 consecutive positions of
  * one sequence.  umb_lat_attend_tiled_ok says (1 / 0) whether the kernel covers a shape and dtype; it has no stream. */
 int umb_lat_attend_tiled(void* out, const float* qa, const UmbPagedKV* kv, const void* sink, const int* seq_slot,
@@ -595,6 +600,8 @@ typedef struct UmbSeqWork {
   void* h2;            /* parallel blocks: normed input of the feed-forward [Tmax][W] dtype */
   float* y2;           /* parallel blocks: feed-forward output; mixers with two output projections: the second [Tmax][W] fp32 */
   float* v_first;      /* values that later layers of the step mix in [Tmax][kv_heads vdim] fp32 (null when no layer does) */
+  float* part;         /* partial results of split keys of latent layers, 256 * 16 * (kv_rank + 2) floats hold them all (null: none are split) */
+  int64_t part_floats;
 } UmbSeqWork;
 
 typedef struct UmbSeqStep {

@@ -274,7 +274,7 @@ class UmbSeqWork(C.Structure):
                 ("Tmax", C.c_int32), ("Rmax", C.c_int32), ("moe_sel", C.c_void_p), ("moe_wt", C.c_void_p),
                 ("moe_pos", C.c_void_p), ("moe_tiles", C.c_void_p), ("moe_xs", C.c_void_p), ("moe_act", C.c_void_p),
                 ("moe_y", C.c_void_p), ("moe_max_tiles", C.c_int32), ("y_rows", C.c_int32), ("aux_floats", C.c_int64),
-                ("h2", C.c_void_p), ("y2", C.c_void_p), ("v_first", C.c_void_p)]
+                ("h2", C.c_void_p), ("y2", C.c_void_p), ("v_first", C.c_void_p), ("part", C.c_void_p), ("part_floats", C.c_int64)]
 
 
 class UmbSeqStep(C.Structure):
@@ -311,6 +311,7 @@ SEQ_SIGNATURES = {
     "umb_lat_qsplit": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I],
     "umb_lat_front": [_P, _P, _PKV, _P, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _I],
     "umb_lat_attend": [_P, _P, _PKV, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I],
+    "umb_lat_attend_split": [_P, _P, _PKV, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _L, _I],
     "umb_lat_attend_tiled": [_P, _P, _PKV, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I],
     "umb_lat_attend_tiled_ok": [_I, _I, _I, _I],
     "umb_seq_group_norm": [_P, _P, _P, _P, _P, _I, _I, _I, _F, _I],

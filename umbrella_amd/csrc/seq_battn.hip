@@ -209,7 +209,12 @@ __device__ __forceinline__ AttnKeys attn_keys(int i, int window, const UmbAttnFo
 // end of a workgroup: the partial sums o_s [nact][RH][Ep], maxima and denominators ml_s [nact][RH][2] (and 2 RH floats behind the nw-th)
 // of its waves, added in wave order; nact <= 16: a row's factors are worked out once, by 16 lanes.
 // part: this split's result goes there instead ([token][row][split][E + 2] = o .., maximum, denominator)
-template <typename P, int RH, int NC, int MAPS>
+// a head's sink: fp32, or a latent layer's in storage format
+template <typename P, bool LAT> __device__ __forceinline__ float sink_of(const float* sink, int h) {
+  if constexpr (LAT) return P::to_f(reinterpret_cast<const u16*>(sink)[h]);
+  else return sink[h];
+}
+template <typename P, int RH, int NC, int MAPS, bool LAT = false>
 __device__ __forceinline__ void attn_finish(typename El<P>::type* __restrict__ out, int ldo, const float* o_s, int Ep, float* ml_s,
                                             int nact, int nw, float* __restrict__ part, int split, int nsplit,
                                             const float* __restrict__ proj, int ld, int gate_col, int t, int h0, int H, int E,
@@ -231,11 +236,33 @@ __device__ __forceinline__ void attn_finish(typename El<P>::type* __restrict__ o
     for (int w = 0; w < nact; ++w) o += o_s[(w * RH + r) * Ep + d] * ml_s[(w * RH + r) * 2];
     return o;
   };
-  auto denominator = [&](int r) -> float { return row_s[2 * r + 1] + (form.sink ? expf(form.sink[h0 + r / MAPS] - row_s[2 * r]) : 0.f); };
+  auto denominator = [&](int r) -> float { return row_s[2 * r + 1] + (form.sink ? expf(sink_of<P, LAT>(form.sink, h0 + r / MAPS) - row_s[2 * r]) : 0.f); };
   auto gate_of = [&](int h, int d) {
     return gate_col >= 0 ? 1.f / (1.f + expf(-proj[(long)t * ld + gate_col + (form.gate_elem ? h * E + d : h)])) : 1.f;
   };
-  if (MAPS == 1 || part) {
+  if ((MAPS == 1 || part) && E % 4 == 0 && Ep % 4 == 0) {  // four columns a thread: a column a thread was up to eight rounds of the waves' sums
+    typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
+    const int per = E >> 2;
+    for (int x = threadIdx.x; x < RH * per; x += nw * 64) {
+      const int r = x / per, d = x % per * 4;
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+      for (int w = 0; w < nact; ++w) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(o_s + (w * RH + r) * Ep + d);
+        const float f = ml_s[(w * RH + r) * 2];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] += v[e] * f;
+      }
+      if (part) {
+        float* pr = part + ((((long)t * H + h0) * MAPS + r) * nsplit + split) * (E + 2);
+        *reinterpret_cast<quad*>(pr + d) = o;
+        if (d == 0) { pr[E] = row_s[2 * r]; pr[E + 1] = row_s[2 * r + 1]; }
+        continue;
+      }
+      const float L = denominator(r);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) stf<P>(out + (long)t * ldo + (long)(h0 + r) * E + d + e, out_scale * gate_of(h0 + r, d + e) * (o[e] / L));
+    }
+  } else if (MAPS == 1 || part) {
     for (int x = threadIdx.x; x < RH * E; x += nw * 64) {
       const int r = x / E, d = x % E;
       const float o = merged(r, d);
@@ -420,9 +447,15 @@ __global__ __launch_bounds__(NW * 64) void bsa_attend_kernel(typename El<P>::typ
 // Before -> now, replayed from a graph: 48 tokens behind 40 keys of 64 features 19.1 -> 6.2 us, behind 500 29.4 -> 20.5; one token behind
 // 40 / 2000 keys of 128 features 16.0 -> 7.4 / 19.2 -> 12.8 (spans of 1024: 22.0); two maps, values of 256, one token behind 40 / 1000
 // 23.0 -> 9.5 / 27.2 -> 19.8; 64 tokens behind 1000, 128 features, 81 -> 51 (262 MB of rows, 5.1 TB/s).
-constexpr int ATT_SPAN = 256;
+// Few rows in all go two to a workgroup and not four: a wave's products halve and twice the units have some (one token, two maps of 128 | 256 behind 77 keys 9.7 -> 8.7 us,
+// a sink of 128 7.4 -> 6.3, 32 + 8 heads of 128 behind 2000 12.4 -> 10.2).
+// LAT: latent attention (one row a token for all heads, kv.k; its first E columns are the values).  A round of 16 keys of it is some 4 us of one wave's products,
+// so a span that goes to a workgroup of its own is 64 keys, four waves.  us, rounds of 64 keys with a key a lane and single columns a lane (lat_attend_kernel, which
+// keeps the other shapes) / this with the merge, 32 heads of 512 + 64: one token behind 40 / 300 / 2000 keys (1024 of a window) 23.3 / 30.9 / 57.6 -> 9.9 / 12.1 / 12.8,
+// 16 behind 100 29.5 -> 14.4, 40 behind 100 82 -> 27.6; 16 heads of 256 + 32: one behind 40 / 2000 19.7 / 26.0 -> 7.2 / 9.4, 40 behind 60 23.0 -> 8.4.
+constexpr int ATT_SPAN = 256, LAT_SPAN = 64;
 
-template <typename P, int RH, int LPR, int NW, int MAPS>
+template <typename P, int RH, int LPR, int NW, int MAPS, bool LAT = false>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q, UmbPagedKV kv,
                                                               const float* __restrict__ proj, int ld, int gate_col,
                                                               const float* __restrict__ bias, int n_dist, const int* __restrict__ pos,
@@ -430,6 +463,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
                                                               float out_scale, float softcap, UmbAttnForm form, float* __restrict__ part,
                                                               int nsplit) {
   constexpr int E = LPR * 8, KPI = 64 / LPR, VL = 16 / KPI, RR = RH / MAPS;
+  constexpr int SPAN = LAT ? LAT_SPAN : ATT_SPAN;
+  static_assert(!LAT || MAPS == 1, "one map");
+  const int ldv = LAT ? D : E;                             // elements between two value rows
   extern __shared__ float lds[];
   const int split = blockIdx.z, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, quarter = lane >> 4;
   float* q_s = lds;                                        // [RH][D]
@@ -438,14 +474,16 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
   const int t = blockIdx.x, h0 = blockIdx.y * RR, g = h0 / (H / G);
   const int i = pos[t], slot = slot_[t];
   const AttnKeys keys = attn_keys(i, window, form);
-  const int first = split * ATT_SPAN;
+  const int first = split * SPAN;
   if (first >= keys.n) return;
-  const int nact = min(NW, (min(keys.n - first, ATT_SPAN) + 15) / 16);       // waves that get a round
+  const int nact = min(NW, ((nsplit > 1 ? min(keys.n - first, SPAN) : keys.n) + 15) / 16);       // waves that get a round
   auto key_pos = [&](int kx) { return kx < keys.kept ? kx : keys.j_lo + kx - keys.kept; };
   int base = first + wave * 16;
   unsigned row = 0;
   if (wave < nact) row = pkv_tok_row(kv, slot, key_pos(min(base + j, keys.n - 1)), g, G);
-  for (int x = threadIdx.x; x < RH * D; x += NW * 64) q_s[x] = q[((long)t * H + h0) * MAPS * D + x];
+  typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
+  for (int x = threadIdx.x; x < RH * D / 4; x += NW * 64)      // (D: a multiple of 32)
+    *reinterpret_cast<f32x4*>(q_s + 4 * x) = *reinterpret_cast<const quad*>(q + ((long)t * H + h0) * MAPS * D + 4 * x);
   __syncthreads();
   if (wave < nact) {
     float acc[RH * 8], m_run[RH], l_run[RH];
@@ -453,12 +491,12 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
     for (int r = 0; r < RH; ++r) { m_run[r] = -INFINITY; l_run[r] = 0.f; }
 #pragma unroll
     for (int v = 0; v < RH * 8; ++v) acc[v] = 0.f;
-    const u16* vcol = reinterpret_cast<const u16*>(kv.v) + (lane & (LPR - 1)) * 8;
+    const u16* vcol = reinterpret_cast<const u16*>(LAT ? kv.k : kv.v) + (lane & (LPR - 1)) * 8;
     while (base < keys.n) {
       const int kx = base + j;
       u32x4 vv[VL];
 #pragma unroll
-      for (int u = 0; u < VL; ++u) vv[u] = *reinterpret_cast<const u32x4*>(vcol + (long)(unsigned)__shfl((int)row, KPI * u + lane / LPR, 64) * E);
+      for (int u = 0; u < VL; ++u) vv[u] = *reinterpret_cast<const u32x4*>(vcol + (long)(unsigned)__shfl((int)row, KPI * u + lane / LPR, 64) * ldv);
       const u16* kr = reinterpret_cast<const u16*>(kv.k) + (long)row * (MAPS * D) + quarter * 8;
       const int dist = i - key_pos(min(kx, keys.n - 1));
       float bv[RR];
@@ -467,7 +505,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
       for (int r = 0; r < RR; ++r) bv[r] = bias ? bias[(long)(h0 + r) * n_dist + bi] : 0.f;
       // the next round of this wave: NW rounds on, or in the next of its workgroup's spans
       int next = base + NW * 16;
-      if (nsplit > 1 && next / ATT_SPAN != base / ATT_SPAN) next += (nsplit - 1) * ATT_SPAN;
+      if (nsplit > 1 && next / SPAN != base / SPAN) next += (nsplit - 1) * SPAN;
       unsigned next_row = 0;
       if (next < keys.n) next_row = pkv_tok_row(kv, slot, key_pos(min(next + j, keys.n - 1)), g, G);
       float s[RH];
@@ -534,23 +572,24 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
     store_groups<RH, LPR>(o_s + wave * RH * E, acc, lane);
   }
   __syncthreads();
-  attn_finish<P, RH, (E + 63) / 64, MAPS>(out, ldo, o_s, E, ml_s, nact, NW, keys.n > ATT_SPAN && nsplit > 1 ? part : nullptr, split, nsplit,
+  attn_finish<P, RH, (E + 63) / 64, MAPS, LAT>(out, ldo, o_s, E, ml_s, nact, NW, keys.n > SPAN && nsplit > 1 ? part : nullptr, split, nsplit,
                                           proj, ld, gate_col, t, h0, H, E, out_scale, form);
 }
 
 // the splits of one (token, head) merged: lane s holds split s's maximum and denominator (a split that had no key carries
 // M = -inf, L = 0), the factors go round by shuffles, every sum runs over the splits in order
-template <typename P, int MAPS>
-__global__ __launch_bounds__(64) void bsa_merge_kernel(typename El<P>::type* __restrict__ out, int ldo, const float* __restrict__ part,
+// (one map: a wave for every 64 columns, each with the factors of its own; 64 columns after the other were a round trip each)
+template <typename P, int MAPS, bool LAT = false>
+__global__ __launch_bounds__(MAPS == 1 ? 512 : 64) void bsa_merge_kernel(typename El<P>::type* __restrict__ out, int ldo, const float* __restrict__ part,
                                                        const float* __restrict__ proj, int ld, int gate_col, int H, int E,
                                                        int splits, float out_scale, UmbAttnForm form, const int* __restrict__ pos,
                                                        int window) {
-  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
   int nsplit = splits;
   if (window > 0) {                                       // splits by spans: those that had keys, none if one workgroup did it all
     const int n = attn_keys(pos[t], window, form).n;
-    if (n <= ATT_SPAN) return;
-    nsplit = min(splits, (n + ATT_SPAN - 1) / ATT_SPAN);
+    if (n <= (LAT ? LAT_SPAN : ATT_SPAN)) return;
+    nsplit = min(splits, (n + (LAT ? LAT_SPAN : ATT_SPAN) - 1) / (LAT ? LAT_SPAN : ATT_SPAN));
   }
   auto gate_of = [&](int d) {
     return gate_col >= 0 ? 1.f / (1.f + expf(-proj[(long)t * ld + gate_col + (form.gate_elem ? h * E + d : h)])) : 1.f;
@@ -570,7 +609,7 @@ __global__ __launch_bounds__(64) void bsa_merge_kernel(typename El<P>::type* __r
       f[mp][s] = __shfl(fs, s, 64);
       L += __shfl(ls * fs, s, 64);
     }
-    if (form.sink) L += expf(form.sink[h] - M);
+    if (form.sink) L += expf(sink_of<P, LAT>(form.sink, h) - M);
     inv[mp] = 1.f / L;
   }
   auto column = [&](int mp, int d) -> float {
@@ -584,7 +623,7 @@ __global__ __launch_bounds__(64) void bsa_merge_kernel(typename El<P>::type* __r
   };
   typename El<P>::type* orow = out + (long)t * ldo + (long)h * E;
   if constexpr (MAPS == 1) {
-    for (int d = lane; d < E; d += 64) stf<P>(orow + d, column(0, d) * (out_scale * gate_of(d)));
+    for (int d = threadIdx.x; d < E; d += blockDim.x) stf<P>(orow + d, column(0, d) * (out_scale * gate_of(d)));
   } else {
     float v[BSA_MAXC], ss = 0.f;
 #pragma unroll
@@ -670,12 +709,22 @@ static int bsa_launch(dim3 grid, size_t lds, hipStream_t st, void* out, int ldo,
 // the decode kernel: spans of ATT_SPAN keys dealt to several workgroups only where few items leave the chip idle; 16 waves per item as
 // long as every item gets a compute unit of its own (values of 256: their registers do not hold it), 8 while two share one, 4 beyond
 // (us with 8 / 4 waves, 32 + 8 heads of 128: 1024 items behind 30 / 200 keys 12.8 / 8.4, 30.2 / 27.5; 512 items behind 500 28.8 / 36.7)
+// workgroups that one item's spans of keys are dealt to; most: keys a token can have, floats: of one split of all items
+static inline int decode_splits(int span, long items, long most, long floats, const float* scratch, long scratch_floats) {
+  int nsplit = 1;
+  if (scratch && items <= 64 && most > span) {
+    nsplit = (int)(512 / items) < 16 ? (int)(512 / items) : 16;
+    if (nsplit > (most + span - 1) / span) nsplit = (int)((most + span - 1) / span);
+    while (nsplit > 1 && floats * nsplit > scratch_floats) nsplit >>= 1;
+  }
+  return nsplit;
+}
 template <typename P>
 static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const float* bias,
                        int n_dist, const int* pos, const int* slot, int T, int H, int G, int D, int E, int window, float scale,
                        float out_scale, float softcap, const UmbAttnForm& form, float* scratch, long scratch_floats, hipStream_t st) {
   const int maps = form.maps, hpg = H / G;
-  int rh = 4;
+  int rh = (long)T * H * maps <= 128 ? 2 : 4;
   while (rh > maps && hpg % (rh / maps)) rh >>= 1;
   const int hblocks = H * maps / rh;
   const long items = (long)T * hblocks;
@@ -683,12 +732,7 @@ static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv,
   // span of keys altogether, a single short conversation's: nobody splits there, and the merge behind it would find nothing to do (one token of 8B
   // widths in a cache of 192 positions, three layers 56 us -> 41 without the merges, 4.6 us each).  In a larger pool a short sequence's merge still runs.
   const long most = std::min((long)(form.chunk > 0 && form.chunk < window ? form.chunk : window) + form.keep_first, (long)kv->max_pages * kv->page);
-  int nsplit = 1;
-  if (scratch && items <= 64 && most > ATT_SPAN) {
-    nsplit = (int)(512 / items) < 16 ? (int)(512 / items) : 16;
-    if (nsplit > (most + ATT_SPAN - 1) / ATT_SPAN) nsplit = (int)((most + ATT_SPAN - 1) / ATT_SPAN);
-    while (nsplit > 1 && (long)T * H * maps * nsplit * (E + 2) > scratch_floats) nsplit >>= 1;
-  }
+  const int nsplit = decode_splits(ATT_SPAN, items, most, (long)T * H * maps * (E + 2), scratch, scratch_floats);
   const int nw = items <= 256 && E < 256 ? 16 : (items <= 512 ? 8 : 4);
   const size_t lds = ((size_t)rh * D + (size_t)nw * rh * E + (size_t)(nw + 1) * rh * 2) * sizeof(float);
 #define ATT_GO(RH, LPR, NW, MAPS)                                                                                                     \
@@ -714,11 +758,63 @@ static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv,
       hipLaunchKernelGGL((bsa_merge_kernel<P, 2>), dim3(T, H), dim3(64), 0, st, (u16*)out, ldo, scratch, proj, ld, gate_col, H, E, nsplit,
                          out_scale, form, pos, window);
     else
-      hipLaunchKernelGGL((bsa_merge_kernel<P, 1>), dim3(T, H), dim3(64), 0, st, (u16*)out, ldo, scratch, proj, ld, gate_col, H, E, nsplit,
+      hipLaunchKernelGGL((bsa_merge_kernel<P, 1>), dim3(T, H), dim3((unsigned)std::min(E + 63, 512) & ~63u), 0, st, (u16*)out, ldo, scratch, proj, ld, gate_col, H, E, nsplit,
                          out_scale, form, pos, window);
   }
   UMB_LAUNCH_CHECK();
   return UMB_OK;
+}
+
+// The same for latent rows of 64, 128, 256 or 512 columns and rotary columns behind them, a multiple of 32 in all; false: another kernel's
+static inline bool lat_decode_ok(int kv_rank, int rot_dim, int dtype, const UmbPagedKV* kv) {
+  return dtype != UMB_SEQ_F32 && (kv_rank == 64 || kv_rank == 128 || kv_rank == 256 || kv_rank == 512) && (kv_rank + rot_dim) % 32 == 0 &&
+         kv_rank + rot_dim <= 640 && (uintptr_t)kv->k % 16 == 0;
+}
+template <typename P, int RH, int LPR>
+static int lat_decode_as(void* out, const float* qa, const UmbPagedKV* kv, const void* sink, const int* pos, const int* slot, int T, int H, int Dk, int window,
+                         float scale, float* scratch, long scratch_floats, hipStream_t st) {
+  constexpr int E = LPR * 8;
+  const long items = (long)T * (H / RH);
+  const int nsplit = decode_splits(LAT_SPAN, items, std::min((long)window, (long)kv->max_pages * kv->page), (long)T * H * (E + 2), scratch, scratch_floats);
+  const int nw = nsplit > 1 ? 4 : items <= 256 && E < 256 ? 16 : (items <= 512 ? 8 : 4);
+  const size_t lds = ((size_t)RH * Dk + (size_t)nw * RH * E + (size_t)(nw + 1) * RH * 2) * sizeof(float);
+  const UmbAttnForm form{1, 0, reinterpret_cast<const float*>(sink), 0.f, 0.f, 0, 0};
+#define LAT_GO(NW)                                                                                                                            \
+  do {                                                                                                                                         \
+    if (ensure_dynamic_lds<attn_decode_kernel<P, RH, LPR, NW, 1, true>>(lds) != UMB_OK) return UMB_EHIP;                                       \
+    hipLaunchKernelGGL((attn_decode_kernel<P, RH, LPR, NW, 1, true>), dim3(T, H / RH, nsplit), dim3(NW * 64), lds, st, (u16*)out, H * E, qa, *kv, \
+                       (const float*)nullptr, 0, -1, (const float*)nullptr, 0, pos, slot, H, 1, Dk, window, scale, 1.f, 0.f, form, scratch, nsplit); \
+  } while (0)
+  if constexpr (E < 256) { if (nw == 16) LAT_GO(16); else if (nw == 8) LAT_GO(8); else LAT_GO(4); }
+  else { if (nw == 8) LAT_GO(8); else LAT_GO(4); }
+#undef LAT_GO
+  if (nsplit > 1)
+    hipLaunchKernelGGL((bsa_merge_kernel<P, 1, true>), dim3(T, H), dim3(std::min(E, 512)), 0, st, (u16*)out, H * E, scratch, (const float*)nullptr, 0, -1, H, E, nsplit, 1.f,
+                       form, pos, window);
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
+// -1: not a shape of these
+int lat_decode(void* out, const float* qa, const UmbPagedKV* kv, const void* sink, const int* pos, const int* slot, int T, int H, int kv_rank, int rot_dim,
+               int window, float scale, float* scratch, long scratch_floats, int dtype, hipStream_t st) {
+  if (!lat_decode_ok(kv_rank, rot_dim, dtype, kv)) return -1;
+  const int Dk = kv_rank + rot_dim;
+  const bool two = (long)T * H <= 128;                     // as in attn_decode
+#define LAT_RH(LPR)                                                                                                                     \
+  do {                                                                                                                                   \
+    if (H % 4 == 0 && !two) return lat_decode_as<P, 4, LPR>(out, qa, kv, sink, pos, slot, T, H, Dk, window, scale, scratch, scratch_floats, st); \
+    if (H % 2 == 0) return lat_decode_as<P, 2, LPR>(out, qa, kv, sink, pos, slot, T, H, Dk, window, scale, scratch, scratch_floats, st); \
+    return lat_decode_as<P, 1, LPR>(out, qa, kv, sink, pos, slot, T, H, Dk, window, scale, scratch, scratch_floats, st);                 \
+  } while (0)
+  auto shape = [&](auto p) -> int {
+    using P = decltype(p);
+    if (kv_rank == 64) LAT_RH(8);
+    if (kv_rank == 128) LAT_RH(16);
+    if (kv_rank == 256) LAT_RH(32);
+    LAT_RH(64);
+  };
+  return dtype == UMB_SEQ_BF16 ? shape(BF16{}) : shape(F16{});
+#undef LAT_RH
 }
 
 extern "C" int umb_attn_attend(void* out, int ldo, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col,
@@ -789,7 +885,7 @@ extern "C" int umb_attn_attend(void* out, int ldo, const float* q, const UmbPage
         hipLaunchKernelGGL((bsa_merge_kernel<P, 2>), dim3(T, H), dim3(64), 0, st, (El_*)out, ldo, scratch, proj, ld, gate_col, H, E,
                            nsplit, out_scale, form, pos, 0);
       else
-        hipLaunchKernelGGL((bsa_merge_kernel<P, 1>), dim3(T, H), dim3(64), 0, st, (El_*)out, ldo, scratch, proj, ld, gate_col, H, E,
+        hipLaunchKernelGGL((bsa_merge_kernel<P, 1>), dim3(T, H), dim3((unsigned)std::min(E + 63, 512) & ~63u), 0, st, (El_*)out, ldo, scratch, proj, ld, gate_col, H, E,
                            nsplit, out_scale, form, pos, 0);
     }
   })

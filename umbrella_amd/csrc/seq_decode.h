@@ -1,4 +1,4 @@
-// Attention of single tokens (16-bit storage, key size a multiple of 32, value size 64, 128 or 256): what the decode kernels of
+// Attention of single tokens (16-bit storage, key size a multiple of 32, value size 64, 128 or 256, latents also 512): what the decode kernels of
 // seq_battn.hip and seq_pwattn.hip share.
 //
 // A wave takes ROUNDS of 16 keys.  Scores: lane (key lane % 16, quarter lane / 16) holds every fourth 16-byte piece of its key's row, so
@@ -61,6 +61,11 @@ template <typename P> __device__ __forceinline__ void unpack8(u32x4 v, float* f)
 // partial sums of a wave: acc[N] per lane, N = 8 rows, over the 64 / LPR row groups; written to dst[row][E]
 template <int RH, int LPR> __device__ __forceinline__ void store_groups(float* dst, float (&acc)[RH * 8], int lane) {
   constexpr int E = LPR * 8, N = RH * 8;
+  if constexpr (LPR == 64) {                                 // a row a load: every lane has its columns' sums
+#pragma unroll
+    for (int v = 0; v < N; ++v) dst[(v >> 3) * E + lane * 8 + (v & 7)] = acc[v];
+    return;
+  }
 #pragma unroll
   for (int k = 0; k < N / 2; ++k) {                          // after this register k holds value 2 k + (lane / 32)
     float a = acc[2 * k], b = acc[2 * k + 1];

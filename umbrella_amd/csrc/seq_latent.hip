@@ -760,8 +760,17 @@ extern "C" int umb_lat_front(void* qn, float* qa, const UmbPagedKV* kv, const fl
   return UMB_OK;
 }
 
+// seq_battn.hip
+int lat_decode(void* out, const float* qa, const UmbPagedKV* kv, const void* sink, const int* pos, const int* slot, int T, int H, int kv_rank, int rot_dim,
+               int window, float scale, float* scratch, long scratch_floats, int dtype, hipStream_t st);
+
 extern "C" int umb_lat_attend(void* out, const float* qa, const UmbPagedKV* kv, const void* sink, const int* pos, const int* slot,
                               int T, int H, int kv_rank, int rot_dim, int window, float scale, int dtype, hipStream_t st) {
+  return umb_lat_attend_split(out, qa, kv, sink, pos, slot, T, H, kv_rank, rot_dim, window, scale, nullptr, 0, dtype, st);
+}
+
+extern "C" int umb_lat_attend_split(void* out, const float* qa, const UmbPagedKV* kv, const void* sink, const int* pos, const int* slot, int T, int H,
+                                    int kv_rank, int rot_dim, int window, float scale, float* scratch, long scratch_floats, int dtype, hipStream_t st) {
   if (T < 1 || H < 1 || kv_rank < 1 || kv_rank > 64 * LAT_MAXC || rot_dim < 0 || window < 1 || !out || !qa || !lat_kv_ok(kv) ||
       !pos || !slot)
     return UMB_EINVAL;
@@ -796,6 +805,8 @@ extern "C" int umb_lat_attend(void* out, const float* qa, const UmbPagedKV* kv, 
     UMB_LAUNCH_CHECK();
     return UMB_OK;
   }
+  const int rc = lat_decode(out, qa, kv, sink, pos, slot, T, H, kv_rank, rot_dim, window, scale, scratch, scratch_floats, dtype, st);
+  if (rc != -1) return rc;
   const int Dk = kv_rank + rot_dim, Dp = (Dk + 3) & ~3;
   // heads of one workgroup: all of them share the keys, so as many as the register budget of the partial sums allows
   const int nc = (kv_rank + 63) / 64;

@@ -444,6 +444,10 @@ class SeqMixLM(LLMBase):
         if self._v_width:                               # values that later layers of the step mix in
             b["v_first"] = torch.zeros(T, self._v_width, dtype=f32, device=dev)
             ws.v_first = b["v_first"].data_ptr()
+        ranks = [ly.mixer.kv_rank for ly in c.layers if ly.mixer.kind == "latent_attention"]
+        if ranks and dt != f32:                         # a token's keys over several workgroups (the size does not follow from the step's: neither do sums)
+            b["part"] = torch.zeros(256 * 16 * (max(ranks) + 2), dtype=f32, device=dev)
+            ws.part, ws.part_floats = b["part"].data_ptr(), b["part"].numel()
         if top:
             pairs = T * top
             tiles = (pairs + 15) // 16 + max(ly.experts for ly in c.layers)          # the smallest tile size the forward picks

@@ -600,8 +600,6 @@ typedef struct UmbSeqWork {
   void* h2;            /* parallel blocks: normed input of the feed-forward [Tmax][W] dtype */
   float* y2;           /* parallel blocks: feed-forward output; mixers with two output projections: the second [Tmax][W] fp32 */
   float* v_first;      /* values that later layers of the step mix in [Tmax][kv_heads vdim] fp32 (null when no layer does) */
-  float* part;         /* partial results of split keys of latent layers, 256 * 16 * (kv_rank + 2) floats hold them all (null: none are split) */
-  int64_t part_floats;
 } UmbSeqWork;
 
 typedef struct UmbSeqStep {

@@ -274,7 +274,7 @@ class UmbSeqWork(C.Structure):
                 ("Tmax", C.c_int32), ("Rmax", C.c_int32), ("moe_sel", C.c_void_p), ("moe_wt", C.c_void_p),
                 ("moe_pos", C.c_void_p), ("moe_tiles", C.c_void_p), ("moe_xs", C.c_void_p), ("moe_act", C.c_void_p),
                 ("moe_y", C.c_void_p), ("moe_max_tiles", C.c_int32), ("y_rows", C.c_int32), ("aux_floats", C.c_int64),
-                ("h2", C.c_void_p), ("y2", C.c_void_p), ("v_first", C.c_void_p), ("part", C.c_void_p), ("part_floats", C.c_int64)]
+                ("h2", C.c_void_p), ("y2", C.c_void_p), ("v_first", C.c_void_p)]
 
 
 class UmbSeqStep(C.Structure):

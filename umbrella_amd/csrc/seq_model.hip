@@ -441,7 +441,8 @@ static int run_mixer(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWo
       SEQ_TRY(umb_lat_attend_tiled(ws->act, ws->aux, &ly.kv, ly.sink, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, s->B,
                                    s->max_len, H, Rc, R, ly.window, ly.scale, dt, st));
     else
-      SEQ_TRY(umb_lat_attend_split(ws->act, ws->aux, &ly.kv, ly.sink, s->pos, s->slot, T, H, Rc, R, ly.window, ly.scale, ws->part, ws->part_floats, dt, st));
+      SEQ_TRY(umb_lat_attend_split(ws->act, ws->aux, &ly.kv, ly.sink, s->pos, s->slot, T, H, Rc, R, ly.window, ly.scale, ws->aux + (long)T * H * Dk,
+                                   ws->aux_floats - (long)T * H * Dk, dt, st));
     SEQ_TRY(umb_seq_linear_batched(ws->mix, ws->act, ly.uv, T, Dv, Rc, H * Rc, H * Dv, H, Rc, (long)Dv * Rc, Dv, ly.gate_head ? 7 : 3,
                                    ws->proj + gate_col, ld, ly.gate_head ? 1 : Dv, dt, st));
   } else if (ly.kind == UMB_MIX_MINGRU) {

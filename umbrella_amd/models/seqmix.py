@@ -372,9 +372,10 @@ class SeqMixLM(LLMBase):
             ask(proj=t["proj_w"].shape[0])
             if m.kind == "latent_attention":
                 # act: query latent, then the attended latents; o: queries; mix: unrotated queries, then the gated heads;
-                # aux: queries carried into the latent space
+                # aux: queries carried into the latent space, and room for the partial results of split keys (of 256 rows at most, all of them
+                # whatever T is: how a token's keys are split does not follow from the workspace)
                 ask(act=max(m.q_rank, m.heads * m.kv_rank), o=m.heads * (m.dim + m.rot_dim) if m.q_rank else 1, mix=m.heads * max(m.dim, m.vdim),
-                    aux=m.heads * (m.kv_rank + m.rot_dim))
+                    aux=m.heads * (m.kv_rank + m.rot_dim) + 256 * 16 * (m.kv_rank + 2) // T + 1)
             elif m.kind == "mingru":
                 ask(mix=m.dim, aux=3 * m.dim + m.dim // 16 + 1)     # aux: piece summaries and start states of long stretches
             elif m.kind == "attention_ssd":
@@ -444,10 +445,6 @@ class SeqMixLM(LLMBase):
         if self._v_width:                               # values that later layers of the step mix in
             b["v_first"] = torch.zeros(T, self._v_width, dtype=f32, device=dev)
             ws.v_first = b["v_first"].data_ptr()
-        ranks = [ly.mixer.kv_rank for ly in c.layers if ly.mixer.kind == "latent_attention"]
-        if ranks and dt != f32:                         # a token's keys over several workgroups (the size does not follow from the step's: neither do sums)
-            b["part"] = torch.zeros(256 * 16 * (max(ranks) + 2), dtype=f32, device=dev)
-            ws.part, ws.part_floats = b["part"].data_ptr(), b["part"].numel()
         if top:
             pairs = T * top
             tiles = (pairs + 15) // 16 + max(ly.experts for ly in c.layers)          # the smallest tile size the forward picks

@@ -192,6 +192,10 @@ int umb_pwa_prep(float* q, const UmbPagedKV* kv, const float* proj, int ld, cons
 /* pooled entries of every block whose last position this step wrote: the fp32 mean of the `pool` cached keys / values */
 int umb_pwa_pool(const UmbPagedKV* kv, const int* seq_slot, const int* seq_pos0, const int* seq_len, int B, int max_len, int G,
                  int D, int pool, int dtype, umb_stream_t stream);
+/* both for one token a sequence (token t is sequence t's only one): the blocks that the tokens complete in the launch that prepares them */
+int umb_pwa_prep_step(float* q, const UmbPagedKV* kv, const float* proj, int ld, const int* pos, const int* slot, const float* freq,
+                      const int* seq_slot, const int* seq_pos0, const int* seq_len, int T, int H, int G, int D, int rot_dims, int pool,
+                      float eps, int dtype, umb_stream_t stream);
 /* out[t][h] = sigmoid(gate[t][h]) * sum over visible keys of sigmoid(q.k * scale + pos_bias[h]) * v, in `dtype`.
  * Visible to position i: tokens j with 0 <= i - j < window, and blocks b with b pool + pool - 1 <= i - window. */
 int umb_pwa_attend(void* out, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const void* pos_bias,

@@ -23,26 +23,60 @@
 #include "seq_common.h"
 #include "seq_decode.h"
 
+// feature d (of D) of the sums of a pooled block's first cnt positions, keys and values, in order.  Lane j of a wave looks up position j's row, the rows go
+// round as scalars and sixteen positions are in flight together.  Called by whole waves.
+template <typename P>
+__device__ __forceinline__ void pool_sums(const UmbPagedKV& kv, int slot, int first, int cnt, int g, int G, int D, int d, float& sk, float& sv) {
+  typedef typename El<P>::type E;
+  constexpr int KB = 16;
+  const int lane = threadIdx.x & 63;
+  for (int c = 0; c < cnt; c += 64) {
+    const int some = cnt - c < 64 ? cnt - c : 64;
+    const long off = pkv_tok(kv, slot, first + c + (lane < some ? lane : some - 1), g, G, D);
+    for (int j0 = 0; j0 < some; j0 += KB) {
+      E kk[KB], vv[KB];
+#pragma unroll
+      for (int u = 0; u < KB; ++u) {
+        const int src = j0 + u < some ? j0 + u : some - 1;
+        const unsigned lo = __builtin_amdgcn_readlane((unsigned)off, src), hi = __builtin_amdgcn_readlane((unsigned)(off >> 32), src);
+        const long o = (long)(((unsigned long long)hi << 32) | lo) + d;
+        kk[u] = reinterpret_cast<const E*>(kv.k)[o];
+        vv[u] = reinterpret_cast<const E*>(kv.v)[o];
+      }
+#pragma unroll
+      for (int u = 0; u < KB; ++u)
+        if (j0 + u < some) {
+          sk += ldf<P>(&kk[u]);
+          sv += ldf<P>(&vv[u]);
+        }
+    }
+  }
+}
+
 // ---- rotary + unit RMS + cache append.  One wave per (token, head slot); head slots 0..H-1 are queries, H..H+G-1 keys.
+// pool > 0 (one token a sequence): slots H+G..H+2G-1 are the pooled blocks that the token completes, if it does: the sums of the cached positions in front of
+// it and its own key and value, worked out once more, as they are stored.  us, in a launch of their own (pwa_pool_kernel, below) / here: 16 requests 4.7 + 4.6 -> 7.0,
+// whether one completes a block or not; one request 4.1 + 1.8 -> 4.2.  Their loads in front of the rest: 7.4.
 template <typename P>
 __global__ __launch_bounds__(256) void pwa_prep_kernel(float* __restrict__ q, UmbPagedKV kv, const float* __restrict__ proj, int ld,
                                                        const int* __restrict__ pos, const int* __restrict__ slot,
                                                        const float* __restrict__ freq, int T, int H, int G, int D, int rot_dims,
-                                                       float eps) {
+                                                       float eps, int pool) {
   typedef typename El<P>::type E;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, per = H + G + (pool > 0 ? G : 0);
   const long id = (long)blockIdx.x * 4 + wave;
-  if (id >= (long)T * (H + G)) return;
-  const int t = (int)(id / (H + G)), hs = (int)(id % (H + G));
-  const bool is_q = hs < H;
-  const float* src = proj + (long)t * ld + (is_q ? (long)hs * D : (long)H * D + (long)(hs - H) * D);
-  const int p = pos[t];
+  if (id >= (long)T * per) return;
+  const int t = __builtin_amdgcn_readfirstlane((int)(id / per)), hs = __builtin_amdgcn_readfirstlane((int)(id % per));
+  const bool is_q = hs < H, is_pool = hs >= H + G;
+  const int g = is_q ? 0 : is_pool ? hs - H - G : hs - H, p = pos[t];
+  if (is_pool && (p + 1) % pool) return;
+  const float* src = proj + (long)t * ld + (is_q ? (long)hs * D : (long)(H + g) * D);
   const float pf = (float)p;
   float* qd = is_q ? q + (long)t * H * D + (long)hs * D : nullptr;
   E* kd = nullptr;
   E* vd = nullptr;
-  if (!is_q) {
-    const long off = pkv_tok(kv, slot[t], p, hs - H, G, D);
+  if (!is_q && !is_pool) {
+    const long off = pkv_tok(kv, slot[t], p, g, G, D);
     kd = reinterpret_cast<E*>(kv.k) + off;
     vd = reinterpret_cast<E*>(kv.v) + off;
   }
@@ -52,7 +86,7 @@ __global__ __launch_bounds__(256) void pwa_prep_kernel(float* __restrict__ q, Um
   for (int m = lane; m < pairs; m += 64) {
     const int d0 = 2 * m, d1 = 2 * m + 1;
     float u = src[d0], v = d1 < D ? src[d1] : 0.f;
-    if (!is_q) { stf<P>(vd + d0, u); if (d1 < D) stf<P>(vd + d1, v); }
+    if (vd) { stf<P>(vd + d0, u); if (d1 < D) stf<P>(vd + d1, v); }
     if (d1 < rot_dims) {
       float sn, cs;
       sincosf(pf * freq[m], &sn, &cs);
@@ -63,6 +97,33 @@ __global__ __launch_bounds__(256) void pwa_prep_kernel(float* __restrict__ q, Um
   }
   ss = wave_sum(ss);
   const float f = 1.f / sqrtf(ss / (float)D + eps);
+  if (is_pool) {
+    const int blk = p / pool, sl = slot[t];
+    const long dst = pkv_blk(kv, sl, blk, pool, g, G, D);
+    const float inv = 1.f / (float)pool;
+    for (int d0 = 0; d0 < D; d0 += 64) {                 // a feature a lane, and its partner's turn
+      const int d = min(d0 + lane, D - 1), m = d >> 1, other = min(d ^ 1, D - 1);
+      float sk = 0.f, sv = 0.f;
+      pool_sums<P>(kv, sl, blk * pool, pool - 1, g, G, D, d, sk, sv);
+      const float raw = src[d];
+      float x = raw;
+      if (2 * m + 1 < rot_dims) {
+        float sn, cs;
+        sincosf(pf * freq[m], &sn, &cs);
+        x = d & 1 ? raw * cs + src[other] * sn : raw * cs - src[other] * sn;
+      }
+      E ks, vs;
+      stf<P>(&ks, x * f);
+      stf<P>(&vs, raw);
+      sk += ldf<P>(&ks);
+      sv += ldf<P>(&vs);
+      if (d0 + lane < D) {
+        kv.kp[dst + d] = sk * inv;
+        kv.vp[dst + d] = sv * inv;
+      }
+    }
+    return;
+  }
   for (int m = lane; m < pairs; m += 64) {
     const int d0 = 2 * m, d1 = 2 * m + 1;
     float u = src[d0], v = d1 < D ? src[d1] : 0.f;
@@ -126,14 +187,12 @@ __global__ __launch_bounds__(256) void pwa_prep_four_kernel(float* __restrict__ 
 }
 
 // ---- pooled blocks completed by this step: grid (block-in-step, sequence, kv head), a thread per feature.
-// Latency: a handful of workgroups, each a chain of page lookups and loads.  Lane j of a wave looks up position j's row, the rows go round
-// as scalars and sixteen positions are in flight together (one at a time, each behind its own lookup, 16 positions took 19.3 us, now 4.4).
+// Latency: a handful of workgroups, each a chain of page lookups and loads (pool_sums; one position at a time, each behind its own lookup, 16 positions
+// took 19.3 us, now 4.4).
 template <typename P>
 __global__ __launch_bounds__(256) void pwa_pool_kernel(UmbPagedKV kv, const int* __restrict__ seq_slot,
                                                        const int* __restrict__ seq_pos0, const int* __restrict__ seq_len, int G,
                                                        int D, int pool) {
-  typedef typename El<P>::type E;
-  constexpr int KB = 16;
   const int b = blockIdx.y, g = blockIdx.z, lane = threadIdx.x & 63;
   const int p0 = seq_pos0[b], n = seq_len[b];
   if (n <= 0) return;
@@ -148,27 +207,7 @@ __global__ __launch_bounds__(256) void pwa_pool_kernel(UmbPagedKV kv, const int*
   for (int d0 = threadIdx.x - lane; d0 < D; d0 += blockDim.x) {           // uniform in a wave
     const int d = d0 + lane < D ? d0 + lane : D - 1;
     float sk = 0.f, sv = 0.f;
-    for (int c = 0; c < pool; c += 64) {
-      const int cnt = pool - c < 64 ? pool - c : 64;
-      const long off = pkv_tok(kv, slot, blk * pool + c + (lane < cnt ? lane : cnt - 1), g, G, D);
-      for (int j0 = 0; j0 < cnt; j0 += KB) {
-        E kk[KB], vv[KB];
-#pragma unroll
-        for (int u = 0; u < KB; ++u) {
-          const int src = j0 + u < cnt ? j0 + u : cnt - 1;
-          const unsigned lo = __builtin_amdgcn_readlane((unsigned)off, src), hi = __builtin_amdgcn_readlane((unsigned)(off >> 32), src);
-          const long o = (long)(((unsigned long long)hi << 32) | lo) + d;
-          kk[u] = reinterpret_cast<const E*>(kv.k)[o];
-          vv[u] = reinterpret_cast<const E*>(kv.v)[o];
-        }
-#pragma unroll
-        for (int u = 0; u < KB; ++u)
-          if (j0 + u < cnt) {
-            sk += ldf<P>(&kk[u]);
-            sv += ldf<P>(&vv[u]);
-          }
-      }
-    }
+    pool_sums<P>(kv, slot, blk * pool, pool, g, G, D, d, sk, sv);
     if (d0 + lane < D) {
       kv.kp[dst + d] = sk * inv;
       kv.vp[dst + d] = sv * inv;
@@ -715,13 +754,13 @@ static inline bool pkv_ok(const UmbPagedKV* kv) {
   return kv && kv->k && kv->v && kv->kp && kv->vp && kv->pages && kv->page >= 1 && kv->max_pages >= 1;
 }
 
-extern "C" int umb_pwa_prep(float* q, const UmbPagedKV* kv, const float* proj, int ld, const int* pos, const int* slot,
-                            const float* freq, int T, int H, int G, int D, int rot_dims, float eps, int dtype, hipStream_t st) {
+static inline bool prep_in_fours(long n, int D) { return n >= 16384 && D <= 128 && D % 2 == 0; }      // from two rounds of waves over the chip on
+static int pwa_prep(float* q, const UmbPagedKV* kv, const float* proj, int ld, const int* pos, const int* slot, const float* freq, int T, int H, int G, int D,
+                    int rot_dims, float eps, int pool, int dtype, hipStream_t st) {
   if (T < 1 || H < 1 || G < 1 || D < 1 || rot_dims < 0 || rot_dims > D || (rot_dims & 1) || !q || !pkv_ok(kv) || !proj || !pos ||
       !slot || (rot_dims && !freq))
     return UMB_EINVAL;
-  const long n = (long)T * (H + G);
-  if (n >= 16384 && D <= 128 && D % 2 == 0) {      // from two rounds of waves over the chip on
+  if (prep_in_fours((long)T * (H + G), D)) {
     const int groups = (H + G + 3) / 4;
     DISPATCH_SEQ_DTYPE(dtype, {
       hipLaunchKernelGGL(pwa_prep_four_kernel<P>, dim3((unsigned)(((long)T * groups + 3) / 4)), dim3(256), 0, st, q, *kv, proj, ld, pos, slot,
@@ -730,14 +769,25 @@ extern "C" int umb_pwa_prep(float* q, const UmbPagedKV* kv, const float* proj, i
     UMB_LAUNCH_CHECK();
     return UMB_OK;
   }
+  const long n = (long)T * (H + G + (pool > 0 ? G : 0));
   DISPATCH_SEQ_DTYPE(dtype, {
     hipLaunchKernelGGL(pwa_prep_kernel<P>, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, q, *kv, proj, ld, pos, slot, freq, T, H,
-                       G, D, rot_dims, eps);
+                       G, D, rot_dims, eps, pool);
   })
   UMB_LAUNCH_CHECK();
   return UMB_OK;
 }
-
+extern "C" int umb_pwa_prep(float* q, const UmbPagedKV* kv, const float* proj, int ld, const int* pos, const int* slot,
+                            const float* freq, int T, int H, int G, int D, int rot_dims, float eps, int dtype, hipStream_t st) {
+  return pwa_prep(q, kv, proj, ld, pos, slot, freq, T, H, G, D, rot_dims, eps, 0, dtype, st);
+}
+extern "C" int umb_pwa_prep_step(float* q, const UmbPagedKV* kv, const float* proj, int ld, const int* pos, const int* slot, const float* freq,
+                                 const int* seq_slot, const int* seq_pos0, const int* seq_len, int T, int H, int G, int D, int rot_dims, int pool,
+                                 float eps, int dtype, hipStream_t st) {
+  if (pool < 1 || !seq_slot || !seq_pos0 || !seq_len || !kv || !kv->kp || !kv->vp) return UMB_EINVAL;
+  const int rc = pwa_prep(q, kv, proj, ld, pos, slot, freq, T, H, G, D, rot_dims, eps, pool, dtype, st);
+  return rc == UMB_OK && prep_in_fours((long)T * (H + G), D) ? umb_pwa_pool(kv, seq_slot, seq_pos0, seq_len, T, 1, G, D, pool, dtype, st) : rc;
+}
 extern "C" int umb_pwa_pool(const UmbPagedKV* kv, const int* seq_slot, const int* seq_pos0, const int* seq_len, int B, int max_len,
                             int G, int D, int pool, int dtype, hipStream_t st) {
   if (B < 1 || max_len < 1 || G < 1 || D < 1 || pool < 1 || !pkv_ok(kv) || !seq_slot || !seq_pos0 || !seq_len) return UMB_EINVAL;

@@ -610,7 +610,7 @@ typedef struct UmbSeqStep {
   int32_t T, B, R, max_len;
   const int32_t *tokens, *pos, *slot;                       /* [T] */
   const int32_t *seq_slot, *seq_row0, *seq_pos0, *seq_len;  /* [B] */
-  const int32_t* logit_rows;                                /* [R] rows whose logits are wanted */
+  const int32_t* logit_rows;                                /* [R] rows whose logits are wanted (null: the first R) */
   float* trace;                                             /* optional [L][T][W]: the residual stream after every layer (the sum of the streams) */
 } UmbSeqStep;
 

@@ -530,6 +530,10 @@ extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const
   const float eps = m->eps;
   const bool hyper = m->streams >= 1;          // several residual streams: norms in front only, stream seams
   const int S = m->streams;
+  // Every row's logits are wanted, in order (single tokens, scored texts): the last seam norms them for the head, which a launch of its own did in 5 us and
+  // more.  (Of several streams the head reads the sum: not a seam's output.)
+  const bool whole = s->R == T && !s->logit_rows && (!hyper || S == 1);
+  auto next_norm = [&](int l) { return l < m->L ? first_norm_of(m, l) : whole ? m->final_norm : nullptr; };
   if (hyper) {
     if (!m->layers[0].norm1) return UMB_EINVAL;
     SEQ_TRY(umb_hc_embed(ws->x, ws->h, m->embed, s->tokens, m->embed_scale, m->layers[0].hc1_in, m->layers[0].norm1,
@@ -548,23 +552,23 @@ extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const
     if (!hyper) SEQ_TRY(sublayer_input(m, ws, s, ly.norm1, ly.canon1, ly.canon_state1, h_ready, st));
     SEQ_TRY(lin(ly.proj, ws->proj, ws->h, T, 0, dt, st));
     SEQ_TRY(run_mixer(m, ly, ws, s, st));
-    SEQ_TRY(lin_y(ly.out, ws->y, ws, ws->mix, T, ly.has_mlp ? slabs(ly.norm2, ly.canon2) : slabs(first_norm_of(m, l + 1), nl ? nl->canon1 : nullptr), dt, st));
+    SEQ_TRY(lin_y(ly.out, ws->y, ws, ws->mix, T, ly.has_mlp ? slabs(ly.norm2, ly.canon2) : slabs(next_norm(l + 1), nl ? nl->canon1 : nullptr), dt, st));
     if (hyper) {
       // write of this sublayer and read of the next one (the feed-forward, the next layer's mixer, or nothing) in one launch
       const float* in2 = ly.has_mlp ? ly.hc2_in : (nl ? nl->hc1_in : nullptr);
-      const void* w2 = ly.has_mlp ? ly.norm2 : (nl ? nl->norm1 : nullptr);
+      const void* w2 = ly.has_mlp ? ly.norm2 : (nl ? nl->norm1 : next_norm(l + 1));
       if ((ly.has_mlp || nl) && !w2) return UMB_EINVAL;
       SEQ_TRY(umb_hc_seam_parts(ws->x, ws->h, ws->y, parts, ly.hc1_mix, ly.hc1_out, m->resid_mult, in2, w2, m->norm_offset, T, W, S, eps, dt, st));
       if (ly.has_mlp) {
         SEQ_TRY(feed_forward(m, ly, ws, s, ws->h, ws->y, &parts, st));
         if (nl && !nl->norm1) return UMB_EINVAL;
         SEQ_TRY(umb_hc_seam_parts(ws->x, ws->h, ws->y, parts, ly.hc2_mix, ly.hc2_out, m->resid_mult, nl ? nl->hc1_in : nullptr,
-                                  nl ? nl->norm1 : nullptr, m->norm_offset, T, W, S, eps, dt, st));
+                                  nl ? nl->norm1 : next_norm(l + 1), m->norm_offset, T, W, S, eps, dt, st));
       }
       if (s->trace) SEQ_TRY(umb_hc_read(s->trace + (long)l * T * W, nullptr, ws->x, nullptr, nullptr, nullptr, 0.f, T, W, S, eps, dt, st));
       continue;
     }
-    const void* next = ly.has_mlp ? ly.norm2 : first_norm_of(m, l + 1);
+    const void* next = ly.has_mlp ? ly.norm2 : next_norm(l + 1);
     if (ly.kind == UMB_MIX_ATTN_DELTA) {
       const void* right = static_cast<char*>(ws->mix) + mix_right(ly, T) * seq_elem_bytes(dt);
       SEQ_TRY(lin_y(ly.out2, ws->y2, ws, right, T, &parts2, dt, st));
@@ -576,8 +580,8 @@ extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const
   ly.has_mlp ? ly.canon_state2 : (nl ? nl->canon_state1 : nullptr), &h_ready, st));
     if (ly.has_mlp) {
       SEQ_TRY(sublayer_input(m, ws, s, ly.norm2, ly.canon2, ly.canon_state2, h_ready, st));
-      SEQ_TRY(feed_forward(m, ly, ws, s, ws->h, ws->y, slabs(first_norm_of(m, l + 1), nl ? nl->canon1 : nullptr), st));
-      SEQ_TRY(seam(m, ws, s, parts, ly.norm2b, first_norm_of(m, l + 1), nl ? nl->canon1 : nullptr, nl ? nl->canon_state1 : nullptr,
+      SEQ_TRY(feed_forward(m, ly, ws, s, ws->h, ws->y, slabs(next_norm(l + 1), nl ? nl->canon1 : nullptr), st));
+      SEQ_TRY(seam(m, ws, s, parts, ly.norm2b, next_norm(l + 1), nl ? nl->canon1 : nullptr, nl ? nl->canon_state1 : nullptr,
                    &h_ready, st));
     }
     if (s->trace) {
@@ -587,7 +591,8 @@ extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const
   }
   if (s->R > 0) {
     // final norm of the wanted rows only (of the sum of the streams, where there are several), then the head
-    if (hyper)
+    if (whole) {
+    } else if (hyper)
       SEQ_TRY(umb_hc_read(nullptr, ws->h, ws->x, s->logit_rows, nullptr, m->final_norm, m->norm_offset, s->R, W, S, eps, dt, st));
     else
       SEQ_TRY(umb_seq_group_norm(nullptr, ws->h, ws->x, s->logit_rows, m->final_norm, s->R, W, groups, eps, dt, st));

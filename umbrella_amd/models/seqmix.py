@@ -508,9 +508,11 @@ class SeqMixLM(LLMBase):
         at[T:2 * T] = np.arange(T) + np.repeat(np.asarray(pos0) - first, n_of)
         at[2 * T:3 * T] = np.repeat(np.asarray(seq_slot), n_of)
         at[3 * T:3 * T + 4 * B] = seq_slot + row0 + pos0 + lens
-        at[3 * T + 4 * B:] = np.asarray(rows, dtype=np.int64) + np.repeat(first, counts)
+        wanted = np.asarray(rows, dtype=np.int64) + np.repeat(first, counts)
+        at[3 * T + 4 * B:] = wanted
+        every = R == T and bool((wanted == np.arange(T)).all())             # every row, in order: the last seam norms them for the head
         graphed = self.use_graph and not trace and T == B and str(dev).startswith("cuda")     # a pure decode step
-        key = (T, R)
+        key = (T, R, every)
         if graphed:
             entry = self._graphs.get(key)
             if entry is None:
@@ -524,6 +526,8 @@ class SeqMixLM(LLMBase):
         s = UmbSeqStep()
         s.T, s.B, s.R, s.max_len = T, B, R, max(lens)
         s.tokens, s.pos, s.slot, s.seq_slot, s.seq_row0, s.seq_pos0, s.seq_len, s.logit_rows = (p + 4 * v for v in o)
+        if every:
+            s.logit_rows = None
         tr = torch.empty(len(self.config.layers), T, self.config.width, dtype=torch.float32, device=dev) if trace else None
         s.trace = tr.data_ptr() if trace else None
         self._keep = meta

@@ -364,6 +364,12 @@ int umb_attn_attend(void* out, int ldo, const float* q, const UmbPagedKV* kv, co
                     const float* bias, int n_dist, const int* pos, const int* slot, int T, int H, int G, int D, int E, int window,
                     float scale, float out_scale, float softcap, const UmbAttnForm* form, float* scratch, long scratch_floats,
                     int dtype, umb_stream_t stream);
+/* both for steps of one token a sequence (q: scratch of T maps H D floats, left as it is where the two are one launch) */
+int umb_attn_step(void* out, int ldo, float* q, const UmbPagedKV* kv, const float* proj, int ld, int append, const void* w_q, const void* w_k,
+                  int norm_qk, int norm_v, const float* freq, int rot_dims, int layout, float rot_mult, float temp_coef, int temp_every,
+                  float eps, const UmbValueMix* mix, int gate_col, const float* bias, int n_dist, const int* pos, const int* slot, int T,
+                  int H, int G, int D, int E, int window, float scale, float out_scale, float softcap, const UmbAttnForm* form,
+                  float* scratch, long scratch_floats, int dtype, umb_stream_t stream);
 int umb_attn_attend_tiled(void* out, int ldo, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col,
                           const float* bias, int n_dist, const int* seq_slot, const int* seq_row0, const int* seq_pos0,
                           const int* seq_len, int B, int max_len, int H, int G, int D, int E, int window, float scale,

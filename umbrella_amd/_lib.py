@@ -346,6 +346,8 @@ SEQ_SIGNATURES = {
     "umb_attn_prep": [_P, _PKV, _P, _I, _I, _P, _P, _I, _I, _P, _P, _P, _I, _I, _F, _I, _I, _I, _I, _I, _I, _F, _I, _F, _I],
     "umb_attn_prep_mix": [_P, _PKV, _P, _I, _I, _P, _P, _I, _I, _P, _P, _P, _I, _I, _F, _I, _I, _I, _I, _I, _I, _F, _I, _F, _P, _I],
     "umb_attn_attend": [_P, _I, _P, _PKV, _P, _I, _I, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _F, _FORM, _P, _L, _I],
+    "umb_attn_step": [_P, _I, _P, _PKV, _P, _I, _I, _P, _P, _I, _I, _P, _I, _I, _F, _F, _I, _F, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _F,
+                      _FORM, _P, _L, _I],
     "umb_attn_attend_tiled": [_P, _I, _P, _PKV, _P, _I, _I, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _F, _FORM, _I],
     "umb_seq_pair_resid_norm": [_P, _P, _P, _P, _P, _P, _F, _P, _P, _I, _I, _F, _I],
     "umb_delta_step": [_P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I],

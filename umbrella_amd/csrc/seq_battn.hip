@@ -45,49 +45,31 @@ struct AttnPrep {
   UmbValueMix mix;                         // first: values to mix in; keep: where this layer's own go (fp32 rows of G E); null: neither
 };
 
-template <typename P>
-__global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, UmbPagedKV kv, const float* __restrict__ proj, int ld,
-                                                        const typename El<P>::type* __restrict__ w_q,
-                                                        const typename El<P>::type* __restrict__ w_k, const int* __restrict__ pos,
-                                                        const int* __restrict__ slot, const float* __restrict__ freq, int T,
-                                                        AttnPrep a) {
-  typedef typename El<P>::type El_;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int per = a.HQ + a.GK + a.GV;
-  const long item = (long)blockIdx.x * 4 + wave;
-  if (item >= (long)T * per) return;
-  const int t = (int)(item / per), hs = (int)(item % per);
-  const bool is_v = hs >= a.HQ + a.GK, is_q = hs < a.HQ;
-  const int n = is_v ? a.E : a.D, D = a.D;
-  const int col = is_v ? (a.HQ + a.GK) * D + (hs - a.HQ - a.GK) * a.E : hs * D;
-  const float* src = proj + (long)t * ld + col;
-  float f = 1.f;
-  if (is_v ? a.norm_v : a.norm_qk) {
-    float ss = 0.f;
-    for (int i = lane; i < n; i += 64) { const float v = src[i]; ss += v * v; }
-    ss = wave_sum(ss);
-    f = 1.f / sqrtf(ss / (float)n + a.eps);
+// a wave's: one row of n values or one row of D queries or keys, put(i, value) for each.  p: the token's position, temp: on queries
+__device__ __forceinline__ float attn_prep_scale(const float* __restrict__ src, int n, int norm, float eps) {
+  float ss = 0.f;
+  const int lane = threadIdx.x & 63;
+  if (!norm) return 1.f;
+  for (int i = lane; i < n; i += 64) { const float v = src[i]; ss += v * v; }
+  ss = wave_sum(ss);
+  return 1.f / sqrtf(ss / (float)n + eps);
+}
+template <typename Put>
+__device__ __forceinline__ void attn_prep_value(const float* __restrict__ src, const AttnPrep& a, long o, bool keep, Put put) {
+  const float f = attn_prep_scale(src, a.E, a.norm_v, a.eps);
+  for (int i = threadIdx.x & 63; i < a.E; i += 64) {
+    float v = src[i] * f;
+    if (keep && a.mix.keep) a.mix.keep[o + i] = v;
+    if (a.mix.first) v = (1.f - a.mix.lambda) * v + a.mix.lambda * a.mix.first[o + i];
+    put(i, v);
   }
-  const int p = pos[t];
-  if (is_v) {
-    const int g = hs - a.HQ - a.GK;
-    El_* row = reinterpret_cast<El_*>(kv.v) + pkv_tok(kv, slot[t], p, g, a.G, a.E);
-    const long o = ((long)t * a.G + g) * a.E;
-    for (int i = lane; i < n; i += 64) {
-      float v = src[i] * f;
-      if (a.mix.keep) a.mix.keep[o + i] = v;
-      if (a.mix.first) v = (1.f - a.mix.lambda) * v + a.mix.lambda * a.mix.first[o + i];
-      stf<P>(row + i, v);
-    }
-    return;
-  }
-  const El_* w = is_q ? w_q : w_k;
-  const float temp = is_q && a.temp_every > 0 ? 1.f + a.temp_coef * logf((float)((p + 1) / a.temp_every + 1)) : 1.f;
-  const int ks = hs - a.HQ;
-  El_* krow = is_q ? nullptr : reinterpret_cast<El_*>(kv.k) + pkv_tok(kv, slot[t], p, ks / a.maps, a.G, a.maps * D) + (ks % a.maps) * D;
-  float* qrow = q + ((long)t * a.HQ + (is_q ? hs : 0)) * D;
+}
+template <typename P, typename Put>
+__device__ __forceinline__ void attn_prep_row(const float* __restrict__ src, const AttnPrep& a, const typename El<P>::type* __restrict__ w,
+                                              const float* __restrict__ freq, int p, float temp, Put put) {
+  const float f = attn_prep_scale(src, a.D, a.norm_qk, a.eps);
   const int half = a.rot_dims >> 1;
-  for (int i = lane; i < n; i += 64) {
+  for (int i = threadIdx.x & 63; i < a.D; i += 64) {
     float v = src[i] * f * (w ? ldf<P>(w + i) : 1.f);
     if (i < a.rot_dims) {
       int fi, other;
@@ -101,9 +83,39 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, U
       cs *= a.rot_mult;
       v = first ? v * cs - u * sn : v * cs + u * sn;
     }
-    if (is_q) qrow[i] = v * temp;
-    else stf<P>(krow + i, v);
+    put(i, v * temp);
   }
+}
+__device__ __forceinline__ float attn_temp(const AttnPrep& a, int p) { return a.temp_every > 0 ? 1.f + a.temp_coef * logf((float)((p + 1) / a.temp_every + 1)) : 1.f; }
+
+template <typename P>
+__global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, UmbPagedKV kv, const float* __restrict__ proj, int ld,
+                                                        const typename El<P>::type* __restrict__ w_q,
+                                                        const typename El<P>::type* __restrict__ w_k, const int* __restrict__ pos,
+                                                        const int* __restrict__ slot, const float* __restrict__ freq, int T,
+                                                        AttnPrep a) {
+  typedef typename El<P>::type El_;
+  const int wave = threadIdx.x >> 6;
+  const int per = a.HQ + a.GK + a.GV;
+  const long item = (long)blockIdx.x * 4 + wave;
+  if (item >= (long)T * per) return;
+  const int t = (int)(item / per), hs = (int)(item % per);
+  const bool is_v = hs >= a.HQ + a.GK, is_q = hs < a.HQ;
+  const int D = a.D, p = pos[t];
+  const float* src = proj + (long)t * ld + (is_v ? (a.HQ + a.GK) * D + (hs - a.HQ - a.GK) * a.E : hs * D);
+  if (is_v) {
+    const int g = hs - a.HQ - a.GK;
+    El_* row = reinterpret_cast<El_*>(kv.v) + pkv_tok(kv, slot[t], p, g, a.G, a.E);
+    attn_prep_value(src, a, ((long)t * a.G + g) * a.E, true, [&](int i, float v) { stf<P>(row + i, v); });
+    return;
+  }
+  const int ks = hs - a.HQ;
+  El_* krow = is_q ? nullptr : reinterpret_cast<El_*>(kv.k) + pkv_tok(kv, slot[t], p, ks / a.maps, a.G, a.maps * D) + (ks % a.maps) * D;
+  float* qrow = q + ((long)t * a.HQ + (is_q ? hs : 0)) * D;
+  attn_prep_row<P>(src, a, is_q ? w_q : w_k, freq, p, is_q ? attn_temp(a, p) : 1.f, [&](int i, float v) {
+    if (is_q) qrow[i] = v;
+    else stf<P>(krow + i, v);
+  });
 }
 
 // The same for many items (rows of at most 128): a wave takes four neighbouring slots of one token, the loads of all four in flight, and
@@ -455,13 +467,17 @@ __global__ __launch_bounds__(NW * 64) void bsa_attend_kernel(typename El<P>::typ
 // 16 behind 100 29.5 -> 14.4, 40 behind 100 82 -> 27.6; 16 heads of 256 + 32: one behind 40 / 2000 19.7 / 26.0 -> 7.2 / 9.4, 40 behind 60 23.0 -> 8.4.
 constexpr int ATT_SPAN = 256, LAT_SPAN = 64;
 
-template <typename P, int RH, int LPR, int NW, int MAPS, bool LAT = false>
+// PREP: steps of one token a sequence.  The queries come from the projection and the token's key and value with them (attn_prep above, which a launch of
+// its own did in 4 - 5 us): the key and value stand in LDS for this workgroup, whose last round takes them from there -- what the cache holds at the token's
+// position is not there yet -- and the group's first workgroup appends them.
+struct DecodePrep { AttnPrep a; const void *w_q, *w_k; const float* freq; };
+template <typename P, int RH, int LPR, int NW, int MAPS, bool LAT = false, bool PREP = false>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q, UmbPagedKV kv,
                                                               const float* __restrict__ proj, int ld, int gate_col,
                                                               const float* __restrict__ bias, int n_dist, const int* __restrict__ pos,
                                                               const int* __restrict__ slot_, int H, int G, int D, int window, float scale,
                                                               float out_scale, float softcap, UmbAttnForm form, float* __restrict__ part,
-                                                              int nsplit) {
+                                                              int nsplit, DecodePrep prep) {
   constexpr int E = LPR * 8, KPI = 64 / LPR, VL = 16 / KPI, RR = RH / MAPS;
   constexpr int SPAN = LAT ? LAT_SPAN : ATT_SPAN;
   static_assert(!LAT || MAPS == 1, "one map");
@@ -469,7 +485,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
   extern __shared__ float lds[];
   const int split = blockIdx.z, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, quarter = lane >> 4;
   float* q_s = lds;                                        // [RH][D]
-  float* o_s = lds + RH * D;                               // [NW][RH][E]
+  u16* new_k = reinterpret_cast<u16*>(lds + RH * D);       // [MAPS][D], the token's own, and its value [E]
+  u16* new_v = new_k + MAPS * D;
+  float* o_s = lds + RH * D + (PREP ? (MAPS * D + E) / 2 : 0);               // [NW][RH][E]
   float* ml_s = o_s + NW * RH * E;                         // [NW][RH][2], [RH][2]
   const int t = blockIdx.x, h0 = blockIdx.y * RR, g = h0 / (H / G);
   const int i = pos[t], slot = slot_[t];
@@ -482,8 +500,35 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
   unsigned row = 0;
   if (wave < nact) row = pkv_tok_row(kv, slot, key_pos(min(base + j, keys.n - 1)), g, G);
   typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
-  for (int x = threadIdx.x; x < RH * D / 4; x += NW * 64)      // (D: a multiple of 32)
-    *reinterpret_cast<f32x4*>(q_s + 4 * x) = *reinterpret_cast<const quad*>(q + ((long)t * H + h0) * MAPS * D + 4 * x);
+  if constexpr (PREP) {
+    const AttnPrep& a = prep.a;
+    const float* src = proj + (long)t * ld;
+    const bool append = split == 0 && h0 % (H / G) == 0;
+    const float temp = attn_temp(a, i);
+    for (int task = wave; task < RH + (a.GK ? MAPS + 1 : 0); task += NW) {       // a row a wave
+      if (task < RH)
+        attn_prep_row<P>(src + (h0 * MAPS + task) * D, a, reinterpret_cast<const u16*>(prep.w_q), prep.freq, i, temp, [&](int x, float v) { q_s[task * D + x] = v; });
+      else if (task < RH + MAPS) {
+        const int mp = task - RH;
+        u16* row_k = reinterpret_cast<u16*>(kv.k) + pkv_tok(kv, slot, i, g, G, MAPS * D) + mp * D;
+        attn_prep_row<P>(src + (a.HQ + g * MAPS + mp) * D, a, reinterpret_cast<const u16*>(prep.w_k), prep.freq, i, 1.f, [&](int x, float v) {
+          const u16 b = P::from_f(v);
+          new_k[mp * D + x] = b;
+          if (append) row_k[x] = b;
+        });
+      } else {
+        u16* row_v = reinterpret_cast<u16*>(kv.v) + pkv_tok(kv, slot, i, g, G, E);
+        attn_prep_value(src + (a.HQ + a.GK) * D + g * E, a, ((long)t * G + g) * E, append, [&](int x, float v) {
+          const u16 b = P::from_f(v);
+          new_v[x] = b;
+          if (append) row_v[x] = b;
+        });
+      }
+    }
+  } else {
+    for (int x = threadIdx.x; x < RH * D / 4; x += NW * 64)      // (D: a multiple of 32)
+      *reinterpret_cast<f32x4*>(q_s + 4 * x) = *reinterpret_cast<const quad*>(q + ((long)t * H + h0) * MAPS * D + 4 * x);
+  }
   __syncthreads();
   if (wave < nact) {
     float acc[RH * 8], m_run[RH], l_run[RH];
@@ -497,6 +542,13 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
       u32x4 vv[VL];
 #pragma unroll
       for (int u = 0; u < VL; ++u) vv[u] = *reinterpret_cast<const u32x4*>(vcol + (long)(unsigned)__shfl((int)row, KPI * u + lane / LPR, 64) * ldv);
+      // the round with the token's own key: it and the lanes behind the last key (whose weights are 0) take what LDS has
+      const bool own = PREP && prep.a.GK && base + 16 >= keys.n;
+      if (own) {
+#pragma unroll
+        for (int u = 0; u < VL; ++u)
+          if (base + KPI * u + lane / LPR >= keys.n - 1) vv[u] = *reinterpret_cast<const u32x4*>(new_v + (lane & (LPR - 1)) * 8);
+      }
       const u16* kr = reinterpret_cast<const u16*>(kv.k) + (long)row * (MAPS * D) + quarter * 8;
       const int dist = i - key_pos(min(kx, keys.n - 1));
       float bv[RR];
@@ -517,6 +569,13 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
         for (int mp = 0; mp < MAPS; ++mp)
 #pragma unroll
           for (int u = 0; u < 4; ++u) kk[mp][u] = *reinterpret_cast<const u32x4*>(kr + mp * D + (d + 32 * u < D ? d + 32 * u : 0));
+        if (own) {
+#pragma unroll
+          for (int mp = 0; mp < MAPS; ++mp)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              if (kx >= keys.n - 1) kk[mp][u] = *reinterpret_cast<const u32x4*>(new_k + mp * D + (d + 32 * u < D ? d + 32 * u : 0) + quarter * 8);
+        }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           if (d + 32 * u >= D) break;
@@ -646,16 +705,23 @@ __global__ __launch_bounds__(MAPS == 1 ? 512 : 64) void bsa_merge_kernel(typenam
 static inline bool form_ok(const UmbAttnForm* f) { return !f || ((f->maps == 1 || f->maps == 2) && f->chunk >= 0 && f->keep_first >= 0); }
 static inline int form_gate_cols(const UmbAttnForm& f, int H, int E) { return f.gate_elem ? H * E : H; }
 
+static inline bool prep_ok(const UmbPagedKV* kv, const float* proj, int ld, int append, const int* pos, const int* slot, const float* freq, int rot_dims,
+                           int layout, int T, int H, int G, int D, int E, int maps) {
+  return !(T < 1 || H < 1 || G < 1 || H % G || D < 1 || E < 1 || maps < 1 || maps > 2 || rot_dims < 0 || rot_dims > D || (rot_dims & 1) ||
+           (rot_dims && !freq) || layout < 0 || layout > 1 || (append && !bsa_kv_ok(kv)) || !proj || !pos || !slot ||
+           ld < maps * H * D + (append ? maps * G * D + G * E : 0));
+}
+static inline AttnPrep prep_of(int append, int norm_qk, int norm_v, int rot_dims, int layout, float rot_mult, int H, int G, int D, int E, int maps,
+                               float temp_coef, int temp_every, float eps, const UmbValueMix* mix) {
+  return AttnPrep{maps * H, append ? maps * G : 0, G, append ? G : 0, D, E, maps, norm_qk, norm_v, rot_dims, layout, rot_mult,
+                  temp_coef, temp_every, eps, mix ? *mix : UmbValueMix{nullptr, nullptr, 0.f, 0.f}};
+}
 extern "C" int umb_attn_prep_mix(float* q, const UmbPagedKV* kv, const float* proj, int ld, int append, const void* w_q, const void* w_k,
                                  int norm_qk, int norm_v, const int* pos, const int* slot, const float* freq, int rot_dims, int layout,
                                  float rot_mult, int T, int H, int G, int D, int E, int maps, float temp_coef, int temp_every, float eps,
                                  const UmbValueMix* mix, int dtype, hipStream_t st) {
-  if (T < 1 || H < 1 || G < 1 || H % G || D < 1 || E < 1 || maps < 1 || maps > 2 || rot_dims < 0 || rot_dims > D || (rot_dims & 1) ||
-      (rot_dims && !freq) || layout < 0 || layout > 1 || !q || (append && !bsa_kv_ok(kv)) || !proj || !pos || !slot ||
-      ld < maps * H * D + (append ? maps * G * D + G * E : 0))
-    return UMB_EINVAL;
-  AttnPrep a{maps * H, append ? maps * G : 0, G, append ? G : 0, D, E, maps, norm_qk, norm_v, rot_dims, layout, rot_mult,
-             temp_coef, temp_every, eps, mix ? *mix : UmbValueMix{nullptr, nullptr, 0.f, 0.f}};
+  if (!q || !prep_ok(kv, proj, ld, append, pos, slot, freq, rot_dims, layout, T, H, G, D, E, maps)) return UMB_EINVAL;
+  const AttnPrep a = prep_of(append, norm_qk, norm_v, rot_dims, layout, rot_mult, H, G, D, E, maps, temp_coef, temp_every, eps, mix);
   const UmbPagedKV none{};
   const long items = (long)T * (a.HQ + a.GK + a.GV);
   // from three rounds of waves over the chip on (us, a wave each / four: 17600 items of two maps 9.2 / 10.5, 19200 of 64 10.2 / 9.9, 30800 of two maps
@@ -722,7 +788,8 @@ static inline int decode_splits(int span, long items, long most, long floats, co
 template <typename P>
 static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const float* bias,
                        int n_dist, const int* pos, const int* slot, int T, int H, int G, int D, int E, int window, float scale,
-                       float out_scale, float softcap, const UmbAttnForm& form, float* scratch, long scratch_floats, hipStream_t st) {
+                       float out_scale, float softcap, const UmbAttnForm& form, float* scratch, long scratch_floats, hipStream_t st,
+                       const DecodePrep* prep = nullptr) {
   const int maps = form.maps, hpg = H / G;
   int rh = (long)T * H * maps <= 128 ? 2 : 4;
   while (rh > maps && hpg % (rh / maps)) rh >>= 1;
@@ -734,13 +801,14 @@ static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv,
   const long most = std::min((long)(form.chunk > 0 && form.chunk < window ? form.chunk : window) + form.keep_first, (long)kv->max_pages * kv->page);
   const int nsplit = decode_splits(ATT_SPAN, items, most, (long)T * H * maps * (E + 2), scratch, scratch_floats);
   const int nw = items <= 256 && E < 256 ? 16 : (items <= 512 ? 8 : 4);
-  const size_t lds = ((size_t)rh * D + (size_t)nw * rh * E + (size_t)(nw + 1) * rh * 2) * sizeof(float);
-#define ATT_GO(RH, LPR, NW, MAPS)                                                                                                     \
+  const size_t lds = ((size_t)rh * D + (prep ? (size_t)(maps * D + E) / 2 : 0) + (size_t)nw * rh * E + (size_t)(nw + 1) * rh * 2) * sizeof(float);
+#define ATT_GO_AS(RH, LPR, NW, MAPS, PREP, ARG)                                                                                       \
   do {                                                                                                                               \
-    if (ensure_dynamic_lds<attn_decode_kernel<P, RH, LPR, NW, MAPS>>(lds) != UMB_OK) return UMB_EHIP;                                 \
-    hipLaunchKernelGGL((attn_decode_kernel<P, RH, LPR, NW, MAPS>), dim3(T, hblocks, nsplit), dim3(NW * 64), lds, st, (u16*)out, ldo, q,   \
-                       *kv, proj, ld, gate_col, bias, n_dist, pos, slot, H, G, D, window, scale, out_scale, softcap, form, scratch, nsplit); \
+    if (ensure_dynamic_lds<attn_decode_kernel<P, RH, LPR, NW, MAPS, false, PREP>>(lds) != UMB_OK) return UMB_EHIP;                    \
+    hipLaunchKernelGGL((attn_decode_kernel<P, RH, LPR, NW, MAPS, false, PREP>), dim3(T, hblocks, nsplit), dim3(NW * 64), lds, st, (u16*)out, ldo, q, \
+                       *kv, proj, ld, gate_col, bias, n_dist, pos, slot, H, G, D, window, scale, out_scale, softcap, form, scratch, nsplit, ARG); \
   } while (0)
+#define ATT_GO(RH, LPR, NW, MAPS) do { if (prep) ATT_GO_AS(RH, LPR, NW, MAPS, true, *prep); else ATT_GO_AS(RH, LPR, NW, MAPS, false, DecodePrep{}); } while (0)
 #define ATT_NW(RH, LPR, MAPS) do { if (nw == 16) ATT_GO(RH, (LPR < 32 ? LPR : 16), 16, MAPS); else if (nw == 8) ATT_GO(RH, LPR, 8, MAPS); else ATT_GO(RH, LPR, 4, MAPS); } while (0)
 #define ATT_RH(LPR)                                                                                  \
   do {                                                                                               \
@@ -753,6 +821,7 @@ static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv,
 #undef ATT_RH
 #undef ATT_NW
 #undef ATT_GO
+#undef ATT_GO_AS
   if (nsplit > 1) {
     if (maps == 2)
       hipLaunchKernelGGL((bsa_merge_kernel<P, 2>), dim3(T, H), dim3(64), 0, st, (u16*)out, ldo, scratch, proj, ld, gate_col, H, E, nsplit,
@@ -783,7 +852,7 @@ static int lat_decode_as(void* out, const float* qa, const UmbPagedKV* kv, const
   do {                                                                                                                                         \
     if (ensure_dynamic_lds<attn_decode_kernel<P, RH, LPR, NW, 1, true>>(lds) != UMB_OK) return UMB_EHIP;                                       \
     hipLaunchKernelGGL((attn_decode_kernel<P, RH, LPR, NW, 1, true>), dim3(T, H / RH, nsplit), dim3(NW * 64), lds, st, (u16*)out, H * E, qa, *kv, \
-                       (const float*)nullptr, 0, -1, (const float*)nullptr, 0, pos, slot, H, 1, Dk, window, scale, 1.f, 0.f, form, scratch, nsplit); \
+                       (const float*)nullptr, 0, -1, (const float*)nullptr, 0, pos, slot, H, 1, Dk, window, scale, 1.f, 0.f, form, scratch, nsplit, DecodePrep{}); \
   } while (0)
   if constexpr (E < 256) { if (nw == 16) LAT_GO(16); else if (nw == 8) LAT_GO(8); else LAT_GO(4); }
   else { if (nw == 8) LAT_GO(8); else LAT_GO(4); }
@@ -895,6 +964,29 @@ extern "C" int umb_attn_attend(void* out, int ldo, const float* q, const UmbPage
 #undef SEQ_TRY_
   UMB_LAUNCH_CHECK();
   return UMB_OK;
+}
+
+extern "C" int umb_attn_step(void* out, int ldo, float* q, const UmbPagedKV* kv, const float* proj, int ld, int append, const void* w_q, const void* w_k,
+                             int norm_qk, int norm_v, const float* freq, int rot_dims, int layout, float rot_mult, float temp_coef, int temp_every, float eps,
+                             const UmbValueMix* mix, int gate_col, const float* bias, int n_dist, const int* pos, const int* slot, int T, int H, int G,
+                             int D, int E, int window, float scale, float out_scale, float softcap, const UmbAttnForm* form_, float* scratch,
+                             long scratch_floats, int dtype, hipStream_t st) {
+  const UmbAttnForm form = form_ ? *form_ : UmbAttnForm{1, 0, nullptr, 0.f, 0.f, 0, 0};
+  if (!form_ok(form_) || !bsa_kv_ok(kv) || !out || !prep_ok(kv, proj, ld, append, pos, slot, freq, rot_dims, layout, T, H, G, D, E, form.maps) || window < 1 ||
+      ldo < H * E || (bias && n_dist < 1) || (gate_col >= 0 && ld < gate_col + form_gate_cols(form, H, E)))
+    return UMB_EINVAL;
+  if (decode_rows_ok(D, E, dtype, kv)) {
+    const DecodePrep prep{prep_of(append, norm_qk, norm_v, rot_dims, layout, rot_mult, H, G, D, E, form.maps, temp_coef, temp_every, eps, mix), w_q, w_k, freq};
+    if (dtype == UMB_SEQ_BF16)
+      return attn_decode<BF16>(out, ldo, nullptr, kv, proj, ld, gate_col, bias, n_dist, pos, slot, T, H, G, D, E, window, scale, out_scale, softcap, form,
+                               scratch, scratch_floats, st, &prep);
+    return attn_decode<F16>(out, ldo, nullptr, kv, proj, ld, gate_col, bias, n_dist, pos, slot, T, H, G, D, E, window, scale, out_scale, softcap, form,
+                            scratch, scratch_floats, st, &prep);
+  }
+  const int rc = umb_attn_prep_mix(q, kv, proj, ld, append, w_q, w_k, norm_qk, norm_v, pos, slot, freq, rot_dims, layout, rot_mult, T, H, G, D, E, form.maps,
+                                   temp_coef, temp_every, eps, mix, dtype, st);
+  return rc != UMB_OK ? rc : umb_attn_attend(out, ldo, q, kv, proj, ld, gate_col, bias, n_dist, pos, slot, T, H, G, D, E, window, scale, out_scale, softcap,
+                                             form_, scratch, scratch_floats, dtype, st);
 }
 
 extern "C" int umb_bsa_attend(void* out, int ldo, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col,

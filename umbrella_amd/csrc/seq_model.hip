@@ -309,6 +309,21 @@ static int attend(const UmbSeqLayer& ly, void* out, const float* q, const UmbSeq
                          out_scale, 0.f, &form, scratch_floats > 0 ? scratch : nullptr, scratch_floats, dt, st);
 }
 
+// what the attention mixers ask of the rows in front of their attention
+struct PrepForm { int append; const void *w_q, *w_k; int norm_qk; const float* freq; int rot_dims, layout; float rot_mult; const UmbValueMix* mix; };
+// both: the rows' preparation and the attention, in one launch where every sequence brings one token
+static int prep_and_attend(const UmbSeqLayer& ly, const UmbSeqWork* ws, const UmbSeqStep* s, float* q, const PrepForm& p, int ld, int H, int G, int D, int E,
+                           float out_scale, const UmbAttnForm& form, float* scratch, int gate_col, float eps, int dt, hipStream_t st) {
+  const long scratch_floats = ws->aux_floats - (long)(scratch - ws->aux);
+  if (s->max_len == 1)
+    return umb_attn_step(ws->mix, H * E, q, &ly.kv, ws->proj, ld, p.append, p.w_q, p.w_k, p.norm_qk, 0, p.freq, p.rot_dims, p.layout, p.rot_mult, 0.f, 0, eps,
+                         p.mix, gate_col, ly.dist_bias, ly.n_dist, s->pos, s->slot, s->T, H, G, D, E, ly.window, ly.scale, out_scale, 0.f, &form,
+                         scratch_floats > 0 ? scratch : nullptr, scratch_floats, dt, st);
+  SEQ_TRY(umb_attn_prep_mix(q, &ly.kv, ws->proj, ld, p.append, p.w_q, p.w_k, p.norm_qk, 0, s->pos, s->slot, p.freq, p.rot_dims, p.layout, p.rot_mult, s->T, H, G,
+                            D, E, form.maps, 0.f, 0, eps, p.mix, dt, st));
+  return attend(ly, ws->mix, q, s, H, G, D, E, ly.window, out_scale, form, scratch, scratch_floats, dt, st, ws->proj, ld, gate_col);
+}
+
 // softmax attention by form: one map; norms, rotary, bias by distance, window with kept first tokens or chunks, sink, element-wise
 // gate and value mixing, each where the layer asks for it
 static int mix_softmax(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWork* ws, const UmbSeqStep* s, hipStream_t st) {
@@ -320,11 +335,9 @@ static int mix_softmax(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeq
   float* q = ws->aux;                                        // [T][H D] | scratch
   float* spare = q + al4((long)T * H * D);
   const UmbValueMix mix{ly.v_mix == 2 ? ws->v_first : nullptr, ly.v_mix == 1 ? ws->v_first : nullptr, ly.v_lambda, 0.f};
-  SEQ_TRY(umb_attn_prep_mix(q, &ly.kv, ws->proj, ld, 1, ly.q_norm, ly.k_norm, ly.q_norm != nullptr, 0, s->pos, s->slot, ly.rot_freq, ly.rot_dims,
-                            ly.rot_layout, ly.rot_mult, T, H, G, D, E, 1, 0.f, 0, m->eps, &mix, dt, st));
   const UmbAttnForm form{1, ly.chunk, ly.attn_sink, 0.f, 0.f, ly.keep_first, ly.gate_elem};
-  return attend(ly, ws->mix, q, s, H, G, D, E, ly.window, 1.f, form, spare, ws->aux_floats - (long)(spare - ws->aux), dt, st, ws->proj, ld,
-                ly.gate_elem ? gate_col : -1);
+  return prep_and_attend(ly, ws, s, q, PrepForm{1, ly.q_norm, ly.k_norm, ly.q_norm != nullptr, ly.rot_freq, ly.rot_dims, ly.rot_layout, ly.rot_mult, &mix}, ld, H, G,
+                         D, E, 1.f, form, spare, ly.gate_elem ? gate_col : -1, m->eps, dt, st);
 }
 
 // differential attention: two maps per head over the same values; with kv_shared the keys and values are another layer's
@@ -333,10 +346,9 @@ static int mix_diff_attn(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbS
   if (H < 1 || G < 1 || ld != 2 * H * D + (ly.kv_shared ? 0 : 2 * G * D + G * E) || ly.out.K != H * E) return UMB_EINVAL;
   float* q = ws->aux;                                        // [T][H][2][D] | scratch
   float* spare = q + al4((long)T * 2 * H * D);
-  SEQ_TRY(umb_attn_prep(q, &ly.kv, ws->proj, ld, !ly.kv_shared, nullptr, nullptr, 0, 0, s->pos, s->slot, ly.rot_freq, ly.rot_dims,
-                        ly.rot_layout, ly.rot_mult, T, H, G, D, E, 2, 0.f, 0, m->eps, dt, st));
   const UmbAttnForm form{2, ly.chunk, nullptr, ly.diff_lambda, m->eps, 0, 0};
-  return attend(ly, ws->mix, q, s, H, G, D, E, ly.window, ly.out_mult, form, spare, ws->aux_floats - (long)(spare - ws->aux), dt, st);
+  return prep_and_attend(ly, ws, s, q, PrepForm{!ly.kv_shared, nullptr, nullptr, 0, ly.rot_freq, ly.rot_dims, ly.rot_layout, ly.rot_mult, nullptr}, ld, H, G, D, E,
+                         ly.out_mult, form, spare, -1, m->eps, dt, st);
 }
 
 static inline int up16(int n) { return (n + 15) & ~15; }
@@ -353,10 +365,8 @@ static int mix_attn_delta(const UmbSeqModel* m, const UmbSeqLayer& ly, const Umb
   if (ld != col0 + C + Hv * Es + 2 * Hv || ly.out.K != H * E || ly.out2.K != Hv * Es || !ly.state) return UMB_EINVAL;
   float* q = ws->aux;                                        // [T][H D] | dq | dk | dv | beta | log g | scratch
   float* spare = q + al4((long)T * H * D);
-  SEQ_TRY(umb_attn_prep(q, &ly.kv, ws->proj, ld, 1, ly.q_norm, ly.k_norm, 1, 0, s->pos, s->slot, nullptr, 0, 0, 1.f, T, H, G, D, E, 1, 0.f, 0,
-                        m->eps, dt, st));
   const UmbAttnForm form{1, 0, ly.attn_sink, 0.f, 0.f, 0, 0};
-  SEQ_TRY(attend(ly, ws->mix, q, s, H, G, D, E, ly.window, 1.f, form, spare, ws->aux_floats - (long)(spare - ws->aux), dt, st));
+  SEQ_TRY(prep_and_attend(ly, ws, s, q, PrepForm{1, ly.q_norm, ly.k_norm, 1, nullptr, 0, 0, 1.f, nullptr}, ld, H, G, D, E, 1.f, form, spare, -1, m->eps, dt, st));
   if (s->max_len == 1)
     SEQ_TRY(umb_delta_step(ws->o, ly.state, ws->proj, ld, col0, ly.s_conv, ly.s_conv_state, ly.s_dt_bias, ly.s_a_log, s->pos, s->slot, T, Hk,
                            Hv, Ds, Es, ly.s_taps, dt, st));

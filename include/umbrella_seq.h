@@ -205,6 +205,10 @@ int umb_pwa_attend(void* out, const float* q, const UmbPagedKV* kv, const float*
 /* The same attention for steps that bring whole stretches of a sequence (prompts), on the matrix pipe: 16-bit storage only,
  * D a multiple of 32 (<= 256); workgroups own 16 consecutive positions of one sequence.  Scores and weights keep fp32
  * accuracy: the fp32 factors (q, pooled means, weights) enter as high + low 16-bit halves. */
+/* all of it for steps of one token a sequence (q: scratch of T H D floats, left as it is where it is one launch) */
+int umb_pwa_step(void* out, float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const void* pos_bias, const int* pos,
+                 const int* slot, const float* freq, const int* seq_slot, const int* seq_pos0, const int* seq_len, int T, int H, int G,
+                 int D, int rot_dims, int window, int pool, float scale, float eps, int dtype, umb_stream_t stream);
 int umb_pwa_attend_tiled(void* out, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col,
                          const void* pos_bias, const int* seq_slot, const int* seq_row0, const int* seq_pos0, const int* seq_len,
                          int B, int max_len, int H, int G, int D, int window, int pool, float scale, int dtype,

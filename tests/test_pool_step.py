@@ -38,3 +38,48 @@ def test_completed_blocks(dtype, B, H, G, D, rot, pool, page):
     # last of the fp32 sums behind it (sizes below 16: a step of 2^-20, half of it on either side), and the mean (2^-24 of itself on either side)
     ulp = {torch.bfloat16: 2.0 ** -4, torch.float16: 2.0 ** -7, torch.float32: 2.0 ** -20}[dtype]
     assert float((a["kp"] - b["kp"]).abs().max()) <= (ulp + 2.0 ** -20) / pool + 2.0 ** -23 * float(a["kp"].abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("H,G,D,rot,window,pool,lens", [(32, 8, 64, 64, 512, 16, [2000]), (32, 8, 128, 128, 64, 16, [96 + i for i in range(16)]),
+                                                        (6, 2, 64, 32, 40, 7, [1, 7, 14, 41, 48, 49, 300]), (4, 4, 256, 0, 16, 16, [16, 17, 32, 33, 1024]),
+                                                        (8, 1, 128, 64, 2 ** 30, 3, [3, 50, 600]), (16, 2, 64, 64, 33, 16, [30 + i for i in range(120)]),
+                                                        (6, 2, 24, 16, 40, 7, [42, 49, 5])])
+def test_step_as_three_launches(dtype, H, G, D, rot, window, pool, lens):
+    """the whole of a step in one launch; the cache holds NaN at the tokens' own positions until they are appended"""
+    from umbrella_amd import _lib
+    from umbrella_amd.attn.cache import PagedSeqCache
+    code, T, ld = _lib.seq_dtype_code(dtype), len(lens), (H + G) * D + H
+    g = torch.Generator(device="cuda").manual_seed(H + D + T)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")                                              # noqa: E731
+    proj, freq, bias = rnd(T, ld), torch.rand(max(rot // 2, 1), generator=g, device="cuda"), rnd(H).to(dtype)
+    pos, one = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device="cuda"), torch.ones(T, dtype=torch.int32, device="cuda")
+    fill, outs = None, []
+    for step in (False, True):
+        c = PagedSeqCache([(G, D, pool)], [], sum(lens) + 50, T, "cuda", dtype, page=32)
+        for b, n in enumerate(lens):
+            c.open(b), c.extend(b, n)
+        kv = c.kv[0]
+        fill = fill or {z: rnd(*kv[z].shape).to(kv[z].dtype) for z in ("k", "v", "kp", "vp")}
+        for z in fill:
+            kv[z].copy_(fill[z])
+        for b, n in enumerate(lens):
+            page = c.seqs[b]["pages"][(n - 1) // 32]
+            kv["k"][page, :, (n - 1) % 32], kv["v"][page, :, (n - 1) % 32] = float("nan"), float("nan")
+        slot = torch.tensor([c.slot(b) for b in range(T)], dtype=torch.int32, device="cuda")
+        q, out = torch.zeros(T, H * D, device="cuda"), torch.full((T + 1, H * D), 3.0, dtype=dtype, device="cuda")
+        if step:
+            _lib.seq_call("umb_pwa_step", out, q, c.struct(0), proj, ld, (H + G) * D, bias, pos, slot, freq, slot, pos, one, T, H, G, D, rot, window, pool,
+                          D ** -0.5, 1e-6, code)
+        else:
+            _lib.seq_call("umb_pwa_prep", q, c.struct(0), proj, ld, pos, slot, freq, T, H, G, D, rot, 1e-6, code)
+            _lib.seq_call("umb_pwa_pool", c.struct(0), slot, pos, one, T, 1, G, D, pool, code)
+            _lib.seq_call("umb_pwa_attend", out, q, c.struct(0), proj, ld, (H + G) * D, bias, pos, slot, T, H, G, D, window, pool, D ** -0.5, code)
+        assert bool((out[T] == 3.0).all()) and bool(torch.isfinite(out).all())
+        outs.append((out[:T].float(), kv["k"].float(), kv["v"].float(), kv["kp"].clone(), kv["vp"].clone()))
+    a, b = outs
+    step_of = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -22}[dtype]           # one step of the storage type, of keys below 16
+    assert torch.equal(a[2], b[2]) and torch.equal(a[4], b[4])
+    assert bool(((a[1] - b[1]).abs() <= step_of * a[1].abs()).all()) and bool(((a[3] - b[3]).abs() <= 16 * step_of / pool + 2.0 ** -19).all())
+    # the rotation and the norm may be contracted otherwise, the sums are of up to 600 weights below 1 in the same order
+    assert bool(((a[0] - b[0]).abs() <= 2 * step_of * a[0].abs() + 2.0 ** -18 * min(window, max(lens))).all())

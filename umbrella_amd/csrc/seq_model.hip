@@ -398,13 +398,11 @@ static int run_mixer(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWo
   if (ly.kind == UMB_MIX_POOLED_WINDOW) {
     const int H = ly.heads, G = ly.kv_heads, D = ly.dim;
     if (ly.vdim != D || ld != H * D + G * D + H) return UMB_EINVAL;
-    if (s->max_len == 1) {                     // a token a sequence: the blocks it may complete in the same launch
-      SEQ_TRY(umb_pwa_prep_step(ws->aux, &ly.kv, ws->proj, ld, s->pos, s->slot, ly.rot_freq, s->seq_slot, s->seq_pos0, s->seq_len, T, H, G, D, ly.rot_dims,
-                                ly.pool, eps, dt, st));
-    } else {
-      SEQ_TRY(umb_pwa_prep(ws->aux, &ly.kv, ws->proj, ld, s->pos, s->slot, ly.rot_freq, T, H, G, D, ly.rot_dims, eps, dt, st));
-      SEQ_TRY(umb_pwa_pool(&ly.kv, s->seq_slot, s->seq_pos0, s->seq_len, s->B, s->max_len, G, D, ly.pool, dt, st));
-    }
+    if (s->max_len == 1)                       // a token a sequence: all of it in one launch where the shape allows it
+      return umb_pwa_step(ws->mix, ws->aux, &ly.kv, ws->proj, ld, H * D + G * D, ly.pos_bias, s->pos, s->slot, ly.rot_freq, s->seq_slot, s->seq_pos0, s->seq_len,
+                          T, H, G, D, ly.rot_dims, ly.window, ly.pool, ly.scale, eps, dt, st);
+    SEQ_TRY(umb_pwa_prep(ws->aux, &ly.kv, ws->proj, ld, s->pos, s->slot, ly.rot_freq, T, H, G, D, ly.rot_dims, eps, dt, st));
+    SEQ_TRY(umb_pwa_pool(&ly.kv, s->seq_slot, s->seq_pos0, s->seq_len, s->B, s->max_len, G, D, ly.pool, dt, st));
     // steps that bring stretches of a sequence (prompts) take the matrix-pipe kernel where the shape allows it
     if (dt != UMB_SEQ_F32 && D % 32 == 0 && D <= 256 && s->max_len >= 16)
       SEQ_TRY(umb_pwa_attend_tiled(ws->mix, ws->aux, &ly.kv, ws->proj, ld, H * D + G * D, ly.pos_bias, s->seq_slot, s->seq_row0,

@@ -53,6 +53,86 @@ __device__ __forceinline__ void pool_sums(const UmbPagedKV& kv, int slot, int fi
   }
 }
 
+// one row of D features by a wave, turned and normed: put(d, value) for each, a pair a lane; raw(d, value) as projected
+template <typename Raw, typename Put>
+__device__ __forceinline__ void pwa_row(const float* __restrict__ src, int D, int rot_dims, const float* __restrict__ freq, int p, float eps, Raw raw, Put put) {
+  const float pf = (float)p;
+  const int lane = threadIdx.x & 63, pairs = (D + 1) / 2;
+  auto turned = [&](int m, float& u, float& v) {
+    if (2 * m + 1 < rot_dims) {
+      float sn, cs;
+      sincosf(pf * freq[m], &sn, &cs);
+      const float ru = u * cs - v * sn, rv = v * cs + u * sn;
+      u = ru; v = rv;
+    }
+  };
+  // pass 1: rotate pairs, sum of squares (each lane owns whole pairs: features 2m, 2m+1 for m = lane, lane + 64, ...)
+  float ss = 0.f;
+  for (int m = lane; m < pairs; m += 64) {
+    const int d0 = 2 * m, d1 = 2 * m + 1;
+    float u = src[d0], v = d1 < D ? src[d1] : 0.f;
+    raw(d0, u);
+    if (d1 < D) raw(d1, v);
+    turned(m, u, v);
+    ss += u * u + (d1 < D ? v * v : 0.f);
+  }
+  ss = wave_sum(ss);
+  const float f = 1.f / sqrtf(ss / (float)D + eps);
+  for (int m = lane; m < pairs; m += 64) {
+    const int d0 = 2 * m, d1 = 2 * m + 1;
+    float u = src[d0], v = d1 < D ? src[d1] : 0.f;
+    turned(m, u, v);
+    put(d0, u * f);
+    if (d1 < D) put(d1, v * f);
+  }
+}
+// the pooled block that the token at p completes, by a wave: the sums of the cached positions in front of it and its own key and value as they are stored
+template <typename P>
+__device__ __forceinline__ void pool_with(const UmbPagedKV& kv, int slot, const float* __restrict__ src, int g, int G, int D, int rot_dims,
+                                          const float* __restrict__ freq, int p, float eps, int pool) {
+  typedef typename El<P>::type E;
+  const int lane = threadIdx.x & 63, blk = p / pool;
+  const float pf = (float)p, inv = 1.f / (float)pool;
+  float f = 0.f;
+  {
+    float ss = 0.f;
+    for (int m = lane; m < (D + 1) / 2; m += 64) {
+      const int d0 = 2 * m, d1 = 2 * m + 1;
+      float u = src[d0], v = d1 < D ? src[d1] : 0.f;
+      if (d1 < rot_dims) {
+        float sn, cs;
+        sincosf(pf * freq[m], &sn, &cs);
+        const float ru = u * cs - v * sn, rv = v * cs + u * sn;
+        u = ru; v = rv;
+      }
+      ss += u * u + (d1 < D ? v * v : 0.f);
+    }
+    f = 1.f / sqrtf(wave_sum(ss) / (float)D + eps);
+  }
+  const long dst = pkv_blk(kv, slot, blk, pool, g, G, D);
+  for (int d0 = 0; d0 < D; d0 += 64) {                   // a feature a lane, and its partner's turn
+    const int d = min(d0 + lane, D - 1), m = d >> 1, other = min(d ^ 1, D - 1);
+    float sk = 0.f, sv = 0.f;
+    pool_sums<P>(kv, slot, blk * pool, pool - 1, g, G, D, d, sk, sv);
+    const float raw = src[d];
+    float x = raw;
+    if (2 * m + 1 < rot_dims) {
+      float sn, cs;
+      sincosf(pf * freq[m], &sn, &cs);
+      x = d & 1 ? raw * cs + src[other] * sn : raw * cs - src[other] * sn;
+    }
+    E ks, vs;
+    stf<P>(&ks, x * f);
+    stf<P>(&vs, raw);
+    sk += ldf<P>(&ks);
+    sv += ldf<P>(&vs);
+    if (d0 + lane < D) {
+      kv.kp[dst + d] = sk * inv;
+      kv.vp[dst + d] = sv * inv;
+    }
+  }
+}
+
 // ---- rotary + unit RMS + cache append.  One wave per (token, head slot); head slots 0..H-1 are queries, H..H+G-1 keys.
 // pool > 0 (one token a sequence): slots H+G..H+2G-1 are the pooled blocks that the token completes, if it does: the sums of the cached positions in front of
 // it and its own key and value, worked out once more, as they are stored.  us, in a launch of their own (pwa_pool_kernel, below) / here: 16 requests 4.7 + 4.6 -> 7.0,
@@ -63,79 +143,26 @@ __global__ __launch_bounds__(256) void pwa_prep_kernel(float* __restrict__ q, Um
                                                        const float* __restrict__ freq, int T, int H, int G, int D, int rot_dims,
                                                        float eps, int pool) {
   typedef typename El<P>::type E;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, per = H + G + (pool > 0 ? G : 0);
+  const int wave = threadIdx.x >> 6, per = H + G + (pool > 0 ? G : 0);
   const long id = (long)blockIdx.x * 4 + wave;
   if (id >= (long)T * per) return;
   const int t = __builtin_amdgcn_readfirstlane((int)(id / per)), hs = __builtin_amdgcn_readfirstlane((int)(id % per));
   const bool is_q = hs < H, is_pool = hs >= H + G;
   const int g = is_q ? 0 : is_pool ? hs - H - G : hs - H, p = pos[t];
-  if (is_pool && (p + 1) % pool) return;
   const float* src = proj + (long)t * ld + (is_q ? (long)hs * D : (long)(H + g) * D);
-  const float pf = (float)p;
-  float* qd = is_q ? q + (long)t * H * D + (long)hs * D : nullptr;
-  E* kd = nullptr;
-  E* vd = nullptr;
-  if (!is_q && !is_pool) {
-    const long off = pkv_tok(kv, slot[t], p, g, G, D);
-    kd = reinterpret_cast<E*>(kv.k) + off;
-    vd = reinterpret_cast<E*>(kv.v) + off;
-  }
-  // pass 1: rotate pairs, sum of squares (each lane owns whole pairs: features 2m, 2m+1 for m = lane, lane + 64, ...)
-  float ss = 0.f;
-  const int pairs = (D + 1) / 2;
-  for (int m = lane; m < pairs; m += 64) {
-    const int d0 = 2 * m, d1 = 2 * m + 1;
-    float u = src[d0], v = d1 < D ? src[d1] : 0.f;
-    if (vd) { stf<P>(vd + d0, u); if (d1 < D) stf<P>(vd + d1, v); }
-    if (d1 < rot_dims) {
-      float sn, cs;
-      sincosf(pf * freq[m], &sn, &cs);
-      const float ru = u * cs - v * sn, rv = v * cs + u * sn;
-      u = ru; v = rv;
-    }
-    ss += u * u + (d1 < D ? v * v : 0.f);
-  }
-  ss = wave_sum(ss);
-  const float f = 1.f / sqrtf(ss / (float)D + eps);
   if (is_pool) {
-    const int blk = p / pool, sl = slot[t];
-    const long dst = pkv_blk(kv, sl, blk, pool, g, G, D);
-    const float inv = 1.f / (float)pool;
-    for (int d0 = 0; d0 < D; d0 += 64) {                 // a feature a lane, and its partner's turn
-      const int d = min(d0 + lane, D - 1), m = d >> 1, other = min(d ^ 1, D - 1);
-      float sk = 0.f, sv = 0.f;
-      pool_sums<P>(kv, sl, blk * pool, pool - 1, g, G, D, d, sk, sv);
-      const float raw = src[d];
-      float x = raw;
-      if (2 * m + 1 < rot_dims) {
-        float sn, cs;
-        sincosf(pf * freq[m], &sn, &cs);
-        x = d & 1 ? raw * cs + src[other] * sn : raw * cs - src[other] * sn;
-      }
-      E ks, vs;
-      stf<P>(&ks, x * f);
-      stf<P>(&vs, raw);
-      sk += ldf<P>(&ks);
-      sv += ldf<P>(&vs);
-      if (d0 + lane < D) {
-        kv.kp[dst + d] = sk * inv;
-        kv.vp[dst + d] = sv * inv;
-      }
-    }
+    if ((p + 1) % pool == 0) pool_with<P>(kv, slot[t], src, g, G, D, rot_dims, freq, p, eps, pool);
     return;
   }
-  for (int m = lane; m < pairs; m += 64) {
-    const int d0 = 2 * m, d1 = 2 * m + 1;
-    float u = src[d0], v = d1 < D ? src[d1] : 0.f;
-    if (d1 < rot_dims) {
-      float sn, cs;
-      sincosf(pf * freq[m], &sn, &cs);
-      const float ru = u * cs - v * sn, rv = v * cs + u * sn;
-      u = ru; v = rv;
-    }
-    if (is_q) { qd[d0] = u * f; if (d1 < D) qd[d1] = v * f; }
-    else { stf<P>(kd + d0, u * f); if (d1 < D) stf<P>(kd + d1, v * f); }
+  if (is_q) {
+    float* qd = q + (long)t * H * D + (long)hs * D;
+    pwa_row(src, D, rot_dims, freq, p, eps, [](int, float) {}, [&](int d, float v) { qd[d] = v; });
+    return;
   }
+  const long off = pkv_tok(kv, slot[t], p, g, G, D);
+  E* kd = reinterpret_cast<E*>(kv.k) + off;
+  E* vd = reinterpret_cast<E*>(kv.v) + off;
+  pwa_row(src, D, rot_dims, freq, p, eps, [&](int d, float v) { stf<P>(vd + d, v); }, [&](int d, float v) { stf<P>(kd + d, v); });
 }
 
 // The same for many items (heads of at most 128, an even number): a wave takes four neighbouring head slots of one token, reads them once,
@@ -395,14 +422,18 @@ __global__ __launch_bounds__(NW * 64) void pwa_attend_kernel(typename El<P>::typ
 // tokens, dealt to the workgroup's waves; weights need no maximum, so the waves' sums are simply added.
 // Before -> now, replayed from a graph, D 128: one token behind 40 / 2000 keys 10.7 -> 4.9 / 30.8 -> 18.0 us, 48 tokens behind 40 20.9 -> 5.7,
 // 64 behind 1000 77 -> 45.
-template <typename P, int RH, int LPR, int NW>
+// PREP: steps of one token a sequence, as in seq_battn.hip: the queries come from the projection, the token's key and value stand in LDS for the round that
+// needs them, and the group's first workgroup appends them and the block that they complete.
+struct PwaPrep { const float* freq; int rot_dims; float eps; };
+template <typename P, int RH, int LPR, int NW, bool PREP>
 __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ out, const float* __restrict__ q, UmbPagedKV kv,
                                                              const float* __restrict__ proj, int ld, int gate_col,
                                                              const u16* __restrict__ pos_bias, const int* __restrict__ pos,
                                                              const int* __restrict__ slot_, int H, int G, int Dr, int window, int pool,
-                                                             float scale) {
+                                                             float scale, PwaPrep prep) {
   constexpr int D = LPR * 8, KPI = 64 / LPR, VL = 16 / KPI;      // Dr = D, but not at compile time: or a round's queries are all read ahead
   __shared__ __attribute__((aligned(16))) float q_s[RH * D];
+  __shared__ __attribute__((aligned(16))) u16 new_k[PREP ? D : 8], new_v[PREP ? D : 8];
   extern __shared__ float o_s[];                           // [NW][RH][D]
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, quarter = lane >> 4;
   const int t = blockIdx.x, h0 = blockIdx.y * RH, g = h0 / (H / G);
@@ -417,7 +448,25 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
   };
   unsigned row = 0;
   if (wave < nact) row = row_of(wave);
-  for (int x = threadIdx.x; x < RH * D; x += NW * 64) q_s[x] = q[((long)t * H + h0) * D + x];
+  if constexpr (PREP) {
+    const float* src = proj + (long)t * ld;
+    const bool append = h0 % (H / G) == 0;
+    for (int task = wave; task < RH + 2; task += NW) {     // a row a wave
+      if (task < RH)
+        pwa_row(src + (h0 + task) * D, Dr, prep.rot_dims, prep.freq, i, prep.eps, [](int, float) {}, [&](int d, float v) { q_s[task * D + d] = v; });
+      else if (task == RH) {
+        const long off = pkv_tok(kv, slot, i, g, G, D);
+        u16* kd = reinterpret_cast<u16*>(kv.k) + off;
+        u16* vd = reinterpret_cast<u16*>(kv.v) + off;
+        pwa_row(src + (H + g) * D, Dr, prep.rot_dims, prep.freq, i, prep.eps,
+                [&](int d, float v) { const u16 b = P::from_f(v); new_v[d] = b; if (append) vd[d] = b; },
+                [&](int d, float v) { const u16 b = P::from_f(v); new_k[d] = b; if (append) kd[d] = b; });
+      } else if (append && (i + 1) % pool == 0)
+        pool_with<P>(kv, slot, src + (H + g) * D, g, G, Dr, prep.rot_dims, prep.freq, i, prep.eps, pool);
+    }
+  } else {
+    for (int x = threadIdx.x; x < RH * D; x += NW * 64) q_s[x] = q[((long)t * H + h0) * D + x];
+  }
   float bias[RH];
 #pragma unroll
   for (int r = 0; r < RH; ++r) bias[r] = pos_bias ? P::to_f(pos_bias[h0 + r]) : 0.f;
@@ -502,10 +551,22 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
       u32x4 vv[VL];
 #pragma unroll
       for (int u = 0; u < VL; ++u) vv[u] = *reinterpret_cast<const u32x4*>(vc + (long)(unsigned)__shfl((int)row, KPI * u + lane / LPR, 64) * D);
+      // the round with the token's own key: it and the lanes behind it (whose weights are 0) take what LDS has, the cache does not have it yet
+      const int key0 = (rd - br) * 16;
+      const bool own = PREP && key0 + 16 >= n_tok;
+      if (own) {
+#pragma unroll
+        for (int u = 0; u < VL; ++u)
+          if (key0 + KPI * u + lane / LPR >= n_tok - 1) vv[u] = *reinterpret_cast<const u32x4*>(new_v + (lane & (LPR - 1)) * 8);
+      }
       for (int d = 0; d < Dr; d += 128) {
         u32x4 kk[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) kk[u] = *reinterpret_cast<const u32x4*>(kr + (d + 32 * u < Dr ? d + 32 * u : 0));
+        if (own && key0 + j >= n_tok - 1) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) kk[u] = *reinterpret_cast<const u32x4*>(new_k + (d + 32 * u < Dr ? d + 32 * u : 0) + quarter * 8);
+        }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           if (d + 32 * u >= Dr) break;
@@ -799,38 +860,45 @@ extern "C" int umb_pwa_pool(const UmbPagedKV* kv, const int* seq_slot, const int
   return UMB_OK;
 }
 
+// single tokens (seq_decode.h); prep: prepared here, of one token a sequence
+static int pwa_decode(void* out, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const void* pos_bias, const int* pos,
+                    const int* slot, int T, int H, int G, int D, int window, int pool, float scale, int dtype, const PwaPrep* prep, hipStream_t st) {
+  const int R = H / G;
+  // 16 waves per item as long as every item gets a compute unit of its own, 8 while two share one, 4 beyond (us with 8 / 4 waves, 32 + 8 heads of
+  // 64: 1024 items behind 30 / 200 keys 12.7 / 7.8, 24.9 / 20.1, 768 behind 200 19.1 / 12.9; 512 items of 128 behind 500 25.4 / 30.0)
+  const int rh = R % 4 == 0 && (long)T * H > 128 ? 4 : (R % 2 == 0 ? 2 : 1);       // few rows in all: two a workgroup, as in seq_battn.hip
+  const long items = (long)T * (H / rh);
+  const int nw = items <= 256 ? 16 : (items <= 512 ? 8 : 4);
+  const size_t lds = (size_t)nw * rh * D * sizeof(float);
+#define PWD_GO_AS(RH, LPR, NW, PREP, ARG)                                                                                       \
+  do {                                                                                                                          \
+  if (ensure_dynamic_lds<pwa_decode_kernel<P, RH, LPR, NW, PREP>>(lds) != UMB_OK) return UMB_EHIP;                            \
+  hipLaunchKernelGGL((pwa_decode_kernel<P, RH, LPR, NW, PREP>), dim3(T, H / rh), dim3(NW * 64), lds, st, (u16*)out, q, *kv, proj, ld, \
+                     gate_col, (const u16*)pos_bias, pos, slot, H, G, D, window, pool, scale, ARG);                           \
+  } while (0)
+#define PWD_GO(RH, LPR, NW) do { if (prep) PWD_GO_AS(RH, LPR, NW, true, *prep); else PWD_GO_AS(RH, LPR, NW, false, PwaPrep{}); } while (0)
+#define PWD_NW(RH, LPR) do { if (nw == 16) PWD_GO(RH, LPR, 16); else if (nw == 8) PWD_GO(RH, LPR, 8); else PWD_GO(RH, LPR, 4); } while (0)
+#define PWD_RH(LPR) do { if (rh == 4) PWD_NW(4, LPR); else if (rh == 2) PWD_NW(2, LPR); else PWD_NW(1, LPR); } while (0)
+#define PWD_D() do { if (D == 64) PWD_RH(8); else if (D == 128) PWD_RH(16); else PWD_RH(32); } while (0)
+  if (dtype == UMB_SEQ_BF16) { using P = BF16; PWD_D(); }
+  else { using P = F16; PWD_D(); }
+#undef PWD_D
+#undef PWD_RH
+#undef PWD_NW
+#undef PWD_GO
+#undef PWD_GO_AS
+  UMB_LAUNCH_CHECK();
+  return UMB_OK;
+}
 extern "C" int umb_pwa_attend(void* out, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col,
                               const void* pos_bias, const int* pos, const int* slot, int T, int H, int G, int D, int window,
                               int pool, float scale, int dtype, hipStream_t st) {
   if (T < 1 || H < 1 || G < 1 || H % G || D < 1 || D > 64 * PWA_MAXC || window < 1 || pool < 1 || !out || !q || !pkv_ok(kv) ||
       !proj || !pos || !slot)
     return UMB_EINVAL;
+  if (decode_rows_ok(D, D, dtype, kv))
+    return pwa_decode(out, q, kv, proj, ld, gate_col, pos_bias, pos, slot, T, H, G, D, window, pool, scale, dtype, nullptr, st);
   const int R = H / G;
-  if (decode_rows_ok(D, D, dtype, kv)) {
-    // 16 waves per item as long as every item gets a compute unit of its own, 8 while two share one, 4 beyond (us with 8 / 4 waves, 32 + 8 heads of
-    // 64: 1024 items behind 30 / 200 keys 12.7 / 7.8, 24.9 / 20.1, 768 behind 200 19.1 / 12.9; 512 items of 128 behind 500 25.4 / 30.0)
-    const int rh = R % 4 == 0 ? 4 : (R % 2 == 0 ? 2 : 1);
-    const long items = (long)T * (H / rh);
-    const int nw = items <= 256 ? 16 : (items <= 512 ? 8 : 4);
-    const size_t lds = (size_t)nw * rh * D * sizeof(float);
-#define PWD_GO(RH, LPR, NW)                                                                                                     \
-  do {                                                                                                                          \
-    if (ensure_dynamic_lds<pwa_decode_kernel<P, RH, LPR, NW>>(lds) != UMB_OK) return UMB_EHIP;                                  \
-    hipLaunchKernelGGL((pwa_decode_kernel<P, RH, LPR, NW>), dim3(T, H / rh), dim3(NW * 64), lds, st, (u16*)out, q, *kv, proj, ld,   \
-                       gate_col, (const u16*)pos_bias, pos, slot, H, G, D, window, pool, scale);                                \
-  } while (0)
-#define PWD_NW(RH, LPR) do { if (nw == 16) PWD_GO(RH, LPR, 16); else if (nw == 8) PWD_GO(RH, LPR, 8); else PWD_GO(RH, LPR, 4); } while (0)
-#define PWD_RH(LPR) do { if (rh == 4) PWD_NW(4, LPR); else if (rh == 2) PWD_NW(2, LPR); else PWD_NW(1, LPR); } while (0)
-#define PWD_D() do { if (D == 64) PWD_RH(8); else if (D == 128) PWD_RH(16); else PWD_RH(32); } while (0)
-    if (dtype == UMB_SEQ_BF16) { using P = BF16; PWD_D(); }
-    else { using P = F16; PWD_D(); }
-#undef PWD_D
-#undef PWD_RH
-#undef PWD_NW
-#undef PWD_GO
-    UMB_LAUNCH_CHECK();
-    return UMB_OK;
-  }
   const int rh = R % 8 == 0 ? 8 : (R % 4 == 0 ? 4 : (R % 2 == 0 ? 2 : 1));     // heads of one group per workgroup
   const int Dp = (D + 3) & ~3;
   const dim3 grid(T, H / rh);
@@ -860,6 +928,20 @@ extern "C" int umb_pwa_attend(void* out, const float* q, const UmbPagedKV* kv, c
 #undef PWA_LAUNCH
   UMB_LAUNCH_CHECK();
   return UMB_OK;
+}
+
+extern "C" int umb_pwa_step(void* out, float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const void* pos_bias, const int* pos,
+                            const int* slot, const float* freq, const int* seq_slot, const int* seq_pos0, const int* seq_len, int T, int H, int G, int D,
+                            int rot_dims, int window, int pool, float scale, float eps, int dtype, hipStream_t st) {
+  if (T < 1 || H < 1 || G < 1 || H % G || D < 1 || D > 64 * PWA_MAXC || window < 1 || pool < 1 || rot_dims < 0 || rot_dims > D || (rot_dims & 1) || !out || !q ||
+      !pkv_ok(kv) || !proj || !pos || !slot || (rot_dims && !freq) || !seq_slot || !seq_pos0 || !seq_len)
+    return UMB_EINVAL;
+  if (decode_rows_ok(D, D, dtype, kv)) {
+    const PwaPrep prep{freq, rot_dims, eps};
+    return pwa_decode(out, nullptr, kv, proj, ld, gate_col, pos_bias, pos, slot, T, H, G, D, window, pool, scale, dtype, &prep, st);
+  }
+  const int rc = umb_pwa_prep_step(q, kv, proj, ld, pos, slot, freq, seq_slot, seq_pos0, seq_len, T, H, G, D, rot_dims, pool, eps, dtype, st);
+  return rc != UMB_OK ? rc : umb_pwa_attend(out, q, kv, proj, ld, gate_col, pos_bias, pos, slot, T, H, G, D, window, pool, scale, dtype, st);
 }
 
 extern "C" int umb_pwa_attend_tiled(void* out, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col,

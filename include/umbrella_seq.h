@@ -287,6 +287,8 @@ int umb_lin_scan(float* o, float* state, const float* q, int ldq, const float* k
                  const int* seq_pos0, const int* seq_len, int B, int H, int D, int Dv, float qscale, umb_stream_t stream);
 /* a step of ONE token per sequence (row t at position pos[t] of slot[t]; position 0 starts from S = 0), sums in the order of umb_lin_scan; v and
  * state 16-byte aligned, Dv and ldv multiples of four */
+int umb_gla_step(void* out, float* state, const float* proj, int ld, const void* w_a2, const void* b_a2, const void* w_norm, const int* pos,
+                 const int* slot, int T, int H, int D, int Dv, int rank, float tau, float qscale, float eps, int dtype, umb_stream_t stream);
 int umb_lin_step(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* alpha,
                  int alpha_per_head, int qk_heads, const int* pos, const int* slot, int T, int H, int D, int Dv, float qscale,
                  umb_stream_t stream);

@@ -413,6 +413,9 @@ static int run_mixer(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWo
   } else if (ly.kind == UMB_MIX_GLA) {
     const int H = ly.heads, D = ly.dim, Dv = ly.vdim, HD = H * D;
     if (ld != 2 * HD + 2 * H * Dv + ly.rank || !ly.state) return UMB_EINVAL;
+    if (s->max_len == 1 && D <= 256 && Dv % 4 == 0 && Dv <= 256 && T <= 65535 && (uintptr_t)ly.state % 16 == 0)      // a token a sequence: one launch
+      return umb_gla_step(ws->mix, ly.state, ws->proj, ld, ly.a2.w, ly.a2.bias, ly.head_norm, s->pos, s->slot, T, H, D, Dv, ly.rank, ly.tau, ly.qscale, eps,
+                          dt, st);
     // aux: decays (their logarithms) [T][HD] | scratch of the chunked form
     float* spare = ws->aux + al4((long)T * HD);
     const long spare_floats = ws->aux_floats - (long)(spare - ws->aux), need = umb_gla_scan_chunked_floats(T, s->B, H, D, Dv);
@@ -423,7 +426,7 @@ static int run_mixer(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWo
     if (chunked)
       SEQ_TRY(umb_gla_scan_chunked(ws->o, ly.state, ws->proj, ld, ws->aux, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, T, s->B, s->max_len,
                                    H, D, Dv, ly.qscale, spare, spare_floats, st));
-    else if (s->max_len == 1 && lin_step_ok(ws->proj + 2L * HD, ld, ly.state, Dv))
+    else if (s->max_len == 1 && lin_step_ok(ws->proj + 2L * HD, ld, ly.state, Dv))      // (heads of more columns)
       SEQ_TRY(umb_lin_step(ws->o, ly.state, ws->proj, ld, ws->proj + HD, ld, ws->proj + 2L * HD, ld, ws->aux, 0, H, s->pos, s->slot, T, H, D, Dv,
                            ly.qscale, st));
     else

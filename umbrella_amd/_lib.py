@@ -336,6 +336,7 @@ SEQ_SIGNATURES = {
     "umb_mingru_scan": [_P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _P, _L, _I],
     "umb_gla_step": [_P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _F, _I],
     "umb_lin_step": [_P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _I, _I, _I, _I, _F],
+    "umb_lin_scan_rows": [_P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F],
     "umb_lin_scan": [_P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _F],
     "umb_ssd_prep": [_P, _I, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I],
     "umb_ssd_scan_chunked_floats": [_I, _I, _I, _I, _I],

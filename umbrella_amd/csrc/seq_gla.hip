@@ -37,7 +37,7 @@ constexpr int GLA_MAXR = 16;     // rows per lane: D <= 256
 constexpr int GLA_TC = 16;       // tokens per staged chunk
 constexpr int GLA_COLS = 16;     // value columns per workgroup (4 per wave)
 
-// Workgroup = (sequence, head, 16 value columns), 4 waves of 4 columns.  The token loop is serial, so its inputs must not
+// Workgroup = (sequence, head, 16 NC value columns), a lane NC of them 16 apart.  The token loop is serial, so its inputs must not
 // cost a memory round trip per token: chunks of 16 tokens (alpha, k, q rows of the head and the 16 v columns) are staged
 // through a double-buffered LDS tile -- the global loads of chunk c + 1 are in flight while chunk c is consumed from LDS.
 // V4: D, Dv and the row stride of proj are multiples of 4 -> the staging moves 16-byte pieces (a quarter of the address
@@ -45,7 +45,7 @@ constexpr int GLA_COLS = 16;     // value columns per workgroup (4 per wave)
 // Operand placement is general: q and k rows hold groups of D shared by `hpg` consecutive heads each (1: a group per head),
 // and the decay is per key channel (alpha [T][H D]) or, with aph, one number per head (alpha [T][H]) that fills the staged
 // row -- the state-space layers with a scalar decay per head run on the same kernel.
-template <int NR, bool V4>
+template <int NR, bool V4, int NC>
 __global__ __launch_bounds__(256) void gla_scan_kernel(float* __restrict__ o, float* __restrict__ state,
                                                        const float* __restrict__ qp, int ldq, const float* __restrict__ kp,
                                                        int ldk, const float* __restrict__ vp, int ldv,
@@ -55,23 +55,24 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(float* __restrict__ o, fl
                                                        int D, int Dv, float qscale) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int VW = V4 ? 4 : 1;                        // floats per staged piece
-  constexpr int STG = (3 * NR + 1 + VW - 1) / VW;       // staged pieces per thread: TC (3 D + 16) / 256 <= 3 NR + 1 floats
+  constexpr int WGC = GLA_COLS * NC;                    // the workgroup's columns; a thread's are 16 apart
+  constexpr int STG = (3 * NR + NC + VW - 1) / VW;      // staged pieces per thread: TC (3 D + 16 NC) / 256 <= 3 NR + NC floats
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15;
-  const int cbase = blockIdx.x * GLA_COLS, cl = wave * 4 + (lane >> 4), c = cbase + cl;
+  const int cbase = blockIdx.x * WGC, cl = wave * 4 + (lane >> 4), c = cbase + cl;
   const int h = blockIdx.y, b = blockIdx.z, hq = h / hpg;
   const int n = seq_len[b];
   if (n <= 0) return;
-  const bool c_ok = c < Dv;
   const int slot = seq_slot[b], row0 = seq_row0[b];
-  float* sp = state + (((long)slot * H + h) * D) * Dv + (c_ok ? c : 0);
-  float S[NR];
+  float* sp = state + (((long)slot * H + h) * D) * Dv + c;
+  float S[NR][NC];
   const bool fresh = seq_pos0[b] == 0;
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     const int d = r * NR + i;
-    S[i] = (!fresh && c_ok && d < D) ? sp[(long)d * Dv] : 0.f;
+#pragma unroll
+    for (int x = 0; x < NC; ++x) S[i][x] = (!fresh && c + 16 * x < Dv && d < D) ? sp[(long)d * Dv + 16 * x] : 0.f;
   }
-  const int HD = H * D, rowlen = 3 * D + GLA_COLS, chunk = GLA_TC * rowlen;
+  const int HD = H * D, rowlen = 3 * D + WGC, chunk = GLA_TC * rowlen;
   const int nch = (n + GLA_TC - 1) / GLA_TC;
   typedef typename std::conditional<V4, f32x4, float>::type piece;
   piece stage[STG];
@@ -123,13 +124,15 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(float* __restrict__ o, fl
     const float* buf = lds + (ch & 1) * chunk;
     if (ch + 1 < nch) fetch(ch + 1);
     const int cnt = n - ch * GLA_TC < GLA_TC ? n - ch * GLA_TC : GLA_TC;
-    float pt[GLA_TC];                                   // this lane's share (its rows) of every token's read-out
+    float pt[NC][GLA_TC];                               // this lane's share (its rows) of every token's read-out
 #pragma unroll
     for (int tt = 0; tt < GLA_TC; ++tt) {
-      float acc = 0.f;
+      float acc[NC] = {};
       if (tt < cnt) {
         const float* row = buf + tt * rowlen;
-        const float v = row[3 * D + cl];
+        float v[NC];
+#pragma unroll
+        for (int x = 0; x < NC; ++x) v[x] = row[3 * D + cl + 16 * x];
         float al[NR], kk[NR], qq[NR];
         bool got = false;
         if constexpr (NR % 4 == 0) {
@@ -155,44 +158,51 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(float* __restrict__ o, fl
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
           if (r * NR + i < D) {
-            S[i] = al[i] * S[i] + kk[i] * v;
-            acc += S[i] * qq[i];
+#pragma unroll
+            for (int x = 0; x < NC; ++x) {
+              S[i][x] = al[i] * S[i][x] + kk[i] * v[x];
+              acc[x] += S[i][x] * qq[i];
+            }
           }
         }
       }
-      pt[tt] = acc;
+#pragma unroll
+      for (int x = 0; x < NC; ++x) pt[x][tt] = acc[x];
     }
     // sum over the 16 row lanes, all 16 tokens at once: a transposing butterfly (15 exchanges instead of 64).  At the step with
     // mask m a lane keeps the half of its values whose token bit m equals its own lane bit and hands the other half to its
     // partner; lane r ends up with the whole sum of token r.  Every token's sum has the same tree (pairs by 8, 4, 2, 1).
-    float p8[8], p4[4], p2[2];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const bool up = r & 8;
-      p8[j] = (up ? pt[j + 8] : pt[j]) + __shfl_xor(up ? pt[j] : pt[j + 8], 8, 64);
-    }
+    for (int x = 0; x < NC; ++x) {
+      float p8[8], p4[4], p2[2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bool up = r & 4;
-      p4[j] = (up ? p8[j + 4] : p8[j]) + __shfl_xor(up ? p8[j] : p8[j + 4], 4, 64);
-    }
+      for (int j = 0; j < 8; ++j) {
+        const bool up = r & 8;
+        p8[j] = (up ? pt[x][j + 8] : pt[x][j]) + __shfl_xor(up ? pt[x][j] : pt[x][j + 8], 8, 64);
+      }
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const bool up = r & 2;
-      p2[j] = (up ? p4[j + 2] : p4[j]) + __shfl_xor(up ? p4[j] : p4[j + 2], 2, 64);
+      for (int j = 0; j < 4; ++j) {
+        const bool up = r & 4;
+        p4[j] = (up ? p8[j + 4] : p8[j]) + __shfl_xor(up ? p8[j] : p8[j + 4], 4, 64);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const bool up = r & 2;
+        p2[j] = (up ? p4[j + 2] : p4[j]) + __shfl_xor(up ? p4[j] : p4[j + 2], 2, 64);
+      }
+      const bool up1 = r & 1;
+      const float mine = ((up1 ? p2[1] : p2[0]) + __shfl_xor(up1 ? p2[0] : p2[1], 1, 64)) * qscale;
+      if (r < cnt && c + 16 * x < Dv) o[(long)(row0 + ch * GLA_TC + r) * (H * Dv) + (long)h * Dv + c + 16 * x] = mine;
     }
-    const bool up1 = r & 1;
-    const float mine = ((up1 ? p2[1] : p2[0]) + __shfl_xor(up1 ? p2[0] : p2[1], 1, 64)) * qscale;
-    if (r < cnt && c_ok) o[(long)(row0 + ch * GLA_TC + r) * (H * Dv) + (long)h * Dv + c] = mine;
     if (ch + 1 < nch) stash(lds + ((ch + 1) & 1) * chunk);
     __syncthreads();
   }
-  if (c_ok) {
 #pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int d = r * NR + i;
-      if (d < D) sp[(long)d * Dv] = S[i];
-    }
+  for (int i = 0; i < NR; ++i) {
+    const int d = r * NR + i;
+#pragma unroll
+    for (int x = 0; x < NC; ++x)
+      if (d < D && c + 16 * x < Dv) sp[(long)d * Dv + 16 * x] = S[i][x];
   }
 }
 
@@ -238,37 +248,57 @@ extern "C" int umb_gla_decay_log(float* log_alpha, const float* proj, int ld, in
   return gla_decay_launch<true>(log_alpha, proj, ld, a_col, w_a2, b_a2, T, HD, rank, tau, dtype, st);
 }
 
-extern "C" int umb_lin_scan(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
-                            const float* alpha, int alpha_per_head, int qk_heads, const int* seq_slot, const int* seq_row0,
-                            const int* seq_pos0, const int* seq_len, int B, int H, int D, int Dv, float qscale, hipStream_t st) {
-  if (B < 1 || H < 1 || D < 1 || D > 16 * GLA_MAXR || Dv < 1 || qk_heads < 1 || H % qk_heads || !o || !state || !q || !k || !v ||
-      !alpha || ldq < qk_heads * D || ldk < qk_heads * D || ldv < H * Dv)
+extern "C" int umb_lin_scan_rows(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
+                                 const float* alpha, int alpha_per_head, int qk_heads, const int* seq_slot, const int* seq_row0,
+                                 const int* seq_pos0, const int* seq_len, int T, int B, int max_len, int H, int D, int Dv, float qscale,
+                                 hipStream_t st) {
+  if (T < 1 || B < 1 || max_len < 1 || max_len > T || H < 1 || D < 1 || D > 16 * GLA_MAXR || Dv < 1 || qk_heads < 1 || H % qk_heads || !o || !state ||
+      !q || !k || !v || !alpha || ldq < qk_heads * D || ldk < qk_heads * D || ldv < H * Dv)
     return UMB_EINVAL;
-  const dim3 grid((Dv + GLA_COLS - 1) / GLA_COLS, H, B);
   const int nr = (D + 15) / 16, aph = alpha_per_head ? 1 : 0, hpg = H / qk_heads;
-  const size_t lds = 2 * (size_t)GLA_TC * (3 * D + GLA_COLS) * sizeof(float);
   const bool v4 = D % 4 == 0 && Dv % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 &&
                   ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (aph ? 0 : (uintptr_t)alpha)) % 16 == 0;
-#define GLA_SCAN_LAUNCH(NR, V4)                                                                                           \
+  const int nc = v4 ? lin_scan_cols(T, max_len, H, D, Dv) : 1;
+  const dim3 grid((Dv + GLA_COLS * nc - 1) / (GLA_COLS * nc), H, B);
+#define GLA_SCAN_LAUNCH(NR, V4, NC)                                                                                       \
   do {                                                                                                                    \
-    if (ensure_dynamic_lds<gla_scan_kernel<NR, V4>>(lds) != UMB_OK) return UMB_EHIP;                                      \
-    hipLaunchKernelGGL((gla_scan_kernel<NR, V4>), grid, dim3(256), lds, st, o, state, q, ldq, k, ldk, v, ldv, alpha, aph, \
-                       hpg, seq_slot, seq_row0, seq_pos0, seq_len, H, D, Dv, qscale);                                      \
+    const size_t lds = 2 * (size_t)GLA_TC * (3 * D + GLA_COLS * NC) * sizeof(float);                                      \
+    if (ensure_dynamic_lds<gla_scan_kernel<NR, V4, NC>>(lds) != UMB_OK) return UMB_EHIP;                                  \
+    hipLaunchKernelGGL((gla_scan_kernel<NR, V4, NC>), grid, dim3(256), lds, st, o, state, q, ldq, k, ldk, v, ldv, alpha, aph, \
+                       hpg, seq_slot, seq_row0, seq_pos0, seq_len, H, D, Dv, qscale);                                     \
   } while (0)
 #define GLA_SCAN_CASE(NR)                                                                                                 \
   case NR:                                                                                                                \
-    if (v4) GLA_SCAN_LAUNCH(NR, true); else GLA_SCAN_LAUNCH(NR, false);                                                   \
+    if (v4) GLA_SCAN_LAUNCH(NR, true, 1); else GLA_SCAN_LAUNCH(NR, false, 1);                                             \
     break;
-  switch (nr) {
-    GLA_SCAN_CASE(1) GLA_SCAN_CASE(2) GLA_SCAN_CASE(3) GLA_SCAN_CASE(4) GLA_SCAN_CASE(5) GLA_SCAN_CASE(6) GLA_SCAN_CASE(7)
-    GLA_SCAN_CASE(8) GLA_SCAN_CASE(9) GLA_SCAN_CASE(10) GLA_SCAN_CASE(11) GLA_SCAN_CASE(12) GLA_SCAN_CASE(13)
-    GLA_SCAN_CASE(14) GLA_SCAN_CASE(15) GLA_SCAN_CASE(16)
-    default: return UMB_EINVAL;
+#define GLA_SCAN_WIDE(NR)                                                                                                 \
+  case NR:                                                                                                                \
+    if (nc == 4) GLA_SCAN_LAUNCH(NR, true, 4); else GLA_SCAN_LAUNCH(NR, true, 2);                                         \
+    break;
+  if (nc > 1) {
+    switch (nr) {
+      GLA_SCAN_WIDE(4) GLA_SCAN_WIDE(8) GLA_SCAN_WIDE(12) GLA_SCAN_WIDE(16)
+    }
+  } else {
+    switch (nr) {
+      GLA_SCAN_CASE(1) GLA_SCAN_CASE(2) GLA_SCAN_CASE(3) GLA_SCAN_CASE(4) GLA_SCAN_CASE(5) GLA_SCAN_CASE(6) GLA_SCAN_CASE(7)
+      GLA_SCAN_CASE(8) GLA_SCAN_CASE(9) GLA_SCAN_CASE(10) GLA_SCAN_CASE(11) GLA_SCAN_CASE(12) GLA_SCAN_CASE(13)
+      GLA_SCAN_CASE(14) GLA_SCAN_CASE(15) GLA_SCAN_CASE(16)
+      default: return UMB_EINVAL;
+    }
   }
 #undef GLA_SCAN_CASE
+#undef GLA_SCAN_WIDE
 #undef GLA_SCAN_LAUNCH
   UMB_LAUNCH_CHECK();
   return UMB_OK;
+}
+
+extern "C" int umb_lin_scan(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
+                            const float* alpha, int alpha_per_head, int qk_heads, const int* seq_slot, const int* seq_row0,
+                            const int* seq_pos0, const int* seq_len, int B, int H, int D, int Dv, float qscale, hipStream_t st) {
+  return umb_lin_scan_rows(o, state, q, ldq, k, ldk, v, ldv, alpha, alpha_per_head, qk_heads, seq_slot, seq_row0, seq_pos0, seq_len, 1, B, 1, H, D, Dv,
+                           qscale, st);
 }
 
 extern "C" int umb_gla_scan(float* o, float* state, const float* proj, int ld, const float* alpha, const int* seq_slot,

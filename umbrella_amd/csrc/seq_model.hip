@@ -153,14 +153,15 @@ static inline bool lin_step_ok(const float* v, int ldv, const float* state, int 
 }
 
 // Whether a step's gated linear attention runs in chunks: from three whole chunks on, where their time is the lesser one.  Token by token it
-// is the longest stretch's serial walk or all rows' share of the chip; in chunks every stretch, however short, is a chunk of full cost per
-// head, and the grid has the longest stretch's chunks for each of them (both fitted, us, one MI355X).  Token by token / in chunks, heads x
-// keys x values 8 x 128 x 256: 192 tokens 68 / 47, 2000 654 / 95, 8 stretches of 200 155 / 104, one of 192 beside 15 single tokens 72 / 113 (16 heads
-// 76 / 187), 300 beside 20 of 20 111 / 148; 32 x 64 x 64: 192 52 / 33, 192 beside 15 of 100 77 / 120, 32 of 192 207 / 290.
+// is the longest stretch's serial walk (slower with more columns a thread) or all rows' share of the chip; in chunks every stretch, however short, is a
+// chunk of full cost per head, and the grid has the longest stretch's chunks for each of them (both fitted, us, one MI355X).  Token by token / in chunks,
+// heads x keys x values 8 x 128 x 256: 192 tokens 64 / 45, 2000 654 / 95, 8 stretches of 192 93 / 87, 16 of 200 134 / 186, 8 of 400 188 / 146, one of 192 beside 15
+// single tokens 67 / 111 (16 heads 70 / 185), 300 beside 20 of 20 105 / 145; 32 x 64 x 64: 192 48 / 31, 192 beside 15 of 100 69 / 116, 32 of 192 159 / 287.
 static inline bool gla_chunks_pay(int T, int B, int max_len, int H, int D, int Dv) {
-  const double serial = max_len * (0.17 + 0.0013 * D), rows = 3.4e-7 * T * H * (double)D * Dv;
-  const double chunks = 30 + 1e-5 * (T / 64 + B) * H * (double)D * Dv + 5e-4 * ((max_len + 63) / 64) * (double)B * H * D;
-  return max_len >= 192 && chunks < (serial > rows ? serial : rows);
+  const int nc = lin_scan_cols(T, max_len, H, D, Dv);
+  const double walk = max_len * (0.17 + 0.0013 * D) * (nc == 4 ? 1.75 : nc == 2 ? 1.4 : 1.0), rows = 1.55e-7 * T * H * (double)D * Dv;
+  const double chunks = 30 + 0.7e-5 * (T / 64 + B) * H * (double)D * Dv + 5e-4 * ((max_len + 63) / 64) * (double)B * H * D;
+  return max_len >= 192 && chunks < (walk > rows ? walk : rows);
 }
 
 // softmax attention with a distance bias beside a state-space layer; both read the projection of the same input and write
@@ -206,8 +207,8 @@ static int mix_attn_ssd(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSe
   else if (single && lin_step_ok(sx, lds, ly.state, sDv))
     SEQ_TRY(umb_lin_step(ws->o, ly.state, sx + inner + sG * N, lds, sx + inner, lds, sx, lds, alpha, 1, sG, s->pos, s->slot, T, sH, N, sDv, 1.f, st));
   else
-    SEQ_TRY(umb_lin_scan(ws->o, ly.state, sx + inner + sG * N, lds, sx + inner, lds, sx, lds, alpha, 1, sG, s->seq_slot, s->seq_row0,
-                         s->seq_pos0, s->seq_len, s->B, sH, N, sDv, 1.f, st));
+    SEQ_TRY(umb_lin_scan_rows(ws->o, ly.state, sx + inner + sG * N, lds, sx + inner, lds, sx, lds, alpha, 1, sG, s->seq_slot, s->seq_row0,
+                              s->seq_pos0, s->seq_len, T, s->B, s->max_len, sH, N, sDv, 1.f, st));
   void* right = static_cast<char*>(ws->mix) + (size_t)H * E * seq_elem_bytes(dt);
   return umb_ssd_gate(right, ldo, ws->o, sx, lds, C, ws->proj, ld, col0, ly.s_d, ly.s_norm, T, sH, sDv, ly.s_norm_groups, m->eps,
                       ly.mix_scale_b, dt, st);
@@ -226,8 +227,8 @@ static int scan_per_head(float* o, float* state, const float* q, int ldq, const 
                                 s->max_len, H, D, P, scratch, scratch_floats, st);
   if (s->max_len == 1 && lin_step_ok(v, ldv, state, P))
     return umb_lin_step(o, state, q, ldq, k, ldk, v, ldv, alpha, 1, H, s->pos, s->slot, s->T, H, D, P, 1.f, st);
-  return umb_lin_scan(o, state, q, ldq, k, ldk, v, ldv, alpha, 1, H, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, s->B, H, D, P,
-                      1.f, st);
+  return umb_lin_scan_rows(o, state, q, ldq, k, ldk, v, ldv, alpha, 1, H, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, s->T, s->B,
+                           s->max_len, H, D, P, 1.f, st);
 }
 
 // retention: proj = [q | k | v | g]; rotary on q and k (k times its constant), the scan with the heads' fixed decays, per-head
@@ -430,8 +431,8 @@ static int run_mixer(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWo
       SEQ_TRY(umb_lin_step(ws->o, ly.state, ws->proj, ld, ws->proj + HD, ld, ws->proj + 2L * HD, ld, ws->aux, 0, H, s->pos, s->slot, T, H, D, Dv,
                            ly.qscale, st));
     else
-      SEQ_TRY(umb_gla_scan(ws->o, ly.state, ws->proj, ld, ws->aux, s->seq_slot, s->seq_row0, s->seq_pos0, s->seq_len, s->B, H, D,
-                           Dv, ly.qscale, st));
+      SEQ_TRY(umb_lin_scan_rows(ws->o, ly.state, ws->proj, ld, ws->proj + HD, ld, ws->proj + 2L * HD, ld, ws->aux, 0, H, s->seq_slot, s->seq_row0,
+                                s->seq_pos0, s->seq_len, T, s->B, s->max_len, H, D, Dv, ly.qscale, st));
     SEQ_TRY(umb_gla_gate(ws->mix, ws->o, ws->proj, ld, 2 * HD + H * Dv, ly.head_norm, T, H, Dv, eps, dt, st));
   } else if (ly.kind == UMB_MIX_LATENT) {
     // proj = [dq | dkv (latent + rotated key part) | gate]; the query latent goes up to the heads, its unrotated parts are

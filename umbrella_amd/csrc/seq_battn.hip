@@ -1011,6 +1011,10 @@ extern "C" int umb_bsa_attend(void* out, int ldo, const float* q, const UmbPaged
 // reads free to move ahead, and steps that every query sees whole left untested, 1999 positions, 32 + 8 heads of 128 went from 212 us to 141, two
 // maps over 617 positions, 64 | 128, from 104 to 71; rows by LDS-DMA, transposed reads in place of 2-byte stores, one barrier a step and fragments read
 // ahead of their products: 117 and 59, two maps of 128 | 256 over 2000 positions 252 -> 182.
+// What bounds it is vector instructions, half of which were addresses: 345 a step of 32 keys with a bias (32 products beside them).  Rows that fill
+// their tile are fetched by a lane's own place plus constants (RowLanes: 76 -> 9 a step), a bias walks by distance (91 -> 32) and is asked for where the
+// step before has used its own: with a bias 1999 positions, 32 + 8 heads of 128 159 us -> 136, of 64 116 -> 94, without 138 -> 123, two maps of
+// 128 | 256 245 -> 213.  Held to four waves a SIMD the loop spills (36 registers of heads of 128): 211.
 // FULL: D and E fill them, staging then tests nothing (2000 positions of 128: 158 us, 162 without).  us, run-time / these counts, 2000 positions: heads of 96 86 / 75, of 112 242 / 202, of 256 216 / 156, two maps of 128 | 128 273 / 179.
 // Two heads a wave, sharing the value fragments, are behind wherever a launch is not several rounds of workgroups: 600 positions, 64 + 8 heads
 // of 128 67 against 55, of 64 42 / 35 (2000 positions 195 / 198, 134 / 121).
@@ -1077,8 +1081,15 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
   const u16* vbase = reinterpret_cast<const u16*>(kv.v);
   auto key_at = [&](int kx) { return kx < kept ? kx : j_off + kx; };
   auto row_pos = [&](int kx) { return key_at(min(kx, total - 1)); };            // behind the last key the last one again, masked
+  RowLanes<4 * NSM * MAPS, 4> key_rows(kbase, wave, lane);
+  RowLanes<2 * NVM, 4> value_rows(vbase, wave, lane);
   auto issue = [&](int st) __attribute__((always_inline)) {
     const unsigned to = lds0 + (unsigned)(st & 1) * Tile::STEP;
+    if constexpr (FULL && key_rows.OK && value_rows.OK) {
+      key_rows.issue(tab + (st & 1) * 32, to, wave);
+      value_rows.issue(tab + (st & 1) * 32, to + Tile::Keys::BYTES, wave);
+      return;
+    }
     auto row_of = [&](int r) { return tab[(st & 1) * 32 + r]; };
     rows_issue<4 * NSM * MAPS, 4>(kbase, DK, to, wave, lane, row_of, [&](int c) {
       if (FULL && Tile::Keys::CH == 4 * NSM * MAPS) return c;
@@ -1090,6 +1101,16 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
   const int hd = g * hpg + (active ? hl : hpg - 1);
   float bnext[8];
   auto ask_bias = [&](int base) __attribute__((always_inline)) {
+    if (base >= kept) {                               // the walk itself: distances in a row from the lane's first one
+      const int d0 = i_j - j_off - base - 4 * g4;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const unsigned at = 4u * (unsigned)min(max(d0 - 16 * (e >> 2) - (e & 3), 0), n_dist - 1);
+        bnext[e] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(bias + (long)hd * n_dist) + at);
+      }
+      asm volatile("");                               // (or the loads are merged with those below, each with an address in two registers)
+      return;
+    }
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int dd = i_j - key_at(base + 16 * (e >> 2) + 4 * g4 + (e & 3)), di = dd < 0 ? 0 : (dd < n_dist ? dd : n_dist - 1);
@@ -1137,15 +1158,9 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
     // the step's rows have landed and nobody reads the step before any more: its buffer and its half of the table are free
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    float bv[8];
-    if (bias) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) bv[e] = bnext[e];
-    }
     if (threadIdx.x < 32) tab[(st & 1) * 32 + threadIdx.x] = next.row(kv, g, G);      // (in front of the issue: a wait for the look-up must not wait for that)
     if (st + 1 < steps) issue(st + 1);
     if (threadIdx.x < 32) next.ask(kv, slot, row_pos(base + 96 + threadIdx.x));
-    if (bias) ask_bias(base + 32);
     if (!active) continue;
     keys.at_step(lds0 + (unsigned)(st & 1) * Tile::STEP);
     values.at_step(lds0 + (unsigned)(st & 1) * Tile::STEP + Tile::Keys::BYTES);
@@ -1185,8 +1200,9 @@ __global__ __launch_bounds__(256) void bsa_attend_mfma_kernel(u16* __restrict__ 
       }
       if (bias) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sv[e] += bv[e] * BSA_LOG2E;
+        for (int e = 0; e < 8; ++e) sv[e] += bnext[e] * BSA_LOG2E;
       }
+      if (bias && hh == HPW - 1) ask_bias(base + 32);
       if (!whole) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {

@@ -50,6 +50,22 @@ __device__ __forceinline__ void rows_issue(const u16* base, long ld, unsigned ld
     }
   }
 }
+// The same where every row fills its tile and a piece is whole rows: a piece's row and chunk are then a lane's own plus a constant, and an address is
+// the look-up, a shift and an add.  (Put together from the piece's number they were 19 vector instructions a piece.)
+template <int CHUNKS, int NW> struct RowLanes {
+  typedef RowTile<CHUNKS> R;
+  static constexpr bool OK = CHUNKS == R::CH && (R::CH & (R::CH - 1)) == 0 && R::CH <= 64 && R::PIECES % NW == 0;
+  static constexpr int STEP = NW * 64 / R::CH;                  // rows from a wave's piece to its next
+  const char* base;
+  unsigned r0, c0;                                              // the first piece's row, and the place of its chunk in bytes
+  __device__ __forceinline__ RowLanes(const u16* base, int wave, int lane)
+      : base(reinterpret_cast<const char*>(base)), r0((unsigned)(wave * 64 + lane) / R::CH), c0(((unsigned)lane % R::CH ^ (r0 & R::XM)) * 16u) {}
+  __device__ __forceinline__ void issue(const unsigned* rows, unsigned lds, int wave) const {
+#pragma unroll
+    for (int i = 0; i < R::PIECES / NW; ++i)
+      rows_dma(base + (c0 ^ (unsigned)(STEP * i & R::XM) * 16u) + (size_t)rows[r0 + STEP * i] * R::ROW, lds + (unsigned)(wave + NW * i) * 1024u);
+  }
+};
 // A operand of 16 rows (16 u ..) x 32 columns (chunks 4 s ..): lane (j, g) reads chunk 4 s + g of row j.  at_step: the addresses of a step's buffer, of
 // which every read is one and a constant (opaque: put together from parts that do not change, each read's own would be kept over all steps)
 template <int CHUNKS> struct RowKeys {

@@ -22,6 +22,7 @@
 // items), so the same token in another batch, or of a prompt cut elsewhere, agrees to fp32 rounding and not bit for bit.
 #include "seq_common.h"
 #include "seq_decode.h"
+#include "seq_rows.h"
 
 // feature d (of D) of the sums of a pooled block's first cnt positions, keys and values, in order.  Lane j of a wave looks up position j's row, the rows go
 // round as scalars and sixteen positions are in flight together.  Called by whole waves.
@@ -601,13 +602,15 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
 // Key list of the tile: pooled blocks 0 .. nb(last position), then the tokens from the first position's window start to the last
 // position, in steps of 32 keys.  A step is staged ONCE for the four waves: key rows as cached (the A operand of S^T = K Q^T), values
 // transposed (the A operand of O^T += V^T P^T); pooled rows, held in fp32, as high and low halves.  The next step's rows are in flight
-// in registers while this one is used.  Per step and head:
+// while this one is used.  Per step and head:
 //   S^T as two 16-key MFMA tiles; P = visible ? sigmoid(S scale + bias) : 0 in fp32, lane (query j, key quad g) holding keys 4g .. 4g+3
 //   of both tiles -- which IS the lane's share of the B operand of the value product.
 // Scores and weights stay fp32-exact on a bf16 / f16 matrix pipe by splitting the fp32 factor into a high and a low 16-bit
 // half (x = hi + lo to 2^-17 in bf16, 2^-22 in fp16): q, the pooled means (held in fp32) and the weights go through two MFMAs instead of one.
 // It is bound by the vector work between the products.  With every wave staging its own values, gathering them two bytes at a time and
 // testing every key: 38 vector instructions a matrix instruction and 121 us at 2048 positions, 32 + 8 heads of 64, window 512; now 57.
+// Token rows that fill their tile (heads of 64, 128, 256) come by LDS-DMA a step ahead, values by transposed reads (seq_rows.h), instead of through registers
+// and 2-byte stores: 56.9 us -> 54.1, heads of 128 88.7 -> 82.3, of 256 (16 + 4) 131 -> 112.
 // A quarter of that is the sigmoid: with the exponential and the reciprocal as the units give them 45, but its error then grows with the score
 // (relative, root mean square in 2^-24: 1.7 within scores of 8 and 6.1 within 30; as below 0.64 and 0.56, a full divide the same).
 // 1 / (1 + e^-x): the quotient by one Newton step, which rounds as the divide does
@@ -637,7 +640,9 @@ __global__ __launch_bounds__(256) void pwa_attend_mfma_kernel(u16* __restrict__ 
   u16* v_hi = k_hi + 32 * LD;                              // [D][LT]
   u16* k_lo = v_hi + D * LT;                               // the low halves of pooled rows
   u16* v_lo = k_lo + 32 * LD;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
+  typedef RowLanes<4 * NS, 4> KeyLanes;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, j = lane & 15, g4 = lane >> 4;
+  const KeyLanes key_rows(reinterpret_cast<const u16*>(kv.k), wave, lane), value_rows(reinterpret_cast<const u16*>(kv.v), wave, lane);
   const int b = blockIdx.y, g = blockIdx.z;
   const int n = seq_len[b], q0 = blockIdx.x * 16;
   if (q0 >= n) return;                                     // the whole workgroup
@@ -755,35 +760,13 @@ __global__ __launch_bounds__(256) void pwa_attend_mfma_kernel(u16* __restrict__ 
     }
 
     // ---- tokens
-    u32x4 tk[NL], tv[NL];
-    auto fetch_tokens = [&](int base) {
-      const long off = (long)pkv_tok_row(kv, slot, j_lo + min(base + sm, n_tok - 1), g, G) * D;
-#pragma unroll
-      for (int u = 0; u < NL; ++u) {
-        const int ch = sc + 8 * u;
-        if (D % 64 == 0 || ch < D / 8) {
-          tk[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const u16*>(kv.k) + off + 8 * ch);
-          tv[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const u16*>(kv.v) + off + 8 * ch);
-        }
-      }
-    };
-    fetch_tokens(0);
-    for (int base = 0; base < n_tok; base += 32) {
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < NL; ++u) {
-        const int ch = sc + 8 * u;
-        if (D % 64 == 0 || ch < D / 8) put(k_hi, v_hi, ch, tk[u], tv[u]);
-      }
-      __syncthreads();
-      if (base + 32 < n_tok) fetch_tokens(base + 32);
-      if (!active) continue;
+    auto token_step = [&](int base, auto key_of, auto value_of) __attribute__((always_inline)) {
       f32x4 s2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int s = 0; s < NS; ++s)
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const u32x4 kh = key_tile(k_hi, u, s);
+          const u32x4 kh = key_of(u, s);
           s2[u] = P::mfma(kh, qlo[s], s2[u]);
           s2[u] = P::mfma(kh, qhi[s], s2[u]);
         }
@@ -792,9 +775,65 @@ __global__ __launch_bounds__(256) void pwa_attend_mfma_kernel(u16* __restrict__ 
       weights(s2, jt + 31 <= i_first && jt > i_last - window, [&](int k) { return jt + k <= i_j && jt + k > i_j - window; }, phi, plo);
 #pragma unroll
       for (int dt = 0; dt < 2 * NS; ++dt) {
-        const u32x4 vh = value_tile(v_hi, dt);
+        const u32x4 vh = value_of(dt);
         o[dt] = P::mfma(vh, plo, o[dt]);
         o[dt] = P::mfma(vh, phi, o[dt]);
+      }
+    };
+    if constexpr (KeyLanes::OK) {                          // by LDS-DMA, a step ahead (seq_rows.h)
+      constexpr unsigned HALF = KeyLanes::R::BYTES, BUF = 2 * HALF;
+      const unsigned lds0 = (unsigned)(size_t)(lds_char*)pwa_lds;
+      unsigned* tab = reinterpret_cast<unsigned*>(pwa_lds + BUF);          // [2][32] behind two buffers of a step's key rows and value rows
+      const int steps = (n_tok + 31) / 32;
+      auto row_pos = [&](int x) { return j_lo + min(x, n_tok - 1); };
+      auto issue = [&](int st) __attribute__((always_inline)) {
+        key_rows.issue(tab + (st & 1) * 32, lds0 + (unsigned)(st & 1) * BUF, wave);
+        value_rows.issue(tab + (st & 1) * 32, lds0 + (unsigned)(st & 1) * BUF + HALF, wave);
+      };
+      RowKeys<4 * NS> keys(j, g4);
+      RowValues<4 * NS> values(j, g4);
+      RowAsked next{};
+      __syncthreads();                                     // every wave is done with what stood there
+      if (threadIdx.x < 64) tab[threadIdx.x] = pkv_tok_row(kv, slot, row_pos(threadIdx.x), g, G);
+      if (threadIdx.x < 32) next.ask(kv, slot, row_pos(64 + threadIdx.x));
+      __syncthreads();
+      issue(0);
+      for (int st = 0; st < steps; ++st) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");        // the step's rows have landed, the step before is read
+        __builtin_amdgcn_s_barrier();
+        if (threadIdx.x < 32) tab[(st & 1) * 32 + threadIdx.x] = next.row(kv, g, G);
+        if (st + 1 < steps) issue(st + 1);
+        if (threadIdx.x < 32) next.ask(kv, slot, row_pos(32 * st + 96 + threadIdx.x));
+        if (!active) continue;
+        keys.at_step(lds0 + (unsigned)(st & 1) * BUF);
+        values.at_step(lds0 + (unsigned)(st & 1) * BUF + HALF);
+        token_step(32 * st, keys, values);
+      }
+    } else {
+      u32x4 tk[NL], tv[NL];
+      auto fetch_tokens = [&](int base) {
+        const long off = (long)pkv_tok_row(kv, slot, j_lo + min(base + sm, n_tok - 1), g, G) * D;
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+          const int ch = sc + 8 * u;
+          if (D % 64 == 0 || ch < D / 8) {
+            tk[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const u16*>(kv.k) + off + 8 * ch);
+            tv[u] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const u16*>(kv.v) + off + 8 * ch);
+          }
+        }
+      };
+      fetch_tokens(0);
+      for (int base = 0; base < n_tok; base += 32) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+          const int ch = sc + 8 * u;
+          if (D % 64 == 0 || ch < D / 8) put(k_hi, v_hi, ch, tk[u], tv[u]);
+        }
+        __syncthreads();
+        if (base + 32 < n_tok) fetch_tokens(base + 32);
+        if (!active) continue;
+        token_step(base, [&](int u, int s) { return key_tile(k_hi, u, s); }, [&](int dt) { return value_tile(v_hi, dt); });
       }
     }
     // lane holds O^T[d = 16 dt + 4 g4 + rr][query j]
@@ -952,7 +991,7 @@ extern "C" int umb_pwa_attend_tiled(void* out, const float* q, const UmbPagedKV*
       !pkv_ok(kv) || !proj || !seq_slot || !seq_row0 || !seq_pos0 || !seq_len || dtype == UMB_SEQ_F32)
     return UMB_EINVAL;
   const dim3 grid((max_len + 15) / 16, B, G);
-  const size_t lds = 2 * ((size_t)32 * (D + 8) + (size_t)D * 36) * sizeof(u16);
+  const size_t lds = 2 * ((size_t)32 * (D + 8) + (size_t)D * 36) * sizeof(u16);      // pooled tiles; two steps of token rows and their table are less
 #define PWA_MFMA_CASE(NS)                                                                                                  \
   case NS:                                                                                                                 \
     if (ensure_dynamic_lds<pwa_attend_mfma_kernel<P, NS>>(lds) != UMB_OK) return UMB_EHIP;                                 \

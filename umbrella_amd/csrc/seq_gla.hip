@@ -5,8 +5,8 @@
 // state, the products that enter it and the read-out.  The state lives in a slot array [slots][H][D][Dv] and is carried from
 // step to step; a sequence whose first row is at position 0 starts from zero whatever its slot held before.
 //
-// scan kernel: one WAVE owns four value columns of one (sequence, head): lane (r = lane % 16, c = lane / 16) keeps NR
-// consecutive rows (r NR ...) of column c in registers, so the update is register-local and the read-out sum over rows is a
+// scan kernel: one WAVE owns four value columns of one (sequence, head), or twice or four times as many (lin_scan_cols): lane (r = lane % 16, c = lane / 16)
+// keeps NR consecutive rows (r NR ...) of column c in registers, so the update is register-local and the read-out sum over rows is a
 // butterfly inside 16 lanes, and the order of every sum is fixed by (D) alone -- a token's output never depends on how the
 // sequence was cut into steps.  The token loop is the only serial dimension; its inputs are independent of the recurrence and
 // are staged ahead through LDS in chunks of 16 tokens.

@@ -774,8 +774,8 @@ extern "C" int umb_lat_attend_split(void* out, const float* qa, const UmbPagedKV
   if (T < 1 || H < 1 || kv_rank < 1 || kv_rank > 64 * LAT_MAXC || rot_dim < 0 || window < 1 || !out || !qa || !lat_kv_ok(kv) ||
       !pos || !slot)
     return UMB_EINVAL;
-  // Few tokens: the vector-pipe kernel below spreads a token's keys over sixteen waves and its heads over several workgroups
-  // and finishes sooner; from a few dozen tokens on the chip is full either way and sharing each key fragment among sixteen
+  // Few tokens: on the vector pipe (lat_decode; other shapes and fp32 the kernel below) a token's keys are spread over sixteen waves, its heads and, with
+  // scratch, its key spans over several workgroups, and it finishes sooner; from a few dozen tokens on the chip is full either way and sharing each key fragment among sixteen
   // heads wins (batch 128 at 1024 keys, kv_rank 512: 1.17 ms a step against 2.40).  UMB_LAT_DEC_MIN moves the switch.
   const char* env = getenv("UMB_LAT_DEC_MIN");
   const int lat_dec_min = env ? atoi(env) : 48;

@@ -252,13 +252,13 @@ extern "C" int umb_lin_scan_rows(float* o, float* state, const float* q, int ldq
                                  const float* alpha, int alpha_per_head, int qk_heads, const int* seq_slot, const int* seq_row0,
                                  const int* seq_pos0, const int* seq_len, int T, int B, int max_len, int H, int D, int Dv, float qscale,
                                  hipStream_t st) {
-  if (T < 1 || B < 1 || max_len < 1 || max_len > T || H < 1 || D < 1 || D > 16 * GLA_MAXR || Dv < 1 || qk_heads < 1 || H % qk_heads || !o || !state ||
+  if (B < 1 || H < 1 || D < 1 || D > 16 * GLA_MAXR || Dv < 1 || qk_heads < 1 || H % qk_heads || !o || !state ||
       !q || !k || !v || !alpha || ldq < qk_heads * D || ldk < qk_heads * D || ldv < H * Dv)
     return UMB_EINVAL;
   const int nr = (D + 15) / 16, aph = alpha_per_head ? 1 : 0, hpg = H / qk_heads;
   const bool v4 = D % 4 == 0 && Dv % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 &&
                   ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (aph ? 0 : (uintptr_t)alpha)) % 16 == 0;
-  const int nc = v4 ? lin_scan_cols(T, max_len, H, D, Dv) : 1;
+  const int nc = v4 && max_len > 0 ? lin_scan_cols(T, max_len, H, D, Dv) : 1;
   const dim3 grid((Dv + GLA_COLS * nc - 1) / (GLA_COLS * nc), H, B);
 #define GLA_SCAN_LAUNCH(NR, V4, NC)                                                                                       \
   do {                                                                                                                    \

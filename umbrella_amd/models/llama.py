@@ -632,13 +632,13 @@ class Llama(LLMBase):
         return self._bufs["h"]
 
     # ------------------------------------------------------------------ forward
-    def _run(self, step: UmbStep, logits: torch.Tensor = None):
+    def _run(self, step: UmbStep, logits: int = None):
         lib = _lib.load()
         st = _lib.stream_ptr()
         ws = self._ws
         if logits is not None:                      # the head's rows go there and not into the workspace's
             ws = UmbWorkspace.from_buffer_copy(ws)
-            ws.logits = logits.data_ptr()
+            ws.logits = logits
         if self._tp is not None:
             assert self._off is None, "tensor-parallel shards are device resident"
             rc = lib.umb_model_forward_tp(C.byref(self._m), C.byref(ws), C.byref(step), C.byref(self._tp), st)
@@ -664,8 +664,8 @@ class Llama(LLMBase):
 
     def forward_explicit(self, tokens, positions, slots, prefix_len, mask_bits=None, mask_words=0, n_mask_keys=None,
                          head_from=0, layer_range=None, skip_embed=False, logits=None):
-        """Explicit-mode step: int32 device arrays tokens/positions/slots [T], prefix_len int32[1].  logits: where the head's fp32 rows go (the
-        workspace's buffer)."""
+        """Explicit-mode step: int32 device arrays tokens/positions/slots [T], prefix_len int32[1].  logits: the address the head's fp32 rows go to
+        (the workspace's buffer)."""
         T = tokens.shape[0]
         s = UmbStep()
         s.T = T
@@ -735,10 +735,12 @@ class Llama(LLMBase):
         out = torch.empty(T, V, dtype=torch.float32, device=dev)
         for lo in range(0, T, self.logit_rows):
             hi = min(T, lo + self.logit_rows)
-            # straight into the result where the head's stores are aligned there (257 rows of 128256: 45 us of copying)
-            direct = self.is_last and out[lo].data_ptr() % 16 == 0
+            # straight into the result where the head's stores are aligned there (257 rows of 128256: 45 us of copying;
+            # the address by arithmetic: what stands in front of the launches is waited for, and two slices more were 3 us of a call of 520)
+            to = out.data_ptr() + 4 * lo * V
+            direct = self.is_last and to % 16 == 0
             self.forward_explicit(idx[lo:hi], idx[T + lo:T + hi], idx[2 * T + lo:2 * T + hi], pre,
-                                  mask_bits=bits[lo:hi], mask_words=W, n_mask_keys=nmk, head_from=0, logits=out[lo:hi] if direct else None)
+                                  mask_bits=bits[lo:hi], mask_words=W, n_mask_keys=nmk, head_from=0, logits=to if direct else None)
             if not direct:
                 out[lo:hi] = self._bufs["logits"][:hi - lo]
         last = scan[2 * nb] if slots.shape[0] == T else int(slots.max().item())

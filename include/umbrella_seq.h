@@ -205,7 +205,8 @@ int umb_pwa_attend(void* out, const float* q, const UmbPagedKV* kv, const float*
 /* The same attention for steps that bring whole stretches of a sequence (prompts), on the matrix pipe: 16-bit storage only,
  * D a multiple of 32 (<= 256); workgroups own 16 consecutive positions of one sequence.  Scores and weights keep fp32
  * accuracy: the fp32 factors (q, pooled means, weights) enter as high + low 16-bit halves. */
-/* all of it for steps of one token a sequence (q: scratch of T H D floats, left as it is where it is one launch) */
+/* all of it for steps of one token a sequence, every slot once (one launch appends and attends; q: scratch of T H D floats, left as it is where it is
+ * one launch) */
 int umb_pwa_step(void* out, float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const void* pos_bias, const int* pos,
                  const int* slot, const float* freq, const int* seq_slot, const int* seq_pos0, const int* seq_len, int T, int H, int G,
                  int D, int rot_dims, int window, int pool, float scale, float eps, int dtype, umb_stream_t stream);
@@ -375,7 +376,8 @@ int umb_attn_attend(void* out, int ldo, const float* q, const UmbPagedKV* kv, co
                     const float* bias, int n_dist, const int* pos, const int* slot, int T, int H, int G, int D, int E, int window,
                     float scale, float out_scale, float softcap, const UmbAttnForm* form, float* scratch, long scratch_floats,
                     int dtype, umb_stream_t stream);
-/* both for steps of one token a sequence (q: scratch of T maps H D floats, left as it is where the two are one launch) */
+/* both for steps of one token a sequence, every slot once (one launch appends and attends; q: scratch of T maps H D floats, left as it is where the two
+ * are one launch) */
 int umb_attn_step(void* out, int ldo, float* q, const UmbPagedKV* kv, const float* proj, int ld, int append, const void* w_q, const void* w_k,
                   int norm_qk, int norm_v, const float* freq, int rot_dims, int layout, float rot_mult, float temp_coef, int temp_every,
                   float eps, const UmbValueMix* mix, int gate_col, const float* bias, int n_dist, const int* pos, const int* slot, int T,
@@ -623,6 +625,8 @@ typedef struct UmbSeqWork {
   float* v_first;      /* values that later layers of the step mix in [Tmax][kv_heads vdim] fp32 (null when no layer does) */
 } UmbSeqWork;
 
+/* Each slot is one sequence of the step, its rows stand together: single tokens (max_len 1) are appended beside the attention of the step's other
+ * rows, and a recurrent state has one owner a step. */
 typedef struct UmbSeqStep {
   int32_t T, B, R, max_len;
   const int32_t *tokens, *pos, *slot;                       /* [T] */

@@ -51,6 +51,21 @@ def _linear(w, b=None) -> UmbSeqLinear:
     return s
 
 
+def _one_stretch_each(toks, seq_slot, row0, pos0, lens):
+    """A step's parts with those of one sequence put together, in the order of their first ones: no mixer takes two stretches of a sequence (single
+    tokens are appended beside the attention of the step's other rows, and a recurrent state has one owner a step).  Returns the tokens, the parts'
+    first rows, where every row of the parts went, and the stretches' (slot, first row, first position, length)."""
+    order = sorted(range(len(lens)), key=lambda i: seq_slot.index(seq_slot[i]))
+    came = np.concatenate([np.arange(row0[i], row0[i] + lens[i]) for i in order])        # the row of the parts that stands in each place
+    back = np.empty_like(came)
+    back[came] = np.arange(len(came))
+    first = back[row0]
+    heads = [i for i in order if seq_slot.index(seq_slot[i]) == i]
+    slots = [seq_slot[i] for i in heads]
+    total = [sum(n for n, other in zip(lens, seq_slot) if other == slot) for slot in slots]
+    return [toks[r] for r in came], first, back, (slots, [int(first[i]) for i in heads], [pos0[i] for i in heads], total)
+
+
 class SeqMixLM(LLMBase):
     """Subclasses provide ``read_config(path)``, ``layer_tensors(i, layer_cfg, get)`` and ``top_tensors(get)``."""
 
@@ -475,8 +490,8 @@ class SeqMixLM(LLMBase):
     # ------------------------------------------------------------------ forward
     @torch.inference_mode()
     def forward_batch(self, parts, want=None, trace: bool = False):
-        """One step of a ragged batch.  parts: [(seq_id, token ids)], each the NEXT tokens of an open sequence; want: per
-        part the indices (into that part) whose logits are asked for (default: the last one).  Returns the fp32 logits
+        """One step of a ragged batch.  parts: [(seq_id, token ids)], each the NEXT tokens of an open sequence (several parts of one sequence
+        are one stretch of it, in their order); want: per part the indices (into that part) whose logits are asked for (default: the last one).  Returns the fp32 logits
         [rows wanted, V] (a view of the workspace, valid until the next step) in the order of parts and of want; with
         trace also the residual stream after every layer [L, T, W]."""
         cache, dev = self.kv_cache, self.device
@@ -496,16 +511,19 @@ class SeqMixLM(LLMBase):
                 rows.extend(w), counts.append(len(w)), toks.extend(ids)
         finally:                                     # a part that is refused leaves those before it extended
             cache.write_pages(entries)
-        T, B, R = len(toks), len(parts), len(rows)
+        first, back = np.asarray(row0), None         # the parts' first rows, from which `rows` count
+        if len(set(seq_slot)) < len(parts):          # a sequence named again: its parts are one stretch, whose rows stand together
+            toks, first, back, (seq_slot, row0, pos0, lens) = _one_stretch_each(toks, seq_slot, row0, pos0, lens)
+        T, B, R = len(toks), len(lens), len(rows)
         self.reserve(T, max(R, 1))
         # tokens, their positions and slots | per sequence: slot, first row, first position, length | rows whose logits are wanted.  Up to a few
         # thousand rows: filled by array operations, and sent without waiting -- a copy that waits for the stream leaves the device idle
         # while the host makes the step's launches, and a step's host work cannot run beside the step before it
         meta_host = torch.empty(3 * T + 4 * B + R, dtype=torch.int32)
         at = meta_host.numpy()
-        first, n_of = np.asarray(row0), np.asarray(lens)
+        n_of = np.asarray(lens)
         at[:T] = toks
-        at[T:2 * T] = np.arange(T) + np.repeat(np.asarray(pos0) - first, n_of)
+        at[T:2 * T] = np.arange(T) + np.repeat(np.asarray(pos0) - np.asarray(row0), n_of)
         at[2 * T:3 * T] = np.repeat(np.asarray(seq_slot), n_of)
         at[3 * T:3 * T + 4 * B] = seq_slot + row0 + pos0 + lens
         wanted = np.asarray(rows, dtype=np.int64) + np.repeat(first, counts)
@@ -551,6 +569,8 @@ class SeqMixLM(LLMBase):
             if graphed:
                 entry["runs"] += 1
         logits = self._bufs["logits"][:R]
+        if trace and back is not None:
+            tr = tr[:, torch.from_numpy(back).to(dev)]
         return (logits, tr) if trace else logits
 
     # ---- the reference's single-sequence face (umbrella/models/base.py:4-32): tokens continue ONE sequence

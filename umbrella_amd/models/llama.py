@@ -187,13 +187,20 @@ def mask_rows(mask: torch.Tensor, T: int):
     return mask, (mask.stride(0) if T > 1 else Cn)
 
 
+class PromptChunk:
+    """Prompt tokens per forward when the workspace allows."""
+    PACKED = 1024   # the matrix-bound verify GEMM streams the weights once per chunk (70B-AWQ, 2048-token prompt: 4.2 k tok/s at 128, 6.1 k at 256,
+                    # 6.7 k at 512, 7.0 k at 1024; 1B: 53 k / 94 k / 155 k / 211 k)
+    DENSE = 2048    # the same of 16-bit weights, whose products have no limit of 1024 rows: fewer partial sums, whole rounds of tiles, one walk
+                    # over the keys (8B widths, 2048-token prompt and one token: 8526 -> 7751 us)
+
+    def __get__(self, model, owner=None):
+        return self.PACKED if model is None or model.config.awq else self.DENSE
+
+
 class Llama(LLMBase):
     CHUNK = 64          # rows of the default workspace (tree / generic forwards)
-    PREFILL_CHUNK = 1024  # prompt tokens per forward when the workspace allows: the matrix-bound verify GEMM streams the
-                          # weights once per chunk (70B-AWQ, 2048-token prompt: 4.2 k tok/s at 128, 6.1 k at 256, 6.7 k at
-                          # 512, 7.0 k at 1024; 1B: 53 k / 94 k / 155 k / 211 k)
-    PREFILL_CHUNK_DENSE = 2048   # the same of 16-bit weights, whose products have no limit of 1024 rows: fewer partial sums, whole rounds of tiles, one walk
-                                 # over the keys (8B widths, 2048-token prompt and one token: 8526 -> 7751 us)
+    PREFILL_CHUNK = PromptChunk()       # a class or a model may set a number of its own
 
     def __init__(self, model_name: str, batch_size: int = 1, max_length: int = 256, device: str = "cuda:0",
                  dtype=torch.float16, offload: bool = False, cuda_graph: bool = False, state_dict=None,
@@ -231,8 +238,6 @@ class Llama(LLMBase):
         if self.sched == "auto":
             self.sched = "split" if (self.config.awq or self.config.hidden_size >= 4096) else "ll"
         c = self.config
-        if not c.awq:
-            self.PREFILL_CHUNK = self.PREFILL_CHUNK_DENSE
         if c.attention_bias:
             self.fused = False                    # projection bias: default / low-latency schedules only
         self.hidden_size, self.num_heads, self.head_dim = c.hidden_size, c.num_attention_heads, c.head_dim

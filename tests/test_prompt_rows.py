@@ -3,6 +3,7 @@ import pytest
 
 from umbrella_amd.models.config import LlamaCfg
 from umbrella_amd.models.llama import Llama
+from umbrella_amd.parallel import prefill_chunk
 
 
 def config(awq):
@@ -29,3 +30,17 @@ def test_what_a_class_or_a_model_says_stands(awq, rows, monkeypatch):
     assert m.PREFILL_CHUNK == rows
     monkeypatch.setattr(Llama, "PREFILL_CHUNK", rows)
     assert model(awq).PREFILL_CHUNK == rows
+
+
+@pytest.mark.parametrize("first,last", [(True, False), (False, False), (False, True)])
+def test_a_stage_of_several_sends_messages_that_overlap(first, last):
+    """a prompt of 2048 tokens is two messages, so that the stages work side by side; a stage that holds every layer has nobody to send to"""
+    m = model(False)
+    m.is_first, m.is_last, m.ws_tokens = first, last, 4096
+    assert m.PREFILL_CHUNK == 1024 and prefill_chunk(m) == 1024
+    m.PREFILL_CHUNK = 512
+    assert prefill_chunk(m) == 512
+    m = model(False)
+    m.is_first = m.is_last = True
+    m.ws_tokens = 4096
+    assert prefill_chunk(m) == 2048

@@ -193,9 +193,13 @@ class PromptChunk:
                     # 6.7 k at 512, 7.0 k at 1024; 1B: 53 k / 94 k / 155 k / 211 k)
     DENSE = 2048    # the same of 16-bit weights, whose products have no limit of 1024 rows: fewer partial sums, whole rounds of tiles, one walk
                     # over the keys (8B widths, 2048-token prompt and one token: 8526 -> 7751 us)
+    STAGE = 1024    # and of a pipeline stage, whose chunks are the messages to the next one: 2048 tokens in two of them keep two stages busy
 
     def __get__(self, model, owner=None):
-        return self.PACKED if model is None or model.config.awq else self.DENSE
+        if model is None or model.config.awq:
+            return self.PACKED
+        whole = getattr(model, "is_first", True) and getattr(model, "is_last", True)
+        return self.DENSE if whole else self.STAGE
 
 
 class Llama(LLMBase):

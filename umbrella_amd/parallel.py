@@ -233,7 +233,8 @@ class PipelinedTarget:
 
 
 def prefill_chunk(model) -> int:
-    """rows per prompt message: the stage model's prompt chunk (1024 when the workspace allows)"""
+    """rows per prompt message: the stage model's prompt chunk (1024 between stages, 2048 where one holds every layer of 16-bit weights,
+    when the workspace allows)"""
     return max(model.CHUNK, min(model.PREFILL_CHUNK, model.ws_tokens))
 
 

@@ -2,7 +2,7 @@
 import pytest
 
 from umbrella_amd.models.config import LlamaCfg
-from umbrella_amd.models.llama import Llama
+from umbrella_amd.models.llama import Llama, workspace_rows
 from umbrella_amd.parallel import prefill_chunk
 
 
@@ -44,3 +44,26 @@ def test_a_stage_of_several_sends_messages_that_overlap(first, last):
     m.is_first = m.is_last = True
     m.ws_tokens = 4096
     assert prefill_chunk(m) == 2048
+
+
+@pytest.mark.parametrize("awq", [False, True])
+def test_no_workspace_for_prompts_that_a_model_cannot_hold(awq):
+    short, long = model(awq, max_length=300), model(awq, max_length=8192)
+    assert short.max_length == 320 and workspace_rows(short, 64) == 320
+    assert workspace_rows(long, 64) == long.PREFILL_CHUNK
+    assert workspace_rows(short, 769) == 784 and workspace_rows(long, 4100) == 4112        # a tree's rows are kept, whole tiles of 16
+    for m, rows in ((short, 1), (short, 769), (long, 64), (long, 4100)):
+        m.ws_tokens = workspace_rows(m, rows)
+        assert prefill_chunk(m) <= m.ws_tokens                                             # every message fits the buffers that are made for it
+    long.PREFILL_CHUNK = 256
+    assert workspace_rows(long, 64) == 256
+
+
+@pytest.mark.gpu
+def test_an_engine_reserves_what_its_models_can_hold():
+    import torch
+    from helpers import load_golden
+    from hip_helpers import static_engine
+    eng, _ = static_engine(load_golden(), "cuda:0", torch.float16, self_draft=True, max_length=256)
+    for m in (eng.draft_model, eng.target_model):
+        assert m.ws_tokens == 256

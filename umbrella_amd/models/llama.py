@@ -202,6 +202,12 @@ class PromptChunk:
         return self.DENSE if whole else self.STAGE
 
 
+def workspace_rows(model, rows: int) -> int:
+    """Rows of a model's workspace for whole prompt chunks (of what it can hold: partial sums of 2048 rows beside a context of 300 are 0.5 GB at 8B widths
+    that nobody uses) and for the `rows` of its trees, in whole tiles."""
+    return _align(max(min(model.PREFILL_CHUNK, model.max_length), rows), 16)
+
+
 class Llama(LLMBase):
     CHUNK = 64          # rows of the default workspace (tree / generic forwards)
     PREFILL_CHUNK = PromptChunk()       # a class or a model may set a number of its own

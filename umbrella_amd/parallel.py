@@ -357,7 +357,7 @@ def build_pipelined_engine(device: str, dtype=torch.float16, seed: int = 0, **co
     import json as _json
 
     from .models.config import KNOWN, LlamaCfg
-    from .models.llama import Llama, pack_mask_bits
+    from .models.llama import Llama, pack_mask_bits, workspace_rows
     from .speculation.static_speculation_engine import resolve_growmap_path
     kind = config.pop("engine", "static")
     assert kind in ("static", "dynamic"), kind
@@ -385,9 +385,10 @@ def build_pipelined_engine(device: str, dtype=torch.float16, seed: int = 0, **co
         T, max_path = W * Dp + 1, Dp + 1
         depth = torch.tensor([0] + [i + 1 for i in range(Dp) for _ in range(W)], dtype=torch.int32, device=device)
         mask_bits = torch.zeros(T, (T + 63) // 64, dtype=torch.int64, device=device)
-    stage.reserve(max(stage.PREFILL_CHUNK, T), logit_rows=max(stage.CHUNK, T))
+    rows = workspace_rows(stage, max(stage.CHUNK, T))
+    stage.reserve(rows, logit_rows=max(stage.CHUNK, T))
     host_staging = dist.get_backend() == "gloo"
-    comm = PipelineComm(rank, world, device, cfg.hidden_size, dtype, max(stage.PREFILL_CHUNK, T), max_path,
+    comm = PipelineComm(rank, world, device, cfg.hidden_size, dtype, rows, max_path,
                         host_staging=host_staging)
     if rank != 0:
         tables = dict(depth=depth, mask_bits=mask_bits, n_dev=torch.zeros(1, dtype=torch.int32, device=device),

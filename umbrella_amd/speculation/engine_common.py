@@ -22,6 +22,7 @@ import torch
 from .. import _lib
 from ..logging_config import setup_logger
 from ..models import AutoModelLM
+from ..models.llama import workspace_rows
 from ..utils import TextColors
 from .base import BaseEngine
 from .speculation_utils import IdTokenizer, is_sentence_complete_regex
@@ -116,7 +117,7 @@ class HipEngine(BaseEngine):
         # final workspace sizes before any graph capture: wide prompt chunks, logits only for tree rows
         for mdl, rows in ((self.draft_model, max(self.draft_rows, 2)), (self.target_model, tree_size)):
             rows = max(mdl.CHUNK, rows)
-            mdl.reserve(max(mdl.PREFILL_CHUNK, rows), logit_rows=rows)
+            mdl.reserve(workspace_rows(mdl, rows), logit_rows=rows)
 
     # ------------------------------------------------------------------ text API
     def prefill(self, text: str):

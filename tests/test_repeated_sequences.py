@@ -41,7 +41,8 @@ def host_model(monkeypatch, steps):
     return m
 
 
-@pytest.mark.parametrize("parts,want", [([("a", [7]), ("a", [8])], [[0], [0]]), (PARTS, WANT), (PARTS, None), ([("b", [1]), ("a", [2])], None)])
+@pytest.mark.parametrize("parts,want", [([("a", [7]), ("a", [8])], [[0], [0]]), (PARTS, WANT), (PARTS, None), ([("b", [1]), ("a", [2])], None),
+                                        ([("b", [1]), ("a", [2])], [[0, 0], []]), ([("b", [1]), ("c", [2]), ("a", [3])], [[0], [0], [0]])])
 def test_each_sequence_is_one_stretch(monkeypatch, parts, want):
     steps, before = [], {"a": 3, "b": 0, "c": 6}
     m = host_model(monkeypatch, steps)

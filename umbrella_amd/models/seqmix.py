@@ -511,24 +511,26 @@ class SeqMixLM(LLMBase):
                 rows.extend(w), counts.append(len(w)), toks.extend(ids)
         finally:                                     # a part that is refused leaves those before it extended
             cache.write_pages(entries)
-        first, back = np.asarray(row0), None         # the parts' first rows, from which `rows` count
+        first, back = row0, None                     # the parts' first rows, from which `rows` count
         if len(set(seq_slot)) < len(parts):          # a sequence named again: its parts are one stretch, whose rows stand together
             toks, first, back, (seq_slot, row0, pos0, lens) = _one_stretch_each(toks, seq_slot, row0, pos0, lens)
         T, B, R = len(toks), len(lens), len(rows)
         self.reserve(T, max(R, 1))
-        # tokens, their positions and slots | per sequence: slot, first row, first position, length | rows whose logits are wanted.  Up to a few
-        # thousand rows: filled by array operations, and sent without waiting -- a copy that waits for the stream leaves the device idle
-        # while the host makes the step's launches, and a step's host work cannot run beside the step before it
-        meta_host = torch.empty(3 * T + 4 * B + R, dtype=torch.int32)
-        at = meta_host.numpy()
-        n_of = np.asarray(lens)
-        at[:T] = toks
-        at[T:2 * T] = np.arange(T) + np.repeat(np.asarray(pos0) - np.asarray(row0), n_of)
-        at[2 * T:3 * T] = np.repeat(np.asarray(seq_slot), n_of)
-        at[3 * T:3 * T + 4 * B] = seq_slot + row0 + pos0 + lens
-        wanted = np.asarray(rows, dtype=np.int64) + np.repeat(first, counts)
-        at[3 * T + 4 * B:] = wanted
-        every = R == T and bool((wanted == np.arange(T)).all())             # every row, in order: the last seam norms them for the head
+        # tokens, their positions and slots | per sequence: slot, first row, first position, length | rows whose logits are wanted.  Sent without
+        # waiting -- a copy that waits for the stream leaves the device idle while the host makes the step's launches, and a step's host work
+        # cannot run beside the step before it
+        if T == B and counts == lens and not any(rows):                     # a token a sequence, the logits of each
+            every, meta_host = True, torch.tensor(toks + pos0 + seq_slot + seq_slot + row0 + pos0 + lens + row0, dtype=torch.int32)
+        else:                                        # up to a few thousand rows: by array operations (of which a step as above had 11 us)
+            meta_host = torch.empty(3 * T + 4 * B + R, dtype=torch.int32)
+            at, n_of = meta_host.numpy(), np.asarray(lens)
+            at[:T] = toks
+            at[T:2 * T] = np.arange(T) + np.repeat(np.asarray(pos0) - np.asarray(row0), n_of)
+            at[2 * T:3 * T] = np.repeat(np.asarray(seq_slot), n_of)
+            at[3 * T:3 * T + 4 * B] = seq_slot + row0 + pos0 + lens
+            wanted = np.asarray(rows, dtype=np.int64) + np.repeat(np.asarray(first), counts)
+            at[3 * T + 4 * B:] = wanted
+            every = R == T and bool((wanted == np.arange(T)).all())         # every row, in order: the last seam norms them for the head
         graphed = self.use_graph and not trace and T == B and str(dev).startswith("cuda")     # a pure decode step
         key = (T, R, every)
         if graphed:

@@ -286,11 +286,13 @@ int umb_mingru_scan(void* out, float* state, const float* proj, int ld, int z_co
 int umb_lin_scan(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
                  const float* alpha, int alpha_per_head, int qk_heads, const int* seq_slot, const int* seq_row0,
                  const int* seq_pos0, const int* seq_len, int B, int H, int D, int Dv, float qscale, umb_stream_t stream);
-/* the same of a step of T rows whose longest stretch has max_len: more columns a thread where the rows fill the chip (umb_lin_scan: one) */
+/* the same of a step of T rows whose longest stretch has max_len: more columns a thread where the rows fill the chip (umb_lin_scan, and
+ * max_len 0: one) */
 int umb_lin_scan_rows(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
                       const float* alpha, int alpha_per_head, int qk_heads, const int* seq_slot, const int* seq_row0,
                       const int* seq_pos0, const int* seq_len, int T, int B, int max_len, int H, int D, int Dv, float qscale,
                       umb_stream_t stream);
+int umb_lin_scan_columns(int T, int max_len, int H, int D, int Dv);   /* how many, where the operands move in 16-byte pieces (no stream) */
 /* a step of ONE token per sequence (row t at position pos[t] of slot[t]; position 0 starts from S = 0), sums in the order of umb_lin_scan; v and
  * state 16-byte aligned, Dv and ldv multiples of four */
 int umb_gla_step(void* out, float* state, const float* proj, int ld, const void* w_a2, const void* b_a2, const void* w_norm, const int* pos,

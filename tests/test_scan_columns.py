@@ -2,9 +2,8 @@
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
 
-
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,groups,D,Dv,per_head", [(16, 16, 128, 256, 0), (16, 16, 128, 68, 0), (32, 8, 64, 84, 1), (9, 3, 256, 132, 0), (64, 64, 52, 16, 1), (24, 24, 184, 100, 0)])
 @pytest.mark.parametrize("lens", [[17, 1, 16, 0], [33] * 5, [20] * 40])
 def test_columns_of_a_thread(lens, H, groups, D, Dv, per_head):
@@ -44,3 +43,14 @@ def test_columns_of_a_thread(lens, H, groups, D, Dv, per_head):
         assert bool((o[T] == 7.0).all())
     if D % 64 == 0:                              # whole quads of rows: the same sums, whatever a thread's columns (contractions aside)
         assert float((out[0][0] - out[1][0]).abs().max()) <= 2.0 ** -20 * float(want.abs().max())
+
+
+def test_the_plain_scan_is_one_column():
+    """umb_lin_scan asks with max_len 0, of which no rows that fill the chip follow, however many heads; (rows, longest): the lines of the rule"""
+    from umbrella_amd import _lib
+    cols = _lib.load_seq().umb_lin_scan_columns
+    for H, D, Dv in ((64, 256, 256), (32, 256, 256), (16, 128, 256), (1024, 52, 64)):
+        assert cols(1, 0, H, D, Dv) == 1
+    assert [cols(n * 96, 96, 16, 128, 256) for n in (1, 3, 4, 7, 8)] == [1, 1, 2, 2, 4]
+    assert cols(800, 96, 16, 120, 256) == 4 and cols(800, 96, 16, 112, 256) == 1           # a lane's rows in whole quads
+    assert cols(0, 1, 1, 1, 1) < 0 and cols(1, 1, 1, 257, 1) < 0

@@ -336,6 +336,7 @@ SEQ_SIGNATURES = {
     "umb_mingru_scan": [_P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _I, _I, _I, _P, _L, _I],
     "umb_gla_step": [_P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _F, _I],
     "umb_lin_step": [_P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _I, _I, _I, _I, _F],
+    "umb_lin_scan_columns": [_I, _I, _I, _I, _I],
     "umb_lin_scan_rows": [_P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F],
     "umb_lin_scan": [_P, _P, _P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P, _I, _I, _I, _I, _F],
     "umb_ssd_prep": [_P, _I, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I],
@@ -379,7 +380,7 @@ SEQ_SIGNATURES = {
     "umb_sample_rows": [_P, _P, _I, _I, _P, _P, _F, _F, _I, _F, _P, _I, _P, _P],
     "umb_seq_version": [],
 }
-_SEQ_NO_STREAM = {"umb_lat_attend_tiled_ok", "umb_seq_linear_split", "umb_seq_tile_kind", "umb_seq_tile_mix", "umb_seq_resid_canon_step_ok", "umb_bsa_attend_tiled_ok", "umb_mingru_scratch_floats",
+_SEQ_NO_STREAM = {"umb_lat_attend_tiled_ok", "umb_seq_linear_split", "umb_seq_tile_kind", "umb_seq_tile_mix", "umb_lin_scan_columns", "umb_seq_resid_canon_step_ok", "umb_bsa_attend_tiled_ok", "umb_mingru_scratch_floats",
                   "umb_ssd_scan_chunked_floats", "umb_delta_scan_floats", "umb_gla_scan_chunked_floats"}          # predicates: no stream argument, the value is the answer
 _seq_lib = None
 

@@ -153,9 +153,10 @@ constexpr long QUAD_ROWS = 400;
 // columns, and those reads are the time where the rows of all stretches fill the chip; where the longest stretch's walk is the time, more columns make
 // its steps longer.  The line: workgroups of 16 columns that the rows keep busy over that walk, times rows a lane (keys / 16).  us with 1 / 2 / 4 columns,
 // heads x keys x values: 16 x 128 x 256, one stretch of 96 36 / 44 / 61, 2 41 / 46 / 61, 4 74 / 51 / 64, 8 116 / 93 / 70, 16 of 51 - 96 184 / 133 / 117; 8 x 256 x 256, 2
-// of 100 66 / 80 / 113, 8 252 / 158 / 116; 32 x 64 x 64, 8 of 100 39 / 39 / 46, 32 113 / 92 / 92.
+// of 100 66 / 80 / 113, 8 252 / 158 / 116; 32 x 64 x 64, 8 of 100 39 / 39 / 46, 32 113 / 92 / 92.  max_len 0: nothing is known of the stretches, one column.
 static inline int lin_scan_cols(int T, int max_len, int H, int D, int Dv) {
   const int nr = (D + 15) / 16;
+  if (max_len < 1) return 1;
   const double busy = (double)T / max_len * H * ((Dv + 15) / 16) * nr;
   return nr % 4 ? 1 : busy >= 16384 ? 4 : busy >= 8192 ? 2 : 1;
 }

@@ -248,6 +248,10 @@ extern "C" int umb_gla_decay_log(float* log_alpha, const float* proj, int ld, in
   return gla_decay_launch<true>(log_alpha, proj, ld, a_col, w_a2, b_a2, T, HD, rank, tau, dtype, st);
 }
 
+extern "C" int umb_lin_scan_columns(int T, int max_len, int H, int D, int Dv) {
+  return T < 1 || H < 1 || D < 1 || D > 16 * GLA_MAXR || Dv < 1 ? UMB_EINVAL : lin_scan_cols(T, max_len, H, D, Dv);
+}
+
 extern "C" int umb_lin_scan_rows(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
                                  const float* alpha, int alpha_per_head, int qk_heads, const int* seq_slot, const int* seq_row0,
                                  const int* seq_pos0, const int* seq_len, int T, int B, int max_len, int H, int D, int Dv, float qscale,
@@ -258,7 +262,7 @@ extern "C" int umb_lin_scan_rows(float* o, float* state, const float* q, int ldq
   const int nr = (D + 15) / 16, aph = alpha_per_head ? 1 : 0, hpg = H / qk_heads;
   const bool v4 = D % 4 == 0 && Dv % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 &&
                   ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (aph ? 0 : (uintptr_t)alpha)) % 16 == 0;
-  const int nc = v4 && max_len > 0 ? lin_scan_cols(T, max_len, H, D, Dv) : 1;
+  const int nc = v4 ? lin_scan_cols(T, max_len, H, D, Dv) : 1;
   const dim3 grid((Dv + GLA_COLS * nc - 1) / (GLA_COLS * nc), H, B);
 #define GLA_SCAN_LAUNCH(NR, V4, NC)                                                                                       \
   do {                                                                                                                    \
@@ -297,7 +301,7 @@ extern "C" int umb_lin_scan_rows(float* o, float* state, const float* q, int ldq
 extern "C" int umb_lin_scan(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv,
                             const float* alpha, int alpha_per_head, int qk_heads, const int* seq_slot, const int* seq_row0,
                             const int* seq_pos0, const int* seq_len, int B, int H, int D, int Dv, float qscale, hipStream_t st) {
-  return umb_lin_scan_rows(o, state, q, ldq, k, ldk, v, ldv, alpha, alpha_per_head, qk_heads, seq_slot, seq_row0, seq_pos0, seq_len, 1, B, 1, H, D, Dv,
+  return umb_lin_scan_rows(o, state, q, ldq, k, ldk, v, ldv, alpha, alpha_per_head, qk_heads, seq_slot, seq_row0, seq_pos0, seq_len, 1, B, 0, H, D, Dv,
                            qscale, st);
 }
 

@@ -495,8 +495,8 @@ __global__ __launch_bounds__(256 * CG) void gla_step_kernel(typename El<P>::type
 
 extern "C" int umb_gla_step(void* out, float* state, const float* proj, int ld, const void* w_a2, const void* b_a2, const void* w_norm, const int* pos,
                             const int* slot, int T, int H, int D, int Dv, int rank, float tau, float qscale, float eps, int dtype, hipStream_t st) {
-  if (T < 1 || T > 65535 || H < 1 || D < 1 || D > 16 * GLA_MAXR || Dv < 4 || Dv % 4 || Dv > 256 || rank < 1 || !(tau > 0.f) || !out || !state || !proj || !w_a2 ||
-      !w_norm || !pos || !slot || (long)ld < 2L * H * D + 2L * H * Dv + rank || (uintptr_t)state % 16)
+  if (T < 1 || T > 65535 || H < 1 || D < 1 || D > 16 * GLA_MAXR || Dv < 4 || Dv % 4 || Dv > 256 || rank < 1 || rank > 8192 || !(tau > 0.f) || !out || !state || !proj ||
+      !w_a2 || !w_norm || !pos || !slot || (long)ld < 2L * H * D + 2L * H * Dv + rank || (uintptr_t)state % 16)
     return UMB_EINVAL;
   const int nr = (D + 15) / 16;
 #define GLA_STEP(R, CG)                                                                                                                       \

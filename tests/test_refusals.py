@@ -20,3 +20,21 @@ def gla_step(rank, ld=None, **kw):
 def test_gla_step(kw):
     """decays of a rank above 8192 are refused for prompts too"""
     assert gla_step(**kw) == EINVAL
+
+
+@pytest.mark.parametrize("rows", [None, AT])
+@pytest.mark.parametrize("streams,block", [(0, 0), (1, 0), (0, 1)])
+def test_logits_without_a_final_norm(rows, streams, block):
+    """also where every row is wanted and the last seam norms them: nothing would write what the head reads"""
+    layer, m, ws, s = _lib.UmbSeqLayer(), _lib.UmbSeqModel(), _lib.UmbSeqWork(), _lib.UmbSeqStep()
+    m.dtype, m.L, m.W, m.V, m.groups, m.eps, m.streams, m.block = 1, 1, 64, 64, 1, 1e-6, streams, block
+    m.embed, m.layers = AT, C.pointer(layer)
+    layer.norm1 = AT
+    for k in ("x", "h", "proj", "aux", "o", "mix", "act", "y", "logits", "h2", "y2"):
+        setattr(ws, k, AT)
+    ws.Tmax, ws.Rmax, ws.aux_floats, ws.y_rows = 16, 16, 1 << 20, 16
+    s.T, s.B, s.R, s.max_len = 1, 1, 1, 1
+    for k in ("tokens", "pos", "slot", "seq_slot", "seq_row0", "seq_pos0", "seq_len"):
+        setattr(s, k, AT)
+    s.logit_rows = rows
+    assert _lib.load_seq().umb_seq_forward(C.byref(m), C.byref(ws), C.byref(s), None) == EINVAL

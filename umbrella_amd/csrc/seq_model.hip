@@ -535,7 +535,7 @@ static int forward_parallel_blocks(const UmbSeqModel* m, const UmbSeqWork* ws, c
 }
 
 extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const UmbSeqStep* s, hipStream_t st) {
-  if (!m || !ws || !s || m->L < 1 || !m->layers || s->T < 1 || s->T > ws->Tmax || s->B < 1 || s->R < 0 || s->R > ws->Rmax)
+  if (!m || !ws || !s || m->L < 1 || !m->layers || s->T < 1 || s->T > ws->Tmax || s->B < 1 || s->R < 0 || s->R > ws->Rmax || (s->R > 0 && !m->final_norm))
     return UMB_EINVAL;
   if (m->block == UMB_BLOCK_PARALLEL) return forward_parallel_blocks(m, ws, s, st);
   const int T = s->T, W = m->W, dt = m->dtype, groups = m->groups;

@@ -192,7 +192,8 @@ int umb_pwa_prep(float* q, const UmbPagedKV* kv, const float* proj, int ld, cons
 /* pooled entries of every block whose last position this step wrote: the fp32 mean of the `pool` cached keys / values */
 int umb_pwa_pool(const UmbPagedKV* kv, const int* seq_slot, const int* seq_pos0, const int* seq_len, int B, int max_len, int G,
                  int D, int pool, int dtype, umb_stream_t stream);
-/* both for one token a sequence (token t is sequence t's only one): the blocks that the tokens complete in the launch that prepares them */
+/* both for one token a sequence (token t is sequence t's only one, every slot once): the blocks that the tokens complete in the launch that prepares
+ * them */
 int umb_pwa_prep_step(float* q, const UmbPagedKV* kv, const float* proj, int ld, const int* pos, const int* slot, const float* freq,
                       const int* seq_slot, const int* seq_pos0, const int* seq_len, int T, int H, int G, int D, int rot_dims, int pool,
                       float eps, int dtype, umb_stream_t stream);
@@ -205,15 +206,15 @@ int umb_pwa_attend(void* out, const float* q, const UmbPagedKV* kv, const float*
 /* The same attention for steps that bring whole stretches of a sequence (prompts), on the matrix pipe: 16-bit storage only,
  * D a multiple of 32 (<= 256); workgroups own 16 consecutive positions of one sequence.  Scores and weights keep fp32
  * accuracy: the fp32 factors (q, pooled means, weights) enter as high + low 16-bit halves. */
-/* all of it for steps of one token a sequence, every slot once (one launch appends and attends; q: scratch of T H D floats, left as it is where it is
- * one launch) */
-int umb_pwa_step(void* out, float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const void* pos_bias, const int* pos,
-                 const int* slot, const float* freq, const int* seq_slot, const int* seq_pos0, const int* seq_len, int T, int H, int G,
-                 int D, int rot_dims, int window, int pool, float scale, float eps, int dtype, umb_stream_t stream);
 int umb_pwa_attend_tiled(void* out, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col,
                          const void* pos_bias, const int* seq_slot, const int* seq_row0, const int* seq_pos0, const int* seq_len,
                          int B, int max_len, int H, int G, int D, int window, int pool, float scale, int dtype,
                          umb_stream_t stream);
+/* preparation, pooled blocks and attention for steps of one token a sequence, every slot once (one launch appends and attends; any D up to 512 and
+ * fp32 too, as two launches; q: scratch of T H D floats, left as it is where it is one launch) */
+int umb_pwa_step(void* out, float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const void* pos_bias, const int* pos,
+                 const int* slot, const float* freq, const int* seq_slot, const int* seq_pos0, const int* seq_len, int T, int H, int G,
+                 int D, int rot_dims, int window, int pool, float scale, float eps, int dtype, umb_stream_t stream);
 
 /* ---- latent attention: queries and keys/values go through low-rank latents; the cache holds, per token, the normed
  * key/value latent c [kv_rank] and one rotated key part [rot_dim] shared by all heads (one row of kv_rank + rot_dim in
@@ -295,11 +296,14 @@ int umb_lin_scan_rows(float* o, float* state, const float* q, int ldq, const flo
 int umb_lin_scan_columns(int T, int max_len, int H, int D, int Dv);   /* how many, where the operands move in 16-byte pieces (no stream) */
 /* a step of ONE token per sequence (row t at position pos[t] of slot[t]; position 0 starts from S = 0), sums in the order of umb_lin_scan; v and
  * state 16-byte aligned, Dv and ldv multiples of four */
-int umb_gla_step(void* out, float* state, const float* proj, int ld, const void* w_a2, const void* b_a2, const void* w_norm, const int* pos,
-                 const int* slot, int T, int H, int D, int Dv, int rank, float tau, float qscale, float eps, int dtype, umb_stream_t stream);
 int umb_lin_step(float* o, float* state, const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, const float* alpha,
                  int alpha_per_head, int qk_heads, const int* pos, const int* slot, int T, int H, int D, int Dv, float qscale,
                  umb_stream_t stream);
+/* gated linear attention of one token per sequence (every slot once), decay, recurrence, per-head norm and gate in one launch, sums in the order of
+ * umb_gla_scan: proj rows [q | k | v | gate | W_a1 h] of any ld >= 2 H D + 2 H Dv + rank; state 16-byte aligned; D and Dv <= 256, Dv a multiple of
+ * four, rank <= 8192, T <= 65535; out [T][H Dv] in `dtype`, b_a2 may be null */
+int umb_gla_step(void* out, float* state, const float* proj, int ld, const void* w_a2, const void* b_a2, const void* w_norm, const int* pos,
+                 const int* slot, int T, int H, int D, int Dv, int rank, float tau, float qscale, float eps, int dtype, umb_stream_t stream);
 
 /* ---- selective state space with a scalar decay per head (state-space duality).  proj fp32 [T][ld]; from column col0:
  * [z (H Dv) | x (H Dv) | B (G N) | C (G N) | dt (H)].  prep: x, B, C through a causal convolution per channel (w [C][taps],

@@ -218,14 +218,14 @@ __device__ __forceinline__ AttnKeys attn_keys(int i, int window, const UmbAttnFo
   return AttnKeys{j_lo, kept, kept + i - j_lo + 1};
 }
 
-// end of a workgroup: the partial sums o_s [nact][RH][Ep], maxima and denominators ml_s [nact][RH][2] (and 2 RH floats behind the nw-th)
-// of its waves, added in wave order; nact <= 16: a row's factors are worked out once, by 16 lanes.
-// part: this split's result goes there instead ([token][row][split][E + 2] = o .., maximum, denominator)
 // a head's sink: fp32, or a latent layer's in storage format
 template <typename P, bool LAT> __device__ __forceinline__ float sink_of(const float* sink, int h) {
   if constexpr (LAT) return P::to_f(reinterpret_cast<const u16*>(sink)[h]);
   else return sink[h];
 }
+// end of a workgroup: the partial sums o_s [nact][RH][Ep], maxima and denominators ml_s [nact][RH][2] (and 2 RH floats behind the nw-th)
+// of its waves, added in wave order; nact <= 16: a row's factors are worked out once, by 16 lanes.
+// part: this split's result goes there instead ([token][row][split][E + 2] = o .., maximum, denominator)
 template <typename P, int RH, int NC, int MAPS, bool LAT = false>
 __device__ __forceinline__ void attn_finish(typename El<P>::type* __restrict__ out, int ldo, const float* o_s, int Ep, float* ml_s,
                                             int nact, int nw, float* __restrict__ part, int split, int nsplit,
@@ -772,9 +772,6 @@ static int bsa_launch(dim3 grid, size_t lds, hipStream_t st, void* out, int ldo,
   return UMB_OK;
 }
 
-// the decode kernel: spans of ATT_SPAN keys dealt to several workgroups only where few items leave the chip idle; 16 waves per item as
-// long as every item gets a compute unit of its own (values of 256: their registers do not hold it), 8 while two share one, 4 beyond
-// (us with 8 / 4 waves, 32 + 8 heads of 128: 1024 items behind 30 / 200 keys 12.8 / 8.4, 30.2 / 27.5; 512 items behind 500 28.8 / 36.7)
 // workgroups that one item's spans of keys are dealt to; most: keys a token can have, floats: of one split of all items
 static inline int decode_splits(int span, long items, long most, long floats, const float* scratch, long scratch_floats) {
   int nsplit = 1;
@@ -785,6 +782,9 @@ static inline int decode_splits(int span, long items, long most, long floats, co
   }
   return nsplit;
 }
+// the decode kernel: spans of ATT_SPAN keys dealt to several workgroups only where few items leave the chip idle; 16 waves per item as
+// long as every item gets a compute unit of its own (values of 256: their registers do not hold it), 8 while two share one, 4 beyond
+// (us with 8 / 4 waves, 32 + 8 heads of 128: 1024 items behind 30 / 200 keys 12.8 / 8.4, 30.2 / 27.5; 512 items behind 500 28.8 / 36.7)
 template <typename P>
 static int attn_decode(void* out, int ldo, const float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const float* bias,
                        int n_dist, const int* pos, const int* slot, int T, int H, int G, int D, int E, int window, float scale,

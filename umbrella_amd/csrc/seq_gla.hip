@@ -7,8 +7,9 @@
 //
 // scan kernel: one WAVE owns four value columns of one (sequence, head), or twice or four times as many (lin_scan_cols): lane (r = lane % 16, c = lane / 16)
 // keeps NR consecutive rows (r NR ...) of column c in registers, so the update is register-local and the read-out sum over rows is a
-// butterfly inside 16 lanes, and the order of every sum is fixed by (D) alone -- a token's output never depends on how the
-// sequence was cut into steps.  The token loop is the only serial dimension; its inputs are independent of the recurrence and
+// butterfly inside 16 lanes, and the order of every sum is fixed by (D) alone, in the kernels of single tokens too: how a sequence
+// was cut into steps moves a token's output by the compiler's contractions at most (by the sums of the chunked form where a long stretch takes
+// that).  The token loop is the only serial dimension; its inputs are independent of the recurrence and
 // are staged ahead through LDS in chunks of 16 tokens.
 #include "seq_common.h"
 #include <type_traits>

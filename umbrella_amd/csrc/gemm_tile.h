@@ -60,6 +60,7 @@ template <int WM, int WN, int RA, int RB, int KS> struct TileShape {
 
 // The tiles a launch chooses from, and what a 64-k stage of a whole round of 256 workgroups takes (us; one MI355X, bf16, random data).  Few sizes
 // of a prompt fill rounds of one tile; between 0.46 (256 x 256) and 1.4 ns a stage, row and token the right one is the one that fills best.
+// (Of one whole round, between K 4096 and 8192, the first two are down to 1.36 and 1.19 with three slots of A; the rules were fitted with these.)
 //                       rows tokens stage
 enum { TILE_256 = 0,  //  256   256  1.42
        TILE_192 = 1,  //  256   192  1.20
@@ -69,13 +70,14 @@ enum { TILE_256 = 0,  //  256   256  1.42
        TILE_128 = 5,  //  128   128  0.49
        TILE_64K = 6,  //  128    64  0.38   K over two groups of waves
        TILE_KINDS = 7 };
+struct Tile { int bn, bt; double us; };
+constexpr Tile TILES[TILE_KINDS] = {{256, 256, 1.42}, {256, 192, 1.20}, {256, 160, 1.04}, {256, 128, 0.86}, {256, 96, 0.73}, {128, 128, 0.49}, {128, 64, 0.38}};
 // us of a launch: 4, and for each round its stages, 2 in front of them and 14 for 256 x 256 outputs behind them; a last round that is not
 // full takes a little less (its share of the memory path is larger).  rows: of A; stages: of one slab; S: slabs
 static inline double tile_cost(int kind, int T, int rows, int stages, int S) {
-  static const struct { int bn, bt; double us; } k[TILE_KINDS] = {{256, 256, 1.42}, {256, 192, 1.20}, {256, 160, 1.04}, {256, 128, 0.86},
-                                                                 {256, 96, 0.73}, {128, 128, 0.49}, {128, 64, 0.38}};
-  const long wgs = (long)((rows + k[kind].bn - 1) / k[kind].bn) * ((T + k[kind].bt - 1) / k[kind].bt) * S, rest = wgs % 256;
-  const double load = rest / 256.0, products = stages * k[kind].us, out = 2.1e-4 * k[kind].bn * k[kind].bt;
+  const Tile k = TILES[kind];
+  const long wgs = (long)((rows + k.bn - 1) / k.bn) * ((T + k.bt - 1) / k.bt) * S, rest = wgs % 256;
+  const double load = rest / 256.0, products = stages * k.us, out = 2.1e-4 * k.bn * k.bt;
   return 4.0 + (wgs / 256) * (products + out + 2.0) + (rest ? products * (0.8 + 0.2 * load) + out * load + 2.0 : 0.0);
 }
 // the least of them (the K-split one takes an even number of stages)
@@ -92,20 +94,20 @@ static inline int tile_kind(int T, int rows, int stages, int S, bool even, doubl
 // What it may save is the last round's idle share, so it has to be 3 % ahead.
 struct TileMix { int columns, tail; };
 static inline TileMix tile_mix(int T, int rows, int stages, double single) {
-  static const struct { int kind, bt; double us; } k[4] = {{TILE_192, 192, 1.20}, {TILE_160, 160, 1.04}, {TILE_128W, 128, 0.86}, {TILE_96, 96, 0.73}};
   const long nbt = (T + 255) / 256, all = (rows + 255L) / 256 * nbt, rounds = all / 256;
   TileMix best{0, 0};
   if (rounds == 0 || all % 256 == 0 || nbt > 256) return best;
   const int columns = (int)(256 * rounds / nbt);
   const long tail = (rows + 255) / 256 - columns, spare = 256 * rounds - columns * nbt;
   if (tail <= 0) return best;
-  const double main = 4.0 + rounds * (stages * 1.42 + 2.1e-4 * 256 * 256 + 2.0);
+  const double main = 4.0 + rounds * (stages * TILES[TILE_256].us + 2.1e-4 * 256 * 256 + 2.0);
   double least = 0.97 * single;
-  for (int i = 0; i < 4; ++i) {
-    const long wgs = tail * ((T + k[i].bt - 1) / k[i].bt) - spare, rest = wgs > 0 ? wgs % 256 : 0;
-    const double load = rest / 256.0, products = stages * k[i].us, out = 2.1e-4 * 256 * k[i].bt;
+  for (int i = TILE_192; i <= TILE_96; ++i) {              // the others of 256 rows
+    const Tile k = TILES[i];
+    const long wgs = tail * ((T + k.bt - 1) / k.bt) - spare, rest = wgs > 0 ? wgs % 256 : 0;
+    const double load = rest / 256.0, products = stages * k.us, out = 2.1e-4 * 256 * k.bt;
     const double us = main + (wgs > 0 ? wgs / 256 * (products + out + 2.0) : 0.0) + (rest ? products * (0.8 + 0.2 * load) + out * load + 2.0 : 0.0);
-    if (us < least) { least = us; best = TileMix{columns, k[i].kind}; }
+    if (us < least) { least = us; best = TileMix{columns, i}; }
   }
   return best;
 }

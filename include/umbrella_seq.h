@@ -210,7 +210,7 @@ int umb_pwa_attend_tiled(void* out, const float* q, const UmbPagedKV* kv, const 
                          const void* pos_bias, const int* seq_slot, const int* seq_row0, const int* seq_pos0, const int* seq_len,
                          int B, int max_len, int H, int G, int D, int window, int pool, float scale, int dtype,
                          umb_stream_t stream);
-/* preparation, pooled blocks and attention for steps of one token a sequence, every slot once (one launch appends and attends; any D up to 512 and
+/* preparation, pooled blocks and attention for steps of one token a sequence, every slot once (one launch appends and attends; any D up to 256 and
  * fp32 too, as two launches; q: scratch of T H D floats, left as it is where it is one launch) */
 int umb_pwa_step(void* out, float* q, const UmbPagedKV* kv, const float* proj, int ld, int gate_col, const void* pos_bias, const int* pos,
                  const int* slot, const float* freq, const int* seq_slot, const int* seq_pos0, const int* seq_len, int T, int H, int G,

@@ -4,7 +4,9 @@ import torch
 
 import potosun_helpers
 import seqmix_helpers
+import tomopel_helpers
 import tutunex_helpers
+import zusuvik_helpers
 
 pytestmark = pytest.mark.gpu
 
@@ -13,7 +15,12 @@ MODELS = {"grouped norms": lambda dt: seqmix_helpers.build(seqmix_helpers.config
           "two mixers": lambda dt: tutunex_helpers.build(tutunex_helpers.config([tutunex_helpers.layer(tutunex_helpers.attention()),
                                                                                   tutunex_helpers.layer(tutunex_helpers.parallel())]), dt),
           "one stream": lambda dt: potosun_helpers.build(potosun_helpers.config([potosun_helpers.layer(potosun_helpers.biased()),
-                                                                                 potosun_helpers.layer(potosun_helpers.latent())]), dt)}
+                                                                                 potosun_helpers.layer(potosun_helpers.latent())]), dt),
+          # the null row list of these goes to the launch that reads the sum of the streams, or the one stream of parallel blocks
+          "two streams": lambda dt: tomopel_helpers.build(tomopel_helpers.config([tomopel_helpers.layer(tomopel_helpers.parallel()),
+                                                                                  tomopel_helpers.layer(tomopel_helpers.mingru())]), dt),
+          "parallel blocks": lambda dt: zusuvik_helpers.build(zusuvik_helpers.config([zusuvik_helpers.layer(zusuvik_helpers.retention()),
+                                                                                      zusuvik_helpers.layer(zusuvik_helpers.parallel(), mlp=None)]), dt)}
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

@@ -83,3 +83,38 @@ def test_step_as_three_launches(dtype, H, G, D, rot, window, pool, lens):
     assert bool(((a[1] - b[1]).abs() <= step_of * a[1].abs()).all()) and bool(((a[3] - b[3]).abs() <= 16 * step_of / pool + 2.0 ** -19).all())
     # the rotation and the norm may be contracted otherwise, the sums are of up to 600 weights below 1 in the same order
     assert bool(((a[0] - b[0]).abs() <= 2 * step_of * a[0].abs() + 2.0 ** -18 * min(window, max(lens))).all())
+
+
+def test_sequences_that_bring_nothing_stand_in_front(monkeypatch):
+    """a caller of the library may list sequences of length 0: the blocks of those behind them are pooled too, also where pooling is a launch over the
+    list (from 16384 head slots on)"""
+    import types
+    from umbrella_amd import _lib
+    import seqmix_helpers
+    B, pool = 2100, 3
+    cfg = seqmix_helpers.config([seqmix_helpers.attn_layer(heads=6, kv_heads=2, dim=12, window=2, pool=pool, ff=16)], width=16, vocab=20, groups=1)
+    m, _ = seqmix_helpers.build(cfg, torch.float32, batch=B + 1, max_length=16, max_tokens=16 * (B + 1))
+    real, keep, got = _lib.load_seq(), [], []
+
+    def forward(model, work, step, stream):
+        s = step._obj
+        if s.max_len == 1:
+            for k, first in (("seq_slot", m.kv_cache.slot("empty")), ("seq_row0", 0), ("seq_pos0", 0), ("seq_len", 0)):
+                own = (m._keep[3 * s.T + ("seq_slot", "seq_row0", "seq_pos0", "seq_len").index(k) * s.B:][:s.B])
+                keep.append(torch.cat([torch.tensor([first], dtype=torch.int32, device="cuda"), own]))
+                setattr(s, k, keep[-1].data_ptr())
+            s.B += 1
+        return real.umb_seq_forward(model, work, step, stream)
+    for listed in (False, True):
+        m.clear()
+        for i in ["empty"] + list(range(B)):
+            m.open(i)
+        m.forward_batch([(i, [i % 7, i % 5]) for i in range(B)])
+        if listed:
+            monkeypatch.setattr(_lib, "load_seq", lambda: types.SimpleNamespace(umb_seq_forward=forward))
+        m.kv_cache.kv[0]["kp"].fill_(9.0)
+        m.forward_batch([(i, [i % 11]) for i in range(B)])
+        got.append([m.kv_cache.pooled_rows(0, i, [0])[0] for i in (0, B // 2, B - 1)])
+    assert len(keep) == 4
+    for a, b in zip(*got):
+        assert torch.equal(a, b) and bool((a != 9.0).all())

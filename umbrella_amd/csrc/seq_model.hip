@@ -399,7 +399,8 @@ static int run_mixer(const UmbSeqModel* m, const UmbSeqLayer& ly, const UmbSeqWo
   if (ly.kind == UMB_MIX_POOLED_WINDOW) {
     const int H = ly.heads, G = ly.kv_heads, D = ly.dim;
     if (ly.vdim != D || ld != H * D + G * D + H) return UMB_EINVAL;
-    if (s->max_len == 1)                       // a token a sequence: all of it in one launch where the shape allows it
+    // a token a sequence, and no sequence listed that brings none (the step takes the list as long as the tokens): one launch where the shape allows it
+    if (s->max_len == 1 && s->B == T)
       return umb_pwa_step(ws->mix, ws->aux, &ly.kv, ws->proj, ld, H * D + G * D, ly.pos_bias, s->pos, s->slot, ly.rot_freq, s->seq_slot, s->seq_pos0, s->seq_len,
                           T, H, G, D, ly.rot_dims, ly.window, ly.pool, ly.scale, eps, dt, st);
     SEQ_TRY(umb_pwa_prep(ws->aux, &ly.kv, ws->proj, ld, s->pos, s->slot, ly.rot_freq, T, H, G, D, ly.rot_dims, eps, dt, st));

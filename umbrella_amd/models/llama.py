@@ -191,8 +191,12 @@ class PromptChunk:
     """Prompt tokens per forward when the workspace allows."""
     PACKED = 1024   # the matrix-bound verify GEMM streams the weights once per chunk (70B-AWQ, 2048-token prompt: 4.2 k tok/s at 128, 6.1 k at 256,
                     # 6.7 k at 512, 7.0 k at 1024; 1B: 53 k / 94 k / 155 k / 211 k)
-    DENSE = 2048    # the same of 16-bit weights, whose products have no limit of 1024 rows: fewer partial sums, whole rounds of tiles, one walk
-                    # over the keys (8B widths, 2048-token prompt and one token: 8526 -> 7751 us)
+    # the same of 16-bit weights, whose products have no limit of 1024 rows: fewer partial sums, whole rounds of tiles, one walk over the keys.  us at
+    # 1024 / 1536 / 2048 / 3072 / 4096 rows a forward, four layers of 8B widths: 1500 tokens 3070 / 2637 / 2656 / 2658 / 2640, 2048 tokens 3844 / 3829 /
+    # 3389 / 3378 / 3376, 3000 tokens 5738 / 5307 / 5280 / 5077 / 5061, 4096 tokens 7897 / 7467 / 6976 / 7213 / 6647, 6000 tokens 12288 / 11580 / 10799 /
+    # 10768 / 10517; eight of 1B widths, 2048 tokens 3101 / 3176 / 2566 / 2569 / 2567, 4096 tokens 6706 / 6287 / 5580 / 5633 / 5041.  4096 would take 3 - 10 %
+    # off prompts of more than 2048 tokens for twice the partial sums.
+    DENSE = 2048
     STAGE = 1024    # and of a pipeline stage, whose chunks are the messages to the next one: 2048 tokens in two of them keep two stages busy
 
     def __get__(self, model, owner=None):

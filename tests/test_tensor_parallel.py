@@ -109,7 +109,7 @@ def _tp_worker(rank, world, port, q):
     logits = _tp_forward_torch(cfg, local, rank, world, ids, pos, mask, comm.all_reduce)
     full = torch.empty(n, cfg.vocab_size)
     comm.all_gather_columns(logits.contiguous(), full)
-    q.put((rank, logits, full.argmax(-1)))
+    q.put((rank, logits.numpy(), full.argmax(-1).numpy()))           # by value: a tensor's storage is fetched from its process, which may have ended
     dist.barrier()
     dist.destroy_process_group()
 
@@ -123,7 +123,7 @@ def test_tp_forward_gloo_world2():
     procs = [ctx.Process(target=_tp_worker, args=(r, world, port, q)) for r in range(world)]
     for p in procs:
         p.start()
-    got = sorted((q.get(timeout=120) for _ in range(world)), key=lambda t: t[0])
+    got = sorted(((r, torch.from_numpy(a), torch.from_numpy(b)) for r, a, b in (q.get(timeout=120) for _ in range(world))), key=lambda t: t[0])
     for p in procs:
         p.join(timeout=60)
         assert p.exitcode == 0

@@ -1,0 +1,28 @@
+"""Streaming products at the lines between their rings and grids (launch_stream), against a product in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# blocks of 16 rows around 256, 400, 512, 1024 and beyond, K of two chunks of 512 bytes to some dozens, every token tile
+@pytest.mark.parametrize("dtype,K", [(torch.bfloat16, 512), (torch.float16, 768), (torch.bfloat16, 2304), (torch.float32, 384), (torch.float32, 1280)])
+@pytest.mark.parametrize("rows", [4096, 4112, 6400, 6401, 8192, 8200, 16384, 16400, 18432, 24577])
+@pytest.mark.parametrize("T,gated", [(1, False), (8, True), (9, False), (16, True), (17, True), (32, False)])
+def test_rings(dtype, K, rows, T, gated):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(rows + K + T)
+    N = 2 * rows if gated else rows
+    x, w = torch.randn(T, K, generator=g, device="cuda").to(dtype), (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(dtype)
+    bias = torch.randn(N, generator=g, device="cuda").to(dtype)
+    out = torch.full((T + 1, rows), 7.0, dtype=dtype if gated else torch.float32, device="cuda")
+    _lib.seq_call("umb_seq_linear", out, x, w, bias, T, N, K, 2 if gated else 0, _lib.seq_dtype_code(dtype))
+    want = x.double() @ w.double().T + bias.double()
+    size = x.double().abs() @ w.double().abs().T + bias.double().abs()                     # what a sum's rounding goes with
+    bound = 2.0 ** -24 * (K / 8 + 16) * size
+    if gated:
+        gate, up = want[:, :rows], want[:, rows:]
+        want = torch.nn.functional.silu(gate) * up
+        bound = 1.1 * bound[:, :rows] * up.abs() + bound[:, rows:] * gate.abs() + {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -21}[dtype] * want.abs() + 1e-7
+    assert bool((out[T] == 7.0).all())
+    assert bool(((out[:T].double() - want).abs() <= bound).all())

@@ -71,6 +71,29 @@ int umb_seq_tile_mix(int T, int rows, int K);
 int umb_seq_linear_parts(float* out, const void* x, const void* w, const void* bias, int T, int N, int K, int parts, int dtype,
                          umb_stream_t stream);
 
+/* A few rows' seam inside the product that reads them: x_out [T][W] (another buffer than f->x) and out = the product of umb_seq_linear's form with the rows
+ * h that the seam leaves, K = W:
+ *   UMB_FRONT_SEAM    umb_seq_resid_norm_parts (x, y in `parts` slabs, w_post, w_next, groups)
+ *   UMB_FRONT_STREAM  umb_hc_seam_parts of one stream (x, y, mix, out, m, in, w_next, offset)
+ *   UMB_FRONT_PAIR    umb_seq_pair_resid_norm_parts (x, y, y2, w1, w2, coef, w_post, w_next)
+ *   UMB_FRONT_EMBED   umb_seq_embed_norm, or umb_hc_embed of one stream (tokens, embed, scale, in, w_next, offset, groups)
+ * The bits are those of the two launches.  epi as umb_seq_linear, 5 (limit, alpha: umb_seq_linear_glu) or 8 (limit: umb_seq_linear_cap).
+ * umb_seq_front_ok: whether the launch covers them (up to 16 rows of some 4096 elements together, W % 8 == 0; no stream); else UMB_EINVAL. */
+enum { UMB_FRONT_SEAM = 0, UMB_FRONT_STREAM = 1, UMB_FRONT_PAIR = 2, UMB_FRONT_EMBED = 3 };
+typedef struct UmbSeqFront {
+  int32_t kind, W, groups, V;
+  int32_t parts, parts2;
+  const float *x, *y, *y2;
+  const void *w_post, *w_next, *w1, *w2, *embed;
+  const int32_t* tokens;
+  const float *mix, *out, *in;
+  float coef, m, offset, scale, eps;
+  int32_t pad_;
+} UmbSeqFront;
+int umb_seq_front_ok(const UmbSeqFront* f, const void* w, int T, int N, int epi, int dtype);
+int umb_seq_front_linear(void* out, float* x_out, const UmbSeqFront* f, const void* w, const void* bias, int T, int N, int epi, float limit, float alpha,
+                         int dtype, umb_stream_t stream);
+
 /* The same product for `batch` independent problems (blockIdx.z): problem b reads x + b sx (rows ldx apart), weights
  * w + b sw ([N][K]) and writes out + b so (rows ldo apart); strides in elements; no bias.  epi 0 / 1 as above;
  * epi 3: out in `dtype` = acc * sigmoid(gate[t ldg + b sg + n]) (gate fp32); epi 7: the same with ONE gate per row and problem,

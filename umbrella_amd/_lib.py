@@ -284,6 +284,13 @@ class UmbSeqStep(C.Structure):
                 ("trace", C.c_void_p)]
 
 
+class UmbSeqFront(C.Structure):
+    _fields_ = [(n, C.c_int32) for n in ("kind", "W", "groups", "V", "parts", "parts2")] + \
+        [(n, C.c_void_p) for n in ("x", "y", "y2", "w_post", "w_next", "w1", "w2", "embed", "tokens", "mix", "out", "in_")] + \
+        [(n, C.c_float) for n in ("coef", "m", "offset", "scale", "eps")] + [("pad_", C.c_int32)]
+
+
+FRONT_SEAM, FRONT_STREAM, FRONT_PAIR, FRONT_EMBED = range(4)
 _PKV = C.POINTER(UmbPagedKV)
 _FORM = C.POINTER(UmbAttnForm)
 SEQ_SIGNATURES = {
@@ -291,6 +298,8 @@ SEQ_SIGNATURES = {
     "umb_seq_linear_split": [_P, _P, _I, _I, _I, _I],
     "umb_seq_tile_kind": [_I, _I, _I, _I], "umb_seq_tile_mix": [_I, _I, _I],
     "umb_seq_linear_parts": [_P, _P, _P, _P, _I, _I, _I, _I, _I],
+    "umb_seq_front_ok": [C.POINTER(UmbSeqFront), _P, _I, _I, _I, _I],
+    "umb_seq_front_linear": [_P, _P, C.POINTER(UmbSeqFront), _P, _P, _I, _I, _I, _F, _F, _I],
     "umb_seq_resid_norm_parts": [_P, _P, _P, _I, _P, _P, _I, _I, _I, _F, _I],
     "umb_seq_pair_resid_norm_parts": [_P, _P, _P, _I, _P, _I, _P, _P, _F, _P, _P, _I, _I, _F, _I],
     "umb_hc_seam_parts": [_P, _P, _P, _I, _P, _P, _F, _P, _P, _F, _I, _I, _I, _F, _I],
@@ -380,7 +389,7 @@ SEQ_SIGNATURES = {
     "umb_sample_rows": [_P, _P, _I, _I, _P, _P, _F, _F, _I, _F, _P, _I, _P, _P],
     "umb_seq_version": [],
 }
-_SEQ_NO_STREAM = {"umb_lat_attend_tiled_ok", "umb_seq_linear_split", "umb_seq_tile_kind", "umb_seq_tile_mix", "umb_lin_scan_columns", "umb_seq_resid_canon_step_ok", "umb_bsa_attend_tiled_ok", "umb_mingru_scratch_floats",
+_SEQ_NO_STREAM = {"umb_lat_attend_tiled_ok", "umb_seq_front_ok", "umb_seq_linear_split", "umb_seq_tile_kind", "umb_seq_tile_mix", "umb_lin_scan_columns", "umb_seq_resid_canon_step_ok", "umb_bsa_attend_tiled_ok", "umb_mingru_scratch_floats",
                   "umb_ssd_scan_chunked_floats", "umb_delta_scan_floats", "umb_gla_scan_chunked_floats"}          # predicates: no stream argument, the value is the answer
 _seq_lib = None
 

@@ -103,6 +103,20 @@ template <int NE, typename Off> __device__ __forceinline__ void add_parts(f32x4 
 }
 __device__ __forceinline__ float sq4(f32x4 v) { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3]; }
 
+// One residual stream's write, mx x + ot (m y), in the order of roundings that few rows have in every kernel
+__device__ __forceinline__ f32x4 stream_write(float mx, f32x4 x, float ot, float m, f32x4 y) {
+  f32x4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = fmaf(ot, m * y[e], mx * x[e]);
+  return r;
+}
+// and of two outputs side by side, a fa wa + b fb wb
+__device__ __forceinline__ f32x4 pair_sum(f32x4 a, float fa, f32x4 wa, f32x4 b, float fb, f32x4 wb) {
+  f32x4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = fmaf(b[e] * fb, wb[e], a[e] * fa * wa[e]);
+  return r;
+}
 // block_sum of a row's squares with the waves' sums added in pairs: with 16 of them one after the other the scale of a row of 4096 was off by
 // 0.795 x 2^-24 in the mean (root mean square), in pairs by 0.698 -- as good as four waves with more elements each
 template <int NT> __device__ __forceinline__ float row_sum(float v, float* red /* >= NT / 64 floats of LDS */) {

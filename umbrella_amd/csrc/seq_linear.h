@@ -1,4 +1,4 @@
-// What the few-token products share: fragments, epilogues, the pieces of
+// What the few-token products share (seq_linear.hip, and seq_front.hip where a norm stands in front of them): fragments, epilogues, the pieces of
 // the streaming kernels and where those pay.
 #pragma once
 #include "gemm_tile.h"

@@ -535,35 +535,124 @@ static int forward_parallel_blocks(const UmbSeqModel* m, const UmbSeqWork* ws, c
   return UMB_OK;
 }
 
-extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const UmbSeqStep* s, hipStream_t st) {
-  if (!m || !ws || !s || m->L < 1 || !m->layers || s->T < 1 || s->T > ws->Tmax || s->B < 1 || s->R < 0 || s->R > ws->Rmax || (s->R > 0 && !m->final_norm))
+// A seam that has not run: what it needs, until the sublayer in front of it asks for its input.  A product of few rows takes the seam along
+// (seq_front.hip; its residual goes to the other of two buffers, x and spare); anything else has it run in place first.
+struct Pending {
+  UmbSeqFront f;
+  bool on = false;
+  float* spare = nullptr;
+};
+static int run_seam(const UmbSeqModel* m, const UmbSeqWork* ws, const UmbSeqStep* s, Pending& p, hipStream_t st) {
+  if (!p.on) return UMB_OK;
+  p.on = false;
+  const UmbSeqFront& f = p.f;
+  const int T = s->T, W = m->W, dt = m->dtype;
+  float *y = const_cast<float*>(f.y), *y2 = const_cast<float*>(f.y2);
+  switch (f.kind) {
+    case UMB_FRONT_SEAM: return umb_seq_resid_norm_parts(ws->x, ws->h, y, f.parts, f.w_post, f.w_next, T, W, f.groups, f.eps, dt, st);
+    case UMB_FRONT_STREAM:
+      return umb_hc_seam_parts(ws->x, ws->h, y, f.parts, f.mix, f.out, f.m, f.in, f.w_next, f.offset, T, W, m->streams, f.eps, dt, st);
+    case UMB_FRONT_PAIR:
+      return umb_seq_pair_resid_norm_parts(ws->x, ws->h, y, f.parts, y2, f.parts2, f.w1, f.w2, f.coef, f.w_post, f.w_next, T, W, f.eps, dt, st);
+    default:
+      if (m->streams >= 1) return umb_hc_embed(ws->x, ws->h, f.embed, f.tokens, f.scale, f.in, f.w_next, f.offset, T, W, f.V, m->streams, f.eps, dt, st);
+      return umb_seq_embed_norm(ws->x, ws->h, f.embed, f.tokens, f.scale, f.w_next, T, W, f.V, f.groups, f.eps, dt, st);
+  }
+}
+// the product l of T rows with the seam in front of it: *done, and the residual's buffers have changed places; otherwise the seam has run
+static int front_product(const UmbSeqModel* m, UmbSeqWork* ws, const UmbSeqStep* s, Pending& p, const UmbSeqLinear& l, void* out, int epi, float limit, float alpha,
+                         bool* done, hipStream_t st) {
+  *done = false;
+  if (!p.on) return UMB_OK;
+  p.f.x = ws->x;
+  if (!p.spare || l.K != m->W || !umb_seq_front_ok(&p.f, l.w, s->T, l.N, epi, m->dtype)) return run_seam(m, ws, s, p, st);
+  p.on = false;
+  SEQ_TRY(umb_seq_front_linear(out, p.spare, &p.f, l.w, l.bias, s->T, l.N, epi, limit, alpha, m->dtype, st));
+  float* const x = ws->x;
+  ws->x = p.spare;
+  p.spare = x;
+  *done = true;
+  return UMB_OK;
+}
+
+extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* given, const UmbSeqStep* s, hipStream_t st) {
+  if (!m || !given || !s || m->L < 1 || !m->layers || s->T < 1 || s->T > given->Tmax || s->B < 1 || s->R < 0 || s->R > given->Rmax ||
+      (s->R > 0 && !m->final_norm))
     return UMB_EINVAL;
-  if (m->block == UMB_BLOCK_PARALLEL) return forward_parallel_blocks(m, ws, s, st);
+  if (m->block == UMB_BLOCK_PARALLEL) return forward_parallel_blocks(m, given, s, st);
   const int T = s->T, W = m->W, dt = m->dtype, groups = m->groups;
   const float eps = m->eps;
   const bool hyper = m->streams >= 1;          // several residual streams: norms in front only, stream seams
   const int S = m->streams;
+  UmbSeqWork work = *given;                    // (its residual rows are where the last seam left them)
+  UmbSeqWork* const ws = &work;
+  Pending pend;
+  if (S <= 1 && !s->trace && T <= given->Tmax / 2) pend.spare = given->x + (size_t)T * W;
   // Every row's logits are wanted, in order (single tokens, scored texts): the last seam norms them for the head, which a launch of its own did in 5 us and
   // more.  (Of several streams the head reads the sum: not a seam's output.)
   const bool whole = s->R == T && !s->logit_rows && (!hyper || S == 1);
   auto next_norm = [&](int l) { return l < m->L ? first_norm_of(m, l) : whole ? m->final_norm : nullptr; };
-  if (hyper) {
-    if (!m->layers[0].norm1) return UMB_EINVAL;
-    SEQ_TRY(umb_hc_embed(ws->x, ws->h, m->embed, s->tokens, m->embed_scale, m->layers[0].hc1_in, m->layers[0].norm1,
-                         m->norm_offset, T, W, m->V, S, eps, dt, st));
-  } else if (m->layers[0].norm1)
-    SEQ_TRY(umb_seq_embed_norm(ws->x, ws->h, m->embed, s->tokens, m->embed_scale, m->layers[0].norm1, T, W, m->V, groups, eps, dt, st));
-  else
+  auto front = [&](int kind, const void* w_next) -> UmbSeqFront& {
+    pend.on = true;
+    pend.f = UmbSeqFront{};
+    pend.f.kind = kind;
+    pend.f.W = W;
+    pend.f.groups = hyper ? 1 : groups;
+    pend.f.V = m->V;
+    pend.f.w_next = w_next;
+    pend.f.eps = eps;
+    return pend.f;
+  };
+  if (hyper && !m->layers[0].norm1) return UMB_EINVAL;
+  if (m->layers[0].norm1) {
+    UmbSeqFront& f = front(UMB_FRONT_EMBED, m->layers[0].norm1);
+    f.embed = m->embed;
+    f.tokens = s->tokens;
+    f.scale = m->embed_scale;
+    if (hyper) {
+      f.in = m->layers[0].hc1_in;
+      f.offset = m->norm_offset;
+    }
+  } else
     SEQ_TRY(umb_seq_embed(ws->x, m->embed, s->tokens, m->embed_scale, T, W, m->V, dt, st));
-  bool h_ready = false;
+  bool h_ready = false, done = false;
   int parts = 1, parts2 = 1;
   // where the slabs of the sublayer's output are counted; a next sublayer that reads through a convolution takes whole sums (its seam's kernel)
   auto slabs = [&](const void* w_next, const void* canon) { parts = 1; return !hyper && !w_next && canon ? nullptr : &parts; };
+  // the seam behind a sublayer: kept for the product that reads it, or run where none does
+  auto stream_seam = [&](const float* mix, const float* out, const float* in, const void* w_next) -> int {
+    UmbSeqFront& f = front(UMB_FRONT_STREAM, w_next);
+    f.y = ws->y;
+    f.parts = parts;
+    f.mix = mix;
+    f.out = out;
+    f.in = in;
+    f.m = m->resid_mult;
+    f.offset = m->norm_offset;
+    return w_next ? UMB_OK : run_seam(m, ws, s, pend, st);
+  };
+  auto plain_seam = [&](const void* w_post, const void* w_next, const void* next_canon, float* next_state) -> int {
+    if (!w_next) return seam(m, ws, s, parts, w_post, w_next, next_canon, next_state, &h_ready, st);
+    UmbSeqFront& f = front(UMB_FRONT_SEAM, w_next);
+    f.y = ws->y;
+    f.parts = parts;
+    f.w_post = w_post;
+    h_ready = false;
+    return UMB_OK;
+  };
+  auto ff = [&](const UmbSeqLayer& ly, int* p) -> int {
+    const int epi = ly.act_kind == UMB_ACT_CLAMP_GLU ? 5 : act_epi(ly.act_kind);
+    if (ly.ff_kind == UMB_FF_GATED) SEQ_TRY(front_product(m, ws, s, pend, ly.gu, ws->act, epi, ly.act_limit, ly.act_alpha, &done, st));
+    else SEQ_TRY(run_seam(m, ws, s, pend, st));
+    if (ly.ff_kind == UMB_FF_GATED && done) return lin_y(ly.down, ws->y, ws, ws->act, T, p, dt, st);
+    return feed_forward(m, ly, ws, s, ws->h, ws->y, p, st);
+  };
   for (int l = 0; l < m->L; ++l) {
     const UmbSeqLayer& ly = m->layers[l];
     const UmbSeqLayer* nl = l + 1 < m->L ? &m->layers[l + 1] : nullptr;
     if (!hyper) SEQ_TRY(sublayer_input(m, ws, s, ly.norm1, ly.canon1, ly.canon_state1, h_ready, st));
-    SEQ_TRY(lin(ly.proj, ws->proj, ws->h, T, 0, dt, st));
+    SEQ_TRY(front_product(m, ws, s, pend, ly.proj, ws->proj, 0, 0.f, 0.f, &done, st));
+    if (!done) SEQ_TRY(lin(ly.proj, ws->proj, ws->h, T, 0, dt, st));
     SEQ_TRY(run_mixer(m, ly, ws, s, st));
     SEQ_TRY(lin_y(ly.out, ws->y, ws, ws->mix, T, ly.has_mlp ? slabs(ly.norm2, ly.canon2) : slabs(next_norm(l + 1), nl ? nl->canon1 : nullptr), dt, st));
     if (hyper) {
@@ -571,33 +660,42 @@ extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const
       const float* in2 = ly.has_mlp ? ly.hc2_in : (nl ? nl->hc1_in : nullptr);
       const void* w2 = ly.has_mlp ? ly.norm2 : (nl ? nl->norm1 : next_norm(l + 1));
       if ((ly.has_mlp || nl) && !w2) return UMB_EINVAL;
-      SEQ_TRY(umb_hc_seam_parts(ws->x, ws->h, ws->y, parts, ly.hc1_mix, ly.hc1_out, m->resid_mult, in2, w2, m->norm_offset, T, W, S, eps, dt, st));
+      SEQ_TRY(stream_seam(ly.hc1_mix, ly.hc1_out, in2, w2));
       if (ly.has_mlp) {
-        SEQ_TRY(feed_forward(m, ly, ws, s, ws->h, ws->y, &parts, st));
+        SEQ_TRY(ff(ly, &parts));
         if (nl && !nl->norm1) return UMB_EINVAL;
-        SEQ_TRY(umb_hc_seam_parts(ws->x, ws->h, ws->y, parts, ly.hc2_mix, ly.hc2_out, m->resid_mult, nl ? nl->hc1_in : nullptr,
-                                  nl ? nl->norm1 : next_norm(l + 1), m->norm_offset, T, W, S, eps, dt, st));
+        SEQ_TRY(stream_seam(ly.hc2_mix, ly.hc2_out, nl ? nl->hc1_in : nullptr, nl ? nl->norm1 : next_norm(l + 1)));
       }
-      if (s->trace) SEQ_TRY(umb_hc_read(s->trace + (long)l * T * W, nullptr, ws->x, nullptr, nullptr, nullptr, 0.f, T, W, S, eps, dt, st));
+      if (s->trace) {
+        SEQ_TRY(run_seam(m, ws, s, pend, st));
+        SEQ_TRY(umb_hc_read(s->trace + (long)l * T * W, nullptr, ws->x, nullptr, nullptr, nullptr, 0.f, T, W, S, eps, dt, st));
+      }
       continue;
     }
     const void* next = ly.has_mlp ? ly.norm2 : next_norm(l + 1);
     if (ly.kind == UMB_MIX_ATTN_DELTA) {
       const void* right = static_cast<char*>(ws->mix) + mix_right(ly, T) * seq_elem_bytes(dt);
       SEQ_TRY(lin_y(ly.out2, ws->y2, ws, right, T, &parts2, dt, st));
-      SEQ_TRY(umb_seq_pair_resid_norm_parts(ws->x, ws->h, ws->y, parts, ws->y2, parts2, ly.out_norm_a, ly.out_norm_b, ly.pair_coef, ly.norm1b,
-                                            next, T, W, eps, dt, st));
+      UmbSeqFront& f = front(UMB_FRONT_PAIR, next);
+      f.y = ws->y;
+      f.y2 = ws->y2;
+      f.parts = parts;
+      f.parts2 = parts2;
+      f.w1 = ly.out_norm_a;
+      f.w2 = ly.out_norm_b;
+      f.coef = ly.pair_coef;
+      f.w_post = ly.norm1b;
+      if (!next) SEQ_TRY(run_seam(m, ws, s, pend, st));
       h_ready = false;
     } else
-      SEQ_TRY(seam(m, ws, s, parts, ly.norm1b, next, ly.has_mlp ? ly.canon2 : (nl ? nl->canon1 : nullptr),
-  ly.has_mlp ? ly.canon_state2 : (nl ? nl->canon_state1 : nullptr), &h_ready, st));
+      SEQ_TRY(plain_seam(ly.norm1b, next, ly.has_mlp ? ly.canon2 : (nl ? nl->canon1 : nullptr), ly.has_mlp ? ly.canon_state2 : (nl ? nl->canon_state1 : nullptr)));
     if (ly.has_mlp) {
       SEQ_TRY(sublayer_input(m, ws, s, ly.norm2, ly.canon2, ly.canon_state2, h_ready, st));
-      SEQ_TRY(feed_forward(m, ly, ws, s, ws->h, ws->y, slabs(next_norm(l + 1), nl ? nl->canon1 : nullptr), st));
-      SEQ_TRY(seam(m, ws, s, parts, ly.norm2b, next_norm(l + 1), nl ? nl->canon1 : nullptr, nl ? nl->canon_state1 : nullptr,
-                   &h_ready, st));
+      SEQ_TRY(ff(ly, slabs(next_norm(l + 1), nl ? nl->canon1 : nullptr)));
+      SEQ_TRY(plain_seam(ly.norm2b, next_norm(l + 1), nl ? nl->canon1 : nullptr, nl ? nl->canon_state1 : nullptr));
     }
     if (s->trace) {
+      SEQ_TRY(run_seam(m, ws, s, pend, st));
       if (hipMemcpyAsync(s->trace + (long)l * T * W, ws->x, (size_t)T * W * sizeof(float), hipMemcpyDeviceToDevice, st) != hipSuccess)
         return UMB_EHIP;
     }
@@ -605,6 +703,10 @@ extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* ws, const
   if (s->R > 0) {
     // final norm of the wanted rows only (of the sum of the streams, where there are several), then the head
     if (whole) {
+      const bool scaled = m->logit_scale != 0.f && m->logit_scale != 1.f;
+      if (scaled) SEQ_TRY(run_seam(m, ws, s, pend, st));
+      else SEQ_TRY(front_product(m, ws, s, pend, m->head, ws->logits, m->logit_cap > 0.f ? 8 : 0, m->logit_cap, 0.f, &done, st));
+      if (!scaled && done) return UMB_OK;
     } else if (hyper)
       SEQ_TRY(umb_hc_read(nullptr, ws->h, ws->x, s->logit_rows, nullptr, m->final_norm, m->norm_offset, s->R, W, S, eps, dt, st));
     else

@@ -158,7 +158,7 @@ static int dgemm_narrow(int T, int N, int K, int S, double* us) {
 }
 
 // the tile by tile_kind (gemm_tile.h)
-static int dgemm_tile(int T, int N, int K, int S, double* us = nullptr) { return tile_kind(T, N, (K / 64 + S - 1) / S, S, K % (128 * S) == 0, us); }
+static int dgemm_tile(int T, int N, int K, int S, double* us = nullptr) { return tile_kind(T, N, (K / 64 + S - 1) / S, S, K % (128 * S) == 0, us, TILE_KINDS); }
 
 template <typename P>
 static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int S, int epi, const GemmFused& fx, hipStream_t st) {
@@ -184,6 +184,7 @@ static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, i
 #undef MIXED
   }
   switch (kind) {
+    case TILE_288: return dgemm_launch<P, 4, 2, 4, 9, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     case TILE_256: return dgemm_launch<P, 4, 2, 4, 8, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     case TILE_192: return dgemm_launch<P, 4, 2, 4, 6, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);
     case TILE_160: return dgemm_launch<P, 4, 2, 4, 5, 1>(wp, x, ldx, out, T, N, K, S, epi, fx, st);

@@ -41,6 +41,12 @@ __device__ __forceinline__ void tile_dma_once(unsigned voff, const void* sbase, 
                :: "v"(voff), "s"(sbase), "s"(ldsaddr) : "memory", "m0");
 }
 
+// a KiB's lines on their way to L2: a word of every 16 bytes to LDS that nobody reads
+__device__ __forceinline__ void tile_touch(unsigned voff, const void* sbase, unsigned ldsaddr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+               :: "v"(voff), "s"(sbase), "s"(ldsaddr) : "memory", "m0");
+}
+
 template <int WM, int WN, int RA, int RB, int KS> struct TileShape {
   static constexpr int NW = WM * WN;                          // waves of one K group
   static constexpr int BN = 16 * WM * RA, BT = 16 * WN * RB;  // rows of A, tokens of B
@@ -69,9 +75,10 @@ enum { TILE_256 = 0,  //  256   256  1.42
        TILE_96 = 4,   //  256    96  0.73
        TILE_128 = 5,  //  128   128  0.49
        TILE_64K = 6,  //  128    64  0.38   K over two groups of waves
-       TILE_KINDS = 7 };
+       TILE_288 = 7,  //  256   288  2.06   A in fragments, many rounds: 257 tokens of 128256 x 8192 650 -> 565 us (two tiles of 160 before), 288 of x 4096 330 -> 299
+       TILE_KINDS = 8 };
 struct Tile { int bn, bt; double us; };
-constexpr Tile TILES[TILE_KINDS] = {{256, 256, 1.42}, {256, 192, 1.20}, {256, 160, 1.04}, {256, 128, 0.86}, {256, 96, 0.73}, {128, 128, 0.49}, {128, 64, 0.38}};
+constexpr Tile TILES[TILE_KINDS] = {{256, 256, 1.42}, {256, 192, 1.20}, {256, 160, 1.04}, {256, 128, 0.86}, {256, 96, 0.73}, {128, 128, 0.49}, {128, 64, 0.38}, {256, 288, 2.06}};
 // us of a launch: 4, and for each round its stages, 2 in front of them and 14 for 256 x 256 outputs behind them; a last round that is not
 // full takes a little less (its share of the memory path is larger).  rows: of A; stages: of one slab; S: slabs
 static inline double tile_cost(int kind, int T, int rows, int stages, int S) {
@@ -80,10 +87,10 @@ static inline double tile_cost(int kind, int T, int rows, int stages, int S) {
   const double load = rest / 256.0, products = stages * k.us, out = 2.1e-4 * k.bn * k.bt;
   return 4.0 + (wgs / 256) * (products + out + 2.0) + (rest ? products * (0.8 + 0.2 * load) + out * load + 2.0 : 0.0);
 }
-// the least of them (the K-split one takes an even number of stages)
-static inline int tile_kind(int T, int rows, int stages, int S, bool even, double* us = nullptr) {
+// the least of them (the K-split one takes an even number of stages); kinds: TILE_288 too where A lies in fragments
+static inline int tile_kind(int T, int rows, int stages, int S, bool even, double* us = nullptr, int kinds = TILE_288) {
   int best = 0;
-  for (int i = 1; i < TILE_KINDS; ++i)
+  for (int i = 1; i < kinds; ++i)
     if ((i != TILE_64K || even) && tile_cost(i, T, rows, stages, S) < tile_cost(best, T, rows, stages, S)) best = i;
   if (us) *us = tile_cost(best, T, rows, stages, S);
   return best;
@@ -136,16 +143,29 @@ __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned cha
                                               const unsigned (&voff)[TileShape<WM, WN, RA, RB, KS>::NPW], int nst, int wave, int ks) {
   typedef TileShape<WM, WN, RA, RB, KS> S;
   constexpr int NW = S::NW, NPA = S::NPA, NPW = S::NPW, PA = NPA / NW, PB = NPW - PA, NF = RA + RB, NM = RA * RB, NSA = S::NSA, NSB = S::NSB;
+  // 144 sums a lane: the fragments of two phases are too many beside them, so B's are given up one by one (A's innermost) while the next are read, one
+  // per 2.8 products, and A's offsets stand in scalar registers (59 values spilled without, now 3)
+  constexpr bool SPREAD = RB > 8;
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4, wm = wave / WN, wn = wave % WN;
   const unsigned lds0 = (unsigned)(size_t)(lds_char*)smem + (unsigned)ks * S::RINGS, lds1 = lds0 + NSA * S::SA;
   const int n = nst / KS;                                     // stages of this group
+  unsigned aoff[PA];                                          // fragments: a piece's offset is the wave's, its lanes 16 bytes apart
+#pragma unroll
+  for (int i = 0; i < PA; ++i) aoff[i] = SPREAD && FRAG ? __builtin_amdgcn_readfirstlane(voff[i]) : 0;
   auto issue = [&](int st, unsigned slot, int i) {            // pieces 0 .. PA - 1 are A's; slot: of the ring they go to
     const unsigned p = (unsigned)(wave + NW * i);
     unsigned dst = i < PA ? lds0 + slot + p * 1024u : lds1 + slot + (p - NPA) * 1024u;
     if (!S::EVEN && i == NPW - 1 && wave + NW * i >= NPA + S::NPB) dst = lds0 + S::RINGS;
     const long s = (long)min(st, n - 1) * KS + ks;
-    if (i < PA) tile_dma(voff[i], static_cast<const char*>(abase) + s * astep, dst);
+    if (SPREAD && FRAG && i < PA) tile_dma((unsigned)lane * 16u, static_cast<const char*>(abase) + s * astep + aoff[i], dst);
+    else if (i < PA) tile_dma(voff[i], static_cast<const char*>(abase) + s * astep, dst);
     else tile_dma(voff[i], static_cast<const char*>(bbase) + s * 128, dst);
+  };
+  // Two slots leave a piece of A less than a stage, and it may come from memory: its lines are asked for a stage and a half earlier (30 us of the 565)
+  constexpr bool TOUCH = SPREAD && FRAG;
+  static_assert(!TOUCH || !S::EVEN, "a KiB of nobody's");
+  auto touch = [&](int st, int i) {
+    tile_touch((unsigned)lane * 16u, static_cast<const char*>(abase) + ((long)min(st, n - 1) * KS + ks) * astep + aoff[i], lds0 + S::RINGS);
   };
   // fragment (16 rows, 32 k) of two row pieces: lane (j, g) reads row j, 16-byte column 4 kh + g
   unsigned foff[2];
@@ -158,7 +178,10 @@ __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned cha
   u32x4 fa[2][RA], fb[2][RB];
   auto read = [&](unsigned sa, unsigned sb, int kh, int i) {  // the i-th fragment of a phase, in the order the products want them
     const unsigned ao = lds0 + sa + (FRAG ? (unsigned)(kh * 1024 + lane * 16) : foff[kh]), bo = lds1 + sb + foff[kh];
-    if (i == 0) fa[kh][0] = *reinterpret_cast<const lds_u32x4*>((size_t)(ao + (unsigned)(wm * RA) * 2048u));
+    if (SPREAD) {
+      if (i < RA) fa[kh][i] = *reinterpret_cast<const lds_u32x4*>((size_t)(ao + (unsigned)(wm * RA + i) * 2048u));
+      else fb[kh][i - RA] = *reinterpret_cast<const lds_u32x4*>((size_t)(bo + (unsigned)(wn * RB + i - RA) * 2048u));
+    } else if (i == 0) fa[kh][0] = *reinterpret_cast<const lds_u32x4*>((size_t)(ao + (unsigned)(wm * RA) * 2048u));
     else if (i <= RB) fb[kh][i - 1] = *reinterpret_cast<const lds_u32x4*>((size_t)(bo + (unsigned)(wn * RB + i - 1) * 2048u));
     else fa[kh][i - RB] = *reinterpret_cast<const lds_u32x4*>((size_t)(ao + (unsigned)(wm * RA + i - RB) * 2048u));
   };
@@ -171,13 +194,17 @@ __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned cha
     static_assert(GAP * (NF - 1) < NM && DG * (NPW - 1) < NM, "every read and every piece has a product to hide behind");
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-      if (READ && m % GAP == 0 && m / GAP < NF) read(KH == 0 ? sa : na, KH == 0 ? sb : nb, KH ^ 1, m / GAP);
+      if constexpr (SPREAD) {
+        if (READ && (m == 0 || m * NF / NM != (m - 1) * NF / NM)) read(KH == 0 ? sa : na, KH == 0 ? sb : nb, KH ^ 1, m * NF / NM);
+      } else if (READ && m % GAP == 0 && m / GAP < NF) read(KH == 0 ? sa : na, KH == 0 ? sb : nb, KH ^ 1, m / GAP);
+      if (TOUCH && KH == 0 && FETCH > 1 && m % (NM / PA) == 1 && m / (NM / PA) < PA) touch(st + NSA + 1, m / (NM / PA));
       if (KH == 1 && m % DG == 0 && m / DG < NPW) {
         const int i = NSA > NSB ? (m / DG < PB ? PA + m / DG : m / DG - PB) : m / DG;            // the shorter ring's pieces first
         if (i >= PA ? FETCH > 0 : FETCH > 1) issue(st + (i < PA ? NSA : NSB), i < PA ? sa : sb, i);
       }
-      acc[m / RB][m % RB] = P::mfma(fa[KH][m / RB], fb[KH][m % RB], acc[m / RB][m % RB]);
-      if ((m + 1) % GAP == 0) __builtin_amdgcn_sched_barrier(0);
+      const int r = SPREAD ? m % RA : m / RB, t = SPREAD ? m / RA : m % RB;
+      acc[r][t] = P::mfma(fa[KH][r], fb[KH][t], acc[r][t]);
+      if (SPREAD || (m + 1) % GAP == 0) __builtin_amdgcn_sched_barrier(0);
     }
   };
   // a stage; LEFT: what may still be on its way when its successor has to be there
@@ -204,7 +231,7 @@ __device__ __forceinline__ bool tile_products(f32x4 (&acc)[RA][RB], unsigned cha
 #pragma unroll
   for (int i = 0; i < NF; ++i) read(0, 0, 0, i);
   int st = 0;
-  for (; st < n - NSA; ++st) stage(std::integral_constant<int, (NSB - 2) * NPW + ALONE>{}, std::integral_constant<int, 2>{}, std::true_type{}, st);
+  for (; st < n - NSA; ++st) stage(std::integral_constant<int, (NSB - 2) * NPW + ALONE + (TOUCH ? PA : 0)>{}, std::integral_constant<int, 2>{}, std::true_type{}, st);
   // the last NSA stages: nothing is asked for that no stage will use
   auto last = [&](auto t_) {
     constexpr int t = decltype(t_)::value, LEFT = (NSB - 2 - t > 0 ? NSB - 2 - t : 0) * NPW + (t == 0 ? ALONE : 0);

@@ -990,7 +990,7 @@ extern "C" int umb_seq_tile_mix(int T, int rows, int K) {
   double us;
   (void)tile_kind(T, rows, K / 64, 1, K % 128 == 0, &us);
   const TileMix mix = tile_mix(T, rows, K / 64, us);
-  return mix.columns * TILE_KINDS + mix.tail;
+  return mix.columns * TILE_288 + mix.tail;              // (TILE_288 is none of this library's)
 }
 
 extern "C" int umb_seq_linear_split(const void* x, const void* w, int T, int N, int K, int dtype) {

@@ -86,6 +86,82 @@ __device__ __forceinline__ void attn_prep_row(const float* __restrict__ src, con
     put(i, v * temp);
   }
 }
+// The same for the decode kernels (D a multiple of 32), compact because what a launch executes once costs its fetch: a pair of features a lane, the angle
+// worked out once for both, in one place for queries and keys; the operands are asked for together, in front of the norm's sum (of the same order).
+template <typename P, typename Put>
+__device__ __forceinline__ void attn_prep_pairs(const float* __restrict__ src, const AttnPrep& a, const typename El<P>::type* __restrict__ w,
+                                                const float* __restrict__ freq, int p, float temp, Put put) {
+  const int lane = threadIdx.x & 63, half = a.rot_dims >> 1, pairs = a.D >> 1;
+  int i0, i1;
+  float u, v, wu, wv, fr;
+  auto get = [&](int m) __attribute__((always_inline)) {
+    m = min(m, pairs - 1);
+    const bool split = a.layout == 0 && m < half;
+    i0 = split ? m : 2 * m;                                  // layout 0: pairs behind the turned ones stand at rot_dims + 2 (m - half) = 2 m too
+    i1 = split ? m + half : 2 * m + 1;
+    u = src[i0];
+    v = src[i1];
+    wu = w ? ldf<P>(w + i0) : 1.f;
+    wv = w ? ldf<P>(w + i1) : 1.f;
+    fr = m < half ? freq[m] : 0.f;
+  };
+  get(lane);
+  float f = 1.f;
+  if (a.norm_qk) {
+    float ss = 0.f;
+#pragma unroll 1
+    for (int i = lane; i < a.D; i += 128) {
+      const float x = src[i], y = i + 64 < a.D ? src[i + 64] : 0.f;
+      ss += x * x;
+      ss += y * y;
+    }
+    f = 1.f / sqrtf(wave_sum(ss) / (float)a.D + a.eps);
+  }
+#pragma unroll 1
+  for (int b = 0;;) {
+    const int m = b + lane;
+    float x = u * f * wu, y = v * f * wv;
+    if (m < half) {
+      float sn, cs;
+      sincosf((float)p * fr, &sn, &cs);
+      sn *= a.rot_mult;
+      cs *= a.rot_mult;
+      const float rx = x * cs - y * sn, ry = y * cs + x * sn;
+      x = rx;
+      y = ry;
+    }
+    if (m < pairs) {
+      put(i0, x * temp);
+      put(i1, y * temp);
+    }
+    b += 64;
+    if (b >= pairs) break;
+    get(b + lane);
+  }
+}
+template <int NC, typename Put>
+__device__ __forceinline__ void attn_prep_value_few(const float* __restrict__ src, const AttnPrep& a, long o, bool keep, Put put) {
+  const int lane = threadIdx.x & 63;
+  float v[NC], m[NC], f = 1.f;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    v[c] = src[lane + 64 * c];
+    m[c] = a.mix.first ? a.mix.first[o + lane + 64 * c] : 0.f;
+  }
+  if (a.norm_v) {
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) ss += v[c] * v[c];
+    f = 1.f / sqrtf(wave_sum(ss) / (float)(64 * NC) + a.eps);
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    float x = v[c] * f;
+    if (keep && a.mix.keep) a.mix.keep[o + lane + 64 * c] = x;
+    if (a.mix.first) x = (1.f - a.mix.lambda) * x + a.mix.lambda * m[c];
+    put(lane + 64 * c, x);
+  }
+}
 __device__ __forceinline__ float attn_temp(const AttnPrep& a, int p) { return a.temp_every > 0 ? 1.f + a.temp_coef * logf((float)((p + 1) / a.temp_every + 1)) : 1.f; }
 
 template <typename P>
@@ -258,6 +334,7 @@ __device__ __forceinline__ void attn_finish(typename El<P>::type* __restrict__ o
     for (int x = threadIdx.x; x < RH * per; x += nw * 64) {
       const int r = x / per, d = x % per * 4;
       f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
       for (int w = 0; w < nact; ++w) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(o_s + (w * RH + r) * Ep + d);
         const float f = ml_s[(w * RH + r) * 2];
@@ -289,12 +366,24 @@ __device__ __forceinline__ void attn_finish(typename El<P>::type* __restrict__ o
   } else {
     // a wave per head: o = a1 - lambda a2 over its root mean square
     for (int rr = threadIdx.x >> 6; rr < RR; rr += nw) {
-      float v[NC], ss = 0.f;
+      float v[NC], u[NC], ss = 0.f;
       const float L1 = denominator(MAPS * rr), L2 = denominator(MAPS * rr + MAPS - 1);
 #pragma unroll
+      for (int c = 0; c < NC; ++c) v[c] = u[c] = 0.f;
+#pragma unroll 1
+      for (int w = 0; w < nact; ++w) {                       // all columns of both maps side by side
+        const int r1 = w * RH + MAPS * rr, r2 = r1 + MAPS - 1;
+        const float f1 = ml_s[r1 * 2], f2 = ml_s[r2 * 2];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const int d = min(lane + 64 * c, E - 1);
+          v[c] += o_s[r1 * Ep + d] * f1;
+          u[c] += o_s[r2 * Ep + d] * f2;
+        }
+      }
+#pragma unroll
       for (int c = 0; c < NC; ++c) {
-        const int d = min(lane + 64 * c, E - 1);
-        const float o = merged(MAPS * rr, d) / L1 - form.lambda * (merged(MAPS * rr + MAPS - 1, d) / L2);
+        const float o = v[c] / L1 - form.lambda * (u[c] / L2);
         v[c] = o;
         if (lane + 64 * c < E) ss += o * o;
       }
@@ -470,6 +559,9 @@ constexpr int ATT_SPAN = 256, LAT_SPAN = 64;
 // PREP: steps of one token a sequence.  The queries come from the projection and the token's key and value with them (attn_prep above, which a launch of
 // its own did in 4 - 5 us): the key and value stand in LDS for this workgroup, whose last round takes them from there -- what the cache holds at the token's
 // position is not there yet -- and the group's first workgroup appends them.
+// A launch is latency, a fifth of it the fetch of code that is executed once: one place for queries and keys, an angle a pair, loops not unrolled where a
+// round is enough; and the first round's rows asked for in front of the preparation (us a launch inside a step, 20 / 16 KB of code: one token, two maps of
+// 128 | 256 10.3 / 7.9, sink heads of 128 8.0 / 7.1; 48 tokens, heads of 64 10.1 / 9.2).
 struct DecodePrep { AttnPrep a; const void *w_q, *w_k; const float* freq; };
 template <typename P, int RH, int LPR, int NW, int MAPS, bool LAT = false, bool PREP = false>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q, UmbPagedKV kv,
@@ -500,25 +592,44 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
   unsigned row = 0;
   if (wave < nact) row = pkv_tok_row(kv, slot, key_pos(min(base + j, keys.n - 1)), g, G);
   typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
+  // The first round's rows are on their way while the token's own are prepared, which is as long as their trip: a lane asks for one word of each, its
+  // quarter's (all lines of a row up to 512 bytes), and the round finds them near.  Held in registers instead they cost the kernel of four rows a wave a SIMD
+  unsigned near_k = 0, near_v = 0;
+  float bv[RR];
+  auto biases = [&]() {
+    const int dist = i - key_pos(min(base + j, keys.n - 1)), bi = dist < n_dist ? dist : n_dist - 1;
+#pragma unroll
+    for (int r = 0; r < RR; ++r) bv[r] = bias ? bias[(long)(h0 + r) * n_dist + bi] : 0.f;
+  };
+  if (wave < nact) {
+    near_k = *reinterpret_cast<const unsigned*>(reinterpret_cast<const u16*>(kv.k) + (long)row * (MAPS * D) + quarter * (MAPS * D / 4));
+    if (!LAT) near_v = *reinterpret_cast<const unsigned*>(reinterpret_cast<const u16*>(kv.v) + (long)row * E + quarter * (E / 4));
+    biases();
+  }
   if constexpr (PREP) {
     const AttnPrep& a = prep.a;
     const float* src = proj + (long)t * ld;
     const bool append = split == 0 && h0 % (H / G) == 0;
     const float temp = attn_temp(a, i);
+#pragma unroll 1
     for (int task = wave; task < RH + (a.GK ? MAPS + 1 : 0); task += NW) {       // a row a wave
-      if (task < RH)
-        attn_prep_row<P>(src + (h0 * MAPS + task) * D, a, reinterpret_cast<const u16*>(prep.w_q), prep.freq, i, temp, [&](int x, float v) { q_s[task * D + x] = v; });
-      else if (task < RH + MAPS) {
+      if (task < RH + MAPS) {
+        const bool is_q = task < RH;
         const int mp = task - RH;
-        u16* row_k = reinterpret_cast<u16*>(kv.k) + pkv_tok(kv, slot, i, g, G, MAPS * D) + mp * D;
-        attn_prep_row<P>(src + (a.HQ + g * MAPS + mp) * D, a, reinterpret_cast<const u16*>(prep.w_k), prep.freq, i, 1.f, [&](int x, float v) {
+        u16* row_k = is_q ? nullptr : reinterpret_cast<u16*>(kv.k) + pkv_tok(kv, slot, i, g, G, MAPS * D) + mp * D;
+        attn_prep_pairs<P>(src + (is_q ? h0 * MAPS + task : a.HQ + g * MAPS + mp) * D, a, reinterpret_cast<const u16*>(is_q ? prep.w_q : prep.w_k), prep.freq, i,
+                           is_q ? temp : 1.f, [&](int x, float v) {
+          if (is_q) {
+            q_s[task * D + x] = v;
+            return;
+          }
           const u16 b = P::from_f(v);
           new_k[mp * D + x] = b;
           if (append) row_k[x] = b;
         });
       } else {
         u16* row_v = reinterpret_cast<u16*>(kv.v) + pkv_tok(kv, slot, i, g, G, E);
-        attn_prep_value(src + (a.HQ + a.GK) * D + g * E, a, ((long)t * G + g) * E, append, [&](int x, float v) {
+        attn_prep_value_few<(E + 63) / 64>(src + (a.HQ + a.GK) * D + g * E, a, ((long)t * G + g) * E, append, [&](int x, float v) {
           const u16 b = P::from_f(v);
           new_v[x] = b;
           if (append) row_v[x] = b;
@@ -550,11 +661,6 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
           if (base + KPI * u + lane / LPR >= keys.n - 1) vv[u] = *reinterpret_cast<const u32x4*>(new_v + (lane & (LPR - 1)) * 8);
       }
       const u16* kr = reinterpret_cast<const u16*>(kv.k) + (long)row * (MAPS * D) + quarter * 8;
-      const int dist = i - key_pos(min(kx, keys.n - 1));
-      float bv[RR];
-      const int bi = dist < n_dist ? dist : n_dist - 1;
-#pragma unroll
-      for (int r = 0; r < RR; ++r) bv[r] = bias ? bias[(long)(h0 + r) * n_dist + bi] : 0.f;
       // the next round of this wave: NW rounds on, or in the next of its workgroup's spans
       int next = base + NW * 16;
       if (nsplit > 1 && next / SPAN != base / SPAN) next += (nsplit - 1) * SPAN;
@@ -563,6 +669,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
       float s[RH];
 #pragma unroll
       for (int r = 0; r < RH; ++r) s[r] = 0.f;
+#pragma unroll 1
       for (int d = 0; d < D; d += 128) {
         u32x4 kk[MAPS][4];
 #pragma unroll
@@ -596,10 +703,14 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
         }
       }
 #pragma unroll
+      for (int r = 0; r < RH; ++r) s[r] = add_rows(s[r]) * scale;
+      if (softcap > 0.f) {
+#pragma unroll
+        for (int r = 0; r < RH; ++r) s[r] = softcap * tanhf(s[r] / softcap);
+      }
+#pragma unroll
       for (int r = 0; r < RH; ++r) {
-        float sc = add_rows(s[r]) * scale;
-        if (softcap > 0.f) sc = softcap * tanhf(sc / softcap);
-        const float sv = kx < keys.n ? sc + bv[r / MAPS] : -INFINITY;
+        const float sv = kx < keys.n ? s[r] + bv[r / MAPS] : -INFINITY;
         const float m_new = fmaxf(m_run[r], row_max16(sv));
         const float m_ref = m_new == -INFINITY ? 0.f : m_new;          // a round of -inf scores alone: weights 0, nothing to rescale
         const float fac = expf(m_run[r] - m_ref);
@@ -622,7 +733,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
       }
       base = next;
       row = next_row;
+      if (base < keys.n) biases();
     }
+    asm volatile("" :: "v"(near_k), "v"(near_v));            // (asked for, whatever they hold)
 #pragma unroll
     for (int r = 0; r < RH; ++r) {
       const float l = row_add16(l_run[r]);

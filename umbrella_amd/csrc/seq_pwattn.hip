@@ -87,6 +87,43 @@ __device__ __forceinline__ void pwa_row(const float* __restrict__ src, int D, in
     if (d1 < D) put(d1, v * f);
   }
 }
+// The same for the decode kernel: D features (a multiple of 32) as NP pairs a lane, asked for together with their frequencies in front of anything that
+// waits, one angle a pair; compact, because what a launch executes once costs its fetch.  put(feature, turned and normed, as projected)
+template <int D, typename Put>
+__device__ __forceinline__ void pwa_row_few(const float* __restrict__ src, int rot_dims, const float* __restrict__ freq, int p, float eps, Put put) {
+  constexpr int NP = (D + 127) / 128;
+  typedef float pair __attribute__((ext_vector_type(2), aligned(4)));
+  const int lane = threadIdx.x & 63;
+  pair raw[NP];
+  float u[NP], v[NP], fr[NP], ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < NP; ++c) {
+    const int m = min(lane + 64 * c, D / 2 - 1);
+    raw[c] = *reinterpret_cast<const pair*>(src + 2 * m);
+    fr[c] = 2 * m + 1 < rot_dims ? freq[m] : 0.f;
+  }
+#pragma unroll
+  for (int c = 0; c < NP; ++c) {
+    const int m = lane + 64 * c;
+    u[c] = raw[c][0];
+    v[c] = raw[c][1];
+    if (2 * m + 1 < rot_dims) {
+      float sn, cs;
+      sincosf((float)p * fr[c], &sn, &cs);
+      const float ru = u[c] * cs - v[c] * sn, rv = v[c] * cs + u[c] * sn;
+      u[c] = ru; v[c] = rv;
+    }
+    if (2 * m < D) ss += u[c] * u[c] + v[c] * v[c];
+  }
+  const float f = 1.f / sqrtf(wave_sum(ss) / (float)D + eps);
+#pragma unroll
+  for (int c = 0; c < NP; ++c) {
+    const int m = lane + 64 * c;
+    if (2 * m >= D) continue;
+    put(2 * m, u[c] * f, raw[c][0]);
+    put(2 * m + 1, v[c] * f, raw[c][1]);
+  }
+}
 // the pooled block that the token at p completes, by a wave: the sums of the cached positions in front of it and its own key and value as they are stored
 template <typename P>
 __device__ __forceinline__ void pool_with(const UmbPagedKV& kv, int slot, const float* __restrict__ src, int g, int G, int D, int rot_dims,
@@ -424,7 +461,8 @@ __global__ __launch_bounds__(NW * 64) void pwa_attend_kernel(typename El<P>::typ
 // Before -> now, replayed from a graph, D 128: one token behind 40 / 2000 keys 10.7 -> 4.9 / 30.8 -> 18.0 us, 48 tokens behind 40 20.9 -> 5.7,
 // 64 behind 1000 77 -> 45.
 // PREP: steps of one token a sequence, as in seq_battn.hip: the queries come from the projection, the token's key and value stand in LDS for the round that
-// needs them, and the group's first workgroup appends them and the block that they complete.
+// needs them, and the group's first workgroup appends them and the block that they complete.  Compact, and the first rows early, as there: 16 tokens, heads of
+// 128, 11.0 -> 10.6 us inside a step.
 struct PwaPrep { const float* freq; int rot_dims; float eps; };
 template <typename P, int RH, int LPR, int NW, bool PREP>
 __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ out, const float* __restrict__ q, UmbPagedKV kv,
@@ -449,19 +487,33 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
   };
   unsigned row = 0;
   if (wave < nact) row = row_of(wave);
+  // the first round's rows are on their way while the token's own are prepared, as in seq_battn.hip
+  unsigned near_k = 0, near_v = 0;
+  if (wave < nact) {
+    const long eb = wave < br ? 4 : 2, at = (long)row * D + quarter * (D / 4);
+    near_k = *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(wave < br ? (const void*)kv.kp : kv.k) + at * eb);
+    near_v = *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(wave < br ? (const void*)kv.vp : kv.v) + at * eb);
+  }
   if constexpr (PREP) {
     const float* src = proj + (long)t * ld;
     const bool append = h0 % (H / G) == 0;
+#pragma unroll 1
     for (int task = wave; task < RH + 2; task += NW) {     // a row a wave
-      if (task < RH)
-        pwa_row(src + (h0 + task) * D, Dr, prep.rot_dims, prep.freq, i, prep.eps, [](int, float) {}, [&](int d, float v) { q_s[task * D + d] = v; });
-      else if (task == RH) {
-        const long off = pkv_tok(kv, slot, i, g, G, D);
+      if (task <= RH) {
+        const bool is_q = task < RH;
+        const long off = is_q ? 0 : pkv_tok(kv, slot, i, g, G, D);
         u16* kd = reinterpret_cast<u16*>(kv.k) + off;
         u16* vd = reinterpret_cast<u16*>(kv.v) + off;
-        pwa_row(src + (H + g) * D, Dr, prep.rot_dims, prep.freq, i, prep.eps,
-                [&](int d, float v) { const u16 b = P::from_f(v); new_v[d] = b; if (append) vd[d] = b; },
-                [&](int d, float v) { const u16 b = P::from_f(v); new_k[d] = b; if (append) kd[d] = b; });
+        pwa_row_few<D>(src + (is_q ? h0 + task : H + g) * D, prep.rot_dims, prep.freq, i, prep.eps, [&](int d, float x, float raw) {
+          if (is_q) {
+            q_s[task * D + d] = x;
+            return;
+          }
+          const u16 kb = P::from_f(x), vb = P::from_f(raw);
+          new_k[d] = kb;
+          new_v[d] = vb;
+          if (append) { kd[d] = kb; vd[d] = vb; }
+        });
       } else if (append && (i + 1) % pool == 0)
         pool_with<P>(kv, slot, src + (H + g) * D, g, G, Dr, prep.rot_dims, prep.freq, i, prep.eps, pool);
     }
@@ -560,6 +612,7 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
         for (int u = 0; u < VL; ++u)
           if (key0 + KPI * u + lane / LPR >= n_tok - 1) vv[u] = *reinterpret_cast<const u32x4*>(new_v + (lane & (LPR - 1)) * 8);
       }
+#pragma unroll 1
       for (int d = 0; d < Dr; d += 128) {
         u32x4 kk[4];
 #pragma unroll
@@ -585,11 +638,13 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
       }
       row = next_row;
     }
+    asm volatile("" :: "v"(near_k), "v"(near_v));            // (asked for, whatever they hold)
     store_groups<RH, LPR>(o_s + wave * RH * D, acc, lane);
   }
   __syncthreads();
   for (int x = threadIdx.x; x < RH * D; x += NW * 64) {
     float o = o_s[x];
+#pragma unroll 4
     for (int w = 1; w < nact; ++w) o += o_s[w * RH * D + x];
     const float gate = 1.f / (1.f + expf(-proj[(long)t * ld + gate_col + h0 + x / D]));
     out[((long)t * H + h0) * D + x] = P::from_f(o * gate);

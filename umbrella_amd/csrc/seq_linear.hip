@@ -823,6 +823,9 @@ static int launch_stream(void* out, const void* x, const void* w, const void* bi
   const long blocks = (long)((N + 15) / 16) * gz, chunks = (long)K * sizeof(typename El<P>::type) / 512;
   // true fp32 of more than 8 tokens stands on its products: as many waves on a unit as before
   constexpr bool F = sizeof(typename El<P>::type) == 4;
+  if constexpr (!F)
+    if (gy == 0 && gz == 1 && ext.parts <= 1 && !ext.tiles && ext.ldx == K && ext.ldo == N && held_pays(T, N, K, epi))
+      return held_stream(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, std::is_same<P, BF16>::value ? UMB_SEQ_BF16 : UMB_SEQ_F16, st);
   if (epi_dual(epi)) {
     // up to some 1.5 blocks a unit they stand side by side: a second one behind the first would leave half of the units idle
     const int held = blocks <= 400 ? 512 : 256;

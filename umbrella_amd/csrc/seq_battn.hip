@@ -194,6 +194,129 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, U
   });
 }
 
+// The same for many items, rows of 64 or 128 whose turned part is whole quads: a wave takes PREP_QUADS quads a lane of one token's neighbouring rows (queries
+// and keys, or values), two or four rows side by side, all loads in flight, and works the angles out once for all of them.
+// Vector work bounded what it replaces (four slots a wave, an element a lane, the angles again for every four: some 250 instructions a slot, quotients and
+// sines among them).  us, that / this, bf16: 2466 tokens, 32 + 8 + 8 slots of 64 33.9 / 16.0 (68 MB, 4.2 TB/s), 1999 tokens, 32 + 8 + 8 of 128 with mixed
+// values 34.8 / 23.2 (98 MB); with a branch between the loads and the sines four times over 18.0 / 25.5.
+constexpr int PREP_QUADS = 4;
+constexpr int prep_rows(int D) { return PREP_QUADS * 256 / D; }      // rows a wave takes
+typedef float quad_u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f32x4 ldq(const float* p) { return *reinterpret_cast<const quad_u*>(p); }
+// 1 / root mean square of a row that D / 4 neighbouring lanes hold
+template <int D> __device__ __forceinline__ float quad_row_scale(f32x4 x, float eps) {
+  float s = row_add16(sq4(x));
+  if constexpr (D == 128) {
+    float b = s;
+    swap16(s, b);
+    s += b;
+  }
+  return 1.f / sqrtf(s / (float)D + eps);
+}
+template <typename P, int D, int E>
+__global__ __launch_bounds__(256) void attn_prep_quads_kernel(float* __restrict__ q, UmbPagedKV kv, const float* __restrict__ proj, int ld,
+                                                              const typename El<P>::type* __restrict__ w_q, const typename El<P>::type* __restrict__ w_k,
+                                                              const int* __restrict__ pos, const int* __restrict__ slot, const float* __restrict__ freq, int T,
+                                                              AttnPrep a, int qk_waves, int waves) {
+  typedef typename El<P>::type El_;
+  const int item = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6))), lane = threadIdx.x & 63;
+  const int t = item / waves, part = item - t * waves;
+  if (t >= T) return;
+  const int p = pos[t], sl = a.GV ? slot[t] : 0;
+  const float* src = proj + (long)t * ld;
+  if (part >= qk_waves) {                                    // values
+    constexpr int ROWS = prep_rows(E);
+    const int sub = lane / (E / 4), e = lane % (E / 4) * 4, first = (part - qk_waves) * ROWS, n = min(ROWS, a.GV - first);
+    const float* vs = src + (a.HQ + a.GK) * D;
+    const long row0 = ((long)t * a.G + first) * E + e, out0 = a.GV ? pkv_tok(kv, sl, p, first, a.G, E) + e : 0;
+    f32x4 v[PREP_QUADS], m[PREP_QUADS];
+#pragma unroll
+    for (int u = 0; u < PREP_QUADS; ++u) {
+      const int r = min(u * (256 / E) + sub, n - 1);
+      v[u] = ldq(vs + (first + r) * E + e);
+    }
+    const float* ms = a.mix.first ? a.mix.first + row0 : vs + first * E + e;      // (no branch between loads: one waits for all of them)
+#pragma unroll
+    for (int u = 0; u < PREP_QUADS; ++u) m[u] = ldq(ms + min(u * (256 / E) + sub, n - 1) * E);
+#pragma unroll
+    for (int u = 0; u < PREP_QUADS; ++u) {
+      const int r = u * (256 / E) + sub;
+      if (a.norm_v) v[u] = v[u] * quad_row_scale<E>(v[u], a.eps);
+      if (r >= n) continue;
+      if (a.mix.keep) *reinterpret_cast<quad_u*>(a.mix.keep + row0 + r * E) = v[u];
+      if (a.mix.first) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[u][i] = (1.f - a.mix.lambda) * v[u][i] + a.mix.lambda * m[u][i];
+      }
+      st4<P>(reinterpret_cast<El_*>(kv.v) + out0 + (long)r * kv.page * E, v[u]);
+    }
+    return;
+  }
+  constexpr int ROWS = prep_rows(D);
+  const int sub = lane / (D / 4), e = lane % (D / 4) * 4, first = part * ROWS, n = min(ROWS, a.HQ + a.GK - first), half = a.rot_dims >> 1;
+  const bool rot = e < a.rot_dims, low = e < half;
+  const int other = a.layout == 0 && rot ? (low ? e + half : e - half) : e;
+  const bool far = a.layout == 0 && a.rot_dims > 0;          // partners in another lane's quad
+  f32x4 x[PREP_QUADS], y[PREP_QUADS];
+#pragma unroll
+  for (int u = 0; u < PREP_QUADS; ++u) {
+    const float* row = src + (first + min(u * (256 / D) + sub, n - 1)) * D;
+    x[u] = ldq(row + e);
+    y[u] = ldq(row + other);                                 // (itself where it is in this lane: no branch between loads, one waits for all of them)
+  }
+  f32x4 cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
+  if (rot) {
+    // a quad's four angles, or two where it holds whole pairs: one place for the sines, the values go round
+    typedef float two __attribute__((ext_vector_type(2), aligned(4)));
+    const int at = a.layout == 0 ? (low ? e : e - half) : e >> 1;
+    const two f0 = *reinterpret_cast<const two*>(freq + at), f1 = *reinterpret_cast<const two*>(freq + (a.layout == 0 ? at + 2 : at));
+    f32x4 fr = {f0[0], f0[1], f1[0], f1[1]};
+#pragma unroll 1
+    for (int i = a.layout == 0 ? 4 : 2; i > 0; --i) {
+      float s, c;
+      sincosf((float)p * fr[0], &s, &c);
+      fr = f32x4{fr[1], fr[2], fr[3], fr[0]};
+      cs = f32x4{cs[1], cs[2], cs[3], c * a.rot_mult};
+      sn = f32x4{sn[1], sn[2], sn[3], s * a.rot_mult};
+    }
+    // x cos - y sin in a pair's first, y cos + x sin in its second
+    if (a.layout == 1) {
+      cs = f32x4{cs[2], cs[2], cs[3], cs[3]};
+      sn = f32x4{-sn[2], sn[2], -sn[3], sn[3]};
+    } else if (low) sn = -sn;
+  }
+  const float temp = attn_temp(a, p);
+  const long k0 = a.GK ? pkv_tok(kv, sl, p, 0, a.G, a.maps * D) : 0, k_group = (long)kv.page * a.maps * D;
+#pragma unroll
+  for (int u = 0; u < PREP_QUADS; ++u) {
+    const int r = u * (256 / D) + sub, hs = first + min(r, n - 1), ks = hs - a.HQ;
+    const bool is_q = ks < 0;
+    if (a.norm_qk) {
+      const float f = quad_row_scale<D>(x[u], a.eps);
+      x[u] = x[u] * f;
+      if (far) y[u] = y[u] * f;
+    }
+    const El_* w = is_q ? w_q : w_k;
+    if (w) {
+      x[u] = x[u] * ld4<P>(w + e);
+      if (far) y[u] = y[u] * ld4<P>(w + other);
+    }
+    if (!far) y[u] = f32x4{x[u][1], x[u][0], x[u][3], x[u][2]};
+    f32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = x[u][i] * cs[i] + y[u][i] * sn[i];
+    if (!rot) o = x[u];
+    if (r >= n) continue;
+    if (is_q) *reinterpret_cast<f32x4*>(q + ((long)t * a.HQ + hs) * D + e) = o * temp;
+    else st4<P>(reinterpret_cast<El_*>(kv.k) + k0 + ks / a.maps * k_group + ks % a.maps * D + e, o);
+  }
+}
+// where it can: whole quads on either side of a pair's distance; weights, queries and cached rows that quads are aligned in
+static inline bool prep_in_quads(const float* q, const UmbPagedKV* kv, const void* w_q, const void* w_k, const AttnPrep& a, int eb) {
+  return (a.D == 64 || a.D == 128) && (a.E == 64 || a.E == 128) && a.rot_dims % (a.layout == 0 ? 8 : 4) == 0 && (uintptr_t)q % 16 == 0 &&
+         ((uintptr_t)w_q | (uintptr_t)w_k) % (4 * eb) == 0 && (!a.GV || ((uintptr_t)kv->k | (uintptr_t)kv->v) % (4 * eb) == 0);
+}
+
 // The same for many items (rows of at most 128): a wave takes four neighbouring slots of one token, the loads of all four in flight, and
 // works the angles out once for them.  A wave per slot was latency times rounds of waves and four times the sines: 1999 tokens of 32 + 16
 // slots of 128 42.5 -> 35.0 us (90 MB, 2.6 TB/s); 2300 tokens, 32 + 16 of 64 34 -> 29.
@@ -839,6 +962,20 @@ extern "C" int umb_attn_prep_mix(float* q, const UmbPagedKV* kv, const float* pr
   const long items = (long)T * (a.HQ + a.GK + a.GV);
   // from three rounds of waves over the chip on (us, a wave each / four: 17600 items of two maps 9.2 / 10.5, 19200 of 64 10.2 / 9.9, 30800 of two maps
   // 13.9 / 13.5, 96000 37.9 / 29.3)
+  if (items >= 24576 && prep_in_quads(q, kv, w_q, w_k, a, dtype == UMB_SEQ_F32 ? 4 : 2)) {
+    const int qk = (a.HQ + a.GK + prep_rows(D) - 1) / prep_rows(D), waves = qk + (a.GV + prep_rows(E) - 1) / prep_rows(E);
+#define QUADS(DD, EE) hipLaunchKernelGGL((attn_prep_quads_kernel<P, DD, EE>), dim3((unsigned)(((long)T * waves + 3) / 4)), dim3(256), 0, st, q, append ? *kv : none, \
+                                         proj, ld, (const typename El<P>::type*)w_q, (const typename El<P>::type*)w_k, pos, slot, freq, T, a, qk, waves)
+    DISPATCH_SEQ_DTYPE(dtype, {
+      if (D == 64 && E == 64) QUADS(64, 64);
+      else if (D == 64) QUADS(64, 128);
+      else if (E == 64) QUADS(128, 64);
+      else QUADS(128, 128);
+    })
+#undef QUADS
+    UMB_LAUNCH_CHECK();
+    return UMB_OK;
+  }
   if (items >= 24576 && D <= 128 && E <= 128) {
     const int groups = (a.HQ + a.GK + a.GV + 3) / 4;
     DISPATCH_SEQ_DTYPE(dtype, {

@@ -19,3 +19,28 @@ def test_attention_slots(dtype, H, G, D, E, maps, layout, rot, append, norm, mix
 @pytest.mark.parametrize("H,G,D,rot", [(15, 1, 64, 32), (16, 8, 128, 128), (20, 4, 64, 0), (17, 1, 128, 60)])
 def test_pooled_slots(dtype, H, G, D, rot):
     prompt.test_many_pooled_slots_are_prepared_as_few_are(dtype, H, G, D, rot)
+
+
+# heads that quads are aligned in, few of them and many, a last wave in part; a normaliser's column behind a head (rows of Dv + 1), weights for all and of each head
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,Dv", [(1, 3, 64), (7, 1, 128), (1, 1, 256), (1800, 11, 64), (2467, 7, 128), (601, 9, 256)])
+@pytest.mark.parametrize("den,weights,kind", [(False, 0, 0), (True, 1, 1), (True, 2, 0)])
+def test_head_gates(dtype, T, H, Dv, den, weights, kind):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + Dv)
+    cols, ld, ldo = Dv + int(den), H * Dv + 5, H * Dv + 4
+    o, proj, mrun = (torch.randn(s, generator=g, device="cuda") for s in ((T, H, cols), (T, ld), (T, H)))
+    w = torch.randn(Dv if weights == 1 else H * Dv, generator=g, device="cuda").to(dtype) if weights else None
+    out = torch.full((T + 1, ldo), 7.0, dtype=dtype, device="cuda")
+    _lib.seq_call("umb_head_gate", out, ldo, o, cols, Dv if den else -1, mrun if den else None, proj, ld, 3, w, int(weights == 2), kind, T, H, Dv, 1e-5, 1.2,
+                  _lib.seq_dtype_code(dtype))
+    v, gate = o[..., :Dv].double(), proj[:, 3:3 + H * Dv].double().view(T, H, Dv)
+    if den:
+        v = v / (torch.maximum(o[..., Dv].double().abs(), torch.exp(-mrun.double())) + 1e-6)[..., None]
+    v = v * 1.2 / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-5)
+    if weights:
+        v = v * (w.double() if weights == 1 else w.double().view(H, Dv))
+    want = (v * torch.sigmoid(gate) * (gate if kind == 0 else 1.0)).view(T, -1)
+    assert bool((out[T] == 7.0).all()) and bool((out[:T, H * Dv:] == 7.0).all())
+    eps = torch.finfo(dtype).eps
+    assert bool(((out[:T, :H * Dv].double() - want).abs() <= 0.51 * eps * want.abs() + 2e-6 * want.abs() + 1e-7).all())

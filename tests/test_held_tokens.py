@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 # second blocks of rows for one workgroup, for most and for all; a last block of one row and of all but one; both ends of the token tiles; both K
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("T,K", [(33, 2048), (48, 2048), (49, 2048), (64, 2048), (33, 4096), (48, 4096)])
+@pytest.mark.parametrize("T,K", [(33, 2048), (48, 2048), (49, 2048), (64, 2048), (33, 4096), (48, 4096), (49, 4096), (64, 4096)])
 @pytest.mark.parametrize("rows,epi", [(4097, 2), (8191, 2), (8200, 0), (16385, 1), (24608, 0), (12300, 2)])
 def test_products(dtype, T, K, rows, epi):
     from umbrella_amd import _lib

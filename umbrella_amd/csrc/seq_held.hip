@@ -5,7 +5,8 @@
 // several blocks of rows keeps what its waves read of the tokens in the first one: K / 4 of each, 192 to 384 registers, which one workgroup a unit leaves
 // to a wave.  From the second block on only weights are fetched, four chunks ahead.
 // us, bf16, cold weights, the streaming kernel / this: 48 tokens 32000 x 2048 31.3 / 26.8 (4.9 TB/s of weights), x 4096 53.7 / 49.4, gate/up 14336 x 4096 52.1 / 43.5,
-// 8192 x 2048 17.0 / 16.7, 5120 x 2048 16.0 / 15.0; 10240 x 2048 16.6 / 15.2; 64 tokens 32000 x 2048 36.8 / 29.4, gate/up 8192 x 2048 19.6 / 18.5.
+// 8192 x 2048 17.0 / 16.7, 5120 x 2048 16.0 / 15.0; 10240 x 2048 16.6 / 15.2; 64 tokens 32000 x 2048 36.8 / 29.4, gate/up 8192 x 2048
+// 19.6 / 18.5, 14336 x 4096 59.1 / 50.3 (ten of the sixteen chunks of 4096 stay: more are more than a wave's registers), 32000 x 4096 62.6 / 53.3.
 // The arithmetic is the streaming kernel's, sum for sum: chunks from the same place on (a workgroup's blocks are 4096 rows and more apart, so that they all
 // begin with the same one), the same wave for the same 32 k, the waves' tiles added in the same order.
 #include "seq_linear.h"
@@ -25,13 +26,14 @@ template <int NT, int TT, bool DUAL> struct HeldShape {
   static constexpr size_t LDS = TOKENS + RB * SLOT_B;
   static_assert(LDS <= 160 * 1024 && S::RED <= RB * SLOT_B && RA >= RB, "the unit's LDS; the waves' tiles in the tokens' ring");
 };
-template <typename P, int NT, int TT, bool DUAL, int NC>
+// HC: the chunks whose tokens stay, from the first on; the others' are fetched with every block's
+template <typename P, int NT, int TT, bool DUAL, int NC, int HC>
 __global__ __launch_bounds__(256, 1) void held_stream_kernel(void* __restrict__ out_, const u16* __restrict__ x, const u16* __restrict__ w,
                                                              const u16* __restrict__ bias, int T, int N, int epi, float limit, float alpha) {
   typedef HeldShape<NT, TT, DUAL> H;
   constexpr int K = NC * 256, STEP = 256, AT = H::AT, PA = H::PA, PB = H::PB, RA = H::RA, RB = H::RB;
   constexpr unsigned PIECE = H::PIECE, SLOT_A = H::SLOT_A, SLOT_B = H::SLOT_B;
-  static_assert(NC >= RA && STEP * 16 % 1024 == 0, "a ring's chunks are of two blocks at most; blocks that begin with the same chunk");
+  static_assert(NC >= RA && HC >= RB && STEP * 16 % 1024 == 0, "a ring's chunks are of two blocks at most; blocks that begin with the same chunk");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, g = lane >> 4;
   const unsigned lds0 = (unsigned)(size_t)(lds_char*)smem, lds1 = lds0 + H::TOKENS;
@@ -73,17 +75,17 @@ __global__ __launch_bounds__(256, 1) void held_stream_kernel(void* __restrict__ 
   auto frag = [&](unsigned base, int s) __attribute__((always_inline)) {
     return *reinterpret_cast<const lds_u32x4*>((size_t)(base + row + (((unsigned)(s * 4 + g)) ^ swz) * 16u));
   };
-  u32x4 held[NC][2][TT];                                     // this wave's tokens: two steps of 32 k of every chunk
+  u32x4 held[HC][2][TT];                                     // this wave's tokens: two steps of 32 k of a chunk
   f32x4 acc[AT][TT];
   int slot = 0;
   auto chunk = [&](auto c_, auto first_) __attribute__((always_inline)) {
     constexpr int c = decltype(c_)::value;
-    constexpr bool first = decltype(first_)::value;
-    // what was asked for behind this chunk's last piece: in the first block its tokens', with RB - 1 chunks of weights and RB - 2 of tokens behind
-    constexpr int T_LEFT = NC - 1 - c < RB - 2 ? NC - 1 - c : RB - 2, LEFT = first ? (RB - 1) * PA + T_LEFT * PB : (RA - 2) * PA;
+    constexpr bool first = decltype(first_)::value, fetched = first || c >= HC;
+    // what was asked for behind this chunk's last piece: its tokens', with RB - 1 chunks of weights and RB - 2 of tokens behind, or its weights'
+    constexpr int T_LEFT = NC - 1 - c < RB - 2 ? NC - 1 - c : RB - 2, LEFT = fetched ? (RB - 1) * PA + T_LEFT * PB : (RA - 2) * PA;
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(LEFT) : "memory");
     __builtin_amdgcn_s_barrier();
-    if constexpr (first && c + RB - 1 < NC) tokens(c + RB - 1);
+    if constexpr ((first || c + RB - 1 >= HC) && c + RB - 1 < NC) tokens(c + RB - 1);
     weights(slot == 0 ? RA - 1 : slot - 1);
     const unsigned base = lds0 + (unsigned)slot * SLOT_A;
 #pragma unroll
@@ -92,14 +94,20 @@ __global__ __launch_bounds__(256, 1) void held_stream_kernel(void* __restrict__ 
       u32x4 a[AT];
 #pragma unroll
       for (int i = 0; i < AT; ++i) a[i] = frag(base + (unsigned)(8 * i) * PIECE, s);
-      if constexpr (first) {
+      u32x4 t[TT];
+      if constexpr (fetched) {
 #pragma unroll
-        for (int tt = 0; tt < TT; ++tt) held[c][u][tt] = frag(lds1 + (unsigned)(c % RB) * SLOT_B + (unsigned)(8 * tt) * PIECE, s);
+        for (int tt = 0; tt < TT; ++tt) t[tt] = frag(lds1 + (unsigned)(c % RB) * SLOT_B + (unsigned)(8 * tt) * PIECE, s);
+      }
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        if constexpr (first && c < HC) held[c][u][tt] = t[tt];
+        if constexpr (!fetched) t[tt] = held[c][u][tt];
       }
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-        for (int i = 0; i < AT; ++i) acc[i][tt] = P::mfma(a[i], held[c][u][tt], acc[i][tt]);
+        for (int i = 0; i < AT; ++i) acc[i][tt] = P::mfma(a[i], t[tt], acc[i][tt]);
     }
     slot = slot + 1 == RA ? 0 : slot + 1;
   };
@@ -109,7 +117,7 @@ __global__ __launch_bounds__(256, 1) void held_stream_kernel(void* __restrict__ 
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt) acc[i][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
     unrolled<0, NC>([&](auto c_) __attribute__((always_inline)) { chunk(c_, first_); });
-    // the waves' tiles are added in the tokens' ring, which nobody reads behind the first block's last chunk
+    // the waves' tiles are added in the tokens' ring: nobody reads it behind a block's last chunk, and its pieces are asked for again behind the next's first
     if (b + STEP >= nb) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // behind the last block no piece may be on its way any more
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -154,11 +162,11 @@ __global__ __launch_bounds__(256, 1) void held_stream_kernel(void* __restrict__ 
   for (int b = blockIdx.x + STEP; b < nb; b += STEP) block(b, std::false_type{});
 }
 
-template <typename P, int NT, int TT, bool DUAL, int NC>
+template <typename P, int NT, int TT, bool DUAL, int NC, int HC = NC>
 static int held_launch(void* out, const void* x, const void* w, const void* bias, int T, int N, int epi, float limit, float alpha, hipStream_t st) {
   constexpr size_t lds = HeldShape<NT, TT, DUAL>::LDS;
-  if (ensure_dynamic_lds<held_stream_kernel<P, NT, TT, DUAL, NC>>(lds) != UMB_OK) return UMB_EHIP;
-  hipLaunchKernelGGL((held_stream_kernel<P, NT, TT, DUAL, NC>), dim3(256), dim3(256), lds, st, out, (const u16*)x, (const u16*)w, (const u16*)bias, T, N, epi,
+  if (ensure_dynamic_lds<held_stream_kernel<P, NT, TT, DUAL, NC, HC>>(lds) != UMB_OK) return UMB_EHIP;
+  hipLaunchKernelGGL((held_stream_kernel<P, NT, TT, DUAL, NC, HC>), dim3(256), dim3(256), lds, st, out, (const u16*)x, (const u16*)w, (const u16*)bias, T, N, epi,
                      limit, alpha);
   UMB_LAUNCH_CHECK();
   return UMB_OK;
@@ -169,9 +177,11 @@ int held_stream(void* out, const void* x, const void* w, const void* bias, int T
   auto run = [&](auto tag) -> int {
     typedef decltype(tag) P;
     if (epi_dual(epi)) {
+      if (K == 4096 && T > 48) return held_launch<P, 1, 4, true, 16, 10>(out, x, w, bias, T, N, epi, limit, alpha, st);
       if (K == 4096) return held_launch<P, 1, 3, true, 16>(out, x, w, bias, T, N, epi, limit, alpha, st);
       return T <= 48 ? held_launch<P, 1, 3, true, 8>(out, x, w, bias, T, N, epi, limit, alpha, st) : held_launch<P, 1, 4, true, 8>(out, x, w, bias, T, N, epi, limit, alpha, st);
     }
+    if (K == 4096 && T > 48) return held_launch<P, 2, 4, false, 16, 10>(out, x, w, bias, T, N, epi, limit, alpha, st);
     if (K == 4096) return held_launch<P, 2, 3, false, 16>(out, x, w, bias, T, N, epi, limit, alpha, st);
     return T <= 48 ? held_launch<P, 2, 3, false, 8>(out, x, w, bias, T, N, epi, limit, alpha, st) : held_launch<P, 2, 4, false, 8>(out, x, w, bias, T, N, epi, limit, alpha, st);
   };

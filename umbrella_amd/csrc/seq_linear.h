@@ -140,9 +140,9 @@ static inline bool stream_pays(int T, int N, int K, int epi, int gz, int eb) {
 }
 
 // Streaming products of 33 to 64 tokens whose tokens stay in a workgroup's registers (seq_held.hip): where its 256 workgroups have more than one block of
-// rows each (with one there is nothing to keep for), and K is as many chunks as they hold: 8, or 16 up to 48 tokens, at 450 of 512 registers.
+// rows each (with one there is nothing to keep for), and K is as many chunks as they hold: 8, or 16, of which beyond 48 tokens ten stay, at 450 of 512 registers.
 static inline bool held_pays(int T, int N, int K, int epi) {
   if (T <= 32 || T > 64 || !(epi_dual(epi) || epi == EPI_F32 || epi == EPI_DT || epi == EPI_CAP)) return false;
-  return (K == 2048 || (K == 4096 && T <= 48)) && (N + 15) / 16 > (epi_dual(epi) ? 256 : 512);
+  return (K == 2048 || K == 4096) && (N + 15) / 16 > (epi_dual(epi) ? 256 : 512);
 }
 int held_stream(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, float limit, float alpha, int dtype, hipStream_t st);

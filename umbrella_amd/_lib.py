@@ -7,6 +7,7 @@ returns non-zero, this raises.  Build with ``python -c "import __graft_entry__ a
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import os
 
@@ -460,6 +461,16 @@ class UmbError(RuntimeError):
 def check(rc: int, what: str = ""):
     if rc != 0:
         raise UmbError(f"libumbrella_hip {what} failed with code {rc}")
+
+
+@contextlib.contextmanager
+def capturing(graph):
+    """torch.cuda.graph for launches of this library.  Entered outside inference mode: what the first capture allocates for the random generator, and every
+    later one writes while a graph is alive, would be inference tensors otherwise, which a capture outside that mode may not write.  The body runs in the mode
+    of the caller.  thread_local: other threads go on asking for events (a process group's watchdog), which a capture in global mode turns into an error."""
+    mode = torch.is_inference_mode_enabled()
+    with torch.inference_mode(False), torch.cuda.graph(graph, capture_error_mode="thread_local"), torch.inference_mode(mode):
+        yield
 
 
 def stream_ptr() -> C.c_void_p:

@@ -562,7 +562,7 @@ class SeqMixLM(LLMBase):
             # the second step of this shape: everything it launches has run once (function attributes are set), so the
             # step can be captured -- capturing executes nothing -- and replayed from now on
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, capture_error_mode="thread_local"):       # (other threads go on asking for events: a process group's watchdog)
+            with _lib.capturing(g):
                 launch()
             entry["graph"] = g
             g.replay()

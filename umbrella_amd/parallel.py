@@ -239,6 +239,7 @@ def prefill_chunk(model) -> int:
 
 
 def _capture(run, device):
+    from . import _lib
     s = torch.cuda.Stream(device=device)
     s.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(s):
@@ -246,7 +247,7 @@ def _capture(run, device):
     torch.cuda.current_stream().wait_stream(s)
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g, capture_error_mode="thread_local"):       # (other threads go on asking for events: a process group's watchdog)
+    with _lib.capturing(g):
         run()
     torch.cuda.synchronize()
     return g

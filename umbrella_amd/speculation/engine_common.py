@@ -250,9 +250,7 @@ class HipEngine(BaseEngine):
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
-        # thread_local: a process group's watchdog thread may still be asking for the warm-up's collectives, which a capture in
-        # global mode turns into an error that ends the process
-        with torch.cuda.graph(g, capture_error_mode="thread_local"):
+        with _lib.capturing(g):
             self._iteration_launch()
         torch.cuda.synchronize()
         self.n_dev.copy_(n_save)

@@ -9,7 +9,9 @@ from __future__ import annotations
 
 import contextlib
 import ctypes as C
+import gc
 import os
+import threading
 
 import torch
 
@@ -463,13 +465,37 @@ def check(rc: int, what: str = ""):
         raise UmbError(f"libumbrella_hip {what} failed with code {rc}")
 
 
+_captures_lock, _captures, _collector_was_on = threading.Lock(), 0, False
+
+
+@contextlib.contextmanager
+def _collector_off():
+    """Nothing is collected while a capture is open, in whichever thread: a dead engine stands in reference cycles (a pipeline's engine and its target hold one
+    another), and the graph that goes with it synchronises the device as it is freed.  A thread that captures may not, and the error leaves a destructor, which
+    ends the process.  Behind the last capture the collector is what it was; what has died meanwhile waits for it.  (A collection in front is no substitute, as
+    the body may start another, and none is needed beside this: 50 ms of a process that serves, for every captured shape.)"""
+    global _captures, _collector_was_on
+    with _captures_lock:
+        if _captures == 0:
+            _collector_was_on = gc.isenabled()
+            gc.disable()
+        _captures += 1
+    try:
+        yield
+    finally:
+        with _captures_lock:
+            _captures -= 1
+            if _captures == 0 and _collector_was_on:
+                gc.enable()
+
+
 @contextlib.contextmanager
 def capturing(graph):
-    """torch.cuda.graph for launches of this library.  Entered outside inference mode: what the first capture allocates for the random generator, and every
-    later one writes while a graph is alive, would be inference tensors otherwise, which a capture outside that mode may not write.  The body runs in the mode
-    of the caller.  thread_local: other threads go on asking for events (a process group's watchdog), which a capture in global mode turns into an error."""
+    """torch.cuda.graph for launches of this library, the collector off (_collector_off).  Entered outside inference mode: what the first capture allocates for
+    the random generator, and every later one writes while a graph is alive, would be inference tensors otherwise, which a capture outside that mode may not
+    write.  The body runs in the mode of the caller.  thread_local: other threads go on asking for events (a process group's watchdog), which a capture in global mode turns into an error."""
     mode = torch.is_inference_mode_enabled()
-    with torch.inference_mode(False), torch.cuda.graph(graph, capture_error_mode="thread_local"), torch.inference_mode(mode):
+    with _collector_off(), torch.inference_mode(False), torch.cuda.graph(graph, capture_error_mode="thread_local"), torch.inference_mode(mode):
         yield
 
 

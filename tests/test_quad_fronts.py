@@ -44,3 +44,62 @@ def test_head_gates(dtype, T, H, Dv, den, weights, kind):
     assert bool((out[T] == 7.0).all()) and bool((out[:T, H * Dv:] == 7.0).all())
     eps = torch.finfo(dtype).eps
     assert bool(((out[:T, :H * Dv].double() - want).abs() <= 0.51 * eps * want.abs() + 2e-6 * want.abs() + 1e-7).all())
+
+
+# ---- the same bits as the kernels that take what quads are not aligned in (an element or a pair a lane)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("H,G,D,E,maps,layout,rot,append,norm,mixed", [(8, 2, 64, 64, 1, 0, 64, 1, 1, True), (9, 3, 128, 64, 2, 1, 80, 1, 0, False),
+                                                                       (17, 17, 64, 128, 1, 1, 36, 1, 1, True), (30, 2, 128, 128, 1, 0, 48, 0, 1, False),
+                                                                       (32, 8, 128, 128, 2, 0, 128, 1, 1, False), (32, 8, 64, 64, 1, 1, 0, 1, 1, False)])
+def test_attention_slots_bit_by_bit(dtype, H, G, D, E, maps, layout, rot, append, norm, mixed):
+    from umbrella_amd import _lib
+    T, code = 2880, _lib.seq_dtype_code(dtype)
+    g = torch.Generator(device="cuda").manual_seed(D + E)
+    HQ, GK, GV = maps * H, append * maps * G, append * G
+    ld = HQ * D + GK * D + GV * E + 5
+    proj, freq, firsts = torch.randn(T, ld, generator=g, device="cuda"), torch.rand(64, generator=g, device="cuda"), torch.randn(T, G * E, generator=g, device="cuda")
+    wq, wk = (torch.randn(D, generator=g, device="cuda").to(dtype) for _ in range(2))
+    pos, slot = torch.arange(T, device="cuda", dtype=torch.int32), torch.zeros(T, device="cuda", dtype=torch.int32)
+    outs = []
+    for shift in (0, 1):                                       # q 4 bytes behind 16: no quads
+        c, _, _, _ = prompt._decode_store([T], G, maps * D, E, 0, dtype, 32, 1)
+        q, keep = torch.zeros(T * HQ * D + 4, device="cuda"), torch.zeros(T, G * E, device="cuda")
+        m = _lib.UmbValueMix(firsts.data_ptr(), keep.data_ptr(), 0.3, 0.0) if mixed else None
+        _lib.seq_call("umb_attn_prep_mix", q[shift:], c.struct(0), proj, ld, append, wq if norm else None, wk if norm else None, norm, norm, pos, slot,
+                      freq if rot else None, rot, layout, 1.1, T, H, G, D, E, maps, 0.1, 100, 1e-5, m, code)
+        outs.append([q[shift:shift + T * HQ * D].clone(), keep, c.kv[0]["k"], c.kv[0]["v"]])
+    assert all(torch.equal(x, y) for x, y in zip(*outs))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("H,G,D,rot", [(32, 8, 64, 64), (16, 8, 128, 128), (20, 4, 64, 0), (17, 1, 128, 60)])
+def test_pooled_slots_bit_by_bit(dtype, H, G, D, rot):
+    from umbrella_amd import _lib
+    T, code = 1700, _lib.seq_dtype_code(dtype)
+    g = torch.Generator(device="cuda").manual_seed(D)
+    proj, freq = torch.randn(T, (H + G) * D + 3, generator=g, device="cuda"), torch.rand(64, generator=g, device="cuda")
+    pos, slot = torch.arange(T, device="cuda", dtype=torch.int32), torch.zeros(T, device="cuda", dtype=torch.int32)
+    outs = []
+    for shift in (0, 1):
+        c, _, _, _ = prompt._decode_store([T], G, D, D, 5, dtype, 32, 1)
+        q = torch.zeros(T * H * D + 4, device="cuda")
+        _lib.seq_call("umb_pwa_prep", q[shift:], c.struct(0), proj, proj.shape[1], pos, slot, freq if rot else None, T, H, G, D, rot, 1e-5, code)
+        outs.append([q[shift:shift + T * H * D].clone(), c.kv[0]["k"], c.kv[0]["v"]])
+    assert all(torch.equal(x, y) for x, y in zip(*outs))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,Dv", [(1800, 11, 64), (2467, 7, 128), (601, 9, 256), (1, 16, 256), (7, 1, 128)])
+@pytest.mark.parametrize("den,weights,kind", [(False, 0, 0), (True, 1, 1), (True, 2, 0)])
+def test_head_gates_bit_by_bit(dtype, T, H, Dv, den, weights, kind):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + Dv)
+    cols, ld, outs = Dv + int(den), H * Dv + 5, []
+    o, proj, mrun = (torch.randn(s, generator=g, device="cuda") for s in ((T, H, cols), (T, ld), (T, H)))
+    w = torch.randn(Dv if weights == 1 else H * Dv, generator=g, device="cuda").to(dtype) if weights else None
+    for ldo in (H * Dv, H * Dv + 1):
+        out = torch.zeros((T, ldo), dtype=dtype, device="cuda")
+        _lib.seq_call("umb_head_gate", out, ldo, o, cols, Dv if den else -1, mrun if den else None, proj, ld, 3, w, int(weights == 2), kind, T, H, Dv, 1e-5, 1.2,
+                      _lib.seq_dtype_code(dtype))
+        outs.append(out[:, :H * Dv])
+    assert torch.equal(*outs)

@@ -197,22 +197,15 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, U
 // The same for many items, rows of 64 or 128 whose turned part is whole quads: a wave takes PREP_QUADS quads a lane of one token's neighbouring rows (queries
 // and keys, or values), two or four rows side by side, all loads in flight, and works the angles out once for all of them.
 // Vector work bounded what it replaces (four slots a wave, an element a lane, the angles again for every four: some 250 instructions a slot, quotients and
-// sines among them).  us, that / this, bf16: 2466 tokens, 32 + 8 + 8 slots of 64 33.9 / 16.0 (68 MB, 4.2 TB/s), 1999 tokens, 32 + 8 + 8 of 128 with mixed
-// values 34.8 / 23.2 (98 MB); with a branch between the loads and the sines four times over 18.0 / 25.5.
+// sines among them).  us, that / this, bf16: 2466 tokens, 32 + 8 + 8 slots of 64 33.9 / 16.2 (68 MB, 4.2 TB/s), 1999 tokens, 32 + 8 + 8 of 128 with mixed
+// values 34.8 / 24.9 (98 MB).  The sums and roundings are those of that kernel (quads_square, two_products): in the order that quads would take by themselves
+// 15.6 / 22.4, and the cached rows of a prompt were others.
 constexpr int PREP_QUADS = 4;
 constexpr int prep_rows(int D) { return PREP_QUADS * 256 / D; }      // rows a wave takes
 typedef float quad_u __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ f32x4 ldq(const float* p) { return *reinterpret_cast<const quad_u*>(p); }
 // 1 / root mean square of a row that D / 4 neighbouring lanes hold
-template <int D> __device__ __forceinline__ float quad_row_scale(f32x4 x, float eps) {
-  float s = row_add16(sq4(x));
-  if constexpr (D == 128) {
-    float b = s;
-    swap16(s, b);
-    s += b;
-  }
-  return 1.f / sqrtf(s / (float)D + eps);
-}
+template <int D> __device__ __forceinline__ float quad_row_scale(f32x4 x, float eps) { return 1.f / sqrtf(quads_square<D, true>(x) / (float)D + eps); }
 template <typename P, int D, int E>
 __global__ __launch_bounds__(256) void attn_prep_quads_kernel(float* __restrict__ q, UmbPagedKV kv, const float* __restrict__ proj, int ld,
                                                               const typename El<P>::type* __restrict__ w_q, const typename El<P>::type* __restrict__ w_k,
@@ -246,7 +239,7 @@ __global__ __launch_bounds__(256) void attn_prep_quads_kernel(float* __restrict_
       if (a.mix.keep) *reinterpret_cast<quad_u*>(a.mix.keep + row0 + r * E) = v[u];
       if (a.mix.first) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[u][i] = (1.f - a.mix.lambda) * v[u][i] + a.mix.lambda * m[u][i];
+        for (int i = 0; i < 4; ++i) v[u][i] = fmaf(1.f - a.mix.lambda, v[u][i], a.mix.lambda * m[u][i]);
       }
       st4<P>(reinterpret_cast<El_*>(kv.v) + out0 + (long)r * kv.page * E, v[u]);
     }
@@ -304,7 +297,7 @@ __global__ __launch_bounds__(256) void attn_prep_quads_kernel(float* __restrict_
     if (!far) y[u] = f32x4{x[u][1], x[u][0], x[u][3], x[u][2]};
     f32x4 o;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = x[u][i] * cs[i] + y[u][i] * sn[i];
+    for (int i = 0; i < 4; ++i) o[i] = two_products(x[u][i], cs[i], y[u][i], sn[i]);
     if (!rot) o = x[u];
     if (r >= n) continue;
     if (is_q) *reinterpret_cast<f32x4*>(q + ((long)t * a.HQ + hs) * D + e) = o * temp;

@@ -41,6 +41,44 @@ __device__ __forceinline__ float add_rows(float v) {
   return a + b;
 }
 
+// Sum of squares of a row of 64, 128 or 256 that D / 4 neighbouring lanes hold in quads, in every lane of them.  The order is that of a wave with an element a lane:
+// those 64 apart, one after the other (LAST_FIRST: the last rounded first), then those 32, 16, .. 1 apart; a row is scaled by the same bits whichever kernel
+// prepares it.  (fmaf with 0: a product alone would be contracted into the sum behind it.)
+template <int D, bool LAST_FIRST> __device__ __forceinline__ float quads_square(f32x4 x) {
+  float s[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (D == 64) s[k] = fmaf(x[k], x[k], 0.f);
+    else if constexpr (D == 128) {
+      float a = x[k], b = x[k];
+      swap16(a, b);
+      s[k] = LAST_FIRST ? fmaf(a, a, fmaf(b, b, 0.f)) : fmaf(b, b, fmaf(a, a, 0.f));
+    } else {
+      static_assert(D == 256 && !LAST_FIRST);
+      float a = x[k], c = x[k];
+      swap32(a, c);
+      float b = a, d = c;
+      swap16(a, b);
+      swap16(c, d);
+      s[k] = fmaf(d, d, fmaf(c, c, fmaf(b, b, fmaf(a, a, 0.f))));
+    }
+    s[k] = row_add16(s[k]);
+  }
+  return (s[0] + s[2]) + (s[1] + s[3]);
+}
+// a b + c d, both products rounded
+__device__ __forceinline__ float two_products(float a, float b, float c, float d) {
+#pragma clang fp contract(off)
+  return a * b + c * d;
+}
+
+// A product that is rounded to fp32 in front of a conversion to fp16 (v_fma_mixlo_f16 would round it once): opaque to the compiler
+__device__ __forceinline__ f32x4 rounded(f32x4 v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm("" : "+v"(v[i]));
+  return v;
+}
+
 // row number of a token's / a pooled block's vectors in the paged store
 __device__ __forceinline__ unsigned pkv_tok_row(const UmbPagedKV& kv, int slot, int pos, int g, int G) {
   const int pg = kv.pages[(long)slot * kv.max_pages + pos / kv.page];

@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void pwa_prep_four_kernel(float* __restrict__ 
 
 // The same where rows are 64 or 128 long and turned in whole quads: a wave takes PREP_QUADS quads a lane of one token's neighbouring slots, two or four side
 // by side, all loads in flight, the angles worked out once for all of them; bound by its bytes, where four slots a wave were by their vector work (seq_battn.hip): 2048 tokens,
-// 32 + 8 slots of 64 18.9 -> 10.2 us.
+// 32 + 8 slots of 64 18.9 -> 10.8 us (10.2 with the sums of squares in another order than that kernel's).
 constexpr int PREP_QUADS = 4;
 constexpr int prep_rows(int D) { return PREP_QUADS * 256 / D; }      // slots a wave takes
 template <typename P, int D>
@@ -288,22 +288,28 @@ __global__ __launch_bounds__(256) void pwa_prep_quads_kernel(float* __restrict__
     if (e < rot_dims) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        o[2 * i] = x[k][2 * i] * cs[i] - x[k][2 * i + 1] * sn[i];
-        o[2 * i + 1] = x[k][2 * i + 1] * cs[i] + x[k][2 * i] * sn[i];
+        o[2 * i] = fmaf(x[k][2 * i], cs[i], -(x[k][2 * i + 1] * sn[i]));
+        o[2 * i + 1] = fmaf(x[k][2 * i + 1], cs[i], x[k][2 * i] * sn[i]);
       }
     }
-    float s = row_add16(sq4(o));
-    if constexpr (D == 128) {
-      float b = s;
-      swap16(s, b);
-      s += b;
+    float sq[2];                                             // pairs, in the order of a wave with a pair a lane
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      sq[i] = fmaf(o[2 * i], o[2 * i], fmaf(o[2 * i + 1], o[2 * i + 1], 0.f));
+      if constexpr (D == 128) {
+        float b = sq[i];
+        swap16(sq[i], b);
+        sq[i] += b;
+      }
+      sq[i] = row_add16(sq[i]);
     }
-    const float f = 1.f / sqrtf(s / (float)D + eps);
+    const float f = 1.f / sqrtf((sq[0] + sq[1]) / (float)D + eps);
     if (r >= n) continue;
-    if (hs < H) *reinterpret_cast<f32x4*>(q + ((long)t * H + hs) * D + e) = o * f;
+    o = rounded(o * f);
+    if (hs < H) *reinterpret_cast<f32x4*>(q + ((long)t * H + hs) * D + e) = o;
     else {
       const long off = kv0 + (long)(hs - H) * kv.page * D;
-      st4<P>(reinterpret_cast<E*>(kv.k) + off, o * f);
+      st4<P>(reinterpret_cast<E*>(kv.k) + off, o);
       st4<P>(reinterpret_cast<E*>(kv.v) + off, x[k]);
     }
   }

@@ -76,7 +76,8 @@ __global__ __launch_bounds__(256) void head_gate_kernel(typename El<P>::type* __
 
 // The same for heads of 64, 128 or 256 columns: a quad a lane, LPH = Dv / 4 lanes a head, NU heads of every 64 / LPH side by side one after the other, read-outs
 // and gates of all asked for together (in two walks over single columns a wave's second trip waited for the first, and a head's 25 instructions of quotient and
-// root were a wave's: they are two or four heads').  2466 tokens, 16 heads of 128, bf16: 27.1 -> 12.6 us (50 MB); one token, 32 heads: level.
+// root were a wave's: they are two or four heads').  2466 tokens, 16 heads of 128, bf16: 27.1 -> 13.3 us (50 MB; 12.3 with
+// the sum of squares in another order than a wave's); one token, 32 heads: level.
 template <typename P, int LPH, int NU>
 __global__ __launch_bounds__(256) void head_gate_quad_kernel(typename El<P>::type* __restrict__ out, int ldo, const float* __restrict__ o, int Pc, int den_col,
                                                              const float* __restrict__ mrun, const float* __restrict__ proj, int ld, int g_col,
@@ -101,13 +102,7 @@ __global__ __launch_bounds__(256) void head_gate_quad_kernel(typename El<P>::typ
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     if (den_col >= 0) v[u] = v[u] * (1.f / (fmaxf(fabsf(den[u]), expf(-mrun[(long)t[u] * H + h[u]])) + 1e-6f));
-    float s = row_add16(sq4(v[u]));
-    if constexpr (LPH == 32) {
-      float b = s;
-      swap16(s, b);
-      s += b;
-    } else if constexpr (LPH == 64) s = add_rows(s);
-    const float f = out_scale / sqrtf(s / (float)Dv + eps);
+    const float f = out_scale / sqrtf(quads_square<Dv, false>(v[u]) / (float)Dv + eps);
     f32x4 y = v[u] * f;
     if (w) y = y * ld4<P>(w + (long)h[u] * w_stride + e);
 #pragma unroll

@@ -69,3 +69,40 @@ def test_step_as_two_launches(dtype, H, G, D, E, maps, lens, window, chunk, keep
     for x, y in zip(a[1:], b[1:]):
         assert bool(((x.float() - y.float()).abs() <= step_of * x.float().abs() + 1e-6).all())
     assert bool(((a[0].float() - b[0].float()).abs() <= 2 * step_of * a[0].float().abs() + 1e-5).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,E,maps,rot,layout,norm_v", [(32, 8, 128, 128, 1, 128, 0, 1), (32, 8, 64, 256, 1, 64, 1, 1), (32, 8, 64, 64, 1, 64, 1, 0), (16, 4, 256, 256, 1, 256, 1, 0),
+                                                            (16, 4, 128, 256, 2, 128, 0, 1), (8, 2, 96, 128, 1, 50, 1, 0)])
+def test_step_appends_what_a_launch_of_its_own_does(dtype, H, G, D, E, maps, rot, layout, norm_v):
+    """keys, values and the first layer's kept ones, bit by bit: a token's cached rows do not depend on the launch that prepared them"""
+    import ctypes as C
+    from umbrella_amd import _lib
+    from umbrella_amd.attn.cache import PagedSeqCache
+    code, T = _lib.seq_dtype_code(dtype), 150
+    ld = maps * H * D + maps * G * D + G * E
+    g = torch.Generator(device="cuda").manual_seed(H + D + E)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")                                              # noqa: E731
+    proj, freq, first = rnd(T, ld), torch.rand(rot // 2, generator=g, device="cuda"), rnd(T, G * E)
+    wq, wk = (1.0 + 0.1 * rnd(D)).to(dtype), (1.0 + 0.1 * rnd(D)).to(dtype)
+    lens = [1 + i % 70 for i in range(T)]
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device="cuda")
+    outs = []
+    for step in (False, True):
+        c = PagedSeqCache([(G, maps * D, 0, E)], [], sum(lens) + 100, T, "cuda", dtype, page=32)
+        for b, n in enumerate(lens):
+            c.open(b), c.extend(b, n)
+        c.kv[0]["k"].zero_(), c.kv[0]["v"].zero_()
+        slot = torch.tensor([c.slot(b) for b in range(T)], dtype=torch.int32, device="cuda")
+        q, kept, out = torch.zeros(T, maps * H * D, device="cuda"), torch.zeros(T, G * E, device="cuda"), torch.zeros(T, H * E, dtype=dtype, device="cuda")
+        form, mix = _lib.UmbAttnForm(), _lib.UmbValueMix(first.data_ptr(), kept.data_ptr(), 0.4, 0.0)
+        form.maps, form.eps, form.lambda_ = maps, 1e-6, 0.3
+        kv = c.struct(0)
+        if step:
+            _lib.seq_call("umb_attn_step", out, H * E, q, kv, proj, ld, 1, wq, wk, 1, norm_v, freq, rot, layout, 1.1, 0.0, 0, 1e-6, C.byref(mix), -1, None, 0, pos,
+                          slot, T, H, G, D, E, 2 ** 30, D ** -0.5, 1.0, 0.0, form, None, 0, code)
+        else:
+            _lib.seq_call("umb_attn_prep_mix", q, kv, proj, ld, 1, wq, wk, 1, norm_v, pos, slot, freq, rot, layout, 1.1, T, H, G, D, E, maps, 0.0, 0, 1e-6,
+                          C.byref(mix), code)
+        outs.append((kept, c.kv[0]["k"], c.kv[0]["v"]))
+    assert float(outs[0][0].abs().sum()) > 0.0 and all(torch.equal(x, y) for x, y in zip(*outs))

@@ -118,3 +118,32 @@ def test_sequences_that_bring_nothing_stand_in_front(monkeypatch):
     assert len(keep) == 4
     for a, b in zip(*got):
         assert torch.equal(a, b) and bool((a != 9.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,rot", [(32, 8, 64, 64), (16, 4, 128, 128), (4, 4, 256, 0), (8, 2, 256, 200), (6, 2, 96, 40)])
+def test_step_appends_what_a_launch_of_its_own_does(dtype, H, G, D, rot):
+    """keys and values bit by bit: a token's cached rows do not depend on the launch that prepared them"""
+    from umbrella_amd import _lib
+    from umbrella_amd.attn.cache import PagedSeqCache
+    code, T, ld, pool = _lib.seq_dtype_code(dtype), 150, (H + G) * D + H, 16
+    g = torch.Generator(device="cuda").manual_seed(H + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")                                              # noqa: E731
+    proj, freq, bias = rnd(T, ld), torch.rand(max(rot // 2, 1), generator=g, device="cuda"), rnd(H).to(dtype)
+    lens = [1 + i % 70 for i in range(T)]
+    pos, one, outs = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device="cuda"), torch.ones(T, dtype=torch.int32, device="cuda"), []
+    for step in (False, True):
+        c = PagedSeqCache([(G, D, pool)], [], sum(lens) + 50, T, "cuda", dtype, page=32)
+        for b, n in enumerate(lens):
+            c.open(b), c.extend(b, n)
+        for z in ("k", "v", "kp", "vp"):
+            c.kv[0][z].zero_()
+        slot = torch.tensor([c.slot(b) for b in range(T)], dtype=torch.int32, device="cuda")
+        q, out = torch.zeros(T, H * D, device="cuda"), torch.zeros(T, H * D, dtype=dtype, device="cuda")
+        if step:
+            _lib.seq_call("umb_pwa_step", out, q, c.struct(0), proj, ld, (H + G) * D, bias, pos, slot, freq, slot, pos, one, T, H, G, D, rot, 64, pool, D ** -0.5,
+                          1e-6, code)
+        else:
+            _lib.seq_call("umb_pwa_prep", q, c.struct(0), proj, ld, pos, slot, freq, T, H, G, D, rot, 1e-6, code)
+        outs.append((c.kv[0]["k"], c.kv[0]["v"]))
+    assert all(torch.equal(x, y) for x, y in zip(*outs))

@@ -112,8 +112,7 @@ __device__ __forceinline__ void attn_prep_pairs(const float* __restrict__ src, c
 #pragma unroll 1
     for (int i = lane; i < a.D; i += 128) {
       const float x = src[i], y = i + 64 < a.D ? src[i + 64] : 0.f;
-      ss += x * x;
-      ss += y * y;
+      ss = fmaf(y, y, fmaf(x, x, ss));
     }
     f = 1.f / sqrtf(wave_sum(ss) / (float)a.D + a.eps);
   }
@@ -126,7 +125,7 @@ __device__ __forceinline__ void attn_prep_pairs(const float* __restrict__ src, c
       sincosf((float)p * fr, &sn, &cs);
       sn *= a.rot_mult;
       cs *= a.rot_mult;
-      const float rx = x * cs - y * sn, ry = y * cs + x * sn;
+      const float rx = fmaf(x, cs, -(y * sn)), ry = fmaf(y, cs, x * sn);
       x = rx;
       y = ry;
     }
@@ -151,14 +150,14 @@ __device__ __forceinline__ void attn_prep_value_few(const float* __restrict__ sr
   if (a.norm_v) {
     float ss = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) ss += v[c] * v[c];
+    for (int c = 0; c < NC; ++c) ss = fmaf(v[c], v[c], ss);
     f = 1.f / sqrtf(wave_sum(ss) / (float)(64 * NC) + a.eps);
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     float x = v[c] * f;
     if (keep && a.mix.keep) a.mix.keep[o + lane + 64 * c] = x;
-    if (a.mix.first) x = (1.f - a.mix.lambda) * x + a.mix.lambda * m[c];
+    if (a.mix.first) x = fmaf(1.f - a.mix.lambda, x, a.mix.lambda * m[c]);
     put(lane + 64 * c, x);
   }
 }

@@ -11,6 +11,7 @@
 // ONE wave as ten dependent memory trips while the other fifteen waves of its workgroup were idle: 19 to 23 us at 40 keys.
 #pragma once
 #include "seq_common.h"
+#include <type_traits>
 
 // a = {a.lo, b.lo}, b = {a.hi, b.hi} in halves of 32 lanes / in rows of 16 lanes, pairwise.  Written out: the builtin's second result came
 // back as its first.  Volatile: not to be moved under a narrower execution mask.
@@ -72,11 +73,19 @@ __device__ __forceinline__ float two_products(float a, float b, float c, float d
   return a * b + c * d;
 }
 
-// A product that is rounded to fp32 in front of a conversion to fp16 (v_fma_mixlo_f16 would round it once): opaque to the compiler
+// The same values in 16 bits either way of rounding, whatever the compiler would make of a product in front of a conversion.  fp16: the product rounded to fp32 first
+// (opaque, so that it is), or once, as v_fma_mixlo_f16 does; bf16 has no such instruction.
 __device__ __forceinline__ f32x4 rounded(f32x4 v) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) asm("" : "+v"(v[i]));
   return v;
+}
+template <typename P> __device__ __forceinline__ u16 product_once(float a, float b) {
+  if constexpr (std::is_same<P, F16>::value) {
+    unsigned r;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
+    return (u16)r;
+  } else return P::from_f(a * b);
 }
 
 // row number of a token's / a pooled block's vectors in the paged store

@@ -88,7 +88,7 @@ __device__ __forceinline__ void pwa_row(const float* __restrict__ src, int D, in
   }
 }
 // The same for the decode kernel: D features (a multiple of 32) as NP pairs a lane, asked for together with their frequencies in front of anything that
-// waits, one angle a pair; compact, because what a launch executes once costs its fetch.  put(feature, turned and normed, as projected)
+// waits, one angle a pair; compact, because what a launch executes once costs its fetch.  put(feature, turned, what norms it, as projected)
 template <int D, typename Put>
 __device__ __forceinline__ void pwa_row_few(const float* __restrict__ src, int rot_dims, const float* __restrict__ freq, int p, float eps, Put put) {
   constexpr int NP = (D + 127) / 128;
@@ -110,18 +110,18 @@ __device__ __forceinline__ void pwa_row_few(const float* __restrict__ src, int r
     if (2 * m + 1 < rot_dims) {
       float sn, cs;
       sincosf((float)p * fr[c], &sn, &cs);
-      const float ru = u[c] * cs - v[c] * sn, rv = v[c] * cs + u[c] * sn;
+      const float ru = fmaf(u[c], cs, -(v[c] * sn)), rv = fmaf(v[c], cs, u[c] * sn);
       u[c] = ru; v[c] = rv;
     }
-    if (2 * m < D) ss += u[c] * u[c] + v[c] * v[c];
+    if (2 * m < D) ss += fmaf(u[c], u[c], fmaf(v[c], v[c], 0.f));
   }
   const float f = 1.f / sqrtf(wave_sum(ss) / (float)D + eps);
 #pragma unroll
   for (int c = 0; c < NP; ++c) {
     const int m = lane + 64 * c;
     if (2 * m >= D) continue;
-    put(2 * m, u[c] * f, raw[c][0]);
-    put(2 * m + 1, v[c] * f, raw[c][1]);
+    put(2 * m, u[c], f, raw[c][0]);
+    put(2 * m + 1, v[c], f, raw[c][1]);
   }
 }
 // the pooled block that the token at p completes, by a wave: the sums of the cached positions in front of it and its own key and value as they are stored
@@ -568,12 +568,12 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
         const long off = is_q ? 0 : pkv_tok(kv, slot, i, g, G, D);
         u16* kd = reinterpret_cast<u16*>(kv.k) + off;
         u16* vd = reinterpret_cast<u16*>(kv.v) + off;
-        pwa_row_few<D>(src + (is_q ? h0 + task : H + g) * D, prep.rot_dims, prep.freq, i, prep.eps, [&](int d, float x, float raw) {
+        pwa_row_few<D>(src + (is_q ? h0 + task : H + g) * D, prep.rot_dims, prep.freq, i, prep.eps, [&](int d, float x, float f, float raw) {
           if (is_q) {
-            q_s[task * D + d] = x;
+            q_s[task * D + d] = x * f;
             return;
           }
-          const u16 kb = P::from_f(x), vb = P::from_f(raw);
+          const u16 kb = product_once<P>(x, f), vb = P::from_f(raw);
           new_k[d] = kb;
           new_v[d] = vb;
           if (append) { kd[d] = kb; vd[d] = vb; }

@@ -9,6 +9,11 @@ import torch
 from umbrella_amd import _lib
 
 
+class Graph:
+    def register_generator_state(self, generator):
+        self.registered_in_mode = torch.is_inference_mode_enabled()
+
+
 class Dead:
     """stands in a cycle, as an engine and its target do; says on its end whether a capture was open"""
     def __init__(self, log, open_):
@@ -30,6 +35,8 @@ def stand_in(monkeypatch):
         finally:
             open_[0] -= 1
     monkeypatch.setattr(torch.cuda, "graph", graph)
+    monkeypatch.setattr(torch.cuda, "default_generators", (None,))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     was = gc.isenabled()
     yield open_
     (gc.enable if was else gc.disable)()
@@ -47,7 +54,7 @@ def test_nothing_is_freed_inside(stand_in, on, fails):
     log = []
     Dead(log, stand_in)
     with pytest.raises(KeyError) if fails else contextlib.nullcontext():
-        with _lib.capturing(object()):
+        with _lib.capturing(Graph()):
             _allocate()
             assert not gc.isenabled()
             if fails:
@@ -63,12 +70,12 @@ def test_captures_of_two_threads(stand_in):
     entered, leave, seen = threading.Event(), threading.Event(), []
 
     def other():
-        with _lib.capturing(object()):
+        with _lib.capturing(Graph()):
             entered.set()
             leave.wait(20)
             seen.append(gc.isenabled())
     t = threading.Thread(target=other)
-    with _lib.capturing(object()):
+    with _lib.capturing(Graph()):
         t.start()
         assert entered.wait(20)
     assert not gc.isenabled()

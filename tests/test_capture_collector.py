@@ -82,3 +82,14 @@ def test_captures_of_two_threads(stand_in):
     leave.set()
     t.join()
     assert seen == [False] and gc.isenabled()
+
+
+@pytest.mark.parametrize("inference", [True, False])
+@pytest.mark.parametrize("grad", [True, False])
+def test_the_body_runs_in_the_modes_of_the_caller(stand_in, inference, grad):
+    g = Graph()
+    with torch.inference_mode(inference), torch.set_grad_enabled(grad):
+        with _lib.capturing(g):
+            assert torch.is_inference_mode_enabled() == inference and torch.is_grad_enabled() == grad
+        assert torch.is_inference_mode_enabled() == inference and torch.is_grad_enabled() == grad
+    assert g.registered_in_mode is False

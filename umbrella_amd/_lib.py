@@ -493,12 +493,13 @@ def _collector_off():
 def capturing(graph):
     """torch.cuda.graph for launches of this library, the collector off (_collector_off).  The random generator has tensors that its first graph allocates and every
     capture writes while a graph is alive.  They are allocated outside inference mode, so that captures outside it may write them, and written inside it, where
-    those of a caller's own graph that was captured in the mode may be written too.  The body runs in the mode of the caller.  thread_local: other threads go on
+    those of a caller's own graph that was captured in the mode may be written too.  The body runs in the modes of the caller.  thread_local: other threads go on
     asking for events (a process group's watchdog), which a capture in global mode turns into an error."""
-    mode = torch.is_inference_mode_enabled()
+    mode, grad = torch.is_inference_mode_enabled(), torch.is_grad_enabled()
     with torch.inference_mode(False):
         graph.register_generator_state(torch.cuda.default_generators[torch.cuda.current_device()])
-    with _collector_off(), torch.inference_mode(True), torch.cuda.graph(graph, capture_error_mode="thread_local"), torch.inference_mode(mode):
+    with _collector_off(), torch.inference_mode(True), torch.cuda.graph(graph, capture_error_mode="thread_local"), torch.inference_mode(mode), \
+            torch.set_grad_enabled(grad):                      # (leaving inference mode turns gradients on)
         yield
 
 

@@ -627,7 +627,8 @@ typedef struct UmbSeqModel {
 
 /* activations of one step (caller-owned, sized for Tmax rows) */
 typedef struct UmbSeqWork {
-  float* x;        /* residual stream [Tmax][W] fp32 ([Tmax][streams][W] with several streams) */
+  float* x;        /* residual stream [Tmax][W] fp32 ([Tmax][streams][W] with several streams); of a step of T <= Tmax / 2 rows, rows T .. 2T - 1 are
+                      scratch too, and the last residual may stand there */
   void* h;         /* normed input of the current sublayer [Tmax][W] dtype */
   float* proj;     /* fused projection output [Tmax][max proj N] fp32 */
   float* aux;      /* q / alpha [Tmax][max heads*dim] fp32 */

@@ -86,3 +86,31 @@ def test_refuses_what_it_does_not_cover():
     assert rc(1, lambda f, t: setattr(f, "y", t["y"].data_ptr() + 4)) != 0
     assert rc(1, lambda f, t: setattr(f, "parts", 5)) != 0
     assert rc(1, lambda f, t: setattr(f, "groups", 3)) != 0
+
+
+@pytest.mark.parametrize("width,groups", [(64, 1), (192, 3)])
+def test_residuals_at_any_address(width, groups, monkeypatch):
+    """a step of a few rows whose workspace is not 16-byte aligned runs its seams by themselves"""
+    import types
+    import seqmix_helpers
+    from umbrella_amd import _lib
+    cfg = seqmix_helpers.config([seqmix_helpers.attn_layer(heads=6, kv_heads=2, dim=12, window=20, pool=3, ff=32)] * 2, width=width, vocab=50, groups=groups)
+    m, _ = seqmix_helpers.build(cfg, torch.float32, batch=2, max_length=32, max_tokens=64)
+    real, got, shifted = _lib.load_seq(), [], []
+
+    def forward(model, work, step, stream):
+        w = work._obj
+        shifted.append(torch.full((w.Tmax * width + 4,), 3.0, device="cuda"))
+        was, w.x = w.x, shifted[-1].data_ptr() + 4
+        try:
+            return real.umb_seq_forward(model, work, step, stream)
+        finally:
+            w.x = was
+    for shift in (False, True):
+        m.clear()
+        m.open(0)
+        if shift:
+            monkeypatch.setattr(_lib, "load_seq", lambda: types.SimpleNamespace(umb_seq_forward=forward))
+        got.append(torch.cat([m.forward_batch([(0, [7, 8, 9])]).clone(), m.forward_batch([(0, [5])]).clone()]).float())
+    assert len(shifted) == 2 and all(float(x[0]) == 3.0 and bool((x[-3:] == 3.0).all()) for x in shifted)
+    assert bool(torch.isfinite(got[0]).all()) and float((got[0] - got[1]).norm() / got[0].norm()) <= 1e-5

@@ -587,7 +587,8 @@ extern "C" int umb_seq_forward(const UmbSeqModel* m, const UmbSeqWork* given, co
   UmbSeqWork work = *given;                    // (its residual rows are where the last seam left them)
   UmbSeqWork* const ws = &work;
   Pending pend;
-  if (S <= 1 && !s->trace && T <= given->Tmax / 2) pend.spare = given->x + (size_t)T * W;
+  // (rows that the products can leave; a workspace without them goes to the seams, which take any alignment and refuse what is not there)
+  if (S <= 1 && !s->trace && T <= given->Tmax / 2 && given->x && given->h && (uintptr_t)given->x % 16 == 0) pend.spare = given->x + (size_t)T * W;
   // Every row's logits are wanted, in order (single tokens, scored texts): the last seam norms them for the head, which a launch of its own did in 5 us and
   // more.  (Of several streams the head reads the sum: not a seam's output.)
   const bool whole = s->R == T && !s->logit_rows && (!hyper || S == 1);

@@ -114,3 +114,19 @@ def test_residuals_at_any_address(width, groups, monkeypatch):
         got.append(torch.cat([m.forward_batch([(0, [7, 8, 9])]).clone(), m.forward_batch([(0, [5])]).clone()]).float())
     assert len(shifted) == 2 and all(float(x[0]) == 3.0 and bool((x[-3:] == 3.0).all()) for x in shifted)
     assert bool(torch.isfinite(got[0]).all()) and float((got[0] - got[1]).norm() / got[0].norm()) <= 1e-5
+
+
+@pytest.mark.parametrize("T,W,several", [(1, 4096, False), (410, 1024, False), (410, 2048, True), (600, 4096, True), (3, 6144, True)])
+def test_roundings_of_a_seams_two_products(T, W, several):
+    """written down, not the compiler's choice: which product of a sum of two is rounded by itself follows from how many quads a thread has"""
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + W)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")                                              # noqa: E731
+    x, y, mix, out, one, h = rnd(T, W), rnd(1, T, W), rnd(1), rnd(1), torch.ones(W, dtype=torch.bfloat16, device="cuda"), torch.empty(T, W, dtype=torch.bfloat16, device="cuda")
+    new = x.clone()
+    _lib.seq_call("umb_hc_seam_parts", new, h, y, 1, mix, out, 0.7, None, one, 0.0, T, W, 1, 1e-6, 1)
+    my = torch.tensor(0.7, device="cuda") * y[0]
+    want = [(mix.double() * x.double() + (out * my).double()).float(), (out.double() * my.double() + (mix * x).double()).float()]
+    # the fused product in 64 bits, rounded twice: another value than one rounding's in one of 2^29 sums
+    wrong = [int((new != w).sum()) for w in want]
+    assert wrong[not several] <= 2 < wrong[several], wrong

@@ -103,18 +103,21 @@ template <int NE, typename Off> __device__ __forceinline__ void add_parts(f32x4 
 }
 __device__ __forceinline__ float sq4(f32x4 v) { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3]; }
 
-// One residual stream's write, mx x + ot (m y), in the order of roundings that few rows have in every kernel
-__device__ __forceinline__ f32x4 stream_write(float mx, f32x4 x, float ot, float m, f32x4 y) {
+// One residual stream's write, mx x + ot (m y), by kernels with NE quads a thread.  The order of the two roundings is written down, and not the same in both:
+// the first product is rounded by itself where a thread has one quad (few rows, and those of up to 1024 elements; the products that form a seam's rows among
+// them), the second where it has several (from QUAD_ROWS rows on, and beyond 4096 elements).  A longer step's residual may so differ from a shorter one's in its
+// last bit.
+template <int NE> __device__ __forceinline__ f32x4 stream_write(float mx, f32x4 x, float ot, float m, f32x4 y) {
   f32x4 r;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) r[e] = fmaf(ot, m * y[e], mx * x[e]);
+  for (int e = 0; e < 4; ++e) r[e] = NE == 1 ? fmaf(ot, m * y[e], mx * x[e]) : fmaf(mx, x[e], ot * (m * y[e]));
   return r;
 }
 // and of two outputs side by side, a fa wa + b fb wb
-__device__ __forceinline__ f32x4 pair_sum(f32x4 a, float fa, f32x4 wa, f32x4 b, float fb, f32x4 wb) {
+template <int NE> __device__ __forceinline__ f32x4 pair_sum(f32x4 a, float fa, f32x4 wa, f32x4 b, float fb, f32x4 wb) {
   f32x4 r;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) r[e] = fmaf(b[e] * fb, wb[e], a[e] * fa * wa[e]);
+  for (int e = 0; e < 4; ++e) r[e] = NE == 1 ? fmaf(b[e] * fb, wb[e], a[e] * fa * wa[e]) : fmaf(a[e] * fa, wa[e], b[e] * fb * wb[e]);
   return r;
 }
 // block_sum of a row's squares with the waves' sums added in pairs: with 16 of them one after the other the scale of a row of 4096 was off by

@@ -73,8 +73,8 @@ __device__ __forceinline__ float two_products(float a, float b, float c, float d
   return a * b + c * d;
 }
 
-// The same values in 16 bits either way of rounding, whatever the compiler would make of a product in front of a conversion.  fp16: the product rounded to fp32 first
-// (opaque, so that it is), or once, as v_fma_mixlo_f16 does; bf16 has no such instruction.
+// The same values in 16 bits either way of rounding, whatever the compiler would make of a product in front of a conversion.  fp16: the product rounded to fp32
+// first (opaque, so that it is), or once, as v_fma_mixlo_f16 does; bf16 has no such instruction.
 __device__ __forceinline__ f32x4 rounded(f32x4 v) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) asm("" : "+v"(v[i]));

@@ -7,7 +7,7 @@
 // are waited for on a counter of their own: in the same wave a wait for the rows would be one for the weights in front of them).  Of a product's
 // workgroups each reads all rows, so this is for rows of a few thousand elements together: front_covers.
 // The arithmetic is the seams' and the products', sum for sum: a step's results are the same bits whichever way its seams run, and do not depend on
-// how many rows it has.  The residual is read by every workgroup and therefore not written in place: x_out is another buffer.
+// how many of these few rows it has.  The residual is read by every workgroup and therefore not written in place: x_out is another buffer.
 #include "seq_linear.h"
 
 constexpr int FRONT_MAX = 16;      // sets of 64 quads in all rows
@@ -160,7 +160,7 @@ __device__ __forceinline__ void front_rows(const UmbSeqFront& f, int T, unsigned
     factors(g, f.coef, 0);
     factors(gb, f.coef, 1);
 #pragma unroll
-    for (int i = 0; i < SETS; ++i) y[i] = pair_sum(y[i], g[i], w1[i].get(), y2[i], gb[i], w2[i].get());
+    for (int i = 0; i < SETS; ++i) y[i] = pair_sum<1>(y[i], g[i], w1[i].get(), y2[i], gb[i], w2[i].get());
     squares(y, 2);
     __syncthreads();
     factors(g, 1.f, 2);
@@ -174,7 +174,7 @@ __device__ __forceinline__ void front_rows(const UmbSeqFront& f, int T, unsigned
     const float mx = KIND == UMB_FRONT_STREAM && f.mix ? f.mix[0] : 1.f, ot = KIND == UMB_FRONT_STREAM && f.out ? f.out[0] : 1.f;
 #pragma unroll
     for (int i = 0; i < SETS; ++i) {
-      if constexpr (KIND == UMB_FRONT_STREAM) x[i] = stream_write(mx, x[i], ot, f.m, y[i]);
+      if constexpr (KIND == UMB_FRONT_STREAM) x[i] = stream_write<1>(mx, x[i], ot, f.m, y[i]);
       leave(i);
       x[i] = in0 * x[i];
     }

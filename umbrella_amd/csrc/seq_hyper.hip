@@ -249,9 +249,7 @@ __global__ __launch_bounds__(NT) void hc_seam_quad_kernel(float* __restrict__ x,
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int q = (int)threadIdx.x + NT * e;
-    f32x4 a;
-    if constexpr (NE == 1) a = stream_write(mx, xv[e], ot, m, yv[e]);
-    else a = mx * xv[e] + ot * (m * yv[e]);
+    const f32x4 a = stream_write<NE>(mx, xv[e], ot, m, yv[e]);
     xv[e] = in0 * a;
     if (q < nq) { *reinterpret_cast<f32x4*>(x + o + 4 * q) = a; ss += sq4(xv[e]); }
   }

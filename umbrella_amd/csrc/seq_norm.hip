@@ -442,8 +442,7 @@ __global__ __launch_bounds__(NT) void pair_resid_norm_quad_kernel(float* __restr
   float sm = 0.f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
-    if constexpr (NE == 1) a[e] = pair_sum(a[e], fa, wa[e], b[e], fb, wb[e]);
-    else a[e] = a[e] * fa * wa[e] + b[e] * fb * wb[e];
+    a[e] = pair_sum<NE>(a[e], fa, wa[e], b[e], fb, wb[e]);
     sm += (int)threadIdx.x + NT * e < nq ? sq4(a[e]) : 0.f;
   }
   const float fm = 1.f / sqrtf(row_sum<NT>(sm, red[2]) / (float)W + eps);

@@ -42,3 +42,25 @@ def test_capped_logits():
     _lib.seq_call("umb_seq_linear_cap", out, x, w, None, T, N, K, 30.0, _lib.seq_dtype_code(torch.bfloat16))
     want = 30.0 * torch.tanh(x.double() @ w.double().T / 30.0)
     assert bool((out[T] == 7.0).all()) and float((out[:T].double() - want).abs().max()) <= 2.0 ** -24 * (K / 8 + 64) * float((x.double().abs() @ w.double().abs().T).max())
+
+
+# chunks of 256 from the fewest on (5), either side of eight and of the ten that stay beyond 48 tokens; the squared activation
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T", [33, 48, 49, 64])
+@pytest.mark.parametrize("K", [1280, 1792, 2304, 2560, 2816, 3072, 3840])
+@pytest.mark.parametrize("rows,epi", [(4097, 2), (8200, 0), (16385, 4)])
+def test_products_of_any_chunks(dtype, T, K, rows, epi):
+    if epi != 4:
+        return test_products(dtype, T, K, rows, epi)
+    from umbrella_amd import _lib
+    code = _lib.seq_dtype_code(dtype)
+    g = torch.Generator(device="cuda").manual_seed(rows + K + T)
+    x, w = torch.randn(T, K, generator=g, device="cuda").to(dtype), (torch.randn(rows, K, generator=g, device="cuda") * K ** -0.5).to(dtype)
+    out, few = torch.full((T + 1, rows), 7.0, dtype=dtype, device="cuda"), torch.empty((32, rows), dtype=dtype, device="cuda")
+    _lib.seq_call("umb_seq_linear", out, x, w, None, T, rows, K, 4, code)
+    want, size = (x.double() @ w.double().T).relu(), x.double().abs() @ w.double().abs().T
+    bound = 2.0 ** -24 * (K / 8 + 16) * size                       # of a sum, as above; of its square twice the sum's times it
+    bound = 2.1 * bound * want + bound * bound + {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype] * want * want + 1e-7
+    assert bool((out[T] == 7.0).all()) and bool(((out[:T].double() - want * want).abs() <= bound).all())
+    _lib.seq_call("umb_seq_linear", few, x, w, None, 32, rows, K, 4, code)
+    assert torch.equal(out[:32], few)

@@ -140,9 +140,12 @@ static inline bool stream_pays(int T, int N, int K, int epi, int gz, int eb) {
 }
 
 // Streaming products of 33 to 64 tokens whose tokens stay in a workgroup's registers (seq_held.hip): where its 256 workgroups have more than one block of
-// rows each (with one there is nothing to keep for), and K is as many chunks as they hold: 8, or 16, of which beyond 48 tokens ten stay, at 450 of 512 registers.
+// rows each (with one there is nothing to keep for), and K is 5 chunks (as long as the weights' ring) to 16, all that stay with a wave up to 48 tokens at 450 of
+// 512 registers; of 64 tokens ten stay, the others are fetched again.  us, the streaming kernel / this, 33 / 48 / 64 tokens, gate/up 14336: K 1280 22.3 / 19.6,
+// 22.3 / 19.0, 26.7 / 21.1; 2560 37.3 / 30.0, 39.7 / 31.7, 45.0 / 33.9; 3584 48.7 / 39.4, 49.2 / 40.8, 55.7 / 47.0; 12304 rows: 1280 13.0 / 12.6, 13.5 / 12.8, 15.7 / 14.2.
+constexpr int HELD_MIN = 5, HELD_MAX = 16;
 static inline bool held_pays(int T, int N, int K, int epi) {
-  if (T <= 32 || T > 64 || !(epi_dual(epi) || epi == EPI_F32 || epi == EPI_DT || epi == EPI_CAP)) return false;
-  return (K == 2048 || K == 4096) && (N + 15) / 16 > (epi_dual(epi) ? 256 : 512);
+  return T > 32 && T <= 64 && (epi_plain(epi) || epi == EPI_CLAMP_GLU || epi == EPI_CAP) && K >= HELD_MIN * 256 && K <= HELD_MAX * 256 &&
+         (N + 15) / 16 > (epi_dual(epi) ? 256 : 512);
 }
 int held_stream(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, float limit, float alpha, int dtype, hipStream_t st);

@@ -130,3 +130,27 @@ def test_roundings_of_a_seams_two_products(T, W, several):
     # the fused product in 64 bits, rounded twice: another value than one rounding's in one of 2^29 sums
     wrong = [int((new != w).sum()) for w in want]
     assert wrong[not several] <= 2 < wrong[several], wrong
+
+
+# fp32 products that run on in two workgroups a unit; the last rows of weights that the one-tile kernel takes
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("kind", ["seam", "stream"])
+@pytest.mark.parametrize("T,W,groups,parts,N,epi", [(4, 512, 1, 1, 12304, 0), (1, 2048, 1, 1, 16400, 1), (2, 1024, 1, 2, 8208, 8), (1, 1000, 1, 1, 16384, 0), (5, 384, 1, 3, 20000, 4)])
+def test_long_products_as_two_launches(dtype, kind, T, W, groups, parts, N, epi):
+    test_as_two_launches(dtype, kind, T, W, groups, parts, N, epi)
+
+
+def test_where_rows_are_formed_inside():
+    """the lines of the rule, either side"""
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(0)
+
+    def ok(dtype, T, W, N, epi=0):
+        f, _ = _front(_lib, 0, T, W, 1, 1, dtype, g)
+        return _lib.load_seq().umb_seq_front_ok(C.byref(f), 1 << 20, T, N, epi, _lib.seq_dtype_code(dtype))
+    B, S = torch.bfloat16, torch.float32
+    assert ok(B, 1, 1000, 16384) and not ok(B, 1, 1000, 16385) and ok(S, 1, 1000, 16385)
+    assert ok(B, 1, 768, 65536) and not ok(B, 1, 768, 65537) and ok(B, 1, 640, 128256)
+    assert ok(B, 1, 512, 32768, 2) and not ok(B, 1, 512, 32770, 2) and ok(B, 1, 1024, 32770, 2) and ok(B, 1, 2048, 128256)
+    assert ok(S, 1, 4096, 8192) and not ok(S, 1, 4096, 8193) and ok(S, 1, 4096, 32768, 2) and ok(S, 1, 2048, 32000) and ok(B, 1, 4096, 32000)
+    assert ok(B, 2, 2048, 4096) and not ok(B, 2, 2048, 4097)

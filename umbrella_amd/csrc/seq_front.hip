@@ -5,7 +5,7 @@
 // 100 KB.  Every workgroup of the product can form the rows itself in less: its weights are asked for first, and the rows' operands, some 50 KB from
 // the caches, arrive beside them.  Four waves fetch weights and multiply, as in seq_linear.hip; four others form the rows in LDS and end (their loads
 // are waited for on a counter of their own: in the same wave a wait for the rows would be one for the weights in front of them).  Of a product's
-// workgroups each reads all rows, so this is for rows of a few thousand elements together: front_covers.
+// workgroups each reads all rows, so this is for rows of a few thousand elements together: front_form.
 // The arithmetic is the seams' and the products', sum for sum: a step's results are the same bits whichever way its seams run, and do not depend on
 // how many of these few rows it has.  The residual is read by every workgroup and therefore not written in place: x_out is another buffer.
 #include "seq_linear.h"
@@ -401,13 +401,21 @@ static int front_form(const UmbSeqFront* f, const void* w, int T, int N, int epi
   if (gs > 4096 || sets > FRONT_MAX || K % 8) return 0;
   // (front_slabs; a pair of fp32 weights does not fit the registers either way)
   if (sets > 8 && ((f->kind == UMB_FRONT_PAIR && (eb == 4 || f->parts > 1 || f->parts2 > 1)) || (!embed && eb == 4 && f->parts > 1))) return 0;
-  // Where it pays: the rows of several tokens beyond some 2000 elements are more reading in every workgroup than the seam's launch, but where workgroups are
-  // few.  us, the seam and the product / this, bf16: one row of 4096, N 4096 10.9 / 10.1, 6144 13.5 / 13.2, gate/up 28672 40.7 / 40.0; of 2048, N 4096 8.3 / 6.6, 32000
-  // 24.5 / 22.8, gate/up 16384 15.7 / 13.7; two of 2048, N 1024 8.3 / 6.8, 4096 8.4 / 8.1, 6144 9.5 / 9.9, 12304 12.6 / 13.7
-  if (sets > 8 && T > 1 && N > 4096) return 0;
+  // Where it pays: the rows are reading in every workgroup, in place of the seam's launch.  Up to eight sets, in however many rows, that is less wherever the
+  // streaming kernel runs; more sets are where they are one row's, or workgroups few.  us, the seam and the product / this, bf16: one row of 4096, N 4096 10.9 / 10.1,
+  // 6144 13.5 / 13.2, gate/up 28672 40.7 / 40.0; of 2048, N 4096 8.3 / 6.6, 32000 24.5 / 22.8, gate/up 16384 15.7 / 13.7; two of 2048, N 1024 8.3 / 6.8, 4096 8.4 / 8.1, 6144
+  // 9.5 / 9.9, 12304 12.6 / 13.7; four of 512, N 4096 5.6 / 3.9, 32000 13.0 / 10.5; eight of 256 5.1 / 3.8, 9.6 / 7.6; five of 192 4.7 / 3.5, 8.4 / 7.1; sixteen of 256,
+  // N 1024 5.0 / 4.6, 4096 5.4 / 5.2.  fp32: eight of 256, N 4096 5.9 / 4.1, 32000 15.3 / 13.4; one of 2048 10.6 / 8.4, 46 / 43; one of 4096, N 8192 27.7 / 27.1, but
+  // 9000 30.1 / 34.8 (its product is bound by the matrix pipes, and the four waves of a unit of which it has one workgroup are too few for them).
+  const bool dual = epi_dual(epi);
+  if (sets > 8 && ((T > 1 && N > 4096) || (eb == 4 && !dual && N > 8192))) return 0;
   const LinExt ext = lin_dense(N, K);
   if (stream_ok(w, w, N, K, epi, ext, eb) && stream_pays(T, N, K, epi, 1, eb)) return 1;
-  return K <= (epi_dual(epi) ? 1024 : 2048) ? 2 : 0;
+  // The one-tile kernel forms the rows for every 16 rows of weights, however many workgroups a unit works through.  16-bit weights of few steps are read in less than
+  // that takes: one row of 1000, 16400 10.5 / 9.9, 24000 12.8 / 13.2, 128256 45 / 54; of 1536, 12304 12.5 / 11.8, 20000 14.9 / 15.2; of 640, 128256 39.5 / 33.5; two
+  // of 768, 65536 24.3 / 23.2, 128256 41.1 / 42.7; gate/up of 512, 16384 11.3 / 10.6, 32768 15.8 / 15.8 (four rows 16.3 / 16.9).  fp32: 139 / 96 for two of 1000, N 128256.
+  if (eb == 2 && N > 16384 && K >= (dual ? 512 : 641) && (dual || K > 768 || N > 65536)) return 0;
+  return K <= (dual ? 1024 : 2048) ? 2 : 0;
 }
 
 extern "C" int umb_seq_front_ok(const UmbSeqFront* f, const void* w, int T, int N, int epi, int dtype) {
@@ -422,14 +430,15 @@ static int launch_front_as(int form, void* out, float* x_out, const UmbSeqFront&
   const size_t rows = (size_t)T * (K * sizeof(E) + 64);
   if (form == 1) {
     const int nc = (int)(K * sizeof(E) / 512);
-    // slots and workgroups as in launch_stream; more blocks than those run on inside one workgroup a unit, whose rows are formed once
+    // slots and workgroups as in launch_stream; more blocks than those run on inside one workgroup a unit, whose rows are formed once, or two of fp32 (one and
+    // two, us: four rows of 512, N 12304 9.8 / 8.4, 32000 18.2 / 14.4, the seam and the product 16.5; one of 2048 22.1 / 19.2, 43.6 / 42.3, 46.0)
 #define FRONT_STREAM(SLOTS, RUN, GRID)                                                                                                                   do {                                                                                                                                                     const size_t lds = FrontRing<DUAL, SLOTS>::R * FrontRing<DUAL, SLOTS>::SLOT + rows;                                                                   if (ensure_dynamic_lds<front_stream_kernel<P, DUAL, KIND, SETS, SLOTS, RUN>>(lds) != UMB_OK) return UMB_EHIP;                                         hipLaunchKernelGGL((front_stream_kernel<P, DUAL, KIND, SETS, SLOTS, RUN>), dim3(GRID), dim3(512), lds, st, out, (const E*)w, (const E*)bias, T, N, K, epi,                        limit, alpha, GRID, nc >= 8 ? 7 : 0, x_out, f);                                                                                   } while (0)
     if constexpr (DUAL) {
       if (blocks > 400 && nc >= 3) FRONT_STREAM(3, true, 256);
       else FRONT_STREAM(3, false, blocks);
     } else {
-      if (blocks > 512 && nc >= 5) FRONT_STREAM(5, true, 256);
-      else if (blocks > 512 && nc >= 3) FRONT_STREAM(3, true, 256);
+      if (blocks > 512 && nc >= 5 && sizeof(E) == 2) FRONT_STREAM(5, true, 256);
+      else if (blocks > 512 && nc >= 3) FRONT_STREAM(3, true, sizeof(E) == 2 ? 256 : 512);
       else if (blocks > 256) FRONT_STREAM(3, false, blocks);
       else FRONT_STREAM(4, false, blocks);
     }

@@ -827,8 +827,9 @@ static int launch_stream(void* out, const void* x, const void* w, const void* bi
     if (gy == 0 && gz == 1 && ext.parts <= 1 && !ext.tiles && ext.ldx == K && ext.ldo == N && held_pays(T, N, K, epi))
       return held_stream(out, x, w, bias, T, N, K, epi, ext.limit, ext.alpha, std::is_same<P, BF16>::value ? UMB_SEQ_BF16 : UMB_SEQ_F16, st);
   if (epi_dual(epi)) {
-    // up to some 1.5 blocks a unit they stand side by side: a second one behind the first would leave half of the units idle
-    const int held = blocks <= 400 ? 512 : 256;
+    // up to some 1.5 blocks a unit they stand side by side: a second one behind the first would leave half of the units idle (fp32: 1.75; 6912 x 1024 of
+    // one token side by side / behind one another 12.3 / 12.9, 8192 14.0 / 13.6)
+    const int held = blocks <= (F ? 448 : 400) ? 512 : 256;
     if (T <= 8) STREAM(1, 1, 4, true, 3, true, held);
     if (T <= 16) STREAM(1, 1, 8, true, 3, true, F ? 1 << 30 : held);
     if (T <= 32) {
@@ -856,7 +857,8 @@ static int launch_stream(void* out, const void* x, const void* w, const void* bi
   const bool narrow = stream_narrow(N, gy > 0 ? (gy + 1) / 2 : (T + 63) / 64, gz);    // about half of a tile list is in use
   if (T <= 32) {
     if (narrow) STREAM(1, 2, 16, false, 3, false, 0);
-    if (blocks <= 512 || (!F && stream_held((blocks + 1) / 2) == 256)) STREAM(2, 2, 16, false, 3, true, 256);
+    // (K of two chunks cannot run on in a ring of three: 24 tokens, 16400 x 512 10.7 / 7.7, 50000 x 512 26.6 / 15.8)
+    if (blocks <= 512 || (!F && chunks >= 3 && stream_held((blocks + 1) / 2) == 256)) STREAM(2, 2, 16, false, 3, true, 256);
     STREAM(2, 2, 16, false, 2, true, 512);
   }
   if (T <= 48) {

@@ -74,6 +74,8 @@ int umb_gemm_wide_split(int T, int N, int S_plan);
  * blocks (one block per CU sharing one staged copy of the activations). */
 int umb_gemm(void* out, const void* x, int ldx, const void* wpacked, const void* meta, int T, int N, int K,
              int awq, int S, int R, int epi, int dtype, umb_stream_t stream);
+/* the staged tile (csrc/gemm_tile.h's TILE_*) of such a product of more than 128 tokens with dense weights, where no mix of two tiles is ahead of it */
+int umb_gemm_tile_kind(int T, int N, int K, int S);
 
 /* Fused work around the GEMM.  RMSNorm is split in two: the producer of the residual stream folds the norm WEIGHT
  * into the activations it hands over (hw = h * w) and leaves per-64-column sums of squares (ssq [T][stride]); the

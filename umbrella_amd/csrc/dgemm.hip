@@ -160,6 +160,11 @@ static int dgemm_narrow(int T, int N, int K, int S, double* us) {
 // the tile by tile_kind (gemm_tile.h)
 static int dgemm_tile(int T, int N, int K, int S, double* us = nullptr) { return tile_kind(T, N, (K / 64 + S - 1) / S, S, K % (128 * S) == 0, us, TILE_KINDS); }
 
+extern "C" int umb_gemm_tile_kind(int T, int N, int K, int S) {
+  if (T <= 128 || N < 1 || K < 64 || S < 1) return UMB_EINVAL;
+  return dgemm_tile(T, N, K, S);
+}
+
 template <typename P>
 static int dgemm_any(const void* wp, const u16* x, int ldx, float* out, int T, int N, int K, int S, int epi, const GemmFused& fx, hipStream_t st) {
   if (T <= 128) {

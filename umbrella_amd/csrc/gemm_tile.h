@@ -75,7 +75,8 @@ enum { TILE_256 = 0,  //  256   256  1.42
        TILE_96 = 4,   //  256    96  0.73
        TILE_128 = 5,  //  128   128  0.49
        TILE_64K = 6,  //  128    64  0.38   K over two groups of waves
-       TILE_288 = 7,  //  256   288  2.06   A in fragments, many rounds: 257 tokens of 128256 x 8192 650 -> 565 us (two tiles of 160 before), 288 of x 4096 330 -> 299
+       TILE_288 = 7,  //  256   288  2.06   A in fragments: tokens that fill 288s in fewer rounds, us before / with it: 257 of 128256 x 8192 650 / 565 (two tiles of
+                      //                    160), 288 of x 4096 330 / 299, gate/up 28672 x 4096 of 513 138 / 117, 16384 x 2048 of 1130 78 / 68, 8192 x 4096 of 2250 142 / 120
        TILE_KINDS = 8 };
 struct Tile { int bn, bt; double us; };
 constexpr Tile TILES[TILE_KINDS] = {{256, 256, 1.42}, {256, 192, 1.20}, {256, 160, 1.04}, {256, 128, 0.86}, {256, 96, 0.73}, {128, 128, 0.49}, {128, 64, 0.38}, {256, 288, 2.06}};

@@ -64,3 +64,27 @@ def test_products_of_any_chunks(dtype, T, K, rows, epi):
     assert bool((out[T] == 7.0).all()) and bool(((out[:T].double() - want * want).abs() <= bound).all())
     _lib.seq_call("umb_seq_linear", few, x, w, None, 32, rows, K, 4, code)
     assert torch.equal(out[:32], few)
+
+
+@pytest.mark.parametrize("T,K,epi", [(48, 2048, 0), (64, 4096, 2), (49, 2816, 4)])
+def test_infinities_and_nan_stay_in_their_rows(T, K, epi):
+    from umbrella_amd import _lib
+    code, rows, bad, odd = _lib.seq_dtype_code(torch.bfloat16), 12300, (5, 20, 31, T - 1), (0, 4100, 12299)
+    g = torch.Generator(device="cuda").manual_seed(K + T)
+    N = 2 * rows if epi == 2 else rows
+    x, w = torch.randn(T, K, generator=g, device="cuda").bfloat16(), (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    out, few, clean = (torch.empty((t, rows), dtype=torch.bfloat16 if epi else torch.float32, device="cuda") for t in (T, 32, T))
+    _lib.seq_call("umb_seq_linear", clean, x, w, None, T, N, K, epi, code)
+    for t, v in zip(bad, (float("inf"), float("nan"), float("-inf"), float("nan"))):
+        x[t, (t * 37) % K] = v
+    for n, v in zip(odd, (float("nan"), float("inf"), float("nan"))):
+        w[n, K - 1 - n % 7] = v
+    _lib.seq_call("umb_seq_linear", out, x, w, None, T, N, K, epi, code)
+    _lib.seq_call("umb_seq_linear", few, x, w, None, 32, N, K, epi, code)
+    same = torch.isnan(out[:32]) == torch.isnan(few)
+    assert bool(same.all()) and torch.equal(out[:32][~torch.isnan(few)], few[~torch.isnan(few)])
+    rest = torch.ones(T, rows, dtype=torch.bool, device="cuda")
+    rest[list(bad)] = False
+    rest[:, list(odd)] = False
+    assert torch.equal(out[rest], clean[rest]) and bool(torch.isfinite(clean).all())
+    assert epi == 4 or not bool(torch.isfinite(out[:, 0]).any())         # (relu squared: fmaxf gives 0 for NaN, in every kernel)

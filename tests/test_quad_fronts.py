@@ -103,3 +103,74 @@ def test_head_gates_bit_by_bit(dtype, T, H, Dv, den, weights, kind):
                       _lib.seq_dtype_code(dtype))
         outs.append(out[:, :H * Dv])
     assert torch.equal(*outs)
+
+
+# ---- infinities, NaN and the ends of the range: where the kernels that take an element a lane have them, in no other row
+def _ends(x, seed):
+    """every eleventh row of x [rows, cols] with one of them somewhere"""
+    g = torch.Generator().manual_seed(seed)
+    for k, r in enumerate(range(3, x.shape[0], 11)):
+        x[r, int(torch.randint(x.shape[1], (1,), generator=g))] = (float("inf"), float("-inf"), float("nan"), 3e38, 0.0)[k % 5]
+        if k % 5 == 4:
+            x[r] = 0.0
+    return x
+
+
+def _same(a, b):
+    return torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(a[~torch.isnan(a)], b[~torch.isnan(b)])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("H,G,D,E,layout,rot,norm,mixed", [(32, 8, 64, 64, 0, 40, 1, True), (32, 8, 128, 128, 1, 64, 0, False), (16, 8, 128, 64, 0, 128, 1, False)])
+def test_ends_of_the_range_in_attention_slots(dtype, H, G, D, E, layout, rot, norm, mixed):
+    from umbrella_amd import _lib
+    T, code, ld = 1600, _lib.seq_dtype_code(dtype), (H + G) * D + G * E
+    g = torch.Generator(device="cuda").manual_seed(D + E)
+    proj, freq, firsts = torch.randn(T, ld, generator=g, device="cuda"), torch.rand(64, generator=g, device="cuda"), torch.randn(T, G * E, generator=g, device="cuda")
+    _ends(proj, D), _ends(firsts, E)
+    wq, wk = (torch.randn(D, generator=g, device="cuda").to(dtype) for _ in range(2))
+    pos, slot, outs = torch.arange(T, device="cuda", dtype=torch.int32), torch.zeros(T, device="cuda", dtype=torch.int32), []
+    for shift in (0, 1):
+        c, _, _, _ = prompt._decode_store([T], G, D, E, 0, dtype, 32, 1)
+        q, keep = torch.zeros(T * H * D + 4, device="cuda"), torch.zeros(T, G * E, device="cuda")
+        m = _lib.UmbValueMix(firsts.data_ptr(), keep.data_ptr(), 0.3, 0.0) if mixed else None
+        _lib.seq_call("umb_attn_prep_mix", q[shift:], c.struct(0), proj, ld, 1, wq if norm else None, wk if norm else None, norm, norm, pos, slot, freq, rot, layout,
+                      1.1, T, H, G, D, E, 1, 0.1, 100, 1e-5, m, code)
+        outs.append([q[shift:shift + T * H * D].clone(), keep, c.kv[0]["k"].float(), c.kv[0]["v"].float()])
+    assert all(_same(x, y) for x, y in zip(*outs))
+    rows = outs[0][0].view(T, H * D)
+    assert bool(torch.isfinite(rows[0]).all()) and 0 < int((~torch.isfinite(rows)).any(1).sum()) <= 4 * (T // 11 + 1) // 5 + 1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,rot", [(32, 8, 64, 64), (16, 8, 128, 60)])
+def test_ends_of_the_range_in_pooled_slots(dtype, H, G, D, rot):
+    from umbrella_amd import _lib
+    T, code = 1700, _lib.seq_dtype_code(dtype)
+    g = torch.Generator(device="cuda").manual_seed(D)
+    proj, freq = _ends(torch.randn(T, (H + G) * D, generator=g, device="cuda"), D), torch.rand(64, generator=g, device="cuda")
+    pos, slot, outs = torch.arange(T, device="cuda", dtype=torch.int32), torch.zeros(T, device="cuda", dtype=torch.int32), []
+    for shift in (0, 1):
+        c, _, _, _ = prompt._decode_store([T], G, D, D, 5, dtype, 32, 1)
+        q = torch.zeros(T * H * D + 4, device="cuda")
+        _lib.seq_call("umb_pwa_prep", q[shift:], c.struct(0), proj, proj.shape[1], pos, slot, freq, T, H, G, D, rot, 1e-5, code)
+        outs.append([q[shift:shift + T * H * D].clone(), c.kv[0]["k"].float(), c.kv[0]["v"].float()])
+    assert all(_same(x, y) for x, y in zip(*outs)) and bool(torch.isnan(outs[0][0]).any())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,Dv", [(1800, 11, 64), (2467, 7, 128), (601, 9, 256)])
+@pytest.mark.parametrize("den,kind", [(False, 0), (True, 1)])
+def test_ends_of_the_range_in_head_gates(dtype, T, H, Dv, den, kind):
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(T + Dv)
+    cols, outs = Dv + int(den), []
+    o, proj, mrun = (torch.randn(s, generator=g, device="cuda") for s in ((T * H, cols), (T, H * Dv), (T, H)))
+    _ends(o, Dv), _ends(proj, T)
+    mrun[5], mrun[6], mrun[7] = float("inf"), float("-inf"), float("nan")
+    for ldo in (H * Dv, H * Dv + 1):
+        out = torch.zeros((T, ldo), dtype=dtype, device="cuda")
+        _lib.seq_call("umb_head_gate", out, ldo, o, cols, Dv if den else -1, mrun if den else None, proj, H * Dv, 0, None, 0, kind, T, H, Dv, 1e-5, 1.2,
+                      _lib.seq_dtype_code(dtype))
+        outs.append(out[:, :H * Dv].float())
+    assert _same(*outs) and bool(torch.isnan(outs[0]).any()) and bool(torch.isfinite(outs[0]).any())

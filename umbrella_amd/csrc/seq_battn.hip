@@ -678,8 +678,11 @@ constexpr int ATT_SPAN = 256, LAT_SPAN = 64;
 // round is enough; and the first round's rows asked for in front of the preparation (us a launch inside a step, 20 / 16 KB of code: one token, two maps of
 // 128 | 256 10.3 / 7.9, sink heads of 128 8.0 / 7.1; 48 tokens, heads of 64 10.1 / 9.2).
 struct DecodePrep { AttnPrep a; const void *w_q, *w_k; const float* freq; };
+// (One map, values of 256 by four waves, prepared: three workgroups a unit, which the registers of the preparation alone would make two: 400 tokens, heads of
+// 256, 300 keys 112 / 125 us.)
 template <typename P, int RH, int LPR, int NW, int MAPS, bool LAT = false, bool PREP = false>
-__global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q, UmbPagedKV kv,
+__global__ __launch_bounds__(NW * 64, PREP && MAPS == 1 && LPR == 32 && NW == 4 ? 3 : 1)
+void attn_decode_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q, UmbPagedKV kv,
                                                               const float* __restrict__ proj, int ld, int gate_col,
                                                               const float* __restrict__ bias, int n_dist, const int* __restrict__ pos,
                                                               const int* __restrict__ slot_, int H, int G, int D, int window, float scale,
@@ -708,7 +711,10 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
   if (wave < nact) row = pkv_tok_row(kv, slot, key_pos(min(base + j, keys.n - 1)), g, G);
   typedef float quad __attribute__((ext_vector_type(4), aligned(4)));
   // The first round's rows are on their way while the token's own are prepared, which is as long as their trip: a lane asks for one word of each, its
-  // quarter's (all lines of a row up to 512 bytes), and the round finds them near.  Held in registers instead they cost the kernel of four rows a wave a SIMD
+  // quarter's (all lines of a row up to 512 bytes), and the round finds them near.  Held in registers instead they cost the kernel of four rows a wave a SIMD.
+  // Only where a wave has one round: of more the first is a small part, and asking twice took longer than it gave (two maps of 64, 2000 keys of two tokens
+  // 25.4 / 27.6 us).
+  const bool early = PREP && keys.n <= NW * 16;
   unsigned near_k = 0, near_v = 0;
   float bv[RR];
   auto biases = [&]() {
@@ -717,9 +723,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
     for (int r = 0; r < RR; ++r) bv[r] = bias ? bias[(long)(h0 + r) * n_dist + bi] : 0.f;
   };
   if (wave < nact) {
-    near_k = *reinterpret_cast<const unsigned*>(reinterpret_cast<const u16*>(kv.k) + (long)row * (MAPS * D) + quarter * (MAPS * D / 4));
-    if (!LAT) near_v = *reinterpret_cast<const unsigned*>(reinterpret_cast<const u16*>(kv.v) + (long)row * E + quarter * (E / 4));
-    biases();
+    if (early) near_k = *reinterpret_cast<const unsigned*>(reinterpret_cast<const u16*>(kv.k) + (long)row * (MAPS * D) + quarter * (MAPS * D / 4));
+    if (early && !LAT) near_v = *reinterpret_cast<const unsigned*>(reinterpret_cast<const u16*>(kv.v) + (long)row * E + quarter * (E / 4));
+    if (PREP) biases();
   }
   if constexpr (PREP) {
     const AttnPrep& a = prep.a;
@@ -757,6 +763,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
   }
   __syncthreads();
   if (wave < nact) {
+    if (PREP) asm volatile("" :: "v"(near_k), "v"(near_v));  // (asked for, whatever they hold; no registers in the rounds)
     float acc[RH * 8], m_run[RH], l_run[RH];
 #pragma unroll
     for (int r = 0; r < RH; ++r) { m_run[r] = -INFINITY; l_run[r] = 0.f; }
@@ -776,6 +783,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
           if (base + KPI * u + lane / LPR >= keys.n - 1) vv[u] = *reinterpret_cast<const u32x4*>(new_v + (lane & (LPR - 1)) * 8);
       }
       const u16* kr = reinterpret_cast<const u16*>(kv.k) + (long)row * (MAPS * D) + quarter * 8;
+      if (!PREP) biases();                                   // (a round ahead, two maps of 128 | 256, 400 tokens of 16 keys: 38.5 -> 46.7 us)
       // the next round of this wave: NW rounds on, or in the next of its workgroup's spans
       int next = base + NW * 16;
       if (nsplit > 1 && next / SPAN != base / SPAN) next += (nsplit - 1) * SPAN;
@@ -848,9 +856,8 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(u16* __restrict__ 
       }
       base = next;
       row = next_row;
-      if (base < keys.n) biases();
+      if (PREP && base < keys.n) biases();
     }
-    asm volatile("" :: "v"(near_k), "v"(near_v));            // (asked for, whatever they hold)
 #pragma unroll
     for (int r = 0; r < RH; ++r) {
       const float l = row_add16(l_run[r]);

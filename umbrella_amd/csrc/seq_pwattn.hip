@@ -525,8 +525,8 @@ __global__ __launch_bounds__(NW * 64) void pwa_attend_kernel(typename El<P>::typ
 // Before -> now, replayed from a graph, D 128: one token behind 40 / 2000 keys 10.7 -> 4.9 / 30.8 -> 18.0 us, 48 tokens behind 40 20.9 -> 5.7,
 // 64 behind 1000 77 -> 45.
 // PREP: steps of one token a sequence, as in seq_battn.hip: the queries come from the projection, the token's key and value stand in LDS for the round that
-// needs them, and the group's first workgroup appends them and the block that they complete.  Compact, and the first rows early, as there: 16 tokens, heads of
-// 128, 11.0 -> 10.6 us inside a step.
+// needs them, and the group's first workgroup appends them and the block that they complete.  Compact, as there: 16 tokens, heads of 128,
+// 11.0 -> 10.6 us inside a step (asking for the first rows early as well gives nothing there and took 45 -> 51 us of 48 tokens behind 2000 keys).
 struct PwaPrep { const float* freq; int rot_dims; float eps; };
 template <typename P, int RH, int LPR, int NW, bool PREP>
 __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ out, const float* __restrict__ q, UmbPagedKV kv,
@@ -551,13 +551,6 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
   };
   unsigned row = 0;
   if (wave < nact) row = row_of(wave);
-  // the first round's rows are on their way while the token's own are prepared, as in seq_battn.hip
-  unsigned near_k = 0, near_v = 0;
-  if (wave < nact) {
-    const long eb = wave < br ? 4 : 2, at = (long)row * D + quarter * (D / 4);
-    near_k = *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(wave < br ? (const void*)kv.kp : kv.k) + at * eb);
-    near_v = *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(wave < br ? (const void*)kv.vp : kv.v) + at * eb);
-  }
   if constexpr (PREP) {
     const float* src = proj + (long)t * ld;
     const bool append = h0 % (H / G) == 0;
@@ -702,7 +695,6 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
       }
       row = next_row;
     }
-    asm volatile("" :: "v"(near_k), "v"(near_v));            // (asked for, whatever they hold)
     store_groups<RH, LPR>(o_s + wave * RH * D, acc, lane);
   }
   __syncthreads();

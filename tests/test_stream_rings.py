@@ -26,3 +26,26 @@ def test_rings(dtype, K, rows, T, gated):
         bound = 1.1 * bound[:, :rows] * up.abs() + bound[:, rows:] * gate.abs() + {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -21}[dtype] * want.abs() + 1e-7
     assert bool((out[T] == 7.0).all())
     assert bool(((out[:T].double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("rows,gated", [(6500, True), (8300, True), (16500, False), (12304, False)])
+@pytest.mark.parametrize("T", [1, 9, 24, 40])
+def test_a_single_tile_of_a_group(rows, gated, T):
+    """a tile list of one tile: its blocks run on inside a unit's workgroups as a dense launch's do"""
+    from umbrella_amd import _lib
+    K, groups, dtype = 1280, 3, torch.bfloat16
+    code, N = _lib.seq_dtype_code(dtype), 2 * rows if gated else rows
+    g = torch.Generator(device="cuda").manual_seed(rows + T)
+    x, w = torch.randn(T + 5, K, generator=g, device="cuda").to(dtype), (torch.randn(groups, N, K, generator=g, device="cuda") * K ** -0.5).to(dtype)
+    made = dtype if gated else torch.float32
+    out = torch.full((T + 6, rows), 7.0, dtype=made, device="cuda")
+    tiles = torch.tensor([[2, 3, T]], dtype=torch.int32, device="cuda")
+    _lib.seq_call("umb_seq_linear_grouped", out, x, w, tiles, 1, 64, N * K, N, K, 2 if gated else 0, code)
+    xs = x[3:3 + T].contiguous()
+    full, size = xs.double() @ w[2].double().T, xs.double().abs() @ w[2].double().abs().T
+    bound = 2.0 ** -24 * (K / 8 + 16) * size
+    if gated:
+        gate, up = full[:, :rows], full[:, rows:]
+        full = torch.nn.functional.silu(gate) * up
+        bound = 1.1 * bound[:, :rows] * up.abs() + bound[:, rows:] * gate.abs() + 2.0 ** -8 * full.abs() + 1e-7
+    assert bool((out[:3] == 7.0).all()) and bool((out[3 + T:] == 7.0).all()) and bool(((out[3:3 + T].double() - full).abs() <= bound).all())

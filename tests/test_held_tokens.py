@@ -48,7 +48,7 @@ def test_capped_logits():
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T", [33, 48, 49, 64])
 @pytest.mark.parametrize("K", [1280, 1792, 2304, 2560, 2816, 3072, 3840])
-@pytest.mark.parametrize("rows,epi", [(4097, 2), (8200, 0), (16385, 4)])
+@pytest.mark.parametrize("rows,epi", [(4097, 2), (8200, 0), (16385, 4), (5121, 2), (10241, 0)])
 def test_products_of_any_chunks(dtype, T, K, rows, epi):
     if epi != 4:
         return test_products(dtype, T, K, rows, epi)

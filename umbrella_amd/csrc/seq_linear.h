@@ -143,9 +143,11 @@ static inline bool stream_pays(int T, int N, int K, int epi, int gz, int eb) {
 // rows each (with one there is nothing to keep for), and K is 5 chunks (as long as the weights' ring) to 16, all that stay with a wave up to 48 tokens at 450 of
 // 512 registers; of 64 tokens ten stay, the others are fetched again.  us, the streaming kernel / this, 33 / 48 / 64 tokens, gate/up 14336: K 1280 22.3 / 19.6,
 // 22.3 / 19.0, 26.7 / 21.1; 2560 37.3 / 30.0, 39.7 / 31.7, 45.0 / 33.9; 3584 48.7 / 39.4, 49.2 / 40.8, 55.7 / 47.0; 12304 rows: 1280 13.0 / 12.6, 13.5 / 12.8, 15.7 / 14.2.
+// Five chunks and a second block for an eighth of the workgroups or fewer: not (gate/up of 4112 and 4400, 48 tokens 9.5 / 10.4, 10.6 / 11.4; 5120 ahead).
 constexpr int HELD_MIN = 5, HELD_MAX = 16;
 static inline bool held_pays(int T, int N, int K, int epi) {
+  const int one = epi_dual(epi) ? 256 : 512;
   return T > 32 && T <= 64 && (epi_plain(epi) || epi == EPI_CLAMP_GLU || epi == EPI_CAP) && K >= HELD_MIN * 256 && K <= HELD_MAX * 256 &&
-         (N + 15) / 16 > (epi_dual(epi) ? 256 : 512);
+         (N + 15) / 16 > (K == HELD_MIN * 256 ? one + one / 8 : one);
 }
 int held_stream(void* out, const void* x, const void* w, const void* bias, int T, int N, int K, int epi, float limit, float alpha, int dtype, hipStream_t st);

@@ -526,7 +526,7 @@ __global__ __launch_bounds__(NW * 64) void pwa_attend_kernel(typename El<P>::typ
 // 64 behind 1000 77 -> 45.
 // PREP: steps of one token a sequence, as in seq_battn.hip: the queries come from the projection, the token's key and value stand in LDS for the round that
 // needs them, and the group's first workgroup appends them and the block that they complete.  Compact, as there: 16 tokens, heads of 128,
-// 11.0 -> 10.6 us inside a step (asking for the first rows early as well gives nothing there and took 45 -> 51 us of 48 tokens behind 2000 keys).
+// 11.0 -> 10.4 us inside a step.
 struct PwaPrep { const float* freq; int rot_dims; float eps; };
 template <typename P, int RH, int LPR, int NW, bool PREP>
 __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ out, const float* __restrict__ q, UmbPagedKV kv,
@@ -551,6 +551,14 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
   };
   unsigned row = 0;
   if (wave < nact) row = row_of(wave);
+  // The first round's rows are on their way while the token's own are prepared, where it is the only round, as in seq_battn.hip, and a unit has one workgroup
+  // (us a launch inside a step, without / with: 16 tokens, heads of 128 10.7 / 10.4; 128 tokens from a warm cache 15.9 / 17.6)
+  unsigned near_k = 0, near_v = 0;
+  if (PREP && NW == 16 && rounds <= NW && wave < nact) {
+    const long eb = wave < br ? 4 : 2, at = (long)row * D + quarter * (D / 4);
+    near_k = *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(wave < br ? (const void*)kv.kp : kv.k) + at * eb);
+    near_v = *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(wave < br ? (const void*)kv.vp : kv.v) + at * eb);
+  }
   if constexpr (PREP) {
     const float* src = proj + (long)t * ld;
     const bool append = h0 % (H / G) == 0;
@@ -582,6 +590,7 @@ __global__ __launch_bounds__(NW * 64) void pwa_decode_kernel(u16* __restrict__ o
   for (int r = 0; r < RH; ++r) bias[r] = pos_bias ? P::to_f(pos_bias[h0 + r]) : 0.f;
   __syncthreads();
   if (wave < nact) {
+    if (PREP && NW == 16) asm volatile("" :: "v"(near_k), "v"(near_v));      // (asked for, whatever they hold; no registers in the rounds)
     float acc[RH * 8];
 #pragma unroll
     for (int v = 0; v < RH * 8; ++v) acc[v] = 0.f;

@@ -51,9 +51,9 @@ def test_head_gates(dtype, T, H, Dv, den, weights, kind):
 @pytest.mark.parametrize("H,G,D,E,maps,layout,rot,append,norm,mixed", [(8, 2, 64, 64, 1, 0, 64, 1, 1, True), (9, 3, 128, 64, 2, 1, 80, 1, 0, False),
                                                                        (17, 17, 64, 128, 1, 1, 36, 1, 1, True), (30, 2, 128, 128, 1, 0, 48, 0, 1, False),
                                                                        (32, 8, 128, 128, 2, 0, 128, 1, 1, False), (32, 8, 64, 64, 1, 1, 0, 1, 1, False)])
-def test_attention_slots_bit_by_bit(dtype, H, G, D, E, maps, layout, rot, append, norm, mixed):
+def test_attention_slots_bit_by_bit(dtype, H, G, D, E, maps, layout, rot, append, norm, mixed, T=2880):
     from umbrella_amd import _lib
-    T, code = 2880, _lib.seq_dtype_code(dtype)
+    code = _lib.seq_dtype_code(dtype)
     g = torch.Generator(device="cuda").manual_seed(D + E)
     HQ, GK, GV = maps * H, append * maps * G, append * G
     ld = HQ * D + GK * D + GV * E + 5
@@ -69,6 +69,16 @@ def test_attention_slots_bit_by_bit(dtype, H, G, D, E, maps, layout, rot, append
                       freq if rot else None, rot, layout, 1.1, T, H, G, D, E, maps, 0.1, 100, 1e-5, m, code)
         outs.append([q[shift:shift + T * HQ * D].clone(), keep, c.kv[0]["k"], c.kv[0]["v"]])
     assert all(torch.equal(x, y) for x, y in zip(*outs))
+
+
+# few slots a token: the fewest that go in quads, one fewer, and waves whose last rows are none
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("H,G,D,E,maps,layout,rot,append,norm,mixed", [(3, 1, 128, 128, 1, 0, 128, 1, 1, True), (2, 1, 128, 64, 1, 1, 64, 1, 1, False), (2, 1, 64, 128, 1, 0, 32, 1, 1, True),
+                                                                       (1, 1, 64, 64, 1, 1, 64, 1, 1, False), (1, 1, 64, 64, 2, 0, 64, 0, 1, False),
+                                                                       (1, 1, 128, 128, 1, 1, 128, 0, 1, False), (3, 3, 64, 64, 1, 1, 64, 1, 0, True)])
+def test_few_attention_slots_bit_by_bit(dtype, H, G, D, E, maps, layout, rot, append, norm, mixed):
+    slots = maps * (H + append * G) + append * G
+    test_attention_slots_bit_by_bit(dtype, H, G, D, E, maps, layout, rot, append, norm, mixed, T=24576 // slots + 7)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])

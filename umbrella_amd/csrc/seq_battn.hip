@@ -197,7 +197,8 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(float* __restrict__ q, U
 // and keys, or values), two or four rows side by side, all loads in flight, and works the angles out once for all of them.
 // Vector work bounded what it replaces (four slots a wave, an element a lane, the angles again for every four: some 250 instructions a slot, quotients and
 // sines among them).  us, that / this, bf16: 2466 tokens, 32 + 8 + 8 slots of 64 33.9 / 16.2 (68 MB, 4.2 TB/s), 1999 tokens, 32 + 8 + 8 of 128 with mixed
-// values 34.8 / 24.9 (98 MB).  The sums and roundings are those of that kernel (quads_square, two_products): in the order that quads would take by themselves
+// values 34.8 / 24.9 (98 MB).  A wave's rows that are none are left out: two queries of 64, normed, of 28972 tokens 30.4 -> 20.5,
+// 8 + 2 + 2 slots of 64 of 7653 16.3 -> 14.8.  The sums and roundings are those of that kernel (quads_square, two_products): in the order that quads would take by themselves
 // 15.6 / 22.4, and the cached rows of a prompt were others.
 constexpr int PREP_QUADS = 4;
 constexpr int prep_rows(int D) { return PREP_QUADS * 256 / D; }      // rows a wave takes
@@ -232,6 +233,7 @@ __global__ __launch_bounds__(256) void attn_prep_quads_kernel(float* __restrict_
     for (int u = 0; u < PREP_QUADS; ++u) m[u] = ldq(ms + min(u * (256 / E) + sub, n - 1) * E);
 #pragma unroll
     for (int u = 0; u < PREP_QUADS; ++u) {
+      if (u * (256 / E) >= n) break;
       const int r = u * (256 / E) + sub;
       if (a.norm_v) v[u] = v[u] * quad_row_scale<E>(v[u], a.eps);
       if (r >= n) continue;
@@ -281,6 +283,7 @@ __global__ __launch_bounds__(256) void attn_prep_quads_kernel(float* __restrict_
   const long k0 = a.GK ? pkv_tok(kv, sl, p, 0, a.G, a.maps * D) : 0, k_group = (long)kv.page * a.maps * D;
 #pragma unroll
   for (int u = 0; u < PREP_QUADS; ++u) {
+    if (u * (256 / D) >= n) break;
     const int r = u * (256 / D) + sub, hs = first + min(r, n - 1), ks = hs - a.HQ;
     const bool is_q = ks < 0;
     if (a.norm_qk) {
@@ -303,9 +306,12 @@ __global__ __launch_bounds__(256) void attn_prep_quads_kernel(float* __restrict_
     else st4<P>(reinterpret_cast<El_*>(kv.k) + k0 + ks / a.maps * k_group + ks % a.maps * D + e, o);
   }
 }
-// where it can: whole quads on either side of a pair's distance; weights, queries and cached rows that quads are aligned in
+// Where it can: whole quads on either side of a pair's distance; weights, queries and cached rows that quads are aligned in.  And where it pays: from five
+// slots a token on, of 64 from four, without values from two.  Fewer are one wave of four slots, but two of quads, mostly empty (us, slots four by four / quads,
+// bf16, normed, turned, slots of 128: two queries, a key and a value of 67474 tokens 84.5 / 99.3, a query, a key and a value of 85519 112 / 131; three queries, a key
+// and a value of 41399 83.6 / 64.6; two queries, a key and a value of 64 of 47362 56.7 / 53.0; two queries of 64 of 28972 23.4 / 20.5).
 static inline bool prep_in_quads(const float* q, const UmbPagedKV* kv, const void* w_q, const void* w_k, const AttnPrep& a, int eb) {
-  return (a.D == 64 || a.D == 128) && (a.E == 64 || a.E == 128) && a.rot_dims % (a.layout == 0 ? 8 : 4) == 0 && (uintptr_t)q % 16 == 0 &&
+  return a.HQ + a.GK + a.GV >= (!a.GV ? 2 : a.D == 64 ? 4 : 5) && (a.D == 64 || a.D == 128) && (a.E == 64 || a.E == 128) && a.rot_dims % (a.layout == 0 ? 8 : 4) == 0 && (uintptr_t)q % 16 == 0 &&
          ((uintptr_t)w_q | (uintptr_t)w_k) % (4 * eb) == 0 && (!a.GV || ((uintptr_t)kv->k | (uintptr_t)kv->v) % (4 * eb) == 0);
 }
 

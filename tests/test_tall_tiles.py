@@ -10,8 +10,8 @@ def test_one_tile_of_288_rows(T, N, K):
     tiles.test_every_tile_of_packed_weights(T, N, K, 1)
 
 
-# several tiles of 288 tokens, the last of them in part, against fewer weight rows; K in slabs: of one stage each, two and three, and one past the last stage
-MORE = [(545, 28688, 384, 1), (576, 28672, 128, 1), (1150, 16384, 256, 1), (2250, 8176, 128, 1), (280, 28688, 128, 2), (288, 16400, 256, 2), (280, 65552, 384, 2), (280, 20496, 256, 3)]
+# several tiles of 288 tokens, the last of them in part, against fewer weight rows; K in slabs: of five stages, the fewest, six and seven, and a shorter last slab
+MORE = [(545, 28688, 384, 1), (576, 28672, 128, 1), (1150, 16384, 256, 1), (2250, 8176, 128, 1), (280, 28688, 640, 2), (560, 14352, 768, 2), (288, 18448, 896, 3), (280, 20496, 1280, 3)]
 
 
 def test_shapes_get_the_tile_of_288_rows():
@@ -19,6 +19,7 @@ def test_shapes_get_the_tile_of_288_rows():
     kind = _lib.load().umb_gemm_tile_kind
     assert all(kind(*s, 1) == 7 for s in [(257, 130064, 256), (288, 131056, 128), (273, 131072, 128), (288, 130064, 384)])
     assert all(kind(*s) == 7 for s in MORE) and kind(289, 130064, 256, 1) != 7 and kind(256, 130064, 256, 1) != 7
+    assert all(kind(*s) != 7 for s in [(280, 28688, 512, 2), (288, 16400, 256, 2), (280, 65552, 384, 2), (280, 20496, 256, 3)])      # slabs of fewer than five stages
     assert kind(128, 130064, 256, 1) < 0 and kind(300, 256, 0, 1) < 0
 
 

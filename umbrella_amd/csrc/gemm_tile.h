@@ -88,11 +88,13 @@ static inline double tile_cost(int kind, int T, int rows, int stages, int S) {
   const double load = rest / 256.0, products = stages * k.us, out = 2.1e-4 * k.bn * k.bt;
   return 4.0 + (wgs / 256) * (products + out + 2.0) + (rest ? products * (0.8 + 0.2 * load) + out * load + 2.0 : 0.0);
 }
-// the least of them (the K-split one takes an even number of stages); kinds: TILE_288 too where A lies in fragments
+// The least of them (the K-split one takes an even number of stages); kinds: TILE_288 too where A lies in fragments, with K whole or in slabs of five stages and
+// more: in shorter ones its two slots of B stand bare (those that the costs give to it, time without / with it: K whole 1.12 in the mean, 2094 of 2106 0.97 or more; slabs
+// of five stages and more 1.10, 2001 of 2066; shorter ones 1.03, a sixth of them under 0.97, 280 tokens of 22432 x 512 in three slabs 29.2 / 37.7 us).
 static inline int tile_kind(int T, int rows, int stages, int S, bool even, double* us = nullptr, int kinds = TILE_288) {
   int best = 0;
   for (int i = 1; i < kinds; ++i)
-    if ((i != TILE_64K || even) && tile_cost(i, T, rows, stages, S) < tile_cost(best, T, rows, stages, S)) best = i;
+    if ((i != TILE_64K || even) && (i != TILE_288 || S == 1 || stages >= 5) && tile_cost(i, T, rows, stages, S) < tile_cost(best, T, rows, stages, S)) best = i;
   if (us) *us = tile_cost(best, T, rows, stages, S);
   return best;
 }

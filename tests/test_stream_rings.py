@@ -28,6 +28,12 @@ def test_rings(dtype, K, rows, T, gated):
     assert bool(((out[:T].double() - want).abs() <= bound).all())
 
 
+# fp32 gate and up of more than 12 chunks, a workgroup a block; single matrices a few blocks beyond two rounds of 32 rows, and of none
+@pytest.mark.parametrize("T,K,rows,gated", [(1, 1664, 7184, True), (8, 1792, 12321, True), (4, 2048, 8200, True), (17, 1536, 20480, False), (32, 256, 18000, False), (32, 384, 20496, False)])
+def test_rings_of_fp32(T, K, rows, gated):
+    test_rings(torch.float32, K, rows, T, gated)
+
+
 @pytest.mark.parametrize("rows,gated", [(6500, True), (8300, True), (16500, False), (12304, False)])
 @pytest.mark.parametrize("T", [1, 9, 24, 40])
 def test_a_single_tile_of_a_group(rows, gated, T):

@@ -830,6 +830,9 @@ static int launch_stream(void* out, const void* x, const void* w, const void* bi
     // up to some 1.5 blocks a unit they stand side by side: a second one behind the first would leave half of the units idle (fp32: 1.75; 6912 x 1024 of
     // one token side by side / behind one another 12.3 / 12.9, 8192 14.0 / 13.6)
     const int held = blocks <= (F ? 448 : 400) ? 512 : 256;
+    // fp32 of more than 12 chunks: a workgroup a block, two on a unit -- one alone is too few waves for its products (us, one block behind the other / this: 2 tokens,
+    // 12320 x 1792 41.4 / 36.0, 5 tokens, 15328 x 1792 43.7 / 40.2; over 3000 launches of 450 to 2048 blocks 1 % behind to 5 % ahead in the median of a size)
+    if (F && chunks > 12 && T <= 8) STREAM(1, 1, 4, true, 3, false, 0);
     if (T <= 8) STREAM(1, 1, 4, true, 3, true, held);
     if (T <= 16) STREAM(1, 1, 8, true, 3, true, F ? 1 << 30 : held);
     if (T <= 32) {

@@ -154,3 +154,17 @@ def test_where_rows_are_formed_inside():
     assert ok(B, 1, 512, 32768, 2) and not ok(B, 1, 512, 32770, 2) and ok(B, 1, 1024, 32770, 2) and ok(B, 1, 2048, 128256)
     assert ok(S, 1, 4096, 8192) and not ok(S, 1, 4096, 8193) and ok(S, 1, 4096, 32768, 2) and ok(S, 1, 2048, 32000) and ok(B, 1, 4096, 32000)
     assert ok(B, 2, 2048, 4096) and not ok(B, 2, 2048, 4097)
+
+
+def test_where_a_pairs_rows_are_formed_inside():
+    """a pair's are more than a seam's: fewer rows of weights where every 16 of them form the rows"""
+    from umbrella_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(0)
+
+    def ok(dtype, T, W, N, epi=0, kind=2):
+        f, _ = _front(_lib, kind, T, W, 1, 1, dtype, g)
+        return _lib.load_seq().umb_seq_front_ok(C.byref(f), 1 << 20, T, N, epi, _lib.seq_dtype_code(dtype))
+    B, S = torch.bfloat16, torch.float32
+    assert ok(B, 1, 256, 8192) and not ok(B, 1, 256, 8193) and ok(B, 1, 256, 8193, kind=0) and ok(S, 1, 128, 8192) and not ok(S, 1, 128, 8193)
+    assert ok(B, 1, 384, 12288) and not ok(B, 1, 384, 12289) and ok(B, 1, 384, 16384, 2) and not ok(B, 1, 384, 16386, 2) and not ok(S, 1, 200, 8193)
+    assert ok(S, 1, 384, 32000) and ok(B, 1, 2048, 32000) and ok(B, 1, 4096, 28672, 2)               # a ring that runs on forms them once a workgroup

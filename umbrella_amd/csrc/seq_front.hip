@@ -410,7 +410,13 @@ static int front_form(const UmbSeqFront* f, const void* w, int T, int N, int epi
   const bool dual = epi_dual(epi);
   if (sets > 8 && ((T > 1 && N > 4096) || (eb == 4 && !dual && N > 8192))) return 0;
   const LinExt ext = lin_dense(N, K);
-  if (stream_ok(w, w, N, K, epi, ext, eb) && stream_pays(T, N, K, epi, 1, eb)) return 1;
+  const bool ring = stream_ok(w, w, N, K, epi, ext, eb) && stream_pays(T, N, K, epi, 1, eb);
+  // A pair's rows are twice the sums and four barriers: formed for every 16 rows of weights (the one-tile kernel, and a ring whose K is too short to run on) they
+  // are more than the seam's launch from 8192 rows of weights on, of single matrices and 384 elements from 12288.  16 bits: one row of 64, 9168 5.6 / 6.5, 21536
+  // 7.0 / 9.9; of 192, 33520 10.1 / 14.6; of 384, 10400 7.5 / 7.9 in four slabs, 1.05 ahead in the mean there, two rows, 23792 10.8 / 12.8; of 768, 39120 19.6 / 24.2;
+  // gate/up, two of 64, 14272 6.8 / 8.3; fp32, one of 128, 10768 7.5 / 9.2, 38256 14.0 / 23.2.
+  if (f->kind == UMB_FRONT_PAIR && N > (!dual && eb == 2 && K >= 384 ? 12288 : 8192) && (!ring || (long)K * eb < 3 * 512)) return 0;
+  if (ring) return 1;
   // The one-tile kernel forms the rows for every 16 rows of weights, however many workgroups a unit works through.  16-bit weights of few steps are read in less than
   // that takes: one row of 1000, 16400 10.5 / 9.9, 24000 12.8 / 13.2, 128256 45 / 54; of 1536, 12304 12.5 / 11.8, 20000 14.9 / 15.2; of 640, 128256 39.5 / 33.5; two
   // of 768, 65536 24.3 / 23.2, 128256 41.1 / 42.7; gate/up of 512, 16384 11.3 / 10.6, 32768 15.8 / 15.8 (four rows 16.3 / 16.9).  fp32: 139 / 96 for two of 1000, N 128256.

@@ -684,10 +684,14 @@ constexpr int ATT_SPAN = 256, LAT_SPAN = 64;
 // round is enough; and the first round's rows asked for in front of the preparation (us a launch inside a step, 20 / 16 KB of code: one token, two maps of
 // 128 | 256 10.3 / 7.9, sink heads of 128 8.0 / 7.1; 48 tokens, heads of 64 10.1 / 9.2).
 struct DecodePrep { AttnPrep a; const void *w_q, *w_k; const float* freq; };
-// (One map, values of 256 by four waves, prepared: three workgroups a unit, which the registers of the preparation alone would make two: 400 tokens, heads of
-// 256, 300 keys 112 / 125 us.)
+// (One map, by four waves, prepared: as many workgroups a unit as an element a lane's preparation left, of which the pairs' registers would cost one -- three for
+// values of 256: 400 tokens, heads of 256, 300 keys 112 / 125 us; four for values of 128 in fp16: 32 heads of 64 | 128, 125 tokens of 12 keys 10.3 / 15.7, 99 of 2463
+// keys 187 / 234.  In bf16 they are three either way: held to four some values spill, 118 tokens of 11 keys 15.9 -> 10.5, but 150 of 1464 keys 167 -> 199.)
+template <typename P> constexpr int decode_waves(int LPR, int NW, int MAPS, bool PREP) {
+  return !PREP || MAPS > 1 || NW != 4 ? 1 : LPR == 32 ? 3 : LPR == 16 && std::is_same<P, F16>::value ? 4 : 1;
+}
 template <typename P, int RH, int LPR, int NW, int MAPS, bool LAT = false, bool PREP = false>
-__global__ __launch_bounds__(NW * 64, PREP && MAPS == 1 && LPR == 32 && NW == 4 ? 3 : 1)
+__global__ __launch_bounds__(NW * 64, decode_waves<P>(LPR, NW, MAPS, PREP))
 void attn_decode_kernel(u16* __restrict__ out, int ldo, const float* __restrict__ q, UmbPagedKV kv,
                                                               const float* __restrict__ proj, int ld, int gate_col,
                                                               const float* __restrict__ bias, int n_dist, const int* __restrict__ pos,
